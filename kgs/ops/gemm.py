@@ -12,6 +12,7 @@ in-pod workload runs on the hand-written MFMA kernel.
 from __future__ import annotations
 
 import os
+from functools import lru_cache
 
 import torch
 
@@ -73,23 +74,28 @@ def gemm_nt(
         _check_operand(out, "out")
         if tuple(out.shape) != (M, N):
             raise ValueError(f"out has shape {tuple(out.shape)}, expected {(M, N)}")
-    rc = _lib.lib().kgs_gemm_bf16_nt(
-        a.data_ptr(),
-        b.data_ptr(),
-        out.data_ptr(),
-        bias.data_ptr() if bias is not None else None,
-        M,
-        N,
-        K,
-        a.stride(0),
-        b.stride(0),
-        out.stride(0),
-        epi,
-        VARIANTS[variant],
-        _lib.stream_handle(a.device),
-    )
+    ptrs = (a.data_ptr(), b.data_ptr(), out.data_ptr(), bias.data_ptr() if bias is not None else None, M, N, K,
+            a.stride(0), b.stride(0), out.stride(0), epi)
+    if variant == "auto":
+        ws = _scratch(M, N, K, a.device)
+        rc = _lib.lib().kgs_gemm_bf16_nt_auto(*ptrs, None if ws is None else ws.data_ptr(), _lib.stream_handle(a.device))
+    else:
+        rc = _lib.lib().kgs_gemm_bf16_nt(*ptrs, VARIANTS[variant], _lib.stream_handle(a.device))
     _lib.check(rc, f"gemm_nt[{M}x{N}x{K}]")
     return out
+
+
+@lru_cache(maxsize=4096)
+def _scratch_floats(m: int, n: int, k: int) -> int:
+    return int(_lib.lib().kgs_gemm_bf16_nt_scratch(m, n, k))
+
+
+def _scratch(m: int, n: int, k: int, device) -> torch.Tensor | None:
+    """Scratch for a product's K slices, None where it has none. Each call's own, from the
+    caching allocator (in a hipGraph capture from the graph's pool), so that products on
+    several streams or threads never share it."""
+    need = _scratch_floats(m, n, k)
+    return torch.empty(need, dtype=torch.float32, device=device) if need else None
 
 
 _SPLITK_WS: dict = {}
@@ -520,6 +526,28 @@ TR_READ_A = False        # route K-major A through ds_read_b64_tr_b16 (else tran
 TR_READ_B_MAX_M = 4096   # K-major B: tr reads up to this M, transpose + NT above
 
 
+@lru_cache(maxsize=4096)
+def _tr_slices(m: int, n: int, k: int, ta: bool, tb: bool) -> int:
+    return int(_lib.lib().kgs_gemm_bf16_tr_slices(m, n, k, int(ta), int(tb)))
+
+
+def _rows16(t: torch.Tensor) -> bool:
+    """Rows of whole, aligned 16-byte chunks."""
+    return t.stride(0) % 8 == 0 and t.data_ptr() % 16 == 0
+
+
+def _gemm_tr(a, b, out, M, N, K, ta, tb, ns) -> torch.Tensor:
+    """K-major operands read in place on small tiles, over ``ns`` K slices (gemm_any.hip)."""
+    if out is None:
+        out = torch.empty((M, N), dtype=torch.bfloat16, device=a.device)
+    ws = torch.empty(ns * M * ((N + 7) // 8 * 8), dtype=torch.float32, device=a.device) if ns > 1 else None
+    rc = _lib.lib().kgs_gemm_bf16_tr(a.data_ptr(), b.data_ptr(), out.data_ptr(), M, N, K, a.stride(0), b.stride(0),
+                                     out.stride(0), ta, tb, ns, None if ws is None else ws.data_ptr(),
+                                     _lib.stream_handle(a.device))
+    _lib.check(rc, f"gemm_tr[{M}x{N}x{K}, ta={ta}, tb={tb}]")
+    return out
+
+
 def gemm_bf16(a: torch.Tensor, b: torch.Tensor, trans_a: bool = False, trans_b: bool = False,
          bias: torch.Tensor | None = None, act: str | None = None, out: torch.Tensor | None = None) -> torch.Tensor:
     """``op(a) @ op(b)`` for row-major bf16 matrices, any of the four layouts:
@@ -540,6 +568,12 @@ def gemm_bf16(a: torch.Tensor, b: torch.Tensor, trans_a: bool = False, trans_b: 
     if K != K2:
         raise ValueError(f"inner dims differ: op(a) {M}x{K}, op(b) {K2}x{N}")
     ta, tb = int(trans_a), int(not trans_b)  # kernel flags: 1 = operand stored [K][rows]
+    if (ta or tb) and bias is None and act in (None, "none") and not TR_READ_A and _rows16(a) and _rows16(b) and \
+            a.shape[1] % 8 == 0 and b.shape[1] % 8 == 0 and (out is None or tuple(out.shape) == (M, N)) and \
+            M and N and 0 < (K + 128) * max(a.stride(0), b.stride(0)) < 1 << 30:
+        ns = _tr_slices(M, N, K, bool(ta), bool(tb))
+        if ns:
+            return _gemm_tr(a, b, out, M, N, K, ta, tb, ns)
     if ta and not TR_READ_A:
         # measured: the tr-read A path runs ~20 % behind a 6.3 TB/s transpose + NT
         # at 8192^3 and ties at 4096^3 (profiles/gemm_layouts.json)

@@ -1,0 +1,654 @@
+// bf16 NT GEMM for any M, N and K % 8 == 0 on the four-wave K-step of gemm_w4.h: the kernel
+// behind kgs_gemm_bf16_nt wherever the persistent 256x256 grid does not apply -- ragged sizes,
+// and products of too few 256x256 tiles to fill the chip.
+//
+//   C[M, N] = epilogue(A[M, K] . B[N, K]^T + bias)
+//
+// What bounds such a product is the number of CUs that get a tile and the length of one
+// workgroup's serial chain of K-steps, so the tile (256x256, 256x128 or 128x128) and the number
+// of K slices are chosen by sizes (any_plan below). 128x128 tiles keep a quarter of the AGPRs, so
+// two workgroups share a CU and one's barriers and loads hide behind the other's MFMAs.
+//
+// Ragged sizes cost two selects per K-step: rows past M or N lie outside the buffer resources,
+// which end at the last valid element, and a lane whose 16-byte chunk of K lies past K gets an
+// offset outside them too; all of these arrive in LDS as zeros. K is walked in whole pairs of
+// 64-wide steps. Stores are predicated by row and column; a C whose rows are not 16-byte aligned
+// takes 2-byte stores.
+//
+// The order of the products in every accumulator is gemm_w4.h's, so without K slices the result
+// is bitwise the aligned kernels'. With slices each one writes fp32 partial tiles, which
+// any_reduce sums in a fixed order before the epilogue.
+#include <utility>
+
+#include "gemm_w4.h"
+
+namespace kgs {
+namespace any {
+
+using w4::BK;
+using w4::Ctx;
+using w4::Frag;
+
+constexpr int OOB = 0x7FFFFFF0;  // above every buffer resource's size (any_ok)
+
+// What a launch stores. DUAL: C gets bf16(acc + bias) and C2 the activation of that bf16 value
+// (a training forward pass, whose backward pass needs both).
+struct Args {
+  const unsigned short* A;
+  const unsigned short* B;
+  void* C;                     // bf16 [M, ldc], or fp32 partials [slices][M][ldc]
+  unsigned short* C2;          // DUAL
+  const unsigned short* bias;  // null: none
+  int M, N, K, lda, ldb, ldc;
+  int ks;                      // K of a slice, a multiple of 128
+  int tall;                    // tile groups along N (M > N): see launch
+  int vec;                     // 16-B stores: ldc % 8 == 0 and C (C2) 16-B aligned
+};
+
+template <int BM, int BN>
+constexpr int waves_per_simd() { return BM == 128 && BN == 128 ? 2 : 1; }
+
+template <int EPI>
+__device__ __forceinline__ unsigned pack_epi(float a, float b, float ba, float bb) {
+  return pack_bf16x2(epilogue<EPI>(a, ba), epilogue<EPI>(b, bb));
+}
+
+// the activation of an already rounded pre-activation; a NaN stays one
+template <int EPI>
+__device__ __forceinline__ float act_of(unsigned short z) {
+  const float v = bf2f(z);
+  if constexpr (EPI == EPI_BIAS_RELU) return v < 0.f ? 0.f : v;
+  return epilogue<EPI>(v, 0.f);
+}
+template <int EPI>
+__device__ __forceinline__ unsigned act_pair(unsigned z) {
+  return pack_bf16x2(act_of<EPI>((unsigned short)(z & 0xffff)), act_of<EPI>((unsigned short)(z >> 16)));
+}
+
+// 8 columns from `col` of a row: one 16-B store, or the valid columns one by one
+__device__ __forceinline__ void store8(unsigned short* row, int col, int N, int vec, uint4 v) {
+  if (vec && col + 8 <= N) {
+    *(uint4*)(row + col) = v;
+    return;
+  }
+  const unsigned u[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+  for (int e = 0; e < 8; ++e)
+    if (col + e < N) row[col + e] = (unsigned short)(u[e >> 1] >> (16 * (e & 1)));
+}
+
+template <int EPI, int BM, int BN, bool SPLIT, bool DUAL>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(waves_per_simd<BM, BN>(), waves_per_simd<BM, BN>())))
+void gemm_nt_any(Args a) {
+  using S = w4::Shape<BM, BN>;
+  using Kn = w4::Knobs<BM, BN>;
+  constexpr int MA = S::MA, NB = S::NB, ND = w4::dma_per_stage<BM, BN>();
+  __shared__ __attribute__((aligned(1024))) char smem[2 * S::STAGE];
+  const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int ntm = (a.M + BM - 1) / BM, ntn = (a.N + BN - 1) / BN;
+  int slice, tm, tn;
+  if (a.tall) w4::tile_of<40000000, SPLIT>((int)blockIdx.x, (int)gridDim.x, ntm, ntn, slice, tm, tn);
+  else w4::tile_of<0, SPLIT>((int)blockIdx.x, (int)gridDim.x, ntm, ntn, slice, tm, tn);
+  const int m0 = tm * BM, n0 = tn * BN;
+  const int k0 = SPLIT ? slice * a.ks : 0;
+  const int kn = SPLIT ? min(a.K - k0, a.ks) : a.K;  // this slice's valid K
+
+  Ctx c;
+  c.smem = smem;
+  c.w = w;
+  c.wr = w >> 1;
+  c.wc = w & 1;
+  c.nt = (kn + 2 * BK - 1) / (2 * BK) * 2;
+  // resources end with the last valid element: nothing outside the operands is ever read
+  const int ra = min(a.M - m0, BM), rb = min(a.N - n0, BN);
+  c.ra = __builtin_amdgcn_make_buffer_rsrc((void*)(a.A + (long)m0 * a.lda + k0), 0, ((ra - 1) * a.lda + kn) * 2, 0x00020000);
+  c.rb = __builtin_amdgcn_make_buffer_rsrc((void*)(a.B + (long)n0 * a.ldb + k0), 0, ((rb - 1) * a.ldb + kn) * 2, 0x00020000);
+  c.sa32 = 32 * a.lda * 2;
+  c.sb32 = 32 * a.ldb * 2;
+  const int row = w * 8 + (lane >> 3);
+  const int ch = ((lane & 7) ^ ((row >> 1) & 7)) * 8;  // first column of this lane's chunk in a K-tile
+  const int voa = (row * a.lda + ch) * 2, vob = (row * a.ldb + ch) * 2;
+  const int fr = lane & 15, fq = lane >> 4;
+  c.ro0 = fr * 128 + ((fq ^ (fr >> 1)) * 16);
+  c.ro1 = fr * 128 + (((4 + fq) ^ (fr >> 1)) * 16);
+  // offsets of the next DMAs: outside the resources where K-tile kt's chunk lies past K
+  auto aim = [&](int kt) {
+    const bool in = kt * BK + ch < kn;
+    c.voa = in ? voa : OOB;
+    c.vob = in ? vob : OOB;
+  };
+
+  if constexpr (BM == 128 && BN == 128) KGS_ACC_RESERVE_QUARTER();
+  else KGS_ACC_RESERVE();
+  w4::static_for<0, MA * NB>([](auto q) { accr::zero<decltype(q)::value>(); });
+
+#pragma unroll
+  for (int st = 0; st < 2; ++st) {
+    aim(st);
+#pragma unroll
+    for (int j = 0; j < ND; ++j) w4::dma_any<BM, BN, 0>(c, st, j, st * BK);
+  }
+  w4::wait_vm<ND>();
+  w4::bar();
+  Frag<MA, NB> f0, f1;
+  {
+    const char* pa = w4::abase<BM, BN, 0>(c, 0);
+    const char* pb = w4::bbase<BM, BN, 0>(c, 0);
+#pragma unroll
+    for (int e = 0; e < S::NR; ++e) {
+      const int x = w4::rd_idx(Kn::ORD, MA, NB, e);
+      if (w4::rd_isa(Kn::ORD, MA, NB, e)) f0.a[x] = w4::frag(pa + x * 2048);
+      else f0.b[x] = w4::frag(pb + x * 2048);
+    }
+  }
+  __builtin_amdgcn_s_waitcnt(0xc07f);
+
+  for (int t = 0; t < c.nt; t += 2) {
+    aim(min(t + 2, c.nt - 1));
+    w4::kstep<BM, BN, 0, Kn::B1, Kn::R, Kn::P, Kn::ORD, 0>(c, f0, f1, t);
+    aim(min(t + 3, c.nt - 1));
+    w4::kstep<BM, BN, 1, Kn::B1, Kn::R, Kn::P, Kn::ORD, 0>(c, f0, f1, t + 1);
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // drain the tail re-loads before LDS is released
+  asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 3" ::: "memory");  // MFMA -> v_accvgpr_read hazard
+
+  const int mw = m0 + c.wr * (BM / 2) + fr, nw = n0 + c.wc * (BN / 2);
+  if constexpr (SPLIT) {
+    // ldc is a multiple of 8: a fragment's four columns are inside the row or all outside
+    float* part = (float*)a.C + (long)slice * a.M * a.ldc;
+    w4::static_for<0, MA>([&](auto ic) {
+      constexpr int i = decltype(ic)::value;
+      f32x4 v[NB];
+      w4::read_row<NB, i>(v);
+      if (mw + i * 16 >= a.M) return;
+      float* prow = part + (long)(mw + i * 16) * a.ldc;
+#pragma unroll
+      for (int n = 0; n < NB; ++n) {
+        const int col = nw + n * 16 + fq * 4;
+        if (col < a.ldc) *(f32x4*)(prow + col) = v[n];
+      }
+    });
+    return;
+  }
+  float bv[NB][4];
+#pragma unroll
+  for (int n = 0; n < NB; ++n) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) bv[n][e] = 0.f;
+    if constexpr (epi_bias<EPI>()) {
+      const int col = nw + n * 16 + fq * 4;
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (a.bias && col + e < a.N) bv[n][e] = bf2f(a.bias[col + e]);
+    }
+  }
+  const int lc = (fq & 1) * 16 + (fq >> 1) * 8;  // this lane's 8 of a fragment pair's 32 columns
+  w4::static_for<0, MA>([&](auto ic) {
+    constexpr int i = decltype(ic)::value;
+    const int r = mw + i * 16;
+    const bool row_ok = r < a.M;
+    unsigned short* crow = (unsigned short*)a.C + (long)r * a.ldc;
+    uint4 old[NB / 2];
+    if constexpr (EPI == EPI_ADDC) {  // N % 8 == 0 and 16-B rows (kgs_gemm_bf16_nt_any)
+#pragma unroll
+      for (int p = 0; p < NB / 2; ++p) {
+        const int col = nw + p * 32 + lc;
+        old[p] = row_ok && col < a.N ? *(const uint4*)(crow + col) : make_uint4(0, 0, 0, 0);
+      }
+    }
+    f32x4 v[NB];
+    w4::read_row<NB, i>(v);
+#pragma unroll
+    for (int n = 0; n < NB; n += 2) {
+      uint2 o[2];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        constexpr int E = DUAL ? EPI_BIAS : EPI;
+        o[h].x = pack_epi<E>(v[n + h][0], v[n + h][1], bv[n + h][0], bv[n + h][1]);
+        o[h].y = pack_epi<E>(v[n + h][2], v[n + h][3], bv[n + h][2], bv[n + h][3]);
+      }
+      auto sx = __builtin_amdgcn_permlane16_swap(o[0].x, o[1].x, false, false);
+      auto sy = __builtin_amdgcn_permlane16_swap(o[0].y, o[1].y, false, false);
+      uint4 q = make_uint4(sx[0], sy[0], sx[1], sy[1]);
+      const int col = nw + n * 16 + lc;
+      if (row_ok && col < a.N) {
+        if constexpr (EPI == EPI_ADDC) q = add_bf16x8(old[n / 2], q);
+        store8(crow, col, a.N, a.vec, q);
+        if constexpr (DUAL)
+          store8(a.C2 + (long)r * a.ldc, col, a.N, a.vec,
+                 make_uint4(act_pair<EPI>(q.x), act_pair<EPI>(q.y), act_pair<EPI>(q.z), act_pair<EPI>(q.w)));
+      }
+    }
+  });
+}
+
+// Products with operands stored K-major (A as [K, M], B as [K, N]): Linear's backward pass, whose
+// dX = dY . W reads W that way and dW = dY^T . X both operands, at the sizes where transposing them
+// first costs more than a smaller tile does (layout_plan below). 128x128 tiles, two workgroups
+// per CU, one barrier per 64-wide K-step: K-tile t + 1 is on its way while t is multiplied.
+//
+// A K-major K-tile is 64 rows of 128 columns (256 B). The 16-byte chunk c of row r lies at
+// c ^ 2 (r & 3 | (r >> 3 & 1) << 2), so that the 16 chunks that a half wave of transposed reads
+// touches are on 16 bank groups. Rows past K lie outside the resource and arrive as zeros; columns
+// past M or N only reach outputs that are not stored.
+struct TrArgs {
+  const unsigned short* A;
+  const unsigned short* B;
+  void* C;
+  int M, N, K, lda, ldb, ldc, ks, vec;
+};
+
+// Four fragments (16 columns each) of k-sub KS of a K-major operand: eight transposed reads and
+// their wait in one block, so that no read is in flight where the compiler does not see it.
+template <int KS>
+__device__ __forceinline__ void tr_read4(bf16x8 (&f)[4], const unsigned (&ad)[4]) {
+  bf16x4 v[8];
+  asm volatile(
+      "ds_read_b64_tr_b16 %0, %8 offset:%c12\n\tds_read_b64_tr_b16 %1, %8 offset:%c13\n\t"
+      "ds_read_b64_tr_b16 %2, %9 offset:%c12\n\tds_read_b64_tr_b16 %3, %9 offset:%c13\n\t"
+      "ds_read_b64_tr_b16 %4, %10 offset:%c12\n\tds_read_b64_tr_b16 %5, %10 offset:%c13\n\t"
+      "ds_read_b64_tr_b16 %6, %11 offset:%c12\n\tds_read_b64_tr_b16 %7, %11 offset:%c13\n\t"
+      "s_waitcnt lgkmcnt(0)"
+      : "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2]), "=&v"(v[3]), "=&v"(v[4]), "=&v"(v[5]), "=&v"(v[6]), "=&v"(v[7])
+      : "v"(ad[0]), "v"(ad[1]), "v"(ad[2]), "v"(ad[3]), "n"(KS * 8192), "n"(KS * 8192 + 1024)
+      : "memory");
+#pragma unroll
+  for (int i = 0; i < 4; ++i) f[i] = __builtin_shufflevector(v[2 * i], v[2 * i + 1], 0, 1, 2, 3, 4, 5, 6, 7);
+}
+
+// One operand of the K-major kernel: TR as described, else K-contiguous as in gemm_nt_any.
+template <bool TR>
+struct Operand {
+  __amdgpu_buffer_rsrc_t r;
+  int vo, step, kstep;  // lane's byte offset, bytes between DMA instructions and between K-tiles
+  int ch, kn;
+  unsigned ro[4];       // fragment reads: byte offsets inside a stage's operand
+
+  __device__ void init(const unsigned short* P, int ld, int p0, int rows, int k0, int kn_, int w, int lane, int half) {
+    kn = kn_;
+    const int fr = lane & 15, fq = lane >> 4;
+    const int n = min(rows - p0, 128);
+    if constexpr (TR) {
+      r = __builtin_amdgcn_make_buffer_rsrc((void*)(P + (long)k0 * ld + p0), 0, ((kn - 1) * ld + n) * 2, 0x00020000);
+      const int row = w * 4 + (lane >> 4);  // of the 16 rows that the four waves' instruction brings
+      const int c = (lane & 15) ^ (2 * ((row & 3) | ((row >> 3) & 1) << 2));
+      vo = row * ld * 2 + c * 16;
+      step = 16 * ld * 2;
+      kstep = BK * ld * 2;
+      const int q = (lane >> 2) & 3, p = lane & 3, kr = 8 * fq + q;  // a read's row, and its place in it
+      const int x = 2 * ((kr & 3) | ((kr >> 3) & 1) << 2);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) ro[i] = kr * 256 + (((half * 8 + 2 * i) ^ x) + (p >> 1)) * 16 + (p & 1) * 8;
+    } else {
+      r = __builtin_amdgcn_make_buffer_rsrc((void*)(P + (long)p0 * ld + k0), 0, ((n - 1) * ld + kn) * 2, 0x00020000);
+      const int row = w * 8 + (lane >> 3);
+      ch = ((lane & 7) ^ ((row >> 1) & 7)) * 8;
+      vo = (row * ld + ch) * 2;
+      step = 32 * ld * 2;
+      kstep = BK * 2;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) ro[i] = (half * 64 + i * 16 + fr) * 128 + ((fq ^ (fr >> 1)) * 16);
+    }
+  }
+  // K-tile t into the 16 KiB at dst
+  __device__ void load(char* dst, int t, int w) const {
+    const int v = TR || t * BK + ch < kn ? vo : OOB;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (KGS_LDS void*)(dst + (j * 4 + w) * 1024), 16, v, j * step + t * kstep, 0, 0);
+  }
+  template <int KS>
+  __device__ void read(bf16x8 (&f)[4], const char* src) const {
+    if constexpr (TR) {
+      const unsigned b = (unsigned)(uintptr_t)(const KGS_LDS char*)src;
+      const unsigned ad[4] = {b + ro[0], b + ro[1], b + ro[2], b + ro[3]};
+      tr_read4<KS>(f, ad);
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) f[i] = *(const bf16x8*)(src + (KS ? ro[i] ^ 64 : ro[i]));
+    }
+  }
+};
+
+template <bool TA, bool TB, bool SPLIT>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_tr(TrArgs a) {
+  __shared__ __attribute__((aligned(1024))) char smem[2 * 32768];
+  const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int ntm = (a.M + 127) / 128, ntn = (a.N + 127) / 128;
+  int slice, tm, tn;
+  w4::tile_of<0, SPLIT>((int)blockIdx.x, (int)gridDim.x, ntm, ntn, slice, tm, tn);
+  const int m0 = tm * 128, n0 = tn * 128, k0 = SPLIT ? slice * a.ks : 0;
+  const int kn = SPLIT ? min(a.K - k0, a.ks) : a.K, nt = (kn + BK - 1) / BK;
+  Operand<TA> oa;
+  Operand<TB> ob;
+  oa.init(a.A, a.lda, m0, a.M, k0, kn, w, lane, w >> 1);
+  ob.init(a.B, a.ldb, n0, a.N, k0, kn, w, lane, w & 1);
+  f32x4 acc[4][4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int n = 0; n < 4; ++n) acc[i][n] = f32x4{0.f, 0.f, 0.f, 0.f};
+  oa.load(smem, 0, w);
+  ob.load(smem + 16384, 0, w);
+  for (int t = 0; t < nt; ++t) {
+    char* st = smem + (t & 1) * 32768;
+    char* nx = smem + ((t & 1) ^ 1) * 32768;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // own part of K-tile t
+    w4::bar();  // every wave's part, and every wave has read K-tile t - 1
+    if (t + 1 < nt) {
+      oa.load(nx, t + 1, w);
+      ob.load(nx + 16384, t + 1, w);
+    }
+    bf16x8 fa[4], fb[4];
+    oa.template read<0>(fa, st);
+    ob.template read<0>(fb, st + 16384);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int n = 0; n < 4; ++n) acc[i][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[n], fa[i], acc[i][n], 0, 0, 0);
+    bf16x8 ga[4], gb[4];
+    oa.template read<1>(ga, st);
+    ob.template read<1>(gb, st + 16384);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int n = 0; n < 4; ++n) acc[i][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(gb[n], ga[i], acc[i][n], 0, 0, 0);
+  }
+  const int fr = lane & 15, fq = lane >> 4;
+  const int mw = m0 + (w >> 1) * 64 + fr, nw = n0 + (w & 1) * 64;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int r = mw + i * 16;
+    if constexpr (SPLIT) {
+      float* prow = (float*)a.C + ((long)slice * a.M + r) * a.ldc;
+#pragma unroll
+      for (int n = 0; n < 4; ++n) {
+        const int col = nw + n * 16 + fq * 4;
+        if (r < a.M && col < a.ldc) *(f32x4*)(prow + col) = acc[i][n];
+      }
+    } else {
+      unsigned short* crow = (unsigned short*)a.C + (long)r * a.ldc;
+#pragma unroll
+      for (int n = 0; n < 4; n += 2) {
+        uint2 o[2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+          o[h] = make_uint2(pack_bf16x2(acc[i][n + h][0], acc[i][n + h][1]), pack_bf16x2(acc[i][n + h][2], acc[i][n + h][3]));
+        auto sx = __builtin_amdgcn_permlane16_swap(o[0].x, o[1].x, false, false);
+        auto sy = __builtin_amdgcn_permlane16_swap(o[0].y, o[1].y, false, false);
+        const int col = nw + n * 16 + (fq & 1) * 16 + (fq >> 1) * 8;
+        if (r < a.M && col < a.N) store8(crow, col, a.N, a.vec, make_uint4(sx[0], sy[0], sx[1], sy[1]));
+      }
+    }
+  }
+}
+
+// Sum of the K slices' partial tiles (fp32 [ns][M][ldp]) and the epilogue: a thread's 8 columns
+// of one row, every slice's loads issued before the first add. Bound by memory: ns + 0.5 passes.
+template <int EPI, bool DUAL>
+__global__ __launch_bounds__(256) void any_reduce(const float* __restrict__ P, unsigned short* __restrict__ C,
+                                                  unsigned short* __restrict__ C2, const unsigned short* __restrict__ bias,
+                                                  int M, int N, int ldc, int ldp, int ns, int vec) {
+  const int per = ldp / 8;
+  const long id = (long)blockIdx.x * 256 + threadIdx.x;
+  if (id >= (long)M * per) return;
+  const int row = (int)(id / per), col = (int)(id - (long)row * per) * 8;
+  const float* p = P + (long)row * ldp + col;
+  const long step = (long)M * ldp;
+  f32x4 s0 = *(const f32x4*)p, s1 = *(const f32x4*)(p + 4);
+  for (int s = 1; s < ns; s += 4) {
+    f32x4 u[4], v[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float* q = p + min(s + e, ns - 1) * step;
+      u[e] = *(const f32x4*)q;
+      v[e] = *(const f32x4*)(q + 4);
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (s + e < ns) {
+        s0 += u[e];
+        s1 += v[e];
+      }
+  }
+  float b[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    b[e] = 0.f;
+    if constexpr (epi_bias<EPI>())
+      if (bias && col + e < N) b[e] = bf2f(bias[col + e]);
+  }
+  constexpr int E = DUAL ? EPI_BIAS : EPI;
+  uint4 q = make_uint4(pack_epi<E>(s0[0], s0[1], b[0], b[1]), pack_epi<E>(s0[2], s0[3], b[2], b[3]),
+                       pack_epi<E>(s1[0], s1[1], b[4], b[5]), pack_epi<E>(s1[2], s1[3], b[6], b[7]));
+  unsigned short* crow = C + (long)row * ldc;
+  if constexpr (EPI == EPI_ADDC) q = add_bf16x8(*(const uint4*)(crow + col), q);
+  store8(crow, col, N, vec, q);
+  if constexpr (DUAL)
+    store8(C2 + (long)row * ldc, col, N, vec,
+           make_uint4(act_pair<EPI>(q.x), act_pair<EPI>(q.y), act_pair<EPI>(q.z), act_pair<EPI>(q.w)));
+}
+
+struct Plan {
+  int bm, bn, ns;
+};
+
+inline int ceil_div(long a, long b) { return (int)((a + b - 1) / b); }
+
+// Microseconds of a launch, as measured on an MI355X (weights streamed from HBM).
+inline double cost(long M, long N, long K, int bm, int bn, int ns, int cus) {
+  const int pairs = ceil_div(K, 128), steps = 2 * ceil_div(pairs, ns);
+  const long wg = (long)ceil_div(M, bm) * ceil_div(N, bn) * ns;
+  const int share = bm == 128 && bn == 128 ? 2 : 1;  // workgroups that one CU runs at a time
+  const double full = (double)wg / cus;
+  // a K-step's time by how full the chip is, one workgroup per CU
+  const double busy = full < 1 ? full : 1;
+  double step = bm == 256 ? (bn == 256 ? 0.92 + 0.30 * busy : 0.62 + 0.18 * busy) : 0.46 + 0.08 * busy;
+  double rounds = ceil_div(wg, cus);
+  if (share == 2 && full > 1) {  // pairs of workgroups overlap
+    const int two = (int)(wg / (2L * cus)), rest = (int)(wg - 2L * cus * two);
+    rounds = two * 1.5 + (rest > cus ? 1.5 : rest > 0 ? 1 : 0);
+  }
+  double t = 4 + rounds * steps * step;
+  if (ns > 1) t += 4 + (2.0 * ns + 0.5) * M * N * 4 / 5.5e6;
+  return t;
+}
+
+// The tile and the slices of a product. A slice keeps at least 512 of K: the partial tiles of
+// shorter ones cost as much as they save (300 x 304 x 2400: 10.6 us in slices of 640, 9.9 of 384).
+// Slices have to promise 15 %: below that the estimate is not sure of them (1024 x 768 x 2048), and
+// without them the result keeps the bits that it has in every other layout.
+inline Plan plan(long M, long N, long K, bool split, int cus) {
+  Plan best{256, 256, 1};
+  double t0 = 1e30;
+  const int shapes[3][2] = {{256, 256}, {256, 128}, {128, 128}};
+  for (auto& s : shapes)
+    for (int ns = 1; ns <= 16; ++ns) {
+      if (ns > 1 && (!split || K < 512L * ns)) break;
+      const double t = cost(M, N, K, s[0], s[1], ns, cus) * (ns > 1 ? 1.15 : 1.0);
+      if (t < t0) {
+        t0 = t;
+        best = {s[0], s[1], ns};
+      }
+    }
+  return best;
+}
+
+// Slices with which gemm_tr is the fastest way to a product with K-major operands, 0 where
+// another one is. The others transpose the operands first (a launch and a pass over memory each)
+// and run cost()'s best tile, or, for aligned sizes and a K-major B alone, the 256x256 kernel that
+// reads it transposed. Measured, us: 2048^3 both K-major 26 here, 42 with transposes; 4096^3 128
+// and 105; 64 x 512 x 2048 9.5 in 8 slices and 33. Slices have to promise a quarter of the time
+// here: they cost the result the bits that it has in every other layout.
+inline int layout_plan(long M, long N, long K, int ta, int tb, int cus) {
+  const long wg = (long)ceil_div(M, 128) * ceil_div(N, 128);
+  double t0 = 1e30;
+  int best = 1;
+  for (int ns = 1; ns <= 16; ++ns) {
+    if (ns > 1 && K < 512L * ns) break;
+    const long n = wg * ns;
+    const double busy = n < cus ? (double)n / cus : 1, step = 0.58 + 0.12 * busy;
+    const int two = (int)(n / (2L * cus)), rest = (int)(n - 2L * cus * two);
+    const double rounds = two * 1.42 + (rest > cus ? 1.42 : rest > 0 ? 1 : 0);
+    double t = 4 + rounds * 2 * ceil_div(ceil_div(K, 128), ns) * step;
+    if (ns > 1) t = 1.35 * (t + 4 + (2.0 * ns + 0.5) * M * N * 4 / 5.5e6);
+    if (t < t0) {
+      t0 = t;
+      best = ns;
+    }
+  }
+  const double turn_a = ta ? 4 + 4.0 * M * K / 5e6 : 0, turn_b = tb ? 4 + 4.0 * N * K / 5e6 : 0;
+  double nt = 1e30;
+  for (auto& s : {std::pair<int, int>{256, 256}, {256, 128}, {128, 128}}) {
+    const double t = cost(M, N, K, s.first, s.second, 1, cus);
+    nt = t < nt ? t : nt;
+  }
+  if (K % 8) return best;  // nothing else reads such operands 16 bytes at a time
+  if (t0 > nt + turn_a + turn_b) return 0;
+  if (M % 256 == 0 && N % 256 == 0 && K % 128 == 0 && tb && M <= 4096) {
+    const long g = (M / 256) * (N / 256);
+    const double busy = g < cus ? (double)g / cus : 1;
+    if (t0 > 4 + ceil_div(g, cus) * (K / 64) * (0.98 + 0.32 * busy) + turn_a) return 0;
+  }
+  return best;
+}
+
+template <int EPI, int BM, int BN, bool DUAL>
+void launch_tile(const Args& a, int ns, hipStream_t s) {
+  const dim3 grid((unsigned)(ceil_div(a.M, BM) * ceil_div(a.N, BN) * ns));
+  if (ns > 1) hipLaunchKernelGGL((gemm_nt_any<EPI_NONE, BM, BN, true, false>), grid, dim3(256), 0, s, a);
+  else hipLaunchKernelGGL((gemm_nt_any<EPI, BM, BN, false, DUAL>), grid, dim3(256), 0, s, a);
+}
+
+template <int EPI, bool DUAL>
+int launch(Args a, Plan p, float* ws, hipStream_t s) {
+  Args g = a;
+  const int ldp = (a.N + 7) / 8 * 8;
+  g.ks = ceil_div(ceil_div(a.K, 128), p.ns) * 128;
+  p.ns = ceil_div(a.K, g.ks);  // no empty slice
+  if (p.ns > 1) {
+    g.C = ws;
+    g.ldc = ldp;
+  }
+  if (p.bm == 128) launch_tile<EPI, 128, 128, DUAL>(g, p.ns, s);
+  else if (p.bn == 128) launch_tile<EPI, 256, 128, DUAL>(g, p.ns, s);
+  else launch_tile<EPI, 256, 256, DUAL>(g, p.ns, s);
+  if (p.ns > 1)
+    hipLaunchKernelGGL((any_reduce<EPI, DUAL>), dim3((unsigned)ceil_div((long)a.M * (ldp / 8), 256)), dim3(256), 0, s, ws,
+                       (unsigned short*)a.C, a.C2, a.bias, a.M, a.N, a.ldc, ldp, p.ns, a.vec);
+  return (int)hipGetLastError();
+}
+
+}  // namespace any
+
+int cu_count();  // gemm_bf16.hip
+
+// The operands gemm_tr takes. K-major: whole 16-byte chunks of columns, 32-bit offsets over K.
+int gemm_tr_ok(const void* A, const void* B, int M, int N, int K, int lda, int ldb, int ta, int tb) {
+  if (M <= 0 || N <= 0 || K <= 0 || lda % 8 || ldb % 8 || lda < (ta ? M : K) || ldb < (tb ? N : K)) return 0;
+  if ((uintptr_t)A % 16 || (uintptr_t)B % 16) return 0;
+  if ((ta ? M : K) % 8 || (tb ? N : K) % 8) return 0;
+  const long ea = ta ? (long)(K + 128) * lda : 256L * lda, eb = tb ? (long)(K + 128) * ldb : 256L * ldb;
+  if (2 * ea >= any::OOB || 2 * eb >= any::OOB) return 0;
+  return ((long)M + 127) / 128 * (((long)N + 127) / 128) * 64 < (1L << 31);
+}
+
+int gemm_tr(const void* A, const void* B, void* C, int M, int N, int K, int lda, int ldb, int ldc, int ta, int tb, int ns,
+            float* ws, hipStream_t s) {
+  using namespace any;
+  TrArgs a{(const unsigned short*)A, (const unsigned short*)B, C, M, N, K, lda, ldb, ldc, 0,
+           ldc % 8 == 0 && (uintptr_t)C % 16 == 0};
+  const int ldp = (N + 7) / 8 * 8, vec = a.vec;
+  a.ks = ceil_div(ceil_div(K, 128), ns) * 128;
+  ns = ceil_div(K, a.ks);
+  if (ns > 1) {
+    if (!ws) return KGS_ERR_ARG;
+    a.C = ws;
+    a.ldc = ldp;
+  }
+  const dim3 grid((unsigned)(ceil_div(M, 128) * ceil_div(N, 128) * ns));
+#define KGS_TR(TA, TB)                                                                        \
+  if (ns > 1) hipLaunchKernelGGL((any::gemm_tr<TA, TB, true>), grid, dim3(256), 0, s, a);    \
+  else hipLaunchKernelGGL((any::gemm_tr<TA, TB, false>), grid, dim3(256), 0, s, a)
+  if (ta && tb) { KGS_TR(true, true); }
+  else if (ta) { KGS_TR(true, false); }
+  else if (tb) { KGS_TR(false, true); }
+  else return KGS_ERR_ARG;
+#undef KGS_TR
+  if (ns > 1)
+    hipLaunchKernelGGL((any_reduce<EPI_NONE, false>), dim3((unsigned)ceil_div((long)M * (ldp / 8), 256)), dim3(256), 0, s, ws,
+                       (unsigned short*)C, nullptr, nullptr, M, N, ldc, ldp, ns, vec);
+  return (int)hipGetLastError();
+}
+
+// The operands the kernel takes: 16-byte rows and chunks, 32-bit offsets over a tile's rows.
+int gemm_any_ok(const void* A, const void* B, int M, int N, int K, int lda, int ldb) {
+  if (M <= 0 || N <= 0 || K <= 0 || K % 8 || lda % 8 || ldb % 8) return 0;
+  if ((uintptr_t)A % 16 || (uintptr_t)B % 16) return 0;
+  if ((long)lda * 512 >= any::OOB || (long)ldb * 512 >= any::OOB) return 0;
+  return ((long)M + 127) / 128 * (((long)N + 127) / 128) * 16 < (1L << 31);
+}
+
+// C2: DUAL's second output, else null. bm, bn, ns: 0 for the plan's choice. ws: fp32 scratch for
+// the plan's slices (kgs_gemm_bf16_nt_any_ws), null: no slices.
+int gemm_any(const void* A, const void* B, void* C, void* C2, const void* bias, int M, int N, int K, int lda, int ldb,
+             int ldc, int epi, int bm, int bn, int ns, float* ws, hipStream_t s) {
+  using namespace any;
+  const int vec = ldc % 8 == 0 && (uintptr_t)C % 16 == 0 && (uintptr_t)C2 % 16 == 0;
+  if (epi == EPI_ADDC && (!vec || N % 8)) return KGS_ERR_ALIGN;
+  Plan p = bm ? Plan{bm, bn, ns} : plan(M, N, K, ws != nullptr, cu_count());
+  if (p.ns > 1 && ws == nullptr) return KGS_ERR_ARG;
+  const Args a{(const unsigned short*)A, (const unsigned short*)B, C, (unsigned short*)C2, (const unsigned short*)bias,
+               M, N, K, lda, ldb, ldc, 0, M > N, vec};
+  if (C2) {
+    switch (epi) {
+      case EPI_BIAS_GELU: return launch<EPI_BIAS_GELU, true>(a, p, ws, s);
+      case EPI_BIAS_RELU: return launch<EPI_BIAS_RELU, true>(a, p, ws, s);
+      case EPI_BIAS_SILU: return launch<EPI_BIAS_SILU, true>(a, p, ws, s);
+      default: return KGS_ERR_ARG;
+    }
+  }
+  switch (epi) {
+    case EPI_NONE: return launch<EPI_NONE, false>(a, p, ws, s);
+    case EPI_BIAS: return launch<EPI_BIAS, false>(a, p, ws, s);
+    case EPI_BIAS_GELU: return launch<EPI_BIAS_GELU, false>(a, p, ws, s);
+    case EPI_BIAS_RELU: return launch<EPI_BIAS_RELU, false>(a, p, ws, s);
+    case EPI_BIAS_SILU: return launch<EPI_BIAS_SILU, false>(a, p, ws, s);
+    case EPI_ADDC: return launch<EPI_ADDC, false>(a, p, ws, s);
+    default: return KGS_ERR_ARG;
+  }
+}
+
+// fp32 values of scratch that a product's slices need (0: it has none)
+long gemm_any_ws(int M, int N, int K) {
+  const any::Plan p = any::plan(M, N, K, true, cu_count());
+  return p.ns > 1 ? (long)p.ns * M * ((N + 7) / 8 * 8) : 0;
+}
+
+}  // namespace kgs
+
+// A product with K-major operands (ta, tb: stored [K][rows]) read in place on 128 x 128 tiles over
+// ns K slices (ws: ns M (N rounded up to 8) fp32 values when ns > 1).
+KGS_EXPORT int kgs_gemm_bf16_tr(const void* A, const void* B, void* C, int M, int N, int K, int lda, int ldb, int ldc,
+                                int ta, int tb, int ns, float* ws, hipStream_t s) {
+  if (M <= 0 || N <= 0 || K <= 0 || ldc < N || ns < 1 || ns > 64) return KGS_ERR_SHAPE;
+  if (!kgs::gemm_tr_ok(A, B, M, N, K, lda, ldb, ta, tb) || (uintptr_t)ws % 16) return KGS_ERR_ALIGN;
+  return kgs::gemm_tr(A, B, C, M, N, K, lda, ldb, ldc, ta, tb, ns, ws, s);
+}
+
+// Slices for kgs_gemm_bf16_tr, 0 where another route is faster (layout_plan).
+KGS_EXPORT int kgs_gemm_bf16_tr_slices(int M, int N, int K, int ta, int tb) {
+  return M > 0 && N > 0 && K > 0 ? kgs::any::layout_plan(M, N, K, ta, tb, kgs::cu_count()) : 0;
+}
+
+// Z = bf16(A . B^T + bias) and Y = act(Z) from one launch (epi: the activations' epilogues; bias
+// may be null), both [M, N] with rows ldc apart. ws: kgs_gemm_bf16_nt_scratch values, or null.
+KGS_EXPORT int kgs_gemm_bf16_nt_act(const void* A, const void* B, void* Z, void* Y, const void* bias, int M, int N, int K,
+                                    int lda, int ldb, int ldc, int epi, float* ws, hipStream_t s) {
+  if (M <= 0 || N <= 0 || K <= 0 || lda < K || ldb < K || ldc < N) return KGS_ERR_SHAPE;
+  if (!Y || epi < kgs::EPI_BIAS_GELU || epi > kgs::EPI_BIAS_SILU) return KGS_ERR_ARG;
+  if (!kgs::gemm_any_ok(A, B, M, N, K, lda, ldb) || (uintptr_t)ws % 16) return KGS_ERR_ALIGN;
+  return kgs::gemm_any(A, B, Z, Y, bias, M, N, K, lda, ldb, ldc, epi, 0, 0, 0, ws, s);
+}

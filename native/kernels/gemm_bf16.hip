@@ -154,7 +154,7 @@ __global__ __launch_bounds__(256) void gemm_nt_generic(const unsigned short* __r
 }  // namespace gen
 
 // Compute units of the current device (the persistent grid size), cached per device.
-static int cu_count() {
+int cu_count() {
   static int n[64] = {};
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = 0;
@@ -164,6 +164,12 @@ static int cu_count() {
   }
   return n[dev];
 }
+
+// gemm_any.hip
+int gemm_any_ok(const void* A, const void* B, int M, int N, int K, int lda, int ldb);
+int gemm_any(const void* A, const void* B, void* C, void* C2, const void* bias, int M, int N, int K, int lda, int ldb,
+             int ldc, int epi, int bm, int bn, int ns, float* ws, hipStream_t s);
+long gemm_any_ws(int M, int N, int K);
 
 // gemm_persistent.hip
 hipError_t launch_w4p_swiglu(const unsigned short* A, const unsigned short* B, unsigned short* C, int M, int N,
@@ -292,10 +298,9 @@ KGS_EXPORT int kgs_gemm_bf16_nt_w4x_ex(const void* A, const void* B, void* C, fl
 //          kernel's one-shot grid (one workgroup
 //          per tile), 16 = force the bounded 256x256 pipeline. Anything else
 //          is rejected.
-// Auto on a grid of at most 128 256x256 tiles (half the CUs or fewer) runs the
-// four-wave kernel on smaller tiles: 256x128 / 128x256 up to 128 tiles, 128x128
-// up to 64 -- 1.13-1.23x hipBLASLt there, where 256x256 tiles leave CUs idle
-// (profiles/r3/gemm_small_grid.json).
+// Auto takes aligned products of more than 128 256x256 tiles (half the CUs) to variant 3, and
+// every other one whose rows are 16-byte aligned to gemm_any.hip, which chooses its tile and, with
+// scratch (kgs_gemm_bf16_nt_auto), its K slices by sizes.
 // C[M, N] = bf16(C + bf16(A . B^T)): a projection with the residual add in its
 // epilogue (EPI_ADDC; the prompt pass's o / down, whose add_rmsnorm becomes a
 // plain rmsnorm -- same roundings, so bitwise the unfused pair). The aligned
@@ -332,8 +337,8 @@ KGS_EXPORT int kgs_gemm_bf16_nt_addc(const void* A, const void* B, void* C, int 
   return (int)hipGetLastError();
 }
 
-KGS_EXPORT int kgs_gemm_bf16_nt(const void* A, const void* B, void* C, const void* bias, int M, int N, int K, int lda,
-                                int ldb, int ldc, int epi, int variant, hipStream_t stream) {
+static int gemm_nt(const void* A, const void* B, void* C, const void* bias, int M, int N, int K, int lda, int ldb,
+                   int ldc, int epi, int variant, float* ws, hipStream_t stream) {
   if (M <= 0 || N <= 0 || K <= 0) return KGS_ERR_SHAPE;
   if (lda < K || ldb < K || ldc < N) return KGS_ERR_SHAPE;
   if (epi != kgs::EPI_NONE && bias == nullptr) return KGS_ERR_ARG;
@@ -343,21 +348,16 @@ KGS_EXPORT int kgs_gemm_bf16_nt(const void* A, const void* B, void* C, const voi
   const int w4 = kgs_gemm_bf16_nt_w4_ok(A, B, C, M, N, K, lda, ldb, ldc) && bias_ok;
   const int bounded = kgs_gemm_bf16_nt_bounded_ok(A, B, C, M, N, K, lda, ldb, ldc) && bias_ok;
   int v;
-  if (variant == 0) v = w4 ? 3 : fast ? 1 : bounded ? 16 : 2;
-  else if (variant == 3 || variant == 4) { if (!w4) return KGS_ERR_ALIGN; v = variant; }
+  if (variant == 0) {
+    const bool large = w4 && (long)(M / 256) * (N / 256) > 128;
+    if (!large && kgs::gemm_any_ok(A, B, M, N, K, lda, ldb))
+      return kgs::gemm_any(A, B, C, nullptr, bias, M, N, K, lda, ldb, ldc, epi, 0, 0, 0, ws, stream);
+    v = large ? 3 : 2;
+  } else if (variant == 3 || variant == 4) { if (!w4) return KGS_ERR_ALIGN; v = variant; }
   else if (variant == 16) { if (!bounded) return KGS_ERR_ALIGN; v = 16; }
   else if (variant == 1) { if (!fast) return KGS_ERR_ALIGN; v = 1; }
   else if (variant == 2) v = 2;
   else return KGS_ERR_ARG;
-  if (variant == 0 && v == 3 && epi == kgs::EPI_NONE) {
-    const long tiles = (long)(M / 256) * (N / 256);
-    if (tiles <= 64) return kgs_gemm_bf16_nt_w4x_ex(A, B, C, nullptr, M, N, K, lda, ldb, ldc, 128, 1, 128, 0, stream);
-    if (tiles <= 128) {
-      const bool wide = M < N;
-      return kgs_gemm_bf16_nt_w4x_ex(A, B, C, nullptr, M, N, K, lda, ldb, ldc, wide ? 256 : 128, 1, wide ? 128 : 256,
-                                     0, stream);
-    }
-  }
   auto a = (const unsigned short*)A;
   auto b = (const unsigned short*)B;
   auto c = (unsigned short*)C;
@@ -372,6 +372,35 @@ KGS_EXPORT int kgs_gemm_bf16_nt(const void* A, const void* B, void* C, const voi
     default: return KGS_ERR_ARG;
   }
   return (int)e;
+}
+
+KGS_EXPORT int kgs_gemm_bf16_nt(const void* A, const void* B, void* C, const void* bias, int M, int N, int K, int lda,
+                                int ldb, int ldc, int epi, int variant, hipStream_t stream) {
+  return gemm_nt(A, B, C, bias, M, N, K, lda, ldb, ldc, epi, variant, nullptr, stream);
+}
+
+// fp32 values of scratch with which kgs_gemm_bf16_nt_auto can slice this product's K (0: no slices).
+KGS_EXPORT long kgs_gemm_bf16_nt_scratch(int M, int N, int K) {
+  return M > 0 && N > 0 && K > 0 ? kgs::gemm_any_ws(M, N, K) : 0;
+}
+
+// Variant 0 with scratch (kgs_gemm_bf16_nt_scratch values, or null).
+KGS_EXPORT int kgs_gemm_bf16_nt_auto(const void* A, const void* B, void* C, const void* bias, int M, int N, int K,
+                                     int lda, int ldb, int ldc, int epi, float* ws, hipStream_t stream) {
+  if ((uintptr_t)ws % 16) return KGS_ERR_ALIGN;
+  return gemm_nt(A, B, C, bias, M, N, K, lda, ldb, ldc, epi, 0, ws, stream);
+}
+
+// gemm_any.hip's kernel on tiles bm x bn (256 x 256, 256 x 128 or 128 x 128) over ns K slices (ws:
+// ns M (N rounded up to 8) values when ns > 1), for tests and measurements.
+KGS_EXPORT int kgs_gemm_bf16_nt_any(const void* A, const void* B, void* C, const void* bias, int M, int N, int K,
+                                    int lda, int ldb, int ldc, int epi, int bm, int bn, int ns, float* ws,
+                                    hipStream_t stream) {
+  if (M <= 0 || N <= 0 || K <= 0 || lda < K || ldb < K || ldc < N) return KGS_ERR_SHAPE;
+  if (epi < 0 || epi > kgs::EPI_BIAS_SILU || (epi != kgs::EPI_NONE && !bias)) return KGS_ERR_ARG;
+  if (!((bm == 256 && (bn == 256 || bn == 128)) || (bm == 128 && bn == 128)) || ns < 1 || ns > 64) return KGS_ERR_ARG;
+  if (!kgs::gemm_any_ok(A, B, M, N, K, lda, ldb) || (uintptr_t)ws % 16) return KGS_ERR_ALIGN;
+  return kgs::gemm_any(A, B, C, nullptr, bias, M, N, K, lda, ldb, ldc, epi, bm, bn, ns, ws, stream);
 }
 
 // ---------------------------------------------------------------------------

@@ -102,6 +102,7 @@ def main() -> None:
         ]
     clob = ", ".join(f'"a{r}"' for r in range(4 * NQ))
     half = ", ".join(f'"a{r}"' for r in range(2 * NQ))
+    quarter = ", ".join(f'"a{r}"' for r in range(NQ))
     lines += [
         "",
         "}  // namespace accr",
@@ -111,6 +112,8 @@ def main() -> None:
         f'#define KGS_ACC_RESERVE() asm volatile("s_nop 0" ::: {clob})',
         "// ... or only a0..a127 (accumulators 0..31)",
         f'#define KGS_ACC_RESERVE_HALF() asm volatile("s_nop 0" ::: {half})',
+        "// ... or only a0..a63 (accumulators 0..15)",
+        f'#define KGS_ACC_RESERVE_QUARTER() asm volatile("s_nop 0" ::: {quarter})',
         "",
     ]
     with open(os.path.join(HERE, "acc_regs.h"), "w") as f:

@@ -1,0 +1,104 @@
+"""The GEMM for any size (native/kernels/gemm_any.hip) and its K-major form at the edges of tiles,
+slices and vectors, against float64 products of the same bf16 operands."""
+import pytest
+
+torch = pytest.importorskip("torch")
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+# bf16 has 8 significant bits: rounding moves a value by up to 2^-8 of its size, so a result by no
+# more in the 2-norm (2^-8 / 2.3 on average); fp32 sums of K products add K 2^-24 at most
+REL = 2.0 ** -8
+
+
+def rnd(*shape):
+    return (torch.rand(*shape, device=DEV) * 2 - 1).bfloat16()
+
+
+def rel(got, want):
+    return float((got.double() - want).norm() / want.norm())
+
+
+def run_any(a, b, c, bm, bn, ns, bias=None, epi=0):
+    from kgs.ops import _lib
+
+    (M, K), N = a.shape, b.shape[0]
+    ws = torch.empty(ns * M * ((N + 7) // 8 * 8), device=DEV)
+    rc = _lib.lib().kgs_gemm_bf16_nt_any(a.data_ptr(), b.data_ptr(), c.data_ptr(), None if bias is None else bias.data_ptr(), M, N, K,
+                                         a.stride(0), b.stride(0), c.stride(0), epi, bm, bn, ns, ws.data_ptr(), _lib.stream_handle(a.device))
+    assert rc == 0, rc
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 8, 8), (5, 16, 64), (127, 129, 72), (129, 251, 1096), (256, 256, 128), (257, 264, 136), (40, 520, 2056)])
+@pytest.mark.parametrize("bm,bn", [(256, 256), (256, 128), (128, 128)])
+@pytest.mark.parametrize("ns", [1, 2, 3])
+def test_any_tile_and_slices(M, N, K, bm, bn, ns):
+    a, b, bias = rnd(M, K), rnd(N, K), torch.randn(N, device=DEV).bfloat16()
+    want = a.double() @ b.double().T
+    big = torch.full((M + 1, N + 3), 7.0, device=DEV, dtype=torch.bfloat16)  # rows that are not 16-byte aligned
+    run_any(a, b, big[:M, :N], bm, bn, ns)
+    assert rel(big[:M, :N], want) < REL
+    assert bool((big[M] == 7).all()) and bool((big[:, N:] == 7).all())  # nothing written outside
+    c = torch.empty(M, N, device=DEV, dtype=torch.bfloat16)
+    run_any(a, b, c, bm, bn, ns, bias, 2)
+    assert rel(c, torch.nn.functional.gelu(want + bias.double(), approximate="tanh")) < 2 * REL
+
+
+def test_any_reads_nothing_past_its_operands():
+    """Views inside larger buffers whose surroundings are NaN: the K tail and the rows past the
+    end have to arrive as zeros."""
+    from kgs.ops import gemm_nt
+
+    M, N, K = 130, 136, 200
+    A, B = (torch.full((r + 2, K + 8), float("nan"), device=DEV, dtype=torch.bfloat16) for r in (M, N))
+    a, b = A[1:M + 1, :K], B[1:N + 1, :K]
+    a.copy_(rnd(M, K))
+    b.copy_(rnd(N, K))
+    assert rel(gemm_nt(a, b), a.double() @ b.double().T) < REL
+
+
+@pytest.mark.parametrize("M,N,K", [(64, 512, 2048), (300, 304, 2400), (128, 640, 4096)])
+def test_sliced_products_on_two_streams_and_in_a_graph(M, N, K):
+    """Every call has scratch of its own: interleaved products keep their results, and a captured
+    one replays to the eager result."""
+    from kgs.ops import gemm_nt
+    from kgs.ops.gemm import _scratch_floats
+
+    assert _scratch_floats(M, N, K) > 0
+    ops = [(rnd(M, K), rnd(N, K)) for _ in range(4)]
+    want = [gemm_nt(a, b) for a, b in ops]
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    torch.cuda.synchronize()
+    got = []
+    for i, (a, b) in enumerate(ops):
+        with torch.cuda.stream(streams[i % 2]):
+            got.append(gemm_nt(a, b))
+    torch.cuda.synchronize()
+    assert all(torch.equal(g, w) for g, w in zip(got, want))
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = gemm_nt(*ops[0])
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        gemm_nt(*ops[1])  # eager work between the replays
+        torch.cuda.synchronize()
+        assert torch.equal(out, want[0])
+
+
+@pytest.mark.parametrize("M,N,K", [(8, 8, 1), (16, 24, 63), (136, 72, 200), (128, 256, 65), (264, 136, 1096), (64, 512, 2056)])
+@pytest.mark.parametrize("ta,tb", [(1, 1), (1, 0), (0, 1)])
+@pytest.mark.parametrize("ns", [1, 3])
+def test_tr_layouts(M, N, K, ta, tb, ns):
+    from kgs.ops import _lib
+
+    if not (ta and tb):
+        K = (K + 7) // 8 * 8  # the K-contiguous operand's chunks
+    a, b = rnd(K, M) if ta else rnd(M, K), rnd(K, N) if tb else rnd(N, K)
+    want = (a.T if ta else a).double() @ (b if tb else b.T).double()
+    ws = torch.empty(ns * M * N, device=DEV)
+    c = torch.full((M + 1, N), 7.0, device=DEV, dtype=torch.bfloat16)
+    rc = _lib.lib().kgs_gemm_bf16_tr(a.data_ptr(), b.data_ptr(), c.data_ptr(), M, N, K, a.stride(0), b.stride(0), N, ta, tb, ns,
+                                     ws.data_ptr(), _lib.stream_handle(a.device))
+    assert rc == 0
+    assert rel(c[:M], want) < REL and bool((c[M] == 7).all())

@@ -611,6 +611,57 @@ def matmul(a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
     return gemm_bf16(a, b)
 
 
+GRADS = ("gelu", "relu", "silu")  # activations whose training passes run on the kernels
+
+
+def gemm_nt_act(a: torch.Tensor, b: torch.Tensor, bias: torch.Tensor | None, act: str
+                ) -> tuple[torch.Tensor, torch.Tensor]:
+    """``z = a @ b.T + bias`` and ``act(z)`` (of the rounded ``z``; ``act``: gelu, relu or silu),
+    both from one GEMM's epilogue."""
+    _check_operand(a, "a")
+    _check_operand(b, "b")
+    M, K = a.shape
+    N = b.shape[0]
+    if K != b.shape[1]:
+        raise ValueError(f"inner dims differ: a {tuple(a.shape)} b {tuple(b.shape)}")
+    if a.device != b.device:
+        raise ValueError("a and b on different devices")
+    if not _rows16(a) or not _rows16(b) or K % 8 or M == 0 or max(a.stride(0), b.stride(0)) >= 1 << 22:
+        z = gemm_nt(a, b, bias=bias)
+        return z, _act(z, act)
+    if bias is not None and (bias.dtype != torch.bfloat16 or bias.numel() != N or not bias.is_contiguous()):
+        raise ValueError("bias must be a contiguous bf16 vector of length N")
+    z, y = (torch.empty((M, N), dtype=torch.bfloat16, device=a.device) for _ in range(2))
+    ws = _scratch(M, N, K, a.device)
+    rc = _lib.lib().kgs_gemm_bf16_nt_act(a.data_ptr(), b.data_ptr(), z.data_ptr(), y.data_ptr(),
+                                         None if bias is None else bias.data_ptr(), M, N, K, a.stride(0), b.stride(0), N,
+                                         EPI[act], None if ws is None else ws.data_ptr(), _lib.stream_handle(a.device))
+    _lib.check(rc, f"gemm_nt_act[{M}x{N}x{K}]")
+    return z, y
+
+
+def act_grad(gy: torch.Tensor, z: torch.Tensor | None, act: str | None, bias: bool, turned: bool
+             ) -> tuple[torch.Tensor, torch.Tensor | None, torch.Tensor | None]:
+    """``gz = gy * act'(z)`` for contiguous bf16 ``gy`` (``act`` None: ``gy`` itself), its transpose
+    if ``turned`` and its column sums if ``bias``, from one pass over memory."""
+    M, N = gy.shape
+    act = act if act in GRADS else None
+    empty = torch.empty
+    gz = gy if act is None else empty((M, N), dtype=torch.bfloat16, device=gy.device)
+    gzt = empty((N, M), dtype=torch.bfloat16, device=gy.device) if turned else None
+    gb = empty(N, dtype=torch.bfloat16, device=gy.device) if bias else None
+    if act is None and gzt is None and gb is None:
+        return gz, None, None
+    if M == 0 or N == 0:
+        return gz, gzt, gb.zero_() if bias else None
+    lib = _lib.lib()
+    parts = lib.kgs_act_grad_parts(M) if bias else 1
+    part = empty((parts, N), dtype=torch.float32, device=gy.device) if parts > 1 else None
+    ptr = [None if t is None else t.data_ptr() for t in (gy, z if act else None, gz if act else None, gzt, part, gb)]
+    _lib.check(lib.kgs_act_grad(*ptr, M, N, EPI[act], _lib.stream_handle(gy.device)), f"act_grad[{M}x{N}]")
+    return gz, gzt, gb
+
+
 class _LinearFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, w, bias, act):
@@ -620,27 +671,28 @@ class _LinearFn(torch.autograd.Function):
             return gemm_nt(x, w, bias=bias)
         if not any(ctx.needs_input_grad[:3]):
             return gemm_nt(x, w, bias=bias, act=act)  # inference: activation fused in the epilogue
-        # training keeps the pre-activation for the backward pass: GEMM with the
-        # bias epilogue, then the activation in torch (cheap, memory-bound)
-        z = gemm_nt(x, w, bias=bias)
-        ctx.z = z
-        return _act(z, act)
+        # training keeps the pre-activation for the backward pass
+        if act in GRADS:
+            ctx.z, y = gemm_nt_act(x, w, bias, act)
+            return y
+        return _act(gemm_nt(x, w, bias=bias), act)
 
     @staticmethod
     def backward(ctx, gy):
         x, w, bias = ctx.saved_tensors
+        need_x, need_w, need_b = ctx.needs_input_grad[:3]
         gy = gy.contiguous()
-        if ctx.act not in (None, "none"):
-            z = ctx.z.float().requires_grad_(True)
-            with torch.enable_grad():
-                y = _act(z, ctx.act)
-            (gz,) = torch.autograd.grad(y, z, gy.float())
-            gy = gz.to(torch.bfloat16).contiguous()
-        # dX[M,K] = dY[M,N] . W[N,K]      (W read K-major: transposed-read path)
-        gx = gemm_bf16(gy, w)
-        # dW[N,K] = dY^T[N,M] . X[M,K]    (both operands M-major)
-        gw = gemm_bf16(gy, x, trans_a=True)
-        gb = gy.float().sum(0).to(torch.bfloat16) if bias is not None else None
+        M, N = gy.shape
+        K = x.shape[1]
+        # dW[N,K] = dY^T[N,M] . X[M,K] (both operands M-major): where it takes dY turned, that is
+        # written by the pass that makes dY
+        turned = need_w and M > 0 and M % 8 == 0 and not _tr_slices(N, K, M, True, True)
+        gz, gzt, gb = act_grad(gy, getattr(ctx, "z", None), ctx.act, need_b and bias is not None, turned)
+        # dX[M,K] = dY[M,N] . W[N,K]      (W read K-major)
+        gx = gemm_bf16(gz, w) if need_x else None
+        gw = None
+        if need_w:
+            gw = gemm_bf16(gzt, x) if turned else gemm_bf16(gz, x, trans_a=True)
         return gx, gw, gb, None
 
 

@@ -1,5 +1,6 @@
-"""The GEMM for any size (native/kernels/gemm_any.hip) and its K-major form at the edges of tiles,
-slices and vectors, against float64 products of the same bf16 operands."""
+"""The GEMM for any size (native/kernels/gemm_any.hip), its K-major form and the linear layer's
+backward pass (native/kernels/linear_grad.hip) at the edges of tiles, slices and vectors, against
+float64 products of the same bf16 operands."""
 import pytest
 
 torch = pytest.importorskip("torch")
@@ -102,3 +103,61 @@ def test_tr_layouts(M, N, K, ta, tb, ns):
                                      ws.data_ptr(), _lib.stream_handle(a.device))
     assert rc == 0
     assert rel(c[:M], want) < REL and bool((c[M] == 7).all())
+
+
+@pytest.mark.parametrize("act", [None, "gelu", "relu", "silu"])
+@pytest.mark.parametrize("M,N", [(1, 8), (7, 3), (64, 64), (65, 136), (513, 72), (1025, 200), (520, 67)])
+def test_act_grad(act, M, N):
+    """The gradient through an activation, its transpose and its column sums."""
+    from kgs.ops.gemm import act_grad
+
+    gy, z = rnd(M, N), 3 * rnd(M, N)
+    z[0, 0] = 0.0
+    want = gy.double()
+    if act:
+        x = z.double().requires_grad_(True)
+        f = {"gelu": lambda v: torch.nn.functional.gelu(v, approximate="tanh"), "relu": torch.relu, "silu": torch.nn.functional.silu}[act]
+        (want,) = torch.autograd.grad(f(x), x, gy.double())
+    gz, gzt, gb = act_grad(gy, z, act, True, True)
+    assert float((gz.double() - want).abs().max()) < 2 * REL * float(want.abs().max())
+    assert torch.equal(gzt, gz.T.contiguous())
+    sums = gz.double().sum(0)
+    assert float((gb.double() - sums).abs().max()) <= REL * float(sums.abs().max()) + M * 2.0 ** -24 * float(gz.double().abs().sum(0).max())
+
+
+@pytest.mark.parametrize("act", [None, "gelu", "relu", "silu"])
+@pytest.mark.parametrize("rows,din,dout,bias", [(64, 512, 2048, True), (1, 64, 72, True), (100, 136, 200, False), (1001, 264, 128, True),
+                                                (33, 7, 10, True), (2048, 256, 512, True)])
+def test_linear_training_step(act, rows, din, dout, bias):
+    """Output, and the gradients of input, weight and bias, against float64."""
+    from kgs.ops import Linear
+
+    lin = Linear(din, dout, bias=bias, act=act, device=DEV)
+    if bias:
+        with torch.no_grad():
+            lin.bias.copy_(torch.randn(dout, device=DEV))
+    x, gy = rnd(rows, din).requires_grad_(True), rnd(rows, dout)
+    y = lin(x)
+    y.backward(gy)
+    p = [t.detach().double().requires_grad_(True) for t in [x, lin.weight] + ([lin.bias] if bias else [])]
+    z = p[0] @ p[1].T + (p[2] if bias else 0.0)
+    f = {None: lambda v: v, "gelu": lambda v: torch.nn.functional.gelu(v, approximate="tanh"), "relu": torch.relu,
+         "silu": torch.nn.functional.silu}[act]
+    # the kernels' activation and its gradient see z rounded to bf16: up to 2^-8 of z on either side
+    want = torch.autograd.grad(f(z), p, gy.double())
+    assert rel(y.detach(), f(z).detach()) < 3 * REL
+    for got, w in zip([x.grad, lin.weight.grad] + ([lin.bias.grad] if bias else []), want):
+        assert rel(got, w) < 8 * REL
+    assert y.dtype == torch.bfloat16
+
+
+def test_linear_keeps_nan_and_skips_what_needs_no_gradient():
+    from kgs.ops import Linear
+
+    lin = Linear(64, 64, act="relu", device=DEV)
+    x = rnd(8, 64)
+    x[3, 5] = float("nan")
+    y = lin(x)  # no gradient for x
+    assert bool(y[3].isnan().all()) and not bool(y[:3].isnan().any())
+    y.backward(torch.ones_like(y))
+    assert x.grad is None and lin.weight.grad is not None

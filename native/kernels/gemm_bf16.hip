@@ -471,7 +471,9 @@ KGS_EXPORT int kgs_gemm_fp8_nt_dev(const void* A, const void* B, void* C, const 
   // over a 256-row panel, more tiles than CUs (round 3, gemm_w4f8.h)
   const int w4p = fast && K >= 768 && (long)(lda / 2) * 512 < (1L << 31) && (long)(ldb / 2) * 512 < (1L << 31);
   int v;
-  if (variant == 0) v = w4p && (M / 256) * (N / 256) > kgs::cu_count() ? 3 : fast ? 1 : 16;
+  // the four-wave kernel wherever it can run: 4096 x 4096 x 14336 (a tile per CU) 145 us, the
+  // eight-wave one 218; 1024 x 4096 x 4096 (a quarter of the CUs) 37 and 65
+  if (variant == 0) v = w4p ? 3 : fast ? 1 : 16;
   else if (variant == 1 || variant == 16) v = variant;
   else if (variant == 3) { if (!w4p) return KGS_ERR_ALIGN; v = 3; }
   else return KGS_ERR_ARG;

@@ -161,3 +161,11 @@ def test_linear_keeps_nan_and_skips_what_needs_no_gradient():
     assert bool(y[3].isnan().all()) and not bool(y[:3].isnan().any())
     y.backward(torch.ones_like(y))
     assert x.grad is None and lin.weight.grad is not None
+
+
+@pytest.mark.parametrize("M,N,K", [(256, 256, 768), (256, 768, 1024), (1024, 1024, 4096)])
+def test_fp8_small_grids_equal_the_eight_wave_kernel(M, N, K):
+    from kgs.ops import gemm_fp8_nt, quantize_fp8
+
+    (a, sa), (b, sb) = quantize_fp8(rnd(M, K)), quantize_fp8(rnd(N, K))
+    assert torch.equal(gemm_fp8_nt(a, b, sa, sb), gemm_fp8_nt(a, b, sa, sb, variant="fast"))

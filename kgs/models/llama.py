@@ -150,13 +150,12 @@ class LlamaModel:
         return self.lm_head(y).reshape(b, s, cfg.vocab)
 
     def _add_norm(self, x, a, proj, w):
-        """x += proj(a) and return rmsnorm(x) * w; on aligned operands the add
-        runs in the GEMM's store (kgs.ops.gemm.gemm_nt_add_, bitwise the same)."""
-        from kgs.ops.gemm import addc_ok, gemm_nt_add_
+        """x += proj(a) and return rmsnorm(x) * w; the add runs in the GEMM's store
+        (kgs.ops.gemm.add_product_, rounded as the two steps round it)."""
+        from kgs.ops.gemm import add_product_
         from kgs.ops.transformer import add_rmsnorm
 
-        if addc_ok(a, proj.w, x):
-            gemm_nt_add_(a, proj.w, x)
+        if add_product_(a, proj.w, x):
             return add_rmsnorm(x, None, w, self.cfg.eps)
         return add_rmsnorm(x, proj(a), w, self.cfg.eps)
 

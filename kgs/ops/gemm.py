@@ -183,6 +183,7 @@ def pack_w4x_weight(w: torch.Tensor, bn: int, swiglu: bool = False) -> PanelWeig
 
 
 GATE_FLAGS = {"silu": 0, "gelu_tanh": 0x40, "clamped": 0x80}
+GATE_ACTS = {"silu": 1, "gelu_tanh": 2, "clamped": 4}  # kgs_common.h GateAct
 
 
 def _w4x_flags(packed: int, stages: int, nt_weights: bool = False) -> int:
@@ -271,6 +272,26 @@ def gemm_nt_add_(a: torch.Tensor, b: torch.Tensor, c: torch.Tensor) -> torch.Ten
                                           c.stride(0), _lib.stream_handle(a.device))
     _lib.check(rc, f"gemm_nt_add_[{M}x{N}x{K}]")
     return c
+
+
+def add_product_(a: torch.Tensor, b: torch.Tensor, c: torch.Tensor) -> bool:
+    """:func:`gemm_nt_add_` on any rows (``N`` and ``K`` multiples of 8, 16-B rows). Returns whether it
+    took the operands; where not, nothing was written."""
+    if addc_ok(a, b, c):
+        gemm_nt_add_(a, b, c)
+        return True
+    if os.environ.get("KGS_PREFILL_ADDC", "1") != "1" or any(
+            not t.is_cuda or t.dtype != torch.bfloat16 or t.dim() != 2 or t.stride(1) != 1 or not _rows16(t) for t in (a, b, c)):
+        return False
+    M, K = a.shape
+    N = b.shape[0]
+    if b.shape[1] != K or tuple(c.shape) != (M, N) or M == 0 or N % 8 or K % 8 or max(a.stride(0), b.stride(0)) >= 1 << 22:
+        return False
+    ws = _scratch(M, N, K, a.device)
+    rc = _lib.lib().kgs_gemm_bf16_nt_add(a.data_ptr(), b.data_ptr(), c.data_ptr(), M, N, K, a.stride(0), b.stride(0),
+                                         c.stride(0), None if ws is None else ws.data_ptr(), _lib.stream_handle(a.device))
+    _lib.check(rc, f"add_product_[{M}x{N}x{K}]")
+    return True
 
 
 def gemm_nt_w4x_partials(a: torch.Tensor, b, bn: int, nslice: int, bm: int = 256, stages: int = 2,
@@ -364,11 +385,18 @@ def swiglu_fused_ok(a: torch.Tensor, w: torch.Tensor) -> bool:
 
 def gemm_swiglu(a: torch.Tensor, w_gate_up: torch.Tensor, act="silu") -> torch.Tensor:
     """Gated MLP input projection ``act(a @ gate.T) * (a @ up.T)`` -> ``[M, I]``:
-    fused into the four-wave GEMM's epilogue (256x256 tiles; 256x128 when
-    ``2I % 256 != 0``) when the shape allows, else GEMM + the elementwise product.
+    fused into the GEMM's epilogue when the shape allows, else GEMM + the elementwise product.
     Same bits either way (silu)."""
     if swiglu_fused_ok(a, w_gate_up):
-        return gemm_nt_w4x_swiglu(a, w_gate_up, bn=256 if w_gate_up.shape[0] % 256 == 0 else 128, act=act)
+        from .activation import Gate
+
+        M, (N, K), gate = a.shape[0], w_gate_up.shape, Gate.of(act)
+        out = torch.empty((M, N // 2), dtype=torch.bfloat16, device=a.device)
+        rc = _lib.lib().kgs_gemm_bf16_nt_swiglu(a.data_ptr(), w_gate_up.data_ptr(), out.data_ptr(), M, N, K, a.stride(0),
+                                                w_gate_up.stride(0), N // 2, GATE_ACTS[gate.act], gate.limit_ptr(a.device),
+                                                _lib.stream_handle(a.device))
+        _lib.check(rc, f"gemm_swiglu[{M}x{N}x{K}]")
+        return out
     from .activation import Gate, act_mul
 
     if Gate.of(act).act != "silu":

@@ -252,16 +252,14 @@ class ServingModel:
         return add_rmsnorm(x, d, w, self.cfg.eps)
 
     def _proj_add_norm(self, a, layer: int, name: str, x, w):
-        """Prompt pass: x += a @ W.T, return rmsnorm(x) * w. On kgs with aligned
-        operands the residual add runs in the GEMM's store (EPI_ADDC) and the
+        """Prompt pass: x += a @ W.T, return rmsnorm(x) * w. On kgs
+        the residual add runs in the GEMM's store (EPI_ADDC) and the
         norm reads x once: bitwise the GEMM + add_rmsnorm pair, with one
         [rows, hidden] tensor fewer through HBM (profiles/r5/prefill_swiglu)."""
         if self.backend == "kgs":
-            from kgs.ops.gemm import addc_ok, gemm_nt_add_
+            from kgs.ops.gemm import add_product_
 
-            wt = self.w[layer][name]
-            if addc_ok(a, wt, x):
-                gemm_nt_add_(a, wt, x)
+            if add_product_(a, self.w[layer][name], x):
                 return self._norm(x, None, w)
         return self._norm(x, self._proj(a, layer, name, False), w)
 
@@ -443,9 +441,9 @@ class ServingModel:
                 else:
                     y = self._norm(x, d, nxt)
                 continue
-            y = self._norm(x, self._proj(a, i, "o", False), self.ln2[i])
+            y = self._proj_add_norm(a, i, "o", x, self.ln2[i])
             act = self._gate_up_act(y, i)
-            y = self._norm(x, self._proj(act, i, "down", False), nxt)
+            y = self._proj_add_norm(act, i, "down", x, nxt)
         rows = [row0 + n - 1 for row0, n, _, _, _, last in chunks if last] + list(range(n_pf, n_pf + nd))
         if not rows:
             return torch.empty((0, c.vocab), dtype=torch.bfloat16, device=x.device)

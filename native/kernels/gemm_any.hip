@@ -77,20 +77,25 @@ __device__ __forceinline__ void store8(unsigned short* row, int col, int N, int 
     if (col + e < N) row[col + e] = (unsigned short)(u[e >> 1] >> (16 * (e & 1)));
 }
 
-template <int EPI, int BM, int BN, bool SPLIT, bool DUAL>
+// SW (a GateAct): B is a fused gate|up weight of N rows, gate rows first, and C [M, N / 2] holds
+// act(gate) * up; a tile stages both halves' rows in turn (gemm_w4.h). `bias` then points to the
+// clamped gate's limit.
+template <int EPI, int BM, int BN, bool SPLIT, bool DUAL, int SW = 0>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(waves_per_simd<BM, BN>(), waves_per_simd<BM, BN>())))
 void gemm_nt_any(Args a) {
+  constexpr int X = SW * 1000000, TN = SW ? BN / 2 : BN;  // TN: output columns of a tile
+  const int cols = SW ? a.N / 2 : a.N;
   using S = w4::Shape<BM, BN>;
   using Kn = w4::Knobs<BM, BN>;
   constexpr int MA = S::MA, NB = S::NB, ND = w4::dma_per_stage<BM, BN>();
   __shared__ __attribute__((aligned(1024))) char smem[2 * S::STAGE];
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int ntm = (a.M + BM - 1) / BM, ntn = (a.N + BN - 1) / BN;
+  const int ntm = (a.M + BM - 1) / BM, ntn = (cols + TN - 1) / TN;
   int slice, tm, tn;
   if (a.tall) w4::tile_of<40000000, SPLIT>((int)blockIdx.x, (int)gridDim.x, ntm, ntn, slice, tm, tn);
   else w4::tile_of<0, SPLIT>((int)blockIdx.x, (int)gridDim.x, ntm, ntn, slice, tm, tn);
-  const int m0 = tm * BM, n0 = tn * BN;
+  const int m0 = tm * BM, n0 = tn * TN;
   const int k0 = SPLIT ? slice * a.ks : 0;
   const int kn = SPLIT ? min(a.K - k0, a.ks) : a.K;  // this slice's valid K
 
@@ -101,9 +106,11 @@ void gemm_nt_any(Args a) {
   c.wc = w & 1;
   c.nt = (kn + 2 * BK - 1) / (2 * BK) * 2;
   // resources end with the last valid element: nothing outside the operands is ever read
-  const int ra = min(a.M - m0, BM), rb = min(a.N - n0, BN);
+  const int ra = min(a.M - m0, BM), rb = min(cols - n0, TN);
   c.ra = __builtin_amdgcn_make_buffer_rsrc((void*)(a.A + (long)m0 * a.lda + k0), 0, ((ra - 1) * a.lda + kn) * 2, 0x00020000);
   c.rb = __builtin_amdgcn_make_buffer_rsrc((void*)(a.B + (long)n0 * a.ldb + k0), 0, ((rb - 1) * a.ldb + kn) * 2, 0x00020000);
+  if constexpr (SW != 0)
+    c.rb2 = __builtin_amdgcn_make_buffer_rsrc((void*)(a.B + ((long)cols + n0) * a.ldb + k0), 0, ((rb - 1) * a.ldb + kn) * 2, 0x00020000);
   c.sa32 = 32 * a.lda * 2;
   c.sb32 = 32 * a.ldb * 2;
   const int row = w * 8 + (lane >> 3);
@@ -127,7 +134,7 @@ void gemm_nt_any(Args a) {
   for (int st = 0; st < 2; ++st) {
     aim(st);
 #pragma unroll
-    for (int j = 0; j < ND; ++j) w4::dma_any<BM, BN, 0>(c, st, j, st * BK);
+    for (int j = 0; j < ND; ++j) w4::dma_any<BM, BN, X>(c, st, j, st * BK);
   }
   w4::wait_vm<ND>();
   w4::bar();
@@ -146,14 +153,43 @@ void gemm_nt_any(Args a) {
 
   for (int t = 0; t < c.nt; t += 2) {
     aim(min(t + 2, c.nt - 1));
-    w4::kstep<BM, BN, 0, Kn::B1, Kn::R, Kn::P, Kn::ORD, 0>(c, f0, f1, t);
+    w4::kstep<BM, BN, 0, Kn::B1, Kn::R, Kn::P, Kn::ORD, X>(c, f0, f1, t);
     aim(min(t + 3, c.nt - 1));
-    w4::kstep<BM, BN, 1, Kn::B1, Kn::R, Kn::P, Kn::ORD, 0>(c, f0, f1, t + 1);
+    w4::kstep<BM, BN, 1, Kn::B1, Kn::R, Kn::P, Kn::ORD, X>(c, f0, f1, t + 1);
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // drain the tail re-loads before LDS is released
   asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 3" ::: "memory");  // MFMA -> v_accvgpr_read hazard
 
-  const int mw = m0 + c.wr * (BM / 2) + fr, nw = n0 + c.wc * (BN / 2);
+  const int mw = m0 + c.wr * (BM / 2) + fr, nw = n0 + c.wc * (TN / 2);
+  const int lc = (fq & 1) * 16 + (fq >> 1) * 8;  // this lane's 8 of a fragment pair's 32 columns
+  if constexpr (SW != 0) {
+    // output fragment q: gate fragment ng = 4 (q / 2) + q % 2 and the up fragment two further
+    const float limit = SW == GATE_CLAMPED ? *(const float*)a.bias : 0.f;
+    w4::static_for<0, MA>([&](auto ic) {
+      constexpr int i = decltype(ic)::value;
+      f32x4 v[NB];
+      w4::read_row<NB, i>(v);
+      if (mw + i * 16 >= a.M) return;
+      unsigned short* crow = (unsigned short*)a.C + (long)(mw + i * 16) * a.ldc;
+#pragma unroll
+      for (int q = 0; q < NB / 2; q += 2) {
+        uint2 o[2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const int ng = 4 * ((q + h) / 2) + (q + h) % 2;
+          float r[4];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) r[e] = gated<SW>(v[ng][e], v[ng + 2][e], limit);
+          o[h] = make_uint2(pack_bf16x2(r[0], r[1]), pack_bf16x2(r[2], r[3]));
+        }
+        auto sx = __builtin_amdgcn_permlane16_swap(o[0].x, o[1].x, false, false);
+        auto sy = __builtin_amdgcn_permlane16_swap(o[0].y, o[1].y, false, false);
+        const int col = nw + q * 16 + lc;
+        if (col < cols) store8(crow, col, cols, a.vec, make_uint4(sx[0], sy[0], sx[1], sy[1]));
+      }
+    });
+    return;
+  }
   if constexpr (SPLIT) {
     // ldc is a multiple of 8: a fragment's four columns are inside the row or all outside
     float* part = (float*)a.C + (long)slice * a.M * a.ldc;
@@ -183,7 +219,6 @@ void gemm_nt_any(Args a) {
         if (a.bias && col + e < a.N) bv[n][e] = bf2f(a.bias[col + e]);
     }
   }
-  const int lc = (fq & 1) * 16 + (fq >> 1) * 8;  // this lane's 8 of a fragment pair's 32 columns
   w4::static_for<0, MA>([&](auto ic) {
     constexpr int i = decltype(ic)::value;
     const int r = mw + i * 16;
@@ -619,6 +654,31 @@ int gemm_any(const void* A, const void* B, void* C, void* C2, const void* bias, 
     case EPI_ADDC: return launch<EPI_ADDC, false>(a, p, ws, s);
     default: return KGS_ERR_ARG;
   }
+}
+
+// C [M, N / 2] = act(A . gate^T) * (A . up^T), B = [gate; up] of N rows (launch_w4p_swiglu for
+// prompts): the largest tile whose grid fills the chip
+int gemm_any_swiglu(const void* A, const void* B, void* C, int M, int N, int K, int lda, int ldb, int ldc, int act,
+                    const float* limit, hipStream_t s) {
+  using namespace any;
+  const Args a{(const unsigned short*)A, (const unsigned short*)B, C, nullptr, (const unsigned short*)limit,
+               M, N, K, lda, ldb, ldc, 0, M > N, ldc % 8 == 0 && (uintptr_t)C % 16 == 0};
+  const Plan p = plan(M, N, K, false, cu_count());
+  const int bm = p.bm, bn = bm == 256 && p.bn == 256 ? 256 : 128;
+  const dim3 grid((unsigned)(ceil_div(M, bm) * ceil_div(N / 2, bn / 2)));
+#define KGS_SWT(ACT)                                                                                                 \
+  if (bm == 128) hipLaunchKernelGGL((gemm_nt_any<EPI_NONE, 128, 128, false, false, ACT>), grid, dim3(256), 0, s, a); \
+  else if (bn == 128) hipLaunchKernelGGL((gemm_nt_any<EPI_NONE, 256, 128, false, false, ACT>), grid, dim3(256), 0, s, a); \
+  else hipLaunchKernelGGL((gemm_nt_any<EPI_NONE, 256, 256, false, false, ACT>), grid, dim3(256), 0, s, a)
+  if (act == GATE_CLAMPED) {
+    KGS_SWT(GATE_CLAMPED);
+  } else if (act == GATE_GELU) {
+    KGS_SWT(GATE_GELU);
+  } else {
+    KGS_SWT(GATE_SILU);
+  }
+#undef KGS_SWT
+  return (int)hipGetLastError();
 }
 
 // fp32 values of scratch that a product's slices need (0: it has none)

@@ -170,6 +170,8 @@ int gemm_any_ok(const void* A, const void* B, int M, int N, int K, int lda, int 
 int gemm_any(const void* A, const void* B, void* C, void* C2, const void* bias, int M, int N, int K, int lda, int ldb,
              int ldc, int epi, int bm, int bn, int ns, float* ws, hipStream_t s);
 long gemm_any_ws(int M, int N, int K);
+int gemm_any_swiglu(const void* A, const void* B, void* C, int M, int N, int K, int lda, int ldb, int ldc, int act,
+                    const float* limit, hipStream_t s);
 
 // gemm_persistent.hip
 hipError_t launch_w4p_swiglu(const unsigned short* A, const unsigned short* B, unsigned short* C, int M, int N,
@@ -178,6 +180,14 @@ hipError_t launch_w4p_swiglu(const unsigned short* A, const unsigned short* B, u
 template <int EPI>
 hipError_t launch_w4p(const unsigned short* A, const unsigned short* B, unsigned short* C, const unsigned short* bias,
                       int M, int N, int K, int lda, int ldb, int ldc, int cus, int* tq, hipStream_t s);
+
+// Ragged rows on the persistent kernel: the fast path's rules but for M, and more tiles than CUs.
+static bool rows_ok(const void* A, const void* B, const void* C, int M, int N, int K, int lda, int ldb, int ldc) {
+  if (M <= 0 || N % 256 || K % 128 || K < 384 || (lda | ldb | ldc) % 8) return false;
+  if (((uintptr_t)A | (uintptr_t)B | (uintptr_t)C) % 16) return false;
+  if ((long)lda * 512 >= (1L << 31) || (long)ldb * 512 >= (1L << 31)) return false;
+  return ((long)M + 255) / 256 * (N / 256) > cu_count();
+}
 
 template <int EPI>
 static hipError_t launch(int variant, const unsigned short* A, const unsigned short* B, unsigned short* C,
@@ -298,8 +308,8 @@ KGS_EXPORT int kgs_gemm_bf16_nt_w4x_ex(const void* A, const void* B, void* C, fl
 //          kernel's one-shot grid (one workgroup
 //          per tile), 16 = force the bounded 256x256 pipeline. Anything else
 //          is rejected.
-// Auto takes aligned products of more than 128 256x256 tiles (half the CUs) to variant 3, and
-// every other one whose rows are 16-byte aligned to gemm_any.hip, which chooses its tile and, with
+// Auto takes aligned products of more than 128 256x256 tiles (half the CUs) to variant 3, ragged
+// rows with more tiles than CUs to its persistent kernel, and every other product whose rows are 16-byte aligned to gemm_any.hip, which chooses its tile and, with
 // scratch (kgs_gemm_bf16_nt_auto), its K slices by sizes.
 // C[M, N] = bf16(C + bf16(A . B^T)): a projection with the residual add in its
 // epilogue (EPI_ADDC; the prompt pass's o / down, whose add_rmsnorm becomes a
@@ -350,6 +360,11 @@ static int gemm_nt(const void* A, const void* B, void* C, const void* bias, int 
   int v;
   if (variant == 0) {
     const bool large = w4 && (long)(M / 256) * (N / 256) > 128;
+    if (!large && epi == kgs::EPI_NONE && kgs::rows_ok(A, B, C, M, N, K, lda, ldb, ldc)) {
+      if (int* tq = kgs::tile_queue(stream))
+        return (int)kgs::launch_w4p<kgs::EPI_NONE>((const unsigned short*)A, (const unsigned short*)B, (unsigned short*)C,
+                                                   nullptr, M, N, K, lda, ldb, ldc, kgs::cu_count(), tq, stream);
+    }
     if (!large && kgs::gemm_any_ok(A, B, M, N, K, lda, ldb))
       return kgs::gemm_any(A, B, C, nullptr, bias, M, N, K, lda, ldb, ldc, epi, 0, 0, 0, ws, stream);
     v = large ? 3 : 2;
@@ -389,6 +404,39 @@ KGS_EXPORT int kgs_gemm_bf16_nt_auto(const void* A, const void* B, void* C, cons
                                      int lda, int ldb, int ldc, int epi, float* ws, hipStream_t stream) {
   if ((uintptr_t)ws % 16) return KGS_ERR_ALIGN;
   return gemm_nt(A, B, C, bias, M, N, K, lda, ldb, ldc, epi, 0, ws, stream);
+}
+
+// In place C = bf16(C + bf16(A . B^T)) as kgs_gemm_bf16_nt_addc, for any M (N, K % 8): the persistent
+// kernel above one tile per CU (never in a capture, as there), else gemm_any.hip's. ws as in
+// kgs_gemm_bf16_nt_auto.
+KGS_EXPORT int kgs_gemm_bf16_nt_add(const void* A, const void* B, void* C, int M, int N, int K, int lda, int ldb, int ldc,
+                                    float* ws, hipStream_t stream) {
+  using namespace kgs;
+  if (M <= 0 || N <= 0 || K <= 0 || lda < K || ldb < K || ldc < N) return KGS_ERR_SHAPE;
+  if (N % 8 || ldc % 8 || (uintptr_t)C % 16 || (uintptr_t)ws % 16 || !gemm_any_ok(A, B, M, N, K, lda, ldb)) return KGS_ERR_ALIGN;
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(stream, &cs) != hipSuccess) return KGS_ERR_ARG;
+  if (cs == hipStreamCaptureStatusNone && rows_ok(A, B, C, M, N, K, lda, ldb, ldc))
+    if (int* tq = tile_queue(stream))
+      return (int)launch_w4p<EPI_ADDC>((const unsigned short*)A, (const unsigned short*)B, (unsigned short*)C, nullptr, M, N,
+                                       K, lda, ldb, ldc, cu_count(), tq, stream);
+  return gemm_any(A, B, C, nullptr, nullptr, M, N, K, lda, ldb, ldc, EPI_ADDC, 0, 0, 0, ws, stream);
+}
+
+// C [M, N / 2] = act(A . gate^T) * (A . up^T) for a fused weight B = [gate; up] of N rows, both products
+// rounded to bf16 first: the persistent kernel above one 256x256 tile per CU, else gemm_any.hip's.
+// act: a GateAct; limit: the clamped gate's, fp32 on the device.
+KGS_EXPORT int kgs_gemm_bf16_nt_swiglu(const void* A, const void* B, void* C, int M, int N, int K, int lda, int ldb,
+                                       int ldc, int act, const float* limit, hipStream_t stream) {
+  using namespace kgs;
+  if (M <= 0 || N <= 0 || K <= 0 || lda < K || ldb < K || ldc < N / 2) return KGS_ERR_SHAPE;
+  if (act != GATE_SILU && act != GATE_GELU && (act != GATE_CLAMPED || !limit || (uintptr_t)limit % 4)) return KGS_ERR_ARG;
+  if (N % 16 || ldc % 8 || (uintptr_t)C % 16 || !gemm_any_ok(A, B, M, N, K, lda, ldb)) return KGS_ERR_ALIGN;
+  if (rows_ok(A, B, C, M, N, K, lda, ldb, ldc))
+    if (int* tq = tile_queue(stream))
+      return (int)launch_w4p_swiglu((const unsigned short*)A, (const unsigned short*)B, (unsigned short*)C, M, N, K, lda,
+                                    ldb, ldc, cu_count(), tq, act, limit, stream);
+  return gemm_any_swiglu(A, B, C, M, N, K, lda, ldb, ldc, act, limit, stream);
 }
 
 // gemm_any.hip's kernel on tiles bm x bn (256 x 256, 256 x 128 or 128 x 128) over ns K slices (ws:

@@ -20,9 +20,23 @@ namespace kgs {
 template <int EPI>
 hipError_t launch_w4p(const unsigned short* A, const unsigned short* B, unsigned short* C, const unsigned short* bias,
                       int M, int N, int K, int lda, int ldb, int ldc, int cus, int* tq, hipStream_t s) {
-  const int tiles = (M / 256) * (N / 256);
+  const int tiles = (M + 255) / 256 * (N / 256);
   const dim3 pg(tiles < cus ? tiles : cus);
   const bool tall = M > N, longk = K > 8192;
+  if (M % 256) {
+    // any M (the prompt rows of a serving step): 8832 x 4096 x 14336 one-shot 867 us
+    if constexpr (EPI == EPI_NONE || EPI == EPI_ADDC) {
+#define KGS_ROWS(X) \
+  hipLaunchKernelGGL((w4p::gemm_nt_w4p<EPI, X, 1, false, false, 0, 0, 2, true>), pg, dim3(256), 0, s, A, B, C, bias, M, N, K, lda, ldb, ldc, tq)
+      if (tall && longk) KGS_ROWS(140000008);
+      else if (tall) KGS_ROWS(140000000);
+      else if (longk) KGS_ROWS(8);
+      else KGS_ROWS(0);
+#undef KGS_ROWS
+      return hipGetLastError();
+    }
+    return hipErrorInvalidValue;  // the callers send ragged rows with other epilogues elsewhere
+  }
   if (tall && longk)
     hipLaunchKernelGGL((w4p::gemm_nt_w4p<EPI, 140000008>), pg, dim3(256), 0, s, A, B, C, bias, M, N, K, lda, ldb, ldc,
                        tq);
@@ -58,17 +72,23 @@ hipError_t launch_w4p(const unsigned short* A, const unsigned short* B, unsigned
 // so the result is bitwise the one-shot kernel's
 hipError_t launch_w4p_swiglu(const unsigned short* A, const unsigned short* B, unsigned short* C, int M, int N,
                              int K, int lda, int ldb, int ldc, int cus, int* tq, int act, const float* limit, hipStream_t s) {
-  const int tiles = (M / 256) * (N / 256);
+  const int tiles = (M + 255) / 256 * (N / 256);
   const dim3 pg(tiles < cus ? tiles : cus);
-  if (act == GATE_CLAMPED)
-    hipLaunchKernelGGL((w4p::gemm_nt_w4p<EPI_NONE, 4000000>), pg, dim3(256), 0, s, A, B, C,
-                       (const unsigned short*)limit, M, N, K, lda, ldb, ldc, tq);
-  else if (act == GATE_GELU)
-    hipLaunchKernelGGL((w4p::gemm_nt_w4p<EPI_NONE, 2000000>), pg, dim3(256), 0, s, A, B, C, nullptr, M, N, K, lda, ldb,
-                       ldc, tq);
-  else
-    hipLaunchKernelGGL((w4p::gemm_nt_w4p<EPI_NONE, 1000000>), pg, dim3(256), 0, s, A, B, C, nullptr, M, N, K, lda, ldb,
-                       ldc, tq);
+  const auto lim = act == GATE_CLAMPED ? (const unsigned short*)limit : nullptr;
+#define KGS_SW(X)                                                                                                     \
+  if (M % 256)                                                                                                        \
+    hipLaunchKernelGGL((w4p::gemm_nt_w4p<EPI_NONE, X, 1, false, false, 0, 0, 2, true>), pg, dim3(256), 0, s, A, B, C, \
+                       lim, M, N, K, lda, ldb, ldc, tq);                                                              \
+  else                                                                                                                \
+    hipLaunchKernelGGL((w4p::gemm_nt_w4p<EPI_NONE, X>), pg, dim3(256), 0, s, A, B, C, lim, M, N, K, lda, ldb, ldc, tq)
+  if (act == GATE_CLAMPED) {
+    KGS_SW(4000000);
+  } else if (act == GATE_GELU) {
+    KGS_SW(2000000);
+  } else {
+    KGS_SW(1000000);
+  }
+#undef KGS_SW
   return hipGetLastError();
 }
 

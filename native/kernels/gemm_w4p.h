@@ -280,9 +280,9 @@ __device__ __forceinline__ void pstep(const Ctx& c, const Ctx& cd, Frag<MA, NB>&
 // Epilogue of one tile, pairs of accumulators (q, q + 1) = (i, n), (i, n + 1):
 // bias + activation, pack to bf16, pair n-tiles with v_permlane16_swap -> one
 // 16-B store per lane (the one-shot kernel's epilogue, reading named AGPRs).
-template <int EPI, int Q, bool NTST = false, int CST = 0>
+template <int EPI, int Q, bool NTST = false, int CST = 0, bool BNDM = false>
 __device__ __forceinline__ void pepi(const Ctx& c, unsigned short* __restrict__ C, int ldc, int tm, int tn,
-                                     const float (&bv)[NB][4]) {
+                                     const float (&bv)[NB][4], int M = 0) {
   if constexpr (Q < MA * NB) {
     constexpr int i = Q / NB, n = Q % NB;
     const int lane = threadIdx.x & 63, fr = lane & 15, fq = lane >> 4;
@@ -305,9 +305,9 @@ __device__ __forceinline__ void pepi(const Ctx& c, unsigned short* __restrict__ 
     } else if constexpr (CST == 1) {
       if (ldc < 0) *dst = qv;  // measurement build: C is never written (ldc > 0), the packing stays
     } else {
-      *dst = qv;
+      if (!BNDM || row < M) *dst = qv;
     }
-    pepi<EPI, Q + 2, NTST, CST>(c, C, ldc, tm, tn, bv);
+    pepi<EPI, Q + 2, NTST, CST, BNDM>(c, C, ldc, tm, tn, bv, M);
   }
 }
 
@@ -387,17 +387,18 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc_c(unsigned short* C, int 
 // before group I's stores, so a tile's epilogue waits out about one memory
 // latency instead of one per store (32 per wave): +15 % on the prompt pass's o
 // projection when each store read its chunk itself.
-template <int I>
+template <int I, bool BNDM = false>
 __device__ __forceinline__ void pepi_addc(const Ctx& c, unsigned short* __restrict__ C, int ldc, int tm, int tn,
-                                          const uint4 (&old)[NB / 2]) {
+                                          const uint4 (&old)[NB / 2], int M = 0) {
   if constexpr (I < MA) {
     const int lane = threadIdx.x & 63, fr = lane & 15, fq = lane >> 4;
-    unsigned short* rowp = C + (long)(tm * BM + c.wr * (BM / 2) + I * 16 + fr) * ldc + tn * BN + c.wc * (BN / 2) +
-                           (fq & 1) * 16 + (fq >> 1) * 8;
+    const int row = tm * BM + c.wr * (BM / 2) + I * 16 + fr;
+    unsigned short* rowp = C + (long)row * ldc + tn * BN + c.wc * (BN / 2) + (fq & 1) * 16 + (fq >> 1) * 8;
     uint4 nxt[NB / 2];
     if constexpr (I + 1 < MA) {
 #pragma unroll
-      for (int p = 0; p < NB / 2; ++p) nxt[p] = *(const uint4*)(rowp + 16L * ldc + p * 32);
+      for (int p = 0; p < NB / 2; ++p)
+        nxt[p] = !BNDM || row + 16 < M ? *(const uint4*)(rowp + 16L * ldc + p * 32) : make_uint4(0, 0, 0, 0);
     }
     w4::static_for<0, NB / 2>([&](auto pc) {
       constexpr int p = decltype(pc)::value, q = I * NB + 2 * p;
@@ -406,9 +407,9 @@ __device__ __forceinline__ void pepi_addc(const Ctx& c, unsigned short* __restri
       const unsigned x1 = pack_bf16x2(v1[0], v1[1]), y1 = pack_bf16x2(v1[2], v1[3]);
       auto sx = __builtin_amdgcn_permlane16_swap(x0, x1, false, false);
       auto sy = __builtin_amdgcn_permlane16_swap(y0, y1, false, false);
-      *(uint4*)(rowp + p * 32) = add_bf16x8(old[p], make_uint4(sx[0], sy[0], sx[1], sy[1]));
+      if (!BNDM || row < M) *(uint4*)(rowp + p * 32) = add_bf16x8(old[p], make_uint4(sx[0], sy[0], sx[1], sy[1]));
     });
-    pepi_addc<I + 1>(c, C, ldc, tm, tn, nxt);
+    pepi_addc<I + 1, BNDM>(c, C, ldc, tm, tn, nxt, M);
   }
 }
 
@@ -429,9 +430,9 @@ __device__ __forceinline__ uint2 swiglu4(float limit) {
   return make_uint2(pack_bf16x2(r[0], r[1]), pack_bf16x2(r[2], r[3]));
 }
 
-template <int I, int QQ, int ACT>
+template <int I, int QQ, int ACT, bool BNDM = false>
 __device__ __forceinline__ void pepi_sw(const Ctx& c, unsigned short* __restrict__ C, int ldc, int tm, int tn,
-                                        float limit) {
+                                        float limit, int M = 0) {
   if constexpr (I < MA) {
     if constexpr (QQ < NB / 2) {
       const int lane = threadIdx.x & 63, fr = lane & 15, fq = lane >> 4;
@@ -441,10 +442,10 @@ __device__ __forceinline__ void pepi_sw(const Ctx& c, unsigned short* __restrict
       const uint4 qv = make_uint4(sx[0], sy[0], sx[1], sy[1]);
       const int row = tm * BM + c.wr * (BM / 2) + I * 16 + fr;
       const int col0 = tn * (BN / 2) + c.wc * (BN / 4) + QQ * 16;
-      *(uint4*)(C + (long)row * ldc + col0 + (fq & 1) * 16 + (fq >> 1) * 8) = qv;
-      pepi_sw<I, QQ + 2, ACT>(c, C, ldc, tm, tn, limit);
+      if (!BNDM || row < M) *(uint4*)(C + (long)row * ldc + col0 + (fq & 1) * 16 + (fq >> 1) * 8) = qv;
+      pepi_sw<I, QQ + 2, ACT, BNDM>(c, C, ldc, tm, tn, limit, M);
     } else {
-      pepi_sw<I + 1, 0, ACT>(c, C, ldc, tm, tn, limit);
+      pepi_sw<I + 1, 0, ACT, BNDM>(c, C, ldc, tm, tn, limit, M);
     }
   }
 }
@@ -462,8 +463,10 @@ __device__ __forceinline__ void mark_bad_ticket(int* q, int raw, int ntx) {
     atomicExch(q + TQ_ERR_WORD, (int)(0x80000000u | ((unsigned)raw & 0x7fffffffu)));
 }
 
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc_a(const unsigned short* A, int tm, int lda) {
-  return __builtin_amdgcn_make_buffer_rsrc((void*)(A + (long)tm * BM * lda), 0, BM * lda * 2, 0x00020000);
+template <bool BNDM = false>
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc_a(const unsigned short* A, int tm, int lda, int M = 0) {
+  const int rows = BNDM ? min(M - tm * BM, BM) : BM;
+  return __builtin_amdgcn_make_buffer_rsrc((void*)(A + (long)tm * BM * lda), 0, rows * lda * 2, 0x00020000);
 }
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc_b(const unsigned short* B, int tn, int ldb) {
   return __builtin_amdgcn_make_buffer_rsrc((void*)(B + (long)tn * BN * ldb), 0, BN * ldb * 2, 0x00020000);
@@ -505,7 +508,10 @@ __device__ __forceinline__ void set_b(Ctx& c, const unsigned short* B, int tn, i
 // (vmcnt(ND + stores)), so it waits for the next tile's K-tile 1 only.
 // DD, SPS: deferred C stores (see pepi_d): SPS 16-B units per lane stored at the end of each of the next
 // tile's first DD K-steps (0 = off, the epilogue stores everything). Needs K / 64 >= PEEL + 2 (below).
-template <int EPI, int X = 0, int DYN = 1, bool NTST = false, bool TS = false, int L = 0, int DD = 0, int SPS = 2>
+// BNDM: any M. The last tile row's A resource ends at row M, so that the rows past it are zeros in
+// LDS, and its stores are predicated.
+template <int EPI, int X = 0, int DYN = 1, bool NTST = false, bool TS = false, int L = 0, int DD = 0, int SPS = 2,
+          bool BNDM = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void gemm_nt_w4p(
     const unsigned short* __restrict__ A, const unsigned short* __restrict__ B, unsigned short* __restrict__ C,
     const unsigned short* __restrict__ bias, int M, int N, int K, int lda, int ldb, int ldc, int* __restrict__ q) {
@@ -520,7 +526,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
   KGS_ACC_RESERVE();
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int ntm = M / BM, ntn = N / BN, ntiles = ntm * ntn;
+  const int ntm = BNDM ? (M + BM - 1) / BM : M / BM, ntn = N / BN, ntiles = ntm * ntn;
+  static_assert(!BNDM || (DD == 0 && !NTST && !TS && L == 0), "any M: plain stores");
   static_assert(!TS || EPI == EPI_NONE, "timing build: bias carries the stamp buffer");
   // X digit 10^6: SwiGLU (B = fused [gate; up], N = 2I rows, C = [M, I]); tiles
   // are 256 B rows = 128 gate + 128 up, ntn = N / 256
@@ -605,7 +612,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
   }
   int sl, tm, tn;
   w4::tile_of<X, false>(DYN ? x + 8 * t : t, ntiles, ntm, ntn, sl, tm, tn);
-  c.ra = rsrc_a(A, tm, lda);
+  c.ra = rsrc_a<BNDM>(A, tm, lda, M);
   set_b<SW>(c, B, tn, ldb, N);
 
   // prologue: K-tiles 0, 1 of the first tile into stages 0, 1; k-sub 0 of K-tile 0 into f0
@@ -673,7 +680,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     int tmn = tm, tnn = tn;
     if (more) w4::tile_of<X, false>(DYN ? x + 8 * tnx : tnx, ntiles, ntm, ntn, sl, tmn, tnn);
     Ctx cn = c;
-    cn.ra = rsrc_a(A, tmn, lda);
+    cn.ra = rsrc_a<BNDM>(A, tmn, lda, M);
     set_b<SW>(cn, B, tnn, ldb, N);
     // the last two K-steps bring the next tile's K-tiles 0 and 1 (no next tile:
     // harmless re-loads of this tile's last K-tile into the freed stages)
@@ -682,7 +689,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 3" ::: "memory");  // MFMA -> v_accvgpr_read
     if constexpr (SW) {
       constexpr int ACT = (X / 1000000) % 10;
-      pepi_sw<0, 0, ACT>(c, C, ldc, tm, tn, ACT == GATE_CLAMPED ? *(const float*)bias : 0.f);
+      pepi_sw<0, 0, ACT, BNDM>(c, C, ldc, tm, tn, ACT == GATE_CLAMPED ? *(const float*)bias : 0.f, M);
     }
     float bv[NB][4];
     if constexpr (!SW) {
@@ -700,17 +707,18 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     }
     if constexpr (EPI == EPI_ADDC) {
       const int fr = lane & 15, fq = lane >> 4;
-      const unsigned short* r0 =
-          C + (long)(tm * BM + c.wr * (BM / 2) + fr) * ldc + tn * BN + c.wc * (BN / 2) + (fq & 1) * 16 + (fq >> 1) * 8;
+      const int row0 = tm * BM + c.wr * (BM / 2) + fr;
+      const unsigned short* r0 = C + (long)row0 * ldc + tn * BN + c.wc * (BN / 2) + (fq & 1) * 16 + (fq >> 1) * 8;
       uint4 old0[NB / 2];
 #pragma unroll
-      for (int p = 0; p < NB / 2; ++p) old0[p] = *(const uint4*)(r0 + p * 32);
-      pepi_addc<0>(c, C, ldc, tm, tn, old0);
+      for (int p = 0; p < NB / 2; ++p)
+        old0[p] = !BNDM || row0 < M ? *(const uint4*)(r0 + p * 32) : make_uint4(0, 0, 0, 0);
+      pepi_addc<0, BNDM>(c, C, ldc, tm, tn, old0, M);
     } else if constexpr (DEF > 0) {
       pepi_d<EPI, 0, UI, DEF, NTST>(c, C, ldc, tm, tn, bv, dq);
       rprev = rsrc_c(C, tm, tn, ldc);
     } else if constexpr (!SW) {
-      pepi<EPI, 0, NTST, CST>(c, C, ldc, tm, tn, bv);
+      pepi<EPI, 0, NTST, CST, BNDM>(c, C, ldc, tm, tn, bv, M);
       if constexpr (CST == 2) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     }
     if constexpr (TS) {

@@ -163,6 +163,43 @@ def test_linear_keeps_nan_and_skips_what_needs_no_gradient():
     assert x.grad is None and lin.weight.grad is not None
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 256, 128), (130, 512, 384), (257, 1024, 512), (4500, 4096, 384), (8320, 2304, 512)])
+def test_products_of_any_rows_add_and_gate_like_their_parts(M, N, K):
+    """The residual add and the gated product in the epilogue, on ragged rows of small and of
+    persistent grids, against the product and a separate pass."""
+    from kgs.ops import gemm_nt
+    from kgs.ops.gemm import _scratch_floats, add_product_, gemm_swiglu
+    from kgs.ops.transformer import silu_mul
+
+    a, b = rnd(M, K), rnd(N, K)
+    c = gemm_nt(a, b)
+    assert rel(c, a.double() @ b.double().T) < REL
+    x = rnd(M, N)
+    want = (x.float() + c.float()).bfloat16()
+    assert add_product_(a, b, x)
+    assert torch.equal(x, want) if not _scratch_floats(M, N, K) else rel(x, want.double()) < REL
+    if N % 128 == 0:
+        assert torch.equal(gemm_swiglu(a, b), silu_mul(gemm_nt(a, b, variant="bounded")))
+
+
+@pytest.mark.parametrize("act", ["gelu_tanh", "clamped"])
+@pytest.mark.parametrize("M", [100, 4500])
+def test_gated_products_of_any_rows(act, M):
+    from kgs.ops.activation import Gate
+    from kgs.ops.gemm import gemm_swiglu
+
+    gate = Gate(act, 0.5 if act == "clamped" else 0.0)
+    a, w = rnd(M, 512), rnd(4096, 512)
+    z = a.double() @ w.double().T
+    g, u = z[:, :2048], z[:, 2048:]
+    if act == "clamped":
+        g, u = g.clamp(max=0.5), u.clamp(-0.5, 0.5)
+        want = g * torch.sigmoid(1.702 * g) * (u + 1)
+    else:
+        want = torch.nn.functional.gelu(g, approximate="tanh") * u
+    assert rel(gemm_swiglu(a, w, gate), want) < 3 * REL
+
+
 @pytest.mark.parametrize("M,N,K", [(256, 256, 768), (256, 768, 1024), (1024, 1024, 4096)])
 def test_fp8_small_grids_equal_the_eight_wave_kernel(M, N, K):
     from kgs.ops import gemm_fp8_nt, quantize_fp8

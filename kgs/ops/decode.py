@@ -585,6 +585,16 @@ def decode_splits(batch: int, kv_heads: int, max_pages: int, cus: int = CUS, min
     return pps, math.ceil(max_pages / pps)
 
 
+def workgroup_splits(batch: int, kv_heads: int, max_pages: int, cus: int = CUS) -> int:
+    """Parts of every sequence's pages for the attention by workgroups. Two workgroups per
+    CU read the cache fastest, so parts are made up to there: of at least 8 pages by the table's
+    width while most CUs idle, of 32 from half the CUs on, where a merge costs as much as
+    the shorter parts save (us, 8 KV heads: one sequence of 4000 tokens 42 / 16 / 11 in 1 / 4 / 16
+    parts; 16 of 1000 15.0 / 17.2 in 1 / 4; 16 unequal ones of up to 4000 27.7 / 22.3)."""
+    groups = batch * kv_heads
+    return min(-(-2 * cus // groups), max(1, max_pages // (8 if 2 * groups < cus else 32)))
+
+
 _AWS: dict = {}
 
 
@@ -673,7 +683,10 @@ def paged_decode_attention(q: torch.Tensor, cache_layer: torch.Tensor, block_tab
     if ctx_lens.dtype != torch.int32 or not ctx_lens.is_contiguous() or ctx_lens.numel() != b:
         raise ValueError("ctx_lens must be contiguous int32 [B]")
     max_pages = block_tables.shape[1]
-    if pages_per_split is None:
+    by_workgroup = pages_per_split is None and pipe is None
+    if by_workgroup:
+        nsplit = workgroup_splits(b, kv_heads, max_pages) if b else 1
+    elif pages_per_split is None:
         pps, nsplit = decode_splits(b, kv_heads, max_pages)
     else:
         pps, nsplit = pages_per_split, math.ceil(max_pages / pages_per_split)
@@ -681,6 +694,15 @@ def paged_decode_attention(q: torch.Tensor, cache_layer: torch.Tensor, block_tab
         out = torch.empty((b, heads * HEAD_DIM), dtype=torch.bfloat16, device=q.device)
     po, pml, cnt = _attn_workspace(b, heads, kv_heads, nsplit, q.device)
     scale = 1.0 / math.sqrt(HEAD_DIM) if scale is None else scale
+    if by_workgroup:
+        rc = _lib.lib().kgs_paged_decode_wg(q.data_ptr(), cache_layer.data_ptr(), block_tables.data_ptr(), ctx_lens.data_ptr(),
+                                            out.data_ptr(), po.data_ptr() if po is not None else None,
+                                            pml.data_ptr() if pml is not None else None,
+                                            cnt.data_ptr() if cnt is not None else None, b, heads, kv_heads, HEAD_DIM,
+                                            max_pages, nsplit, q.stride(0), out.stride(0), float(scale),
+                                            1 if cache_layer.dtype == FP8 else 0, _lib.stream_handle(q.device))
+        _lib.check(rc, "paged_decode_attention")
+        return out
     rc = _lib.lib().kgs_paged_decode_bf16_ex(q.data_ptr(), cache_layer.data_ptr(), block_tables.data_ptr(),
                                              ctx_lens.data_ptr(), out.data_ptr(),
                                              po.data_ptr() if po is not None else None,

@@ -1057,6 +1057,234 @@ __global__ __launch_bounds__(64) void paged_decode(AttnArgs a) {
   store_o(op, o, L > 0.f ? 1.f / L : 0.f);
 }
 
+// Decode attention by workgroups: W waves share a (sequence, KV head), or one of nsplit equal
+// parts of its pages. paged_decode gives every (sequence, KV head, fixed number of pages) one wave,
+// so a batch of unequal contexts waits for the longest one's wave, and at small batches a split
+// costs a merge through memory. Here the pages are dealt to the waves by the sequence's own length
+// (wave w takes pages w, w + W, ..) and the waves merge in LDS. Bound by the HBM reads of K and V:
+// 100 sequences of 60 to 2800 tokens (4 KV heads) 60 -> 42 us at 4.4 TB/s, one of 4000 (8 KV heads)
+// 22 -> 11 us, 256 unequal ones around 1024 329 -> 171 us; 256 equal ones of 1024, which the single
+// waves already read at 6.9 TB/s, 156 -> 163 us.
+//
+// A wave's page ids lie in its lanes (64 at a time, one load), so that no page waits for its id.
+// bf16 pages: eight waves, four on a SIMD hide each other's loads. e4m3 pages (PIPE): four waves
+// that keep the next page on its way in registers while they widen and multiply one (64 sequences
+// around 700 tokens, 8 KV heads: 22 us, 31 without).
+template <bool KV8>
+struct PageRegs;  // a page's K and V as loaded: fragment order, e4m3 pages 8 bytes a lane
+template <>
+struct PageRegs<false> {
+  bf16x8 k[8], v[8];
+  __device__ void load(const void* cache, long region, int lane) {
+    const bf16x8* p = (const bf16x8*)((const unsigned short*)cache + region) + lane;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) k[i] = __builtin_nontemporal_load(p + 64 * i);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = __builtin_nontemporal_load(p + PAGE_ELEMS / 8 + 64 * i);
+  }
+  __device__ bf16x8 kf(int i) const { return k[i]; }
+  __device__ bf16x8 vf(int i) const { return v[i]; }
+};
+template <>
+struct PageRegs<true> {
+  u32x2 k[8], v[8];
+  __device__ void load(const void* cache, long region, int lane) {
+    const u32x2* p = (const u32x2*)((const unsigned char*)cache + region) + lane;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) k[i] = __builtin_nontemporal_load(p + 64 * i);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = __builtin_nontemporal_load(p + PAGE_ELEMS / 8 + 64 * i);
+  }
+  __device__ bf16x8 kf(int i) const { return dequant8(k[i], 1.f); }
+  __device__ bf16x8 vf(int i) const { return dequant8(v[i], 1.f); }
+};
+
+template <bool KV8, int W = KV8 ? 4 : 8, bool PIPE = KV8>
+__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(PIPE ? 2 : 4, PIPE ? 2 : 4))) void paged_wg(AttnArgs a) {
+  constexpr int LDO = HD + 4;  // a row of partial outputs: 16 heads' rows start on different banks
+  __shared__ __attribute__((aligned(16))) float part[W][16][LDO];
+  __shared__ float mls[W][16][2];
+  __shared__ int is_last;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int G = a.H / a.HKV;
+  int id = blockIdx.x;
+  const int sp = id % a.nsplit;
+  id /= a.nsplit;
+  const int kvh = id % a.HKV, b = id / a.HKV;
+  const int g = lane >> 4, n = lane & 15;
+  const int ctx = a.ctx_lens[b];
+  const int npages = min((ctx + PAGE - 1) / PAGE, a.max_pages);
+  const int per = (npages + a.nsplit - 1) / a.nsplit;
+  const int p0 = sp * per, p1 = min(npages, p0 + per);
+  const int h = kvh * G + n;
+  const int mine = p1 > p0 + w ? (p1 - p0 - w + W - 1) / W : 0;  // this wave's pages
+
+  float m = -INFINITY, lsum = 0.f;
+  f32x4v acc[8];
+#pragma unroll
+  for (int dt = 0; dt < 8; ++dt) acc[dt] = f32x4v{0.f, 0.f, 0.f, 0.f};
+  if (mine) {
+    const int* bt = a.block_tables + (long)b * a.max_pages + p0 + w;
+    int ids = lane < mine ? bt[W * lane] : 0;
+    bf16x8 qf[4];
+    const unsigned short* qp = a.q + (long)b * a.ldq + (long)h * HD + 8 * g;
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) qf[ks] = n < G ? *(const bf16x8*)(qp + 32 * ks) : bf16x8{};
+    auto load_page = [&](PageRegs<KV8>& r, int j) {
+      if (j && (j & 63) == 0) ids = j + lane < mine ? bt[W * (j + lane)] : 0;
+      r.load(a.cache, ((long)__builtin_amdgcn_readlane(ids, j & 63) * a.HKV + kvh) * 2 * PAGE_ELEMS, lane);
+    };
+    auto page = [&](const PageRegs<KV8>& r, int j) {
+      f32x4v s[2];
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        s[t] = f32x4v{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) s[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(r.kf(t * 4 + ks), qf[ks], s[t], 0, 0, 0);
+      }
+      const int tok0 = (p0 + w + W * j) * PAGE + 4 * g;  // lane holds S^T[token 16t + 4g + i][head n]
+      float bm = -INFINITY;
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float v = (tok0 + 16 * t + i) < ctx ? s[t][i] * a.sl2 : -INFINITY;
+          s[t][i] = v;
+          bm = fmaxf(bm, v);
+        }
+      bm = wmax16(bm);
+      const float mn = fmaxf(m, bm), alpha = __builtin_amdgcn_exp2f(m - mn);
+      m = mn;
+      bf16x8 pf;
+      float ps = 0.f;
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float p = __builtin_amdgcn_exp2f(s[t][i] - mn);
+          ps += p;
+          pf[4 * t + i] = (short)f2bf(p);
+        }
+      lsum = lsum * alpha + ps;
+#pragma unroll
+      for (int dt = 0; dt < 8; ++dt) {
+        acc[dt] *= alpha;
+        acc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(r.vf(dt), pf, acc[dt], 0, 0, 0);
+      }
+    };
+    if constexpr (PIPE) {
+      PageRegs<KV8> ra, rb;
+      load_page(ra, 0);
+      for (int j = 0; j < mine; j += 2) {
+        if (j + 1 < mine) load_page(rb, j + 1);
+        page(ra, j);
+        if (j + 1 < mine) {
+          if (j + 2 < mine) load_page(ra, j + 2);
+          page(rb, j + 1);
+        }
+      }
+    } else {
+      for (int j = 0; j < mine; ++j) {
+        PageRegs<KV8> r;
+        load_page(r, j);
+        page(r, j);
+      }
+    }
+    lsum = wsum16(lsum);
+  }
+  // lane holds O^T[dim 16dt + 4g + i][head n]
+  if (n < G) {
+#pragma unroll
+    for (int dt = 0; dt < 8; ++dt) *(f32x4v*)&part[w][n][16 * dt + 4 * g] = acc[dt];
+    if (g == 0) {
+      mls[w][n][0] = m;
+      mls[w][n][1] = lsum;
+    }
+  }
+  __syncthreads();
+  const long nrows = (long)a.B * a.H * a.nsplit;
+  const __amdgpu_buffer_rsrc_t por = rsrc(a.po, (unsigned)(nrows * HD * 4));
+  const __amdgpu_buffer_rsrc_t mlr = rsrc(a.pml, (unsigned)(nrows * 8));
+  // a thread's four dims of one head
+  for (int i = threadIdx.x; i < G * (HD / 4); i += 64 * W) {
+    const int hn = i >> 5, d = (i & 31) * 4;
+    float M = -INFINITY;
+#pragma unroll
+    for (int x = 0; x < W; ++x) M = fmaxf(M, mls[x][hn][0]);
+    float L = 0.f;
+    f32x4v o = f32x4v{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int x = 0; x < W; ++x) {
+      const float l = mls[x][hn][1];
+      if (l <= 0.f) continue;
+      const float f = __builtin_amdgcn_exp2f(mls[x][hn][0] - M);
+      L += f * l;
+      o += f * *(const f32x4v*)&part[x][hn][d];
+    }
+    const int hh = kvh * G + hn;
+    if (a.nsplit == 1) {
+      const float inv = L > 0.f ? 1.f / L : 0.f;
+      *(uint2*)(a.o + (long)b * a.ldo + (long)hh * HD + d) =
+          make_uint2(pack_bf16x2(o[0] * inv, o[1] * inv), pack_bf16x2(o[2] * inv, o[3] * inv));
+    } else {
+      const unsigned row = (unsigned)(((long)b * a.H + hh) * a.nsplit + sp);
+      st_sc1(por, (row * HD + d) * 4, o);
+      if (d == 0) {
+        st1_sc1(mlr, row * 8, M);
+        st1_sc1(mlr, row * 8 + 4, L);
+      }
+    }
+  }
+  if (a.nsplit == 1) return;
+  // the split that arrives last merges: partial results written through, then a ticket
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    int* c = a.cnt + (long)b * a.HKV + kvh;
+    const int last = __hip_atomic_fetch_add(c, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == a.nsplit - 1;
+    if (last) {
+      __hip_atomic_store(c, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // re-arm
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    }
+    is_last = last;
+  }
+  __syncthreads();
+  if (!is_last) return;
+  for (int i = threadIdx.x; i < G * (HD / 4); i += 64 * W) {
+    const int hn = i >> 5, d = (i & 31) * 4, hh = kvh * G + hn;
+    const unsigned row = (unsigned)(((long)b * a.H + hh) * a.nsplit);
+    float M = -INFINITY, L = 0.f;
+    f32x4v o = f32x4v{0.f, 0.f, 0.f, 0.f};
+    for (int s0 = 0; s0 < a.nsplit; s0 += 4) {
+      float mv[4], lv[4];
+      f32x4v pv[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        mv[j] = -INFINITY;
+        lv[j] = 0.f;
+        if (s0 + j < a.nsplit) {
+          mv[j] = ld1_sc1(mlr, (row + s0 + j) * 8);
+          lv[j] = ld1_sc1(mlr, (row + s0 + j) * 8 + 4);
+          pv[j] = ld_sc1(por, ((row + s0 + j) * HD + d) * 4);
+        }
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        if (lv[j] <= 0.f) continue;
+        const float mn = fmaxf(M, mv[j]);
+        const float sc = __builtin_amdgcn_exp2f(M - mn), f = __builtin_amdgcn_exp2f(mv[j] - mn);
+        L = L * sc + f * lv[j];
+        o = o * sc + f * pv[j];
+        M = mn;
+      }
+    }
+    const float inv = L > 0.f ? 1.f / L : 0.f;
+    *(uint2*)(a.o + (long)b * a.ldo + (long)hh * HD + d) =
+        make_uint2(pack_bf16x2(o[0] * inv, o[1] * inv), pack_bf16x2(o[2] * inv, o[3] * inv));
+  }
+}
+
 // merge nsplit partials (m in log2 units, l, unnormalised O) of one (b, h):
 // the launch-boundary variant, for batches with many (sequence, KV head)
 // groups -- there an in-launch last-arriver merge costs one L2-invalidating
@@ -1383,6 +1611,26 @@ KGS_EXPORT int kgs_paged_decode_bf16_ex(const void* q, const void* cache, const 
   if (nsplit > 1 && !merge)
     hipLaunchKernelGGL(paged_reduce, dim3((unsigned)(B * H)), dim3(64), 0, s, po, pml, (unsigned short*)o, H, nsplit,
                        ldo);
+  return (int)hipGetLastError();
+}
+
+// Paged decode attention by workgroups, nsplit equal parts of every sequence's pages (paged_wg). Arguments as kgs_paged_decode_bf16; nsplit > 1 needs po, pml and
+// cnt, and merges in the same launch.
+KGS_EXPORT int kgs_paged_decode_wg(const void* q, const void* cache, const int* block_tables, const int* ctx_lens, void* o,
+                                   float* po, float* pml, int* cnt, int B, int H, int HKV, int hd, int max_pages,
+                                   int nsplit, long ldq, long ldo, float scale, int kv8, hipStream_t s) {
+  using namespace kgs::dec;
+  if (B <= 0 || H <= 0 || HKV <= 0 || H % HKV || H / HKV > 16 || hd != HD || max_pages <= 0 || nsplit <= 0) return KGS_ERR_SHAPE;
+  if (ldq < (long)H * HD || ldo < (long)H * HD) return KGS_ERR_SHAPE;
+  if (!al16(q) || !al16(cache) || !al16(o) || ldq % 8 || ldo % 8) return KGS_ERR_ALIGN;
+  if (nsplit > 1 && (!po || !pml || !cnt || !al16(po))) return KGS_ERR_ARG;
+  const long nwg = (long)B * HKV * nsplit;
+  if (nwg > 0x7fffffff || (long)B * H * nsplit * HD * 4 > 0xffffffffL) return KGS_ERR_SHAPE;
+  AttnArgs a{(const unsigned short*)q, (const unsigned short*)cache, block_tables, ctx_lens, (unsigned short*)o, po,
+             pml, cnt, ldq, ldo, B, H, HKV, max_pages, 0, nsplit, 1, scale * 1.4426950408889634f,
+             nullptr, 0, nullptr, nullptr, nullptr, nullptr, nullptr};
+  if (kv8) hipLaunchKernelGGL(paged_wg<true>, dim3((unsigned)nwg), dim3(256), 0, s, a);
+  else hipLaunchKernelGGL(paged_wg<false>, dim3((unsigned)nwg), dim3(512), 0, s, a);
   return (int)hipGetLastError();
 }
 

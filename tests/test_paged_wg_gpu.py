@@ -1,0 +1,85 @@
+"""Decode attention by workgroups (paged_wg in native/kernels/decode.hip) where its parts meet:
+one token, page and wave borders, more parts than pages, one and sixteen query heads per key
+head, contexts of very different lengths, e4m3 pages, replays from a hipGraph."""
+import math
+
+import pytest
+
+torch = pytest.importorskip("torch")
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def setup(lens, hkv, group, fp8=False, seed=0):
+    from kgs.ops import decode as D
+
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    need = [math.ceil(n / 32) for n in lens]
+    cache = torch.randn(sum(need) + 1, hkv, 2, 4096, device=DEV, generator=g).to(D.FP8 if fp8 else torch.bfloat16)
+    ids = 1 + torch.randperm(sum(need), device=DEV, generator=g).int()
+    tables = torch.zeros(len(lens), max(need) + 3, dtype=torch.int32, device=DEV)
+    at = 0
+    for i, n in enumerate(need):
+        tables[i, :n] = ids[at:at + n]
+        at += n
+    q = (2 * torch.randn(len(lens), (group + 2) * hkv * 128, device=DEV, generator=g)).bfloat16()
+    return q, cache, tables, torch.tensor(lens, dtype=torch.int32, device=DEV)
+
+
+def run(q, cache, tables, ctx, heads, hkv, nsplit, out):
+    from kgs.ops import _lib
+    from kgs.ops import decode as D
+
+    ws = D._attn_workspace(q.shape[0], heads, hkv, nsplit, q.device)
+    rc = _lib.lib().kgs_paged_decode_wg(q.data_ptr(), cache.data_ptr(), tables.data_ptr(), ctx.data_ptr(), out.data_ptr(),
+                                        *(None if t is None else t.data_ptr() for t in ws), q.shape[0], heads, hkv, 128,
+                                        tables.shape[1], nsplit, q.stride(0), out.stride(0), 128 ** -0.5,
+                                        int(cache.dtype == D.FP8), _lib.stream_handle(q.device))
+    assert rc == 0
+
+
+# weights and values are bf16 (2^-8 each), so a row moves by at most their product's share of |v| < 6
+TOL = 3e-2
+
+
+@pytest.mark.parametrize("hkv,group", [(8, 4), (1, 16), (4, 1), (2, 7)])
+@pytest.mark.parametrize("nsplit", [1, 2, 5])
+@pytest.mark.parametrize("fp8", [False, True])
+def test_parts_and_lengths(hkv, group, nsplit, fp8):
+    from kgs.ops import decode as D
+
+    lens = [1, 31, 32, 33, 256, 257, 300, 2200]
+    q, cache, tables, ctx = setup(lens, hkv, group, fp8)
+    want = D.ref_paged_decode(q, cache, tables, ctx, hkv * group, hkv)
+    out = torch.full((len(lens) + 1, hkv * group * 128), 7.0, dtype=torch.bfloat16, device=DEV)
+    for _ in range(2):  # the merge leaves its tickets at zero
+        run(q, cache, tables, ctx, hkv * group, hkv, nsplit, out[:len(lens)])
+        assert float((out[:len(lens)].float() - want).abs().max()) < TOL
+    assert bool((out[-1] == 7).all())
+
+
+def test_an_empty_context_gives_zeros_and_a_graph_replays():
+    from kgs.ops import decode as D
+
+    q, cache, tables, ctx = setup([40, 500, 90, 1000], 8, 4)
+    ctx[2] = 0
+    eager = D.paged_decode_attention(q, cache, tables, ctx, 32, 8)
+    assert bool((eager[2] == 0).all())
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = D.paged_decode_attention(q, cache, tables, ctx, 32, 8)
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        D.paged_decode_attention(q, cache, tables, ctx, 32, 8)
+        torch.cuda.synchronize()
+        assert torch.equal(out, eager)
+
+
+@pytest.mark.parametrize("batch,kv,pages", [(1, 8, 1), (1, 8, 32), (1, 1, 4096), (16, 8, 128), (64, 8, 64), (300, 8, 16)])
+def test_split_rule_stays_in_its_bounds(batch, kv, pages):
+    from kgs.ops.decode import workgroup_splits
+
+    n = workgroup_splits(batch, kv, pages)
+    assert 1 <= n <= max(1, pages // 8) and (n == 1 or (n - 1) * batch * kv < 512)

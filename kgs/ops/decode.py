@@ -737,6 +737,24 @@ def ref_cache_write(cache_layer: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
         cache_layer[page[:, None], h, 1, v_idx[tau]] = cvt(v[:, h])
 
 
+def gather_kv_into(cache_layer: torch.Tensor, pages: torch.Tensor, ctx: int, k: torch.Tensor, v: torch.Tensor) -> None:
+    """:func:`gather_kv` into the given row-major bf16 ``k``, ``v`` (of one row stride), in one
+    launch; rows of a page outside the cache come back zero."""
+    rows, hkv = k.shape[0], cache_layer.shape[1]
+    if cache_layer.dtype not in (torch.bfloat16, FP8) or not cache_layer.is_contiguous():
+        raise ValueError("the cache must be contiguous bf16 or e4m3")
+    if pages.numel() < (ctx + PAGE - 1) // PAGE or not 0 <= ctx <= rows:
+        raise ValueError(f"{pages.numel()} pages and {rows} rows for {ctx} tokens")
+    if k.dtype != torch.bfloat16 or v.dtype != torch.bfloat16 or k.shape != v.shape or k.stride() != v.stride() or \
+            k.shape[1] != hkv * HEAD_DIM or k.stride(1) != 1:
+        raise ValueError("k and v must be row-major bf16 [rows, kv_heads * 128] of one row stride")
+    pages = pages.to(cache_layer.device, torch.int32).contiguous()
+    rc = _lib.lib().kgs_gather_kv(cache_layer.data_ptr(), pages.data_ptr(), k.data_ptr(), v.data_ptr(), ctx, rows, hkv, HEAD_DIM,
+                                  cache_layer.shape[0], k.stride(0), 1 if cache_layer.dtype == FP8 else 0,
+                                  _lib.stream_handle(k.device))
+    _lib.check(rc, "gather_kv")
+
+
 _KV_IDX: dict = {}
 
 
@@ -746,7 +764,7 @@ def gather_kv(cache_layer: torch.Tensor, pages: torch.Tensor, ctx: int, rows: in
     ``k``, ``v`` ``[rows, kv_heads * 128]`` bf16 (rows ``ctx .. rows-1`` zero) --
     the keys/values a prefill chunk attends to (``rows`` pads them to the
     chunk's q-blocks). Vectorised torch gathers through the page layout's index
-    tables; an fp8 cache is widened to bf16."""
+    tables; an fp8 cache is widened to bf16. :func:`gather_kv_into` is the one-launch form."""
     rows = ctx if rows is None else rows
     dev = cache_layer.device
     key = (dev.type, dev.index)

@@ -263,6 +263,45 @@ def attention_ragged(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, items: t
     return out
 
 
+QBLOCK = 128  # query rows of an attention_blocks item
+
+
+def attention_blocks(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, items: torch.Tensor, heads: int, kv_heads: int,
+                     out: torch.Tensor, k2: torch.Tensor | None = None, v2: torch.Tensor | None = None,
+                     scale: float | None = None) -> torch.Tensor:
+    """Causal flash attention of sequences of any lengths in one launch (head_dim 128), a block of 128
+    query rows each item. ``items`` int32 ``[n, 4]``: the block's first row in ``q`` / ``out``, the row
+    of its sequence's key 0, the position of the first row (a multiple of 64), and 0 for keys
+    in ``k`` / ``v`` or 1 for keys in ``k2`` / ``v2``. An item reads its position + 128 keys."""
+    for t, n in ((q, "q"), (k, "k"), (v, "v"), (out, "out")):
+        _need(t, n)
+    if items.dtype != torch.int32 or items.dim() != 2 or items.shape[1] != 4 or not items.is_contiguous():
+        raise ValueError("items must be contiguous int32 [n, 4]")
+    if (k2 is None) != (v2 is None) or (k2 is not None and k2.stride() != v2.stride()):
+        raise ValueError("k2 and v2 come together, with one row stride")
+    scale = 1.0 / math.sqrt(128) if scale is None else scale
+    two = (0, 0, 0) if k2 is None else (k2.data_ptr(), v2.data_ptr(), k2.stride(0))
+    rc = _lib.lib().kgs_attn_fwd_blocks_bf16(q.data_ptr(), k.data_ptr(), v.data_ptr(), two[0], two[1], out.data_ptr(),
+                                             items.data_ptr(), items.shape[0], heads, kv_heads, 128, q.stride(0),
+                                             k.stride(0), v.stride(0), two[2], out.stride(0), float(scale),
+                                             _lib.stream_handle(q.device))
+    _lib.check(rc, "attention_blocks")
+    return out
+
+
+def block_items(seqs, rows: int):
+    """Items of :func:`attention_blocks`, heaviest first, for sequences ``(first query row, rows (a
+    multiple of 128), first key row, position of the first row (a multiple of 64), key
+    source)`` among ``rows`` query rows (and keys, for source 0)."""
+    import numpy as np
+
+    for r, n, k0, pos, src in seqs:
+        if n <= 0 or n % QBLOCK or pos % 64 or min(r, k0, pos) < 0 or max(r + n, 0 if src else k0 + pos + n) > rows:
+            raise ValueError(f"a sequence of {n} rows from {r} at position {pos} does not fit blocks of {QBLOCK} in {rows} rows")
+    out = np.array([(r + b, k0, pos + b, src) for r, n, k0, pos, src in seqs for b in range(0, n, QBLOCK)], np.int32)
+    return out[np.argsort(-out[:, 2], kind="stable")]
+
+
 def ref_attention_chunk(q, k, v, heads, kv_heads, head_dim=128, scale=None):
     """fp32 reference of :func:`attention_chunk` (bottom-right causal)."""
     S, Sk = q.shape[0], k.shape[0]

@@ -300,6 +300,7 @@ class ServingModel:
         h, hd = c.hidden, c.head_dim
         if self.prefill_f8 is not None:
             return self._prefill_fp8(tokens, positions, slots, seq_starts, seq_lens, padded_lens)
+        last, items = self._prefill_rows(tokens.numel(), tokens.device, seq_starts, seq_lens, padded_lens)
         x = self.embed[tokens.long()].reshape(-1, h).contiguous()
         y = self._norm(x, None, self.ln1[0])
         T.op("prefill embed+norm")
@@ -308,7 +309,7 @@ class ServingModel:
             T.op(f"prefill L{i} qkv")
             self._rope_cache(qkv, i, positions, slots)
             T.op(f"prefill L{i} rope_cache")
-            a = self._prefill_attention(qkv, seq_starts, seq_lens, padded_lens)
+            a = self._prefill_attention(qkv, seq_starts, seq_lens, padded_lens, items)
             T.op(f"prefill L{i} attention")
             y = self._proj_add_norm(a, i, "o", x, self.ln2[i])
             T.op(f"prefill L{i} o+norm")
@@ -317,7 +318,6 @@ class ServingModel:
             nxt = self.ln1[i + 1] if i + 1 < c.layers else self.norm
             y = self._proj_add_norm(act, i, "down", x, nxt)
             T.op(f"prefill L{i} down+norm")
-        last = torch.as_tensor([int(s) + int(n) - 1 for s, n in zip(seq_starts, seq_lens)], device=y.device)
         yl = y[last].contiguous()
         out = self._proj(yl, None, "lm", True)
         T.op("prefill lm_head")
@@ -330,6 +330,7 @@ class ServingModel:
         from kgs.ops.transformer import add_rmsnorm, add_rmsnorm_fp8, quantize_rows_fp8, silu_mul_fp8
 
         c = self.cfg
+        last, items = self._prefill_rows(tokens.numel(), tokens.device, seq_starts, seq_lens, padded_lens)
         x = self.embed[tokens.long()].reshape(-1, c.hidden).contiguous()
         y8, ys = add_rmsnorm_fp8(x, None, self.ln1[0], c.eps)
         y = None
@@ -337,7 +338,7 @@ class ServingModel:
             F = self.prefill_f8[i]
             qkv = F["qkv"].forward_q(y8, ys)
             self._rope_cache(qkv, i, positions, slots)
-            a8, as_ = quantize_rows_fp8(self._prefill_attention(qkv, seq_starts, seq_lens, padded_lens))
+            a8, as_ = quantize_rows_fp8(self._prefill_attention(qkv, seq_starts, seq_lens, padded_lens, items))
             y8, ys = add_rmsnorm_fp8(x, F["o"].forward_q(a8, as_), self.ln2[i], c.eps)
             m8, ms = silu_mul_fp8(F["gate_up"].forward_q(y8, ys))
             d = F["down"].forward_q(m8, ms)
@@ -345,13 +346,47 @@ class ServingModel:
                 y8, ys = add_rmsnorm_fp8(x, d, self.ln1[i + 1], c.eps)
             else:
                 y = add_rmsnorm(x, d, self.norm, c.eps)
-        last = torch.as_tensor([int(s) + int(n) - 1 for s, n in zip(seq_starts, seq_lens)], device=y.device)
         return self._proj(y[last].contiguous(), None, "lm", True)
 
-    def _prefill_attention(self, qkv, seq_starts, seq_lens, padded_lens):
+    def _prefill_rows(self, tokens, device, seq_starts, seq_lens, padded_lens):
+        """The row of every sequence's last real token, and the attention items of prompts of
+        unequal padded lengths (None for equal ones), from one copy to the device."""
+        last = [int(s) + int(n) - 1 for s, n in zip(seq_starts, seq_lens)]
+        items = None
+        if self.backend != "ref" and len(set(int(p) for p in padded_lens)) > 1:
+            from kgs.ops.transformer import block_items
+
+            items = block_items([(int(s), int(p), int(s), 0, 0) for s, p in zip(seq_starts, padded_lens)], tokens)
+        return self._step_rows(device, last, items)
+
+    @staticmethod
+    def _step_rows(device, rows, items):
+        """Row numbers (int64) and int32 ``[n, 4]`` items (or None) on the device, in one copy."""
+        import numpy as np
+
+        flat = np.asarray(rows, np.int32)
+        if items is not None:
+            flat = np.concatenate([items.reshape(-1), flat])
+        t = torch.from_numpy(flat)
+        if device.type == "cuda":
+            t = t.pin_memory().to(device, non_blocking=True)
+        n = 0 if items is None else items.size
+        return t[n:].long(), None if items is None else t[:n].view(-1, 4)
+
+    def _kv(self, qkv):
+        """The key and the value columns of fused QKV rows."""
+        c = self.cfg
+        q, n = c.heads * c.head_dim, c.kv_heads * c.head_dim
+        return qkv[:, q:q + n], qkv[:, q + n:q + 2 * n]
+
+    def _prefill_attention(self, qkv, seq_starts, seq_lens, padded_lens, items=None):
         c = self.cfg
         hd = c.head_dim
         out = torch.empty((qkv.shape[0], c.heads * hd), dtype=torch.bfloat16, device=qkv.device)
+        if items is not None:  # unequal prompts: one launch over all their query blocks
+            from kgs.ops.transformer import attention_blocks
+
+            return attention_blocks(qkv, *self._kv(qkv), items, c.heads, c.kv_heads, out)
         if self.backend != "ref" and len(set(int(p) for p in padded_lens)) == 1:
             # equal padded lengths, packed back to back: one batched launch
             from kgs.ops.transformer import attention_qkv
@@ -393,6 +428,19 @@ class ServingModel:
         x = self.embed[tokens.long()].reshape(-1, c.hidden).contiguous()
         n_pf = sum(ch[2] for ch in chunks)
         nd = x.shape[0] - n_pf
+        rows = [row0 + n - 1 for row0, n, _, _, _, last in chunks if last] + list(range(n_pf, n_pf + nd))
+        items, past = None, []  # attention items of all chunks; those over a cached context
+        if self.backend != "ref" and chunks:
+            from kgs.ops.transformer import attention_blocks, block_items
+
+            seqs, k0 = [], 0
+            for row0, n, p, ctx0, pages, _ in chunks:
+                seqs.append((row0, p, k0 if ctx0 else row0, ctx0, int(ctx0 > 0)))
+                if ctx0:
+                    past.append((k0, k0 + ctx0 + p, ctx0 + n, pages))
+                    k0 += ctx0 + p
+            items = block_items(seqs, x.shape[0])
+        rows, items = self._step_rows(x.device, rows, items)
         f8 = self.prefill_f8 is not None and n_pf > 0  # W8A8 projections for the whole mixed step
         if f8:
             from kgs.ops.transformer import add_rmsnorm_fp8, quantize_rows_fp8, silu_mul_fp8
@@ -404,23 +452,18 @@ class ServingModel:
             qkv = self.prefill_f8[i]["qkv"].forward_q(y8, ys) if f8 else self._proj(y, i, "qkv", False)
             self._rope_cache(qkv, i, positions, slots)
             a = torch.empty((x.shape[0], c.heads * hd), dtype=torch.bfloat16, device=x.device)
-            j = 0
-            while j < len(chunks):
-                row0, n, p, ctx0, pages, _ = chunks[j]
-                # first chunks (no cached context) of equal padded length sit back to
-                # back: one batched flash-attention launch for the run
-                k = j + 1
-                if ctx0 == 0 and self.backend != "ref":
-                    while k < len(chunks) and chunks[k][3] == 0 and chunks[k][2] == p:
-                        k += 1
-                if k - j > 1:
-                    from kgs.ops.transformer import attention_qkv
-
-                    attention_qkv(qkv[row0:row0 + p * (k - j)], k - j, p, c.heads, c.kv_heads, head_dim=hd,
-                                  causal=True, out=a[row0:row0 + p * (k - j)])
-                else:
+            if items is not None:
+                # every chunk in one launch: keys of first chunks are their own rows, those of later
+                # ones the cached rows (this step's were just written there), gathered
+                k2 = v2 = None
+                if past:
+                    k2, v2 = torch.empty((2, past[-1][1], c.kv_heads * hd), dtype=torch.bfloat16, device=x.device)
+                    for r0, r1, ctx, pages in past:
+                        D.gather_kv_into(self.cache.layer(i), pages, ctx, k2[r0:r1], v2[r0:r1])
+                attention_blocks(qkv, *self._kv(qkv), items, c.heads, c.kv_heads, a, k2, v2)
+            else:
+                for row0, n, p, ctx0, pages, _ in chunks:
                     a[row0:row0 + p] = self._chunk_attention(qkv[row0:row0 + p], i, n, p, ctx0, pages)
-                j = k
             if nd:
                 qd = qkv[n_pf:]
                 if self.backend == "ref":
@@ -444,37 +487,26 @@ class ServingModel:
             y = self._proj_add_norm(a, i, "o", x, self.ln2[i])
             act = self._gate_up_act(y, i)
             y = self._proj_add_norm(act, i, "down", x, nxt)
-        rows = [row0 + n - 1 for row0, n, _, _, _, last in chunks if last] + list(range(n_pf, n_pf + nd))
-        if not rows:
+        if rows.numel() == 0:
             return torch.empty((0, c.vocab), dtype=torch.bfloat16, device=x.device)
-        yl = y[torch.as_tensor(rows, device=y.device)].contiguous()
+        yl = y[rows].contiguous()
         return self._proj(yl, None, "lm", True)
 
     def _chunk_attention(self, blk, layer, n, p, ctx0, pages):
-        """Causal attention of one prompt chunk (rows = positions ctx0 .. ctx0+p-1,
-        n real) over everything cached before it plus itself; padded rows out 0."""
+        """The plain backend's causal attention of one prompt chunk (rows = positions ctx0 ..
+        ctx0+p-1, n real) over everything cached before it plus itself; padded rows out 0."""
         c = self.cfg
         hd = c.head_dim
         if ctx0 == 0:  # first chunk: the whole-prompt path
-            out = torch.empty((p, c.heads * hd), dtype=torch.bfloat16, device=blk.device)
-            if self.backend == "ref":
-                return self._prefill_attention(blk, [0], [n], [p])
-            from kgs.ops.transformer import attention_qkv
+            return self._prefill_attention(blk, [0], [n], [p])
+        from kgs.ops.transformer import ref_attention_chunk
 
-            return attention_qkv(blk, 1, p, c.heads, c.kv_heads, head_dim=hd, causal=True, out=out)
         # keys/values of positions 0 .. ctx0+n-1 (this chunk's rows were just
-        # written to the cache by rope_cache), zero-padded to ctx0 + p rows
-        if self.backend == "ref":
-            from kgs.ops.transformer import ref_attention_chunk
-
-            k, v = D.gather_kv(self.cache.layer(layer), pages, ctx0 + n)
-            o = torch.zeros((p, c.heads * hd), dtype=torch.bfloat16, device=blk.device)
-            o[:n] = ref_attention_chunk(blk[:n], k, v, c.heads, c.kv_heads, hd).to(torch.bfloat16)
-            return o
-        from kgs.ops.transformer import attention_chunk
-
-        k, v = D.gather_kv(self.cache.layer(layer), pages, ctx0 + n, rows=ctx0 + p)
-        return attention_chunk(blk, k, v, c.heads, c.kv_heads, hd)
+        # written to the cache by rope_cache)
+        k, v = D.gather_kv(self.cache.layer(layer), pages, ctx0 + n)
+        o = torch.zeros((p, c.heads * hd), dtype=torch.bfloat16, device=blk.device)
+        o[:n] = ref_attention_chunk(blk[:n], k, v, c.heads, c.kv_heads, hd).to(torch.bfloat16)
+        return o
 
     # ----------------------------------------------------------------- decode
     @torch.no_grad()

@@ -68,7 +68,23 @@ struct Args {
   const int* pos;
   int npos, rot;
   int win;  // a row sees itself and the win - 1 keys before it; 0: all
+  // blocks form: the keys and values of items that bring their own (a chunk's cached context)
+  const unsigned short* k2;
+  const unsigned short* v2;
+  long ld2;
 };
+
+// EQUAL: B equal sequences of S rows, a multiple of QB. RAGGED: any number of query rows per
+// sequence at any position (Args::items), rows and keys past a block's end clamped on load and
+// dropped on store; always causal. BLOCKS: whole blocks of QB rows of sequences of any lengths in
+// one launch, causal, with grouped key heads; one int4 per block -- first query row, first key row
+// of its sequence, position of the first query row (a multiple of KB), and 1 where the keys are
+// rows of k2 / v2. One launch because one per sequence leaves the chip to each sequence's own tail:
+// prompts of a few hundred tokens at 32 heads have fewer workgroups each than the 512 that are
+// resident. A whole prompt step of 16 unequal prompts of about 512 tokens (H 4096) went from 13.76
+// to 12.85 ms; a step of 2048 prompt rows, one chunk of them at 3072 cached tokens, with 40
+// decode rows from 3.90 to 3.60, of it the keys' gather in one launch about half.
+enum Mode { EQUAL = 0, RAGGED_ROWS = 1, BLOCKS = 2 };
 
 // XOR image of a row's 16-B chunks (HD / 8 of them)
 template <int HD>
@@ -82,11 +98,9 @@ __device__ __forceinline__ int off(int r, int c) { return 2 * HD * r + 16 * (c ^
 
 __device__ __forceinline__ bf16x8 pack8(const f32x16& s, int base) { return pack_bf16x8(s, base); }
 
-// RAGGED: any number of query rows per sequence at any position (Args::items),
-// rows and keys past a block's end clamped on load and dropped on store; always
-// causal. Otherwise B equal sequences of S rows, a multiple of QB.
-template <int HD, bool RAGGED, int HR = 0>
+template <int HD, Mode MODE, int HR = 0>
 __global__ __launch_bounds__(256, 2) __attribute__((amdgpu_waves_per_eu(2, 2))) void fwd(Args a) {
+  constexpr bool RAGGED = MODE == RAGGED_ROWS;
   constexpr int TILE_BYTES = KB * HD * 2;  // 16 KB at 128
   constexpr int ND = HD / 32, NK = HD / 16, NR = HR / 16, ROT_BYTES = KB * HR * 2;
   __shared__ __attribute__((aligned(16))) char smem[2][2 * TILE_BYTES + ROT_BYTES];  // [buf]: K, V, rotated K
@@ -94,9 +108,33 @@ __global__ __launch_bounds__(256, 2) __attribute__((amdgpu_waves_per_eu(2, 2))) 
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l32 = lane & 31, hh = lane >> 5;
   int h, kvh, q0, qw, qrow, qoff, nval = QB;
-  long tok0, ktok0;
+  long tok0, ktok0, ldk = a.ldk, ldv = a.ldv;
+  const unsigned short *kp = a.k, *vp = a.v;
   bool causal = true;
-  if constexpr (RAGGED) {
+  // XCD-aware order: 8 consecutive dispatch slots of one XCD take 4 heads of
+  // one KV group; work ids stay heaviest-first in dispatch time.
+  int lid = blockIdx.x;
+  if (!RAGGED && (gridDim.x & 31) == 0) {
+    const int t = lid >> 3, x = lid & 7;
+    lid = ((t >> 2) << 5) | (x << 2) | (t & 3);
+  }
+  if constexpr (MODE == BLOCKS) {
+    const int item = lid / a.H;
+    h = lid - item * a.H;
+    kvh = h / (a.H / a.HKV);
+    const int4 it = a.items[item];
+    tok0 = it.x;
+    ktok0 = it.y;
+    qoff = it.z;
+    if (it.w) {
+      kp = a.k2;
+      vp = a.v2;
+      ldk = ldv = a.ld2;
+    }
+    q0 = 0;
+    qw = 32 * w;
+    qrow = qw + l32;
+  } else if constexpr (RAGGED) {
     const int item = blockIdx.x / a.H;
     h = kvh = blockIdx.x - item * a.H;
     const int4 it = a.items[item];
@@ -109,14 +147,6 @@ __global__ __launch_bounds__(256, 2) __attribute__((amdgpu_waves_per_eu(2, 2))) 
     qrow = qw + l32;
   } else {
     const int nqb = a.S / QB;
-    const int nwg = gridDim.x;
-    // XCD-aware order: 8 consecutive dispatch slots of one XCD take 4 heads of
-    // one KV group; work ids stay heaviest-first in dispatch time.
-    int lid = blockIdx.x;
-    if ((nwg & 31) == 0) {
-      const int t = lid >> 3, x = lid & 7;
-      lid = ((t >> 2) << 5) | (x << 2) | (t & 3);
-    }
     const int per = a.B * a.H;
     const int qi = lid / per, rem = lid - qi * per;
     const int qb = a.causal ? nqb - 1 - qi : qi;
@@ -157,8 +187,8 @@ __global__ __launch_bounds__(256, 2) __attribute__((amdgpu_waves_per_eu(2, 2))) 
     }
   }
 
-  const unsigned short* kbase = a.k + ktok0 * a.ldk + (long)kvh * HD;
-  const unsigned short* vbase = a.v + ktok0 * a.ldv + (long)kvh * HD;
+  const unsigned short* kbase = kp + ktok0 * ldk + (long)kvh * HD;
+  const unsigned short* vbase = vp + ktok0 * ldv + (long)kvh * HD;
   const unsigned short* rbase = a.kr + ktok0 * a.ldr;
   // K/V tile jn -> LDS buffer sb by LDS-DMA (global_load_lds, no staging
   // registers): a 16 KB tile is 16 chunks of 1 KB = 4 rows of 256 B; wave w
@@ -173,8 +203,8 @@ __global__ __launch_bounds__(256, 2) __attribute__((amdgpu_waves_per_eu(2, 2))) 
       const int r = (512 / HD) * ch + lane / (HD / 8), c = (lane & (HD / 8 - 1)) ^ swz<HD>(r);
       long row = (long)jn * KB + r;
       if constexpr (RAGGED) row = min(row, (long)(qoff + nval - 1));
-      glds16(kbase + row * a.ldk + 8 * c, smem[sb] + 1024 * ch);
-      glds16(vbase + row * a.ldv + 8 * c, smem[sb] + TILE_BYTES + 1024 * ch);
+      glds16(kbase + row * ldk + 8 * c, smem[sb] + 1024 * ch);
+      glds16(vbase + row * ldv + 8 * c, smem[sb] + TILE_BYTES + 1024 * ch);
     }
     if constexpr (HR > 0) {
 #pragma unroll
@@ -374,8 +404,8 @@ KGS_EXPORT int kgs_attn_fwd_bf16_ex(const void* q, const void* k, const void* v,
   if (nwg > 0x7fffffff) return KGS_ERR_SHAPE;
   Args a{(const unsigned short*)q, (const unsigned short*)k, (const unsigned short*)v, (unsigned short*)o,
          ldq, ldk, ldv, ldo, B, S, H, HKV, scale * 1.4426950408889634f, causal ? 1 : 0, Sk, Sk - S,
-         nullptr, nullptr, 0, 0, 0, nullptr, 0, nullptr, nullptr, 0, 0, 0};
-  hipLaunchKernelGGL((fwd<HD, false>), dim3((unsigned)nwg), dim3(256), 0, s, a);
+         nullptr, nullptr, 0, 0, 0, nullptr, 0, nullptr, nullptr, 0, 0, 0, nullptr, nullptr, 0};
+  hipLaunchKernelGGL((fwd<HD, EQUAL>), dim3((unsigned)nwg), dim3(256), 0, s, a);
   return (int)hipGetLastError();
 }
 
@@ -410,10 +440,32 @@ KGS_EXPORT int kgs_attn_fwd_ragged_bf16(const void* q, const void* k, const void
   Args a{(const unsigned short*)q, (const unsigned short*)k, (const unsigned short*)v, (unsigned short*)o,
          ldq, ldk, ldv, ldo, 0, 0, H, H, scale * 1.4426950408889634f, 1, 0, 0,
          (const int4*)items, (const unsigned short*)gate, ldg, hg, eg,
-         (const unsigned short*)kr, ldr, (const float*)cs, (const int*)pos, npos, rot, win};
+         (const unsigned short*)kr, ldr, (const float*)cs, (const int*)pos, npos, rot, win, nullptr, nullptr, 0};
   const dim3 grid((unsigned)(nitems * H));
-  auto fn = hd == 128 ? (hr == 0 ? fwd<128, true> : hr == 32 ? fwd<128, true, 32> : fwd<128, true, 64>)
-                      : (hr == 0 ? fwd<64, true> : hr == 32 ? fwd<64, true, 32> : fwd<64, true, 64>);
+  auto fn = hd == 128 ? (hr == 0 ? fwd<128, RAGGED_ROWS> : hr == 32 ? fwd<128, RAGGED_ROWS, 32> : fwd<128, RAGGED_ROWS, 64>)
+                      : (hr == 0 ? fwd<64, RAGGED_ROWS> : hr == 32 ? fwd<64, RAGGED_ROWS, 32> : fwd<64, RAGGED_ROWS, 64>);
   hipLaunchKernelGGL(fn, grid, dim3(256), 0, s, a);
+  return (int)hipGetLastError();
+}
+
+// Causal attention of sequences of any lengths in whole blocks of 128 query rows, head_dim 128,
+// grouped key heads, one launch. items: nitems int4 (first query row, first key row of its
+// sequence, position of the first query row among these, 0: keys in k / v, 1: in k2 / v2), any
+// order (heaviest first keeps the tail short). Every item reads its position + 128 keys.
+KGS_EXPORT int kgs_attn_fwd_blocks_bf16(const void* q, const void* k, const void* v, const void* k2, const void* v2, void* o,
+                                       const void* items, int nitems, int H, int HKV, int hd, long ldq, long ldk,
+                                       long ldv, long ld2, long ldo, float scale, hipStream_t s) {
+  using namespace kgs::attn;
+  if (nitems <= 0 || H <= 0 || HKV <= 0 || H % HKV || hd != 128) return KGS_ERR_SHAPE;
+  const long w = (long)HKV * hd;
+  if (ldq < (long)H * hd || ldk < w || ldv < w || ldo < (long)H * hd || (k2 && ld2 < w)) return KGS_ERR_SHAPE;
+  const uintptr_t al = (uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)o | (uintptr_t)items | (uintptr_t)k2 | (uintptr_t)v2;
+  if ((al & 15) || (ldq | ldk | ldv | ldo | ld2) & 7) return KGS_ERR_ALIGN;
+  if ((long)nitems * H > 0x7fffffff) return KGS_ERR_SHAPE;
+  Args a{(const unsigned short*)q, (const unsigned short*)k, (const unsigned short*)v, (unsigned short*)o,
+         ldq, ldk, ldv, ldo, 0, 0, H, HKV, scale * 1.4426950408889634f, 1, 0, 0,
+         (const int4*)items, nullptr, 0, 0, 0, nullptr, 0, nullptr, nullptr, 0, 0, 0,
+         (const unsigned short*)k2, (const unsigned short*)v2, ld2};
+  hipLaunchKernelGGL((fwd<128, BLOCKS>), dim3((unsigned)(nitems * H)), dim3(256), 0, s, a);
   return (int)hipGetLastError();
 }

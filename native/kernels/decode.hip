@@ -736,6 +736,53 @@ __global__ __launch_bounds__(256) void v_cache_pages(const unsigned short* __res
   }
 }
 
+// The first `ctx` cached tokens of a sequence as row-major K and V, [rows, HKV * 128] each, rows from
+// ctx on zero: the keys a prompt chunk attends to. A workgroup per (page, KV head): both regions go
+// through LDS as they lie, so that the rows leave as 256-byte runs. Bound by memory: 16384 tokens
+// of 8 heads (67 MB read, as much written) take 24 us, 5.5 TB/s, against 176 for the same gather
+// by tensor operations (an index, transpose, zero padding and conversion pass each); 4096
+// tokens, where the launch is most of it, 9 against 70.
+template <bool KV8>
+__global__ __launch_bounds__(256) void gather_kv(const void* __restrict__ cache, const int* __restrict__ pages,
+                                                 unsigned short* __restrict__ ko, unsigned short* __restrict__ vo, int ctx,
+                                                 int rows, int HKV, int npages, long ld) {
+  __shared__ __attribute__((aligned(16))) unsigned short sk[PAGE_ELEMS], sv[PAGE_ELEMS];
+  const int t0 = blockIdx.x * PAGE, kvh = blockIdx.y, tid = threadIdx.x;
+  int valid = ctx - t0;  // tokens of this page
+  const int pg = valid > 0 ? pages[blockIdx.x] : 0;
+  if ((unsigned)pg >= (unsigned)npages) valid = 0;
+  if (valid > 0) {
+    const long region = ((long)pg * HKV + kvh) * 2 * PAGE_ELEMS;
+#pragma unroll
+    for (int i = tid * 8; i < PAGE_ELEMS; i += 256 * 8) {
+      if constexpr (KV8) {
+        const unsigned char* p = (const unsigned char*)cache + region + i;
+        *(bf16x8*)&sk[i] = dequant8(*(const u32x2*)p, 1.f);
+        *(bf16x8*)&sv[i] = dequant8(*(const u32x2*)(p + PAGE_ELEMS), 1.f);
+      } else {
+        const unsigned short* p = (const unsigned short*)cache + region + i;
+        *(bf16x8*)&sk[i] = *(const bf16x8*)p;
+        *(bf16x8*)&sv[i] = *(const bf16x8*)(p + PAGE_ELEMS);
+      }
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = tid; i < PAGE_ELEMS / 8; i += 256) {
+    const int tau = i >> 4, d = (i & 15) * 8;
+    if (t0 + tau >= rows) continue;
+    bf16x8 k = {0, 0, 0, 0, 0, 0, 0, 0}, v = k;
+    if (tau < valid) {
+      k = *(const bf16x8*)&sk[kv_k_index(tau, d)];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = (short)sv[kv_v_index(tau, d + e)];
+    }
+    const long at = (long)(t0 + tau) * ld + kvh * HD + d;
+    *(bf16x8*)(ko + at) = k;
+    *(bf16x8*)(vo + at) = v;
+  }
+}
+
 // ---------------------------------------------------------------------------
 // paged decode attention
 // ---------------------------------------------------------------------------
@@ -1631,6 +1678,21 @@ KGS_EXPORT int kgs_paged_decode_wg(const void* q, const void* cache, const int* 
              nullptr, 0, nullptr, nullptr, nullptr, nullptr, nullptr};
   if (kv8) hipLaunchKernelGGL(paged_wg<true>, dim3((unsigned)nwg), dim3(256), 0, s, a);
   else hipLaunchKernelGGL(paged_wg<false>, dim3((unsigned)nwg), dim3(512), 0, s, a);
+  return (int)hipGetLastError();
+}
+
+// Rows 0 .. rows - 1 of a sequence's cached keys and values, row-major with rows ld apart (16-B
+// aligned): the first ctx from its pages (int32, at least ceil(ctx / 32) of them), the others zero.
+KGS_EXPORT int kgs_gather_kv(const void* cache, const int* pages, void* k, void* v, int ctx, int rows, int HKV, int hd, int npages,
+                             long ld, int kv8, hipStream_t s) {
+  using namespace kgs::dec;
+  if (ctx < 0 || rows < ctx || rows <= 0 || npages <= 0 || HKV <= 0 || HKV > 65535 || hd != HD || ld < (long)HKV * HD) return KGS_ERR_SHAPE;
+  if (!al16(cache) || !al16(k) || !al16(v) || ld % 8) return KGS_ERR_ALIGN;
+  const dim3 grid((unsigned)((rows + PAGE - 1) / PAGE), (unsigned)HKV);
+  auto ko = (unsigned short*)k;
+  auto vo = (unsigned short*)v;
+  if (kv8) hipLaunchKernelGGL(gather_kv<true>, grid, dim3(256), 0, s, cache, pages, ko, vo, ctx, rows, HKV, npages, ld);
+  else hipLaunchKernelGGL(gather_kv<false>, grid, dim3(256), 0, s, cache, pages, ko, vo, ctx, rows, HKV, npages, ld);
   return (int)hipGetLastError();
 }
 

@@ -256,6 +256,38 @@ def w4x_route(m: int, n: int, k: int):
     return W4X_TUNED.get((b, n, k))
 
 
+W4X_RULE_MIN = 33   # rows: skinny GEMM below
+W4X_RULE_MAX = 256
+
+
+def w4x_rule(m: int, n: int, k: int, most: int = 16, cus: int = CUS):
+    """The route (as :func:`w4x_route`) for 33 to 256 rows of a size without measured entries, or None.
+    ``most``: slices that the caller can take.
+
+    128x128 tiles in as many K slices (of at least 256) as fit one workgroup on every CU: a
+    second round of workgroups costs more than finer slices give, wider tiles leave
+    CUs idle. Tiles of 256 rows only where 128-row ones alone are more than the CUs. us at 100
+    rows, weights from HBM, next to the library's product: 3072x2048 8.5 / 12.4 (with 4 slices
+    9.5, with 16 12.8), 2048x2048 7.4 / 11.2, 16384x2048 17.7 / 21.0 (unsplit 24.4), 2048x8192 12.6 /
+    21.2 (8 slices 15.2), 32000x2048 30.5 / 33.1; at 256 rows 2048x8192 18.0 / 27.2, 16384x2048 25.6 /
+    30.1. The slices' sum is left to the norm, rotation or gate that follows; a launch of its own for
+    it costs 3 to 6 us more, and 16 slices there more than they give (``most`` = 8). None where the tiles are more
+    than the CUs, or a K like 11008 that slices badly leaves half of the CUs idle."""
+    if not W4X_RULE_MIN <= m <= W4X_RULE_MAX or n % 128 or k % 128 or (n, k) in _MEASURED:
+        return None
+    bm = 128 if -(-m // 128) * (n // 128) <= cus else 256
+    tiles = -(-m // bm) * (n // 128)
+    ns = 1
+    while 2 * ns <= most and 2 * ns * tiles <= cus and k % (256 * ns) == 0 and k >= 512 * ns:
+        ns *= 2
+    if tiles > cus or (2 * ns * tiles < cus and k >= 512 * ns and 2 * ns <= most):
+        return None
+    return 128, ns, bm
+
+
+_MEASURED = {key[1:] for key in (*W4X_TUNED, *SPLITK_TUNED)}
+
+
 def w4x_stages(route) -> int:
     """LDS stages of a W4X_TUNED route (2 unless the entry names 3 or 4)."""
     return route[3] if len(route) > 3 else 2

@@ -202,9 +202,24 @@ def _packed_operand(b, bn, swiglu):
     return b.data, b.shape, b.shape[1], 1
 
 
+def _partials(op: str, device, need: int, private: bool) -> torch.Tensor:
+    """fp32 room for a split product's partials: a buffer of the call's own (calls on several
+    streams), or the per-GPU workspace."""
+    if private:
+        return torch.empty(need, dtype=torch.float32, device=device)
+    from .decode import device_key
+
+    ws = _SPLITK_WS.get(device_key(device))
+    if ws is None or ws.numel() < need:
+        if torch.cuda.is_current_stream_capturing():
+            raise RuntimeError(f"{op}: reserve_splitk_workspace() before hipGraph capture")
+        ws = reserve_splitk_workspace(device, need)
+    return ws
+
+
 def gemm_nt_w4x(a: torch.Tensor, b, bn: int = 256, nslice: int = 1,
                 out: torch.Tensor | None = None, bm: int = 256, stages: int = 2,
-                nt_weights: bool = False) -> torch.Tensor:
+                nt_weights: bool = False, private: bool = False) -> torch.Tensor:
     """``a @ b.T`` on the four-wave kernel with ``bm`` x ``bn`` tiles (256 or 128
     each), any M (rows past M read as zeros), over ``nslice`` K-slices (fp32
     partials + reduce when > 1): the decode-batch GEMM path.
@@ -212,7 +227,8 @@ def gemm_nt_w4x(a: torch.Tensor, b, bn: int = 256, nslice: int = 1,
     or a :class:`PanelWeight` packed with the same ``bn``. ``stages``: LDS
     stages (3 / 4 keep more K-tiles in flight; only where they fit in 160 KiB).
     ``nt_weights``: ``b``'s loads non-temporal (decode weights each CU streams
-    once), ``a``'s loads default (two stages only)."""
+    once), ``a``'s loads default (two stages only). ``private``: partials in a buffer of
+    this call's own instead of the per-GPU workspace."""
     _check_operand(a, "a")
     b, bshape, ldb, packed = _packed_operand(b, bn, False)
     if not packed:
@@ -223,18 +239,8 @@ def gemm_nt_w4x(a: torch.Tensor, b, bn: int = 256, nslice: int = 1,
         raise ValueError(f"inner dims differ: a {tuple(a.shape)} b {tuple(bshape)}")
     if out is None:
         out = torch.empty((M, N), dtype=torch.bfloat16, device=a.device)
-    ws_ptr = None
-    if nslice > 1:
-        from .decode import device_key
-
-        need = nslice * M * N
-        ws = _SPLITK_WS.get(device_key(a.device))
-        if ws is None or ws.numel() < need:
-            if torch.cuda.is_current_stream_capturing():
-                raise RuntimeError("gemm_nt_w4x: reserve_splitk_workspace() before hipGraph capture")
-            ws = reserve_splitk_workspace(a.device, need)
-        ws_ptr = ws.data_ptr()
-    rc = _lib.lib().kgs_gemm_bf16_nt_w4x_ex(a.data_ptr(), b.data_ptr(), out.data_ptr(), ws_ptr, M, N, K, a.stride(0),
+    ws = _partials("gemm_nt_w4x", a.device, nslice * M * N, private) if nslice > 1 else None
+    rc = _lib.lib().kgs_gemm_bf16_nt_w4x_ex(a.data_ptr(), b.data_ptr(), out.data_ptr(), None if ws is None else ws.data_ptr(), M, N, K, a.stride(0),
                                             ldb, out.stride(0), int(bn), int(nslice), int(bm),
                                             _w4x_flags(packed, stages, nt_weights), _lib.stream_handle(a.device))
     _lib.check(rc, f"gemm_nt_w4x[{M}x{N}x{K} {bm}x{bn}/{nslice}]")
@@ -295,10 +301,10 @@ def add_product_(a: torch.Tensor, b: torch.Tensor, c: torch.Tensor) -> bool:
 
 
 def gemm_nt_w4x_partials(a: torch.Tensor, b, bn: int, nslice: int, bm: int = 256, stages: int = 2,
-                         nt_weights: bool = False) -> torch.Tensor:
+                         nt_weights: bool = False, private: bool = False) -> torch.Tensor:
     """The split-K four-wave GEMM WITHOUT its reduce: returns the fp32 partial
     products ``[nslice, M, N]`` (a view of the per-GPU split-K workspace, valid
-    until the next split-K call on the stream) for a fused consumer --
+    until the next split-K call on the stream, or with ``private`` a tensor of its own) for a fused consumer --
     ``kgs.ops.transformer.splitk_add_rmsnorm`` or ``kgs.ops.decode.rope_cache_``."""
     if nslice < 2:
         raise ValueError("partials need nslice >= 2")
@@ -310,14 +316,8 @@ def gemm_nt_w4x_partials(a: torch.Tensor, b, bn: int, nslice: int, bm: int = 256
     N, K2 = bshape
     if K != K2:
         raise ValueError(f"inner dims differ: a {tuple(a.shape)} b {tuple(bshape)}")
-    from .decode import device_key
-
     need = nslice * M * N
-    ws = _SPLITK_WS.get(device_key(a.device))
-    if ws is None or ws.numel() < need:
-        if torch.cuda.is_current_stream_capturing():
-            raise RuntimeError("gemm_nt_w4x_partials: reserve_splitk_workspace() before hipGraph capture")
-        ws = reserve_splitk_workspace(a.device, need)
+    ws = _partials("gemm_nt_w4x_partials", a.device, need, private)
     rc = _lib.lib().kgs_gemm_bf16_nt_w4x_ex(a.data_ptr(), b.data_ptr(), None, ws.data_ptr(), M, N, K, a.stride(0),
                                             ldb, N, int(bn), int(nslice), int(bm),
                                             _w4x_flags(packed, stages, nt_weights),
@@ -359,12 +359,13 @@ def gemm_nt_w4x_swiglu(a: torch.Tensor, w_gate_up, bn: int = 128,
 
 
 def gemm_nt_w4x_splitk_swiglu(a: torch.Tensor, w_gate_up: torch.Tensor, bn: int = 256, nslice: int = 2,
-                              bm: int = 256, out: torch.Tensor | None = None) -> torch.Tensor:
+                              bm: int = 256, out: torch.Tensor | None = None, nt_weights: bool = False,
+                              private: bool = False) -> torch.Tensor:
     """SwiGLU over a fused gate|up weight as a split-K GEMM (fp32 partials in the
     split-K workspace) + one reduce-and-SwiGLU pass: returns ``[M, I]`` with the
     roundings of ``gemm_nt`` + ``silu_mul``. For decode batches where the
     epilogue-fused kernel (:func:`gemm_nt_w4x_swiglu`) leaves CUs idle."""
-    parts = gemm_nt_w4x_partials(a, w_gate_up, bn=bn, nslice=nslice, bm=bm)
+    parts = gemm_nt_w4x_partials(a, w_gate_up, bn=bn, nslice=nslice, bm=bm, nt_weights=nt_weights, private=private)
     M, N = a.shape[0], w_gate_up.shape[0]
     if out is None:
         out = torch.empty((M, N // 2), dtype=torch.bfloat16, device=a.device)

@@ -17,22 +17,7 @@ from . import decode as D
 from .activation import Gate
 
 SKINNY_MAX_ROWS = 32   # untuned shapes: skinny GEMM up to here
-SPLIT_MAX_ROWS = 512   # four-wave split-K tiles up to here
-TARGET_TILES = 400     # workgroups that fill the CUs about one and a half times
-MAX_PARTIALS = 16 << 20  # fp32 partial products of a split-K call
-
-
-def split_tiles(m: int, n: int, k: int) -> tuple[int, int, int] | None:
-    """(tile width, K slices, tile height) of the four-wave GEMM for ``m`` rows, or
-    None when the shape does not tile."""
-    if n % 128 or k % 128:
-        return None
-    bm = 128 if m <= 128 else 256
-    tiles = n // 128 * -(-m // bm)
-    ns = 1
-    while ns < 8 and 2 * ns * tiles <= TARGET_TILES and k % (256 * ns) == 0 and 2 * ns * m * n <= MAX_PARTIALS:
-        ns *= 2
-    return 128, ns, bm
+SPLIT_MAX_SLICES = 8   # K slices whose sum is a launch of its own
 
 
 class Projection:
@@ -79,22 +64,27 @@ class Projection:
     def _gated(self, x, m):
         from .gemm import gemm_nt_w4x_swiglu, gemm_swiglu, swiglu_fused_ok
 
-        if m > SPLIT_MAX_ROWS:
+        if m > 512:
             return gemm_swiglu(x, self.w, self.gated)
         if not swiglu_fused_ok(x, self.w):
             return None
-        return gemm_nt_w4x_swiglu(x, self.w, bn=128, bm=128 if m <= 128 else 256, nt_weights=D.NT_WEIGHTS,
-                                  act=self.gated)
+        # up to 128 rows one tile high, each weight read once and non-temporal; above, the general
+        # kernel's tiles (us against 256-row ones here: 5120x2048 at 256 rows 22.4 / 28.1, at 512
+        # 22.7 / 28.2; 22016x4096 64.2 / 63.0 and 88.7 / 110.2)
+        if m > 128:
+            return gemm_swiglu(x, self.w, self.gated)
+        return gemm_nt_w4x_swiglu(x, self.w, bn=128, bm=128, nt_weights=D.NT_WEIGHTS, act=self.gated)
 
     def _plain(self, x, m, n, k):
         from .gemm import gemm_nt, gemm_nt_w4x
 
-        if m > SPLIT_MAX_ROWS:
+        if m > 512:
             return gemm_nt(x, self.w)
         if m < D.W4X_MIN_BATCH or x.stride(0) % 8 or x.data_ptr() % 16:
             return None
-        route = D.w4x_route(m, n, k) or split_tiles(m, n, k)
-        if route is None:
-            return gemm_nt(x, self.w) if m >= 128 else None
+        table = D.w4x_route(m, n, k)
+        route = table or D.w4x_rule(m, n, k, SPLIT_MAX_SLICES)
+        if route is None:  # us at 64 rows of 4096x11008, which slices badly: 27 here, 36 by the library
+            return gemm_nt(x, self.w) if m >= 128 or (n % 128 == 0 and k % 128 == 0) else None
         return gemm_nt_w4x(x, self.w, bn=route[0], nslice=route[1], bm=route[2], stages=D.w4x_stages(route),
-                           nt_weights=D.w4x_nt(route))
+                           nt_weights=D.w4x_nt(route), private=table is None)

@@ -16,8 +16,10 @@ Two step kinds, both driven by the native scheduler's plans
   :func:`kgs.ops.decode.skinny_gemm` launches over prepacked weights whose
   epilogues carry the RMSNorms (norm weights folded into the weights, row
   scales from sums of squares the residual-updating GEMMs accumulate), the
-  residual adds and SwiGLU -- no elementwise kernels. Larger batches use
-  add_rmsnorm/silu_mul and hipBLASLt, with the split-K 256x256 GEMM
+  residual adds and SwiGLU -- no elementwise kernels. Larger batches run
+  split-K four-wave tiles (:func:`kgs.ops.decode.w4x_route`, :func:`kgs.ops.decode.w4x_rule`)
+  whose partial sums go into the rotation, norm or gate that follows, and
+  otherwise add_rmsnorm/silu_mul and hipBLASLt, the split-K 256x256 GEMM
   (:func:`kgs.ops.decode.splitk_slices`), the skinny GEMM
   (:func:`kgs.ops.decode.use_skinny`) or the 256x256 GEMM (LM head) where
   those measured faster.
@@ -175,12 +177,13 @@ class ServingModel:
             return (x.float() @ w.float().T).to(torch.bfloat16)
         m = x.shape[0]
         if decode:
-            route = D.w4x_route(m, w.shape[0], w.shape[1])
+            table = D.w4x_route(m, w.shape[0], w.shape[1])
+            route = table or D.w4x_rule(m, w.shape[0], w.shape[1])
             if route is not None:
                 from kgs.ops.gemm import gemm_nt_w4x
 
                 return gemm_nt_w4x(x, w, bn=route[0], nslice=route[1], bm=route[2], stages=D.w4x_stages(route),
-                                   nt_weights=D.w4x_nt(route))
+                                   nt_weights=D.w4x_nt(route), private=table is None)
         if decode:
             ns = D.splitk_slices(m, w.shape[0], w.shape[1])
             if ns == 1:
@@ -209,7 +212,7 @@ class ServingModel:
         if not self.fuse_splitk:
             return None
         w = self.w[layer][name]
-        r = D.w4x_route(m, w.shape[0], w.shape[1])
+        r = D.w4x_route(m, w.shape[0], w.shape[1]) or D.w4x_rule(m, w.shape[0], w.shape[1])
         if r is None or r[1] < 2:
             return None
         if name in ("o", "down") and self.cfg.hidden % 2048:
@@ -233,13 +236,22 @@ class ServingModel:
         return self.w[layer]["gate_up"]
 
     def _swiglu_route(self, m: int):
-        """(bn, 1) when the decode gate|up projection runs unsplit on the
-        four-wave kernel: SwiGLU then goes into its epilogue."""
+        """The route when the decode gate|up projection runs on the four-wave kernel: unsplit,
+        SwiGLU goes into its epilogue, split (no measured entry is), into the slices' sum."""
         if not self.fuse_splitk:
             return None
         w = self.w[0]["gate_up"]
         r = D.w4x_route(m, w.shape[0], w.shape[1])
-        return r if r is not None and r[1] == 1 else None
+        return D.w4x_rule(m, w.shape[0], w.shape[1]) if r is None else r if r[1] == 1 else None
+
+    def _split_proj(self, x, layer: int, name: str, r):
+        """fp32 partial products of a decode projection along route ``r``; a size without measured
+        entries gets a buffer of the call's own."""
+        from kgs.ops.gemm import gemm_nt_w4x_partials
+
+        w = self.w[layer][name]
+        return gemm_nt_w4x_partials(x, self._w4x_weight(layer, name, r[0]), *r, nt_weights=D.w4x_nt(r),
+                                    private=D.w4x_route(x.shape[0], *w.shape) is None)
 
     def _norm(self, x, d, w):
         """x += d (in place, bf16) and return rmsnorm(x) * w."""
@@ -521,7 +533,7 @@ class ServingModel:
         rq, ro, rd = (self._splitk_route(m, 0, n) for n in ("qkv", "o", "down"))  # same shapes in every layer
         rg = self._swiglu_route(m)
         if rq or ro or rd or rg:
-            from kgs.ops.gemm import gemm_nt_w4x_partials, gemm_nt_w4x_swiglu
+            from kgs.ops.gemm import gemm_nt_w4x_splitk_swiglu, gemm_nt_w4x_swiglu
             from kgs.ops.transformer import splitk_add_rmsnorm
         # split-K qkv with KGS_ROPE_ATTN=1: its reduce + RoPE + KV write run
         # inside the attention launch (one launch per layer fewer)
@@ -529,13 +541,13 @@ class ServingModel:
             c.heads // c.kv_heads <= 6
         for i in range(c.layers):
             if fused_attn:
-                part = gemm_nt_w4x_partials(y, self._w4x_weight(i, "qkv", rq[0]), *rq, nt_weights=D.w4x_nt(rq))
+                part = self._split_proj(y, i, "qkv", rq)
                 a = D.rope_paged_decode_attention(part, self.cos, self.sin, positions, slots, self.cache.layer(i),
                                                   block_tables, ctx_lens, c.heads, c.kv_heads,
                                                   pages_per_split=pages_per_split)
                 T.op(f"decode L{i} qkv+rope+attention")
             elif rq:
-                part = gemm_nt_w4x_partials(y, self._w4x_weight(i, "qkv", rq[0]), *rq, nt_weights=D.w4x_nt(rq))
+                part = self._split_proj(y, i, "qkv", rq)
                 qkv = torch.empty((m, part.shape[2]), dtype=torch.bfloat16, device=x.device)
                 D.rope_cache_(qkv, self.cos, self.sin, positions, slots, self.cache.layer(i), c.heads, c.kv_heads,
                               partials=part)
@@ -554,12 +566,14 @@ class ServingModel:
                                              pages_per_split=pages_per_split)
                 T.op(f"decode L{i} attention")
             if ro:
-                y = splitk_add_rmsnorm(gemm_nt_w4x_partials(a, self._w4x_weight(i, "o", ro[0]), *ro,
-                                                            nt_weights=D.w4x_nt(ro)), x, self.ln2[i], c.eps)
+                y = splitk_add_rmsnorm(self._split_proj(a, i, "o", ro), x, self.ln2[i], c.eps)
             else:
                 y = self._norm(x, self._proj(a, i, "o", True), self.ln2[i])
             T.op(f"decode L{i} o+norm")
-            if rg:
+            if rg and rg[1] > 1:
+                act = gemm_nt_w4x_splitk_swiglu(y, self.w[i]["gate_up"], rg[0], rg[1], rg[2], nt_weights=D.w4x_nt(rg),
+                                                private=True)
+            elif rg:
                 act = gemm_nt_w4x_swiglu(y, self._gate_up_weight(i, rg[0]), bn=rg[0], bm=rg[2],
                                          stages=D.w4x_stages(rg), nt_weights=D.w4x_nt(rg))
             else:
@@ -567,8 +581,7 @@ class ServingModel:
             T.op(f"decode L{i} gate_up")
             nxt = self.ln1[i + 1] if i + 1 < c.layers else self.norm
             if rd:
-                y = splitk_add_rmsnorm(gemm_nt_w4x_partials(act, self._w4x_weight(i, "down", rd[0]), *rd,
-                                                            nt_weights=D.w4x_nt(rd)), x, nxt, c.eps)
+                y = splitk_add_rmsnorm(self._split_proj(act, i, "down", rd), x, nxt, c.eps)
             else:
                 y = self._norm(x, self._proj(act, i, "down", True), nxt)
             T.op(f"decode L{i} down+norm")

@@ -1569,6 +1569,7 @@ KGS_EXPORT int kgs_rope_cache_bf16(void* qkv, const float* cosv, const float* si
     case 2: KGS_RCS(KV, 2); break;    \
     case 4: KGS_RCS(KV, 4); break;    \
     case 8: KGS_RCS(KV, 8); break;    \
+    case 16: KGS_RCS(KV, 16); break;  \
     default: KGS_RCS(KV, 0); break;   \
   }
     if (kv8) {
@@ -1586,7 +1587,10 @@ KGS_EXPORT int kgs_rope_cache_bf16(void* qkv, const float* cosv, const float* si
     const dim3 gv((unsigned)((tokens + kgs::dec::PAGE - 1) / kgs::dec::PAGE), (unsigned)HKV);
     hipLaunchKernelGGL(kgs::dec::v_cache_pages, gv, b, 0, s, (const unsigned short*)q, slot, (unsigned short*)cache,
                        tokens, H, HKV, ld);
-  } else if ((H + 2 * HKV) % 8 == 0) {
+  } else if ((H + 2 * HKV) % 8 == 0 && n > 2 * 256 * 256) {
+    // more than two workgroups of the per-head form on every CU: eight heads a thread share the
+    // cos / sin loads; below, their serial work is what takes the time (24 heads, us of
+    // per-head / eight-head: 8 tokens 3.6 / 5.9, 100 4.1 / 6.9, 512 7.0 / 8.3, 1000 10.2 / 10.0)
     const dim3 g8((unsigned)((n / 8 + 255) / 256));
     if (kv8)
       hipLaunchKernelGGL(kgs::dec::rope_cache_g8<true>, g8, b, 0, s, q, cosv, sinv, pos, slot, cache, tokens, H, HKV,

@@ -443,6 +443,7 @@ KGS_EXPORT int kgs_splitk_add_rmsnorm_bf16(const float* P, int nslice, void* x, 
     case 2: KGS_SARN(NJ, 2); break;                               \
     case 4: KGS_SARN(NJ, 4); break;                               \
     case 8: KGS_SARN(NJ, 8); break;                               \
+    case 16: KGS_SARN(NJ, 16); break;                             \
     default: KGS_SARN(NJ, 0); break;                              \
   }
   switch (nj) {

@@ -553,7 +553,7 @@ class PagedKVCache:
 
 def rope_cache_(qkv: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, positions: torch.Tensor,
                 slots: torch.Tensor, cache_layer: torch.Tensor, heads: int, kv_heads: int,
-                partials: torch.Tensor | None = None) -> torch.Tensor:
+                partials: torch.Tensor | None = None, rows: torch.Tensor | None = None) -> torch.Tensor:
     """In place: rotate the q and k heads of every row of the fused ``qkv``
     ``[T, (H + 2 HKV) * 128]`` at ``positions[t]``, and write k, v into cache slot
     ``slots[t]`` (``page * 32 + offset``; < 0 skips the write).
@@ -561,8 +561,15 @@ def rope_cache_(qkv: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, positio
     ``partials`` (fp32 ``[nslice, T, (H + 2 HKV) * 128]``, from
     ``kgs.ops.gemm.gemm_nt_w4x_partials``): the projection arrives as split-K
     partial products; they are reduced (bf16-rounded like the unfused reduce)
-    in the same launch and ``qkv`` is output only."""
+    in the same launch and ``qkv`` is output only.
+
+    ``rows`` (int32, one per token): token ``t`` is row ``rows[t]`` of ``qkv``, none where negative --
+    prompts padded to whole pages whose padding has no rows."""
     t = qkv.shape[0]
+    if rows is not None:
+        t = rows.numel()
+        if rows.dtype != torch.int32 or not rows.is_contiguous() or partials is not None:
+            raise ValueError("rows must be a contiguous int32 vector, without partials")
     if qkv.dtype != torch.bfloat16 or not qkv.is_cuda or qkv.stride(1) != 1:
         raise ValueError("qkv must be a row-major bf16 GPU matrix")
     nslice = 0
@@ -583,7 +590,7 @@ def rope_cache_(qkv: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, positio
                                         slots.data_ptr(), cache_layer.data_ptr(), t, heads, kv_heads, HEAD_DIM,
                                         qkv.stride(0), 1 if cache_layer.dtype == FP8 else 0,
                                         None if partials is None else partials.data_ptr(), nslice,
-                                        _lib.stream_handle(qkv.device))
+                                        None if rows is None else rows.data_ptr(), _lib.stream_handle(qkv.device))
     _lib.check(rc, "rope_cache")
     return qkv
 

@@ -269,10 +269,10 @@ QBLOCK = 128  # query rows of an attention_blocks item
 def attention_blocks(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, items: torch.Tensor, heads: int, kv_heads: int,
                      out: torch.Tensor, k2: torch.Tensor | None = None, v2: torch.Tensor | None = None,
                      scale: float | None = None) -> torch.Tensor:
-    """Causal flash attention of sequences of any lengths in one launch (head_dim 128), a block of 128
-    query rows each item. ``items`` int32 ``[n, 4]``: the block's first row in ``q`` / ``out``, the row
-    of its sequence's key 0, the position of the first row (a multiple of 64), and 0 for keys
-    in ``k`` / ``v`` or 1 for keys in ``k2`` / ``v2``. An item reads its position + 128 keys."""
+    """Causal flash attention of sequences of any lengths in one launch (head_dim 128), a block of up to
+    128 query rows each item. ``items`` int32 ``[n, 4]`` (:func:`block_items`): the block's first row in
+    ``q`` / ``out``, the row of its sequence's key 0, the position of the first row, and twice its
+    number of rows, plus 1 for keys in ``k2`` / ``v2`` instead of ``k`` / ``v``."""
     for t, n in ((q, "q"), (k, "k"), (v, "v"), (out, "out")):
         _need(t, n)
     if items.dtype != torch.int32 or items.dim() != 2 or items.shape[1] != 4 or not items.is_contiguous():
@@ -290,15 +290,17 @@ def attention_blocks(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, items: t
 
 
 def block_items(seqs, rows: int):
-    """Items of :func:`attention_blocks`, heaviest first, for sequences ``(first query row, rows (a
-    multiple of 128), first key row, position of the first row (a multiple of 64), key
-    source)`` among ``rows`` query rows (and keys, for source 0)."""
+    """Items of :func:`attention_blocks`, heaviest first, for sequences ``(first query row, rows,
+    first key row, position of the first row, key source)`` among ``rows`` query rows (and
+    keys, for source 0)."""
     import numpy as np
 
+    out = []
     for r, n, k0, pos, src in seqs:
-        if n <= 0 or n % QBLOCK or pos % 64 or min(r, k0, pos) < 0 or max(r + n, 0 if src else k0 + pos + n) > rows:
-            raise ValueError(f"a sequence of {n} rows from {r} at position {pos} does not fit blocks of {QBLOCK} in {rows} rows")
-    out = np.array([(r + b, k0, pos + b, src) for r, n, k0, pos, src in seqs for b in range(0, n, QBLOCK)], np.int32)
+        if n <= 0 or min(r, k0, pos) < 0 or max(r + n, 0 if src else k0 + pos + n) > rows:
+            raise ValueError(f"a sequence of {n} rows from {r} at position {pos} does not fit {rows} rows")
+        out += [(r + b, k0, pos + b, 2 * min(QBLOCK, n - b) + src) for b in range(0, n, QBLOCK)]
+    out = np.array(out, np.int32).reshape(-1, 4)
     return out[np.argsort(-out[:, 2], kind="stable")]
 
 

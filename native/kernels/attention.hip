@@ -76,9 +76,10 @@ struct Args {
 
 // EQUAL: B equal sequences of S rows, a multiple of QB. RAGGED: any number of query rows per
 // sequence at any position (Args::items), rows and keys past a block's end clamped on load and
-// dropped on store; always causal. BLOCKS: whole blocks of QB rows of sequences of any lengths in
-// one launch, causal, with grouped key heads; one int4 per block -- first query row, first key row
-// of its sequence, position of the first query row (a multiple of KB), and 1 where the keys are
+// dropped on store; always causal. BLOCKS: blocks of up to QB rows of sequences of any lengths in
+// one launch, causal, with grouped key heads, clamped likewise; one int4 per block -- first query
+// row, first key row of its sequence, position of the first query row, and twice the number of
+// rows, plus 1 where the keys are
 // rows of k2 / v2. One launch because one per sequence leaves the chip to each sequence's own tail:
 // prompts of a few hundred tokens at 32 heads have fewer workgroups each than the 512 that are
 // resident. A whole prompt step of 16 unequal prompts of about 512 tokens (H 4096) went from 13.76
@@ -100,7 +101,7 @@ __device__ __forceinline__ bf16x8 pack8(const f32x16& s, int base) { return pack
 
 template <int HD, Mode MODE, int HR = 0>
 __global__ __launch_bounds__(256, 2) __attribute__((amdgpu_waves_per_eu(2, 2))) void fwd(Args a) {
-  constexpr bool RAGGED = MODE == RAGGED_ROWS;
+  constexpr bool RAGGED = MODE == RAGGED_ROWS, PART = MODE != EQUAL;
   constexpr int TILE_BYTES = KB * HD * 2;  // 16 KB at 128
   constexpr int ND = HD / 32, NK = HD / 16, NR = HR / 16, ROT_BYTES = KB * HR * 2;
   __shared__ __attribute__((aligned(16))) char smem[2][2 * TILE_BYTES + ROT_BYTES];  // [buf]: K, V, rotated K
@@ -126,7 +127,8 @@ __global__ __launch_bounds__(256, 2) __attribute__((amdgpu_waves_per_eu(2, 2))) 
     tok0 = it.x;
     ktok0 = it.y;
     qoff = it.z;
-    if (it.w) {
+    nval = it.w >> 1;
+    if (it.w & 1) {
       kp = a.k2;
       vp = a.v2;
       ldk = ldv = a.ld2;
@@ -162,7 +164,7 @@ __global__ __launch_bounds__(256, 2) __attribute__((amdgpu_waves_per_eu(2, 2))) 
     qoff = a.qoff;
     causal = a.causal != 0;
   }
-  const int lrow = RAGGED ? min(qrow, nval - 1) : qrow;  // the row this lane loads
+  const int lrow = PART ? min(qrow, nval - 1) : qrow;  // the row this lane loads
 
   // Q fragments (B operand of S^T = K.Q^T): lane holds Q[qrow][16ks + 8hh .. +7]
   bf16x8 qf[NK + NR];
@@ -202,7 +204,7 @@ __global__ __launch_bounds__(256, 2) __attribute__((amdgpu_waves_per_eu(2, 2))) 
       const int ch = ND * w + i;
       const int r = (512 / HD) * ch + lane / (HD / 8), c = (lane & (HD / 8 - 1)) ^ swz<HD>(r);
       long row = (long)jn * KB + r;
-      if constexpr (RAGGED) row = min(row, (long)(qoff + nval - 1));
+      if constexpr (PART) row = min(row, (long)(qoff + nval - 1));
       glds16(kbase + row * ldk + 8 * c, smem[sb] + 1024 * ch);
       glds16(vbase + row * ldv + 8 * c, smem[sb] + TILE_BYTES + 1024 * ch);
     }
@@ -217,7 +219,7 @@ __global__ __launch_bounds__(256, 2) __attribute__((amdgpu_waves_per_eu(2, 2))) 
     }
   };
 
-  const int ntile = RAGGED ? (qoff + nval - 1) / KB + 1 : causal ? (qoff + q0 + QB) / KB : a.Sk / KB;
+  const int ntile = PART ? (qoff + nval - 1) / KB + 1 : causal ? (qoff + q0 + QB) / KB : a.Sk / KB;
   const int win = RAGGED ? a.win : 0;
   const int j0 = win ? max(0, qoff + q0 - win + 1) / KB : 0;
   dma_tiles(j0, 0);
@@ -357,8 +359,9 @@ __global__ __launch_bounds__(256, 2) __attribute__((amdgpu_waves_per_eu(2, 2))) 
 
   l = xor32_sum(l);
   float inv = 1.0f / l;
-  if constexpr (RAGGED) {
+  if constexpr (PART)
     if (qrow >= nval) return;
+  if constexpr (RAGGED) {
     if (a.gate && !a.eg) inv /= 1.0f + __expf(-bf2f(a.gate[(tok0 + qrow) * a.ldg + (long)h * a.hg]));
   }
   unsigned short* op = a.o + (tok0 + qrow) * a.ldo + (long)h * HD;
@@ -448,10 +451,10 @@ KGS_EXPORT int kgs_attn_fwd_ragged_bf16(const void* q, const void* k, const void
   return (int)hipGetLastError();
 }
 
-// Causal attention of sequences of any lengths in whole blocks of 128 query rows, head_dim 128,
+// Causal attention of sequences of any lengths in blocks of up to 128 query rows, head_dim 128,
 // grouped key heads, one launch. items: nitems int4 (first query row, first key row of its
-// sequence, position of the first query row among these, 0: keys in k / v, 1: in k2 / v2), any
-// order (heaviest first keeps the tail short). Every item reads its position + 128 keys.
+// sequence, position of the first query row among these, 2 * rows (1 to 128) + (0: keys in k / v, 1: in
+// k2 / v2)), any order (heaviest first keeps the tail short). Every item reads its position + rows keys.
 KGS_EXPORT int kgs_attn_fwd_blocks_bf16(const void* q, const void* k, const void* v, const void* k2, const void* v2, void* o,
                                        const void* items, int nitems, int H, int HKV, int hd, long ldq, long ldk,
                                        long ldv, long ld2, long ldo, float scale, hipStream_t s) {

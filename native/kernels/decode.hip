@@ -560,14 +560,17 @@ __global__ __launch_bounds__(256) void rope_cache(unsigned short* __restrict__ q
                                                   const float* __restrict__ sinv, const int* __restrict__ pos,
                                                   const int* __restrict__ slot, void* __restrict__ cache,
                                                   long tokens, int H, int HKV, long ld,
-                                                  const float* __restrict__ P = nullptr, int nslice = 0) {
+                                                  const float* __restrict__ P = nullptr, int nslice = 0,
+                                                  const int* __restrict__ rows = nullptr) {
   const int nh = H + 2 * HKV;
   const long idx = (long)blockIdx.x * 256 + threadIdx.x;
   if (idx >= tokens * nh * 8) return;
   const long t = idx / (nh * 8);
   const int rem = (int)(idx - t * nh * 8);
   const int h = rem >> 3, c = rem & 7;
-  unsigned short* base = qkv + t * ld + (long)h * HD + 8 * c;
+  const long row = rows ? rows[t] : t;
+  if (row < 0) return;
+  unsigned short* base = qkv + row * ld + (long)h * HD + 8 * c;
   bf16x8* p1 = (bf16x8*)base;
   bf16x8* p2 = (bf16x8*)(base + HD / 2);
   // position and cache slot first: the cos/sin loads hang off pos[t], so its
@@ -645,7 +648,8 @@ template <bool KV8, bool VSEP = false>
 __global__ __launch_bounds__(256) void rope_cache_g8(unsigned short* __restrict__ qkv, const float* __restrict__ cosv,
                                                      const float* __restrict__ sinv, const int* __restrict__ pos,
                                                      const int* __restrict__ slot, void* __restrict__ cache,
-                                                     long tokens, int H, int HKV, long ld) {
+                                                     long tokens, int H, int HKV, long ld,
+                                                     const int* __restrict__ rows) {
   const int ng = (H + 2 * HKV) >> 3;
   const long idx = (long)blockIdx.x * 256 + threadIdx.x;
   if (idx >= tokens * ng * 8) return;
@@ -653,9 +657,11 @@ __global__ __launch_bounds__(256) void rope_cache_g8(unsigned short* __restrict_
   const int rem = (int)(idx - t * ng * 8);
   const int g = rem >> 3, c = rem & 7;
   if (VSEP && g * 8 >= H + HKV) return;  // a group of v heads only
+  const long row = rows ? rows[t] : t;
+  if (row < 0) return;
   const int p = pos[t];
   const int sl = slot[t];
-  unsigned short* base = qkv + t * ld + (long)g * 8 * HD + 8 * c;
+  unsigned short* base = qkv + row * ld + (long)g * 8 * HD + 8 * c;
   bf16x8 a[8], b[8];
 #pragma unroll
   for (int j = 0; j < 8; ++j) {
@@ -696,17 +702,18 @@ __global__ __launch_bounds__(256) void rope_cache_g8(unsigned short* __restrict_
 // as kv_write.
 __global__ __launch_bounds__(256) void v_cache_pages(const unsigned short* __restrict__ qkv,
                                                      const int* __restrict__ slot, unsigned short* __restrict__ cache,
-                                                     long tokens, int H, int HKV, long ld) {
+                                                     long tokens, int H, int HKV, long ld,
+                                                     const int* __restrict__ rows) {
   __shared__ unsigned short vs[PAGE][HD + 8];
   __shared__ int sl[PAGE];
   __shared__ int fast;
   const long t0 = (long)blockIdx.x * PAGE;
   const int kvh = blockIdx.y, tid = threadIdx.x;
-  if (tid < PAGE) sl[tid] = t0 + tid < tokens ? slot[t0 + tid] : -1;
+  if (tid < PAGE) sl[tid] = t0 + tid < tokens && (!rows || rows[t0 + tid] >= 0) ? slot[t0 + tid] : -1;
   for (int k = tid; k < PAGE * (HD / 8); k += 256) {
     const int r = k / (HD / 8), ch = k % (HD / 8);
-    const long t = t0 + r;
-    const uint4 v = t < tokens ? *(const uint4*)(qkv + t * ld + (long)(H + HKV + kvh) * HD + ch * 8)
+    const long t = t0 + r, row = t >= tokens ? -1 : rows ? rows[t] : t;
+    const uint4 v = row >= 0 ? *(const uint4*)(qkv + row * ld + (long)(H + HKV + kvh) * HD + ch * 8)
                                : make_uint4(0, 0, 0, 0);
     *(uint4*)&vs[r][ch * 8] = v;
   }
@@ -1549,13 +1556,15 @@ KGS_EXPORT int kgs_skinny_gemm_bf16(const void* wp, const void* x, void* y, floa
 // P != nullptr: the projection is given as nslice fp32 split-K partials
 // [nslice][tokens][(H + 2 HKV) * hd] instead of in qkv; the reduced, rotated
 // rows are written to qkv (which is then output only).
+// rows != nullptr (without P): token t is row rows[t] of qkv, none where negative: prompts padded
+// to whole pages whose padding has no rows, so that a page's run still leaves in 16-byte chunks.
 KGS_EXPORT int kgs_rope_cache_bf16(void* qkv, const float* cosv, const float* sinv, const int* pos, const int* slot,
                                   void* cache, long tokens, int H, int HKV, int hd, long ld, int kv8, const float* P,
-                                  int nslice, hipStream_t s) {
+                                  int nslice, const int* rows, hipStream_t s) {
   if (tokens < 0 || H <= 0 || HKV <= 0 || H % HKV || hd != kgs::dec::HD) return KGS_ERR_SHAPE;
   if (ld < (long)(H + 2 * HKV) * hd) return KGS_ERR_SHAPE;
   if (!al16(qkv) || !al16(cosv) || !al16(sinv) || !al16(cache) || ld % 8) return KGS_ERR_ALIGN;
-  if (P != nullptr && (nslice <= 0 || !al16(P))) return KGS_ERR_ARG;
+  if (P != nullptr && (nslice <= 0 || !al16(P) || rows != nullptr)) return KGS_ERR_ARG;
   const long n = tokens * (H + 2 * HKV) * 8;
   if (n == 0) return 0;
   const dim3 g((unsigned)((n + 255) / 256)), b(256);
@@ -1563,7 +1572,7 @@ KGS_EXPORT int kgs_rope_cache_bf16(void* qkv, const float* cosv, const float* si
   if (P != nullptr) {
 #define KGS_RCS(KV, NSL)                                                                                           \
   hipLaunchKernelGGL((kgs::dec::rope_cache<KV, true, NSL>), g, b, 0, s, q, cosv, sinv, pos, slot, cache, tokens, H, \
-                     HKV, ld, P, nslice)
+                     HKV, ld, P, nslice, nullptr)
 #define KGS_RCS_KV(KV)                \
   switch (nslice) {                   \
     case 2: KGS_RCS(KV, 2); break;    \
@@ -1583,10 +1592,10 @@ KGS_EXPORT int kgs_rope_cache_bf16(void* qkv, const float* cosv, const float* si
     // prompt-sized: the v heads go through the page-run writer
     const dim3 g8((unsigned)((n / 8 + 255) / 256));
     hipLaunchKernelGGL((kgs::dec::rope_cache_g8<false, true>), g8, b, 0, s, q, cosv, sinv, pos, slot, cache, tokens, H,
-                       HKV, ld);
+                       HKV, ld, rows);
     const dim3 gv((unsigned)((tokens + kgs::dec::PAGE - 1) / kgs::dec::PAGE), (unsigned)HKV);
     hipLaunchKernelGGL(kgs::dec::v_cache_pages, gv, b, 0, s, (const unsigned short*)q, slot, (unsigned short*)cache,
-                       tokens, H, HKV, ld);
+                       tokens, H, HKV, ld, rows);
   } else if ((H + 2 * HKV) % 8 == 0 && n > 2 * 256 * 256) {
     // more than two workgroups of the per-head form on every CU: eight heads a thread share the
     // cos / sin loads; below, their serial work is what takes the time (24 heads, us of
@@ -1594,16 +1603,16 @@ KGS_EXPORT int kgs_rope_cache_bf16(void* qkv, const float* cosv, const float* si
     const dim3 g8((unsigned)((n / 8 + 255) / 256));
     if (kv8)
       hipLaunchKernelGGL(kgs::dec::rope_cache_g8<true>, g8, b, 0, s, q, cosv, sinv, pos, slot, cache, tokens, H, HKV,
-                         ld);
+                         ld, rows);
     else
       hipLaunchKernelGGL(kgs::dec::rope_cache_g8<false>, g8, b, 0, s, q, cosv, sinv, pos, slot, cache, tokens, H, HKV,
-                         ld);
+                         ld, rows);
   } else if (kv8) {
     hipLaunchKernelGGL(kgs::dec::rope_cache<true>, g, b, 0, s, q, cosv, sinv, pos, slot, cache, tokens, H, HKV, ld,
-                       nullptr, 0);
+                       nullptr, 0, rows);
   } else {
     hipLaunchKernelGGL(kgs::dec::rope_cache<false>, g, b, 0, s, q, cosv, sinv, pos, slot, cache, tokens, H, HKV, ld,
-                       nullptr, 0);
+                       nullptr, 0, rows);
   }
   return (int)hipGetLastError();
 }

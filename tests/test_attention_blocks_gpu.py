@@ -13,12 +13,32 @@ DEV = "cuda"
 
 
 def test_block_items_order_and_refusals():
-    it = T.block_items([(0, 256, 0, 0, 0), (256, 128, 0, 192, 1)], 384)
-    assert it.tolist() == [[256, 0, 192, 1], [128, 0, 128, 0], [0, 0, 0, 0]]
+    it = T.block_items([(0, 256, 0, 0, 0), (256, 100, 0, 190, 1)], 356)
+    assert it.tolist() == [[256, 0, 190, 201], [128, 0, 128, 256], [0, 0, 0, 256]]
     assert it.dtype == np.int32
-    for bad in ((0, 100, 0, 0, 0), (0, 128, 0, 32, 1), (300, 128, 300, 0, 0), (0, 128, 0, 320, 0), (0, 0, 0, 0, 0)):
+    for bad in ((300, 128, 300, 0, 0), (0, 128, 0, 320, 0), (0, 0, 0, 0, 0), (-1, 4, 0, 0, 0)):
         with pytest.raises(ValueError):
             T.block_items([bad], 384)
+
+
+def test_prompt_rows_cpu():
+    """What is dropped, where each row goes and which are wanted, for prompt portions and decode rows."""
+    from kgs.serve.model import ServingModel
+
+    class M:
+        backend = "kgs"
+
+    seqs, dev = [(0, 20, 128, 0), (128, 130, 256, 64)], torch.device("cpu")
+    p = ServingModel._prompt_rows(M, seqs, 387, dev, tail=3, wanted=[False, True])
+    assert p.n == 153 and p.past == [(0, 194, 194, 1)]
+    assert p.keep.tolist() == [*range(20), *range(128, 258), *range(384, 387)]
+    assert p.last.tolist() == [149, 150, 151, 152]
+    assert all(int(p.rows[k]) == i for i, k in enumerate(p.keep.tolist())) and int((p.rows >= 0).sum()) == 153
+    assert sorted(map(tuple, p.items.tolist())) == [(0, 0, 0, 40), (20, 0, 64, 257), (148, 0, 192, 5)]
+    for kw in ({"drop": False}, {}):  # kept whole where asked, or where no tile of rows is saved
+        q = ServingModel._prompt_rows(M, seqs if kw else [(0, 120, 128, 0), (128, 128, 128, 0)], 384 if kw else 256, dev, **kw)
+        assert q.keep is None and q.rows is None and q.last.tolist() == ([19, 257] if kw else [119, 255])
+    assert q.items is None and q.n == 256  # equal portions: the batched launch
 
 
 @pytest.mark.gpu
@@ -28,7 +48,7 @@ def test_blocks_match_per_sequence_bits(heads, kv):
     several blocks beside chunks whose keys are in other buffers, at contexts that end on a
     block's edge and in its middle."""
     torch.manual_seed(heads)
-    lens, past = [128, 384, 256], [(128, 64), (256, 320), (128, 1024)]
+    lens, past = [128, 384, 256], [(128, 64), (256, 320), (128, 1024)]  # what one launch per sequence takes
     rows = sum(lens) + sum(n for n, _ in past) + 5
     w = 128 * (heads + 2 * kv)
     qkv = torch.randn(rows, w, device=DEV).bfloat16()
@@ -50,6 +70,64 @@ def test_blocks_match_per_sequence_bits(heads, kv):
     T.attention_blocks(qkv, k, v, items, heads, kv, out, k2, v2)
     assert torch.equal(out, want)
     assert not out[r:].any()  # rows of no item stay as they were
+
+
+@pytest.mark.gpu
+def test_partial_blocks_match_whole_ones():
+    """Lengths and positions of no multiple: each row's bits as in blocks padded to 128 rows, where the
+    padding holds other values; nothing past a sequence's rows is written."""
+    torch.manual_seed(3)
+    heads, kv, w = 4, 2, 8 * 128
+    seqs = [(1, 0), (127, 0), (129, 0), (64, 0), (300, 0), (65, 64), (1, 192), (200, 448)]
+    rows = sum(n for n, _ in seqs)
+    qkv = torch.randn(rows, w, device=DEV).bfloat16()
+    k2, v2 = torch.randn(2, sum(c + n for n, c in seqs), 128 * kv, device=DEV).bfloat16()
+    plan, want, r, kr = [], [], 0, 0
+    for n, c in seqs:
+        p = -(-n // 128) * 128
+        q = torch.randn(p, w, device=DEV).bfloat16()
+        q[:n] = qkv[r:r + n]
+        if c:
+            k, v = torch.randn(2, c + p, 128 * kv, device=DEV).bfloat16()
+            k[:c + n], v[:c + n] = k2[kr:kr + c + n], v2[kr:kr + c + n]
+            want.append(T.attention_chunk(q, k, v, heads, kv)[:n])
+            plan.append((r, n, kr, c, 1))
+            kr += c + n
+        else:
+            want.append(T.attention_qkv(q, 1, p, heads, kv, out=torch.empty(p, 128 * heads, device=DEV, dtype=torch.bfloat16))[:n])
+            plan.append((r, n, r, 0, 0))
+        r += n
+    out = torch.full((rows + 9, 128 * heads), 5.0, device=DEV, dtype=torch.bfloat16)
+    items = torch.from_numpy(T.block_items(plan, rows)).to(DEV)
+    T.attention_blocks(qkv, qkv[:, 128 * heads:128 * (heads + kv)], qkv[:, 128 * (heads + kv):], items, heads, kv, out, k2, v2)
+    assert torch.equal(out[:rows], torch.cat(want))
+    assert bool((out[rows:] == 5).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("cache_dtype", [torch.bfloat16, D.FP8])
+@pytest.mark.parametrize("lens", [[5, 33, 1], [20] * 9, [700, 400, 31]])
+def test_rope_rows_match_padded(lens, cache_dtype):
+    """Tokens padded to 128 a prompt whose padding has no rows: the rows and the cache of the padded call."""
+    torch.manual_seed(len(lens))
+    heads, kv = 4, 2
+    total = sum(-(-n // 128) * 128 for n in lens)
+    real = sum(lens)
+    cos, sin = T.rope_tables(1024, 128, 1e4, DEV)
+    pos, slot, rows, at, page, r = np.zeros(total, np.int32), np.full(total, -1, np.int32), np.full(total, -1, np.int32), 0, 1, 0
+    for n in lens:
+        pos[at:at + n] = np.arange(n)
+        slot[at:at + n] = 32 * page + np.arange(n)
+        rows[at:at + n] = r + np.arange(n)
+        at, page, r = at + -(-n // 128) * 128, page + -(-n // 32), r + n
+    pos, slot, rows = (torch.from_numpy(x).to(DEV) for x in (pos, slot, rows))
+    qkv = torch.randn(real, (heads + 2 * kv) * 128, device=DEV).bfloat16()
+    full = torch.randn(total, (heads + 2 * kv) * 128, device=DEV).bfloat16()
+    full[rows >= 0] = qkv
+    ca, cb = (torch.zeros(page + 1, kv, 2, 4096, device=DEV).to(cache_dtype) for _ in range(2))
+    D.rope_cache_(full, cos, sin, pos, slot, ca, heads, kv)
+    D.rope_cache_(qkv, cos, sin, pos, slot, cb, heads, kv, rows=rows)
+    assert torch.equal(qkv, full[rows >= 0]) and torch.equal(ca.view(torch.uint8), cb.view(torch.uint8))
 
 
 @pytest.mark.gpu

@@ -43,8 +43,10 @@ _SIGS = {
     "kgs_gemm_bf16_nt_swiglu": ([_c_void_p] * 3 + [_c_int] * 7 + [_c_void_p] * 2, _c_int),
     "kgs_gemm_bf16_nt_act": ([_c_void_p] * 5 + [_c_int] * 7 + [_c_void_p] * 2, _c_int),
     "kgs_gemm_bf16_tr_slices": ([_c_int] * 5, _c_int),
-    "kgs_act_grad_parts": ([_c_int], _c_int),
-    "kgs_act_grad": ([_c_void_p] * 6 + [_c_int] * 3 + [_c_void_p], _c_int),
+    "kgs_act_grad_parts": ([_c_int] * 2, _c_int),
+    "kgs_act_grad": ([_c_void_p] * 6 + [_c_int] * 4 + [_c_void_p], _c_int),
+    "kgs_pad_rows_bf16": ([_c_void_p] * 2 + [_c_long, _c_int, _c_long] + [_c_void_p] * 2 + [_c_long, _c_int, _c_long, _c_void_p],
+                          _c_int),
     "kgs_gemm_bf16_tr": ([_c_void_p] * 3 + [_c_int] * 9 + [_c_void_p] * 2, _c_int),
     "kgs_gemm_bf16_nt_addc": ([_c_void_p, _c_void_p, _c_void_p] + [_c_int] * 6 + [_c_void_p], _c_int),
     "kgs_tile_queue_stats": ([_c_int, ctypes.POINTER(_c_long)], _c_int),

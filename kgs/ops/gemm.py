@@ -74,6 +74,9 @@ def gemm_nt(
         _check_operand(out, "out")
         if tuple(out.shape) != (M, N):
             raise ValueError(f"out has shape {tuple(out.shape)}, expected {(M, N)}")
+    if variant == "auto" and K > PAD_MIN_K:
+        a, b = _even(a, b)
+        K = a.shape[1]
     ptrs = (a.data_ptr(), b.data_ptr(), out.data_ptr(), bias.data_ptr() if bias is not None else None, M, N, K,
             a.stride(0), b.stride(0), out.stride(0), epi)
     if variant == "auto":
@@ -83,6 +86,26 @@ def gemm_nt(
         rc = _lib.lib().kgs_gemm_bf16_nt(*ptrs, VARIANTS[variant], _lib.stream_handle(a.device))
     _lib.check(rc, f"gemm_nt[{M}x{N}x{K}]")
     return out
+
+
+PAD_MIN_K = 32  # products of shorter rows read them element by element where 16 bytes do not fit
+
+
+def _even(*ts: torch.Tensor) -> tuple[torch.Tensor, ...]:
+    """One or two matrices, each a zero-padded copy where its rows are not whole, aligned 16-byte
+    chunks: what the fast kernels read. One launch for both copies."""
+    odd = [i for i, t in enumerate(ts) if (t.shape[1] % 8 or not _rows16(t)) and t.numel()]
+    if not odd:
+        return ts
+    out, args = list(ts), []
+    for i in odd:
+        t = ts[i]
+        out[i] = torch.empty((t.shape[0], (t.shape[1] + 7) // 8 * 8), dtype=torch.bfloat16, device=t.device)
+        args += [t.data_ptr(), out[i].data_ptr(), t.shape[0], t.shape[1], t.stride(0)]
+    if len(odd) == 1:
+        args += [None, None, 0, 0, 0]
+    _lib.check(_lib.lib().kgs_pad_rows_bf16(*args, _lib.stream_handle(out[odd[0]].device)), "pad_rows")
+    return tuple(out)
 
 
 @lru_cache(maxsize=4096)
@@ -597,12 +620,31 @@ def gemm_bf16(a: torch.Tensor, b: torch.Tensor, trans_a: bool = False, trans_b: 
     if K != K2:
         raise ValueError(f"inner dims differ: op(a) {M}x{K}, op(b) {K2}x{N}")
     ta, tb = int(trans_a), int(not trans_b)  # kernel flags: 1 = operand stored [K][rows]
-    if (ta or tb) and bias is None and act in (None, "none") and not TR_READ_A and _rows16(a) and _rows16(b) and \
-            a.shape[1] % 8 == 0 and b.shape[1] % 8 == 0 and (out is None or tuple(out.shape) == (M, N)) and \
-            M and N and 0 < (K + 128) * max(a.stride(0), b.stride(0)) < 1 << 30:
+    if (ta or tb) and bias is None and act in (None, "none") and not TR_READ_A and M and N and K and \
+            (out is None or tuple(out.shape) == (M, N)):
+        return _product(*_even(a, b), out, M, N, K, ta, tb)
+    return _general(a, b, out, M, N, K, ta, tb, bias, act)
+
+
+def _product(a, b, out, M, N, K, ta, tb) -> torch.Tensor:
+    """The product of operands whose rows are whole 16-byte chunks, at least one of them K-major; what
+    lies between their last column and the next chunk is theirs too, and zero."""
+    if (K + 128) * max(a.stride(0), b.stride(0)) < 1 << 30:
         ns = _tr_slices(M, N, K, bool(ta), bool(tb))
         if ns:
             return _gemm_tr(a, b, out, M, N, K, ta, tb, ns)
+
+    def turn(t, n):
+        return transpose(t if n % 8 == 0 else t.as_strided((t.shape[0], (n + 7) // 8 * 8), t.stride()))[:n]
+
+    if ta:
+        a, ta = turn(a, M), 0
+    if tb and N % 8:
+        b, tb = turn(b, N), 0
+    return _general(a[:, :K], b if tb else b[:, :K], out, M, N, K, ta, tb, None, None)
+
+
+def _general(a, b, out, M, N, K, ta, tb, bias, act) -> torch.Tensor:
     if ta and not TR_READ_A:
         # measured: the tr-read A path runs ~20 % behind a 6.3 TB/s transpose + NT
         # at 8192^3 and ties at 4096^3 (profiles/gemm_layouts.json)
@@ -655,6 +697,9 @@ def gemm_nt_act(a: torch.Tensor, b: torch.Tensor, bias: torch.Tensor | None, act
         raise ValueError(f"inner dims differ: a {tuple(a.shape)} b {tuple(b.shape)}")
     if a.device != b.device:
         raise ValueError("a and b on different devices")
+    if K > PAD_MIN_K:
+        a, b = _even(a, b)
+        K = a.shape[1]
     if not _rows16(a) or not _rows16(b) or K % 8 or M == 0 or max(a.stride(0), b.stride(0)) >= 1 << 22:
         z = gemm_nt(a, b, bias=bias)
         return z, _act(z, act)
@@ -672,23 +717,26 @@ def gemm_nt_act(a: torch.Tensor, b: torch.Tensor, bias: torch.Tensor | None, act
 def act_grad(gy: torch.Tensor, z: torch.Tensor | None, act: str | None, bias: bool, turned: bool
              ) -> tuple[torch.Tensor, torch.Tensor | None, torch.Tensor | None]:
     """``gz = gy * act'(z)`` for contiguous bf16 ``gy`` (``act`` None: ``gy`` itself), its transpose
-    if ``turned`` and its column sums if ``bias``, from one pass over memory."""
+    if ``turned`` and its column sums if ``bias``, from one pass over memory. ``gz``'s rows are
+    whole 16-byte chunks, zeros past ``N`` (a view of them)."""
     M, N = gy.shape
     act = act if act in GRADS else None
     empty = torch.empty
-    gz = gy if act is None else empty((M, N), dtype=torch.bfloat16, device=gy.device)
+    ld = (N + 7) // 8 * 8
+    fresh = act is not None or ld != N or gy.data_ptr() % 16 != 0
+    gz = empty((M, ld), dtype=torch.bfloat16, device=gy.device) if fresh else gy
     gzt = empty((N, M), dtype=torch.bfloat16, device=gy.device) if turned else None
     gb = empty(N, dtype=torch.bfloat16, device=gy.device) if bias else None
-    if act is None and gzt is None and gb is None:
+    if not fresh and gzt is None and gb is None:
         return gz, None, None
     if M == 0 or N == 0:
-        return gz, gzt, gb.zero_() if bias else None
+        return gz[:, :N], gzt, gb.zero_() if bias else None
     lib = _lib.lib()
-    parts = lib.kgs_act_grad_parts(M) if bias else 1
+    parts = lib.kgs_act_grad_parts(M, N) if bias else 1
     part = empty((parts, N), dtype=torch.float32, device=gy.device) if parts > 1 else None
-    ptr = [None if t is None else t.data_ptr() for t in (gy, z if act else None, gz if act else None, gzt, part, gb)]
-    _lib.check(lib.kgs_act_grad(*ptr, M, N, EPI[act], _lib.stream_handle(gy.device)), f"act_grad[{M}x{N}]")
-    return gz, gzt, gb
+    ptr = [None if t is None else t.data_ptr() for t in (gy, z if act else None, gz if fresh else None, gzt, part, gb)]
+    _lib.check(lib.kgs_act_grad(*ptr, M, N, ld, EPI[act], _lib.stream_handle(gy.device)), f"act_grad[{M}x{N}]")
+    return gz if ld == N else gz[:, :N], gzt, gb
 
 
 class _LinearFn(torch.autograd.Function):
@@ -717,11 +765,17 @@ class _LinearFn(torch.autograd.Function):
         # written by the pass that makes dY
         turned = need_w and M > 0 and M % 8 == 0 and not _tr_slices(N, K, M, True, True)
         gz, gzt, gb = act_grad(gy, getattr(ctx, "z", None), ctx.act, need_b and bias is not None, turned)
+        if not (M and N and K):
+            return (gemm_bf16(gz, w) if need_x else None, gemm_bf16(gz, x, trans_a=True) if need_w else None, gb, None)
+        if need_x and need_w:
+            x, w = _even(x, w)
+        elif need_x:
+            (w,) = _even(w)
+        elif need_w:
+            (x,) = _even(x)
         # dX[M,K] = dY[M,N] . W[N,K]      (W read K-major)
-        gx = gemm_bf16(gz, w) if need_x else None
-        gw = None
-        if need_w:
-            gw = gemm_bf16(gzt, x) if turned else gemm_bf16(gz, x, trans_a=True)
+        gx = _product(gz, w, None, M, K, N, 0, 1) if need_x else None
+        gw = _product(gzt if turned else gz, x, None, N, K, M, int(not turned), 1) if need_w else None
         return gx, gw, gb, None
 
 

@@ -266,7 +266,8 @@ void gemm_nt_any(Args a) {
 // A K-major K-tile is 64 rows of 128 columns (256 B). The 16-byte chunk c of row r lies at
 // c ^ 2 (r & 3 | (r >> 3 & 1) << 2), so that the 16 chunks that a half wave of transposed reads
 // touches are on 16 bank groups. Rows past K lie outside the resource and arrive as zeros; columns
-// past M or N only reach outputs that are not stored.
+// past M or N only reach outputs that are not stored. Rows hold whole chunks: sizes of no multiple
+// of 8 come with rows padded to one (zeros where they are contracted over).
 struct TrArgs {
   const unsigned short* A;
   const unsigned short* B;
@@ -305,7 +306,7 @@ struct Operand {
     const int fr = lane & 15, fq = lane >> 4;
     const int n = min(rows - p0, 128);
     if constexpr (TR) {
-      r = __builtin_amdgcn_make_buffer_rsrc((void*)(P + (long)k0 * ld + p0), 0, ((kn - 1) * ld + n) * 2, 0x00020000);
+      r = __builtin_amdgcn_make_buffer_rsrc((void*)(P + (long)k0 * ld + p0), 0, ((kn - 1) * ld + (n + 7) / 8 * 8) * 2, 0x00020000);
       const int row = w * 4 + (lane >> 4);  // of the 16 rows that the four waves' instruction brings
       const int c = (lane & 15) ^ (2 * ((row & 3) | ((row >> 3) & 1) << 2));
       vo = row * ld * 2 + c * 16;
@@ -316,6 +317,7 @@ struct Operand {
 #pragma unroll
       for (int i = 0; i < 4; ++i) ro[i] = kr * 256 + (((half * 8 + 2 * i) ^ x) + (p >> 1)) * 16 + (p & 1) * 8;
     } else {
+      kn = (kn + 7) / 8 * 8;
       r = __builtin_amdgcn_make_buffer_rsrc((void*)(P + (long)p0 * ld + k0), 0, ((n - 1) * ld + kn) * 2, 0x00020000);
       const int row = w * 8 + (lane >> 3);
       ch = ((lane & 7) ^ ((row >> 1) & 7)) * 8;
@@ -466,6 +468,40 @@ __global__ __launch_bounds__(256) void any_reduce(const float* __restrict__ P, u
            make_uint4(act_pair<EPI>(q.x), act_pair<EPI>(q.y), act_pair<EPI>(q.z), act_pair<EPI>(q.w)));
 }
 
+typedef short bf16x8u __attribute__((ext_vector_type(8), aligned(2)));
+
+// Rows of any length at any 2-byte alignment into rows of whole 16-byte chunks, zeros past the
+// last column, of one or two matrices: what the kernels' 16-byte loads can read. Bound by memory
+// (6624 x 2243 5.1 TB/s; small ones the launch, 2.6 us). us by the kernel that reads such operands
+// element by element / by this and the fast tiles: 16 x 64 x 2467 162 / 11, 128 x 128 x 401 55 / 10,
+// 4096 x 4096 x 2467 1204 / 92; they meet near K = 32 (16 x 64 x 33 5.2 / 5.8).
+struct PadArgs {
+  const unsigned short* src[2];
+  unsigned short* dst[2];
+  long rows[2];
+  int cols[2];
+  long ld[2];
+};
+__global__ __launch_bounds__(256) void pad_rows(PadArgs a) {
+  const int per[2] = {(a.cols[0] + 7) / 8, (a.cols[1] + 7) / 8};
+  const long first = a.rows[0] * per[0], all = first + a.rows[1] * per[1];
+  for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < all; i += (long)gridDim.x * 256) {
+    const int o = i >= first;
+    const long j = o ? i - first : i, n = o ? per[1] : per[0], row = j / n;
+    const int c = (int)(j - row * n) * 8, cols = o ? a.cols[1] : a.cols[0];
+    const unsigned short* s = (o ? a.src[1] : a.src[0]) + row * (o ? a.ld[1] : a.ld[0]) + c;
+    bf16x8 v = {0, 0, 0, 0, 0, 0, 0, 0};
+    if (c + 8 <= cols) {
+      v = *(const bf16x8u*)s;
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        if (c + e < cols) v[e] = (short)s[e];
+    }
+    *(bf16x8*)((o ? a.dst[1] : a.dst[0]) + j * 8) = v;
+  }
+}
+
 struct Plan {
   int bm, bn, ns;
 };
@@ -580,11 +616,12 @@ int launch(Args a, Plan p, float* ws, hipStream_t s) {
 
 int cu_count();  // gemm_bf16.hip
 
-// The operands gemm_tr takes. K-major: whole 16-byte chunks of columns, 32-bit offsets over K.
+// The operands gemm_tr takes: rows of whole 16-byte chunks, readable (and zero where contracted
+// over) to the next one, 32-bit offsets over K.
 int gemm_tr_ok(const void* A, const void* B, int M, int N, int K, int lda, int ldb, int ta, int tb) {
+  // lda, ldb are multiples of 8 and so hold the padded rows too
   if (M <= 0 || N <= 0 || K <= 0 || lda % 8 || ldb % 8 || lda < (ta ? M : K) || ldb < (tb ? N : K)) return 0;
   if ((uintptr_t)A % 16 || (uintptr_t)B % 16) return 0;
-  if ((ta ? M : K) % 8 || (tb ? N : K) % 8) return 0;
   const long ea = ta ? (long)(K + 128) * lda : 256L * lda, eb = tb ? (long)(K + 128) * ldb : 256L * ldb;
   if (2 * ea >= any::OOB || 2 * eb >= any::OOB) return 0;
   return ((long)M + 127) / 128 * (((long)N + 127) / 128) * 64 < (1L << 31);
@@ -688,6 +725,21 @@ long gemm_any_ws(int M, int N, int K) {
 }
 
 }  // namespace kgs
+
+// Copies of one or two (src2 null: one) bf16 matrices with rows of cols rounded up to 8, zeros in
+// the added columns. dst 16-B aligned, contiguous.
+KGS_EXPORT int kgs_pad_rows_bf16(const void* src, void* dst, long rows, int cols, long ld, const void* src2, void* dst2,
+                                 long rows2, int cols2, long ld2, hipStream_t s) {
+  using namespace kgs::any;
+  if (!src2) rows2 = cols2 = 0;
+  if (rows <= 0 || cols <= 0 || ld < cols || (src2 && (rows2 <= 0 || cols2 <= 0 || ld2 < cols2))) return KGS_ERR_SHAPE;
+  if ((uintptr_t)src % 2 || (uintptr_t)dst % 16 || (uintptr_t)src2 % 2 || (uintptr_t)dst2 % 16) return KGS_ERR_ALIGN;
+  const PadArgs a{{(const unsigned short*)src, (const unsigned short*)src2}, {(unsigned short*)dst, (unsigned short*)dst2},
+                  {rows, rows2}, {cols, cols2}, {ld, ld2}};
+  const long n = rows * ((cols + 7) / 8) + rows2 * ((cols2 + 7) / 8), wg = (n + 255) / 256;
+  hipLaunchKernelGGL(pad_rows, dim3((unsigned)(wg < 4096 ? wg : 4096)), dim3(256), 0, s, a);
+  return (int)hipGetLastError();
+}
 
 // A product with K-major operands (ta, tb: stored [K][rows]) read in place on 128 x 128 tiles over
 // ns K slices (ws: ns M (N rounded up to 8) fp32 values when ns > 1).

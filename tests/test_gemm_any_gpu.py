@@ -206,3 +206,55 @@ def test_fp8_small_grids_equal_the_eight_wave_kernel(M, N, K):
 
     (a, sa), (b, sb) = quantize_fp8(rnd(M, K)), quantize_fp8(rnd(N, K))
     assert torch.equal(gemm_fp8_nt(a, b, sa, sb), gemm_fp8_nt(a, b, sa, sb, variant="fast"))
+
+
+@pytest.mark.parametrize("rows,cols,off,rows2,cols2", [(1, 1, 0, 1, 9), (7, 33, 1, 130, 33), (300, 2243, 3, 17, 2243), (64, 4097, 7, 1, 8),
+                                                       (513, 64, 1, 2, 5)])
+def test_padded_rows(rows, cols, off, rows2, cols2):
+    """Copies of rows at any 2-byte alignment, zeros up to the next chunk; even rows come back as they are."""
+    from kgs.ops.gemm import _even
+
+    a, b = rnd(rows, cols + off)[:, off:], rnd(rows2, cols2)
+    for t, e in zip((a, b), _even(a, b)):
+        if t.shape[1] % 8 == 0 and t.stride(0) % 8 == 0 and t.data_ptr() % 16 == 0:
+            assert e is t
+        else:
+            assert e.shape[1] % 8 == 0 and torch.equal(e[:, :t.shape[1]], t) and not e[:, t.shape[1]:].any()
+    assert torch.equal(_even(a)[0][:, :cols], a)
+
+
+@pytest.mark.parametrize("M,N,K", [(3, 2, 33), (24, 65, 1555), (128, 130, 2467), (300, 257, 129), (257, 512, 39), (64, 72, 31)])
+@pytest.mark.parametrize("act", [None, "gelu"])
+def test_odd_rows(M, N, K, act):
+    """Rows of no multiple of eight, in every layout, and an aligned K in rows that are not."""
+    from kgs.ops import gemm_nt
+    from kgs.ops.gemm import gemm_bf16
+
+    a, b, bias = rnd(M, K), rnd(N, K), rnd(1, N)[0]
+    want = a.double() @ b.double().T
+    y = gemm_nt(a, b, bias=bias if act else None, act=act)
+    assert rel(y, torch.nn.functional.gelu(want + bias.double(), approximate="tanh") if act else want) < 2 * REL
+    if act:
+        return
+    for ta, tb in ((0, 1), (1, 0), (1, 1)):
+        x, z = (a.T.contiguous() if ta else a), (b.T.contiguous() if tb else b)
+        assert rel(gemm_bf16(x, z, trans_a=bool(ta), trans_b=not tb), want) < REL
+    w = rnd(M, 72)[:, 3:67]
+    v = rnd(N, 64)
+    assert rel(gemm_nt(w, v), w.double() @ v.double().T) < REL
+
+
+@pytest.mark.parametrize("rows,din,dout", [(101, 827, 310), (1024, 310, 54), (56, 2877, 153), (4200, 130, 2049)])
+@pytest.mark.parametrize("frozen", [None, "x", "w"])
+def test_linear_odd_sizes(rows, din, dout, frozen):
+    from kgs.ops import Linear
+
+    lin = Linear(din, dout, act="silu", device=DEV)
+    x, gy = rnd(rows, din).requires_grad_(frozen != "x"), rnd(rows, dout)
+    lin.weight.requires_grad_(frozen != "w")
+    lin(x).backward(gy)
+    p = [t.detach().double().requires_grad_(True) for t in (x, lin.weight, lin.bias)]
+    want = torch.autograd.grad(torch.nn.functional.silu(p[0] @ p[1].T + p[2]), p, gy.double())
+    for t, w in zip((x, lin.weight, lin.bias), want):
+        if t.requires_grad:
+            assert rel(t.grad, w) < 8 * REL  # as test_linear_training_step

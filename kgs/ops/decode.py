@@ -145,11 +145,11 @@ SKINNY_VARIANTS = {
     8: (1, 4, 16), 9: (1, 4, 4), 10: (1, 4, 8), 11: (2, 4, 4), 12: (2, 4, 8),
     13: (2, 8, 2), 14: (2, 8, 4), 15: (4, 8, 2), 16: (1, 8, 4),
     17: (2, 16, 2), 18: (1, 16, 4), 19: (1, 16, 2),
-    20: (1, 1, 8), 21: (2, 1, 8),
+    20: (1, 1, 8), 21: (2, 1, 8), 22: (1, 2, 8), 23: (2, 2, 8), 24: (1, 4, 8), 25: (2, 4, 8),
 }
 # variants whose four waves split one strip's K range (decode.hip skinny KIN):
 # strips of 16 R rows, chunks of 4 x KC k-steps, no cross-workgroup split-K
-KIN_VARIANTS = frozenset({20, 21})
+KIN_VARIANTS = frozenset({20, 21, 22, 23, 24, 25})
 _DEFAULT_VARIANT = {1: 1, 2: 4, 4: 8, 8: 13, 16: 17}
 
 # Measured routing per (MT, N, K) on MI355X with weights streamed from HBM
@@ -160,7 +160,7 @@ _DEFAULT_VARIANT = {1: 1, 2: 4, 4: 8, 8: 13, 16: 17}
 _QKV, _O, _GU, _DOWN, _LM = (6144, 4096), (4096, 4096), (28672, 4096), (4096, 14336), (128256, 4096)
 TUNED: dict = {
     (1, *_QKV): (1, 2), (1, *_O): (20, 1), (1, *_GU): (3, 1), (1, *_DOWN): (1, 4), (1, *_LM): (1, 1),
-    (2, *_QKV): (4, 2), (2, *_O): (4, 4), (2, *_GU): (6, 1), (2, *_DOWN): (4, 4), (2, *_LM): (6, 1),
+    (2, *_QKV): (4, 2), (2, *_GU): (6, 1), (2, *_DOWN): (4, 4), (2, *_LM): (6, 1),
     (4, *_QKV): None, (4, *_O): (9, 4), (4, *_GU): (11, 1), (4, *_DOWN): (10, 4), (4, *_LM): (11, 1),
     (8, *_QKV): None, (8, *_O): None, (8, *_GU): None, (8, *_DOWN): (16, 4), (8, *_LM): None,
     (16, *_QKV): None, (16, *_O): None, (16, *_GU): None, (16, *_DOWN): None, (16, *_LM): None,
@@ -367,14 +367,40 @@ def choose_ksplit(m: int, n: int, k: int, cus: int = CUS, variant: int = 0) -> i
     return best
 
 
+def skinny_rule(m: int, n: int, k: int, one: bool = False) -> tuple[int, int]:
+    """(variant, ksplit) of bf16 weights without a measured entry; ``one``: one W-row tile per wave.
+
+    The K split inside the workgroup (16 rows of W each, no slabs in memory and no ticket, 2 to 3 us
+    of a launch) where its strips are a workgroup per CU or so: up to 6144 rows, two tiles a wave
+    above 4096 from 17 rows of x on. Every workgroup reads all of x, so up to 32 rows of x only K of at
+    most 4096 (8192 in two halves up to 16), beyond those x of 160k values. us at 24 rows, before /
+    so: 3072x2048 10.3 / 6.9, 2048x2048 9.4 / 6.7, 6144x2048 12.4 / 9.9, 4096x4096 14.3 / 11.5; at 1 row 7.6 /
+    5.0, 6.9 / 4.7, 9.7 / 6.9; at 64 rows 2048x2048 13.7 / 11.7, but 4096x4096 18.2 / 20.8.
+    Else x chunks of 8 k-steps instead of 16 from 17 rows on (16384x2048 at 40 rows 22.8 / 18.5,
+    32000x2048 42 / 31)."""
+    mt = _mt(m)
+    strips = n // 16
+    if mt <= 4 and k % 1024 == 0 and n % 32 == 0 and strips <= 384:
+        wide = mt > 1 and strips > 256 and not one
+        v = {1: 20, 2: 23 if wide else 22, 4: 25 if wide else 24}[mt]
+        if mt == 1 and k <= 8192:
+            return v, 2 if k > 4096 and strips < 256 and k % 2048 == 0 else 1
+        if (mt == 2 and k <= 4096) or (mt == 4 and m * k <= 160 << 10):
+            return v, 1
+    v = {2: 5, 4: 10}.get(mt, _DEFAULT_VARIANT[mt])
+    return v, choose_ksplit(m, n, k, variant=v)
+
+
 def skinny_config(m: int, n: int, k: int, fp8: bool = False) -> tuple[int, int]:
-    """(variant, ksplit) for a skinny-GEMM call: the tuned entry, else the defaults."""
+    """(variant, ksplit) for a skinny-GEMM call: the tuned entry, else by rule."""
     tiny = (TUNED_TINY_FP8 if fp8 else TUNED_TINY).get((n, k))
     if tiny is not None and m <= tiny[2]:
         return tiny[:2]
     hit = (TUNED_FP8 if fp8 else TUNED).get((_mt(m), n, k))
     if hit is not None:
         return hit
+    if not fp8:
+        return skinny_rule(m, n, k)
     v = _DEFAULT_VARIANT[_mt(m)]
     return v, choose_ksplit(m, n, k, variant=v)
 
@@ -454,9 +480,8 @@ def skinny_gemm(x: torch.Tensor, w: PackedWeight, out: torch.Tensor | None = Non
     if variant == 0 and ksplit is None:
         variant, ks = skinny_config(m, w.n, k, fp8=w.fp8)
         if rope is not None and SKINNY_VARIANTS[variant][0] != 1:
-            # the RoPE epilogue is built for one-tile waves (R 1): the batch's default variant
-            variant = _DEFAULT_VARIANT[_mt(m)]
-            ks = choose_ksplit(m, w.n, k, variant=variant)
+            # the RoPE epilogue is built for one-tile waves (R 1)
+            variant, ks = skinny_rule(m, w.n, k, one=True)
     else:
         ks = ksplit if ksplit is not None else choose_ksplit(m, w.n, k, variant=variant)
     rps, kpc, mpad = skinny_geometry(m, variant)

@@ -173,7 +173,7 @@ __device__ __forceinline__ bf16x8 dequant8(u32x2 v, float s) {
 // EROPE: the EPI_ROPE instantiation (qkv of the fused decode layer only, so
 // the other projections keep the lean epilogue's registers); its RoPE tables,
 // positions and cache slots are loaded at kernel start, under the main loop.
-// KIN (batch <= 16, MT 1): the four waves share one strip of 16 R rows and
+// KIN (batch <= 64): the four waves share one strip of 16 R rows and
 // split its K range four ways instead of each taking its own rows, so a
 // 4096-row projection fills 256 CUs with no cross-workgroup split-K (the slab
 // stores, the ticket and the last arriver's reduce are ~3-4 us of a 12-14 us
@@ -195,8 +195,8 @@ __global__ __launch_bounds__(256, (MT * KC_ > 32 || R * MT >= 16) ? 1 : 2) void 
   // the only __shared__ object (a second one can make hipcc drain vmcnt before
   // every ds_read, cdna_hip_programming.md s5 trap 4a); the split-K "last
   // arriver" flag reuses its first word after the main loop
-  static_assert(!KIN || (MT == 1 && PF == KC), "KIN: batch <= 16, one ring round per chunk");
-  __shared__ __attribute__((aligned(16))) bf16x8 xs[2][KIN ? 2 * R * 64 : C::CHUNK_SLOTS];
+  static_assert(!KIN || PF == KC, "KIN: one ring round per chunk");
+  __shared__ __attribute__((aligned(16))) bf16x8 xs[2][KIN ? 2 * R * MT * 64 : C::CHUNK_SLOTS];
 
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int nstrip = N / ((KIN ? 16 : 64) * R);
@@ -278,11 +278,15 @@ __global__ __launch_bounds__(256, (MT * KC_ > 32 || R * MT >= 16) ? 1 : 2) void 
     for (int r = 0; r < R; ++r) wf[p][r] = __builtin_nontemporal_load(wrow[r] + (long)min(p, nsteps - 1) * 64);
 
   if constexpr (KIN) {
-    // B fragment of k-step s: lane (column m = lane & 15, k = 8 (lane >> 4) ..)
-    const unsigned short* xr = x + (long)min(lane & 15, M - 1) * ldx + (long)kk0 * 32 + 8 * (lane >> 4);
-    bf16x8 xf[PF];
+    // B fragment of k-step s: lane (column m = 16 c + (lane & 15), k = 8 (lane >> 4) ..)
+    const unsigned short* xr[MT];
 #pragma unroll
-    for (int p = 0; p < PF; ++p) xf[p] = *(const bf16x8*)(xr + p * 32);
+    for (int c = 0; c < MT; ++c) xr[c] = x + (long)min(16 * c + (lane & 15), M - 1) * ldx + (long)kk0 * 32 + 8 * (lane >> 4);
+    bf16x8 xf[PF][MT];
+#pragma unroll
+    for (int p = 0; p < PF; ++p)
+#pragma unroll
+      for (int c = 0; c < MT; ++c) xf[p][c] = *(const bf16x8*)(xr[c] + p * 32);
     for (int s0 = 0; s0 < nsteps; s0 += PF) {
 #pragma unroll
       for (int p = 0; p < PF; ++p) {
@@ -291,12 +295,14 @@ __global__ __launch_bounds__(256, (MT * KC_ > 32 || R * MT >= 16) ? 1 : 2) void 
           bf16x8 wdq;
           if constexpr (W8) wdq = dequant8(wf[p][r], wsc[r]);
           else wdq = wf[p][r];
-          acc[r][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wdq, xf[p], acc[r][0], 0, 0, 0);
+#pragma unroll
+          for (int c = 0; c < MT; ++c) acc[r][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wdq, xf[p][c], acc[r][c], 0, 0, 0);
         }
         const int sn = min(s0 + p + PF, nsteps - 1);
 #pragma unroll
         for (int r = 0; r < R; ++r) wf[p][r] = __builtin_nontemporal_load(wrow[r] + (long)sn * 64);
-        xf[p] = *(const bf16x8*)(xr + sn * 32);
+#pragma unroll
+        for (int c = 0; c < MT; ++c) xf[p][c] = *(const bf16x8*)(xr[c] + sn * 32);
       }
     }
     // the four K quarters of the strip: waves 1-3 hand theirs to wave 0 (slot 0
@@ -304,17 +310,21 @@ __global__ __launch_bounds__(256, (MT * KC_ > 32 || R * MT >= 16) ? 1 : 2) void 
     f32x4v* red = (f32x4v*)&xs[0][1];
     if (w > 0) {
 #pragma unroll
-      for (int r = 0; r < R; ++r) red[((w - 1) * R + r) * 64 + lane] = acc[r][0];
+      for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int c = 0; c < MT; ++c) red[(((w - 1) * R + r) * MT + c) * 64 + lane] = acc[r][c];
     }
     __syncthreads();
     if (w == 0) {
 #pragma unroll
-      for (int r = 0; r < R; ++r) {
-        f32x4v t = acc[r][0];
+      for (int r = 0; r < R; ++r)
 #pragma unroll
-        for (int v = 0; v < 3; ++v) t += red[(v * R + r) * 64 + lane];
-        acc[r][0] = t;
-      }
+        for (int c = 0; c < MT; ++c) {
+          f32x4v t = acc[r][c];
+#pragma unroll
+          for (int v = 0; v < 3; ++v) t += red[((v * R + r) * MT + c) * 64 + lane];
+          acc[r][c] = t;
+        }
     }
   } else {
   load_x(0);
@@ -1386,6 +1396,8 @@ constexpr SkinnyVariant kVariants[] = {
     {2, 8, 2}, {2, 8, 4}, {4, 8, 2}, {1, 8, 4},     // 13-16: M <= 128
     {2, 16, 2}, {1, 16, 4}, {1, 16, 2},             // 17-19: M <= 256
     {1, 1, 8, 1}, {2, 1, 8, 1},                     // 20-21: M <= 16, K split inside the workgroup
+    {1, 2, 8, 1}, {2, 2, 8, 1},                     // 22-23: M <= 32
+    {1, 4, 8, 1}, {2, 4, 8, 1},                     // 24-25: M <= 64
 };
 constexpr int kNumVariants = sizeof(kVariants) / sizeof(kVariants[0]);
 
@@ -1528,6 +1540,14 @@ int skinny_fused(const void* wp, const void* x, void* y, float* ws, int* cnt, in
     case 2 * 20 + 1: return (int)launch_skinny<1, 1, 8, true, true>(wp, x, y, ws, cnt, M, N, K, ldx, ldy, ksplit, cps, ep, s);
     case 2 * 21: return (int)launch_skinny<2, 1, 8, false, true>(wp, x, y, ws, cnt, M, N, K, ldx, ldy, ksplit, cps, ep, s);
     case 2 * 21 + 1: return (int)launch_skinny<2, 1, 8, true, true>(wp, x, y, ws, cnt, M, N, K, ldx, ldy, ksplit, cps, ep, s);
+    case 2 * 22: return (int)launch_skinny<1, 2, 8, false, true>(wp, x, y, ws, cnt, M, N, K, ldx, ldy, ksplit, cps, ep, s);
+    case 2 * 22 + 1: return (int)launch_skinny<1, 2, 8, true, true>(wp, x, y, ws, cnt, M, N, K, ldx, ldy, ksplit, cps, ep, s);
+    case 2 * 23: return (int)launch_skinny<2, 2, 8, false, true>(wp, x, y, ws, cnt, M, N, K, ldx, ldy, ksplit, cps, ep, s);
+    case 2 * 23 + 1: return (int)launch_skinny<2, 2, 8, true, true>(wp, x, y, ws, cnt, M, N, K, ldx, ldy, ksplit, cps, ep, s);
+    case 2 * 24: return (int)launch_skinny<1, 4, 8, false, true>(wp, x, y, ws, cnt, M, N, K, ldx, ldy, ksplit, cps, ep, s);
+    case 2 * 24 + 1: return (int)launch_skinny<1, 4, 8, true, true>(wp, x, y, ws, cnt, M, N, K, ldx, ldy, ksplit, cps, ep, s);
+    case 2 * 25: return (int)launch_skinny<2, 4, 8, false, true>(wp, x, y, ws, cnt, M, N, K, ldx, ldy, ksplit, cps, ep, s);
+    case 2 * 25 + 1: return (int)launch_skinny<2, 4, 8, true, true>(wp, x, y, ws, cnt, M, N, K, ldx, ldy, ksplit, cps, ep, s);
     default: return KGS_ERR_ARG;
   }
 }

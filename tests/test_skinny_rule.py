@@ -1,0 +1,66 @@
+"""Skinny GEMM variants by rule: launchable over sizes, and the forms with the K split inside the
+workgroup for up to 64 rows."""
+from __future__ import annotations
+
+import pytest
+import torch
+
+from kgs.ops import decode as D
+
+DEV = "cuda"
+
+
+def test_rule_is_launchable():
+    for m in (1, 16, 17, 32, 33, 40, 48, 64):
+        for n in (64, 128, 1280, 2048, 4096, 4160, 6144, 6208, 16384):
+            for k in (512, 1024, 1536, 2048, 4096, 5120, 8192, 9216):
+                for one in (False, True):
+                    v, ks = D.skinny_rule(m, n, k, one)
+                    rps, kpc, _ = D.skinny_geometry(m, v)
+                    if n % 64 == 0 and k % 512 == 0:  # what callers pack weights of
+                        assert n % rps == 0 and k % kpc == 0 and (k // kpc) % ks == 0, (m, n, k, v, ks)
+                    assert not one or D.SKINNY_VARIANTS[v][0] == 1 or m > 64
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,v", [(17, 22), (32, 22), (24, 23), (33, 24), (64, 24), (40, 25)])
+def test_k_split_in_the_workgroup(m, v):
+    """Against fp32 for every epilogue: plain, split, RMS + SwiGLU, residual with its sums of squares, and
+    (one-tile waves) RoPE with the cache write, whose bits are the plain output's through rope_cache_."""
+    from kgs.ops.transformer import rope_tables
+
+    torch.manual_seed(m)
+    n, k = 512, 2048
+    x = torch.randn(m, k, device=DEV).bfloat16()
+    w = (torch.randn(n, k, device=DEV) * k ** -0.5).bfloat16()
+    ref = x.float() @ w.float().T
+    # fp32 sums of k exact products (k 2^-24 of their magnitudes) and one rounding to bf16
+    tol = k * 2.0 ** -24 * (x.float().abs() @ w.float().abs().T) + 2.0 ** -8 * ref.abs()
+    pw = D.PackedWeight(w)
+    for ks in (1, 2):
+        y = D.skinny_gemm(x, pw, variant=v, ksplit=ks).float()
+        assert bool(((y - ref).abs() <= tol).all())
+        res = torch.randn(m, n, device=DEV).bfloat16()
+        old, ss = res.float(), torch.zeros(m, device=DEV)
+        D.skinny_gemm(x, pw, out=res, resid_ss=ss, variant=v, ksplit=ks)
+        assert bool(((res.float() - old - ref).abs() <= tol + 2.0 ** -8 * (old + ref).abs()).all())
+        torch.testing.assert_close(ss, res.float().pow(2).sum(-1), rtol=1e-4, atol=1e-3)
+    ss = x.float().pow(2).sum(-1).contiguous()
+    wide = (torch.randn(2 * n, k, device=DEV) * k ** -0.5).bfloat16()
+    xn = x.float() * torch.rsqrt(ss / k + 1e-5)[:, None]
+    g, u = xn @ wide[:n].float().T, xn @ wide[n:].float().T
+    got = D.skinny_gemm(x, D.PackedWeight(wide, swiglu=True, fold=torch.ones(k, device=DEV)), rms=ss, variant=v, ksplit=1)
+    torch.testing.assert_close(got.float(), torch.nn.functional.silu(g) * u, rtol=2e-2, atol=1e-3)
+    if D.SKINNY_VARIANTS[v][0] != 1:
+        return
+    heads, kv = 4, 2
+    wq = (torch.randn((heads + 2 * kv) * 128, k, device=DEV) * k ** -0.5).bfloat16()
+    one = torch.ones(k, device=DEV)
+    cos, sin = rope_tables(256, 128, 1e4, DEV)
+    pos, slot = torch.arange(m, device=DEV, dtype=torch.int32) * 3, torch.arange(m, device=DEV, dtype=torch.int32) - 1
+    ca, cb = (torch.zeros(4, kv, 2, 4096, device=DEV, dtype=torch.bfloat16) for _ in range(2))
+    q1 = D.skinny_gemm(x, D.PackedWeight(wq, fold=one), rms=ss, variant=v, ksplit=1)
+    D.rope_cache_(q1, cos, sin, pos, slot, ca, heads, kv)
+    q2 = D.skinny_gemm(x, D.PackedWeight(wq, fold=one, rope=(heads, kv)), rms=ss, variant=v, ksplit=1,
+                       rope={"cos": cos, "sin": sin, "positions": pos, "slots": slot, "cache": cb})
+    assert torch.equal(q1, q2) and torch.equal(ca, cb)

@@ -6,8 +6,7 @@ library's ``libamdhip64.so.7`` dependency resolves (by SONAME) to the HIP runtim
 torch already loaded -- one HIP runtime per process, shared streams.
 
 There is deliberately no silent fallback: on a machine with a GPU, a missing or
-unloadable library raises ``NativeUnavailable`` (the driver checks that the
-native code is what runs).
+unloadable library raises ``NativeUnavailable``.
 """
 from __future__ import annotations
 
@@ -221,9 +220,14 @@ def check(rc: int, what: str) -> None:
 
 
 def stream_handle(device=None) -> int:
+    """The current stream of ``device`` as a raw handle. Tensors of a device mean that it is set up, so
+    the Stream object that torch would make of it (2 us a launch) is left out."""
     import torch
 
-    return torch.cuda.current_stream(device).cuda_stream
+    index = getattr(device, "index", None)
+    if index is None:
+        return torch.cuda.current_stream(device).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(index)
 
 
 def tile_queue_stats(device: int = 0) -> dict:

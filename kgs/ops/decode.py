@@ -593,15 +593,15 @@ def rope_cache_(qkv: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, positio
     t = qkv.shape[0]
     if rows is not None:
         t = rows.numel()
-        if rows.dtype != torch.int32 or not rows.is_contiguous() or partials is not None:
-            raise ValueError("rows must be a contiguous int32 vector, without partials")
+        if rows.dtype != torch.int32 or not rows.is_contiguous():
+            raise ValueError("rows must be a contiguous int32 vector")
     if qkv.dtype != torch.bfloat16 or not qkv.is_cuda or qkv.stride(1) != 1:
         raise ValueError("qkv must be a row-major bf16 GPU matrix")
     nslice = 0
     if partials is not None:
         if partials.dtype != torch.float32 or partials.dim() != 3 or not partials.is_contiguous() or \
-                tuple(partials.shape[1:]) != (t, (heads + 2 * kv_heads) * HEAD_DIM):
-            raise ValueError("partials must be contiguous fp32 [nslice, T, (H + 2 HKV) * 128]")
+                tuple(partials.shape[1:]) != (qkv.shape[0], (heads + 2 * kv_heads) * HEAD_DIM):
+            raise ValueError("partials must be contiguous fp32 [nslice, rows of qkv, (H + 2 HKV) * 128]")
         nslice = partials.shape[0]
     for v, name in ((positions, "positions"), (slots, "slots")):
         if v.dtype != torch.int32 or not v.is_contiguous() or v.numel() != t:
@@ -615,7 +615,8 @@ def rope_cache_(qkv: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, positio
                                         slots.data_ptr(), cache_layer.data_ptr(), t, heads, kv_heads, HEAD_DIM,
                                         qkv.stride(0), 1 if cache_layer.dtype == FP8 else 0,
                                         None if partials is None else partials.data_ptr(), nslice,
-                                        None if rows is None else rows.data_ptr(), _lib.stream_handle(qkv.device))
+                                        None if rows is None else rows.data_ptr(), qkv.shape[0],
+                                        _lib.stream_handle(qkv.device))
     _lib.check(rc, "rope_cache")
     return qkv
 

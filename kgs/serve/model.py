@@ -258,14 +258,23 @@ class ServingModel:
         r = D.w4x_route(m, w.shape[0], w.shape[1])
         return D.w4x_rule(m, w.shape[0], w.shape[1]) if r is None else r if r[1] == 1 else None
 
-    def _split_proj(self, x, layer: int, name: str, r):
-        """fp32 partial products of a decode projection along route ``r``; a size without measured
-        entries gets a buffer of the call's own."""
+    def _split_proj(self, x, layer: int, name: str, r, private: bool = False):
+        """fp32 partial products of a projection along route ``r``, in a buffer of the call's own if
+        ``private`` (prompts) and for a size without measured entries."""
         from kgs.ops.gemm import gemm_nt_w4x_partials
 
         w = self.w[layer][name]
         return gemm_nt_w4x_partials(x, self._w4x_weight(layer, name, r[0]), *r, nt_weights=D.w4x_nt(r),
-                                    private=D.w4x_route(x.shape[0], *w.shape) is None)
+                                    private=private or D.w4x_route(x.shape[0], *w.shape) is None)
+
+    def _gate_up_split(self, y, layer: int, r):
+        """gate|up and SwiGLU along route ``r`` of :meth:`_swiglu_route`."""
+        from kgs.ops.gemm import gemm_nt_w4x_splitk_swiglu, gemm_nt_w4x_swiglu
+
+        if r[1] > 1:
+            return gemm_nt_w4x_splitk_swiglu(y, self.w[layer]["gate_up"], r[0], r[1], r[2], nt_weights=D.w4x_nt(r), private=True)
+        return gemm_nt_w4x_swiglu(y, self._gate_up_weight(layer, r[0]), bn=r[0], bm=r[2], stages=D.w4x_stages(r),
+                                  nt_weights=D.w4x_nt(r))
 
     def _norm(self, x, d, w):
         """x += d (in place, bf16) and return rmsnorm(x) * w."""
@@ -333,19 +342,40 @@ class ServingModel:
         x = self.embed[tokens.long()].reshape(-1, h).contiguous()
         y = self._norm(x, None, self.ln1[0])
         T.op("prefill embed+norm")
+        m = x.shape[0]
+        # few rows: the decode step's split tiles, whose sums the rotation, norms and gate take (one
+        # prompt of 90 tokens at hidden 4096: 703 us by the general kernel and its own sums, 635 so)
+        few = m <= D.W4X_RULE_MAX
+        rq, ro, rd = (self._splitk_route(m, 0, n) if few else None for n in ("qkv", "o", "down"))
+        rg = self._swiglu_route(m) if few else None
+        if ro or rd:
+            from kgs.ops.transformer import splitk_add_rmsnorm
         for i in range(c.layers):
-            qkv = self._proj(y, i, "qkv", False)
-            T.op(f"prefill L{i} qkv")
-            self._rope_cache(qkv, i, positions, slots, plan.rows)
+            if rq:
+                part = self._split_proj(y, i, "qkv", rq, True)
+                qkv = torch.empty((m, part.shape[2]), dtype=torch.bfloat16, device=x.device)
+                T.op(f"prefill L{i} qkv")
+                D.rope_cache_(qkv, self.cos, self.sin, positions, slots, self.cache.layer(i), c.heads, c.kv_heads,
+                              partials=part, rows=plan.rows)
+            else:
+                qkv = self._proj(y, i, "qkv", False)
+                T.op(f"prefill L{i} qkv")
+                self._rope_cache(qkv, i, positions, slots, plan.rows)
             T.op(f"prefill L{i} rope_cache")
             a = self._prefill_attention(qkv, seq_starts, seq_lens, padded_lens, plan.items)
             T.op(f"prefill L{i} attention")
-            y = self._proj_add_norm(a, i, "o", x, self.ln2[i])
+            if ro:
+                y = splitk_add_rmsnorm(self._split_proj(a, i, "o", ro, True), x, self.ln2[i], c.eps)
+            else:
+                y = self._proj_add_norm(a, i, "o", x, self.ln2[i])
             T.op(f"prefill L{i} o+norm")
-            act = self._gate_up_act(y, i)
+            act = self._gate_up_split(y, i, rg) if rg else self._gate_up_act(y, i)
             T.op(f"prefill L{i} gate_up")
             nxt = self.ln1[i + 1] if i + 1 < c.layers else self.norm
-            y = self._proj_add_norm(act, i, "down", x, nxt)
+            if rd:
+                y = splitk_add_rmsnorm(self._split_proj(act, i, "down", rd, True), x, nxt, c.eps)
+            else:
+                y = self._proj_add_norm(act, i, "down", x, nxt)
             T.op(f"prefill L{i} down+norm")
         yl = y[plan.last].contiguous()
         out = self._proj(yl, None, "lm", True)
@@ -576,8 +606,7 @@ class ServingModel:
         m = x.shape[0]
         rq, ro, rd = (self._splitk_route(m, 0, n) for n in ("qkv", "o", "down"))  # same shapes in every layer
         rg = self._swiglu_route(m)
-        if rq or ro or rd or rg:
-            from kgs.ops.gemm import gemm_nt_w4x_splitk_swiglu, gemm_nt_w4x_swiglu
+        if ro or rd:
             from kgs.ops.transformer import splitk_add_rmsnorm
         # split-K qkv with KGS_ROPE_ATTN=1: its reduce + RoPE + KV write run
         # inside the attention launch (one launch per layer fewer)
@@ -614,12 +643,8 @@ class ServingModel:
             else:
                 y = self._norm(x, self._proj(a, i, "o", True), self.ln2[i])
             T.op(f"decode L{i} o+norm")
-            if rg and rg[1] > 1:
-                act = gemm_nt_w4x_splitk_swiglu(y, self.w[i]["gate_up"], rg[0], rg[1], rg[2], nt_weights=D.w4x_nt(rg),
-                                                private=True)
-            elif rg:
-                act = gemm_nt_w4x_swiglu(y, self._gate_up_weight(i, rg[0]), bn=rg[0], bm=rg[2],
-                                         stages=D.w4x_stages(rg), nt_weights=D.w4x_nt(rg))
+            if rg:
+                act = self._gate_up_split(y, i, rg)
             else:
                 act = self._silu_mul(self._proj(y, i, "gate_up", True))
             T.op(f"decode L{i} gate_up")

@@ -571,7 +571,7 @@ __global__ __launch_bounds__(256) void rope_cache(unsigned short* __restrict__ q
                                                   const int* __restrict__ slot, void* __restrict__ cache,
                                                   long tokens, int H, int HKV, long ld,
                                                   const float* __restrict__ P = nullptr, int nslice = 0,
-                                                  const int* __restrict__ rows = nullptr) {
+                                                  const int* __restrict__ rows = nullptr, long prows = 0) {
   const int nh = H + 2 * HKV;
   const long idx = (long)blockIdx.x * 256 + threadIdx.x;
   if (idx >= tokens * nh * 8) return;
@@ -589,7 +589,7 @@ __global__ __launch_bounds__(256) void rope_cache(unsigned short* __restrict__ q
   const int sl = slot[t];
   bf16x8 a, b;
   if constexpr (SK) {
-    const long MN = tokens * nh * HD, e = t * nh * HD + (long)h * HD + 8 * c;
+    const long MN = prows * nh * HD, e = row * nh * HD + (long)h * HD + 8 * c;
     f32x4 s[4];
     if constexpr (NSL > 0) {
       f32x4 ps[NSL][4];
@@ -1574,17 +1574,17 @@ KGS_EXPORT int kgs_skinny_gemm_bf16(const void* wp, const void* x, void* y, floa
 // [pages][HKV][2][4096] bf16. q and k are rotated in place; k, v land in the cache.
 // kv8: the cache holds e4m3 bytes ([pages][HKV][2][4096] B) instead of bf16.
 // P != nullptr: the projection is given as nslice fp32 split-K partials
-// [nslice][tokens][(H + 2 HKV) * hd] instead of in qkv; the reduced, rotated
+// [nslice][prows][(H + 2 HKV) * hd] instead of in qkv (prows: its rows, tokens without a map); the reduced, rotated
 // rows are written to qkv (which is then output only).
-// rows != nullptr (without P): token t is row rows[t] of qkv, none where negative: prompts padded
+// rows != nullptr: token t is row rows[t] of qkv, none where negative: prompts padded
 // to whole pages whose padding has no rows, so that a page's run still leaves in 16-byte chunks.
 KGS_EXPORT int kgs_rope_cache_bf16(void* qkv, const float* cosv, const float* sinv, const int* pos, const int* slot,
                                   void* cache, long tokens, int H, int HKV, int hd, long ld, int kv8, const float* P,
-                                  int nslice, const int* rows, hipStream_t s) {
+                                  int nslice, const int* rows, long prows, hipStream_t s) {
   if (tokens < 0 || H <= 0 || HKV <= 0 || H % HKV || hd != kgs::dec::HD) return KGS_ERR_SHAPE;
   if (ld < (long)(H + 2 * HKV) * hd) return KGS_ERR_SHAPE;
   if (!al16(qkv) || !al16(cosv) || !al16(sinv) || !al16(cache) || ld % 8) return KGS_ERR_ALIGN;
-  if (P != nullptr && (nslice <= 0 || !al16(P) || rows != nullptr)) return KGS_ERR_ARG;
+  if (P != nullptr && (nslice <= 0 || !al16(P) || prows <= 0 || (!rows && prows != tokens))) return KGS_ERR_ARG;
   const long n = tokens * (H + 2 * HKV) * 8;
   if (n == 0) return 0;
   const dim3 g((unsigned)((n + 255) / 256)), b(256);
@@ -1592,7 +1592,7 @@ KGS_EXPORT int kgs_rope_cache_bf16(void* qkv, const float* cosv, const float* si
   if (P != nullptr) {
 #define KGS_RCS(KV, NSL)                                                                                           \
   hipLaunchKernelGGL((kgs::dec::rope_cache<KV, true, NSL>), g, b, 0, s, q, cosv, sinv, pos, slot, cache, tokens, H, \
-                     HKV, ld, P, nslice, nullptr)
+                     HKV, ld, P, nslice, rows, prows)
 #define KGS_RCS_KV(KV)                \
   switch (nslice) {                   \
     case 2: KGS_RCS(KV, 2); break;    \

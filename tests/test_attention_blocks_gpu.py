@@ -128,6 +128,14 @@ def test_rope_rows_match_padded(lens, cache_dtype):
     D.rope_cache_(full, cos, sin, pos, slot, ca, heads, kv)
     D.rope_cache_(qkv, cos, sin, pos, slot, cb, heads, kv, rows=rows)
     assert torch.equal(qkv, full[rows >= 0]) and torch.equal(ca.view(torch.uint8), cb.view(torch.uint8))
+    # rows that arrive as partial sums
+    parts = torch.randn(4, real, qkv.shape[1], device=DEV)
+    whole = parts[0] + parts[1] + parts[2] + parts[3]
+    qa, qb = whole.bfloat16(), torch.empty_like(qkv)
+    cc, cd = (torch.zeros_like(ca) for _ in range(2))
+    D.rope_cache_(qa, cos, sin, pos, slot, cc, heads, kv, rows=rows)
+    D.rope_cache_(qb, cos, sin, pos, slot, cd, heads, kv, partials=parts, rows=rows)
+    assert torch.equal(qa, qb) and torch.equal(cc.view(torch.uint8), cd.view(torch.uint8))
 
 
 @pytest.mark.gpu

@@ -164,14 +164,15 @@ enum Epi { EPI_NONE = 0, EPI_BIAS = 1, EPI_BIAS_GELU = 2, EPI_BIAS_RELU = 3, EPI
 template <int EPI>
 constexpr bool epi_bias() { return EPI != EPI_NONE && EPI != EPI_ADDC; }
 
+// x (1 + tanh u) / 2 with u = k0 (x + k1 x^3), as x sigmoid(2 u): five products, v_exp and v_rcp
+// (1 ulp; u = -inf .. inf give sigmoid 0 .. 1) instead of two precise divisions' worth, and no
+// cancellation of 1 + tanh on the negative side. 64 values per thread at the end of a GEMM's tile are
+// several us that nothing overlaps: 1000 x 3000 x 1032 17.8 us by tanh, 15.8 so; with its
+// gradient a training step of 8192 rows, 4096 - 14336 - 4096, 4.52 ms against 4.41.
 __device__ __forceinline__ float gelu_tanh(float x) {
-  const float k0 = 0.7978845608028654f, k1 = 0.044715f;
-  float u = k0 * (x + k1 * x * x * x);
-  // tanh via exp: stable for |u| large.
-  float e = __expf(-2.0f * fabsf(u));
-  float t = (1.0f - e) / (1.0f + e);
-  t = u < 0.f ? -t : t;
-  return 0.5f * x * (1.0f + t);
+  constexpr float A = -2.0f * 1.4426950408889634f * 0.7978845608028654f, B = A * 0.044715f;
+  const float e = __builtin_amdgcn_exp2f(x * __builtin_fmaf(B, x * x, A));
+  return x * __builtin_amdgcn_rcpf(1.0f + e);
 }
 
 // activation of a gated feed-forward: 1 silu, 2 tanh gelu of the gate, times up;

@@ -31,9 +31,10 @@ __device__ __forceinline__ float grad(float g, float z) {
     return g * s * (1.0f + z * (1.0f - s));
   }
   if constexpr (ACT == ACT_GELU) {
+    // with s = sigmoid(2 u) from e = exp(-2 |u|): (1 + tanh u) / 2 = s, (1 - tanh^2 u) / 2 = 2 e / (1 + e)^2
     const float k0 = 0.7978845608028654f, k1 = 0.044715f, q = z * z, u = k0 * z * (1.0f + k1 * q);
-    const float e = __expf(-2.0f * fabsf(u)), ta = (1.0f - e) / (1.0f + e), t = u < 0.f ? -ta : ta;
-    return g * (0.5f * (1.0f + t) + 0.5f * z * (1.0f - t * t) * k0 * (1.0f + 3.0f * k1 * q));
+    const float e = __expf(-2.0f * fabsf(u)), r = __builtin_amdgcn_rcpf(1.0f + e), er = e * r;
+    return g * ((u < 0.f ? er : r) + z * (2.0f * er * r) * (k0 * (1.0f + 3.0f * k1 * q)));
   }
   return g;
 }

@@ -5,7 +5,7 @@
 //   C[M, N] = epilogue(A[M, K] . B[N, K]^T + bias)
 //
 // What bounds such a product is the number of CUs that get a tile and the length of one
-// workgroup's serial chain of K-steps, so the tile (256x256, 256x128 or 128x128) and the number
+// workgroup's serial chain of K-steps, so the tile (256x256, 256x128, 128x128 or 64x64) and the number
 // of K slices are chosen by sizes (any_plan below). 128x128 tiles keep a quarter of the AGPRs, so
 // two workgroups share a CU and one's barriers and loads hide behind the other's MFMAs.
 //
@@ -75,6 +75,56 @@ __device__ __forceinline__ void store8(unsigned short* row, int col, int N, int 
 #pragma unroll
   for (int e = 0; e < 8; ++e)
     if (col + e < N) row[col + e] = (unsigned short)(u[e >> 1] >> (16 * (e & 1)));
+}
+
+// A lane's part of a tile's rows: NB fragments of 16 columns, four of each from `col`
+template <int EPI, int NB>
+__device__ __forceinline__ void load_bias(const Args& a, int col, float (&bv)[NB][4]) {
+#pragma unroll
+  for (int n = 0; n < NB; ++n)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      bv[n][e] = 0.f;
+      if constexpr (epi_bias<EPI>())
+        if (a.bias && col + n * 16 + e < a.N) bv[n][e] = bf2f(a.bias[col + n * 16 + e]);
+    }
+}
+// EPI_ADDC's old values, 8 columns from `col` of each fragment pair (N % 8 == 0 and 16-B rows)
+template <int EPI, int NB>
+__device__ __forceinline__ void load_old(const Args& a, int r, int col, uint4 (&old)[NB / 2]) {
+  if constexpr (EPI == EPI_ADDC) {
+    const unsigned short* crow = (const unsigned short*)a.C + (long)r * a.ldc;
+#pragma unroll
+    for (int p = 0; p < NB / 2; ++p)
+      old[p] = r < a.M && col + p * 32 < a.N ? *(const uint4*)(crow + col + p * 32) : make_uint4(0, 0, 0, 0);
+  }
+}
+// Row r of a tile through the epilogue; `col` as in load_old
+template <int EPI, int NB, bool DUAL>
+__device__ __forceinline__ void store_row(const Args& a, int r, int col, const f32x4 (&v)[NB], const float (&bv)[NB][4],
+                                          const uint4 (&old)[NB / 2]) {
+  unsigned short* crow = (unsigned short*)a.C + (long)r * a.ldc;
+#pragma unroll
+  for (int n = 0; n < NB; n += 2) {
+    uint2 o[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      constexpr int E = DUAL ? EPI_BIAS : EPI;
+      o[h].x = pack_epi<E>(v[n + h][0], v[n + h][1], bv[n + h][0], bv[n + h][1]);
+      o[h].y = pack_epi<E>(v[n + h][2], v[n + h][3], bv[n + h][2], bv[n + h][3]);
+    }
+    auto sx = __builtin_amdgcn_permlane16_swap(o[0].x, o[1].x, false, false);
+    auto sy = __builtin_amdgcn_permlane16_swap(o[0].y, o[1].y, false, false);
+    uint4 q = make_uint4(sx[0], sy[0], sx[1], sy[1]);
+    const int c = col + n * 16;
+    if (r < a.M && c < a.N) {
+      if constexpr (EPI == EPI_ADDC) q = add_bf16x8(old[n / 2], q);
+      store8(crow, c, a.N, a.vec, q);
+      if constexpr (DUAL)
+        store8(a.C2 + (long)r * a.ldc, c, a.N, a.vec,
+               make_uint4(act_pair<EPI>(q.x), act_pair<EPI>(q.y), act_pair<EPI>(q.z), act_pair<EPI>(q.w)));
+    }
+  }
 }
 
 // SW (a GateAct): B is a fused gate|up weight of N rows, gate rows first, and C [M, N / 2] holds
@@ -208,54 +258,91 @@ void gemm_nt_any(Args a) {
     return;
   }
   float bv[NB][4];
-#pragma unroll
-  for (int n = 0; n < NB; ++n) {
-#pragma unroll
-    for (int e = 0; e < 4; ++e) bv[n][e] = 0.f;
-    if constexpr (epi_bias<EPI>()) {
-      const int col = nw + n * 16 + fq * 4;
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        if (a.bias && col + e < a.N) bv[n][e] = bf2f(a.bias[col + e]);
-    }
-  }
+  load_bias<EPI, NB>(a, nw + fq * 4, bv);
   w4::static_for<0, MA>([&](auto ic) {
     constexpr int i = decltype(ic)::value;
     const int r = mw + i * 16;
-    const bool row_ok = r < a.M;
-    unsigned short* crow = (unsigned short*)a.C + (long)r * a.ldc;
     uint4 old[NB / 2];
-    if constexpr (EPI == EPI_ADDC) {  // N % 8 == 0 and 16-B rows (kgs_gemm_bf16_nt_any)
-#pragma unroll
-      for (int p = 0; p < NB / 2; ++p) {
-        const int col = nw + p * 32 + lc;
-        old[p] = row_ok && col < a.N ? *(const uint4*)(crow + col) : make_uint4(0, 0, 0, 0);
-      }
-    }
+    load_old<EPI, NB>(a, r, nw + lc, old);
     f32x4 v[NB];
     w4::read_row<NB, i>(v);
-#pragma unroll
-    for (int n = 0; n < NB; n += 2) {
-      uint2 o[2];
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        constexpr int E = DUAL ? EPI_BIAS : EPI;
-        o[h].x = pack_epi<E>(v[n + h][0], v[n + h][1], bv[n + h][0], bv[n + h][1]);
-        o[h].y = pack_epi<E>(v[n + h][2], v[n + h][3], bv[n + h][2], bv[n + h][3]);
-      }
-      auto sx = __builtin_amdgcn_permlane16_swap(o[0].x, o[1].x, false, false);
-      auto sy = __builtin_amdgcn_permlane16_swap(o[0].y, o[1].y, false, false);
-      uint4 q = make_uint4(sx[0], sy[0], sx[1], sy[1]);
-      const int col = nw + n * 16 + lc;
-      if (row_ok && col < a.N) {
-        if constexpr (EPI == EPI_ADDC) q = add_bf16x8(old[n / 2], q);
-        store8(crow, col, a.N, a.vec, q);
-        if constexpr (DUAL)
-          store8(a.C2 + (long)r * a.ldc, col, a.N, a.vec,
-                 make_uint4(act_pair<EPI>(q.x), act_pair<EPI>(q.y), act_pair<EPI>(q.z), act_pair<EPI>(q.w)));
-      }
-    }
+    store_row<EPI, NB, DUAL>(a, r, nw + lc, v, bv, old);
   });
+}
+
+// The same product on 64x64 tiles, for grids that leave CUs idle at 128x128. What bounds such a
+// launch is each workgroup's chain of K-steps; a step of this tile takes 0.27 us against 0.36 (LDS
+// traffic: half the bytes), and four times the workgroups share the epilogue. Four stages of 64-wide
+// K-tiles keep three on their way with one barrier per step (eight: the same time; 64x128 tiles with
+// three stages 0.44 us a step). Accumulators are plain registers, in gemm_w4.h's order of products per
+// element: bitwise the larger tiles' results. us, 128x128 / here: 1024^3 9.4 / 7.4, 256 x 3072 x 2048 15.1 /
+// 11.6, 128 x 5757 x 2080 19.8 / 13.5, 168 x 1760 x 1032 9.7 / 7.2.
+template <int EPI, bool DUAL>
+__global__ __launch_bounds__(256) void gemm_small(Args a) {
+  constexpr int BM = 64, BN = 64, ST = 4;
+  constexpr int FM = BM / 32, FN = BN / 32, LA = BM / 32, LB = BN / 32, STAGE = (BM + BN) * 128;
+  __shared__ __attribute__((aligned(1024))) char smem[ST * STAGE];
+  const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int ntm = (a.M + BM - 1) / BM, ntn = (a.N + BN - 1) / BN;
+  int none, tm, tn;
+  w4::tile_of<0, false>((int)blockIdx.x, (int)gridDim.x, ntm, ntn, none, tm, tn);
+  const int m0 = tm * BM, n0 = tn * BN, K = a.K, nt = (K + BK - 1) / BK;
+  const int na = min(a.M - m0, BM), nb = min(a.N - n0, BN);
+  const auto ra = __builtin_amdgcn_make_buffer_rsrc((void*)(a.A + (long)m0 * a.lda), 0, ((na - 1) * a.lda + K) * 2, 0x00020000);
+  const auto rb = __builtin_amdgcn_make_buffer_rsrc((void*)(a.B + (long)n0 * a.ldb), 0, ((nb - 1) * a.ldb + K) * 2, 0x00020000);
+  const int row = w * 8 + (lane >> 3), ch = ((lane & 7) ^ ((row >> 1) & 7)) * 8;
+  const int va = (row * a.lda + ch) * 2, vb = (row * a.ldb + ch) * 2, sa = 64 * a.lda, sb = 64 * a.ldb;
+  auto load = [&](int t) {  // K-tile t (zeros past K) into its stage
+    char* dst = smem + (t % ST) * STAGE;
+    const bool in = t * BK + ch < K;
+    const int oa = in ? va : OOB, ob = in ? vb : OOB;
+#pragma unroll
+    for (int j = 0; j < LA; ++j)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (KGS_LDS void*)(dst + (j * 4 + w) * 1024), 16, oa, j * sa + t * 128, 0, 0);
+#pragma unroll
+    for (int j = 0; j < LB; ++j)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (KGS_LDS void*)(dst + BM * 128 + (j * 4 + w) * 1024), 16, ob, j * sb + t * 128, 0, 0);
+  };
+  const int fr = lane & 15, fq = lane >> 4;
+  const int ro = fr * 128 + ((fq ^ (fr >> 1)) * 16);
+  const int pa = (w >> 1) * (BM / 2) * 128 + ro, pb = BM * 128 + (w & 1) * (BN / 2) * 128 + ro;
+  f32x4 acc[FM][FN];
+#pragma unroll
+  for (int i = 0; i < FM; ++i)
+#pragma unroll
+    for (int n = 0; n < FN; ++n) acc[i][n] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int t = 0; t < ST - 1; ++t) load(t);
+  for (int t = 0; t < nt; ++t) {
+    w4::wait_vm<(ST - 2) * (LA + LB)>();  // own part of K-tile t
+    w4::bar();  // every wave's part, and every wave has read K-tile t - 1
+    load(t + ST - 1);
+    const char* st = smem + (t % ST) * STAGE;
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+      bf16x8 fa[FM], fb[FN];
+#pragma unroll
+      for (int i = 0; i < FM; ++i) fa[i] = *(const bf16x8*)(st + ((pa + i * 2048) ^ (ks * 64)));
+#pragma unroll
+      for (int n = 0; n < FN; ++n) fb[n] = *(const bf16x8*)(st + ((pb + n * 2048) ^ (ks * 64)));
+#pragma unroll
+      for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int n = 0; n < FN; ++n) acc[i][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[n], fa[i], acc[i][n], 0, 0, 0);
+    }
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the tail's loads land before LDS is released
+  const int mw = m0 + (w >> 1) * (BM / 2) + fr, nw = n0 + (w & 1) * (BN / 2);
+  const int lc = (fq & 1) * 16 + (fq >> 1) * 8;
+  float bv[FN][4];
+  load_bias<EPI, FN>(a, nw + fq * 4, bv);
+#pragma unroll
+  for (int i = 0; i < FM; ++i) {
+    uint4 old[FN / 2];
+    load_old<EPI, FN>(a, mw + i * 16, nw + lc, old);
+    store_row<EPI, FN, DUAL>(a, mw + i * 16, nw + lc, acc[i], bv, old);
+  }
 }
 
 // Products with operands stored K-major (A as [K, M], B as [K, N]): Linear's backward pass, whose
@@ -544,6 +631,9 @@ inline Plan plan(long M, long N, long K, bool split, int cus) {
         best = {s[0], s[1], ns};
       }
     }
+  // 64x64 tiles: a cheaper step, twice as many bytes per product; several share a CU
+  const double full = (double)ceil_div(M, 64) * ceil_div(N, 64) / cus;
+  if (3.5 + ceil_div(K, 64) * (full <= 1 ? 0.34 + 0.06 * full : 0.06 + 0.38 * full) < t0) best = {64, 64, 1};
   return best;
 }
 
@@ -595,6 +685,10 @@ void launch_tile(const Args& a, int ns, hipStream_t s) {
 
 template <int EPI, bool DUAL>
 int launch(Args a, Plan p, float* ws, hipStream_t s) {
+  if (p.bm == 64) {
+    hipLaunchKernelGGL((gemm_small<EPI, DUAL>), dim3((unsigned)(ceil_div(a.M, 64) * ceil_div(a.N, 64))), dim3(256), 0, s, a);
+    return (int)hipGetLastError();
+  }
   Args g = a;
   const int ldp = (a.N + 7) / 8 * 8;
   g.ks = ceil_div(ceil_div(a.K, 128), p.ns) * 128;
@@ -701,7 +795,7 @@ int gemm_any_swiglu(const void* A, const void* B, void* C, int M, int N, int K, 
   const Args a{(const unsigned short*)A, (const unsigned short*)B, C, nullptr, (const unsigned short*)limit,
                M, N, K, lda, ldb, ldc, 0, M > N, ldc % 8 == 0 && (uintptr_t)C % 16 == 0};
   const Plan p = plan(M, N, K, false, cu_count());
-  const int bm = p.bm, bn = bm == 256 && p.bn == 256 ? 256 : 128;
+  const int bm = p.bm == 256 ? 256 : 128, bn = bm == 256 && p.bn == 256 ? 256 : 128;
   const dim3 grid((unsigned)(ceil_div(M, bm) * ceil_div(N / 2, bn / 2)));
 #define KGS_SWT(ACT)                                                                                                 \
   if (bm == 128) hipLaunchKernelGGL((gemm_nt_any<EPI_NONE, 128, 128, false, false, ACT>), grid, dim3(256), 0, s, a); \

@@ -446,7 +446,9 @@ KGS_EXPORT int kgs_gemm_bf16_nt_any(const void* A, const void* B, void* C, const
                                     hipStream_t stream) {
   if (M <= 0 || N <= 0 || K <= 0 || lda < K || ldb < K || ldc < N) return KGS_ERR_SHAPE;
   if (epi < 0 || epi > kgs::EPI_BIAS_SILU || (epi != kgs::EPI_NONE && !bias)) return KGS_ERR_ARG;
-  if (!((bm == 256 && (bn == 256 || bn == 128)) || (bm == 128 && bn == 128)) || ns < 1 || ns > 64) return KGS_ERR_ARG;
+  const bool large = (bm == 256 && (bn == 256 || bn == 128)) || (bm == 128 && bn == 128);
+  const bool small = bm == 64 && bn == 64 && ns == 1;
+  if (!(large || small) || ns < 1 || ns > 64) return KGS_ERR_ARG;
   if (!kgs::gemm_any_ok(A, B, M, N, K, lda, ldb) || (uintptr_t)ws % 16) return KGS_ERR_ALIGN;
   return kgs::gemm_any(A, B, C, nullptr, bias, M, N, K, lda, ldb, ldc, epi, bm, bn, ns, ws, stream);
 }

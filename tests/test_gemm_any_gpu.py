@@ -258,3 +258,42 @@ def test_linear_odd_sizes(rows, din, dout, frozen):
     for t, w in zip((x, lin.weight, lin.bias), want):
         if t.requires_grad:
             assert rel(t.grad, w) < 8 * REL  # as test_linear_training_step
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 8, 8), (64, 64, 64), (65, 63, 72), (130, 200, 1032), (63, 257, 320), (320, 128, 200)])
+@pytest.mark.parametrize("epi", [0, 1, 2, 4])
+def test_small_tiles_keep_the_bits(M, N, K, epi):
+    """64x64 tiles against 128x128 ones: the same products in the same order, every epilogue, edges of
+    tiles, fewer K-tiles than stages; a row below the output stays as it is."""
+    a, b, bias = rnd(M, K), rnd(N, K), rnd(1, N)[0].contiguous()
+    c1, c2 = (torch.full((M + 1, N), 5.0, device=DEV, dtype=torch.bfloat16) for _ in range(2))
+    run_any(a, b, c1[:M], 64, 64, 1, bias if epi else None, epi)
+    run_any(a, b, c2[:M], 128, 128, 1, bias if epi else None, epi)
+    assert torch.equal(c1, c2) and bool((c1[M] == 5).all())
+
+
+def test_gelu_over_its_range():
+    """The epilogue's gelu and its gradient over every finite bf16 value (and the infinities as before)
+    against float64: half a bf16 unit plus a few fp32 units of the exponent's argument."""
+    from kgs.ops import gemm_nt
+    from kgs.ops.gemm import act_grad
+
+    bits = torch.arange(1 << 16, device=DEV, dtype=torch.int32).to(torch.int16)
+    x = bits.view(torch.bfloat16)
+    x = x[x.isfinite() & (x.abs() < 1e18)]  # the square stays finite
+    x = x[:x.numel() // 8 * 8].view(-1, 1).contiguous()
+    one = torch.zeros(8, 8, device=DEV, dtype=torch.bfloat16)
+    one[:, 0] = 1
+    a = torch.zeros(x.shape[0], 8, device=DEV, dtype=torch.bfloat16)
+    a[:, :1] = x
+    got = gemm_nt(a, one, act="gelu")[:, 0].double()
+    z = x[:, 0].double().requires_grad_(True)
+    want = torch.nn.functional.gelu(z, approximate="tanh")
+    # below -8 or so the result is under 1e-14 and its relative error is the exponent's: 2 |u| 2^-23
+    tol = 2.0 ** -8 * want.abs() * 1.01 + 1e-14
+    assert bool(((got - want).abs() <= tol).all())
+    (d,) = torch.autograd.grad(want.sum(), z)
+    gz, _, _ = act_grad(torch.ones_like(a), a, "gelu", False, False)
+    assert bool(((gz[:, 0].double() - d).abs() <= 2.0 ** -8 * d.abs() * 1.01 + 1e-6).all())
+    y = gemm_nt(torch.tensor([[float("inf")] + 7 * [0.0]], device=DEV).bfloat16(), one, act="gelu")
+    assert bool((y == float("inf")).all())

@@ -733,7 +733,7 @@ __global__ __launch_bounds__(256) void splitk_reduce_swiglu(const float* __restr
   for (int k = 0; k < 8; ++k) {
     const float g = bf2f(f2bf(k < 4 ? g0[k] : g1[k - 4]));
     const float u = bf2f(f2bf(k < 4 ? u0[k] : u1[k - 4]));
-    r[k] = g / (1.0f + __expf(-g)) * u;
+    r[k] = silu(g) * u;
   }
   uint4 o;
   o.x = pack_bf16x2(r[0], r[1]);

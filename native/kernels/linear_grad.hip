@@ -27,7 +27,7 @@ template <int ACT>
 __device__ __forceinline__ float grad(float g, float z) {
   if constexpr (ACT == ACT_RELU) return z <= 0.f ? 0.f : g;
   if constexpr (ACT == ACT_SILU) {
-    const float s = 1.0f / (1.0f + __expf(-z));
+    const float s = __builtin_amdgcn_rcpf(1.0f + __expf(-z));
     return g * s * (1.0f + z * (1.0f - s));
   }
   if constexpr (ACT == ACT_GELU) {

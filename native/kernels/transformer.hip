@@ -179,7 +179,7 @@ __global__ __launch_bounds__(256) void silu_mul_q8(const unsigned short* __restr
       for (int e = 0; e < 8; ++e) {
         const float gf = bf2f((unsigned short)g[e]);
         // round through bf16 like the bf16 path, so both paths quantise the same values
-        v[k][e] = bf2f(f2bf(gf / (1.0f + __expf(-gf)) * bf2f((unsigned short)u[e])));
+        v[k][e] = bf2f(f2bf(silu(gf) * bf2f((unsigned short)u[e])));
         am = fmaxf(am, fabsf(v[k][e]));
       }
     }
@@ -247,7 +247,7 @@ __global__ __launch_bounds__(256) void silu_mul(const unsigned short* __restrict
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
     const float gf = bf2f((unsigned short)g[e]);
-    o[e] = (short)f2bf(gf / (1.0f + __expf(-gf)) * bf2f((unsigned short)u[e]));
+    o[e] = (short)f2bf(silu(gf) * bf2f((unsigned short)u[e]));
   }
   ((bf16x8*)(out + r * ld_out))[c] = o;
 }

@@ -455,7 +455,7 @@ GATE_EPI = {"silu": 0, "gelu_tanh": EPI_GELU, "clamped": EPI_CLAMPED}
 def skinny_gemm(x: torch.Tensor, w: PackedWeight, out: torch.Tensor | None = None,
                 ksplit: int | None = None, variant: int = 0, rms: torch.Tensor | None = None,
                 resid_ss: torch.Tensor | None = None, zero: torch.Tensor | None = None,
-                eps: float = 1e-5, rope: dict | None = None) -> torch.Tensor:
+                eps: float = 1e-5, rope: dict | None = None, counters: torch.Tensor | None = None) -> torch.Tensor:
     """``x @ W^T`` (bf16, fp32 accumulate) for ``x: [M <= 256, K]`` row-major;
     ``silu(x @ Wg^T) * (x @ Wu^T)`` for a ``swiglu`` weight. Fused epilogues:
 
@@ -469,7 +469,9 @@ def skinny_gemm(x: torch.Tensor, w: PackedWeight, out: torch.Tensor | None = Non
     * ``rope`` (a ``rope=(H, HKV)``-packed qkv weight): dict of ``cos``, ``sin``
       (fp32 ``[max_pos, 64]``), ``positions`` and ``slots`` (int32 ``[M]``) and
       ``cache`` (the layer's bf16 pages): q / k rotated at their positions, k / v
-      written into their cache slots -- :func:`rope_cache_` in the epilogue."""
+      written into their cache slots -- :func:`rope_cache_` in the epilogue;
+    * ``counters`` (zeroed int32, a value per W strip; left zeroed): instead of the per-GPU ones, with
+      slabs of the call's own -- calls that other streams' calls may overlap."""
     if x.dtype != torch.bfloat16 or not x.is_cuda or x.dim() != 2 or x.stride(1) != 1:
         raise ValueError("x must be a row-major bf16 GPU matrix")
     m, k = x.shape
@@ -497,7 +499,13 @@ def skinny_gemm(x: torch.Tensor, w: PackedWeight, out: torch.Tensor | None = Non
             raise ValueError("resid_ss needs the residual stream as out [M, N] (and no swiglu)")
     if out is None:
         out = torch.empty((m, w.n_out), dtype=torch.bfloat16, device=x.device)
-    ws, cnt = _workspace(x.device, ks * mpad * w.n if ks > 1 else 0, w.n // rps)
+    need = ks * mpad * w.n if ks > 1 else 0
+    if counters is None:
+        ws, cnt = _workspace(x.device, need, w.n // rps)
+    else:
+        if counters.dtype != torch.int32 or not counters.is_contiguous() or counters.numel() < w.n // rps:
+            raise ValueError(f"counters must be at least {w.n // rps} contiguous int32")
+        ws, cnt = torch.empty(max(need, 4), dtype=torch.float32, device=x.device), counters
     if (rope is not None) != bool(w.rope):
         raise ValueError("rope= needs a rope-packed qkv weight (PackedWeight(..., rope=(H, HKV))) and vice versa")
     if rope is not None:

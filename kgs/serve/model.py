@@ -6,7 +6,8 @@ Two step kinds, both driven by the native scheduler's plans
 
 * **prefill** -- the prompts of newly admitted sequences, each padded to a
   multiple of 128 tokens and concatenated (the layers drop the padding where that
-  saves a tile of rows): every projection is one
+  saves a tile of rows; steps of up to ``fused_max_batch`` rows run the FUSED layer
+  below, of up to 256 the split tiles): every projection is one
   :func:`kgs.ops.gemm_nt` (256x256 MFMA pipeline), RoPE + the KV-cache scatter
   is one :func:`kgs.ops.decode.rope_cache_` launch, attention is one
   flash-attention launch over all sequences' query blocks, and only the last real token of each
@@ -335,8 +336,10 @@ class ServingModel:
         h, hd = c.hidden, c.head_dim
         if self.prefill_f8 is not None:
             return self._prefill_fp8(tokens, positions, slots, seq_starts, seq_lens, padded_lens)
-        plan = self._prompt_rows([(int(s), int(n), int(p), 0) for s, n, p in zip(seq_starts, seq_lens, padded_lens)],
-                                 tokens.numel(), tokens.device)
+        seqs = [(int(s), int(n), int(p), 0) for s, n, p in zip(seq_starts, seq_lens, padded_lens)]
+        if self.packed is not None and not self.decode_fp8 and 0 < sum(n for _, n, _, _ in seqs) <= self.fused_max_batch:
+            return self._prefill_fused(tokens, positions, slots, seqs)
+        plan = self._prompt_rows(seqs, tokens.numel(), tokens.device)
         if plan.keep is not None:
             tokens = tokens.reshape(-1)[plan.keep]
         x = self.embed[tokens.long()].reshape(-1, h).contiguous()
@@ -382,6 +385,27 @@ class ServingModel:
         T.op("prefill lm_head")
         return out
 
+    def _prefill_fused(self, tokens, positions, slots, seqs) -> torch.Tensor:
+        """A prompt step of few rows on the fused decode layer (:meth:`_fused_layers`), without its padding:
+        5 launches a layer besides the attention's (one prompt of 20 tokens, hidden 2048: 481 us by the
+        split tiles, 403 so; of 30, hidden 4096: 630 and 546)."""
+        plan = self._prompt_rows(seqs, tokens.numel(), tokens.device, drop=True, force=True)
+        tokens, positions, slots = (t.reshape(-1)[plan.keep] for t in (tokens, positions, slots))
+        c = self.cfg
+        # counters of the step's own: nothing is shared with a decode step on another stream
+        most = max(w.n for w in (*self.packed[0].values(), self.packed_lm))
+        count = torch.zeros(most // 16, dtype=torch.int32, device=tokens.device)
+        from kgs.ops.transformer import attention_blocks
+
+        def attend(qkv, i):
+            a = torch.empty((plan.n, c.heads * c.head_dim), dtype=torch.bfloat16, device=qkv.device)
+            return attention_blocks(qkv, *self._kv(qkv), plan.items, c.heads, c.kv_heads, a)
+
+        x, ss = self._fused_layers(tokens, positions, slots, attend, "prefill", count)
+        out = D.skinny_gemm(x[plan.last], self.packed_lm, rms=ss[plan.last], eps=c.eps, counters=count)
+        T.op("prefill-fused lm_head")
+        return out
+
     def _prefill_fp8(self, tokens, positions, slots, seq_starts, seq_lens, padded_lens) -> torch.Tensor:
         """W8A8 prompt pass: every GEMM input is e4m3 rows with per-row scales from
         its fused producer (add_rmsnorm_fp8, silu_mul_fp8, quantize_rows_fp8);
@@ -408,20 +432,22 @@ class ServingModel:
                 y = add_rmsnorm(x, d, self.norm, c.eps)
         return self._proj(y[plan.last].contiguous(), None, "lm", True)
 
-    def _prompt_rows(self, seqs, total: int, device, drop: bool = True, tail: int = 0, wanted=None) -> "_PromptRows":
+    def _prompt_rows(self, seqs, total: int, device, drop: bool = True, tail: int = 0, wanted=None,
+                     force: bool = False) -> "_PromptRows":
         """What a step's layers need of its prompt portions ``(first row, rows, padded rows, cached tokens
         before)`` and ``tail`` decode rows after them, ``total`` rows as given, in one copy to
         the device. ``wanted``: the portions whose last row is wanted, all by default.
 
         The layers run without the padding wherever that saves a 128-row tile of their products:
         no result depends on it, and it is an eighth of the rows at 500 tokens a prompt (16 such
-        prompts at hidden 4096: 12.85 ms with it, 10.32 without), most of them at 20. Equal portions without cached tokens that need no rows dropped keep the batched
+        prompts at hidden 4096: 12.85 ms with it, 10.32 without), most of them at 20; ``force``: in any
+        case. Equal portions without cached tokens that need no rows dropped keep the batched
         launch."""
         import numpy as np
 
         ref = self.backend == "ref"
         real = sum(n for _, n, _, _ in seqs) + tail
-        drop = drop and not ref and -(-real // 128) < -(-total // 128)
+        drop = drop and not ref and (force or -(-real // 128) < -(-total // 128))
         starts, at = [s for s, _, _, _ in seqs], 0
         if drop:
             starts = []
@@ -664,6 +690,20 @@ class ServingModel:
         ss_a / ss_b carry the residual rows' sums of squares between the
         producing GEMM (residual update) and the consuming one (folded RMSNorm)."""
         c = self.cfg
+
+        def attend(qkv, i):
+            return D.paged_decode_attention(qkv, self.cache.layer(i), block_tables, ctx_lens, c.heads, c.kv_heads,
+                                            pages_per_split=pages_per_split)
+
+        x, ss = self._fused_layers(tokens, positions, slots, attend, "decode", None)
+        out = D.skinny_gemm(x, self.packed_lm, rms=ss, eps=c.eps)
+        T.op("decode-fused lm_head")
+        return out
+
+    def _fused_layers(self, tokens, positions, slots, attend, kind: str, counters):
+        """The residual rows after all layers and their sums of squares; ``attend(qkv, layer)`` is the
+        attention of the rotated rows, whose keys and values are in the cache."""
+        c = self.cfg
         eps = c.eps
         x = self.embed[tokens.long()].reshape(-1, c.hidden).contiguous()  # residual stream
         ss_b = x.float().pow(2).sum(-1)  # statistic for layer 0's qkv
@@ -671,20 +711,17 @@ class ServingModel:
         for i in range(c.layers):
             P = self.packed[i]
             if P["qkv"].rope:
-                qkv = D.skinny_gemm(x, P["qkv"], rms=ss_b, eps=eps,
+                qkv = D.skinny_gemm(x, P["qkv"], rms=ss_b, eps=eps, counters=counters,
                                     rope={"cos": self.cos, "sin": self.sin, "positions": positions, "slots": slots,
                                           "cache": self.cache.layer(i)})
             else:
-                qkv = D.skinny_gemm(x, P["qkv"], rms=ss_b, eps=eps)
+                qkv = D.skinny_gemm(x, P["qkv"], rms=ss_b, eps=eps, counters=counters)
                 self._rope_cache(qkv, i, positions, slots)
-            T.op(f"decode-fused L{i} qkv+rope")
-            a = D.paged_decode_attention(qkv, self.cache.layer(i), block_tables, ctx_lens, c.heads, c.kv_heads,
-                                         pages_per_split=pages_per_split)
-            T.op(f"decode-fused L{i} attention")
-            D.skinny_gemm(a, P["o"], out=x, resid_ss=ss_a, zero=ss_b)
-            act = D.skinny_gemm(x, P["gate_up"], rms=ss_a, eps=eps)
-            D.skinny_gemm(act, P["down"], out=x, resid_ss=ss_b, zero=ss_a)
-            T.op(f"decode-fused L{i} o+mlp")
-        out = D.skinny_gemm(x, self.packed_lm, rms=ss_b, eps=eps)
-        T.op("decode-fused lm_head")
-        return out
+            T.op(f"{kind}-fused L{i} qkv+rope")
+            a = attend(qkv, i)
+            T.op(f"{kind}-fused L{i} attention")
+            D.skinny_gemm(a, P["o"], out=x, resid_ss=ss_a, zero=ss_b, counters=counters)
+            act = D.skinny_gemm(x, P["gate_up"], rms=ss_a, eps=eps, counters=counters)
+            D.skinny_gemm(act, P["down"], out=x, resid_ss=ss_b, zero=ss_a, counters=counters)
+            T.op(f"{kind}-fused L{i} o+mlp")
+        return x, ss_b

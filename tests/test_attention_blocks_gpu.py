@@ -153,3 +153,30 @@ def test_gather_kv_bits(fp8, kv, ctx, rows):
     assert torch.equal(k, wk) and torch.equal(v, wv)
     with pytest.raises(ValueError):
         D.gather_kv_into(cache, pages[:0], 1, k, v)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("lens", [[20, 5], [48], [49], [130, 126], [100, 157], [300, 260]])
+def test_prefill_by_rows(lens):
+    """Either side of the row counts where a prompt step changes its layers: logits and cache of the step
+    against float32 layers on the same weights. Sums round to bf16 at other places on either side: a
+    few 2^-8 in the 2-norm over two layers."""
+    from kgs.models.llama import LlamaConfig
+    from kgs.serve.model import ServingModel
+
+    cfg = LlamaConfig(hidden=2048, intermediate=2048, heads=16, kv_heads=4, layers=2, vocab=1024)
+    ours, ref = (ServingModel(cfg, device=DEV, backend=b, num_pages=40, max_model_len=1024) for b in ("kgs", "ref"))
+    padded = [-(-n // 128) * 128 for n in lens]
+    total, rng = sum(padded), np.random.default_rng(len(lens))
+    tok, pos, slot, at, page, starts = np.zeros(total, np.int32), np.zeros(total, np.int32), np.full(total, -1, np.int32), 0, 1, []
+    for n, p in zip(lens, padded):
+        starts.append(at)
+        tok[at:at + n], pos[at:at + n], slot[at:at + n] = rng.integers(0, 1024, n), np.arange(n), 32 * page + np.arange(n)
+        at, page = at + p, page + -(-n // 32)
+    args = [torch.from_numpy(a).to(DEV) for a in (tok, pos, slot)]
+    got, want = (m.prefill(*args, starts, lens, padded).float() for m in (ours, ref))
+    assert got.shape == want.shape == (len(lens), 1024)
+    assert float((got - want).norm() / want.norm()) < 0.03
+    a, b = ours.cache.data.float(), ref.cache.data.float()
+    assert float((a - b).norm() / b.norm()) < 0.02
+    assert torch.equal(a == 0, b == 0)  # the same slots written

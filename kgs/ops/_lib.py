@@ -111,7 +111,8 @@ _SIGS = {
                               _c_int),
     "kgs_splitk_reduce_swiglu_bf16": ([_c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_void_p], _c_int),
     "kgs_gather_kv": ([_c_void_p] * 4 + [_c_int] * 5 + [_c_long, _c_int, _c_void_p], _c_int),
-    "kgs_attn_fwd_blocks_bf16": ([_c_void_p] * 7 + [_c_int] * 4 + [_c_long] * 5 + [ctypes.c_float, _c_void_p], _c_int),
+    "kgs_attn_fwd_blocks_bf16": ([_c_void_p] * 7 + [_c_int] * 4 + [_c_long] * 5 + [ctypes.c_float, _c_void_p, _c_int, _c_int] +
+                                 [_c_void_p] * 2, _c_int),
     "kgs_paged_decode_wg": ([_c_void_p] * 8 + [_c_int] * 6 + [_c_long, _c_long, ctypes.c_float, _c_int, _c_void_p], _c_int),
     "kgs_paged_decode_bf16_ex": ([_c_void_p] * 8 + [_c_int] * 7 + [_c_long, _c_long, ctypes.c_float, _c_int, _c_int,
                                                                    _c_void_p], _c_int),

@@ -268,23 +268,29 @@ QBLOCK = 128  # query rows of an attention_blocks item
 
 def attention_blocks(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, items: torch.Tensor, heads: int, kv_heads: int,
                      out: torch.Tensor, k2: torch.Tensor | None = None, v2: torch.Tensor | None = None,
-                     scale: float | None = None) -> torch.Tensor:
+                     scale: float | None = None, merges: torch.Tensor | None = None, slots: int = 0) -> torch.Tensor:
     """Causal flash attention of sequences of any lengths in one launch (head_dim 128), a block of up to
     128 query rows each item. ``items`` int32 ``[n, 4]`` (:func:`block_items`): the block's first row in
     ``q`` / ``out``, the row of its sequence's key 0, the position of the first row, and twice its
-    number of rows, plus 1 for keys in ``k2`` / ``v2`` instead of ``k`` / ``v``."""
+    number of rows, plus 1 for keys in ``k2`` / ``v2`` instead of ``k`` / ``v``. ``merges``, ``slots``:
+    those of :func:`split_items`, whose parts of a block's keys are put together in a second launch."""
     for t, n in ((q, "q"), (k, "k"), (v, "v"), (out, "out")):
         _need(t, n)
     if items.dtype != torch.int32 or items.dim() != 2 or items.shape[1] != 4 or not items.is_contiguous():
         raise ValueError("items must be contiguous int32 [n, 4]")
     if (k2 is None) != (v2 is None) or (k2 is not None and k2.stride() != v2.stride()):
         raise ValueError("k2 and v2 come together, with one row stride")
+    if merges is not None and (merges.dtype != torch.int32 or merges.dim() != 2 or merges.shape[1] != 4 or
+                               not merges.is_contiguous() or slots < 2 * merges.shape[0]):
+        raise ValueError("merges must be contiguous int32 [n, 4], with their slots")
     scale = 1.0 / math.sqrt(128) if scale is None else scale
+    ws = None if merges is None else torch.empty(slots * heads * QBLOCK * (128 + 2), dtype=torch.float32, device=q.device)
     two = (0, 0, 0) if k2 is None else (k2.data_ptr(), v2.data_ptr(), k2.stride(0))
     rc = _lib.lib().kgs_attn_fwd_blocks_bf16(q.data_ptr(), k.data_ptr(), v.data_ptr(), two[0], two[1], out.data_ptr(),
                                              items.data_ptr(), items.shape[0], heads, kv_heads, 128, q.stride(0),
                                              k.stride(0), v.stride(0), two[2], out.stride(0), float(scale),
-                                             _lib.stream_handle(q.device))
+                                             None if merges is None else merges.data_ptr(), 0 if merges is None else merges.shape[0],
+                                             slots, None if ws is None else ws.data_ptr(), _lib.stream_handle(q.device))
     _lib.check(rc, "attention_blocks")
     return out
 
@@ -302,6 +308,44 @@ def block_items(seqs, rows: int):
         out += [(r + b, k0, pos + b, 2 * min(QBLOCK, n - b) + src) for b in range(0, n, QBLOCK)]
     out = np.array(out, np.int32).reshape(-1, 4)
     return out[np.argsort(-out[:, 2], kind="stable")]
+
+
+SPLIT_TILES = 24    # 64-key tiles of a block that may be split
+SPLIT_PARTS = 8
+SPLIT_FAIR = 16     # fewest tiles of a part, about
+
+
+def split_items(items, heads: int, cus: int = 256):
+    """``items`` with the longest blocks' keys in parts, for launches whose time is that of one such
+    block: ``(items, merges, slots)``. Two workgroups run on a CU; a block of more than half as many tiles
+    again as each of these would get on average is cut into parts of about that many (blocks of 16 tiles
+    in parts of 8 gain as often as they lose). ``merges``
+    int32 ``[n, 4]``: first row, rows, first slot and parts of a split block; None without any."""
+    import numpy as np
+
+    rows = items[:, 3] >> 1 & 255
+    tiles = (items[:, 2] + rows - 1) // 64 + 1
+    fair = max(SPLIT_FAIR, -(-int(tiles.sum()) * heads // (2 * cus)))
+    long = np.nonzero((tiles >= SPLIT_TILES) & (2 * tiles > 3 * fair))[0]
+    if long.size == 0:
+        return items, None, 0
+    out, left, merges, slot = [], [], [], 0
+    for i, it in enumerate(items.tolist()):
+        t = int(tiles[i])
+        if t < SPLIT_TILES or 2 * t <= 3 * fair:
+            out.append(it)
+            left.append(t)
+            continue
+        n = min(SPLIT_PARTS, max(2, (2 * t + fair) // (2 * fair)))
+        merges.append([it[0], int(rows[i]), slot, n])
+        for p in range(n):
+            out.append([*it[:3], it[3] | p << 9 | n << 13 | slot << 17])
+            left.append(t * (p + 1) // n - t * p // n)
+        slot += n
+    if slot >= 1 << 14:
+        return items, None, 0
+    order = np.argsort(-np.asarray(left), kind="stable")
+    return np.asarray(out, np.int32)[order], np.asarray(merges, np.int32), slot
 
 
 def ref_attention_chunk(q, k, v, heads, kv_heads, head_dim=128, scale=None):

@@ -60,15 +60,15 @@ def gate_up_panel_widths(n: int, k: int) -> set:
 
 class _PromptRows:
     """Rows of a step's layers: ``n`` of them, ``last`` (int64) those whose logits are wanted, attention
-    ``items`` with the gathered contexts ``past`` ``(first row, end, tokens, portion)``, and, where
+    ``items`` (and ``merges``, ``slots`` of their parts) with the gathered contexts ``past`` ``(first row, end, tokens, portion)``, and, where
     the padding was dropped, ``keep`` (int64: the given rows that stay) and ``rows`` (int32: each
     given row's number, -1 for padding)."""
 
-    __slots__ = ("n", "past", "items", "last", "rows", "keep")
+    __slots__ = ("n", "past", "items", "merges", "slots", "last", "rows", "keep")
 
     def __init__(self, n, past):
-        self.n, self.past = n, past
-        self.items = self.last = self.rows = self.keep = None
+        self.n, self.past, self.slots = n, past, 0
+        self.items = self.merges = self.last = self.rows = self.keep = None
 
 
 class ServingModel:
@@ -365,7 +365,7 @@ class ServingModel:
                 T.op(f"prefill L{i} qkv")
                 self._rope_cache(qkv, i, positions, slots, plan.rows)
             T.op(f"prefill L{i} rope_cache")
-            a = self._prefill_attention(qkv, seq_starts, seq_lens, padded_lens, plan.items)
+            a = self._prefill_attention(qkv, seq_starts, seq_lens, padded_lens, plan)
             T.op(f"prefill L{i} attention")
             if ro:
                 y = splitk_add_rmsnorm(self._split_proj(a, i, "o", ro, True), x, self.ln2[i], c.eps)
@@ -399,7 +399,7 @@ class ServingModel:
 
         def attend(qkv, i):
             a = torch.empty((plan.n, c.heads * c.head_dim), dtype=torch.bfloat16, device=qkv.device)
-            return attention_blocks(qkv, *self._kv(qkv), plan.items, c.heads, c.kv_heads, a)
+            return attention_blocks(qkv, *self._kv(qkv), plan.items, c.heads, c.kv_heads, a, merges=plan.merges, slots=plan.slots)
 
         x, ss = self._fused_layers(tokens, positions, slots, attend, "prefill", count)
         out = D.skinny_gemm(x[plan.last], self.packed_lm, rms=ss[plan.last], eps=c.eps, counters=count)
@@ -422,7 +422,7 @@ class ServingModel:
             F = self.prefill_f8[i]
             qkv = F["qkv"].forward_q(y8, ys)
             self._rope_cache(qkv, i, positions, slots)
-            a8, as_ = quantize_rows_fp8(self._prefill_attention(qkv, seq_starts, seq_lens, padded_lens, plan.items))
+            a8, as_ = quantize_rows_fp8(self._prefill_attention(qkv, seq_starts, seq_lens, padded_lens, plan))
             y8, ys = add_rmsnorm_fp8(x, F["o"].forward_q(a8, as_), self.ln2[i], c.eps)
             m8, ms = silu_mul_fp8(F["gate_up"].forward_q(y8, ys))
             d = F["down"].forward_q(m8, ms)
@@ -460,7 +460,7 @@ class ServingModel:
         parts = [np.asarray(last + list(range(at, at + tail)), np.int32)]
         past, items = [], None
         if not ref and seqs and (drop or wanted is not None or len({p for _, _, p, _ in seqs}) > 1):
-            from kgs.ops.transformer import block_items
+            from kgs.ops.transformer import block_items, split_items
 
             blocks, k0 = [], 0
             for j, (r, (_, n, p, ctx)) in enumerate(zip(starts, seqs)):
@@ -469,8 +469,8 @@ class ServingModel:
                 if ctx:
                     past.append((k0, k0 + ctx + m, ctx + n, j))
                     k0 += ctx + m
-            items = block_items(blocks, at)
-            parts.append(items.reshape(-1))
+            items, merges, slots = split_items(block_items(blocks, at), self.cfg.heads)
+            parts.append(items.reshape(-1) if merges is None else np.concatenate([items, merges]).reshape(-1))
         if drop:
             keep = np.concatenate([np.arange(s, s + n, dtype=np.int32) for s, n, _, _ in seqs] +
                                   [np.arange(total - tail, total, dtype=np.int32)])
@@ -484,7 +484,10 @@ class ServingModel:
             t = t.pin_memory().to(device, non_blocking=True)
         out = _PromptRows(at + tail, past)
         n = sizes[1] if items is not None else 0
-        out.items = None if items is None else t[:n].view(-1, 4)
+        if items is not None:
+            out.items = t[:items.size].view(-1, 4)
+            if merges is not None:
+                out.merges, out.slots = t[items.size:n].view(-1, 4), slots
         out.last = t[n:n + sizes[0]].long()
         if drop:
             out.rows, out.keep = t[n + sizes[0]:n + sizes[0] + total], t[n + sizes[0] + total:].long()
@@ -496,14 +499,15 @@ class ServingModel:
         q, n = c.heads * c.head_dim, c.kv_heads * c.head_dim
         return qkv[:, q:q + n], qkv[:, q + n:q + 2 * n]
 
-    def _prefill_attention(self, qkv, seq_starts, seq_lens, padded_lens, items=None):
+    def _prefill_attention(self, qkv, seq_starts, seq_lens, padded_lens, plan=None):
         c = self.cfg
         hd = c.head_dim
         out = torch.empty((qkv.shape[0], c.heads * hd), dtype=torch.bfloat16, device=qkv.device)
-        if items is not None:  # unequal prompts: one launch over all their query blocks
+        if plan is not None and plan.items is not None:  # unequal prompts: one launch over all their query blocks
             from kgs.ops.transformer import attention_blocks
 
-            return attention_blocks(qkv, *self._kv(qkv), items, c.heads, c.kv_heads, out)
+            return attention_blocks(qkv, *self._kv(qkv), plan.items, c.heads, c.kv_heads, out, merges=plan.merges,
+                                    slots=plan.slots)
         if self.backend != "ref" and len(set(int(p) for p in padded_lens)) == 1:
             # equal padded lengths, packed back to back: one batched launch
             from kgs.ops.transformer import attention_qkv
@@ -572,7 +576,8 @@ class ServingModel:
                 # ones the cached rows (this step's were just written there), gathered
                 for r0, r1, ctx, j in plan.past:
                     D.gather_kv_into(self.cache.layer(i), chunks[j][4], ctx, k2[r0:r1], v2[r0:r1])
-                attention_blocks(qkv, *self._kv(qkv), plan.items, c.heads, c.kv_heads, a, k2, v2)
+                attention_blocks(qkv, *self._kv(qkv), plan.items, c.heads, c.kv_heads, a, k2, v2, merges=plan.merges,
+                                 slots=plan.slots)
             else:
                 for row0, n, p, ctx0, pages, _ in chunks:
                     a[row0:row0 + p] = self._chunk_attention(qkv[row0:row0 + p], i, n, p, ctx0, pages)

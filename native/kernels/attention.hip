@@ -72,6 +72,8 @@ struct Args {
   const unsigned short* k2;
   const unsigned short* v2;
   long ld2;
+  float* ws;  // parts of split blocks: [slot][H][QB] rows of HD sums and (maximum, weight sum)
+  int slots;
 };
 
 // EQUAL: B equal sequences of S rows, a multiple of QB. RAGGED: any number of query rows per
@@ -79,12 +81,17 @@ struct Args {
 // dropped on store; always causal. BLOCKS: blocks of up to QB rows of sequences of any lengths in
 // one launch, causal, with grouped key heads, clamped likewise; one int4 per block -- first query
 // row, first key row of its sequence, position of the first query row, and twice the number of
-// rows, plus 1 where the keys are
+// rows (bits 1-8), plus 1 where the keys are
 // rows of k2 / v2. One launch because one per sequence leaves the chip to each sequence's own tail:
 // prompts of a few hundred tokens at 32 heads have fewer workgroups each than the 512 that are
 // resident. A whole prompt step of 16 unequal prompts of about 512 tokens (H 4096) went from 13.76
 // to 12.85 ms; a step of 2048 prompt rows, one chunk of them at 3072 cached tokens, with 40
 // decode rows from 3.90 to 3.60, of it the keys' gather in one launch about half.
+// A block over a long context may come in parts of its key tiles (bits 9-12: which, 13-16: of how
+// many, 17 up: the first part's slot): each leaves fp32 sums, maximum and weight sum in its slot, and
+// merge_parts puts them together. Otherwise a launch takes as long as its longest blocks' serial
+// chain of tiles: steps of 512 rows at 6016 cached tokens (32 heads) 1664 us, 1302 so; of 2048 rows at
+// 4096 (16 heads) 1580 and 1380; of 804 rows at 3072 beside 918 rows of new prompts 3431 and 3390.
 enum Mode { EQUAL = 0, RAGGED_ROWS = 1, BLOCKS = 2 };
 
 // XOR image of a row's 16-B chunks (HD / 8 of them)
@@ -108,7 +115,7 @@ __global__ __launch_bounds__(256, 2) __attribute__((amdgpu_waves_per_eu(2, 2))) 
 
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l32 = lane & 31, hh = lane >> 5;
-  int h, kvh, q0, qw, qrow, qoff, nval = QB;
+  int h, kvh, q0, qw, qrow, qoff, nval = QB, part = 0, parts = 0, slot = 0;
   long tok0, ktok0, ldk = a.ldk, ldv = a.ldv;
   const unsigned short *kp = a.k, *vp = a.v;
   bool causal = true;
@@ -123,11 +130,19 @@ __global__ __launch_bounds__(256, 2) __attribute__((amdgpu_waves_per_eu(2, 2))) 
     const int item = lid / a.H;
     h = lid - item * a.H;
     kvh = h / (a.H / a.HKV);
-    const int4 it = a.items[item];
+    int4 it = a.items[item];  // uniform: kept in scalars
+    it.x = __builtin_amdgcn_readfirstlane(it.x);
+    it.y = __builtin_amdgcn_readfirstlane(it.y);
+    it.z = __builtin_amdgcn_readfirstlane(it.z);
+    it.w = __builtin_amdgcn_readfirstlane(it.w);
     tok0 = it.x;
     ktok0 = it.y;
     qoff = it.z;
-    nval = it.w >> 1;
+    nval = (it.w >> 1) & 255;
+    part = (it.w >> 9) & 15;
+    parts = (it.w >> 13) & 15;
+    slot = (int)((unsigned)it.w >> 17) + part;
+    if (parts && (slot >= a.slots || part >= parts)) return;  // no such slot
     if (it.w & 1) {
       kp = a.k2;
       vp = a.v2;
@@ -203,10 +218,10 @@ __global__ __launch_bounds__(256, 2) __attribute__((amdgpu_waves_per_eu(2, 2))) 
     for (int i = 0; i < ND; ++i) {
       const int ch = ND * w + i;
       const int r = (512 / HD) * ch + lane / (HD / 8), c = (lane & (HD / 8 - 1)) ^ swz<HD>(r);
-      long row = (long)jn * KB + r;
-      if constexpr (PART) row = min(row, (long)(qoff + nval - 1));
-      glds16(kbase + row * ldk + 8 * c, smem[sb] + 1024 * ch);
-      glds16(vbase + row * ldv + 8 * c, smem[sb] + TILE_BYTES + 1024 * ch);
+      int row = jn * KB + r;
+      if constexpr (PART) row = min(row, qoff + nval - 1);
+      glds16(kbase + (long)row * ldk + 8 * c, smem[sb] + 1024 * ch);
+      glds16(vbase + (long)row * ldv + 8 * c, smem[sb] + TILE_BYTES + 1024 * ch);
     }
     if constexpr (HR > 0) {
 #pragma unroll
@@ -219,9 +234,13 @@ __global__ __launch_bounds__(256, 2) __attribute__((amdgpu_waves_per_eu(2, 2))) 
     }
   };
 
-  const int ntile = PART ? (qoff + nval - 1) / KB + 1 : causal ? (qoff + q0 + QB) / KB : a.Sk / KB;
+  int ntile = PART ? (qoff + nval - 1) / KB + 1 : causal ? (qoff + q0 + QB) / KB : a.Sk / KB;
   const int win = RAGGED ? a.win : 0;
-  const int j0 = win ? max(0, qoff + q0 - win + 1) / KB : 0;
+  int j0 = win ? max(0, qoff + q0 - win + 1) / KB : 0;
+  if (MODE == BLOCKS && parts) {
+    j0 = ntile * part / parts;
+    ntile = ntile * (part + 1) / parts;
+  }
   dma_tiles(j0, 0);
   // Q fragments and tile 0 complete before the loop (a vmcnt the waitcnt pass
   // sees, so it does not carry the Q loads into the loop header)
@@ -325,7 +344,7 @@ __global__ __launch_bounds__(256, 2) __attribute__((amdgpu_waves_per_eu(2, 2))) 
 #pragma unroll
         for (int d = 0; d < ND; ++d) o[d] *= alpha;
       }
-      const float msl = RAGGED && m == NEG ? 0.f : m * sl2;  // a row that has seen no key yet: weights 0
+      const float msl = PART && m == NEG ? 0.f : m * sl2;  // a row that has seen no key yet: weights 0
 #pragma unroll
       for (int t = 0; t < 2; ++t)
 #pragma unroll
@@ -361,6 +380,18 @@ __global__ __launch_bounds__(256, 2) __attribute__((amdgpu_waves_per_eu(2, 2))) 
   float inv = 1.0f / l;
   if constexpr (PART)
     if (qrow >= nval) return;
+  if (MODE == BLOCKS && parts) {
+    float* part0 = a.ws + ((long)slot * a.H + h) * (QB * (HD + 2)) + qrow;  // [dim][row]: a wave's 32 rows in a run
+#pragma unroll
+    for (int d = 0; d < ND; ++d)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) part0[(32 * d + 8 * (r >> 2) + 4 * hh + (r & 3)) * QB] = o[d][r];
+    if (hh == 0) {
+      part0[HD * QB] = m;
+      part0[(HD + 1) * QB] = l;
+    }
+    return;
+  }
   if constexpr (RAGGED) {
     if (a.gate && !a.eg) inv /= 1.0f + __expf(-bf2f(a.gate[(tok0 + qrow) * a.ldg + (long)h * a.hg]));
   }
@@ -381,6 +412,45 @@ __global__ __launch_bounds__(256, 2) __attribute__((amdgpu_waves_per_eu(2, 2))) 
       pk.y = pack_bf16x2(o[d][4 * r4 + 2] * inv, o[d][4 * r4 + 3] * inv);
       *(uint2*)(op + dcol) = pk;
     }
+}
+
+// The parts of a split block (x) and head (y): out = sum_p w_p O_p / sum_p w_p l_p with
+// w_p = 2^((m_p - max m) sl2). merges: first row, rows, first slot, parts. A thread per row, 16 dims (z).
+__global__ __launch_bounds__(QB) void merge_parts(const float* __restrict__ ws, const int4* __restrict__ merges,
+                                                  unsigned short* __restrict__ o, int H, long ldo, float sl2) {
+  constexpr int HD = 128, PARTS = 8;
+  const int4 mg = merges[blockIdx.x];
+  const int h = blockIdx.y, r = threadIdx.x, n = min(mg.w, PARTS);
+  if (r >= mg.y) return;
+  const float* p = ws + ((long)mg.z * H + h) * (QB * (HD + 2)) + r;
+  const long step = (long)H * QB * (HD + 2);
+  float w[PARTS], mx = NEG, l = 0.f;
+#pragma unroll
+  for (int i = 0; i < PARTS; ++i) {
+    w[i] = i < n ? p[i * step + HD * QB] : NEG;
+    mx = fmaxf(mx, w[i]);
+  }
+#pragma unroll
+  for (int i = 0; i < PARTS; ++i) {
+    w[i] = __builtin_amdgcn_exp2f((w[i] - mx) * sl2);
+    if (i < n) l = __builtin_fmaf(w[i], p[i * step + (HD + 1) * QB], l);
+  }
+  const float inv = 1.0f / l;
+  float s[16];
+#pragma unroll
+  for (int e = 0; e < 16; ++e) s[e] = 0.f;
+  const int d0 = 16 * blockIdx.z;
+#pragma unroll
+  for (int i = 0; i < PARTS; ++i)
+    if (i < n) {
+#pragma unroll
+      for (int e = 0; e < 16; ++e) s[e] = __builtin_fmaf(w[i], p[i * step + (d0 + e) * QB], s[e]);
+    }
+#pragma unroll
+  for (int e = 0; e < 16; ++e) s[e] *= inv;
+  uint4* out = (uint4*)(o + (mg.x + r) * ldo + (long)h * HD + d0);
+  out[0] = make_uint4(pack_bf16x2(s[0], s[1]), pack_bf16x2(s[2], s[3]), pack_bf16x2(s[4], s[5]), pack_bf16x2(s[6], s[7]));
+  out[1] = make_uint4(pack_bf16x2(s[8], s[9]), pack_bf16x2(s[10], s[11]), pack_bf16x2(s[12], s[13]), pack_bf16x2(s[14], s[15]));
 }
 
 }  // namespace attn
@@ -407,7 +477,7 @@ KGS_EXPORT int kgs_attn_fwd_bf16_ex(const void* q, const void* k, const void* v,
   if (nwg > 0x7fffffff) return KGS_ERR_SHAPE;
   Args a{(const unsigned short*)q, (const unsigned short*)k, (const unsigned short*)v, (unsigned short*)o,
          ldq, ldk, ldv, ldo, B, S, H, HKV, scale * 1.4426950408889634f, causal ? 1 : 0, Sk, Sk - S,
-         nullptr, nullptr, 0, 0, 0, nullptr, 0, nullptr, nullptr, 0, 0, 0, nullptr, nullptr, 0};
+         nullptr, nullptr, 0, 0, 0, nullptr, 0, nullptr, nullptr, 0, 0, 0, nullptr, nullptr, 0, nullptr, 0};
   hipLaunchKernelGGL((fwd<HD, EQUAL>), dim3((unsigned)nwg), dim3(256), 0, s, a);
   return (int)hipGetLastError();
 }
@@ -443,7 +513,7 @@ KGS_EXPORT int kgs_attn_fwd_ragged_bf16(const void* q, const void* k, const void
   Args a{(const unsigned short*)q, (const unsigned short*)k, (const unsigned short*)v, (unsigned short*)o,
          ldq, ldk, ldv, ldo, 0, 0, H, H, scale * 1.4426950408889634f, 1, 0, 0,
          (const int4*)items, (const unsigned short*)gate, ldg, hg, eg,
-         (const unsigned short*)kr, ldr, (const float*)cs, (const int*)pos, npos, rot, win, nullptr, nullptr, 0};
+         (const unsigned short*)kr, ldr, (const float*)cs, (const int*)pos, npos, rot, win, nullptr, nullptr, 0, nullptr, 0};
   const dim3 grid((unsigned)(nitems * H));
   auto fn = hd == 128 ? (hr == 0 ? fwd<128, RAGGED_ROWS> : hr == 32 ? fwd<128, RAGGED_ROWS, 32> : fwd<128, RAGGED_ROWS, 64>)
                       : (hr == 0 ? fwd<64, RAGGED_ROWS> : hr == 32 ? fwd<64, RAGGED_ROWS, 32> : fwd<64, RAGGED_ROWS, 64>);
@@ -457,7 +527,7 @@ KGS_EXPORT int kgs_attn_fwd_ragged_bf16(const void* q, const void* k, const void
 // k2 / v2)), any order (heaviest first keeps the tail short). Every item reads its position + rows keys.
 KGS_EXPORT int kgs_attn_fwd_blocks_bf16(const void* q, const void* k, const void* v, const void* k2, const void* v2, void* o,
                                        const void* items, int nitems, int H, int HKV, int hd, long ldq, long ldk,
-                                       long ldv, long ld2, long ldo, float scale, hipStream_t s) {
+                                       long ldv, long ld2, long ldo, float scale, const void* merges, int nmerge, int slots, float* ws, hipStream_t s) {
   using namespace kgs::attn;
   if (nitems <= 0 || H <= 0 || HKV <= 0 || H % HKV || hd != 128) return KGS_ERR_SHAPE;
   const long w = (long)HKV * hd;
@@ -465,10 +535,15 @@ KGS_EXPORT int kgs_attn_fwd_blocks_bf16(const void* q, const void* k, const void
   const uintptr_t al = (uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)o | (uintptr_t)items | (uintptr_t)k2 | (uintptr_t)v2;
   if ((al & 15) || (ldq | ldk | ldv | ldo | ld2) & 7) return KGS_ERR_ALIGN;
   if ((long)nitems * H > 0x7fffffff) return KGS_ERR_SHAPE;
+  if (merges ? nmerge <= 0 || slots <= 0 || !ws || H > 65535 : slots != 0) return KGS_ERR_ARG;
+  if ((uintptr_t)merges % 16 || (uintptr_t)ws % 16) return KGS_ERR_ALIGN;
   Args a{(const unsigned short*)q, (const unsigned short*)k, (const unsigned short*)v, (unsigned short*)o,
          ldq, ldk, ldv, ldo, 0, 0, H, HKV, scale * 1.4426950408889634f, 1, 0, 0,
          (const int4*)items, nullptr, 0, 0, 0, nullptr, 0, nullptr, nullptr, 0, 0, 0,
-         (const unsigned short*)k2, (const unsigned short*)v2, ld2};
+         (const unsigned short*)k2, (const unsigned short*)v2, ld2, ws, slots};
   hipLaunchKernelGGL((fwd<128, BLOCKS>), dim3((unsigned)(nitems * H)), dim3(256), 0, s, a);
+  if (merges)
+    hipLaunchKernelGGL(merge_parts, dim3((unsigned)nmerge, (unsigned)H, 8), dim3(QB), 0, s, ws, (const int4*)merges,
+                       (unsigned short*)o, H, ldo, a.sl2);
   return (int)hipGetLastError();
 }

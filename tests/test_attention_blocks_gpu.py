@@ -27,6 +27,7 @@ def test_prompt_rows_cpu():
 
     class M:
         backend = "kgs"
+        cfg = type("Cfg", (), {"heads": 8})
 
     seqs, dev = [(0, 20, 128, 0), (128, 130, 256, 64)], torch.device("cpu")
     p = ServingModel._prompt_rows(M, seqs, 387, dev, tail=3, wanted=[False, True])
@@ -39,6 +40,53 @@ def test_prompt_rows_cpu():
         q = ServingModel._prompt_rows(M, seqs if kw else [(0, 120, 128, 0), (128, 128, 128, 0)], 384 if kw else 256, dev, **kw)
         assert q.keep is None and q.rows is None and q.last.tolist() == ([19, 257] if kw else [119, 255])
     assert q.items is None and q.n == 256  # equal portions: the batched launch
+
+
+def test_split_items():
+    """Every key tile of a block is in exactly one part, slots follow one another, short blocks and launches
+    of many rounds stay whole."""
+    it = T.block_items([(0, 300, 0, 3072, 1), (300, 256, 300, 0, 0)], 556)
+    out, merges, slots = T.split_items(it, 32)
+    got = {}
+    for r, k0, pos, w in out.tolist():
+        rows, part, parts, slot, t = w >> 1 & 255, w >> 9 & 15, w >> 13 & 15, w >> 17, (pos + (w >> 1 & 255) - 1) // 64 + 1
+        got.setdefault((r, rows, pos, w & 1), []).append((t * part // parts, t * (part + 1) // parts, slot) if parts else (0, t, None))
+    assert {k for k in got} == {(r, w >> 1, p, w & 1) for r, _, p, w in it.tolist()}
+    for (r, rows, pos, _), ps in got.items():
+        ps.sort()
+        assert ps[0][0] == 0 and ps[-1][1] == (pos + rows - 1) // 64 + 1 and all(a[1] == b[0] for a, b in zip(ps, ps[1:]))
+        assert (len(ps) > 1) == (pos >= 3072) and len({p[2] for p in ps}) == 1
+    assert sorted(m[2] for m in merges.tolist()) == [sum(m[3] for m in merges.tolist()[:i]) for i in range(len(merges))]
+    assert slots == sum(m[3] for m in merges.tolist())
+    assert T.split_items(T.block_items([(0, 8192, 0, 0, 0)], 8192), 32)[1] is None  # 2048 workgroups
+    assert T.split_items(T.block_items([(0, 512, 0, 0, 0)], 512), 8)[1] is None     # nothing long
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,ctx", [(1, 1024), (70, 1500), (300, 3072), (128, 6144)])
+@pytest.mark.parametrize("parts", [2, 3, 8])
+def test_parts_of_long_blocks(rows, ctx, parts):
+    """Blocks cut into parts against whole ones: the sums are fp32 in another order, then rounded to bf16 once
+    on either side (2^-8 of the largest weight's value apart at most)."""
+    torch.manual_seed(rows + parts)
+    heads, kv = 4, 2
+    q = torch.randn(rows, 128 * heads, device=DEV).bfloat16()
+    k, v = torch.randn(2, ctx + rows, 128 * kv, device=DEV).bfloat16()
+    k[0] *= 3  # a few keys outweigh the rest, so that parts' maxima differ
+    items = T.block_items([(0, rows, 0, ctx, 1)], rows)
+    want, got = torch.zeros(2, rows + 2, 128 * heads, device=DEV, dtype=torch.bfloat16)
+    T.attention_blocks(q, k, v, torch.from_numpy(items).to(DEV), heads, kv, want, k, v)
+    out, merges, slot = [], [], 0
+    for it in items.tolist():
+        merges.append([it[0], it[3] >> 1, slot, parts])
+        out += [[*it[:3], it[3] | p << 9 | parts << 13 | slot << 17] for p in range(parts)]
+        slot += parts
+    T.attention_blocks(q, k, v, torch.tensor(out, dtype=torch.int32, device=DEV), heads, kv, got, k, v,
+                       merges=torch.tensor(merges, dtype=torch.int32, device=DEV), slots=slot)
+    assert float((got.float() - want.float()).abs().max()) <= 2.0 ** -7 * float(want.float().abs().max())
+    assert not got[rows:].any()
+    ref = T.ref_attention_chunk(torch.cat([q, q[:, :2 * 128 * kv]], 1), k, v, heads, kv)
+    assert float((got[:rows].float() - ref).norm() / ref.norm()) < 2.0 ** -7  # P and the result in bf16
 
 
 @pytest.mark.gpu

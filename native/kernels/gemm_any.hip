@@ -29,6 +29,7 @@ using w4::BK;
 using w4::Ctx;
 using w4::Frag;
 
+typedef long i64x2 __attribute__((ext_vector_type(2)));
 constexpr int OOB = 0x7FFFFFF0;  // above every buffer resource's size (any_ok)
 
 // What a launch stores. DUAL: C gets bf16(acc + bias) and C2 the activation of that bf16 value
@@ -43,6 +44,8 @@ struct Args {
   int ks;                      // K of a slice, a multiple of 128
   int tall;                    // tile groups along N (M > N): see launch
   int vec;                     // 16-B stores: ldc % 8 == 0 and C (C2) 16-B aligned
+  float alpha;                 // e4m3: a factor of the sums, times *alpha_ptr if that is given
+  const float* alpha_ptr;
 };
 
 template <int BM, int BN>
@@ -277,7 +280,10 @@ void gemm_nt_any(Args a) {
 // three stages 0.44 us a step). Accumulators are plain registers, in gemm_w4.h's order of products per
 // element: bitwise the larger tiles' results. us, 128x128 / here: 1024^3 9.4 / 7.4, 256 x 3072 x 2048 15.1 /
 // 11.6, 128 x 5757 x 2080 19.8 / 13.5, 168 x 1760 x 1032 9.7 / 7.2.
-template <int EPI, bool DUAL>
+// F8: e4m3 operands, seen as rows of 16-bit words (lda, ldb, K in words). A lane's 16-byte chunk is 16
+// values of K, its halves the operands of two MFMAs: which K they are does not matter as long as
+// both operands agree.
+template <int EPI, bool DUAL, bool F8 = false>
 __global__ __launch_bounds__(256) void gemm_small(Args a) {
   constexpr int BM = 64, BN = 64, ST = 4;
   constexpr int FM = BM / 32, FN = BN / 32, LA = BM / 32, LB = BN / 32, STAGE = (BM + BN) * 128;
@@ -329,10 +335,25 @@ __global__ __launch_bounds__(256) void gemm_small(Args a) {
 #pragma unroll
       for (int i = 0; i < FM; ++i)
 #pragma unroll
-        for (int n = 0; n < FN; ++n) acc[i][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[n], fa[i], acc[i][n], 0, 0, 0);
+        for (int n = 0; n < FN; ++n) {
+          if constexpr (F8) {
+            const auto x = __builtin_bit_cast(i64x2, fa[i]), y = __builtin_bit_cast(i64x2, fb[n]);
+            acc[i][n] = __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(y[0], x[0], acc[i][n], 0, 0, 0);
+            acc[i][n] = __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(y[1], x[1], acc[i][n], 0, 0, 0);
+          } else {
+            acc[i][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[n], fa[i], acc[i][n], 0, 0, 0);
+          }
+        }
     }
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the tail's loads land before LDS is released
+  if constexpr (F8) {
+    const float f = a.alpha_ptr ? a.alpha * *a.alpha_ptr : a.alpha;
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int n = 0; n < FN; ++n) acc[i][n] *= f;
+  }
   const int mw = m0 + (w >> 1) * (BM / 2) + fr, nw = n0 + (w & 1) * (BN / 2);
   const int lc = (fq & 1) * 16 + (fq >> 1) * 8;
   float bv[FN][4];
@@ -767,7 +788,7 @@ int gemm_any(const void* A, const void* B, void* C, void* C2, const void* bias, 
   Plan p = bm ? Plan{bm, bn, ns} : plan(M, N, K, ws != nullptr, cu_count());
   if (p.ns > 1 && ws == nullptr) return KGS_ERR_ARG;
   const Args a{(const unsigned short*)A, (const unsigned short*)B, C, (unsigned short*)C2, (const unsigned short*)bias,
-               M, N, K, lda, ldb, ldc, 0, M > N, vec};
+               M, N, K, lda, ldb, ldc, 0, M > N, vec, 1.f, nullptr};
   if (C2) {
     switch (epi) {
       case EPI_BIAS_GELU: return launch<EPI_BIAS_GELU, true>(a, p, ws, s);
@@ -793,7 +814,7 @@ int gemm_any_swiglu(const void* A, const void* B, void* C, int M, int N, int K, 
                     const float* limit, hipStream_t s) {
   using namespace any;
   const Args a{(const unsigned short*)A, (const unsigned short*)B, C, nullptr, (const unsigned short*)limit,
-               M, N, K, lda, ldb, ldc, 0, M > N, ldc % 8 == 0 && (uintptr_t)C % 16 == 0};
+               M, N, K, lda, ldb, ldc, 0, M > N, ldc % 8 == 0 && (uintptr_t)C % 16 == 0, 1.f, nullptr};
   const Plan p = plan(M, N, K, false, cu_count());
   const int bm = p.bm == 256 ? 256 : 128, bn = bm == 256 && p.bn == 256 ? 256 : 128;
   const dim3 grid((unsigned)(ceil_div(M, bm) * ceil_div(N / 2, bn / 2)));
@@ -809,6 +830,27 @@ int gemm_any_swiglu(const void* A, const void* B, void* C, int M, int N, int K, 
     KGS_SWT(GATE_SILU);
   }
 #undef KGS_SWT
+  return (int)hipGetLastError();
+}
+
+// e4m3 operands on 64x64 tiles, sizes in 16-bit words (kgs_gemm_fp8_nt_dev)
+int gemm_any_f8(const void* A, const void* B, void* C, const void* bias, int M, int N, int Kw, int lda, int ldb, int ldc,
+                float alpha, const float* alpha_ptr, int epi, hipStream_t s) {
+  using namespace any;
+  if (!gemm_any_ok(A, B, M, N, Kw, lda, ldb)) return KGS_ERR_ALIGN;
+  const Args a{(const unsigned short*)A, (const unsigned short*)B, C, nullptr, (const unsigned short*)bias, M, N, Kw, lda, ldb,
+               ldc, 0, 0, ldc % 8 == 0 && (uintptr_t)C % 16 == 0, alpha, alpha_ptr};
+  const dim3 grid((unsigned)(ceil_div(M, 64) * ceil_div(N, 64)));
+#define KGS_F8(E) hipLaunchKernelGGL((gemm_small<E, false, true>), grid, dim3(256), 0, s, a)
+  switch (epi) {
+    case EPI_NONE: KGS_F8(EPI_NONE); break;
+    case EPI_BIAS: KGS_F8(EPI_BIAS); break;
+    case EPI_BIAS_GELU: KGS_F8(EPI_BIAS_GELU); break;
+    case EPI_BIAS_RELU: KGS_F8(EPI_BIAS_RELU); break;
+    case EPI_BIAS_SILU: KGS_F8(EPI_BIAS_SILU); break;
+    default: return KGS_ERR_ARG;
+  }
+#undef KGS_F8
   return (int)hipGetLastError();
 }
 

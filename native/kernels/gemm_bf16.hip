@@ -170,6 +170,8 @@ int gemm_any_ok(const void* A, const void* B, int M, int N, int K, int lda, int 
 int gemm_any(const void* A, const void* B, void* C, void* C2, const void* bias, int M, int N, int K, int lda, int ldb,
              int ldc, int epi, int bm, int bn, int ns, float* ws, hipStream_t s);
 long gemm_any_ws(int M, int N, int K);
+int gemm_any_f8(const void* A, const void* B, void* C, const void* bias, int M, int N, int Kw, int lda, int ldb, int ldc,
+                float alpha, const float* alpha_ptr, int epi, hipStream_t s);
 int gemm_any_swiglu(const void* A, const void* B, void* C, int M, int N, int K, int lda, int ldb, int ldc, int act,
                     const float* limit, hipStream_t s);
 
@@ -524,10 +526,21 @@ KGS_EXPORT int kgs_gemm_fp8_nt_dev(const void* A, const void* B, void* C, const 
   // the four-wave kernel wherever it can run: 4096 x 4096 x 14336 (a tile per CU) 145 us, the
   // eight-wave one 218; 1024 x 4096 x 4096 (a quarter of the CUs) 37 and 65
   if (variant == 0) v = w4p ? 3 : fast ? 1 : 16;
-  else if (variant == 1 || variant == 16) v = variant;
+  else if (variant == 1 || variant == 16 || variant == 64) v = variant;
   else if (variant == 3) { if (!w4p) return KGS_ERR_ALIGN; v = 3; }
   else return KGS_ERR_ARG;
-  if (!(v == 16 ? bounded : fast)) return KGS_ERR_ALIGN;
+  if (!(v >= 16 ? bounded : fast)) return KGS_ERR_ALIGN;
+  if (variant == 0) {
+    // 64x64 tiles (0.3 us a 128-deep K-step, several on a CU) against 256x256 ones (1.2 us) by how often
+    // each fills the chip; us, large / small: 256 x 64 x 1024 14.9 / 4.7, 1024^3 16.5 / 5.3, 2048^3 25.3 /
+    // 18.4, 3000 x 2000 x 1504 20.0 / 24.3, 3968 x 2688 x 4160 46 / 93
+    const double small = ((M + 63) / 64) * (double)((N + 63) / 64) / kgs::cu_count();
+    const long large = ((M + 255) / 256) * (long)((N + 255) / 256), steps = (K + 127) / 128;
+    const long rounds = (large + kgs::cu_count() - 1) / kgs::cu_count();
+    if (2.8 + steps * (small <= 1 ? 0.3 : 0.06 + 0.3 * small) < 4 + rounds * steps * 1.2) v = 64;
+  }
+  if (v == 64)
+    return kgs::gemm_any_f8(A, B, C, bias, M, N, K / 2, lda / 2, ldb / 2, ldc, alpha, alpha_ptr, epi, stream);
   auto a = (const unsigned short*)A;
   auto b = (const unsigned short*)B;
   auto c = (unsigned short*)C;

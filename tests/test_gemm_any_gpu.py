@@ -297,3 +297,32 @@ def test_gelu_over_its_range():
     assert bool(((gz[:, 0].double() - d).abs() <= 2.0 ** -8 * d.abs() * 1.01 + 1e-6).all())
     y = gemm_nt(torch.tensor([[float("inf")] + 7 * [0.0]], device=DEV).bfloat16(), one, act="gelu")
     assert bool((y == float("inf")).all())
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 8, 16), (64, 64, 128), (65, 72, 144), (130, 200, 1040), (256, 256, 1024), (63, 264, 640)])
+@pytest.mark.parametrize("epi", [0, 1, 2, 3, 4])
+def test_small_fp8_tiles(M, N, K, epi):
+    """e4m3 operands on 64x64 tiles at their edges, every epilogue, host and device scales; a row below the
+    output stays as it is."""
+    from kgs.ops import _lib
+
+    a, b = (rnd(r, K).to(torch.float8_e4m3fn) for r in (M, N))
+    bias, scale = rnd(1, N)[0].contiguous(), torch.tensor([0.75], device=DEV)
+    z = 0.5 * (a.double() @ b.double().T)
+    for ptr in (None, scale.data_ptr()):
+        c = torch.full((M + 1, N), 5.0, device=DEV, dtype=torch.bfloat16)
+        rc = _lib.lib().kgs_gemm_fp8_nt_dev(a.data_ptr(), b.data_ptr(), c.data_ptr(), bias.data_ptr() if epi else None, M, N, K, K, K, N,
+                                            0.5, ptr, epi, 64, _lib.stream_handle(a.device))
+        assert rc == 0
+        want = z * (0.75 if ptr else 1.0) + (bias.double() if epi else 0.0)
+        f = [lambda v: v, lambda v: v, lambda v: torch.nn.functional.gelu(v, approximate="tanh"), torch.relu, torch.nn.functional.silu][epi]
+        assert rel(c[:M], f(want)) < 2 * REL and bool((c[M] == 5).all())
+
+
+@pytest.mark.parametrize("M,N,K", [(24, 88, 128), (1024, 1024, 1024), (512, 512, 4096), (2560, 3200, 576), (2048, 2048, 2048)])
+def test_fp8_auto_either_side_of_the_rule(M, N, K):
+    from kgs.ops.gemm import gemm_fp8_nt
+
+    a, b = (rnd(r, K).to(torch.float8_e4m3fn) for r in (M, N))
+    want = a.double() @ b.double().T
+    assert rel(gemm_fp8_nt(a, b), want) < REL and rel(gemm_fp8_nt(a, b, variant="bounded"), want) < REL

@@ -337,7 +337,8 @@ class ServingModel:
         if self.prefill_f8 is not None:
             return self._prefill_fp8(tokens, positions, slots, seq_starts, seq_lens, padded_lens)
         seqs = [(int(s), int(n), int(p), 0) for s, n, p in zip(seq_starts, seq_lens, padded_lens)]
-        if self.packed is not None and not self.decode_fp8 and 0 < sum(n for _, n, _, _ in seqs) <= self.fused_max_batch:
+        if self.packed is not None and not self.decode_fp8 and 0 < sum(n for _, n, _, _ in seqs) <= self.fused_max_batch and \
+                all(w.n % 64 == 0 and w.k % 512 == 0 for w in (*self.packed[0].values(), self.packed_lm)):  # skinny_gemm's tiles
             return self._prefill_fused(tokens, positions, slots, seqs)
         plan = self._prompt_rows(seqs, tokens.numel(), tokens.device)
         if plan.keep is not None:

@@ -204,15 +204,16 @@ def test_gather_kv_bits(fp8, kv, ctx, rows):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("lens", [[20, 5], [48], [49], [130, 126], [100, 157], [300, 260]])
-def test_prefill_by_rows(lens):
+@pytest.mark.parametrize("lens,ff", [([20, 5], 2048), ([48], 2048), ([49], 2048), ([130, 126], 2048), ([100, 157], 2048), ([300, 260], 2048),
+                                     ([20, 5], 2304)])  # 2304: no skinny tile of down
+def test_prefill_by_rows(lens, ff):
     """Either side of the row counts where a prompt step changes its layers: logits and cache of the step
     against float32 layers on the same weights. Sums round to bf16 at other places on either side: a
     few 2^-8 in the 2-norm over two layers."""
     from kgs.models.llama import LlamaConfig
     from kgs.serve.model import ServingModel
 
-    cfg = LlamaConfig(hidden=2048, intermediate=2048, heads=16, kv_heads=4, layers=2, vocab=1024)
+    cfg = LlamaConfig(hidden=2048, intermediate=ff, heads=16, kv_heads=4, layers=2, vocab=1024)
     ours, ref = (ServingModel(cfg, device=DEV, backend=b, num_pages=40, max_model_len=1024) for b in ("kgs", "ref"))
     padded = [-(-n // 128) * 128 for n in lens]
     total, rng = sum(padded), np.random.default_rng(len(lens))

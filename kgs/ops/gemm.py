@@ -74,17 +74,21 @@ def gemm_nt(
         _check_operand(out, "out")
         if tuple(out.shape) != (M, N):
             raise ValueError(f"out has shape {tuple(out.shape)}, expected {(M, N)}")
-    if variant == "auto" and K > PAD_MIN_K:
+    pa, pb, lda, ldb = a.data_ptr(), b.data_ptr(), a.stride(0), b.stride(0)
+    if variant == "auto" and K > PAD_MIN_K and (K % 8 or (lda | ldb) % 8 or (pa | pb) % 16):
         a, b = _even(a, b)
         K = a.shape[1]
-    ptrs = (a.data_ptr(), b.data_ptr(), out.data_ptr(), bias.data_ptr() if bias is not None else None, M, N, K,
-            a.stride(0), b.stride(0), out.stride(0), epi)
+        pa, pb, lda, ldb = a.data_ptr(), b.data_ptr(), a.stride(0), b.stride(0)
+    pbias = bias.data_ptr() if bias is not None else None
     if variant == "auto":
         ws = _scratch(M, N, K, a.device)
-        rc = _lib.lib().kgs_gemm_bf16_nt_auto(*ptrs, None if ws is None else ws.data_ptr(), _lib.stream_handle(a.device))
+        rc = _lib.lib().kgs_gemm_bf16_nt_auto(pa, pb, out.data_ptr(), pbias, M, N, K, lda, ldb, out.stride(0), epi,
+                                              None if ws is None else ws.data_ptr(), _lib.stream_handle(a.device))
     else:
-        rc = _lib.lib().kgs_gemm_bf16_nt(*ptrs, VARIANTS[variant], _lib.stream_handle(a.device))
-    _lib.check(rc, f"gemm_nt[{M}x{N}x{K}]")
+        rc = _lib.lib().kgs_gemm_bf16_nt(pa, pb, out.data_ptr(), pbias, M, N, K, lda, ldb, out.stride(0), epi, VARIANTS[variant],
+                                         _lib.stream_handle(a.device))
+    if rc:
+        _lib.check(rc, f"gemm_nt[{M}x{N}x{K}]")
     return out
 
 
@@ -515,7 +519,8 @@ def gemm_fp8_nt(
         a.data_ptr(), b.data_ptr(), out.data_ptr(), bias.data_ptr() if bias is not None else None,
         M, N, K, a.stride(0), b.stride(0), out.stride(0), alpha, alpha_ptr, epi,
         FP8_VARIANTS[variant], _lib.stream_handle(a.device))
-    _lib.check(rc, f"gemm_fp8_nt[{M}x{N}x{K}]")
+    if rc:
+        _lib.check(rc, f"gemm_fp8_nt[{M}x{N}x{K}]")
     return out
 
 

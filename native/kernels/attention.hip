@@ -106,8 +106,8 @@ __device__ __forceinline__ int off(int r, int c) { return 2 * HD * r + 16 * (c ^
 
 __device__ __forceinline__ bf16x8 pack8(const f32x16& s, int base) { return pack_bf16x8(s, base); }
 
-template <int HD, Mode MODE, int HR = 0>
-__global__ __launch_bounds__(256, 2) __attribute__((amdgpu_waves_per_eu(2, 2))) void fwd(Args a) {
+template <int HD, Mode MODE, int HR>
+__device__ __forceinline__ void forward(const Args& a) {
   constexpr bool RAGGED = MODE == RAGGED_ROWS, PART = MODE != EQUAL;
   constexpr int TILE_BYTES = KB * HD * 2;  // 16 KB at 128
   constexpr int ND = HD / 32, NK = HD / 16, NR = HR / 16, ROT_BYTES = KB * HR * 2;
@@ -414,6 +414,14 @@ __global__ __launch_bounds__(256, 2) __attribute__((amdgpu_waves_per_eu(2, 2))) 
     }
 }
 
+template <int HD, Mode MODE, int HR = 0>
+__global__ __launch_bounds__(256, 2) __attribute__((amdgpu_waves_per_eu(2, 2))) void fwd(Args a) {
+  forward<HD, MODE, HR>(a);
+}
+__global__ __launch_bounds__(256, 2) __attribute__((amdgpu_waves_per_eu(2, 2))) void blocks(Args a) {
+  forward<128, BLOCKS, 0>(a);
+}
+
 // The parts of a split block (x) and head (y): out = sum_p w_p O_p / sum_p w_p l_p with
 // w_p = 2^((m_p - max m) sl2). merges: first row, rows, first slot, parts. A thread per row, 16 dims (z).
 __global__ __launch_bounds__(QB) void merge_parts(const float* __restrict__ ws, const int4* __restrict__ merges,
@@ -541,7 +549,7 @@ KGS_EXPORT int kgs_attn_fwd_blocks_bf16(const void* q, const void* k, const void
          ldq, ldk, ldv, ldo, 0, 0, H, HKV, scale * 1.4426950408889634f, 1, 0, 0,
          (const int4*)items, nullptr, 0, 0, 0, nullptr, 0, nullptr, nullptr, 0, 0, 0,
          (const unsigned short*)k2, (const unsigned short*)v2, ld2, ws, slots};
-  hipLaunchKernelGGL((fwd<128, BLOCKS>), dim3((unsigned)(nitems * H)), dim3(256), 0, s, a);
+  hipLaunchKernelGGL(blocks, dim3((unsigned)(nitems * H)), dim3(256), 0, s, a);
   if (merges)
     hipLaunchKernelGGL(merge_parts, dim3((unsigned)nmerge, (unsigned)H, 8), dim3(QB), 0, s, ws, (const int4*)merges,
                        (unsigned short*)o, H, ldo, a.sl2);

@@ -29,11 +29,9 @@
 #   serve_nt_ab  batch-$B serving with nt weight loads off / on / on + SwiGLU-packed gate|up, twice
 #   serve_overlap_ab  batch-$B serving, sequential vs overlapped engine steps, twice
 #   mall_probe   batch-256 decode projections with weights cold (HBM) vs hot (MALL)
-#   serve_nt_rep the round-4 faulting serving configuration (nt on, output 256) x2, nt off, nt on traced
 #   uninit_probe serving under allocator fill patterns 0 / 0x400 (uninitialised reads show as a difference)
 #   serve_rep    batch-256 serving $N times back to back with step breadcrumbs (KGS_STEP_TRACE)
 #   serve_tq     batch-256 serving, ticket pool checked after every step, with and without hipGraphs
-#   prefix_regress  the graph-replay regression test against gpurun_ab/prefix (the pre-fix library)
 #   overlap_rccl_ab persistent (static first ticket) vs one-shot grid against the RCCL-shaped CU hold
 #   lib_ab       this tree's kernel library vs another build ($LIB_B), interleaved, five sweep shapes
 #   fp8_sweep    kgs fp8 vs hipBLASLt fp8, N(0,1) operands ($SHAPES, $VARIANTS: e.g. w4f8_<X>_<B1>_<R>_<P> knobs)
@@ -58,8 +56,6 @@
 #   gemm_tail    per-workgroup start / per-tile end stamps of the persistent GEMM (head, tail, XCD spread)
 #   w4x_sweep    decode-batch GEMM sweep (four-wave tiles, slices, stages vs hipBLASLt)
 #   kt           GPU tests matching $KT (pytest -k)
-#   memset_repro pure-HIP hipGraph memset-node check ($G graphs, $R replays, $P extra nodes; no torch);
-#                memset_repro_torch: the same binary on torch's bundled HIP runtime
 #   attn_bench   flash-attention forward vs SDPA
 #   serve_b16    batch-16 serving; skinny_tune: skinny GEMM variant x split-K tune at batches $MS
 #   online_sweep online serving (Poisson arrivals, 2048-row chunked steps) at 8-96 req/s
@@ -187,16 +183,6 @@ step() {
             done ;;
         rope_probe) run rope_probe 200 python bench/rope_cache_probe.py &&
             (export KGS_KERNELS_LIB=$LIB_B; run rope_probe_libb 200 python bench/rope_cache_probe.py) ;;
-        serve_nt_rep)  # the round-4 faulting configuration (batch $B, output 256, nt on) twice, nt off,
-            # then nt on under a kernel trace (the last dispatches name a faulting kernel)
-            local SB="python -u -m kgs.serve bench --requests ${B:-256} --input-len 512 --output-len 256"
-            SB="$SB --max-batch ${B:-256} --max-model-len 2048"
-            (export KGS_NT_WEIGHTS=1; run serve_nt1_a 300 $SB) &&
-            (export KGS_NT_WEIGHTS=1; run serve_nt1_b 300 $SB) &&
-            (export KGS_NT_WEIGHTS=0; run serve_nt0_a 300 $SB) &&
-            (export KGS_NT_WEIGHTS=1; run serve_nt1_trace 300 rocprofv3 --kernel-trace --stats --output-format csv \
-                -d "$O/nt1_trace" -o d -- python3 -m kgs.serve bench --requests ${B:-256} --input-len 512 \
-                --output-len 256 --max-batch ${B:-256} --max-model-len 2048) ;;
         uninit_probe)  # serving under two allocator fill patterns (bench/uninit_probe.py): must agree bitwise
             (export KGS_STEP_TRACE="$O/steps_u0.log"; run uninit_0 300 python bench/uninit_probe.py --pattern 0 \
                 --out "$O/uninit_0.json") &&
@@ -215,11 +201,6 @@ step() {
             (export KGS_STEP_TRACE="$O/steps_tq_graphs.log" KGS_TQ_CHECK=1; run serve_tq_graphs 300 $SB)
             [ $? -le 1 ] &&
             (export KGS_STEP_TRACE="$O/steps_tq_eager.log" KGS_TQ_CHECK=1; run serve_tq_eager 300 $SB --no-graphs) ;;
-        prefix_regress)  # the replay regression test against the pre-fix library (memset node): expected to fail
-            (export KGS_KERNELS_LIB=gpurun_ab/prefix/libkgs_kernels.so
-             run prefix_regress 300 python -u -m pytest tests/test_kernels_gpu.py -x -v -k captured_persistent \
-                --timeout 120 --timeout-method thread)
-            [ $? -le 1 ] ;;  # 1 = the test failed (the point); a fault / kill still stops the chain
         overlap_rccl_ab) run overlap_rccl_ab 400 python bench/overlap_rccl.py --policies static,oneshot \
             --out "$O/overlap_rccl_ab.json" ;;
         lib_ab)  # two builds of libkgs_kernels.so interleaved in one process ($LIB_B, default the pre-pack build)
@@ -394,12 +375,6 @@ step() {
             for r in 1 2; do
                 run online_seq_$r 300 $OB --overlap off && run online_ovl_$r 300 $OB --overlap on || return 1
             done ;;
-        memset_repro) run memset_repro 300 kgs/_native/kgs-graph-memset-repro ${G:-4} ${R:-200} ${P:-8} ;;
-        memset_repro_torch)  # the same binary on torch's bundled HIP runtime (the one the serving engine used)
-            local th=/tmp/kgs_torchhip
-            mkdir -p $th && ln -sf "$(python3 -c 'import os, torch; print(os.path.join(os.path.dirname(torch.__file__), "lib", "libamdhip64.so"))')" $th/libamdhip64.so.7 &&
-            LD_LIBRARY_PATH=$th${LD_LIBRARY_PATH:+:$LD_LIBRARY_PATH} run memset_repro_torch 300 \
-                kgs/_native/kgs-graph-memset-repro ${G:-4} ${R:-200} ${P:-8} ;;
         kt) run kt 600 python -u -m pytest tests -x -v -m gpu -k "$KT" --timeout 120 --timeout-method thread ;;
         *) echo "unknown step $1" >&2; return 2 ;;
     esac

@@ -624,9 +624,14 @@ def gemm_bf16(a: torch.Tensor, b: torch.Tensor, trans_a: bool = False, trans_b: 
     N, K2 = (b.shape[0], b.shape[1]) if trans_b else (b.shape[1], b.shape[0])
     if K != K2:
         raise ValueError(f"inner dims differ: op(a) {M}x{K}, op(b) {K2}x{N}")
+    if a.device != b.device:
+        raise ValueError("a and b on different devices")
+    if out is not None:
+        _check_operand(out, "out")
+        if tuple(out.shape) != (M, N) or out.device != a.device:
+            raise ValueError(f"out is {tuple(out.shape)} on {out.device}, expected {(M, N)} on {a.device}")
     ta, tb = int(trans_a), int(not trans_b)  # kernel flags: 1 = operand stored [K][rows]
-    if (ta or tb) and bias is None and act in (None, "none") and not TR_READ_A and M and N and K and \
-            (out is None or tuple(out.shape) == (M, N)):
+    if (ta or tb) and bias is None and act in (None, "none") and not TR_READ_A and M and N and K:
         return _product(*_even(a, b), out, M, N, K, ta, tb)
     return _general(a, b, out, M, N, K, ta, tb, bias, act)
 

@@ -405,6 +405,24 @@ def skinny_config(m: int, n: int, k: int, fp8: bool = False) -> tuple[int, int]:
     return v, choose_ksplit(m, n, k, variant=v)
 
 
+def _skinny_plan(m: int, w: "PackedWeight", rope: bool) -> tuple[int, int]:
+    variant, ks = skinny_config(m, w.n, w.k, fp8=w.fp8)
+    if rope and SKINNY_VARIANTS[variant][0] != 1:
+        # the RoPE epilogue is built for one-tile waves (R 1)
+        variant, ks = skinny_rule(m, w.n, w.k, one=True)
+    return variant, ks
+
+
+def skinny_takes(m: int, w: "PackedWeight") -> bool:
+    """Whether :func:`skinny_gemm` runs ``m`` rows of ``w``: up to 256 (64 of an e4m3 weight, and of a
+    RoPE-packed one, whose epilogue is built for these), on the strips and chunks of its choice."""
+    if not 0 < m <= (64 if w.fp8 or w.rope else 256):
+        return False
+    variant, _ = _skinny_plan(m, w, bool(w.rope))
+    strip, chunk, _ = skinny_geometry(m, variant)
+    return w.n % strip == 0 and w.k % chunk == 0
+
+
 def use_skinny(m: int, n: int, k: int) -> bool:
     """Decode routing: True = skinny GEMM, False = the library GEMM (hipBLASLt)."""
     if not 0 < m <= 256:
@@ -480,10 +498,7 @@ def skinny_gemm(x: torch.Tensor, w: PackedWeight, out: torch.Tensor | None = Non
     if w.fp8 and _mt(m) > 4:
         raise ValueError("fp8 (W8A16) skinny GEMM covers batches <= 64")
     if variant == 0 and ksplit is None:
-        variant, ks = skinny_config(m, w.n, k, fp8=w.fp8)
-        if rope is not None and SKINNY_VARIANTS[variant][0] != 1:
-            # the RoPE epilogue is built for one-tile waves (R 1)
-            variant, ks = skinny_rule(m, w.n, k, one=True)
+        variant, ks = _skinny_plan(m, w, rope is not None)
     else:
         ks = ksplit if ksplit is not None else choose_ksplit(m, w.n, k, variant=variant)
     rps, kpc, mpad = skinny_geometry(m, variant)

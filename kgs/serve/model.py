@@ -6,7 +6,7 @@ Two step kinds, both driven by the native scheduler's plans
 
 * **prefill** -- the prompts of newly admitted sequences, each padded to a
   multiple of 128 tokens and concatenated (the layers drop the padding where that
-  saves a tile of rows; steps of up to ``fused_max_batch`` rows run the FUSED layer
+  saves a tile of rows; steps of up to ``fused_max_batch`` rows, 64 at most, run the FUSED layer
   below, of up to 256 the split tiles): every projection is one
   :func:`kgs.ops.gemm_nt` (256x256 MFMA pipeline), RoPE + the KV-cache scatter
   is one :func:`kgs.ops.decode.rope_cache_` launch, attention is one
@@ -337,8 +337,7 @@ class ServingModel:
         if self.prefill_f8 is not None:
             return self._prefill_fp8(tokens, positions, slots, seq_starts, seq_lens, padded_lens)
         seqs = [(int(s), int(n), int(p), 0) for s, n, p in zip(seq_starts, seq_lens, padded_lens)]
-        if self.packed is not None and not self.decode_fp8 and 0 < sum(n for _, n, _, _ in seqs) <= self.fused_max_batch and \
-                all(w.n % 64 == 0 and w.k % 512 == 0 for w in (*self.packed[0].values(), self.packed_lm)):  # skinny_gemm's tiles
+        if self._fused_prompts(sum(n for _, n, _, _ in seqs), len(seqs)):
             return self._prefill_fused(tokens, positions, slots, seqs)
         plan = self._prompt_rows(seqs, tokens.numel(), tokens.device)
         if plan.keep is not None:
@@ -385,6 +384,13 @@ class ServingModel:
         out = self._proj(yl, None, "lm", True)
         T.op("prefill lm_head")
         return out
+
+    def _fused_prompts(self, rows: int, prompts: int) -> bool:
+        """Whether a step of so many prompt rows takes the fused decode layer: as many as a decode step of it,
+        64 at most (what its rotation takes), where its products tile."""
+        if self.packed is None or self.decode_fp8 or not 0 < rows <= min(self.fused_max_batch, 64):
+            return False
+        return all(D.skinny_takes(rows, w) for w in self.packed[0].values()) and D.skinny_takes(prompts, self.packed_lm)
 
     def _prefill_fused(self, tokens, positions, slots, seqs) -> torch.Tensor:
         """A prompt step of few rows on the fused decode layer (:meth:`_fused_layers`), without its padding:

@@ -204,9 +204,10 @@ def test_gather_kv_bits(fp8, kv, ctx, rows):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("lens,ff", [([20, 5], 2048), ([48], 2048), ([49], 2048), ([130, 126], 2048), ([100, 157], 2048), ([300, 260], 2048),
-                                     ([20, 5], 2304)])  # 2304: no skinny tile of down
-def test_prefill_by_rows(lens, ff):
+@pytest.mark.parametrize("lens,ff,fused", [([20, 5], 2048, 48), ([48], 2048, 48), ([49], 2048, 48), ([130, 126], 2048, 48), ([100, 157], 2048, 48),
+                                           ([300, 260], 2048, 48), ([20, 5], 2304, 48),  # 2304: no skinny tile of down
+                                           ([64], 2048, 128), ([65], 2048, 128), ([257], 2048, 300)])
+def test_prefill_by_rows(lens, ff, fused):
     """Either side of the row counts where a prompt step changes its layers: logits and cache of the step
     against float32 layers on the same weights. Sums round to bf16 at other places on either side: a
     few 2^-8 in the 2-norm over two layers."""
@@ -214,7 +215,7 @@ def test_prefill_by_rows(lens, ff):
     from kgs.serve.model import ServingModel
 
     cfg = LlamaConfig(hidden=2048, intermediate=ff, heads=16, kv_heads=4, layers=2, vocab=1024)
-    ours, ref = (ServingModel(cfg, device=DEV, backend=b, num_pages=40, max_model_len=1024) for b in ("kgs", "ref"))
+    ours, ref = (ServingModel(cfg, device=DEV, backend=b, num_pages=40, max_model_len=1024, fused_max_batch=fused) for b in ("kgs", "ref"))
     padded = [-(-n // 128) * 128 for n in lens]
     total, rng = sum(padded), np.random.default_rng(len(lens))
     tok, pos, slot, at, page, starts = np.zeros(total, np.int32), np.zeros(total, np.int32), np.full(total, -1, np.int32), 0, 1, []

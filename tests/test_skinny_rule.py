@@ -22,6 +22,41 @@ def test_rule_is_launchable():
                     assert not one or D.SKINNY_VARIANTS[v][0] == 1 or m > 64
 
 
+class _Weight:
+    def __init__(self, n, k, rope=None, fp8=False):
+        self.n, self.k, self.rope, self.fp8 = n, k, rope, fp8
+
+
+def test_what_the_skinny_gemm_takes():
+    """Its own choice of a variant has to tile the weight, and the rotation's to have one-tile waves."""
+    for m in range(1, 258):
+        for w in (_Weight(3072, 2048), _Weight(3072, 2048, rope=(16, 4)), _Weight(3072, 2048, fp8=True), _Weight(3136, 2048), _Weight(2048, 2304)):
+            most = 64 if w.rope or w.fp8 else 256
+            ok = D.skinny_takes(m, w)
+            if m > most:
+                assert not ok
+                continue
+            v, ks = D._skinny_plan(m, w, bool(w.rope))
+            rps, kpc, _ = D.skinny_geometry(m, v)
+            assert ok == (w.n % rps == 0 and w.k % kpc == 0) and (not ok or (w.k // kpc) % ks == 0)
+            assert not w.rope or D.SKINNY_VARIANTS[v][0] == 1
+    assert D.skinny_takes(64, _Weight(3072, 2048, rope=(16, 4))) and D.skinny_takes(200, _Weight(3072, 2048))
+    assert not D.skinny_takes(200, _Weight(3136, 2048)) and not D.skinny_takes(1, _Weight(2048, 2304))
+
+
+@pytest.mark.parametrize("most,rows,fused", [(48, 48, True), (48, 49, False), (128, 64, True), (128, 65, False), (300, 257, False), (0, 1, False)])
+def test_prompt_rows_of_the_fused_layer(most, rows, fused):
+    """A larger fused_max_batch takes no prompt to products that are not built for it."""
+    from kgs.serve.model import ServingModel
+
+    class M:
+        decode_fp8, fused_max_batch = False, most
+        packed = [{"qkv": _Weight(3072, 2048, rope=(16, 4)), "o": _Weight(2048, 2048), "gate_up": _Weight(16384, 2048), "down": _Weight(2048, 8192)}]
+        packed_lm = _Weight(1024, 2048)
+
+    assert ServingModel._fused_prompts(M, rows, 1) is fused
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("m,v", [(17, 22), (32, 22), (24, 23), (33, 24), (64, 24), (40, 25)])
 def test_k_split_in_the_workgroup(m, v):

@@ -21,6 +21,7 @@ on CPU too and define the cache layout for tests).
 from __future__ import annotations
 
 import math
+from functools import lru_cache
 import os
 
 import torch
@@ -405,22 +406,22 @@ def skinny_config(m: int, n: int, k: int, fp8: bool = False) -> tuple[int, int]:
     return v, choose_ksplit(m, n, k, variant=v)
 
 
-def _skinny_plan(m: int, w: "PackedWeight", rope: bool) -> tuple[int, int]:
-    variant, ks = skinny_config(m, w.n, w.k, fp8=w.fp8)
+def _skinny_plan(m: int, n: int, k: int, fp8: bool, rope: bool) -> tuple[int, int]:
+    variant, ks = skinny_config(m, n, k, fp8=fp8)
     if rope and SKINNY_VARIANTS[variant][0] != 1:
         # the RoPE epilogue is built for one-tile waves (R 1)
-        variant, ks = skinny_rule(m, w.n, w.k, one=True)
+        variant, ks = skinny_rule(m, n, k, one=True)
     return variant, ks
 
 
-def skinny_takes(m: int, w: "PackedWeight") -> bool:
-    """Whether :func:`skinny_gemm` runs ``m`` rows of ``w``: up to 256 (64 of an e4m3 weight, and of a
+@lru_cache(maxsize=4096)
+def skinny_takes(m: int, n: int, k: int, fp8: bool = False, rope: bool = False) -> bool:
+    """Whether :func:`skinny_gemm` runs ``m`` rows of an ``[n, k]`` weight: up to 256 (64 of an e4m3 weight, and of a
     RoPE-packed one, whose epilogue is built for these), on the strips and chunks of its choice."""
-    if not 0 < m <= (64 if w.fp8 or w.rope else 256):
+    if not 0 < m <= (64 if fp8 or rope else 256):
         return False
-    variant, _ = _skinny_plan(m, w, bool(w.rope))
-    strip, chunk, _ = skinny_geometry(m, variant)
-    return w.n % strip == 0 and w.k % chunk == 0
+    strip, chunk, _ = skinny_geometry(m, _skinny_plan(m, n, k, fp8, rope)[0])
+    return n % strip == 0 and k % chunk == 0
 
 
 def use_skinny(m: int, n: int, k: int) -> bool:
@@ -466,7 +467,8 @@ def _workspace(device: torch.device, floats: int, ints: int):
     return ws, cnt
 
 
-EPI_SWIGLU, EPI_RMS, EPI_RESID, EPI_GELU, EPI_CLAMPED = 1, 2, 4, 16, 32
+EPI_SWIGLU, EPI_RMS, EPI_RESID, EPI_GELU, EPI_CLAMPED, EPI_SUMS_IN, EPI_SUMS_OUT = 1, 2, 4, 16, 32, 64, 128
+SUM_WORDS, SUM_MAX_N = 8, 8192  # integers of a row's exact sum of squares (decode.hip add_exact), longest row
 GATE_EPI = {"silu": 0, "gelu_tanh": EPI_GELU, "clamped": EPI_CLAMPED}
 
 
@@ -484,6 +486,9 @@ def skinny_gemm(x: torch.Tensor, w: PackedWeight, out: torch.Tensor | None = Non
       place (``out += x @ W^T``), and the new rows' sums of squares are added
       into ``resid_ss`` (for the next ``rms`` consumer);
     * ``zero`` (fp32 ``[M]``): cleared at kernel start (a consumed statistic);
+    * ``rms``, ``resid_ss`` and ``zero`` may be int64 ``[SUM_WORDS, M]`` instead (``resid_ss`` and ``zero`` alike,
+      rows of at most ``SUM_MAX_N``): exact sums, whose bits do not depend on the order in which
+      workgroups add to them;
     * ``rope`` (a ``rope=(H, HKV)``-packed qkv weight): dict of ``cos``, ``sin``
       (fp32 ``[max_pos, 64]``), ``positions`` and ``slots`` (int32 ``[M]``) and
       ``cache`` (the layer's bf16 pages): q / k rotated at their positions, k / v
@@ -498,7 +503,7 @@ def skinny_gemm(x: torch.Tensor, w: PackedWeight, out: torch.Tensor | None = Non
     if w.fp8 and _mt(m) > 4:
         raise ValueError("fp8 (W8A16) skinny GEMM covers batches <= 64")
     if variant == 0 and ksplit is None:
-        variant, ks = _skinny_plan(m, w, rope is not None)
+        variant, ks = _skinny_plan(m, w.n, k, w.fp8, rope is not None)
     else:
         ks = ksplit if ksplit is not None else choose_ksplit(m, w.n, k, variant=variant)
     rps, kpc, mpad = skinny_geometry(m, variant)
@@ -506,9 +511,17 @@ def skinny_gemm(x: torch.Tensor, w: PackedWeight, out: torch.Tensor | None = Non
         raise ValueError(f"skinny GEMM needs N % {rps} == 0 and K % {kpc} == 0 (N={w.n}, K={k})")
     epi = (EPI_SWIGLU | GATE_EPI[w.act.act] if w.swiglu else 0) | (EPI_RMS if rms is not None else 0) | \
         (EPI_RESID if resid_ss is not None else 0)
-    for t, name in ((rms, "rms"), (resid_ss, "resid_ss"), (zero, "zero")):
-        if t is not None and (t.dtype != torch.float32 or t.numel() < m or not t.is_contiguous()):
-            raise ValueError(f"{name} must be a contiguous fp32 vector of >= M elements")
+    for t, name, sums in ((rms, "rms", EPI_SUMS_IN), (resid_ss, "resid_ss", EPI_SUMS_OUT), (zero, "zero", EPI_SUMS_OUT)):
+        if t is None:
+            continue
+        if t.dtype == torch.int64 and t.shape == (SUM_WORDS, m):
+            epi |= sums
+        elif t.dtype != torch.float32 or t.numel() < m:
+            raise ValueError(f"{name} must be a contiguous fp32 vector of >= M elements, or int64 [{SUM_WORDS}, M]")
+        if not t.is_contiguous():
+            raise ValueError(f"{name} must be contiguous")
+    if epi & EPI_SUMS_OUT and resid_ss is not None and zero is not None and resid_ss.dtype != zero.dtype:
+        raise ValueError("resid_ss and zero must be of one kind")
     if resid_ss is not None:
         if w.swiglu or out is None or tuple(out.shape) != (m, w.n):
             raise ValueError("resid_ss needs the residual stream as out [M, N] (and no swiglu)")
@@ -520,7 +533,7 @@ def skinny_gemm(x: torch.Tensor, w: PackedWeight, out: torch.Tensor | None = Non
     else:
         if counters.dtype != torch.int32 or not counters.is_contiguous() or counters.numel() < w.n // rps:
             raise ValueError(f"counters must be at least {w.n // rps} contiguous int32")
-        ws, cnt = torch.empty(max(need, 4), dtype=torch.float32, device=x.device), counters
+        ws, cnt = torch.empty(need, dtype=torch.float32, device=x.device) if need else None, counters
     if (rope is not None) != bool(w.rope):
         raise ValueError("rope= needs a rope-packed qkv weight (PackedWeight(..., rope=(H, HKV))) and vice versa")
     if rope is not None:
@@ -534,15 +547,15 @@ def skinny_gemm(x: torch.Tensor, w: PackedWeight, out: torch.Tensor | None = Non
             if v.dtype != torch.int32 or not v.is_contiguous() or v.numel() < m:
                 raise ValueError(f"{key} must be a contiguous int32 vector of >= M elements")
         rc = _lib.lib().kgs_skinny_gemm_bf16_rope(
-            w.data.data_ptr(), x.data_ptr(), out.data_ptr(), ws.data_ptr(), cnt.data_ptr(), m, w.n, k, x.stride(0),
-            out.stride(0), ks, variant, EPI_RMS if rms is not None else 0,
+            w.data.data_ptr(), x.data_ptr(), out.data_ptr(), None if ws is None else ws.data_ptr(), cnt.data_ptr(), m, w.n, k, x.stride(0),
+            out.stride(0), ks, variant, epi & (EPI_RMS | EPI_SUMS_IN),
             rms.data_ptr() if rms is not None else None, 1.0 / k, float(eps), rope["cos"].data_ptr(),
             rope["sin"].data_ptr(), rope["positions"].data_ptr(), rope["slots"].data_ptr(), cache.data_ptr(),
             w.rope[0], w.rope[1], _lib.stream_handle(x.device))
         _lib.check(rc, f"skinny_gemm_rope[{m}x{w.n}x{k}, variant={variant}, ksplit={ks}]")
         return out
     rc = _lib.lib().kgs_skinny_gemm_bf16_fused(
-        w.data.data_ptr(), x.data_ptr(), out.data_ptr(), ws.data_ptr(), cnt.data_ptr(), m, w.n, k, x.stride(0),
+        w.data.data_ptr(), x.data_ptr(), out.data_ptr(), None if ws is None else ws.data_ptr(), cnt.data_ptr(), m, w.n, k, x.stride(0),
         out.stride(0), ks, variant, epi, rms.data_ptr() if rms is not None else None,
         resid_ss.data_ptr() if resid_ss is not None else None, zero.data_ptr() if zero is not None else None,
         1.0 / k, float(eps), w.wscale.data_ptr() if w.fp8 else None, w.act.limit, _lib.stream_handle(x.device))

@@ -387,10 +387,12 @@ class ServingModel:
 
     def _fused_prompts(self, rows: int, prompts: int) -> bool:
         """Whether a step of so many prompt rows takes the fused decode layer: as many as a decode step of it,
-        64 at most (what its rotation takes), where its products tile."""
-        if self.packed is None or self.decode_fp8 or not 0 < rows <= min(self.fused_max_batch, 64):
+        64 at most (what its rotation takes), where its products tile and its rows' statistics are exact sums."""
+        if self.packed is None or self.decode_fp8 or not 0 < rows <= min(self.fused_max_batch, 64) or \
+                self.packed[0]["o"].n > D.SUM_MAX_N:
             return False
-        return all(D.skinny_takes(rows, w) for w in self.packed[0].values()) and D.skinny_takes(prompts, self.packed_lm)
+        return all(D.skinny_takes(rows, w.n, w.k, w.fp8, bool(w.rope)) for w in self.packed[0].values()) and \
+            D.skinny_takes(prompts, self.packed_lm.n, self.packed_lm.k)
 
     def _prefill_fused(self, tokens, positions, slots, seqs) -> torch.Tensor:
         """A prompt step of few rows on the fused decode layer (:meth:`_fused_layers`), without its padding:
@@ -408,8 +410,8 @@ class ServingModel:
             a = torch.empty((plan.n, c.heads * c.head_dim), dtype=torch.bfloat16, device=qkv.device)
             return attention_blocks(qkv, *self._kv(qkv), plan.items, c.heads, c.kv_heads, a, merges=plan.merges, slots=plan.slots)
 
-        x, ss = self._fused_layers(tokens, positions, slots, attend, "prefill", count)
-        out = D.skinny_gemm(x[plan.last], self.packed_lm, rms=ss[plan.last], eps=c.eps, counters=count)
+        x, ss = self._fused_layers(tokens, positions, slots, attend, "prefill", count, exact=True)
+        out = D.skinny_gemm(x[plan.last], self.packed_lm, rms=ss.index_select(1, plan.last), eps=c.eps, counters=count)
         T.op("prefill-fused lm_head")
         return out
 
@@ -707,27 +709,31 @@ class ServingModel:
             return D.paged_decode_attention(qkv, self.cache.layer(i), block_tables, ctx_lens, c.heads, c.kv_heads,
                                             pages_per_split=pages_per_split)
 
-        x, ss = self._fused_layers(tokens, positions, slots, attend, "decode", None)
+        x, ss = self._fused_layers(tokens, positions, slots, attend, "decode", None, exact=False)
         out = D.skinny_gemm(x, self.packed_lm, rms=ss, eps=c.eps)
         T.op("decode-fused lm_head")
         return out
 
-    def _fused_layers(self, tokens, positions, slots, attend, kind: str, counters):
+    def _fused_layers(self, tokens, positions, slots, attend, kind: str, counters, exact: bool):
         """The residual rows after all layers and their sums of squares; ``attend(qkv, layer)`` is the
-        attention of the rotated rows, whose keys and values are in the cache."""
+        attention of the rotated rows, whose keys and values are in the cache. ``exact``: statistics whose
+        bits do not depend on the order in which workgroups arrive, so that equal steps give equal bits."""
         c = self.cfg
         eps = c.eps
         x = self.embed[tokens.long()].reshape(-1, c.hidden).contiguous()  # residual stream
-        ss_b = x.float().pow(2).sum(-1)  # statistic for layer 0's qkv
-        ss_a = torch.zeros_like(ss_b)
+        ss_b = ss = x.float().pow(2).sum(-1)  # statistic for layer 0's qkv
+        if exact:
+            ss_a, ss_b = torch.zeros((2, D.SUM_WORDS, x.shape[0]), dtype=torch.int64, device=x.device)
+        else:
+            ss_a = torch.zeros_like(ss)
         for i in range(c.layers):
             P = self.packed[i]
             if P["qkv"].rope:
-                qkv = D.skinny_gemm(x, P["qkv"], rms=ss_b, eps=eps, counters=counters,
+                qkv = D.skinny_gemm(x, P["qkv"], rms=ss, eps=eps, counters=counters,
                                     rope={"cos": self.cos, "sin": self.sin, "positions": positions, "slots": slots,
                                           "cache": self.cache.layer(i)})
             else:
-                qkv = D.skinny_gemm(x, P["qkv"], rms=ss_b, eps=eps, counters=counters)
+                qkv = D.skinny_gemm(x, P["qkv"], rms=ss, eps=eps, counters=counters)
                 self._rope_cache(qkv, i, positions, slots)
             T.op(f"{kind}-fused L{i} qkv+rope")
             a = attend(qkv, i)
@@ -735,5 +741,6 @@ class ServingModel:
             D.skinny_gemm(a, P["o"], out=x, resid_ss=ss_a, zero=ss_b, counters=counters)
             act = D.skinny_gemm(x, P["gate_up"], rms=ss_a, eps=eps, counters=counters)
             D.skinny_gemm(act, P["down"], out=x, resid_ss=ss_b, zero=ss_a, counters=counters)
+            ss = ss_b
             T.op(f"{kind}-fused L{i} o+mlp")
-        return x, ss_b
+        return x, ss

@@ -110,6 +110,12 @@ struct SkinnyCfg {
 //               atomics), the statistic the next EPI_RMS consumer needs.
 //   ss_zero     zeroed by workgroup 0 at kernel start (the sum-of-squares
 //               buffer of the previous layer boundary, already consumed).
+//   EPI_SUMS_IN, EPI_SUMS_OUT
+//               ss_in (ss_out, ss_zero) hold SUM_WORDS integers a row instead of a
+//               float: the exact sum of the workgroups' fp32 sums of squares (add_exact),
+//               so that the order in which these arrive does not show in any bit.
+//               Prompt steps use it: the same prompts give the same logits and cached
+//               keys.
 //   EPI_ROPE    W is the fused qkv weight packed so that in every q / k head
 //               16-row tile t holds dims 8t..8t+7 then 64+8t..64+8t+7
 //               (kgs/ops/decode.py rope_rows): lane l pairs with lane l ^ 32,
@@ -118,9 +124,10 @@ struct SkinnyCfg {
 //               paged cache slot slot[m] -- the rope_cache launch, folded in.
 // Together they remove both add_rmsnorm launches, the SwiGLU launch and the
 // RoPE / KV-write launch from a decode layer (kgs/serve/model.py fused path).
-enum { EPI_SWIGLU = 1, EPI_RMS = 2, EPI_RESID = 4, EPI_ROPE = 8, EPI_GELU = 16, EPI_CLAMPED = 32 };
+enum { EPI_SWIGLU = 1, EPI_RMS = 2, EPI_RESID = 4, EPI_ROPE = 8, EPI_GELU = 16, EPI_CLAMPED = 32, EPI_SUMS_IN = 64, EPI_SUMS_OUT = 128 };
 struct SkinnyEpi {
   int mode;
+  int zero_words;  // 4-byte words of ss_zero
   const float* ss_in;
   float* ss_out;
   float* ss_zero;
@@ -135,6 +142,31 @@ struct SkinnyEpi {
   unsigned short* cache;  // this layer's bf16 pages [pages][HKV][2][4096]
   int H, HKV;
 };
+
+// An exact sum of non-negative floats: a value m 2^(e - 149) (24-bit m) goes, shifted by e % 32, into
+// integer e / 32 of eight, whose addition does not round. 2^24 * 2^31 times 512 values fit 64 bits, so a row takes
+// at most 512 of them (of 16 columns and more: SUM_MAX_N). The last integer's values stay below 2^62: bit 63
+// of it says that an infinity was added, bit 62 a NaN. Integer i of row m lies at [i][m]: the rows of a
+// tile add to the same integer as a rule, and so to one run of memory.
+constexpr int SUM_WORDS = 8, SUM_MAX_N = 8192;
+__device__ __forceinline__ void add_exact(unsigned long long* acc, int rows, float v) {
+  const unsigned b = __float_as_uint(v), e = b >> 23;
+  const bool odd = e >= 255;
+  const unsigned m = e ? (b & 0x7fffff) | 0x800000 : b, sh = e ? e - 1 : 0;
+  if (odd) atomicOr(acc + (SUM_WORDS - 1) * rows, 1ull << (b == 0x7f800000u ? 63 : 62));
+  else if (m) atomicAdd(acc + (sh >> 5) * rows, (unsigned long long)m << (sh & 31));
+}
+// ... as a float: the integers rounded to 53 bits each, added from the smallest
+__device__ __forceinline__ float exact_sum(const unsigned long long* acc, int rows) {
+  unsigned long long w[SUM_WORDS];
+#pragma unroll
+  for (int i = 0; i < SUM_WORDS; ++i) w[i] = acc[i * rows];
+  const unsigned flags = (unsigned)(w[SUM_WORDS - 1] >> 62);
+  double s = 0;
+#pragma unroll
+  for (int i = 0; i < SUM_WORDS; ++i) s += __builtin_ldexp((double)w[i], 32 * i - 149);
+  return flags ? (flags & 1 ? __builtin_nanf("") : __builtin_inff()) : (float)s;
+}
 
 // W8 (weight-only fp8, "W8A16"): W is OCP e4m3 in the same fragment order, 8 B
 // per lane per fragment (512 B wave loads: half the HBM bytes), dequantised to
@@ -180,7 +212,12 @@ __device__ __forceinline__ bf16x8 dequant8(u32x2 v, float s) {
 // batch-1 launch); the waves' partial tiles are summed through LDS. x comes
 // straight from global/L2 through the W ring (no LDS staging): chunk = KC
 // k-steps per wave, k_per_chunk = 4 * 32 * KC.
-template <int R, int MT, int KC_, bool W8 = false, bool EROPE = false, bool KIN = false>
+// SUMS: the instantiations with EPI_SUMS_IN and EPI_SUMS_OUT (bf16 weights, batch <= 64), apart because
+// what they add moves the main loop's register allocation. The rows' scales are made once per workgroup, under the
+// first weights' way from memory, and a workgroup's tiles are summed in LDS before they are added (with each
+// tile's atomics and each output's conversion 1.2 us more a launch). us at 30 rows, floats / exact sums:
+// 28672x4096 43.4 / 43.6, 4096x14336 29.5 / 29.1, 4096x4096 16.9 / 16.5.
+template <int R, int MT, int KC_, bool W8 = false, bool EROPE = false, bool KIN = false, bool SUMS = false>
 __global__ __launch_bounds__(256, (MT * KC_ > 32 || R * MT >= 16) ? 1 : 2) void skinny(const void* __restrict__ wpv, const unsigned short* __restrict__ x,
                                                  unsigned short* __restrict__ y, float* __restrict__ ws,
                                                  int* __restrict__ cnt, int M, int N, int K, long ldx, long ldy,
@@ -197,11 +234,17 @@ __global__ __launch_bounds__(256, (MT * KC_ > 32 || R * MT >= 16) ? 1 : 2) void 
   // arriver" flag reuses its first word after the main loop
   static_assert(!KIN || PF == KC, "KIN: one ring round per chunk");
   __shared__ __attribute__((aligned(16))) bf16x8 xs[2][KIN ? 2 * R * MT * 64 : C::CHUNK_SLOTS];
+  __shared__ float stat[SUMS ? 5 : 1][16 * MT];  // SUMS: the rows' scales; a wave's sums of squares in [1 + wave]
 
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int nstrip = N / ((KIN ? 16 : 64) * R);
   const int strip = blockIdx.x % nstrip, split = blockIdx.x / nstrip;
-  if (ep.ss_zero != nullptr && blockIdx.x == 0 && tid < M) ep.ss_zero[tid] = 0.f;
+  if constexpr (SUMS) {
+    if (ep.ss_zero != nullptr && blockIdx.x == 0)
+      for (int i = tid; i < ep.zero_words; i += 256) ep.ss_zero[i] = 0.f;
+  } else {
+    if (ep.ss_zero != nullptr && blockIdx.x == 0 && tid < M) ep.ss_zero[tid] = 0.f;
+  }
   const int nkk = K / 32;
   // k-steps (of 32) of this wave and where they start
   const int nsteps = chunks_per_split * KC;
@@ -277,6 +320,12 @@ __global__ __launch_bounds__(256, (MT * KC_ > 32 || R * MT >= 16) ? 1 : 2) void 
 #pragma unroll
     for (int r = 0; r < R; ++r) wf[p][r] = __builtin_nontemporal_load(wrow[r] + (long)min(p, nsteps - 1) * 64);
 
+  if constexpr (SUMS) {
+    if ((ep.mode & EPI_RMS) && tid < M) {
+      const float ss = (ep.mode & EPI_SUMS_IN) ? exact_sum((const unsigned long long*)ep.ss_in + tid, M) : ep.ss_in[tid];
+      stat[0][tid] = rsqrtf(ss * ep.inv_k + ep.eps);  // read after the barriers below
+    }
+  }
   if constexpr (KIN) {
     // B fragment of k-step s: lane (column m = 16 c + (lane & 15), k = 8 (lane >> 4) ..)
     const unsigned short* xr[MT];
@@ -365,7 +414,7 @@ __global__ __launch_bounds__(256, (MT * KC_ > 32 || R * MT >= 16) ? 1 : 2) void 
   // (the SWIGLU / RESID exchanges are cross-lane)
   auto emit = [&](f32x4v v, int m, int r) {
     const int ms = m < M ? m : M - 1;
-    if (ep.mode & EPI_RMS) v *= rsqrtf(ep.ss_in[ms] * ep.inv_k + ep.eps);
+    if (ep.mode & EPI_RMS) v *= SUMS ? stat[0][ms] : rsqrtf(ep.ss_in[ms] * ep.inv_k + ep.eps);
     if (ep.mode & EPI_SWIGLU) {
       f32x4v u;
 #pragma unroll
@@ -397,7 +446,10 @@ __global__ __launch_bounds__(256, (MT * KC_ > 32 || R * MT >= 16) ? 1 : 2) void 
         sq = r0 * r0 + r1 * r1 + r2 * r2 + r3 * r3;
       }
       sq = wsum16(sq);  // lanes of one column m (g = 0..3)
-      if (m < M && g == 0) atomicAdd(ep.ss_out + m, sq);
+      if (m < M && g == 0) {
+        if (SUMS && (ep.mode & EPI_SUMS_OUT)) stat[1 + w][m] = r ? stat[1 + w][m] + sq : sq;
+        else atomicAdd(ep.ss_out + m, sq);
+      }
     } else if (EROPE) {
       const int c = m >> 4;
       const int T = nt0 + r, hh = T >> 3, t = T & 7;  // head and 16-row tile within it
@@ -445,12 +497,30 @@ __global__ __launch_bounds__(256, (MT * KC_ > 32 || R * MT >= 16) ? 1 : 2) void 
       *(uint2*)(y + (long)m * ldy + 16 * (nt0 + r) + 4 * g) = pk;
     }
   };
+  // the workgroup's sums of squares, in the order of its waves (KIN: wave 0's alone), to the rows' exact sums
+  auto add_sums = [&] {
+    if constexpr (SUMS) {
+      if (!(ep.mode & EPI_RESID) || !(ep.mode & EPI_SUMS_OUT)) return;
+      if constexpr (KIN) {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // other lanes' values, by the wave's own LDS order
+        __builtin_amdgcn_wave_barrier();
+      } else {
+        __syncthreads();
+      }
+      if (tid < M) {
+        float sq = stat[1][tid];
+        if constexpr (!KIN) sq = ((sq + stat[2][tid]) + stat[3][tid]) + stat[4][tid];
+        add_exact((unsigned long long*)ep.ss_out + tid, M, sq);
+      }
+    }
+  };
   if (ksplit == 1) {
     if (KIN && w != 0) return;
 #pragma unroll
     for (int c = 0; c < MT; ++c)
 #pragma unroll
       for (int r = 0; r < R; ++r) emit(acc[r][c], 16 * c + mc, r);
+    add_sums();
     return;
   }
   // split-K: fp32 slabs ws[split][m][n] stored write-through (sc1); every wave
@@ -506,6 +576,7 @@ __global__ __launch_bounds__(256, (MT * KC_ > 32 || R * MT >= 16) ? 1 : 2) void 
       emit(t, m, r);
     }
   }
+  add_sums();
 }
 
 // ---------------------------------------------------------------------------
@@ -1407,18 +1478,23 @@ int default_variant(int mt) { return mt == 1 ? 1 : mt == 2 ? 4 : mt == 4 ? 8 : m
 template <int R, int MT, int KC, bool W8, bool KIN = false>
 hipError_t launch_skinny(const void* wp, const void* x, void* y, float* ws, int* cnt, int M, int N, int K, long ldx,
                          long ldy, int ksplit, int cps, const kgs::dec::SkinnyEpi& ep, hipStream_t s) {
-  const int nstrip = N / ((KIN ? 16 : 64) * R);
+  using namespace kgs::dec;
+  const dim3 grid(N / ((KIN ? 16 : 64) * R) * ksplit);
+  auto run = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, wp, (const unsigned short*)x, (unsigned short*)y, ws, cnt, M, N, K, ldx, ldy,
+                       ksplit, cps, ep);
+    return hipGetLastError();
+  };
+  const bool rope = ep.mode & EPI_ROPE, sums = ep.mode & (EPI_SUMS_IN | EPI_SUMS_OUT);
   if constexpr (!W8 && MT <= 4 && R == 1) {  // the fused layer's qkv variants (kgs/ops/decode.py rope_variant)
-    if (ep.mode & kgs::dec::EPI_ROPE) {
-      hipLaunchKernelGGL((kgs::dec::skinny<R, MT, KC, false, true, KIN>), dim3(nstrip * ksplit), dim3(256), 0, s, wp,
-                         (const unsigned short*)x, (unsigned short*)y, ws, cnt, M, N, K, ldx, ldy, ksplit, cps, ep);
-      return hipGetLastError();
-    }
+    if (rope) return sums ? run(skinny<R, MT, KC, false, true, KIN, true>) : run(skinny<R, MT, KC, false, true, KIN>);
   }
-  if (ep.mode & kgs::dec::EPI_ROPE) return hipErrorInvalidValue;  // no RoPE instantiation for this variant
-  hipLaunchKernelGGL((kgs::dec::skinny<R, MT, KC, W8, false, KIN>), dim3(nstrip * ksplit), dim3(256), 0, s, wp,
-                     (const unsigned short*)x, (unsigned short*)y, ws, cnt, M, N, K, ldx, ldy, ksplit, cps, ep);
-  return hipGetLastError();
+  if (rope) return hipErrorInvalidValue;  // no RoPE instantiation for this variant
+  if constexpr (!W8 && MT <= 4) {
+    if (sums) return run(skinny<R, MT, KC, false, false, KIN, true>);
+  }
+  if (sums) return hipErrorInvalidValue;
+  return run(skinny<R, MT, KC, W8, false, KIN>);
 }
 }  // namespace
 
@@ -1447,7 +1523,8 @@ KGS_EXPORT int kgs_skinny_geometry(int M, int* rows_per_strip, int* k_per_chunk,
 // with ksplit > 1, ws holds ksplit * mpad * N floats and cnt N / rows_per_strip
 // zero-initialised ints (left zeroed on return). epi: EPI_* flags (SWIGLU: y is
 // [M, N/2]; RMS needs ss_in[M]; RESID accumulates into y and ss_out[M]);
-// ss_zero (optional, [M] floats) is cleared at kernel start.
+// ss_zero (optional, [M] floats) is cleared at kernel start. With EPI_SUMS_IN ss_in, with EPI_SUMS_OUT
+// ss_out and ss_zero hold 64-bit integers [8][M] (16-B aligned), N at most 8192 for ss_out.
 namespace {
 int skinny_fused(const void* wp, const void* x, void* y, float* ws, int* cnt, int M, int N, int K, long ldx, long ldy,
                  int ksplit, int variant, int epi, const float* ss_in, float* ss_out, float* ss_zero, float inv_k,
@@ -1476,7 +1553,7 @@ KGS_EXPORT int kgs_skinny_gemm_bf16_rope(const void* wp, const void* x, void* y,
                                         const float* sinv, const int* pos, const int* slot, void* cache, int H,
                                         int HKV, hipStream_t s) {
   using namespace kgs::dec;
-  if (epi & ~EPI_RMS) return KGS_ERR_ARG;
+  if (epi & ~(EPI_RMS | EPI_SUMS_IN)) return KGS_ERR_ARG;
   if (H <= 0 || HKV <= 0 || H % HKV || N != (H + 2 * HKV) * HD) return KGS_ERR_SHAPE;
   if (!cosv || !sinv || !pos || !slot || !al16(cache)) return KGS_ERR_ARG;
   SkinnyEpi r{};
@@ -1500,7 +1577,7 @@ int skinny_fused(const void* wp, const void* x, void* y, float* ws, int* cnt, in
   const int rc = kgs_skinny_variant_geometry(variant, M, &rps, &kpc, &mpad);
   if (rc) return rc;
   if (variant == 0) variant = default_variant(mt_for(M));
-  if (epi & ~(EPI_SWIGLU | EPI_RMS | EPI_RESID | EPI_ROPE | EPI_GELU | EPI_CLAMPED) ||
+  if (epi & ~(EPI_SWIGLU | EPI_RMS | EPI_RESID | EPI_ROPE | EPI_GELU | EPI_CLAMPED | EPI_SUMS_IN | EPI_SUMS_OUT) ||
       ((epi & (EPI_GELU | EPI_CLAMPED)) && !(epi & EPI_SWIGLU)) || ((epi & EPI_SWIGLU) && (epi & EPI_RESID)))
     return KGS_ERR_ARG;
   if ((epi & EPI_ROPE) && (rope.cache == nullptr || (epi & (EPI_SWIGLU | EPI_RESID)) || wscale != nullptr))
@@ -1508,6 +1585,8 @@ int skinny_fused(const void* wp, const void* x, void* y, float* ws, int* cnt, in
   if (((epi & EPI_RMS) && ss_in == nullptr) || ((epi & EPI_RESID) && ss_out == nullptr)) return KGS_ERR_ARG;
   if (N <= 0 || K <= 0 || N % rps || K % kpc || ldx < K || ldy < ((epi & EPI_SWIGLU) ? N / 2 : N))
     return KGS_ERR_SHAPE;
+  if ((epi & EPI_RESID) && (epi & EPI_SUMS_OUT) && N > SUM_MAX_N) return KGS_ERR_SHAPE;
+  if (((epi & EPI_SUMS_IN) && !al16(ss_in)) || ((epi & EPI_SUMS_OUT) && (!al16(ss_out) || !al16(ss_zero)))) return KGS_ERR_ALIGN;
   const int nchunks = K / kpc;
   if (ksplit <= 0 || nchunks % ksplit) return KGS_ERR_ARG;
   if (ksplit > 1 && (ws == nullptr || cnt == nullptr)) return KGS_ERR_ARG;
@@ -1518,6 +1597,7 @@ int skinny_fused(const void* wp, const void* x, void* y, float* ws, int* cnt, in
   ep.ss_in = ss_in;
   ep.ss_out = ss_out;
   ep.ss_zero = ss_zero;
+  ep.zero_words = (epi & EPI_SUMS_OUT) ? 2 * SUM_WORDS * M : M;
   ep.inv_k = inv_k;
   ep.eps = eps;
   ep.wscale = wscale;

@@ -6,6 +6,7 @@ import numpy as np
 import pytest
 import torch
 
+from kgs.models.llama import LlamaConfig
 from kgs.ops import decode as D
 from kgs.ops import transformer as T
 
@@ -203,19 +204,8 @@ def test_gather_kv_bits(fp8, kv, ctx, rows):
         D.gather_kv_into(cache, pages[:0], 1, k, v)
 
 
-@pytest.mark.gpu
-@pytest.mark.parametrize("lens,ff,fused", [([20, 5], 2048, 48), ([48], 2048, 48), ([49], 2048, 48), ([130, 126], 2048, 48), ([100, 157], 2048, 48),
-                                           ([300, 260], 2048, 48), ([20, 5], 2304, 48),  # 2304: no skinny tile of down
-                                           ([64], 2048, 128), ([65], 2048, 128), ([257], 2048, 300)])
-def test_prefill_by_rows(lens, ff, fused):
-    """Either side of the row counts where a prompt step changes its layers: logits and cache of the step
-    against float32 layers on the same weights. Sums round to bf16 at other places on either side: a
-    few 2^-8 in the 2-norm over two layers."""
-    from kgs.models.llama import LlamaConfig
-    from kgs.serve.model import ServingModel
-
-    cfg = LlamaConfig(hidden=2048, intermediate=ff, heads=16, kv_heads=4, layers=2, vocab=1024)
-    ours, ref = (ServingModel(cfg, device=DEV, backend=b, num_pages=40, max_model_len=1024, fused_max_batch=fused) for b in ("kgs", "ref"))
+def _prompts(lens):
+    """Arguments of a prompt step: prompts padded to 128, each on pages of its own."""
     padded = [-(-n // 128) * 128 for n in lens]
     total, rng = sum(padded), np.random.default_rng(len(lens))
     tok, pos, slot, at, page, starts = np.zeros(total, np.int32), np.zeros(total, np.int32), np.full(total, -1, np.int32), 0, 1, []
@@ -223,10 +213,52 @@ def test_prefill_by_rows(lens, ff, fused):
         starts.append(at)
         tok[at:at + n], pos[at:at + n], slot[at:at + n] = rng.integers(0, 1024, n), np.arange(n), 32 * page + np.arange(n)
         at, page = at + p, page + -(-n // 32)
-    args = [torch.from_numpy(a).to(DEV) for a in (tok, pos, slot)]
-    got, want = (m.prefill(*args, starts, lens, padded).float() for m in (ours, ref))
+    return (*(torch.from_numpy(a).to(DEV) for a in (tok, pos, slot)), starts, lens, padded)
+
+
+@pytest.fixture
+def normed(monkeypatch):
+    """Models whose norm weights are not one, so that a missing or doubled one shows."""
+    from kgs.serve import model as M
+
+    class Normed(M.LlamaModel):
+        def __init__(self, cfg, **kw):
+            super().__init__(cfg, **kw)
+            g = torch.Generator(device=DEV).manual_seed(7)
+            for t in (*(w[n] for w in self.layers for n in ("ln1", "ln2")), self.norm):
+                t.copy_(torch.exp2(torch.rand(t.shape, generator=g, device=DEV) * 4 - 2))
+
+    monkeypatch.setattr(M, "LlamaModel", Normed)
+    return M.ServingModel
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("lens,ff,fused", [([20, 5], 2048, 48), ([48], 2048, 48), ([49], 2048, 48), ([130, 126], 2048, 48), ([100, 157], 2048, 48),
+                                           ([300, 260], 2048, 48), ([20, 5], 2304, 48),  # 2304: no skinny tile of down
+                                           ([64], 2048, 128), ([65], 2048, 128), ([257], 2048, 300)])
+def test_prefill_by_rows(lens, ff, fused, normed):
+    """Either side of the row counts where a prompt step changes its layers: logits and cache of the step
+    against float32 layers on the same weights. Sums round to bf16 at other places on either side: a
+    few 2^-8 in the 2-norm over two layers."""
+    cfg = LlamaConfig(hidden=2048, intermediate=ff, heads=16, kv_heads=4, layers=2, vocab=1024)
+    ours, ref = (normed(cfg, device=DEV, backend=b, num_pages=40, max_model_len=1024, fused_max_batch=fused) for b in ("kgs", "ref"))
+    args = _prompts(lens)
+    got, want = (m.prefill(*args).float() for m in (ours, ref))
     assert got.shape == want.shape == (len(lens), 1024)
     assert float((got - want).norm() / want.norm()) < 0.03
     a, b = ours.cache.data.float(), ref.cache.data.float()
     assert float((a - b).norm() / b.norm()) < 0.02
     assert torch.equal(a == 0, b == 0)  # the same slots written
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("lens,kv", [([1], "bf16"), ([20, 5], "bf16"), ([48], "bf16"), ([33], "fp8"), ([64], "bf16"), ([90], "bf16")])
+def test_a_prompt_step_repeats_its_bits(lens, kv, normed):
+    """The same prompts give the same logits and cached keys every time, whatever order workgroups arrive in."""
+    cfg = LlamaConfig(hidden=2048, intermediate=8192, heads=16, kv_heads=4, layers=4, vocab=1024)
+    model, args, first = normed(cfg, device=DEV, num_pages=8, max_model_len=256, fused_max_batch=64, kv_cache_dtype=kv), _prompts(lens), None
+    for _ in range(40):
+        model.cache.data.zero_()
+        got = model.prefill(*args).clone(), model.cache.data.view(torch.uint8).clone()
+        first = first or got
+        assert all(torch.equal(a, b) for a, b in zip(got, first))

@@ -2,6 +2,8 @@
 workgroup for up to 64 rows."""
 from __future__ import annotations
 
+from fractions import Fraction
+
 import pytest
 import torch
 
@@ -30,18 +32,18 @@ class _Weight:
 def test_what_the_skinny_gemm_takes():
     """Its own choice of a variant has to tile the weight, and the rotation's to have one-tile waves."""
     for m in range(1, 258):
-        for w in (_Weight(3072, 2048), _Weight(3072, 2048, rope=(16, 4)), _Weight(3072, 2048, fp8=True), _Weight(3136, 2048), _Weight(2048, 2304)):
-            most = 64 if w.rope or w.fp8 else 256
-            ok = D.skinny_takes(m, w)
-            if m > most:
+        for n, k, fp8, rope in ((3072, 2048, False, False), (3072, 2048, False, True), (3072, 2048, True, False), (3136, 2048, False, False),
+                                (2048, 2304, False, False)):
+            ok = D.skinny_takes(m, n, k, fp8, rope)
+            if m > (64 if rope or fp8 else 256):
                 assert not ok
                 continue
-            v, ks = D._skinny_plan(m, w, bool(w.rope))
+            v, ks = D._skinny_plan(m, n, k, fp8, rope)
             rps, kpc, _ = D.skinny_geometry(m, v)
-            assert ok == (w.n % rps == 0 and w.k % kpc == 0) and (not ok or (w.k // kpc) % ks == 0)
-            assert not w.rope or D.SKINNY_VARIANTS[v][0] == 1
-    assert D.skinny_takes(64, _Weight(3072, 2048, rope=(16, 4))) and D.skinny_takes(200, _Weight(3072, 2048))
-    assert not D.skinny_takes(200, _Weight(3136, 2048)) and not D.skinny_takes(1, _Weight(2048, 2304))
+            assert ok == (n % rps == 0 and k % kpc == 0) and (not ok or (k // kpc) % ks == 0)
+            assert not rope or D.SKINNY_VARIANTS[v][0] == 1
+    assert D.skinny_takes(64, 3072, 2048, rope=True) and D.skinny_takes(200, 3072, 2048)
+    assert not D.skinny_takes(200, 3136, 2048) and not D.skinny_takes(1, 2048, 2304)
 
 
 @pytest.mark.parametrize("most,rows,fused", [(48, 48, True), (48, 49, False), (128, 64, True), (128, 65, False), (300, 257, False), (0, 1, False)])
@@ -99,3 +101,45 @@ def test_k_split_in_the_workgroup(m, v):
     q2 = D.skinny_gemm(x, D.PackedWeight(wq, fold=one, rope=(heads, kv)), rms=ss, variant=v, ksplit=1,
                        rope={"cos": cos, "sin": sin, "positions": pos, "slots": slot, "cache": cb})
     assert torch.equal(q1, q2) and torch.equal(ca, cb)
+
+
+def _exact(words) -> float:
+    """An exact sum's value from its eight integers (decode.hip add_exact), rounded once."""
+    w = [int(x) & (2 ** 64 - 1) for x in words]
+    if w[-1] >> 62:
+        return float("nan") if w[-1] >> 62 & 1 else float("inf")
+    return float(Fraction(sum(x << 32 * i for i, x in enumerate(w)), 2 ** 149))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [1024, 8192])
+@pytest.mark.parametrize("m,variant,ksplit", [(8, 1, 1), (8, 1, 4), (8, 20, 1), (24, 22, 1), (24, 5, 2), (48, 24, 1), (64, 10, 4), (64, 25, 1), (64, 12, 1)])
+def test_exact_sums_of_squares(m, variant, ksplit, n):
+    """Statistics kept as exact sums: equal integers from every launch, the float64 sum of the stored values but for
+    the tiles' fp32 rounding (16 values each: under 2^-20), and, read back, the bits of the same value as a float."""
+    torch.manual_seed(m)
+    k = 4096
+    w, up = (D.PackedWeight(torch.randn(*s, device=DEV).bfloat16()) for s in ((n, k), (512, n)))
+    x = torch.randn(m, k, device=DEV).bfloat16()
+    y = torch.randn(m, n, device=DEV).bfloat16()
+    x[:5] = 0  # these rows' residual stays what it is
+    y[0], y[1], y[2, ::3], y[3, 7], y[4, 9] = 0, 1e-20, 1e15, 1e20, float("nan")
+    got = []
+    for _ in range(4):
+        sums, old, out = *torch.zeros(2, D.SUM_WORDS, m, dtype=torch.int64, device=DEV), y.clone()
+        old.fill_(7)
+        D.skinny_gemm(x, w, out=out, resid_ss=sums, zero=old, variant=variant, ksplit=ksplit)
+        assert not old.any()
+        got.append(sums)
+    assert all(torch.equal(got[0], g) for g in got)
+    value = [_exact(r) for r in got[0].T.tolist()]
+    want = out.double().pow(2).sum(-1).tolist()
+    assert value[0] == 0 and value[3] == float("inf") and value[4] != value[4]
+    for i in (1, 2, *range(5, m)):
+        assert abs(value[i] - want[i]) <= 2.0 ** -20 * want[i], i
+    a, b = (D.skinny_gemm(out, up, rms=r) for r in (got[0], torch.tensor(value, dtype=torch.float32, device=DEV)))
+    assert torch.equal(a.view(torch.int16), b.view(torch.int16))
+    with pytest.raises(ValueError):
+        D.skinny_gemm(x, w, out=out, resid_ss=got[0], zero=torch.zeros(m, device=DEV))
+    with pytest.raises(ValueError):
+        D.skinny_gemm(out, up, rms=got[0][:, :m - 1].contiguous())

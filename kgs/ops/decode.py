@@ -696,6 +696,24 @@ def workgroup_splits(batch: int, kv_heads: int, max_pages: int, cus: int = CUS) 
     return min(-(-2 * cus // groups), max(1, max_pages // (8 if 2 * groups < cus else 32)))
 
 
+def workgroup_waves(groups: int, max_pages: int, fp8: bool) -> int:
+    """Waves of such a workgroup for ``groups`` (sequence, KV head) pairs, 1 for the kernel of single waves.
+
+    Eight (e4m3 pages four), except where a table so narrow that a wave has a page or two meets so many
+    pairs that a workgroup's fixed cost counts: from 1024 on. us by single waves / as many waves as elsewhere /
+    by this rule, 8 KV heads, contexts as long as the table and uniform up to there: bf16, 256 sequences of 2 pages
+    11.7 / 17.3 / 11.7 and 9.5 / 16.1 / 9.5, of 4 22.0 / 24.5 / 21.6 and 16.7 / 19.0 / 14.7 (in two waves), 1024 of 8
+    170 / 171 / 173 and 110 / 104 / 102 (in four; most of them a few tokens: 43 / 61 / 39); e4m3, 256 of 8 23.3 /
+    26.9 / 23.3 and 17.9 / 21.1 / 17.9, of 16 44.6 / 43.8 / 45.3 and 30.6 / 31.3 / 27.5 (in two), 1024 of 2 26 / 55 / 26
+    and 22 / 52 / 22. At 32 pages the waves of one group even out unequal contexts for more than they cost:
+    bf16, 256 sequences 156 / 163 and 113 / 90, e4m3 84.8 / 81.1 and 58.5 / 50.6."""
+    if groups < 1024:
+        return 4 if fp8 else 8
+    if fp8:
+        return 1 if groups >= 2048 and max_pages <= 8 else 2 if max_pages <= 16 else 4
+    return 1 if groups >= 2048 and max_pages <= 2 else 2 if max_pages <= 4 else 4 if max_pages <= 8 else 8
+
+
 _AWS: dict = {}
 
 
@@ -784,8 +802,9 @@ def paged_decode_attention(q: torch.Tensor, cache_layer: torch.Tensor, block_tab
     if ctx_lens.dtype != torch.int32 or not ctx_lens.is_contiguous() or ctx_lens.numel() != b:
         raise ValueError("ctx_lens must be contiguous int32 [B]")
     max_pages = block_tables.shape[1]
-    by_workgroup = pages_per_split is None and pipe is None
-    if by_workgroup:
+    fp8 = cache_layer.dtype == FP8
+    waves = workgroup_waves(b * kv_heads, max_pages, fp8) if pages_per_split is None and pipe is None else 1
+    if waves > 1:
         nsplit = workgroup_splits(b, kv_heads, max_pages) if b else 1
     elif pages_per_split is None:
         pps, nsplit = decode_splits(b, kv_heads, max_pages)
@@ -795,13 +814,13 @@ def paged_decode_attention(q: torch.Tensor, cache_layer: torch.Tensor, block_tab
         out = torch.empty((b, heads * HEAD_DIM), dtype=torch.bfloat16, device=q.device)
     po, pml, cnt = _attn_workspace(b, heads, kv_heads, nsplit, q.device)
     scale = 1.0 / math.sqrt(HEAD_DIM) if scale is None else scale
-    if by_workgroup:
-        rc = _lib.lib().kgs_paged_decode_wg(q.data_ptr(), cache_layer.data_ptr(), block_tables.data_ptr(), ctx_lens.data_ptr(),
-                                            out.data_ptr(), po.data_ptr() if po is not None else None,
-                                            pml.data_ptr() if pml is not None else None,
-                                            cnt.data_ptr() if cnt is not None else None, b, heads, kv_heads, HEAD_DIM,
-                                            max_pages, nsplit, q.stride(0), out.stride(0), float(scale),
-                                            1 if cache_layer.dtype == FP8 else 0, _lib.stream_handle(q.device))
+    if waves > 1:
+        rc = _lib.lib().kgs_paged_decode_wg_ex(q.data_ptr(), cache_layer.data_ptr(), block_tables.data_ptr(), ctx_lens.data_ptr(),
+                                               out.data_ptr(), po.data_ptr() if po is not None else None,
+                                               pml.data_ptr() if pml is not None else None,
+                                               cnt.data_ptr() if cnt is not None else None, b, heads, kv_heads, HEAD_DIM,
+                                               max_pages, nsplit, q.stride(0), out.stride(0), float(scale),
+                                                  int(fp8), waves, _lib.stream_handle(q.device))
         _lib.check(rc, "paged_decode_attention")
         return out
     rc = _lib.lib().kgs_paged_decode_bf16_ex(q.data_ptr(), cache_layer.data_ptr(), block_tables.data_ptr(),

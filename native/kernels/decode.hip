@@ -1204,7 +1204,8 @@ __global__ __launch_bounds__(64) void paged_decode(AttnArgs a) {
 // A wave's page ids lie in its lanes (64 at a time, one load), so that no page waits for its id.
 // bf16 pages: eight waves, four on a SIMD hide each other's loads. e4m3 pages (PIPE): four waves
 // that keep the next page on its way in registers while they widen and multiply one (64 sequences
-// around 700 tokens, 8 KV heads: 22 us, 31 without).
+// around 700 tokens, 8 KV heads: 22 us, 31 without). Fewer waves where the table holds few pages
+// (kgs/ops/decode.py workgroup_waves).
 template <bool KV8>
 struct PageRegs;  // a page's K and V as loaded: fragment order, e4m3 pages 8 bytes a lane
 template <>
@@ -1774,11 +1775,12 @@ KGS_EXPORT int kgs_paged_decode_bf16_ex(const void* q, const void* cache, const 
   return (int)hipGetLastError();
 }
 
-// Paged decode attention by workgroups, nsplit equal parts of every sequence's pages (paged_wg). Arguments as kgs_paged_decode_bf16; nsplit > 1 needs po, pml and
-// cnt, and merges in the same launch.
-KGS_EXPORT int kgs_paged_decode_wg(const void* q, const void* cache, const int* block_tables, const int* ctx_lens, void* o,
-                                   float* po, float* pml, int* cnt, int B, int H, int HKV, int hd, int max_pages,
-                                   int nsplit, long ldq, long ldo, float scale, int kv8, hipStream_t s) {
+// Paged decode attention by workgroups of `waves` waves (bf16 pages 2, 4 or 8, e4m3 pages 2 or 4), nsplit equal parts
+// of every sequence's pages (paged_wg). Arguments as kgs_paged_decode_bf16; nsplit > 1 needs po, pml and cnt, and
+// merges in the same launch.
+KGS_EXPORT int kgs_paged_decode_wg_ex(const void* q, const void* cache, const int* block_tables, const int* ctx_lens, void* o,
+                                      float* po, float* pml, int* cnt, int B, int H, int HKV, int hd, int max_pages,
+                                      int nsplit, long ldq, long ldo, float scale, int kv8, int waves, hipStream_t s) {
   using namespace kgs::dec;
   if (B <= 0 || H <= 0 || HKV <= 0 || H % HKV || H / HKV > 16 || hd != HD || max_pages <= 0 || nsplit <= 0) return KGS_ERR_SHAPE;
   if (ldq < (long)H * HD || ldo < (long)H * HD) return KGS_ERR_SHAPE;
@@ -1789,9 +1791,18 @@ KGS_EXPORT int kgs_paged_decode_wg(const void* q, const void* cache, const int* 
   AttnArgs a{(const unsigned short*)q, (const unsigned short*)cache, block_tables, ctx_lens, (unsigned short*)o, po,
              pml, cnt, ldq, ldo, B, H, HKV, max_pages, 0, nsplit, 1, scale * 1.4426950408889634f,
              nullptr, 0, nullptr, nullptr, nullptr, nullptr, nullptr};
-  if (kv8) hipLaunchKernelGGL(paged_wg<true>, dim3((unsigned)nwg), dim3(256), 0, s, a);
-  else hipLaunchKernelGGL(paged_wg<false>, dim3((unsigned)nwg), dim3(512), 0, s, a);
+  auto fn = kv8 ? (waves == 4 ? paged_wg<true> : waves == 2 ? paged_wg<true, 2> : nullptr)
+                : (waves == 8 ? paged_wg<false> : waves == 4 ? paged_wg<false, 4> : waves == 2 ? paged_wg<false, 2> : nullptr);
+  if (!fn) return KGS_ERR_ARG;
+  hipLaunchKernelGGL(fn, dim3((unsigned)nwg), dim3(64 * waves), 0, s, a);
   return (int)hipGetLastError();
+}
+
+KGS_EXPORT int kgs_paged_decode_wg(const void* q, const void* cache, const int* block_tables, const int* ctx_lens, void* o,
+                                   float* po, float* pml, int* cnt, int B, int H, int HKV, int hd, int max_pages,
+                                   int nsplit, long ldq, long ldo, float scale, int kv8, hipStream_t s) {
+  return kgs_paged_decode_wg_ex(q, cache, block_tables, ctx_lens, o, po, pml, cnt, B, H, HKV, hd, max_pages, nsplit, ldq, ldo,
+                                scale, kv8, kv8 ? 4 : 8, s);
 }
 
 // Rows 0 .. rows - 1 of a sequence's cached keys and values, row-major with rows ld apart (16-B

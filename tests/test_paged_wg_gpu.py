@@ -83,3 +83,58 @@ def test_split_rule_stays_in_its_bounds(batch, kv, pages):
 
     n = workgroup_splits(batch, kv, pages)
     assert 1 <= n <= max(1, pages // 8) and (n == 1 or (n - 1) * batch * kv < 512)
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("groups,pages", [(1023, 1), (1024, 2), (1024, 5), (2047, 2), (2048, 2), (2048, 3), (2048, 8), (2048, 9), (8192, 16), (8192, 17),
+                                          (1, 4096), (8192, 4096)])
+def test_wave_rule(fp8, groups, pages):
+    """Narrow tables of many pairs by few waves, everything else by as many as elsewhere."""
+    from kgs.ops.decode import workgroup_waves
+
+    w, most = workgroup_waves(groups, pages, fp8), 4 if fp8 else 8
+    assert w in ((1, 2, 4) if fp8 else (1, 2, 4, 8))
+    assert w == most or (groups >= 1024 and pages <= (16 if fp8 else 8))
+    assert w == 1 or w >= min(2, most) and (w > 1 or groups >= 2048)
+    assert w <= workgroup_waves(groups, pages + 1, fp8) and w >= workgroup_waves(groups + 1, pages, fp8)
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("pages", [1, 2, 3, 4, 5, 8, 9, 16])
+@pytest.mark.parametrize("batch", [127, 128, 256])
+def test_few_waves_on_narrow_tables(batch, pages, fp8):
+    """Either side of each border of the rule, contexts of every length that the table holds."""
+    from kgs.ops import decode as D
+
+    g = torch.Generator(device=DEV).manual_seed(pages)
+    ctx = torch.randint(1, 32 * pages + 1, (batch,), generator=g, device=DEV, dtype=torch.int32)
+    ctx[0], ctx[1], ctx[2] = 32 * pages, 1, 0
+    cache = torch.randn(50, 8, 2, 4096, device=DEV, generator=g).to(D.FP8 if fp8 else torch.bfloat16)
+    tables = torch.randint(0, 50, (batch, pages), generator=g, device=DEV, dtype=torch.int32)
+    q = (2 * torch.randn(batch, 16 * 128, device=DEV, generator=g)).bfloat16()
+    got = D.paged_decode_attention(q, cache, tables, ctx, 16, 8)
+    some = [0, 1, 2, *range(3, batch, 17), batch - 1]
+    want = D.ref_paged_decode(q[some], cache, tables[some].contiguous(), ctx[some].clamp(min=1), 16, 8)
+    want[2] = 0
+    assert float((got[some].float() - want).abs().max()) < TOL
+
+
+@pytest.mark.parametrize("fp8,waves", [(False, 2), (False, 4), (True, 2)])
+@pytest.mark.parametrize("nsplit", [1, 3])
+def test_few_waves_in_parts(fp8, waves, nsplit):
+    from kgs.ops import _lib
+    from kgs.ops import decode as D
+
+    lens, hkv = [1, 33, 64, 65, 129, 900, 2200], 4
+    q, cache, tables, ctx = setup(lens, hkv, 4, fp8)
+    out = torch.full((len(lens), 16 * 128), 7.0, dtype=torch.bfloat16, device=DEV)
+    ws = D._attn_workspace(len(lens), 16, hkv, nsplit, q.device)
+
+    def go(w):
+        return _lib.lib().kgs_paged_decode_wg_ex(q.data_ptr(), cache.data_ptr(), tables.data_ptr(), ctx.data_ptr(), out.data_ptr(),
+                                                 *(None if t is None else t.data_ptr() for t in ws), len(lens), 16, hkv, 128, tables.shape[1],
+                                                 nsplit, q.stride(0), out.stride(0), 128 ** -0.5, int(fp8), w, _lib.stream_handle(q.device))
+
+    assert go(waves) == 0
+    assert float((out.float() - D.ref_paged_decode(q, cache, tables, ctx, 16, hkv)).abs().max()) < TOL
+    assert go(3) != 0 and go(8 if fp8 else 1) != 0  # no such kernels

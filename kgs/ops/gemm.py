@@ -310,7 +310,10 @@ def gemm_nt_add_(a: torch.Tensor, b: torch.Tensor, c: torch.Tensor) -> torch.Ten
 def add_product_(a: torch.Tensor, b: torch.Tensor, c: torch.Tensor) -> bool:
     """:func:`gemm_nt_add_` on any rows (``N`` and ``K`` multiples of 8, 16-B rows). Returns whether it
     took the operands; where not, nothing was written."""
-    if addc_ok(a, b, c):
+    # 256x256 tiles alone only where they are more than half the CUs, as in gemm_nt: us by these / by the tiles and
+    # slices below, 512 rows of 4096x4096 71 / 41, 2048 of 2048x8192 129 / 74, of 4096x14336 (128 tiles) 243 / 189;
+    # 2304 of it (144) 246 / 245
+    if a.dim() == 2 and a.shape[0] // 256 * (b.shape[0] // 256) > 128 and addc_ok(a, b, c):
         gemm_nt_add_(a, b, c)
         return True
     if os.environ.get("KGS_PREFILL_ADDC", "1") != "1" or any(

@@ -163,7 +163,8 @@ def test_linear_keeps_nan_and_skips_what_needs_no_gradient():
     assert x.grad is None and lin.weight.grad is not None
 
 
-@pytest.mark.parametrize("M,N,K", [(1, 256, 128), (130, 512, 384), (257, 1024, 512), (4500, 4096, 384), (8320, 2304, 512)])
+@pytest.mark.parametrize("M,N,K", [(1, 256, 128), (130, 512, 384), (257, 1024, 512), (4500, 4096, 384), (8320, 2304, 512),
+                                   (512, 512, 2048), (2048, 4096, 512), (2304, 4096, 256)])
 def test_products_of_any_rows_add_and_gate_like_their_parts(M, N, K):
     """The residual add and the gated product in the epilogue, on ragged rows of small and of
     persistent grids, against the product and a separate pass."""

@@ -1,5 +1,6 @@
-"""What gemm_bf16 refuses before anything is launched, in each of the four layouts (no GPU: tensors that
-only claim to be on one, and a kernel library that must not be reached)."""
+"""What gemm_bf16 refuses before anything is launched, in each of the four layouts, and which kernel a
+residual product asks for (no GPU: tensors that only claim to be on one, and a kernel library that
+must not be reached, or that only says what was called)."""
 import pytest
 import torch
 
@@ -71,3 +72,24 @@ def test_a_good_out_goes_on(ta, tb):
     a, b = operands(ta, tb)
     with pytest.raises(Reached):
         G.gemm_bf16(a, b, trans_a=ta, trans_b=tb, out=claimed(M, N))
+
+
+@pytest.mark.parametrize("m,n,entry", [(512, 4096, "kgs_gemm_bf16_nt_add"), (2048, 4096, "kgs_gemm_bf16_nt_add"), (2304, 4096, "kgs_gemm_bf16_nt_addc"),
+                                       (4000, 4096, "kgs_gemm_bf16_nt_add"), (8192, 4096, "kgs_gemm_bf16_nt_addc")])
+def test_residual_products_of_few_tiles_do_not_take_the_largest_ones(m, n, entry, monkeypatch):
+    """256x256 tiles on fewer than half the CUs take up to three times as long as smaller tiles and slices."""
+    called = []
+
+    class Library:
+        def __getattr__(self, name):
+            def call(*args):
+                called.append(name)
+                return int(name == "kgs_gemm_bf16_nt_w4_ok" and args[3] % 256 == 0)
+
+            return call
+
+    monkeypatch.setattr(_lib, "lib", Library)
+    monkeypatch.setattr(_lib, "stream_handle", lambda device=None: 0)
+    monkeypatch.delenv("KGS_PREFILL_ADDC", raising=False)
+    assert G.add_product_(claimed(m, 128), claimed(n, 128), claimed(m, n))
+    assert called[-1] == entry and not ("nt_addc" in entry) ^ ("kgs_gemm_bf16_nt_addc" in called)

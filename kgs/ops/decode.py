@@ -373,23 +373,42 @@ def skinny_rule(m: int, n: int, k: int, one: bool = False) -> tuple[int, int]:
 
     The K split inside the workgroup (16 rows of W each, no slabs in memory and no ticket, 2 to 3 us
     of a launch) where its strips are a workgroup per CU or so: up to 6144 rows, two tiles a wave
-    above 4096 from 17 rows of x on. Every workgroup reads all of x, so up to 32 rows of x only K of at
-    most 4096 (8192 in two halves up to 16), beyond those x of 160k values. us at 24 rows, before /
+    above 4096 from 17 rows of x on. Every workgroup reads all of x, which bounds K by the rows: up to 16 rows K of
+    8192 (in two halves where that is no second round of workgroups; else, from 64k values of x on, only where slabs
+    would not fill three quarters of the CUs), of 32k values where the strips are more than the CUs; up to 32 rows K of
+    4096 (96k values on less than half of the CUs and in two tiles a wave); beyond them 160k values; from 17 rows on
+    K of 2048 where two tiles a wave leave more than a quarter of the CUs idle. us at 24 rows, before /
     so: 3072x2048 10.3 / 6.9, 2048x2048 9.4 / 6.7, 6144x2048 12.4 / 9.9, 4096x4096 14.3 / 11.5; at 1 row 7.6 /
-    5.0, 6.9 / 4.7, 9.7 / 6.9; at 64 rows 2048x2048 13.7 / 11.7, but 4096x4096 18.2 / 20.8.
+    5.0, 6.9 / 4.7, 9.7 / 6.9; at 64 rows 2048x2048 13.7 / 11.7, but 4096x4096 18.2 / 20.8; at 16 rows 5120x3072
+    10.9 / 13.2 and 3072x8192 14.6 / 16.0 (18.3 in halves), at 32 5120x3072 13.2 / 14.5 and 1024x4096 11.6 / 12.5.
     Else x chunks of 8 k-steps instead of 16 from 17 rows on (16384x2048 at 40 rows 22.8 / 18.5,
-    32000x2048 42 / 31)."""
+    32000x2048 42 / 31), but not up to 32 rows where a grid short of the CUs has 2048 and more of K in a workgroup
+    (5120x10240 at 24 rows 30.2 / 32.2, 9216x3072 17.8 / 18.6), and not in more slices than with 16 where those are
+    shorter than 512 (1024x4096 at 48 rows 15.5 / 18.0 in 16 slices; 3584x3584 at 24 in one 18.9, in two 15.1)."""
     mt = _mt(m)
     strips = n // 16
     if mt <= 4 and k % 1024 == 0 and n % 32 == 0 and strips <= 384:
-        wide = mt > 1 and strips > 256 and not one
+        over = strips > CUS
+        wide = mt > 1 and over and not one
         v = {1: 20, 2: 23 if wide else 22, 4: 25 if wide else 24}[mt]
-        if mt == 1 and k <= 8192:
-            return v, 2 if k > 4096 and strips < 256 and k % 2048 == 0 else 1
-        if (mt == 2 and k <= 4096) or (mt == 4 and m * k <= 160 << 10):
-            return v, 1
+        if mt == 1 and k <= 8192 and (not over or m * k <= 32 << 10):
+            halves = k > 4096 and 2 * strips <= CUS and k % 2048 == 0
+            if halves or k <= 4096 or m * k <= 64 << 10 or 4 * (n // 64) * choose_ksplit(m, n, k) < 3 * CUS:
+                return v, 2 if halves else 1
+        if not over or k <= 2048 or (wide and 4 * (strips // 2) >= 3 * CUS):
+            if mt == 2 and k <= 4096 and (m * k <= 96 << 10 or (2 * strips >= CUS and not wide)):
+                return v, 1
+            if mt == 4 and m * k <= 160 << 10:
+                return v, 1
     v = {2: 5, 4: 10}.get(mt, _DEFAULT_VARIANT[mt])
-    return v, choose_ksplit(m, n, k, variant=v)
+    ks = choose_ksplit(m, n, k, variant=v)
+    if mt in (2, 4) and k % 512 == 0:
+        coarse = choose_ksplit(m, n, k)
+        if mt == 2 and ks == coarse and k // ks >= 2048 and n // 64 * ks < CUS:
+            v = _DEFAULT_VARIANT[mt]
+        elif ks > coarse and k // ks < 512:
+            ks = coarse
+    return v, ks
 
 
 def skinny_config(m: int, n: int, k: int, fp8: bool = False) -> tuple[int, int]:

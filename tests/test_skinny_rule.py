@@ -24,6 +24,24 @@ def test_rule_is_launchable():
                     assert not one or D.SKINNY_VARIANTS[v][0] == 1 or m > 64
 
 
+def test_rule_keeps_to_where_its_forms_are_the_faster():
+    """Where all of x per workgroup, a second round of workgroups or short slices cost more than they give."""
+    kin = set()
+    for m in (1, 8, 16, 17, 24, 32, 40, 64):
+        for n in (1024, 1280, 2048, 3072, 4096, 5120, 6144, 9216):
+            for k in (1024, 2048, 2560, 3072, 4096, 5120, 8192, 10240):
+                v, ks = D.skinny_rule(m, n, k)
+                strips = n // (16 * D.SKINNY_VARIANTS[v][0])
+                if v in D.KIN_VARIANTS:
+                    kin.add((m, n, k))
+                    assert ks * strips <= 384 and (strips <= 256 or m <= 16 and m * k <= 32 << 10)
+                elif m > 16:
+                    assert k // ks >= 512 or ks <= D.choose_ksplit(m, n, k)
+    assert not kin & {(16, 5120, 3072), (16, 5120, 5120), (16, 3072, 8192), (32, 5120, 3072), (32, 1024, 4096), (40, 5120, 3072), (16, 6144, 4096)}
+    assert kin >= {(16, 4096, 4096), (16, 2048, 8192), (8, 6144, 4096), (24, 6144, 2048), (32, 4096, 4096), (40, 6144, 2048), (64, 2048, 2048)}
+    assert D.skinny_rule(24, 5120, 10240)[0] == 4 and D.skinny_rule(24, 16384, 2048)[0] == 5 and D.skinny_rule(48, 1024, 4096) == (10, 8)
+
+
 class _Weight:
     def __init__(self, n, k, rope=None, fp8=False):
         self.n, self.k, self.rope, self.fp8 = n, k, rope, fp8

@@ -368,6 +368,7 @@ def choose_ksplit(m: int, n: int, k: int, cus: int = CUS, variant: int = 0) -> i
     return best
 
 
+@lru_cache(maxsize=4096)
 def skinny_rule(m: int, n: int, k: int, one: bool = False) -> tuple[int, int]:
     """(variant, ksplit) of bf16 weights without a measured entry; ``one``: one W-row tile per wave.
 

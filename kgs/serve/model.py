@@ -192,13 +192,22 @@ class ServingModel:
             return (x.float() @ w.float().T).to(torch.bfloat16)
         m = x.shape[0]
         if decode:
-            table = D.w4x_route(m, w.shape[0], w.shape[1])
-            route = table or D.w4x_rule(m, w.shape[0], w.shape[1])
+            n, k = w.shape
+            table = D.w4x_route(m, n, k)
+            rule = D.w4x_rule(m, n, k) if table is None else None
+            route = table or (rule if rule is not None and rule[1] == 1 else None)
             if route is not None:
                 from kgs.ops.gemm import gemm_nt_w4x
 
                 return gemm_nt_w4x(x, w, bn=route[0], nslice=route[1], bm=route[2], stages=D.w4x_stages(route),
                                    nt_weights=D.w4x_nt(route), private=table is None)
+            # slices whose sum nothing takes: the general kernel's tiles, but for small outputs of a middling K the
+            # library's (us at 96 rows, the rule's slices and their sum / general / library: 1024x1024 9.5 / 7.0 / 8.3,
+            # 2560x7168 18.9 / 17.7 / 20.3, 5120x5120 25.4 / 21.2 / 27.2; 1024x4096 14.5 / 11.5 / 8.9, 2048x2048 11.8 / 11.1 / 8.5)
+            if rule is not None and not (n <= 2048 and 1024 < k <= 4096):
+                from kgs.ops import gemm_nt
+
+                return gemm_nt(x, w)
         if decode:
             ns = D.splitk_slices(m, w.shape[0], w.shape[1])
             if ns == 1:

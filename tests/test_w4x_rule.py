@@ -31,6 +31,29 @@ def test_rule_is_launchable_over_sizes():
         assert all(D.w4x_rule(m, n, k) is None for m in (33, 100, 256))
 
 
+@pytest.mark.parametrize("m,n,k,taken", [(96, 1024, 1024, "general"), (96, 2560, 7168, "general"), (96, 1024, 4096, "library"), (33, 1536, 1536, "library"),
+                                         (100, 32000, 2048, "tiles"), (100, 16384, 4096, "general"), (100, 6144, 4096, "tiles")])
+def test_decode_products_that_nothing_sums_are_not_sliced(m, n, k, taken, monkeypatch):
+    """Slices by rule are for consumers that take their sums: a launch of its own for it costs more than they give
+    (entries measured one by one keep theirs)."""
+    import kgs.ops
+    from kgs.ops import gemm
+    from kgs.serve.model import ServingModel
+
+    calls = []
+    monkeypatch.setattr(gemm, "gemm_nt_w4x", lambda *a, nslice=1, **kw: calls.append(("tiles", nslice)))
+    monkeypatch.setattr(kgs.ops, "gemm_nt", lambda *a, **kw: calls.append(("general", 1)))
+    monkeypatch.setattr(torch, "matmul", lambda *a: calls.append(("library", 1)))
+
+    class M:
+        backend, packed, decode_fp8 = "kgs", None, False
+        w = [{"o": torch.empty(n, k, dtype=torch.bfloat16, device="meta")}]
+
+    ServingModel._proj(M, torch.empty(m, k, dtype=torch.bfloat16, device="meta"), 0, "o", True)
+    assert [c[0] for c in calls] == [taken]
+    assert calls[0][1] == 1 or (n, k) in D._MEASURED
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("m", [33, 128, 129, 256])
 @pytest.mark.parametrize("n,k", [(128, 128), (768, 2048), (3072, 2048), (2048, 8192), (5120, 1408), (32000, 512)])

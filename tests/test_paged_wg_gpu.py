@@ -86,22 +86,22 @@ def test_split_rule_stays_in_its_bounds(batch, kv, pages):
 
 
 @pytest.mark.parametrize("fp8", [False, True])
-@pytest.mark.parametrize("groups,pages", [(1023, 1), (1024, 2), (1024, 5), (2047, 2), (2048, 2), (2048, 3), (2048, 8), (2048, 9), (8192, 16), (8192, 17),
-                                          (1, 4096), (8192, 4096)])
+@pytest.mark.parametrize("groups", [1, 639, 640, 1023, 1024, 1151, 1152, 1535, 1536, 2047, 2048, 8192])
+@pytest.mark.parametrize("pages", [1, 2, 3, 4, 5, 8, 9, 16, 17, 4096])
 def test_wave_rule(fp8, groups, pages):
-    """Narrow tables of many pairs by few waves, everything else by as many as elsewhere."""
+    """Narrow tables by few waves, the fewer the more pairs there are; everything else by as many as elsewhere."""
     from kgs.ops.decode import workgroup_waves
 
     w, most = workgroup_waves(groups, pages, fp8), 4 if fp8 else 8
     assert w in ((1, 2, 4) if fp8 else (1, 2, 4, 8))
-    assert w == most or (groups >= 1024 and pages <= (16 if fp8 else 8))
-    assert w == 1 or w >= min(2, most) and (w > 1 or groups >= 2048)
+    assert w == most or pages <= (16 if fp8 else 8)
     assert w <= workgroup_waves(groups, pages + 1, fp8) and w >= workgroup_waves(groups + 1, pages, fp8)
+    assert w == 1 if pages == 1 and (groups >= 640 or not fp8) else w > 1 or groups >= 1152
 
 
 @pytest.mark.parametrize("fp8", [False, True])
 @pytest.mark.parametrize("pages", [1, 2, 3, 4, 5, 8, 9, 16])
-@pytest.mark.parametrize("batch", [127, 128, 256])
+@pytest.mark.parametrize("batch", [5, 79, 80, 127, 128, 144, 256])
 def test_few_waves_on_narrow_tables(batch, pages, fp8):
     """Either side of each border of the rule, contexts of every length that the table holds."""
     from kgs.ops import decode as D

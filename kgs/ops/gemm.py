@@ -75,15 +75,17 @@ def gemm_nt(
         if tuple(out.shape) != (M, N):
             raise ValueError(f"out has shape {tuple(out.shape)}, expected {(M, N)}")
     pa, pb, lda, ldb = a.data_ptr(), b.data_ptr(), a.stride(0), b.stride(0)
-    if variant == "auto" and K > PAD_MIN_K and (K % 8 or (lda | ldb) % 8 or (pa | pb) % 16):
-        a, b = _even(a, b)
-        K = a.shape[1]
-        pa, pb, lda, ldb = a.data_ptr(), b.data_ptr(), a.stride(0), b.stride(0)
     pbias = bias.data_ptr() if bias is not None else None
     if variant == "auto":
-        ws = _scratch(M, N, K, a.device)
-        rc = _lib.lib().kgs_gemm_bf16_nt_auto(pa, pb, out.data_ptr(), pbias, M, N, K, lda, ldb, out.stride(0), epi,
-                                              None if ws is None else ws.data_ptr(), _lib.stream_handle(a.device))
+        odd_a, odd_b = (bool(K % 8 or ld % 8 or p % 16) for p, ld in ((pa, lda), (pb, ldb)))
+        if (odd_a or odd_b) and _pads(M, N, K):
+            ws = torch.empty(max(4, _padded_floats(M, N, K, odd_a, odd_b)), dtype=torch.float32, device=a.device)
+            rc = _lib.lib().kgs_gemm_bf16_nt_padded(pa, pb, out.data_ptr(), pbias, M, N, K, lda, ldb, out.stride(0), epi,
+                                                    ws.data_ptr(), _lib.stream_handle(a.device))
+        else:
+            ws = _scratch(M, N, K, a.device)
+            rc = _lib.lib().kgs_gemm_bf16_nt_auto(pa, pb, out.data_ptr(), pbias, M, N, K, lda, ldb, out.stride(0), epi,
+                                                  None if ws is None else ws.data_ptr(), _lib.stream_handle(a.device))
     else:
         rc = _lib.lib().kgs_gemm_bf16_nt(pa, pb, out.data_ptr(), pbias, M, N, K, lda, ldb, out.stride(0), epi, VARIANTS[variant],
                                          _lib.stream_handle(a.device))
@@ -92,7 +94,13 @@ def gemm_nt(
     return out
 
 
-PAD_MIN_K = 32  # products of shorter rows read them element by element where 16 bytes do not fit
+def _pads(m: int, n: int, k: int) -> bool:
+    """Whether operands whose rows 16-byte loads do not fit are copied into ones that they do, for the fast
+    tiles; else the product reads them element by element. The copy is a launch and an allocation, so calls in a row
+    take 13 us with it whatever their size, without it 8 (what the host takes) and the kernel's time beyond: 8.7 at 64 x 64 x 63,
+    10.3 at 97, 14.0 at 129; 1624 x 72 10.9 at 43, 13.3 at 65; 512 x 512 14.0 at 33, 17.2 at 63; 4096 x 4096 44 at 33
+    (with it 15). Under a graph the copy is the faster by 1.2 to 2 from 33 on."""
+    return k > (128 if m * n <= 4096 else 64 if min(m, n) <= 96 else 32)
 
 
 def _even(*ts: torch.Tensor) -> tuple[torch.Tensor, ...]:
@@ -115,6 +123,11 @@ def _even(*ts: torch.Tensor) -> tuple[torch.Tensor, ...]:
 @lru_cache(maxsize=4096)
 def _scratch_floats(m: int, n: int, k: int) -> int:
     return int(_lib.lib().kgs_gemm_bf16_nt_scratch(m, n, k))
+
+
+@lru_cache(maxsize=4096)
+def _padded_floats(m: int, n: int, k: int, odd_a: bool, odd_b: bool) -> int:
+    return int(_lib.lib().kgs_gemm_bf16_nt_padded_scratch(m, n, k, int(odd_a), int(odd_b)))
 
 
 def _scratch(m: int, n: int, k: int, device) -> torch.Tensor | None:
@@ -710,7 +723,7 @@ def gemm_nt_act(a: torch.Tensor, b: torch.Tensor, bias: torch.Tensor | None, act
         raise ValueError(f"inner dims differ: a {tuple(a.shape)} b {tuple(b.shape)}")
     if a.device != b.device:
         raise ValueError("a and b on different devices")
-    if K > PAD_MIN_K:
+    if _pads(M, N, K):
         a, b = _even(a, b)
         K = a.shape[1]
     if not _rows16(a) or not _rows16(b) or K % 8 or M == 0 or max(a.stride(0), b.stride(0)) >= 1 << 22:

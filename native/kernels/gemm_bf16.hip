@@ -408,6 +408,40 @@ KGS_EXPORT int kgs_gemm_bf16_nt_auto(const void* A, const void* B, void* C, cons
   return gemm_nt(A, B, C, bias, M, N, K, lda, ldb, ldc, epi, 0, ws, stream);
 }
 
+KGS_EXPORT int kgs_pad_rows_bf16(const void* src, void* dst, long rows, int cols, long ld, const void* src2, void* dst2,
+                                 long rows2, int cols2, long ld2, hipStream_t s);  // gemm_any.hip
+
+// The operands that kgs_pad_rows_bf16 has to copy for the fast kernels: rows that are not whole, aligned 16-byte chunks.
+static bool odd_rows(const void* P, int K, int ld) { return K % 8 || ld % 8 || (uintptr_t)P % 16; }
+
+// fp32 values of scratch for kgs_gemm_bf16_nt_padded: the copies (odd_a, odd_b: which) and the slices.
+KGS_EXPORT long kgs_gemm_bf16_nt_padded_scratch(int M, int N, int K, int odd_a, int odd_b) {
+  if (M <= 0 || N <= 0 || K <= 0) return 0;
+  const int kp = (K + 7) / 8 * 8;
+  return ((odd_a ? (long)M : 0) + (odd_b ? (long)N : 0)) * (kp / 2) + kgs::gemm_any_ws(M, N, kp);
+}
+
+// kgs_gemm_bf16_nt_auto through copies of the operands whose rows its fast kernels cannot read, in ws
+// (kgs_gemm_bf16_nt_padded_scratch values): both launches and one piece of scratch for one call (1024 x 256 x 65
+// in a row 13.3 us, with a call and an allocation for each copy 19.3).
+KGS_EXPORT int kgs_gemm_bf16_nt_padded(const void* A, const void* B, void* C, const void* bias, int M, int N, int K, int lda,
+                                       int ldb, int ldc, int epi, float* ws, hipStream_t stream) {
+  if (M <= 0 || N <= 0 || K <= 0 || lda < K || ldb < K || ldc < N) return KGS_ERR_SHAPE;
+  if (!ws || (uintptr_t)ws % 16) return KGS_ERR_ALIGN;
+  const bool oa = odd_rows(A, K, lda), ob = odd_rows(B, K, ldb);
+  const int kp = (K + 7) / 8 * 8;
+  auto pa = (unsigned short*)ws, pb = pa + (oa ? (long)M * kp : 0);
+  float* rest = (float*)(pb + (ob ? (long)N * kp : 0));
+  if (oa || ob) {
+    const int rc = oa ? kgs_pad_rows_bf16(A, pa, M, K, lda, ob ? B : nullptr, ob ? pb : nullptr, N, K, ldb, stream)
+                      : kgs_pad_rows_bf16(B, pb, N, K, ldb, nullptr, nullptr, 0, 0, 0, stream);
+    if (rc) return rc;
+  }
+  const bool slices = kgs::gemm_any_ws(M, N, kp) > 0;
+  return gemm_nt(oa ? pa : A, ob ? pb : B, C, bias, M, N, kp, oa ? kp : lda, ob ? kp : ldb, ldc, epi, 0, slices ? rest : nullptr,
+                 stream);
+}
+
 // In place C = bf16(C + bf16(A . B^T)) as kgs_gemm_bf16_nt_addc, for any M (N, K % 8): the persistent
 // kernel above one tile per CU (never in a capture, as there), else gemm_any.hip's. ws as in
 // kgs_gemm_bf16_nt_auto.

@@ -327,3 +327,36 @@ def test_fp8_auto_either_side_of_the_rule(M, N, K):
     a, b = (rnd(r, K).to(torch.float8_e4m3fn) for r in (M, N))
     want = a.double() @ b.double().T
     assert rel(gemm_fp8_nt(a, b), want) < REL and rel(gemm_fp8_nt(a, b, variant="bounded"), want) < REL
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 64, 130), (70, 100, 129), (300, 304, 2404), (16, 64, 2467), (513, 1030, 257), (64, 64, 65), (4096, 72, 43)])
+@pytest.mark.parametrize("odd", ["a", "b", "both"])
+@pytest.mark.parametrize("act", [None, "gelu"])
+def test_products_through_copies(M, N, K, odd, act):
+    """The one call that copies odd operands and multiplies: the bits of the two steps, whichever operand is odd (rows of no
+    multiple of 8, or a first value off the 16-byte grid) and with slices."""
+    from kgs.ops.gemm import _even, _pads, gemm_nt
+
+    def operand(rows, is_odd):
+        k = K if odd == "both" else (K + 7) // 8 * 8
+        t = rnd(rows, k + 8)
+        return t[:, 3:3 + k] if is_odd and odd != "both" else t[:, :k].contiguous()
+
+    a, b = operand(M, odd != "b"), operand(N, odd != "a")
+    bias = rnd(1, N)[0] if act else None
+    got, plain = gemm_nt(a, b, bias=bias, act=act), gemm_nt(*_even(a, b), bias=bias, act=act)
+    if _pads(M, N, a.shape[1]):
+        assert torch.equal(got, plain)
+    want = a.double() @ b.double().T
+    if act:
+        want = torch.nn.functional.gelu(want + bias.double(), approximate="tanh")
+    assert rel(got, want) < 2 * REL
+    assert rel(plain, want) < 2 * REL
+
+
+def test_short_odd_rows_are_read_where_they_lie():
+    """A copy is a launch and an allocation more: not for short rows of small products."""
+    from kgs.ops.gemm import _pads
+
+    assert not _pads(64, 64, 97) and not _pads(1624, 72, 43) and not _pads(4096, 4096, 32) and not _pads(1, 64, 128)
+    assert _pads(64, 64, 129) and _pads(1624, 72, 65) and _pads(512, 512, 33) and _pads(4096, 4096, 33)

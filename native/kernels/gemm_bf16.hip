@@ -367,7 +367,11 @@ static int gemm_nt(const void* A, const void* B, void* C, const void* bias, int 
         return (int)kgs::launch_w4p<kgs::EPI_NONE>((const unsigned short*)A, (const unsigned short*)B, (unsigned short*)C,
                                                    nullptr, M, N, K, lda, ldb, ldc, kgs::cu_count(), tq, stream);
     }
-    if (!large && kgs::gemm_any_ok(A, B, M, N, K, lda, ldb))
+    // large outputs of short sums whose rows are not 16-byte aligned: gemm_any's tiles would leave in 2-byte stores
+    // that nothing hides (us, its / the element-wise kernel's: 8192 x 8191 x 128 165 / 131, 3000 x 8001 x 64 65 / 50,
+    // 6272 x 3085 x 128 55 / 49, x 256 57 / 56, x 512 66 / 71; 2048 x 3001 x 128 21 / 21)
+    const bool short_odd = (ldc % 8 || (uintptr_t)C % 16) && K <= 256 && (long)M * N >= 1L << 23;
+    if (!large && !short_odd && kgs::gemm_any_ok(A, B, M, N, K, lda, ldb))
       return kgs::gemm_any(A, B, C, nullptr, bias, M, N, K, lda, ldb, ldc, epi, 0, 0, 0, ws, stream);
     v = large ? 3 : 2;
   } else if (variant == 3 || variant == 4) { if (!w4) return KGS_ERR_ALIGN; v = variant; }

@@ -360,3 +360,17 @@ def test_short_odd_rows_are_read_where_they_lie():
 
     assert not _pads(64, 64, 97) and not _pads(1624, 72, 43) and not _pads(4096, 4096, 32) and not _pads(1, 64, 128)
     assert _pads(64, 64, 129) and _pads(1624, 72, 65) and _pads(512, 512, 33) and _pads(4096, 4096, 33)
+
+
+@pytest.mark.parametrize("M,N,K,short", [(3000, 2801, 64, True), (2901, 2900, 256, True), (3000, 2801, 264, False), (2896, 2896, 64, False), (1000, 2801, 64, False)])
+@pytest.mark.parametrize("act", [None, "silu"])
+def test_large_odd_outputs_of_short_sums(M, N, K, short, act):
+    """Either side of where rows that leave in 2-byte stores go to the element-wise kernel: its bits there."""
+    from kgs.ops import gemm_nt
+
+    a, b, bias = rnd(M, K), rnd(N, K), rnd(1, N)[0] if act else None
+    got, plain = gemm_nt(a, b, bias=bias, act=act), gemm_nt(a, b, bias=bias, act=act, variant="generic")
+    assert torch.equal(got, plain) or not short
+    want = a.double() @ b.double().T
+    want = torch.nn.functional.silu(want + bias.double()) if act else want
+    assert rel(got, want) < 2 * REL and rel(plain, want) < 2 * REL

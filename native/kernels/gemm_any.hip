@@ -18,7 +18,6 @@
 // The order of the products in every accumulator is gemm_w4.h's, so without K slices the result
 // is bitwise the aligned kernels'. With slices each one writes fp32 partial tiles, which
 // any_reduce sums in a fixed order before the epilogue.
-#include <algorithm>
 #include <utility>
 
 #include "gemm_w4.h"
@@ -638,19 +637,16 @@ inline double cost(long M, long N, long K, int bm, int bn, int ns, int cus) {
 
 // The tile and the slices of a product. A slice keeps at least 512 of K: the partial tiles of
 // shorter ones cost as much as they save (300 x 304 x 2400: 10.6 us in slices of 640, 9.9 of 384).
-// Slices have to promise 7 % over a whole large tile, below which the estimate is not sure of them
-// (us unsplit / sliced: 512 x 4096 x 4096 35.8 / 28.7, 1024 x 1832 x 4096 37.2 / 27.9, 512 x 8192 x
-// 11008 110 / 87, 1321 x 5120 x 14336 177 / 166), and 15 % over 64x64 tiles (1024 x 1024 x 3072 15.6 /
-// 20.7, 413 x 2048 x 3072 16.5 / 20.0, 128 x 2048 x 2048 11.1 / 11.9).
+// Slices have to promise 15 %: below that the estimate is not sure of them (1024 x 768 x 2048), and
+// without them the result keeps the bits that it has in every other layout.
 inline Plan plan(long M, long N, long K, bool split, int cus) {
   Plan best{256, 256, 1};
-  double t0 = 1e30, small0 = 1e30;  // small0: what 64x64 tiles have to be below
+  double t0 = 1e30;
   const int shapes[3][2] = {{256, 256}, {256, 128}, {128, 128}};
   for (auto& s : shapes)
     for (int ns = 1; ns <= 16; ++ns) {
       if (ns > 1 && (!split || K < 512L * ns)) break;
-      const double c = cost(M, N, K, s[0], s[1], ns, cus), t = c * (ns > 1 ? 1.07 : 1.0);
-      small0 = std::min(small0, c * (ns > 1 ? 1.15 : 1.0));
+      const double t = cost(M, N, K, s[0], s[1], ns, cus) * (ns > 1 ? 1.15 : 1.0);
       if (t < t0) {
         t0 = t;
         best = {s[0], s[1], ns};
@@ -658,7 +654,7 @@ inline Plan plan(long M, long N, long K, bool split, int cus) {
     }
   // 64x64 tiles: a cheaper step, twice as many bytes per product; several share a CU
   const double full = (double)ceil_div(M, 64) * ceil_div(N, 64) / cus;
-  if (3.5 + ceil_div(K, 64) * (full <= 1 ? 0.34 + 0.06 * full : 0.06 + 0.38 * full) < small0) best = {64, 64, 1};
+  if (3.5 + ceil_div(K, 64) * (full <= 1 ? 0.34 + 0.06 * full : 0.06 + 0.38 * full) < t0) best = {64, 64, 1};
   return best;
 }
 
@@ -783,7 +779,7 @@ int gemm_any_ok(const void* A, const void* B, int M, int N, int K, int lda, int 
 }
 
 // C2: DUAL's second output, else null. bm, bn, ns: 0 for the plan's choice. ws: fp32 scratch for
-// the plan's slices (kgs_gemm_bf16_nt_scratch), null: no slices.
+// the plan's slices (kgs_gemm_bf16_nt_any_ws), null: no slices.
 int gemm_any(const void* A, const void* B, void* C, void* C2, const void* bias, int M, int N, int K, int lda, int ldb,
              int ldc, int epi, int bm, int bn, int ns, float* ws, hipStream_t s) {
   using namespace any;

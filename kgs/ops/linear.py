@@ -84,6 +84,13 @@ class Projection:
             return None
         table = D.w4x_route(m, n, k)
         route = table or D.w4x_rule(m, n, k, SPLIT_MAX_SLICES)
+        if table is None and route is not None and m > 128 and k > 4096 and n <= 16384:
+            # 128-row tiles read the weight twice, and the sum of slices is a launch of its own here: the
+            # general kernel instead, and 256-row tiles in two slices where those nearly fill the CUs. us at
+            # 129 rows, rule / general / two slices: 4096x8192 28.3 / 25.4 / -, 7168x5120 38.7 / 30.6 / -,
+            # 11008x8192 74.5 / 50.4 / -, 14336x5120 60.7 / 50.5 / 48.6, 16384x8192 87.1 / 86.6 / 75.0; at
+            # K = 4096 the rule's are as good or better (8192 at 256 rows 31.1 / 40.4)
+            route = (128, 2, 256) if n > 12800 and k % 256 == 0 else None
         if route is None:  # us at 64 rows of 4096x11008, which slices badly: 27 here, 36 by the library
             return gemm_nt(x, self.w) if m >= 128 or (n % 128 == 0 and k % 128 == 0) else None
         return gemm_nt_w4x(x, self.w, bn=route[0], nslice=route[1], bm=route[2], stages=D.w4x_stages(route),

@@ -54,9 +54,26 @@ def test_decode_products_that_nothing_sums_are_not_sliced(m, n, k, taken, monkey
     assert calls[0][1] == 1 or (n, k) in D._MEASURED
 
 
+@pytest.mark.parametrize("m,n,k,tiles", [(128, 4096, 8192, (8, 128)), (129, 4096, 8192, None), (192, 7168, 5120, None), (256, 5120, 8192, None),
+                                         (129, 11008, 8192, None), (129, 16384, 8192, (2, 256)), (256, 14336, 5120, (2, 256)),
+                                         (256, 14336, 5248, None), (129, 8192, 4096, (2, 128)), (256, 32768, 8192, (1, 256))])
+def test_projections_of_a_long_sum_above_128_rows(m, n, k, tiles, monkeypatch):
+    """There the rule's 128-row tiles take up to 48 % more than the general kernel or two slices
+    of 256-row ones."""
+    from kgs.ops import gemm
+    from kgs.ops.linear import Projection
+
+    calls = []
+    monkeypatch.setattr(gemm, "gemm_nt_w4x", lambda *a, nslice, bm, **kw: calls.append((nslice, bm)) or a[0])
+    monkeypatch.setattr(gemm, "gemm_nt", lambda *a, **kw: calls.append(None) or a[0])
+    p = Projection(torch.empty(n, k, dtype=torch.bfloat16, device="meta"))
+    p._plain(torch.empty(m, k, dtype=torch.bfloat16, device="meta"), m, n, k)
+    assert calls == [tiles]
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("m", [33, 128, 129, 256])
-@pytest.mark.parametrize("n,k", [(128, 128), (768, 2048), (3072, 2048), (2048, 8192), (5120, 1408), (32000, 512)])
+@pytest.mark.parametrize("n,k", [(128, 128), (768, 2048), (3072, 2048), (2048, 8192), (5120, 1408), (32000, 512), (13056, 4352)])
 def test_projection_and_partials(m, n, k):
     """Against the fp64 product: fp32 sums of exact bf16 products in any order (error below
     k 2^-24 of the sum of magnitudes), then one rounding to bf16."""

@@ -720,20 +720,33 @@ def workgroup_waves(groups: int, max_pages: int, fp8: bool) -> int:
     """Waves of such a workgroup for ``groups`` (sequence, KV head) pairs, 1 for the kernel of single waves.
 
     Eight (e4m3 pages four), except where the table is so narrow that a wave has a page or two: a workgroup's fixed
-    cost counts then, more so the more pairs a CU has. us by single waves / as many waves as elsewhere / by this
-    rule, 8 KV heads, contexts as long as the table and uniform up to there: bf16, one page, 256 pairs 3.5 / 3.8 / 3.5, 800
-    3.9 / 6.3 / 3.9; 256 sequences of 2 pages
-    11.7 / 17.3 / 11.7 and 9.5 / 16.1 / 9.5, of 4 22.0 / 24.5 / 21.6 and 16.7 / 19.0 / 14.7 (in two waves), 1024 of 8
-    170 / 171 / 173 and 110 / 104 / 102 (in four; most of them a few tokens: 43 / 61 / 39), 100 of 4 9.7 / 10.6 / 8.9 and 7.0 /
-    8.3 / 6.3 (in four); e4m3, 100 of 2 5.4 / 6.7 / 4.8 and 6.1 / 6.6 / 5.0 (in two), 160 of 4 9.8 / 11.8 / 9.8 and
-    9.4 / 11.1 / 9.4, 256 of 8 23.3 /
-    26.9 / 23.3 and 17.9 / 21.1 / 17.9, of 16 44.6 / 43.8 / 45.3 and 30.6 / 31.3 / 27.5 (in two), 1024 of 2 26 / 55 / 26
-    and 22 / 52 / 22. At 32 pages the waves of one group even out unequal contexts for more than they cost:
-    bf16, 256 sequences 156 / 163 and 113 / 90, e4m3 84.8 / 81.1 and 58.5 / 50.6."""
+    cost counts then, more so the more pairs a CU has. At 32 pages the waves of one group even out unequal contexts
+    for more than they cost. us with 8 KV heads, contexts as long as the table / uniform up to there:
+
+    ======  =========  =====  ==============  ===============  =====================
+    pages    sequences  type  single waves    8 (e4m3: 4)      this rule (waves)
+    ======  =========  =====  ==============  ===============  =====================
+    1        32         bf16  3.5             3.8              3.5 (1)
+    1        100        bf16  3.9             6.3              3.9 (1)
+    2        256        bf16  11.7 / 9.5      17.3 / 16.1      11.7 / 9.5 (1)
+    4        100        bf16  9.7 / 7.0       10.6 / 8.3       8.9 / 6.3 (4)
+    4        256        bf16  22.0 / 16.7     24.5 / 19.0      21.6 / 14.7 (2)
+    8        1024       bf16  170 / 110       171 / 104        173 / 102 (4)
+    32       256        bf16  156 / 113       163 / 90         163 / 90 (8)
+    2        100        e4m3  5.4 / 6.1       6.7 / 6.6        4.8 / 5.0 (2)
+    2        130        e4m3  6.1 / 6.0       8.7 / 8.5        6.1 / 6.0 (1)
+    2        1024       e4m3  26 / 22         55 / 52          26 / 22 (1)
+    4        160        e4m3  9.8 / 9.4       11.8 / 11.1      9.8 / 9.4 (1)
+    8        181        e4m3  19.9 / 16.1     19.7 / 16.0      20.3 / 14.5 (2)
+    8        256        e4m3  23.3 / 17.9     26.9 / 21.1      23.3 / 17.9 (1)
+    16       256        e4m3  44.6 / 30.6     43.8 / 31.3      45.3 / 27.5 (2)
+    32       256        e4m3  84.8 / 58.5     81.1 / 50.6      81.1 / 50.6 (4)
+    ======  =========  =====  ==============  ===============  =====================
+    """
     if fp8:
         if groups < 640:
             return 4
-        if max_pages <= (8 if groups >= 1536 else 4 if groups >= 1152 else 1):
+        if max_pages <= (8 if groups >= 1536 else 4 if groups >= 1152 else 2 if groups >= 1024 else 1):
             return 1
         return 2 if max_pages <= 16 else 4
     if max_pages <= (2 if groups >= 2048 else 1):

@@ -96,7 +96,8 @@ def test_wave_rule(fp8, groups, pages):
     assert w in ((1, 2, 4) if fp8 else (1, 2, 4, 8))
     assert w == most or pages <= (16 if fp8 else 8)
     assert w <= workgroup_waves(groups, pages + 1, fp8) and w >= workgroup_waves(groups + 1, pages, fp8)
-    assert w == 1 if pages == 1 and (groups >= 640 or not fp8) else w > 1 or groups >= 1152
+    assert w == 1 if pages == 1 and (groups >= 640 or not fp8) else w > 1 or groups >= (1152 if pages > 2 else 1024)
+    assert w == 1 or not (fp8 and pages <= 2 and groups >= 1024)
 
 
 @pytest.mark.parametrize("fp8", [False, True])

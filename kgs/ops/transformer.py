@@ -274,15 +274,20 @@ def attention_blocks(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, items: t
     ``q`` / ``out``, the row of its sequence's key 0, the position of the first row, and twice its
     number of rows, plus 1 for keys in ``k2`` / ``v2`` instead of ``k`` / ``v``. ``merges``, ``slots``:
     those of :func:`split_items`, whose parts of a block's keys are put together in a second launch."""
-    for t, n in ((q, "q"), (k, "k"), (v, "v"), (out, "out")):
-        _need(t, n)
-    if items.dtype != torch.int32 or items.dim() != 2 or items.shape[1] != 4 or not items.is_contiguous():
-        raise ValueError("items must be contiguous int32 [n, 4]")
+    for t, n, h in ((q, "q", heads), (k, "k", kv_heads), (v, "v", kv_heads), (out, "out", heads), (k2, "k2", kv_heads), (v2, "v2", kv_heads)):
+        if t is not None:
+            _need(t, n)
+            if t.shape[1] < 128 * h or t.device != q.device:
+                raise ValueError(f"{n} must hold {h} heads of 128, on q's GPU")
+    if out.shape[0] < q.shape[0] or v.shape[0] < k.shape[0] or (v2 is not None and k2 is not None and v2.shape[0] < k2.shape[0]):
+        raise ValueError("out needs q's rows, the values the keys'")
+    if items.dtype != torch.int32 or items.dim() != 2 or items.shape[1] != 4 or not items.is_contiguous() or items.device != q.device:
+        raise ValueError("items must be contiguous int32 [n, 4] on q's GPU")
     if (k2 is None) != (v2 is None) or (k2 is not None and k2.stride() != v2.stride()):
         raise ValueError("k2 and v2 come together, with one row stride")
     if merges is not None and (merges.dtype != torch.int32 or merges.dim() != 2 or merges.shape[1] != 4 or
-                               not merges.is_contiguous() or slots < 2 * merges.shape[0]):
-        raise ValueError("merges must be contiguous int32 [n, 4], with their slots")
+                               not merges.is_contiguous() or merges.device != q.device or slots < 2 * merges.shape[0]):
+        raise ValueError("merges must be contiguous int32 [n, 4] on q's GPU, with their slots")
     scale = 1.0 / math.sqrt(128) if scale is None else scale
     ws = None if merges is None else torch.empty(slots * heads * QBLOCK * (128 + 2), dtype=torch.float32, device=q.device)
     two = (0, 0, 0) if k2 is None else (k2.data_ptr(), v2.data_ptr(), k2.stride(0))

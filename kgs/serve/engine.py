@@ -42,7 +42,7 @@ class SamplingParams:
     presence_penalty: float = 0.0   # OpenAI: minus this once for every token already generated
     frequency_penalty: float = 0.0  # OpenAI: minus this times the token's count in the output
     repetition_penalty: float = 1.0  # CTRL/HF: logits of prompt+output tokens divided (>0) / multiplied (<0)
-    seed: int | None = None          # per-request sampling generator (reproducible regardless of batch mates)
+    seed: int | None = None          # per-request sampling generator (its draws do not depend on batch mates)
 
 
 @dataclass

@@ -457,7 +457,8 @@ class ServingModel:
         the device. ``wanted``: the portions whose last row is wanted, all by default.
 
         The layers run without the padding wherever that saves a 128-row tile of their products:
-        no result depends on it, and it is an eighth of the rows at 500 tokens a prompt (16 such
+        no result takes anything from it (a product of fewer rows may add its K slices in another
+        order, so fp32 sums and the bits after them can differ), and it is an eighth of the rows at 500 tokens a prompt (16 such
         prompts at hidden 4096: 12.85 ms with it, 10.32 without), most of them at 20; ``force``: in any
         case. Equal portions without cached tokens that need no rows dropped keep the batched
         launch."""

@@ -1199,7 +1199,9 @@ __global__ __launch_bounds__(64) void paged_decode(AttnArgs a) {
 // (wave w takes pages w, w + W, ..) and the waves merge in LDS. Bound by the HBM reads of K and V:
 // 100 sequences of 60 to 2800 tokens (4 KV heads) 60 -> 42 us at 4.4 TB/s, one of 4000 (8 KV heads)
 // 22 -> 11 us, 256 unequal ones around 1024 329 -> 171 us; 256 equal ones of 1024, which the single
-// waves already read at 6.9 TB/s, 156 -> 163 us.
+// waves already read at 6.9 TB/s, 156 -> 163 us (the host, which sees the table's width and not the
+// lengths, cannot tell the two; equal lengths lose 4 %, unequal ones gain half). Narrow tables take
+// fewer waves or the single-wave kernel by a rule on the host.
 //
 // A wave's page ids lie in its lanes (64 at a time, one load), so that no page waits for its id.
 // bf16 pages: eight waves, four on a SIMD hide each other's loads. e4m3 pages (PIPE): four waves

@@ -6,7 +6,7 @@
 //
 // What bounds such a product is the number of CUs that get a tile and the length of one
 // workgroup's serial chain of K-steps, so the tile (256x256, 256x128, 128x128 or 64x64) and the number
-// of K slices are chosen by sizes (any_plan below). 128x128 tiles keep a quarter of the AGPRs, so
+// of K slices are chosen by sizes (plan below). 128x128 tiles keep a quarter of the AGPRs, so
 // two workgroups share a CU and one's barriers and loads hide behind the other's MFMAs.
 //
 // Ragged sizes cost two selects per K-step: rows past M or N lie outside the buffer resources,
@@ -30,7 +30,7 @@ using w4::Ctx;
 using w4::Frag;
 
 typedef long i64x2 __attribute__((ext_vector_type(2)));
-constexpr int OOB = 0x7FFFFFF0;  // above every buffer resource's size (any_ok)
+constexpr int OOB = 0x7FFFFFF0;  // above every buffer resource's size (gemm_any_ok)
 
 // What a launch stores. DUAL: C gets bf16(acc + bias) and C2 the activation of that bf16 value
 // (a training forward pass, whose backward pass needs both).
@@ -274,8 +274,9 @@ void gemm_nt_any(Args a) {
 }
 
 // The same product on 64x64 tiles, for grids that leave CUs idle at 128x128. What bounds such a
-// launch is each workgroup's chain of K-steps; a step of this tile takes 0.27 us against 0.36 (LDS
-// traffic: half the bytes), and four times the workgroups share the epilogue. Four stages of 64-wide
+// launch is each workgroup's chain of K-steps; a step of this tile takes 0.26 us in a lone workgroup and
+// 0.27 with one on every CU, against 0.34 and 0.49 (LDS traffic: half the bytes; operands in L2, cost()
+// below has weights from HBM), and four times the workgroups share the epilogue. Four stages of 64-wide
 // K-tiles keep three on their way with one barrier per step (eight: the same time; 64x128 tiles with
 // three stages 0.44 us a step). Accumulators are plain registers, in gemm_w4.h's order of products per
 // element: bitwise the larger tiles' results. us, 128x128 / here: 1024^3 9.4 / 7.4, 256 x 3072 x 2048 15.1 /
@@ -779,7 +780,7 @@ int gemm_any_ok(const void* A, const void* B, int M, int N, int K, int lda, int 
 }
 
 // C2: DUAL's second output, else null. bm, bn, ns: 0 for the plan's choice. ws: fp32 scratch for
-// the plan's slices (kgs_gemm_bf16_nt_any_ws), null: no slices.
+// the plan's slices (kgs_gemm_bf16_nt_scratch), null: no slices.
 int gemm_any(const void* A, const void* B, void* C, void* C2, const void* bias, int M, int N, int K, int lda, int ldb,
              int ldc, int epi, int bm, int bn, int ns, float* ws, hipStream_t s) {
   using namespace any;

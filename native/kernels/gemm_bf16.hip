@@ -311,8 +311,9 @@ KGS_EXPORT int kgs_gemm_bf16_nt_w4x_ex(const void* A, const void* B, void* C, fl
 //          per tile), 16 = force the bounded 256x256 pipeline. Anything else
 //          is rejected.
 // Auto takes aligned products of more than 128 256x256 tiles (half the CUs) to variant 3, ragged
-// rows with more tiles than CUs to its persistent kernel, and every other product whose rows are 16-byte aligned to gemm_any.hip, which chooses its tile and, with
-// scratch (kgs_gemm_bf16_nt_auto), its K slices by sizes.
+// rows with more tiles than CUs to its persistent kernel, and every other product whose rows are 16-byte
+// aligned to gemm_any.hip, which chooses its tile and, with scratch (kgs_gemm_bf16_nt_auto), its K slices by
+// sizes; the rest, and large odd outputs of short sums, to the element-wise kernel (2).
 // C[M, N] = bf16(C + bf16(A . B^T)): a projection with the residual add in its
 // epilogue (EPI_ADDC; the prompt pass's o / down, whose add_rmsnorm becomes a
 // plain rmsnorm -- same roundings, so bitwise the unfused pair). The aligned
@@ -479,8 +480,8 @@ KGS_EXPORT int kgs_gemm_bf16_nt_swiglu(const void* A, const void* B, void* C, in
   return gemm_any_swiglu(A, B, C, M, N, K, lda, ldb, ldc, act, limit, stream);
 }
 
-// gemm_any.hip's kernel on tiles bm x bn (256 x 256, 256 x 128 or 128 x 128) over ns K slices (ws:
-// ns M (N rounded up to 8) values when ns > 1), for tests and measurements.
+// gemm_any.hip's kernels on tiles bm x bn (256 x 256, 256 x 128 or 128 x 128) over ns K slices (ws:
+// ns M (N rounded up to 8) values when ns > 1), or 64 x 64 with ns = 1, for tests and measurements.
 KGS_EXPORT int kgs_gemm_bf16_nt_any(const void* A, const void* B, void* C, const void* bias, int M, int N, int K,
                                     int lda, int ldb, int ldc, int epi, int bm, int bn, int ns, float* ws,
                                     hipStream_t stream) {
@@ -511,8 +512,8 @@ hipError_t launch_fp8_w4p(const unsigned short* A, const unsigned short* B, unsi
 
 namespace {
 
-// v 3: the four-wave persistent kernel (aligned, Kw >= 384 words, more tiles
-// than CUs); falls back to the 8-wave aligned kernel without a ticket slot
+// v 3: the four-wave persistent kernel (aligned, Kw >= 384 words, any number of
+// tiles); falls back to the 8-wave aligned kernel without a ticket slot
 template <int EPI>
 hipError_t launch_fp8(int v, const unsigned short* A, const unsigned short* B, unsigned short* C,
                       const unsigned short* bias, int M, int N, int Kw, int ldaw, int ldbw, int ldc, float alpha,
@@ -558,11 +559,12 @@ KGS_EXPORT int kgs_gemm_fp8_nt_dev(const void* A, const void* B, void* C, const 
   const int fast = kgs_gemm_fp8_nt_ok(A, B, C, M, N, K, lda, ldb, ldc, 0);
   const int bounded = kgs_gemm_fp8_nt_ok(A, B, C, M, N, K, lda, ldb, ldc, 1);
   // the four-wave persistent kernel: K >= 768 fp8 (384 words), 32-bit offsets
-  // over a 256-row panel, more tiles than CUs (round 3, gemm_w4f8.h)
+  // over a 256-row panel (gemm_w4f8.h)
   const int w4p = fast && K >= 768 && (long)(lda / 2) * 512 < (1L << 31) && (long)(ldb / 2) * 512 < (1L << 31);
   int v;
-  // the four-wave kernel wherever it can run: 4096 x 4096 x 14336 (a tile per CU) 145 us, the
-  // eight-wave one 218; 1024 x 4096 x 4096 (a quarter of the CUs) 37 and 65
+  // the four-wave kernel wherever it can run, us next to the eight-wave one: 4096 x 4096 x 14336 (a tile
+  // per CU) 145 / 217 on one set of operands, 158 / 289 on four in turn; 1024 x 4096 x 4096 (a quarter
+  // of the CUs) 37 / 65
   if (variant == 0) v = w4p ? 3 : fast ? 1 : 16;
   else if (variant == 1 || variant == 16 || variant == 64) v = variant;
   else if (variant == 3) { if (!w4p) return KGS_ERR_ALIGN; v = 3; }

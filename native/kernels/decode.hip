@@ -328,30 +328,50 @@ __global__ __launch_bounds__(256, (MT * KC_ > 32 || R * MT >= 16) ? 1 : 2) void 
   }
   if constexpr (KIN) {
     // B fragment of k-step s: lane (column m = 16 c + (lane & 15), k = 8 (lane >> 4) ..)
-    const unsigned short* xr[MT];
+    // e4m3 weights with up to 16 rows in a form of its own: from the general one the compiler drains every load in
+    // the middle of a chunk (us at 1 / 16 rows: 4096x4096 8.0 / 9.8, here 7.4 / 8.5; 6144x4096 10.2 / 14.5, here 9.6 / 13.0)
+    if constexpr (W8 && MT == 1) {
+      const unsigned short* xr = x + (long)min(lane & 15, M - 1) * ldx + (long)kk0 * 32 + 8 * (lane >> 4);
+      bf16x8 xf[PF];
 #pragma unroll
-    for (int c = 0; c < MT; ++c) xr[c] = x + (long)min(16 * c + (lane & 15), M - 1) * ldx + (long)kk0 * 32 + 8 * (lane >> 4);
-    bf16x8 xf[PF][MT];
+      for (int p = 0; p < PF; ++p) xf[p] = *(const bf16x8*)(xr + p * 32);
+      for (int s0 = 0; s0 < nsteps; s0 += PF) {
 #pragma unroll
-    for (int p = 0; p < PF; ++p)
+        for (int p = 0; p < PF; ++p) {
 #pragma unroll
-      for (int c = 0; c < MT; ++c) xf[p][c] = *(const bf16x8*)(xr[c] + p * 32);
-    for (int s0 = 0; s0 < nsteps; s0 += PF) {
+          for (int r = 0; r < R; ++r) acc[r][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(dequant8(wf[p][r], wsc[r]), xf[p], acc[r][0], 0, 0, 0);
+          const int sn = min(s0 + p + PF, nsteps - 1);
 #pragma unroll
-      for (int p = 0; p < PF; ++p) {
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-          bf16x8 wdq;
-          if constexpr (W8) wdq = dequant8(wf[p][r], wsc[r]);
-          else wdq = wf[p][r];
-#pragma unroll
-          for (int c = 0; c < MT; ++c) acc[r][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wdq, xf[p][c], acc[r][c], 0, 0, 0);
+          for (int r = 0; r < R; ++r) wf[p][r] = __builtin_nontemporal_load(wrow[r] + (long)sn * 64);
+          xf[p] = *(const bf16x8*)(xr + sn * 32);
         }
-        const int sn = min(s0 + p + PF, nsteps - 1);
+      }
+    } else {
+      const unsigned short* xr[MT];
 #pragma unroll
-        for (int r = 0; r < R; ++r) wf[p][r] = __builtin_nontemporal_load(wrow[r] + (long)sn * 64);
+      for (int c = 0; c < MT; ++c) xr[c] = x + (long)min(16 * c + (lane & 15), M - 1) * ldx + (long)kk0 * 32 + 8 * (lane >> 4);
+      bf16x8 xf[PF][MT];
 #pragma unroll
-        for (int c = 0; c < MT; ++c) xf[p][c] = *(const bf16x8*)(xr[c] + sn * 32);
+      for (int p = 0; p < PF; ++p)
+#pragma unroll
+        for (int c = 0; c < MT; ++c) xf[p][c] = *(const bf16x8*)(xr[c] + p * 32);
+      for (int s0 = 0; s0 < nsteps; s0 += PF) {
+#pragma unroll
+        for (int p = 0; p < PF; ++p) {
+#pragma unroll
+          for (int r = 0; r < R; ++r) {
+            bf16x8 wdq;
+            if constexpr (W8) wdq = dequant8(wf[p][r], wsc[r]);
+            else wdq = wf[p][r];
+#pragma unroll
+            for (int c = 0; c < MT; ++c) acc[r][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wdq, xf[p][c], acc[r][c], 0, 0, 0);
+          }
+          const int sn = min(s0 + p + PF, nsteps - 1);
+#pragma unroll
+          for (int r = 0; r < R; ++r) wf[p][r] = __builtin_nontemporal_load(wrow[r] + (long)sn * 64);
+#pragma unroll
+          for (int c = 0; c < MT; ++c) xf[p][c] = *(const bf16x8*)(xr[c] + sn * 32);
+        }
       }
     }
     // the four K quarters of the strip: waves 1-3 hand theirs to wave 0 (slot 0

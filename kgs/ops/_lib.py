@@ -37,6 +37,7 @@ _SIGS = {
     "kgs_gemm_bf16_nt": ([_c_void_p, _c_void_p, _c_void_p, _c_void_p] + [_c_int] * 8 + [_c_void_p], _c_int),
     "kgs_gemm_bf16_nt_scratch": ([_c_int] * 3, _c_long),
     "kgs_gemm_bf16_nt_auto": ([_c_void_p] * 4 + [_c_int] * 7 + [_c_void_p] * 2, _c_int),
+    "kgs_gemm_bf16_nt_off_lines": ([_c_void_p] + [_c_int] * 5, _c_int),
     "kgs_gemm_bf16_nt_padded_scratch": ([_c_int] * 5, _c_long),
     "kgs_gemm_bf16_nt_padded": ([_c_void_p] * 4 + [_c_int] * 7 + [_c_void_p] * 2, _c_int),
     "kgs_gemm_bf16_nt_any": ([_c_void_p] * 4 + [_c_int] * 10 + [_c_void_p] * 2, _c_int),

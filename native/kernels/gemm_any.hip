@@ -659,6 +659,21 @@ inline Plan plan(long M, long N, long K, bool split, int cus) {
   return best;
 }
 
+// Whether 256x256 tiles are plan's choice, or so near it that the eight-wave kernel of such tiles
+// (gemm_pipeline.h: the same bits) is the faster one where the rows of A start off the 128-byte lines. A K-step of
+// the tiles here then waits for twice the lines: 4 to 15 % of a product, of smaller tiles more; the
+// eight-wave kernel's loads do not show it. us, tiles by plan / eight waves, A's rows 16 bytes off a line or more
+// (both on lines): 3812 x 2240 x 4208 90 / 84 (80 / 80), 7738 x 1320 x 7584 163 / 141, 3653 x 2784 x 712 25.3 / 24.3, 10155 x 4216
+// x 3424 256 / 239 (222 / 228); where plan takes smaller tiles 1653 x 14544 x 3552 194 / 157, 3495 x 5248 x 4944 222 / 203, but
+// 3508 x 4928 x 888 47 / 49, 1752 x 9960 x 520 32 / 37: the estimates may differ by 3 % above K = 512, 14 % from
+// 3072 on, and shorter sums than 256 keep plan's tiles (8121 x 1312 x 160 13.5 / 14.9). B's rows do not matter
+// (72.3 / 71.9).
+inline bool wide(long M, long N, long K, bool split, int cus) {
+  const Plan p = plan(M, N, K, split, cus);
+  if (K < 256 || p.ns > 1 || p.bm == 64) return false;
+  return cost(M, N, K, 256, 256, 1, cus) <= cost(M, N, K, p.bm, p.bn, 1, cus) * (K >= 3072 ? 1.14 : K > 512 ? 1.03 : 1);
+}
+
 // Slices with which gemm_tr is the fastest way to a product with K-major operands, 0 where
 // another one is. The others transpose the operands first (a launch and a pass over memory each)
 // and run cost()'s best tile, or, for aligned sizes and a K-major B alone, the 256x256 kernel that
@@ -854,6 +869,8 @@ int gemm_any_f8(const void* A, const void* B, void* C, const void* bias, int M, 
 #undef KGS_F8
   return (int)hipGetLastError();
 }
+
+bool gemm_any_wide(int M, int N, int K, bool split) { return any::wide(M, N, K, split, cu_count()); }
 
 // fp32 values of scratch that a product's slices need (0: it has none)
 long gemm_any_ws(int M, int N, int K) {

@@ -170,6 +170,7 @@ int gemm_any_ok(const void* A, const void* B, int M, int N, int K, int lda, int 
 int gemm_any(const void* A, const void* B, void* C, void* C2, const void* bias, int M, int N, int K, int lda, int ldb,
              int ldc, int epi, int bm, int bn, int ns, float* ws, hipStream_t s);
 long gemm_any_ws(int M, int N, int K);
+bool gemm_any_wide(int M, int N, int K, bool split);
 int gemm_any_f8(const void* A, const void* B, void* C, const void* bias, int M, int N, int Kw, int lda, int ldb, int ldc,
                 float alpha, const float* alpha_ptr, int epi, hipStream_t s);
 int gemm_any_swiglu(const void* A, const void* B, void* C, int M, int N, int K, int lda, int ldb, int ldc, int act,
@@ -313,7 +314,8 @@ KGS_EXPORT int kgs_gemm_bf16_nt_w4x_ex(const void* A, const void* B, void* C, fl
 // Auto takes aligned products of more than 128 256x256 tiles (half the CUs) to variant 3, ragged
 // rows with more tiles than CUs to its persistent kernel, and every other product whose rows are 16-byte
 // aligned to gemm_any.hip, which chooses its tile and, with scratch (kgs_gemm_bf16_nt_auto), its K slices by
-// sizes; the rest, and large odd outputs of short sums, to the element-wise kernel (2).
+// sizes (256x256 tiles of an A whose rows start off the 128-byte lines: variant 16); the rest, and large odd outputs
+// of short sums, to the element-wise kernel (2).
 // C[M, N] = bf16(C + bf16(A . B^T)): a projection with the residual add in its
 // epilogue (EPI_ADDC; the prompt pass's o / down, whose add_rmsnorm becomes a
 // plain rmsnorm -- same roundings, so bitwise the unfused pair). The aligned
@@ -350,6 +352,12 @@ KGS_EXPORT int kgs_gemm_bf16_nt_addc(const void* A, const void* B, void* C, int 
   return (int)hipGetLastError();
 }
 
+// Whether auto runs a product that gemm_any could take on the eight-wave kernel of 256x256 tiles (its operands
+// permitting): A's rows off the 128-byte lines, and tiles of that size (any::wide). split: with scratch for slices.
+KGS_EXPORT int kgs_gemm_bf16_nt_off_lines(const void* A, int M, int N, int K, int lda, int split) {
+  return M > 0 && N > 0 && K > 0 && (lda % 64 || (uintptr_t)A % 128) && kgs::gemm_any_wide(M, N, K, split != 0);
+}
+
 static int gemm_nt(const void* A, const void* B, void* C, const void* bias, int M, int N, int K, int lda, int ldb,
                    int ldc, int epi, int variant, float* ws, hipStream_t stream) {
   if (M <= 0 || N <= 0 || K <= 0) return KGS_ERR_SHAPE;
@@ -372,9 +380,10 @@ static int gemm_nt(const void* A, const void* B, void* C, const void* bias, int 
     // that nothing hides (us, its / the element-wise kernel's: 8192 x 8191 x 128 165 / 131, 3000 x 8001 x 64 65 / 50,
     // 6272 x 3085 x 128 55 / 49, x 256 57 / 56, x 512 66 / 71; 2048 x 3001 x 128 21 / 21)
     const bool short_odd = (ldc % 8 || (uintptr_t)C % 16) && K <= 256 && (long)M * N >= 1L << 23;
-    if (!large && !short_odd && kgs::gemm_any_ok(A, B, M, N, K, lda, ldb))
+    const bool off = !large && bounded && kgs_gemm_bf16_nt_off_lines(A, M, N, K, lda, ws != nullptr);
+    if (!large && !short_odd && !off && kgs::gemm_any_ok(A, B, M, N, K, lda, ldb))
       return kgs::gemm_any(A, B, C, nullptr, bias, M, N, K, lda, ldb, ldc, epi, 0, 0, 0, ws, stream);
-    v = large ? 3 : 2;
+    v = large ? 3 : off ? 16 : 2;
   } else if (variant == 3 || variant == 4) { if (!w4) return KGS_ERR_ALIGN; v = variant; }
   else if (variant == 16) { if (!bounded) return KGS_ERR_ALIGN; v = 16; }
   else if (variant == 1) { if (!fast) return KGS_ERR_ALIGN; v = 1; }

@@ -374,3 +374,24 @@ def test_large_odd_outputs_of_short_sums(M, N, K, short, act):
     want = a.double() @ b.double().T
     want = torch.nn.functional.silu(want + bias.double()) if act else want
     assert rel(got, want) < 2 * REL and rel(plain, want) < 2 * REL
+
+
+@pytest.mark.parametrize("M,N,K,pad,off,taken", [(2560, 3912, 264, 0, 0, True), (2560, 3912, 248, 0, 0, False), (2576, 3584, 712, 0, 0, True), (2576, 3584, 704, 0, 0, False), (2576, 3584, 704, 8, 0, True),
+                                                 (2576, 3584, 704, 0, 8, True), (1500, 12344, 3080, 0, 0, True), (259, 264, 264, 0, 0, False)])
+@pytest.mark.parametrize("act", [None, "gelu", "silu"])
+def test_rows_off_the_lines(M, N, K, pad, off, taken, act):
+    """Rows of A that start off the 128-byte lines take the eight-wave kernel where the tiles are as large as its
+    own: the same bits as the tiles that any such product can have."""
+    from kgs.ops import _lib, gemm_nt
+    from kgs.ops.gemm import EPI
+
+    a = torch.full((M + 1, K + pad), float("nan"), device=DEV, dtype=torch.bfloat16).reshape(-1)[off:off + M * (K + pad)].view(M, K + pad)[:, :K]
+    b, bias = rnd(N, K), None if act is None else rnd(N)
+    a.copy_(rnd(M, K))
+    lib = _lib.lib()
+    assert lib.kgs_gemm_bf16_nt_off_lines(a.data_ptr(), M, N, K, a.stride(0), 0) == taken
+    got, tiles = gemm_nt(a, b, bias=bias, act=act), torch.empty(M, N, device=DEV, dtype=torch.bfloat16)
+    run_any(a, b, tiles, 256, 256, 1, bias, EPI[act])
+    if lib.kgs_gemm_bf16_nt_scratch(M, N, K) == 0:
+        assert torch.equal(got, tiles)
+    assert rel(got if act is None else gemm_nt(a, b), a.double() @ b.double().T) < REL

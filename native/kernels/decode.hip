@@ -534,6 +534,25 @@ __global__ __launch_bounds__(256, (MT * KC_ > 32 || R * MT >= 16) ? 1 : 2) void 
       }
     }
   };
+  // Above 128 rows the unrolled epilogues are 25 thousand instructions, and a product that has none fetched its way
+  // through them, 2 to 3 us of a launch: it stores by itself. us at 256 rows, through them / so: 4096x4096 63.6 /
+  // 59.9, 6144x4096 68.9 / 63.5, 5120x5120 79.5 / 76.5. (Apart from the rest: a change to what fewer rows' kernels hold
+  // here moves their register allocation, 28672x4096 at 16 rows 44 / 79.)
+  [[maybe_unused]] auto store = [&](f32x4v v, int m, int r) {
+    uint2 pk;
+    pk.x = pack_bf16x2(v[0], v[1]);
+    pk.y = pack_bf16x2(v[2], v[3]);
+    if (m < M) *(uint2*)(y + (long)m * ldy + 16 * (nt0 + r) + 4 * g) = pk;
+  };
+  if constexpr (MT > 8) {
+    if (ksplit == 1 && ep.mode == 0) {
+#pragma unroll
+      for (int c = 0; c < MT; ++c)
+#pragma unroll
+        for (int r = 0; r < R; ++r) store(acc[r][c], 16 * c + mc, r);
+      return;
+    }
+  }
   if (ksplit == 1) {
     if (KIN && w != 0) return;
 #pragma unroll
@@ -574,6 +593,30 @@ __global__ __launch_bounds__(256, (MT * KC_ > 32 || R * MT >= 16) ? 1 : 2) void 
   }
   __syncthreads();
   if (!*flag || (KIN && w != 0)) return;
+  if constexpr (MT > 8) {
+    if (ep.mode == 0) {
+#pragma unroll
+      for (int c = 0; c < MT; ++c) {
+        const int m = 16 * c + mc;
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          const unsigned at = (unsigned)((min(m, M - 1) * mstride + 16 * (nt0 + r) + 4 * g) * 4);
+          f32x4v t = f32x4v{0.f, 0.f, 0.f, 0.f};
+          for (int sp0 = 0; sp0 < ksplit; sp0 += 4) {  // four slabs' loads in flight, as below
+            f32x4v pv[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+              if (sp0 + j < ksplit) pv[j] = ld_sc1(wr, at + (unsigned)((sp0 + j) * sstride * 4));
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+              if (sp0 + j < ksplit) t += pv[j];
+          }
+          store(t, m, r);
+        }
+      }
+      return;
+    }
+  }
 #pragma unroll
   for (int c = 0; c < MT; ++c) {
     const int m = 16 * c + mc;

@@ -161,3 +161,24 @@ def test_exact_sums_of_squares(m, variant, ksplit, n):
         D.skinny_gemm(x, w, out=out, resid_ss=got[0], zero=torch.zeros(m, device=DEV))
     with pytest.raises(ValueError):
         D.skinny_gemm(out, up, rms=got[0][:, :m - 1].contiguous())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m", [129, 160, 241, 256])
+@pytest.mark.parametrize("ks", [1, 2, 7])
+def test_plain_products_above_128_rows_store_what_the_epilogues_do(m, ks):
+    """They have a way out of their own; the general one with a row scale of one gives the same bits, and rows and
+    columns outside the output stay as they were."""
+    n, k = 256, 512 * ks
+    x, w = (torch.rand(r, k, device=DEV) * 2 - 1 for r in (m, n))
+    pw, x, ss = D.PackedWeight(w.bfloat16()), x.bfloat16(), torch.full((m,), float(k), device=DEV)
+    for v in D.skinny_variants(m):
+        buf = torch.full((m + 1, n + 8), 7.0, device=DEV, dtype=torch.bfloat16)
+        D.skinny_gemm(x, pw, out=buf[:m, :n], variant=v, ksplit=ks)
+        want = x.double() @ w.bfloat16().double().T
+        # rsqrt(k * (1 / k)) is exactly one for powers of two
+        scaled = D.skinny_gemm(x, pw, rms=ss, eps=0.0, variant=v, ksplit=ks)
+        if k & (k - 1) == 0:
+            assert torch.equal(buf[:m, :n], scaled)
+        assert float((buf[:m, :n].double() - want).norm() / want.norm()) < 2.0 ** -8
+        assert bool((buf[m] == 7).all()) and bool((buf[:, n:] == 7).all())

@@ -5,7 +5,7 @@
 //   C[M, N] = epilogue(A[M, K] . B[N, K]^T + bias)
 //
 // What bounds such a product is the number of CUs that get a tile and the length of one
-// workgroup's serial chain of K-steps, so the tile (256x256, 256x128, 128x128 or 64x64) and the number
+// workgroup's serial chain of K-steps, so the tile (64x64, or 128x128 to 256x256 in steps of 32 and 64) and the number
 // of K slices are chosen by sizes (plan below). 128x128 tiles keep a quarter of the AGPRs, so
 // two workgroups share a CU and one's barriers and loads hide behind the other's MFMAs.
 //
@@ -133,9 +133,8 @@ __device__ __forceinline__ void store_row(const Args& a, int r, int col, const f
 // SW (a GateAct): B is a fused gate|up weight of N rows, gate rows first, and C [M, N / 2] holds
 // act(gate) * up; a tile stages both halves' rows in turn (gemm_w4.h). `bias` then points to the
 // clamped gate's limit.
-template <int EPI, int BM, int BN, bool SPLIT, bool DUAL, int SW = 0>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(waves_per_simd<BM, BN>(), waves_per_simd<BM, BN>())))
-void gemm_nt_any(Args a) {
+template <int EPI, int BM, int BN, bool SPLIT, bool DUAL, int SW>
+__device__ __forceinline__ void tile_product(const Args& a) {
   constexpr int X = SW * 1000000, TN = SW ? BN / 2 : BN;  // TN: output columns of a tile
   const int cols = SW ? a.N / 2 : a.N;
   using S = w4::Shape<BM, BN>;
@@ -271,6 +270,17 @@ void gemm_nt_any(Args a) {
     w4::read_row<NB, i>(v);
     store_row<EPI, NB, DUAL>(a, r, nw + lc, v, bv, old);
   });
+}
+
+// gemm_nt_any: the tiles of plan, with or without slices; gemm_nt_mid: those between them (refine), one workgroup a CU
+template <int EPI, int BM, int BN, bool SPLIT, bool DUAL, int SW = 0>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(waves_per_simd<BM, BN>(), waves_per_simd<BM, BN>())))
+void gemm_nt_any(Args a) {
+  tile_product<EPI, BM, BN, SPLIT, DUAL, SW>(a);
+}
+template <int EPI, int BM, int BN, bool DUAL, int SW = 0>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void gemm_nt_mid(Args a) {
+  tile_product<EPI, BM, BN, false, DUAL, SW>(a);
 }
 
 // The same product on 64x64 tiles, for grids that leave CUs idle at 128x128. What bounds such a
@@ -659,6 +669,64 @@ inline Plan plan(long M, long N, long K, bool split, int cus) {
   return best;
 }
 
+// A tile's time in an unsliced product, us, fitted to 310 sizes of 160 to 10000 rows (half of the errors below 6 %; the
+// tile that these estimates choose takes 0.8 % more than the best one): start, what each round of workgroups
+// after the first adds, and a K-step alone on a CU and what the chip's filling adds to it. 128x128 tiles: of two
+// workgroups on a CU, and of the single ones that remain.
+struct Tile {
+  int bm, bn;
+  double start, again, step, fill;
+};
+constexpr Tile TILES[] = {{256, 256, 7.12, 7.31, 0.88, 0.50}, {256, 128, 4.61, 4.53, 0.55, 0.29}, {128, 128, 3.5, 3.2, 0.97, 0},
+                          {192, 128, 4.15, 2.97, 0.44, 0.25}, {224, 128, 4.27, 3.53, 0.49, 0.28}, {192, 192, 5.02, 4.65, 0.56, 0.29},
+                          {224, 192, 5.40, 5.14, 0.61, 0.35}, {256, 192, 5.90, 5.94, 0.67, 0.38}, {224, 256, 6.49, 6.69, 0.78, 0.43}};
+inline double tile_cost(const Tile& t, long M, long N, long K, int cus) {
+  const long wg = (long)ceil_div(M, t.bm) * ceil_div(N, t.bn);
+  const int steps = 2 * ceil_div(K, 128);
+  if (t.bm == 128) {
+    const int two = (int)(wg / (2L * cus)), rest = (int)(wg - 2L * cus * two), pairs = two + (rest > cus);
+    const double one = rest > 0 && rest <= cus ? 0.34 + 0.26 * rest / cus : 0;
+    return t.start + steps * (pairs * t.step + one) + (two ? t.again * (two - (rest == 0)) : 0);
+  }
+  const int full = (int)(wg / cus), rest = (int)(wg - (long)full * cus), rounds = full + (rest > 0);
+  return t.start + (rounds - 1) * t.again + steps * (rounds * t.step + (full + (double)rest / cus) * t.fill);
+}
+inline double tile_cost(int bm, int bn, long M, long N, long K, int cus) {
+  for (const Tile& t : TILES)
+    if (t.bm == bm && t.bn == bn) return tile_cost(t, M, N, K, cus);
+  return 1e30;
+}
+
+// The tile of an unsliced product: plan's, or one between its three that leaves fewer CUs idle in the last round. What
+// such a product loses is that round (7 x 24 tiles of 256x256 are 168 of 256 CUs, 8 x 32 of 224x192 all of them);
+// a K-step of any of these tiles is bound by its operands' way into LDS, 60 bytes per ns and CU, so that the smaller ones are little
+// slower per product. The bits are the same. us, plan's tile / this one: 1762 x 6144 x 4096 81 / 66, 2830 x 6144 x 5504 199 / 145,
+// 1762 x 28672 x 4096 349 / 309, 590 x 11776 x 3472 75 / 57, 1382 x 6144 x 1152 28 / 21. sw: a gated product's tiles, whose
+// waves hold gate and up columns in turn, are 128 or 256 wide.
+inline Plan refine(Plan p, long M, long N, long K, int cus, bool sw = false) {
+  if (p.ns > 1 || p.bm == 64) return p;
+  double t0 = tile_cost(p.bm, p.bn, M, N, K, cus) * 0.97;
+  for (const Tile& t : TILES) {
+    if (sw && t.bn == 192) continue;
+    const double c = tile_cost(t, M, N, K, cus);
+    if (c < t0) {
+      t0 = c;
+      p.bm = t.bm;
+      p.bn = t.bn;
+    }
+  }
+  return p;
+}
+
+// Whether a product that the aligned, the persistent or the eight-wave 256x256 kernels take is better off on refine's
+// tile here: those keep a little (persistent tiles 3 % on average, 9 % at most) that a tile has to win back first. Of rows off
+// the 128-byte lines (wide below), us by eight waves / so: 1598 x 5680 x 4144 87 / 72, 2310 x 3384 x 8568 165 / 130, where
+// the estimate promises 8 % 3567 x 15328 x 928 108 / 111, 1505 x 8296 x 4336 103 / 98.
+inline bool finer(long M, long N, long K, int cus, bool sw = false) {
+  const Plan p = refine({256, 256, 1}, M, N, K, cus, sw);
+  return p.bm * p.bn < 65536 && tile_cost(p.bm, p.bn, M, N, K, cus) < 0.93 * tile_cost(TILES[0], M, N, K, cus);
+}
+
 // Whether 256x256 tiles are plan's choice, or so near it that the eight-wave kernel of such tiles
 // (gemm_pipeline.h: the same bits) is the faster one where the rows of A start off the 128-byte lines. A K-step of
 // the tiles here then waits for twice the lines: 4 to 15 % of a product, of smaller tiles more; the
@@ -734,9 +802,24 @@ int launch(Args a, Plan p, float* ws, hipStream_t s) {
     g.C = ws;
     g.ldc = ldp;
   }
-  if (p.bm == 128) launch_tile<EPI, 128, 128, DUAL>(g, p.ns, s);
-  else if (p.bn == 128) launch_tile<EPI, 256, 128, DUAL>(g, p.ns, s);
-  else launch_tile<EPI, 256, 256, DUAL>(g, p.ns, s);
+  if (p.ns > 1 && (p.bn == 192 || (p.bm != 128 && p.bm != 256))) return KGS_ERR_ARG;  // slices run on plan's tiles
+#define KGS_MID(BM, BN)                                                                                                \
+  case BM << 16 | BN:                                                                                                  \
+    hipLaunchKernelGGL((gemm_nt_mid<EPI, BM, BN, DUAL>), dim3((unsigned)(ceil_div(a.M, BM) * ceil_div(a.N, BN))), dim3(256), 0, s, g); \
+    break
+  switch (p.bm << 16 | p.bn) {
+    case 128 << 16 | 128: launch_tile<EPI, 128, 128, DUAL>(g, p.ns, s); break;
+    case 256 << 16 | 128: launch_tile<EPI, 256, 128, DUAL>(g, p.ns, s); break;
+    case 256 << 16 | 256: launch_tile<EPI, 256, 256, DUAL>(g, p.ns, s); break;
+    KGS_MID(192, 128);
+    KGS_MID(224, 128);
+    KGS_MID(192, 192);
+    KGS_MID(224, 192);
+    KGS_MID(256, 192);
+    KGS_MID(224, 256);
+    default: return KGS_ERR_ARG;
+  }
+#undef KGS_MID
   if (p.ns > 1)
     hipLaunchKernelGGL((any_reduce<EPI, DUAL>), dim3((unsigned)ceil_div((long)a.M * (ldp / 8), 256)), dim3(256), 0, s, ws,
                        (unsigned short*)a.C, a.C2, a.bias, a.M, a.N, a.ldc, ldp, p.ns, a.vec);
@@ -801,7 +884,7 @@ int gemm_any(const void* A, const void* B, void* C, void* C2, const void* bias, 
   using namespace any;
   const int vec = ldc % 8 == 0 && (uintptr_t)C % 16 == 0 && (uintptr_t)C2 % 16 == 0;
   if (epi == EPI_ADDC && (!vec || N % 8)) return KGS_ERR_ALIGN;
-  Plan p = bm ? Plan{bm, bn, ns} : plan(M, N, K, ws != nullptr, cu_count());
+  const Plan p = bm ? Plan{bm, bn, ns} : refine(plan(M, N, K, ws != nullptr, cu_count()), M, N, K, cu_count());
   if (p.ns > 1 && ws == nullptr) return KGS_ERR_ARG;
   const Args a{(const unsigned short*)A, (const unsigned short*)B, C, (unsigned short*)C2, (const unsigned short*)bias,
                M, N, K, lda, ldb, ldc, 0, M > N, vec, 1.f, nullptr};
@@ -831,21 +914,31 @@ int gemm_any_swiglu(const void* A, const void* B, void* C, int M, int N, int K, 
   using namespace any;
   const Args a{(const unsigned short*)A, (const unsigned short*)B, C, nullptr, (const unsigned short*)limit,
                M, N, K, lda, ldb, ldc, 0, M > N, ldc % 8 == 0 && (uintptr_t)C % 16 == 0, 1.f, nullptr};
-  const Plan p = plan(M, N, K, false, cu_count());
-  const int bm = p.bm == 256 ? 256 : 128, bn = bm == 256 && p.bn == 256 ? 256 : 128;
-  const dim3 grid((unsigned)(ceil_div(M, bm) * ceil_div(N / 2, bn / 2)));
-#define KGS_SWT(ACT)                                                                                                 \
-  if (bm == 128) hipLaunchKernelGGL((gemm_nt_any<EPI_NONE, 128, 128, false, false, ACT>), grid, dim3(256), 0, s, a); \
-  else if (bn == 128) hipLaunchKernelGGL((gemm_nt_any<EPI_NONE, 256, 128, false, false, ACT>), grid, dim3(256), 0, s, a); \
-  else hipLaunchKernelGGL((gemm_nt_any<EPI_NONE, 256, 256, false, false, ACT>), grid, dim3(256), 0, s, a)
+  Plan p = plan(M, N, K, false, cu_count());
+  if (p.bm == 64) p = {128, 128, 1};
+  p = refine(p, M, N, K, cu_count(), true);
+  const dim3 grid((unsigned)(ceil_div(M, p.bm) * ceil_div(N / 2, p.bn / 2)));
+#define KGS_SWK(BM, BN, ...) \
+  case BM << 16 | BN: hipLaunchKernelGGL((__VA_ARGS__>), grid, dim3(256), 0, s, a); break
+#define KGS_SWT(ACT)           \
+  switch (p.bm << 16 | p.bn) { \
+    KGS_SWK(128, 128, gemm_nt_any<EPI_NONE, 128, 128, false, false, ACT); \
+    KGS_SWK(256, 128, gemm_nt_any<EPI_NONE, 256, 128, false, false, ACT); \
+    KGS_SWK(256, 256, gemm_nt_any<EPI_NONE, 256, 256, false, false, ACT); \
+    KGS_SWK(192, 128, gemm_nt_mid<EPI_NONE, 192, 128, false, ACT);        \
+    KGS_SWK(224, 128, gemm_nt_mid<EPI_NONE, 224, 128, false, ACT);        \
+    KGS_SWK(224, 256, gemm_nt_mid<EPI_NONE, 224, 256, false, ACT);        \
+    default: return KGS_ERR_ARG;                                          \
+  }
   if (act == GATE_CLAMPED) {
-    KGS_SWT(GATE_CLAMPED);
+    KGS_SWT(GATE_CLAMPED)
   } else if (act == GATE_GELU) {
-    KGS_SWT(GATE_GELU);
+    KGS_SWT(GATE_GELU)
   } else {
-    KGS_SWT(GATE_SILU);
+    KGS_SWT(GATE_SILU)
   }
 #undef KGS_SWT
+#undef KGS_SWK
   return (int)hipGetLastError();
 }
 
@@ -869,6 +962,8 @@ int gemm_any_f8(const void* A, const void* B, void* C, const void* bias, int M, 
 #undef KGS_F8
   return (int)hipGetLastError();
 }
+
+bool gemm_any_finer(int M, int N, int K, bool sw) { return any::finer(M, N, K, cu_count(), sw); }
 
 bool gemm_any_wide(int M, int N, int K, bool split) { return any::wide(M, N, K, split, cu_count()); }
 

@@ -171,6 +171,7 @@ int gemm_any(const void* A, const void* B, void* C, void* C2, const void* bias, 
              int ldc, int epi, int bm, int bn, int ns, float* ws, hipStream_t s);
 long gemm_any_ws(int M, int N, int K);
 bool gemm_any_wide(int M, int N, int K, bool split);
+bool gemm_any_finer(int M, int N, int K, bool sw);
 int gemm_any_f8(const void* A, const void* B, void* C, const void* bias, int M, int N, int Kw, int lda, int ldb, int ldc,
                 float alpha, const float* alpha_ptr, int epi, hipStream_t s);
 int gemm_any_swiglu(const void* A, const void* B, void* C, int M, int N, int K, int lda, int ldb, int ldc, int act,
@@ -184,12 +185,19 @@ template <int EPI>
 hipError_t launch_w4p(const unsigned short* A, const unsigned short* B, unsigned short* C, const unsigned short* bias,
                       int M, int N, int K, int lda, int ldb, int ldc, int cus, int* tq, hipStream_t s);
 
-// Ragged rows on the persistent kernel: the fast path's rules but for M, and more tiles than CUs.
-static bool rows_ok(const void* A, const void* B, const void* C, int M, int N, int K, int lda, int ldb, int ldc) {
+// Ragged rows on the persistent kernel: the fast path's rules but for M, more tiles than CUs, and no finer tile
+// that fills them better (sw: a gated product's).
+static bool rows_ok(const void* A, const void* B, const void* C, int M, int N, int K, int lda, int ldb, int ldc, bool sw = false) {
   if (M <= 0 || N % 256 || K % 128 || K < 384 || (lda | ldb | ldc) % 8) return false;
   if (((uintptr_t)A | (uintptr_t)B | (uintptr_t)C) % 16) return false;
   if ((long)lda * 512 >= (1L << 31) || (long)ldb * 512 >= (1L << 31)) return false;
-  return ((long)M + 255) / 256 * (N / 256) > cu_count();
+  return ((long)M + 255) / 256 * (N / 256) > cu_count() && !gemm_any_finer(M, N, K, sw);
+}
+
+// Aligned products of up to one 256x256 tile per CU that a finer tile fills better. Above that they stay on the
+// persistent kernel, on which the tests of its ticket slots and captured graphs launch such sizes through gemm_nt.
+static bool aligned_finer(int M, int N, int K) {
+  return (long)(M / 256) * (N / 256) <= cu_count() && gemm_any_finer(M, N, K, false);
 }
 
 template <int EPI>
@@ -311,22 +319,24 @@ KGS_EXPORT int kgs_gemm_bf16_nt_w4x_ex(const void* A, const void* B, void* C, fl
 //          kernel's one-shot grid (one workgroup
 //          per tile), 16 = force the bounded 256x256 pipeline. Anything else
 //          is rejected.
-// Auto takes aligned products of more than 128 256x256 tiles (half the CUs) to variant 3, ragged
-// rows with more tiles than CUs to its persistent kernel, and every other product whose rows are 16-byte
+// Auto takes aligned products of more than 128 256x256 tiles (half the CUs) to variant 3 (up to one per CU unless a
+// finer tile fills the CUs better), ragged rows with more tiles than CUs to its persistent kernel (unless a finer tile does), and every other product whose rows are 16-byte
 // aligned to gemm_any.hip, which chooses its tile and, with scratch (kgs_gemm_bf16_nt_auto), its K slices by
 // sizes (256x256 tiles of an A whose rows start off the 128-byte lines: variant 16); the rest, and large odd outputs
 // of short sums, to the element-wise kernel (2).
 // C[M, N] = bf16(C + bf16(A . B^T)): a projection with the residual add in its
 // epilogue (EPI_ADDC; the prompt pass's o / down, whose add_rmsnorm becomes a
 // plain rmsnorm -- same roundings, so bitwise the unfused pair). The aligned
-// four-wave path only (kgs_gemm_bf16_nt_w4_ok); persistent with more tiles
-// than CUs on an eager stream, else (and in any hipGraph capture) the one-shot
+// four-wave path's operands only (kgs_gemm_bf16_nt_w4_ok); gemm_any.hip's tiles where they fill the CUs better, else
+// persistent with more tiles than CUs on an eager stream, else (and in any hipGraph capture) the one-shot
 // grid (tall problems in the mirrored order).
 KGS_EXPORT int kgs_gemm_bf16_nt_addc(const void* A, const void* B, void* C, int M, int N, int K, int lda, int ldb,
                                      int ldc, hipStream_t stream) {
   using namespace kgs;
   if (M <= 0 || N <= 0 || K <= 0 || lda < K || ldb < K || ldc < N) return KGS_ERR_SHAPE;
   if (!kgs_gemm_bf16_nt_w4_ok(A, B, C, M, N, K, lda, ldb, ldc)) return KGS_ERR_ALIGN;
+  if (aligned_finer(M, N, K))
+    return gemm_any(A, B, C, nullptr, nullptr, M, N, K, lda, ldb, ldc, EPI_ADDC, 0, 0, 0, nullptr, stream);
   auto a = (const unsigned short*)A;
   auto b = (const unsigned short*)B;
   auto c = (unsigned short*)C;
@@ -353,7 +363,8 @@ KGS_EXPORT int kgs_gemm_bf16_nt_addc(const void* A, const void* B, void* C, int 
 }
 
 // Whether auto runs a product that gemm_any could take on the eight-wave kernel of 256x256 tiles (its operands
-// permitting): A's rows off the 128-byte lines, and tiles of that size (any::wide). split: with scratch for slices.
+// permitting) unless a finer tile fills the CUs better: A's rows off the 128-byte lines, and tiles of that size (any::wide).
+// split: with scratch for slices.
 KGS_EXPORT int kgs_gemm_bf16_nt_off_lines(const void* A, int M, int N, int K, int lda, int split) {
   return M > 0 && N > 0 && K > 0 && (lda % 64 || (uintptr_t)A % 128) && kgs::gemm_any_wide(M, N, K, split != 0);
 }
@@ -370,7 +381,7 @@ static int gemm_nt(const void* A, const void* B, void* C, const void* bias, int 
   const int bounded = kgs_gemm_bf16_nt_bounded_ok(A, B, C, M, N, K, lda, ldb, ldc) && bias_ok;
   int v;
   if (variant == 0) {
-    const bool large = w4 && (long)(M / 256) * (N / 256) > 128;
+    const bool large = w4 && (long)(M / 256) * (N / 256) > 128 && !kgs::aligned_finer(M, N, K);
     if (!large && epi == kgs::EPI_NONE && kgs::rows_ok(A, B, C, M, N, K, lda, ldb, ldc)) {
       if (int* tq = kgs::tile_queue(stream))
         return (int)kgs::launch_w4p<kgs::EPI_NONE>((const unsigned short*)A, (const unsigned short*)B, (unsigned short*)C,
@@ -380,7 +391,7 @@ static int gemm_nt(const void* A, const void* B, void* C, const void* bias, int 
     // that nothing hides (us, its / the element-wise kernel's: 8192 x 8191 x 128 165 / 131, 3000 x 8001 x 64 65 / 50,
     // 6272 x 3085 x 128 55 / 49, x 256 57 / 56, x 512 66 / 71; 2048 x 3001 x 128 21 / 21)
     const bool short_odd = (ldc % 8 || (uintptr_t)C % 16) && K <= 256 && (long)M * N >= 1L << 23;
-    const bool off = !large && bounded && kgs_gemm_bf16_nt_off_lines(A, M, N, K, lda, ws != nullptr);
+    const bool off = !large && bounded && kgs_gemm_bf16_nt_off_lines(A, M, N, K, lda, ws != nullptr) && !kgs::gemm_any_finer(M, N, K, false);
     if (!large && !short_odd && !off && kgs::gemm_any_ok(A, B, M, N, K, lda, ldb))
       return kgs::gemm_any(A, B, C, nullptr, bias, M, N, K, lda, ldb, ldc, epi, 0, 0, 0, ws, stream);
     v = large ? 3 : off ? 16 : 2;
@@ -482,7 +493,7 @@ KGS_EXPORT int kgs_gemm_bf16_nt_swiglu(const void* A, const void* B, void* C, in
   if (M <= 0 || N <= 0 || K <= 0 || lda < K || ldb < K || ldc < N / 2) return KGS_ERR_SHAPE;
   if (act != GATE_SILU && act != GATE_GELU && (act != GATE_CLAMPED || !limit || (uintptr_t)limit % 4)) return KGS_ERR_ARG;
   if (N % 16 || ldc % 8 || (uintptr_t)C % 16 || !gemm_any_ok(A, B, M, N, K, lda, ldb)) return KGS_ERR_ALIGN;
-  if (rows_ok(A, B, C, M, N, K, lda, ldb, ldc))
+  if (rows_ok(A, B, C, M, N, K, lda, ldb, ldc, true))
     if (int* tq = tile_queue(stream))
       return (int)launch_w4p_swiglu((const unsigned short*)A, (const unsigned short*)B, (unsigned short*)C, M, N, K, lda,
                                     ldb, ldc, cu_count(), tq, act, limit, stream);
@@ -490,13 +501,14 @@ KGS_EXPORT int kgs_gemm_bf16_nt_swiglu(const void* A, const void* B, void* C, in
 }
 
 // gemm_any.hip's kernels on tiles bm x bn (256 x 256, 256 x 128 or 128 x 128) over ns K slices (ws:
-// ns M (N rounded up to 8) values when ns > 1), or 64 x 64 with ns = 1, for tests and measurements.
+// ns M (N rounded up to 8) values when ns > 1), or with ns = 1 on 64 x 64 and the tiles of launch there, for tests
+// and measurements.
 KGS_EXPORT int kgs_gemm_bf16_nt_any(const void* A, const void* B, void* C, const void* bias, int M, int N, int K,
                                     int lda, int ldb, int ldc, int epi, int bm, int bn, int ns, float* ws,
                                     hipStream_t stream) {
   if (M <= 0 || N <= 0 || K <= 0 || lda < K || ldb < K || ldc < N) return KGS_ERR_SHAPE;
   if (epi < 0 || epi > kgs::EPI_BIAS_SILU || (epi != kgs::EPI_NONE && !bias)) return KGS_ERR_ARG;
-  const bool large = (bm == 256 && (bn == 256 || bn == 128)) || (bm == 128 && bn == 128);
+  const bool large = bm >= 128 && bm <= 256 && bn >= 128 && bn <= 256;  // which of them: launch()
   const bool small = bm == 64 && bn == 64 && ns == 1;
   if (!(large || small) || ns < 1 || ns > 64) return KGS_ERR_ARG;
   if (!kgs::gemm_any_ok(A, B, M, N, K, lda, ldb) || (uintptr_t)ws % 16) return KGS_ERR_ALIGN;

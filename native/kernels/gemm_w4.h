@@ -76,12 +76,12 @@ constexpr int GM = 4;  // tile-group height (production choice)
 
 template <int BM, int BN>
 struct Shape {
-  static_assert(BN == 256 || BN == 128, "BN must be 256 or 128");
-  static_assert(BM == 256 || BM == 128, "BM must be 256 or 128");
-  static constexpr int MA = BM / 32;         // A fragments per wave per k-sub (8 or 4)
-  static constexpr int NB = BN / 32;         // B fragments per wave per k-sub (8 or 4)
-  static constexpr int OPA = BM * BK * 2;    // A operand of one stage: 32 or 16 KiB
-  static constexpr int OPB = BN * BK * 2;    // B operand of one stage: 32 or 16 KiB
+  static_assert(BN == 256 || BN == 192 || BN == 128, "BN must be 256, 192 or 128: whole fragment pairs per wave");
+  static_assert(BM % 32 == 0 && BM >= 128 && BM <= 256, "BM must be whole DMA groups of 32 rows, 128 to 256");
+  static constexpr int MA = BM / 32;         // A fragments per wave per k-sub (4 to 8)
+  static constexpr int NB = BN / 32;         // B fragments per wave per k-sub (4, 6 or 8)
+  static constexpr int OPA = BM * BK * 2;    // A operand of one stage: 16 to 32 KiB
+  static constexpr int OPB = BN * BK * 2;    // B operand of one stage: 16 to 32 KiB
   static constexpr int STAGE = OPA + OPB;
   static constexpr int LDS_BYTES = 2 * STAGE;
   static constexpr int HM = MA * NB;         // MFMAs per k-sub
@@ -351,7 +351,10 @@ __device__ __forceinline__ void kstep(const Ctx& c, Frag<BM / 32, BN / 32>& f0, 
 // Production knobs per tile shape: barrier 1 after MFMA B1, R MFMAs after
 // barrier 2, P reads per MFMA there, growing-square order, GROUP_M 4.
 template <int BM, int BN>
-struct Knobs;
+struct Knobs {  // the shapes between those below (gemm_any.hip): their proportions of a k-sub's reads
+  static constexpr int NR = Shape<BM, BN>::NR;
+  static constexpr int B1 = NR * 3 / 2, R = NR * 5 / 4, P = 1, ORD = 1, X = 0;
+};
 template <>
 struct Knobs<256, 256> {
   static constexpr int B1 = 24, R = 20, P = 1, ORD = 1, X = 0;

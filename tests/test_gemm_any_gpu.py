@@ -45,6 +45,56 @@ def test_any_tile_and_slices(M, N, K, bm, bn, ns):
     assert rel(c, torch.nn.functional.gelu(want + bias.double(), approximate="tanh")) < 2 * REL
 
 
+MID = [(192, 128), (224, 128), (192, 192), (224, 192), (256, 192), (224, 256)]
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 8, 8), (225, 200, 72), (193, 385, 136), (448, 264, 1096), (450, 392, 264)])
+@pytest.mark.parametrize("bm,bn", MID)
+def test_mid_tiles_repeat_the_large_tile_bits(M, N, K, bm, bn):
+    """The tiles between plan's three, at their edges: the 256x256 tile's bits, through views whose rows are not 16-byte
+    aligned in C and longer than K in A and B; nothing outside is written."""
+    A, B = rnd(M + 1, K + 16), rnd(N + 1, K + 8)
+    a, b, bias = A[:M, :K], B[1:, :K], torch.randn(N, device=DEV).bfloat16()
+    for epi in (0, 2):
+        want = torch.empty(M, N, device=DEV, dtype=torch.bfloat16)
+        run_any(a, b, want, 256, 256, 1, bias, epi)
+        big = torch.full((M + 1, N + 3), 7.0, device=DEV, dtype=torch.bfloat16)
+        run_any(a, b, big[:M, :N], bm, bn, 1, bias, epi)
+        assert torch.equal(big[:M, :N], want)
+        assert bool((big[M] == 7).all()) and bool((big[:, N:] == 7).all())
+    assert rel(want, torch.nn.functional.gelu(a.double() @ b.double().T + bias.double(), approximate="tanh")) < 2 * REL
+
+
+# sizes whose tile, by the rule, is each of MID
+@pytest.mark.parametrize("M,N,K", [(642, 5480, 128), (965, 5456, 136), (1541, 5008, 128), (1543, 5408, 128), (2035, 4832, 128),
+                                   (2054, 5392, 128)])
+def test_mid_tiles_with_every_epilogue(M, N, K):
+    """What is stored beside the product: the residual sum, both outputs of a training pass."""
+    from kgs.ops import gemm_nt
+    from kgs.ops.gemm import add_product_, gemm_nt_act, gemm_swiglu
+
+    a, b, bias = rnd(M, K), rnd(N, K), torch.randn(N, device=DEV).bfloat16()
+    z = a.double() @ b.double().T
+    assert rel(gemm_nt(a, b), z) < REL
+    c0 = rnd(M, N)
+    c = c0.clone()
+    assert add_product_(a, b, c) and rel(c, z + c0.double()) < 2 * REL
+    pre, y = gemm_nt_act(a, b, bias, "silu")
+    assert rel(pre, z + bias.double()) < REL
+    assert rel(y, torch.nn.functional.silu(pre.double())) < REL
+
+
+@pytest.mark.parametrize("M,N", [(642, 5504), (965, 5504), (1541, 5120)])
+@pytest.mark.parametrize("act", ["silu", "gelu_tanh"])
+def test_mid_tiles_of_gated_products(M, N, act):
+    from kgs.ops.gemm import gemm_swiglu
+
+    a, b = rnd(M, 128), rnd(N, 128)
+    g, u = (a.double() @ b.double().T).bfloat16().double().chunk(2, 1)
+    f = torch.nn.functional.silu(g) if act == "silu" else torch.nn.functional.gelu(g, approximate="tanh")
+    assert rel(gemm_swiglu(a, b, act), f * u) < 2 * REL
+
+
 def test_any_reads_nothing_past_its_operands():
     """Views inside larger buffers whose surroundings are NaN: the K tail and the rows past the
     end have to arrive as zeros."""

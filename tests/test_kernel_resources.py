@@ -278,6 +278,20 @@ def test_named_agpr_kernels_never_touch_agprs_outside_asm(gemm_build):
         assert not stray, (name, stray[:5])
 
 
+def test_tiles_between_the_three_keep_their_accumulators(gemm_build):
+    """gemm_nt_mid: six tiles x (6 epilogues, 3 with two outputs) and three of them x 3 gates; the rules of gemm_nt_any."""
+    res, asm = gemm_build
+    funcs = _functions(asm, r"gemm_nt_midI")
+    assert len(funcs) == 6 * (6 + 3) + 3 * 3, len(funcs)
+    for name, body in funcs.items():
+        bm, bn = map(int, re.search(r"gemm_nt_midILi\dELi(\d+)ELi(\d+)E", name).groups())
+        seen, stray = _stray_agpr_lines(body)
+        assert seen >= bm // 32 * (bn // 32) * 4 and not stray, (name, seen, stray[:5])
+        assert not any("v_accvgpr_mov" in ln for ln in body.splitlines()), name
+        r = res[name]
+        assert r["VGPRs Spill"] == 0 and r["SGPRs Spill"] == 0 and r["LDS Size"] == 2 * (bm + bn) * 128, (name, r)
+
+
 def _vregs(text: str) -> set:
     out = set()
     for a, b in re.findall(r"(?<![\w.])v\[(\d+):(\d+)\]", text):

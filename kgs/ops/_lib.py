@@ -208,6 +208,21 @@ def lib() -> ctypes.CDLL:
     return so
 
 
+@lru_cache(maxsize=1)
+def autograd():
+    """The native autograd nodes (``native/autograd``), on the kernels of :func:`lib`."""
+    so = lib()
+    try:
+        from .._native import _autograd
+    except ImportError as e:
+        raise NativeUnavailable(f"cannot load kgs/_native/_autograd: {e}; build it with `python -m kgs.utils.build`") from e
+    names = ("kgs_gemm_bf16_nt_auto", "kgs_gemm_bf16_nt_padded", "kgs_gemm_bf16_nt_act", "kgs_pad_rows_bf16", "kgs_act_grad",
+             "kgs_gemm_bf16_tr", "kgs_gemm_bf16_nt_scratch", "kgs_gemm_bf16_nt_padded_scratch", "kgs_act_grad_parts",
+             "kgs_gemm_bf16_tr_slices")
+    _autograd.bind({n: ctypes.cast(getattr(so, n), ctypes.c_void_p).value for n in names})
+    return _autograd
+
+
 def available() -> bool:
     try:
         lib()

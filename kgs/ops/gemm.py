@@ -818,7 +818,12 @@ def _act(z: torch.Tensor, act: str) -> torch.Tensor:
 
 
 def linear(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None, act: str | None = None):
-    """Differentiable ``act(x @ w.T + bias)`` on the HIP GEMM (x: [M,K], w: [N,K])."""
+    """Differentiable ``act(x @ w.T + bias)`` on the HIP GEMM (x: [M,K], w: [N,K]): by the native node
+    (``native/autograd/linear.cpp``) where the host bounds the layer, else by :class:`_LinearFn`."""
+    if x.is_cuda and act in EPI:
+        y = _lib.autograd().linear(x, w, bias, EPI[act])
+        if y is not None:
+            return y
     return _LinearFn.apply(x, w, bias, act)
 
 
@@ -835,6 +840,8 @@ class Linear(torch.nn.Module):
         self.act = act
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
+        if x.dim() == 2:
+            return linear(x.contiguous(), self.weight, self.bias, self.act)
         shp = x.shape
         y = linear(x.reshape(-1, shp[-1]).contiguous(), self.weight, self.bias, self.act)
         return y.reshape(*shp[:-1], y.shape[-1])

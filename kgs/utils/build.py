@@ -20,6 +20,9 @@ Builds, with the ROCm toolchain in ``/opt/rocm``:
   plugin's health path; loaded only through ``KGS_AMDSMI_LIB``.
 * ``kgs/_native/_serve*.so`` -- the continuous-batching scheduler and paged-KV
   block allocator of ``kgs.serve`` (C++17, pybind11).
+* ``kgs/_native/_autograd*.so`` -- the autograd node of ``kgs.ops.Linear`` for
+  layers that the host bounds (C++17 against torch's headers; it calls the
+  kernels at the addresses that ``kgs/ops/_lib.py`` hands it).
 * ``kgs/_native/kgs-rccl-bench`` -- single-process multi-GPU RCCL all-reduce
   sweep (ncclCommInitAll), the C++ twin of ``kgs.parallel.allreduce``.
 
@@ -118,6 +121,14 @@ def _py_ext_suffix() -> str:
     import sysconfig
 
     return sysconfig.get_config_var("EXT_SUFFIX") or ".so"
+
+
+def _torch_dir() -> Path | None:
+    """The installed torch package's folder (found, not imported), None without one."""
+    import importlib.util
+
+    spec = importlib.util.find_spec("torch")
+    return Path(spec.origin).parent if spec and spec.origin else None
 
 
 # ``--only`` group names: the device-plugin image builds ``gpuinfo`` (the three
@@ -238,6 +249,19 @@ def targets(out: Path | None = None) -> list[Target]:
             optional=True,
         ),
     ]
+    torch_dir = _torch_dir()
+    if torch_dir is not None:
+        inc = torch_dir / "include"
+        ts.insert(-1, Target(
+            "autograd",
+            odir / f"_autograd{_py_ext_suffix()}",
+            [NATIVE / "autograd" / "linear.cpp"],
+            CXX,
+            flags=["-O2", "-std=c++17", "-fPIC", "-Wall", "-Wno-unknown-pragmas", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
+                   "-DTORCH_EXTENSION_NAME=_autograd", "-DTORCH_API_INCLUDE_EXTENSION_H", f"-isystem{inc}",
+                   f"-isystem{inc / 'torch' / 'csrc' / 'api' / 'include'}", f"-isystem{ROCM / 'include'}"] + _pybind_includes(),
+            link_flags=[f"-L{torch_dir / 'lib'}", "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch", "-ltorch_python"],
+        ))
     return [t for t in ts if all(s.exists() for s in t.sources)]
 
 

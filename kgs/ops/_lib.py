@@ -117,6 +117,7 @@ _SIGS = {
     "kgs_attn_fwd_blocks_bf16": ([_c_void_p] * 7 + [_c_int] * 4 + [_c_long] * 5 + [ctypes.c_float, _c_void_p, _c_int, _c_int] +
                                  [_c_void_p] * 2, _c_int),
     "kgs_paged_decode_wg": ([_c_void_p] * 8 + [_c_int] * 6 + [_c_long, _c_long, ctypes.c_float, _c_int, _c_void_p], _c_int),
+    "kgs_paged_decode_wg_bal": ([_c_void_p] * 8 + [_c_int] * 7 + [_c_long, _c_long, ctypes.c_float, _c_int, _c_void_p], _c_int),
     "kgs_paged_decode_wg_ex": ([_c_void_p] * 8 + [_c_int] * 6 + [_c_long, _c_long, ctypes.c_float, _c_int, _c_int, _c_void_p], _c_int),
     "kgs_paged_decode_bf16_ex": ([_c_void_p] * 8 + [_c_int] * 7 + [_c_long, _c_long, ctypes.c_float, _c_int, _c_int,
                                                                    _c_void_p], _c_int),

@@ -960,6 +960,8 @@ struct AttnArgs {
   const int* pos;               // [B]
   const int* slot;              // [B] cache slot of the new token (< 0: no write)
   void* cache_w;                // the same layer base as cache, writable
+  // parts by length (paged_wg BAL): units (parts of a sequence) to deal the pages to, a part's least pages, units at most
+  int target, least, units;
 };
 
 // store O^T[dim 16dt + 4g + i][head] * inv for the lane's head
@@ -1260,7 +1262,7 @@ __global__ __launch_bounds__(64) void paged_decode(AttnArgs a) {
 // so a batch of unequal contexts waits for the longest one's wave, and at small batches a split
 // costs a merge through memory. Here the pages are dealt to the waves by the sequence's own length
 // (wave w takes pages w, w + W, ..) and the waves merge in LDS. Bound by the HBM reads of K and V:
-// 100 sequences of 60 to 2800 tokens (4 KV heads) 60 -> 42 us at 4.4 TB/s, one of 4000 (8 KV heads)
+// 100 sequences of 60 to 2800 tokens (4 KV heads) 60 -> 38 us, one of 4000 (8 KV heads)
 // 22 -> 11 us, 256 unequal ones around 1024 329 -> 171 us; 256 equal ones of 1024, which the single
 // waves already read at 6.9 TB/s, 156 -> 163 us (the host, which sees the table's width and not the
 // lengths, cannot tell the two; equal lengths lose 4 %, unequal ones gain half). Narrow tables take
@@ -1271,6 +1273,18 @@ __global__ __launch_bounds__(64) void paged_decode(AttnArgs a) {
 // that keep the next page on its way in registers while they widen and multiply one (64 sequences
 // around 700 tokens, 8 KV heads: 22 us, 31 without). Fewer waves where the table holds few pages
 // (kgs/ops/decode.py workgroup_waves).
+// Inclusive sums over the wave's lanes, all of them active: shifts by 1, 2, 4 and 8 within rows of 16, then the last
+// lane of row 0 (of 2) to row 1 (3) and of lane 31 to the upper half
+__device__ __forceinline__ int scan64(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);
+  return v;
+}
+
 template <bool KV8>
 struct PageRegs;  // a page's K and V as loaded: fragment order, e4m3 pages 8 bytes a lane
 template <>
@@ -1300,7 +1314,12 @@ struct PageRegs<true> {
   __device__ bf16x8 vf(int i) const { return dequant8(v[i], 1.f); }
 };
 
-template <bool KV8, int W = KV8 ? 4 : 8, bool PIPE = KV8>
+//
+// BAL: the parts follow the lengths, so that a long context is no longer one workgroup's (100 sequences of 60 to 2800 tokens, 4
+// KV heads: 38.1 -> 29.9 us, 70 of 4000 at most 44.9 -> 32.2; the rule is length_parts). All workgroups read all of them (a lane holds BAL of each 64) and cut
+// every sequence into equal parts of at most P pages, P such that `target` parts of P hold
+// them all (at least `least`): unit u of the grid is the u-th such part.
+template <bool KV8, int W = KV8 ? 4 : 8, bool PIPE = KV8, int BAL = 0>
 __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(PIPE ? 2 : 4, PIPE ? 2 : 4))) void paged_wg(AttnArgs a) {
   constexpr int LDO = HD + 4;  // a row of partial outputs: 16 heads' rows start on different banks
   __shared__ __attribute__((aligned(16))) float part[W][16][LDO];
@@ -1308,14 +1327,47 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(PIPE ? 2
   __shared__ int is_last;
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int G = a.H / a.HKV;
-  int id = blockIdx.x;
-  const int sp = id % a.nsplit;
-  id /= a.nsplit;
-  const int kvh = id % a.HKV, b = id / a.HKV;
+  int id = blockIdx.x, sp, kvh, b, nsplit = a.nsplit, first = 0;  // first: the sequence's first unit (BAL)
   const int g = lane >> 4, n = lane & 15;
+  if constexpr (BAL) {
+    kvh = id % a.HKV;
+    id /= a.HKV;
+    int pages[BAL], total = 0;
+#pragma unroll
+    for (int i = 0; i < BAL; ++i) {
+      const int at = 64 * i + lane;
+      pages[i] = at < a.B ? max(0, min((a.ctx_lens[at] + PAGE - 1) / PAGE, a.max_pages)) : 0;
+      total += pages[i];
+    }
+    total = __builtin_amdgcn_readlane(scan64(total), 63);
+    const int P = (max(a.least, (int)((unsigned)(total + a.target - 1) / (unsigned)a.target)) + W - 1) / W * W;  // whole rounds of the waves
+    b = -1;
+    int before = 0;
+#pragma unroll
+    for (int i = 0; i < BAL; ++i) {
+      const int parts = 64 * i + lane < a.B ? max(1u, (unsigned)(pages[i] + P - 1) / (unsigned)P) : 0;
+      const int upto = before + scan64(parts);
+      const unsigned long long hit = __ballot(parts && id >= upto - parts && id < upto);
+      if (hit) {
+        const int l = __builtin_ctzll(hit);
+        b = 64 * i + l;
+        nsplit = __builtin_amdgcn_readlane(parts, l);
+        first = __builtin_amdgcn_readlane(upto, l) - nsplit;
+        sp = id - first;
+        break;
+      }
+      before = __builtin_amdgcn_readlane(upto, 63);
+    }
+    if (b < 0) return;
+  } else {
+    sp = id % nsplit;
+    id /= nsplit;
+    kvh = id % a.HKV;
+    b = id / a.HKV;
+  }
   const int ctx = a.ctx_lens[b];
   const int npages = min((ctx + PAGE - 1) / PAGE, a.max_pages);
-  const int per = (npages + a.nsplit - 1) / a.nsplit;
+  const int per = (npages + nsplit - 1) / nsplit;
   const int p0 = sp * per, p1 = min(npages, p0 + per);
   const int h = kvh * G + n;
   const int mine = p1 > p0 + w ? (p1 - p0 - w + W - 1) / W : 0;  // this wave's pages
@@ -1403,7 +1455,10 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(PIPE ? 2
     }
   }
   __syncthreads();
-  const long nrows = (long)a.B * a.H * a.nsplit;
+  // rows of partial results: part s of head hh
+  const long nrows = (long)(BAL ? a.units : a.B * nsplit) * a.H;
+  const unsigned next = BAL ? a.H : 1;
+  auto row_of = [&](int hh) { return BAL ? (unsigned)(first * a.H + hh) : (unsigned)(((long)b * a.H + hh) * nsplit); };
   const __amdgpu_buffer_rsrc_t por = rsrc(a.po, (unsigned)(nrows * HD * 4));
   const __amdgpu_buffer_rsrc_t mlr = rsrc(a.pml, (unsigned)(nrows * 8));
   // a thread's four dims of one head
@@ -1423,12 +1478,12 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(PIPE ? 2
       o += f * *(const f32x4v*)&part[x][hn][d];
     }
     const int hh = kvh * G + hn;
-    if (a.nsplit == 1) {
+    if (nsplit == 1) {
       const float inv = L > 0.f ? 1.f / L : 0.f;
       *(uint2*)(a.o + (long)b * a.ldo + (long)hh * HD + d) =
           make_uint2(pack_bf16x2(o[0] * inv, o[1] * inv), pack_bf16x2(o[2] * inv, o[3] * inv));
     } else {
-      const unsigned row = (unsigned)(((long)b * a.H + hh) * a.nsplit + sp);
+      const unsigned row = row_of(hh) + sp * next;
       st_sc1(por, (row * HD + d) * 4, o);
       if (d == 0) {
         st1_sc1(mlr, row * 8, M);
@@ -1436,13 +1491,13 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(PIPE ? 2
       }
     }
   }
-  if (a.nsplit == 1) return;
+  if (nsplit == 1) return;
   // the split that arrives last merges: partial results written through, then a ticket
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
   if (threadIdx.x == 0) {
     int* c = a.cnt + (long)b * a.HKV + kvh;
-    const int last = __hip_atomic_fetch_add(c, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == a.nsplit - 1;
+    const int last = __hip_atomic_fetch_add(c, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == nsplit - 1;
     if (last) {
       __hip_atomic_store(c, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // re-arm
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
@@ -1452,22 +1507,59 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(PIPE ? 2
   }
   __syncthreads();
   if (!is_last) return;
-  for (int i = threadIdx.x; i < G * (HD / 4); i += 64 * W) {
-    const int hn = i >> 5, d = (i & 31) * 4, hh = kvh * G + hn;
-    const unsigned row = (unsigned)(((long)b * a.H + hh) * a.nsplit);
-    float M = -INFINITY, L = 0.f;
-    f32x4v o = f32x4v{0.f, 0.f, 0.f, 0.f};
-    for (int s0 = 0; s0 < a.nsplit; s0 += 4) {
+  if constexpr (!BAL) {
+    for (int i = threadIdx.x; i < G * (HD / 4); i += 64 * W) {
+      const int hn = i >> 5, d = (i & 31) * 4, hh = kvh * G + hn;
+      const unsigned row = (unsigned)(((long)b * a.H + hh) * a.nsplit);
+      float M = -INFINITY, L = 0.f;
+      f32x4v o = f32x4v{0.f, 0.f, 0.f, 0.f};
+      for (int s0 = 0; s0 < a.nsplit; s0 += 4) {
+        float mv[4], lv[4];
+        f32x4v pv[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          mv[j] = -INFINITY;
+          lv[j] = 0.f;
+          if (s0 + j < a.nsplit) {
+            mv[j] = ld1_sc1(mlr, (row + s0 + j) * 8);
+            lv[j] = ld1_sc1(mlr, (row + s0 + j) * 8 + 4);
+            pv[j] = ld_sc1(por, ((row + s0 + j) * HD + d) * 4);
+          }
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          if (lv[j] <= 0.f) continue;
+          const float mn = fmaxf(M, mv[j]);
+          const float sc = __builtin_amdgcn_exp2f(M - mn), f = __builtin_amdgcn_exp2f(mv[j] - mn);
+          L = L * sc + f * lv[j];
+          o = o * sc + f * pv[j];
+          M = mn;
+        }
+      }
+      const float inv = L > 0.f ? 1.f / L : 0.f;
+      *(uint2*)(a.o + (long)b * a.ldo + (long)hh * HD + d) =
+          make_uint2(pack_bf16x2(o[0] * inv, o[1] * inv), pack_bf16x2(o[2] * inv, o[3] * inv));
+    }
+    return;
+  }
+  const int tasks = G * (HD / 4);  // a thread's four dims of one head
+  // parts pg, pg + groups, ..: four rows on their way at once
+  auto merge = [&](int ii, int pg, int groups, float& M, float& L, f32x4v& o) {
+    const unsigned row = row_of(kvh * G + (ii >> 5)), d = (ii & 31) * 4;
+    M = -INFINITY, L = 0.f;
+    o = f32x4v{0.f, 0.f, 0.f, 0.f};
+    for (int s0 = pg; s0 < nsplit; s0 += 4 * groups) {
       float mv[4], lv[4];
       f32x4v pv[4];
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         mv[j] = -INFINITY;
         lv[j] = 0.f;
-        if (s0 + j < a.nsplit) {
-          mv[j] = ld1_sc1(mlr, (row + s0 + j) * 8);
-          lv[j] = ld1_sc1(mlr, (row + s0 + j) * 8 + 4);
-          pv[j] = ld_sc1(por, ((row + s0 + j) * HD + d) * 4);
+        const int sj = s0 + j * groups;
+        if (sj < nsplit) {
+          mv[j] = ld1_sc1(mlr, (row + sj * next) * 8);
+          lv[j] = ld1_sc1(mlr, (row + sj * next) * 8 + 4);
+          pv[j] = ld_sc1(por, ((row + sj * next) * HD + d) * 4);
         }
       }
 #pragma unroll
@@ -1480,9 +1572,46 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(PIPE ? 2
         M = mn;
       }
     }
+  };
+  auto store = [&](int ii, float L, const f32x4v& o) {
     const float inv = L > 0.f ? 1.f / L : 0.f;
-    *(uint2*)(a.o + (long)b * a.ldo + (long)hh * HD + d) =
+    *(uint2*)(a.o + (long)b * a.ldo + (long)(kvh * G + (ii >> 5)) * HD + (ii & 31) * 4) =
         make_uint2(pack_bf16x2(o[0] * inv, o[1] * inv), pack_bf16x2(o[2] * inv, o[3] * inv));
+  };
+  float M, L;
+  f32x4v o;
+  if (nsplit <= 8) {
+    for (int i = threadIdx.x; i < tasks; i += 64 * W) {
+      merge(i, 0, 1, M, L, o);
+      store(i, L, o);
+    }
+    return;
+  }
+  // many parts by as many groups of threads as there are, then through LDS
+  const int groups = max(1, min(W, 64 * W / tasks));
+  for (int i = threadIdx.x; i < tasks * groups; i += 64 * W) {
+    const int pg = i / tasks, ii = i - pg * tasks;
+    merge(ii, pg, groups, M, L, o);
+    *(f32x4v*)&part[pg][ii >> 5][(ii & 31) * 4] = o;
+    if ((ii & 31) == 0) {
+      mls[pg][ii >> 5][0] = M;
+      mls[pg][ii >> 5][1] = L;
+    }
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < tasks; i += 64 * W) {
+    const int hn = i >> 5;
+    M = -INFINITY, L = 0.f;
+    o = f32x4v{0.f, 0.f, 0.f, 0.f};
+    for (int x = 0; x < groups; ++x) M = fmaxf(M, mls[x][hn][0]);
+    for (int x = 0; x < groups; ++x) {
+      const float l = mls[x][hn][1];
+      if (l <= 0.f) continue;
+      const float f = __builtin_amdgcn_exp2f(mls[x][hn][0] - M);
+      L += f * l;
+      o += f * *(const f32x4v*)&part[x][hn][(i & 31) * 4];
+    }
+    store(i, L, o);
   }
 }
 
@@ -1860,6 +1989,29 @@ KGS_EXPORT int kgs_paged_decode_wg_ex(const void* q, const void* cache, const in
                 : (waves == 8 ? paged_wg<false> : waves == 4 ? paged_wg<false, 4> : waves == 2 ? paged_wg<false, 2> : nullptr);
   if (!fn) return KGS_ERR_ARG;
   hipLaunchKernelGGL(fn, dim3((unsigned)nwg), dim3(64 * waves), 0, s, a);
+  return (int)hipGetLastError();
+}
+
+// The same with parts by the sequences' lengths (paged_wg BAL): at most 128 sequences, 8 (e4m3: 4) waves; po and pml hold
+// B + target rows of H heads.
+KGS_EXPORT int kgs_paged_decode_wg_bal(const void* q, const void* cache, const int* block_tables, const int* ctx_lens, void* o,
+                                       float* po, float* pml, int* cnt, int B, int H, int HKV, int hd, int max_pages, int target,
+                                       int least, long ldq, long ldo, float scale, int kv8, hipStream_t s) {
+  using namespace kgs::dec;
+  if (B <= 0 || B > 128 || H <= 0 || HKV <= 0 || H % HKV || H / HKV > 16 || hd != HD || max_pages <= 0) return KGS_ERR_SHAPE;
+  if (target <= 0 || target > 1 << 16 || least <= 0 || max_pages > 1 << 22) return KGS_ERR_SHAPE;
+  if (ldq < (long)H * HD || ldo < (long)H * HD) return KGS_ERR_SHAPE;
+  if (!al16(q) || !al16(cache) || !al16(o) || ldq % 8 || ldo % 8) return KGS_ERR_ALIGN;
+  if (!po || !pml || !cnt || !al16(po)) return KGS_ERR_ARG;
+  // parts of at most P pages: sum of ceil(pages / P) <= B + total / P <= B + target
+  const int units = B + target;
+  if ((long)units * HKV > 0x7fffffff || (long)units * H * HD * 4 > 0xffffffffL) return KGS_ERR_SHAPE;
+  AttnArgs a{(const unsigned short*)q, (const unsigned short*)cache, block_tables, ctx_lens, (unsigned short*)o, po,
+             pml, cnt, ldq, ldo, B, H, HKV, max_pages, 0, 1, 1, scale * 1.4426950408889634f,
+             nullptr, 0, nullptr, nullptr, nullptr, nullptr, nullptr, target, least, units};
+  auto fn = kv8 ? (B > 64 ? paged_wg<true, 4, true, 2> : paged_wg<true, 4, true, 1>)
+                : (B > 64 ? paged_wg<false, 8, false, 2> : paged_wg<false, 8, false, 1>);
+  hipLaunchKernelGGL(fn, dim3((unsigned)(units * HKV)), dim3(kv8 ? 256 : 512), 0, s, a);
   return (int)hipGetLastError();
 }
 

@@ -139,3 +139,49 @@ def test_few_waves_in_parts(fp8, waves, nsplit):
     assert go(waves) == 0
     assert float((out.float() - D.ref_paged_decode(q, cache, tables, ctx, 16, hkv)).abs().max()) < TOL
     assert go(3) != 0 and go(8 if fp8 else 1) != 0  # no such kernels
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("hkv,group", [(8, 4), (1, 16), (4, 1)])
+@pytest.mark.parametrize("batch,target", [(1, 7), (9, 1), (9, 3), (64, 40), (65, 40), (128, 300)])
+def test_parts_that_follow_the_lengths(batch, target, hkv, group, fp8):
+    """One part each, parts of one round, more than eight of a sequence, empty contexts, both sides of 64 sequences; rows and
+    tables past the batch stay as they are, and tickets end at zero."""
+    from kgs.ops import _lib
+    from kgs.ops import decode as D
+
+    g = torch.Generator(device="cpu").manual_seed(batch)
+    lens = torch.randint(1, 400, (batch,), generator=g).tolist()
+    lens[0], lens[-1] = 2200, 1 if batch > 1 else 2200
+    q, cache, tables, ctx = setup(lens, hkv, group, fp8)
+    if batch > 2:
+        ctx[2] = 0
+    heads = hkv * group
+    want = D.ref_paged_decode(q, cache, tables, ctx.clamp(min=1), heads, hkv)
+    out = torch.full((batch + 1, heads * 128), 7.0, dtype=torch.bfloat16, device=DEV)
+    rows = batch + target
+    po, pml = torch.full(((rows * heads + 1) * 128,), 7.0, device=DEV), torch.full((rows * heads * 2 + 2,), 7.0, device=DEV)
+    cnt = torch.zeros(batch * hkv, dtype=torch.int32, device=DEV)
+    for least in (1, 8, 64):
+        rc = _lib.lib().kgs_paged_decode_wg_bal(q.data_ptr(), cache.data_ptr(), tables.data_ptr(), ctx.data_ptr(), out.data_ptr(),
+                                                po.data_ptr(), pml.data_ptr(), cnt.data_ptr(), batch, heads, hkv, 128, tables.shape[1],
+                                                target, least, q.stride(0), out.stride(0), 128 ** -0.5, int(fp8),
+                                                _lib.stream_handle(q.device))
+        assert rc == 0
+        got = out[:batch].float()
+        if batch > 2:
+            assert bool((got[2] == 0).all())
+            got[2] = want[2]
+        assert float((got - want).abs().max()) < TOL
+        assert bool((out[-1] == 7).all()) and bool((po[-128:] == 7).all()) and bool((pml[-2:] == 7).all()) and not bool(cnt.any())
+
+
+def test_length_rule_has_room_for_its_parts():
+    from kgs.ops.decode import length_parts
+
+    for batch in (1, 2, 3, 31, 32, 64, 128, 129):
+        for kv in (1, 4, 8, 300):
+            for fp8 in (False, True):
+                n = length_parts(batch, kv, 64, 4 if fp8 else 8, fp8)
+                assert (n > 0) == (2 < batch <= 128) and n * kv <= max(384, kv)
+                assert length_parts(batch, kv, 63, 4 if fp8 else 8, fp8) == 0 == length_parts(batch, kv, 64, 2, fp8)

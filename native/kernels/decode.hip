@@ -960,7 +960,7 @@ struct AttnArgs {
   const int* pos;               // [B]
   const int* slot;              // [B] cache slot of the new token (< 0: no write)
   void* cache_w;                // the same layer base as cache, writable
-  // parts by length (paged_wg BAL): units (parts of a sequence) to deal the pages to, a part's least pages, units at most
+  // parts by length (paged_parts): units (parts of a sequence) to deal the pages to, a part's least pages, units at most
   int target, least, units;
 };
 
@@ -1315,12 +1315,12 @@ struct PageRegs<true> {
 };
 
 //
-// BAL: the parts follow the lengths, so that a long context is no longer one workgroup's (100 sequences of 60 to 2800 tokens, 4
+// BAL (paged_parts): the parts follow the lengths, so that a long context is no longer one workgroup's (100 sequences of 60 to 2800 tokens, 4
 // KV heads: 38.1 -> 29.9 us, 70 of 4000 at most 44.9 -> 32.2; the rule is length_parts). All workgroups read all of them (a lane holds BAL of each 64) and cut
 // every sequence into equal parts of at most P pages, P such that `target` parts of P hold
 // them all (at least `least`): unit u of the grid is the u-th such part.
-template <bool KV8, int W = KV8 ? 4 : 8, bool PIPE = KV8, int BAL = 0>
-__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(PIPE ? 2 : 4, PIPE ? 2 : 4))) void paged_wg(AttnArgs a) {
+template <bool KV8, int W, bool PIPE, int BAL>
+__device__ __forceinline__ void paged_waves(const AttnArgs& a) {
   constexpr int LDO = HD + 4;  // a row of partial outputs: 16 heads' rows start on different banks
   __shared__ __attribute__((aligned(16))) float part[W][16][LDO];
   __shared__ float mls[W][16][2];
@@ -1613,6 +1613,16 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(PIPE ? 2
     }
     store(i, L, o);
   }
+}
+
+template <bool KV8, int W = KV8 ? 4 : 8, bool PIPE = KV8>
+__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(PIPE ? 2 : 4, PIPE ? 2 : 4))) void paged_wg(AttnArgs a) {
+  paged_waves<KV8, W, PIPE, 0>(a);
+}
+
+template <bool KV8, int BAL>
+__global__ __launch_bounds__(KV8 ? 256 : 512) __attribute__((amdgpu_waves_per_eu(KV8 ? 2 : 4, KV8 ? 2 : 4))) void paged_parts(AttnArgs a) {
+  paged_waves<KV8, KV8 ? 4 : 8, KV8, BAL>(a);
 }
 
 // merge nsplit partials (m in log2 units, l, unnormalised O) of one (b, h):
@@ -1992,7 +2002,7 @@ KGS_EXPORT int kgs_paged_decode_wg_ex(const void* q, const void* cache, const in
   return (int)hipGetLastError();
 }
 
-// The same with parts by the sequences' lengths (paged_wg BAL): at most 128 sequences, 8 (e4m3: 4) waves; po and pml hold
+// The same with parts by the sequences' lengths (paged_parts): at most 128 sequences, 8 (e4m3: 4) waves; po and pml hold
 // B + target rows of H heads.
 KGS_EXPORT int kgs_paged_decode_wg_bal(const void* q, const void* cache, const int* block_tables, const int* ctx_lens, void* o,
                                        float* po, float* pml, int* cnt, int B, int H, int HKV, int hd, int max_pages, int target,
@@ -2009,8 +2019,8 @@ KGS_EXPORT int kgs_paged_decode_wg_bal(const void* q, const void* cache, const i
   AttnArgs a{(const unsigned short*)q, (const unsigned short*)cache, block_tables, ctx_lens, (unsigned short*)o, po,
              pml, cnt, ldq, ldo, B, H, HKV, max_pages, 0, 1, 1, scale * 1.4426950408889634f,
              nullptr, 0, nullptr, nullptr, nullptr, nullptr, nullptr, target, least, units};
-  auto fn = kv8 ? (B > 64 ? paged_wg<true, 4, true, 2> : paged_wg<true, 4, true, 1>)
-                : (B > 64 ? paged_wg<false, 8, false, 2> : paged_wg<false, 8, false, 1>);
+  auto fn = kv8 ? (B > 64 ? paged_parts<true, 2> : paged_parts<true, 1>)
+                : (B > 64 ? paged_parts<false, 2> : paged_parts<false, 1>);
   hipLaunchKernelGGL(fn, dim3((unsigned)(units * HKV)), dim3(kv8 ? 256 : 512), 0, s, a);
   return (int)hipGetLastError();
 }

@@ -160,6 +160,16 @@ def test_decode_attention_by_workgroups_fits_its_waves(builds):
         assert r["LDS Size"] <= 80 * 1024, (name, r)
 
 
+def test_decode_attention_in_parts_by_length_fits_its_waves(builds):
+    """The same occupancies as paged_wg's."""
+    wg = {n: r for n, r in builds["decode.hip"].result()[0].items() if "paged_partsI" in n}
+    assert len(wg) == 2 * 2, sorted(wg)
+    for name, r in wg.items():
+        assert r["VGPRs Spill"] == 0 and r["SGPRs Spill"] == 0, (name, r)
+        assert r["VGPRs"] + r["AGPRs"] <= (256 if "paged_partsILb1" in name else 128), (name, r)
+        assert r["LDS Size"] <= 80 * 1024, (name, r)
+
+
 def test_skinny_gemms_do_not_spill(builds):
     res = builds["decode.hip"].result()[0]
     skinny = {n: r for n, r in res.items() if "3dec6skinnyI" in n}

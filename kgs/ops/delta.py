@@ -58,7 +58,7 @@ class RaggedSeqs:
     """Sequences of a call (int32, device): each row's sequence, and per sequence
     its first row, rows, first position and state slot. ``chunks`` / ``cseqs`` (see
     :func:`chunk_plan`): the sequences that go by chunks; ``step_rows`` /
-    ``step_seqs``: rows and numbers of the others, None when that is all of them."""
+    ``step_seqs``: rows and numbers of the others, None when that is all of them. ``longest`` picks a kernel only."""
     row_seq: torch.Tensor
     row0: torch.Tensor
     n: torch.Tensor
@@ -68,6 +68,7 @@ class RaggedSeqs:
     cseqs: torch.Tensor | None = None
     step_rows: torch.Tensor | None = None
     step_seqs: torch.Tensor | None = None
+    longest: int = 0  # chunks of the longest sequence that goes by chunks, 0: not known
 
 
 def chunk_plan(row0, n, pos0, slot) -> dict:
@@ -123,8 +124,9 @@ def delta_forward(z: torch.Tensor, offs: tuple[int, int, int, int], a2: torch.Te
         state.conv.data_ptr(), opt(seqs.step_rows), opt(seqs.step_seqs), opt(seqs.chunks), opt(seqs.cseqs), *ptr(work, 6))
     pairs = not (K % 2 or V % 2 or z.stride(0) % 2 or a2.stride(0) % 2 or any(x % 2 for x in offs[:3]) or
                  z.data_ptr() % 4 or a2.data_ptr() % 4)
-    dims = (ctypes.c_long * 20)(z.stride(0), a2.stride(0), *offs, sh.taps, G, H, K, V, sh.kp, B, T,
-                                int(z.dtype == torch.float32), *nstep, nc, seqs.cseqs.shape[0] if nc else 0, int(pairs))
+    dims = (ctypes.c_long * 21)(z.stride(0), a2.stride(0), *offs, sh.taps, G, H, K, V, sh.kp, B, T,
+                                int(z.dtype == torch.float32), *nstep, nc, seqs.cseqs.shape[0] if nc else 0, int(pairs),
+                                seqs.longest)
     _lib.check(_lib.lib().kgs_delta_forward(ptrs, dims, _lib.stream_handle(dev)), f"delta_forward[{T}x{H}x{K}x{V}]")
     return o
 

@@ -191,14 +191,16 @@ class RaggedModel:
         row_seq = np.repeat(order, n[order])
         pos = pos0[row_seq] + np.arange(len(tokens)) - row0[row_seq]
         refs = [pk.add(a) for a in (tokens, slots, row_seq, row0, n, pos0, slot, bt, logit_rows, pos)]
-        split = {k: pk.add(v) for k, v in chunk_plan(row0, n, pos0, slot).items()} if self.delta_chunks else {}
+        plan = chunk_plan(row0, n, pos0, slot) if self.delta_chunks else {}
+        split = {k: pk.add(v) for k, v in plan.items()}
+        longest = int(plan["cseqs"][0][2]) if plan else 0
         host = {g: g.host_plan(pk, row0, n, pos0, bt, row_seq, pos, refs) for g in self.geometries}
         get = pk.send()
         d = [get(r) for r in refs]
         plans = {g: build(get) for g, build in host.items()}
         return Batch(dev_tokens.to(torch.int32).contiguous() if dev_tokens is not None else d[0], d[1],
-                     RaggedSeqs(d[2], d[3], d[4], d[5], d[6], **{k: get(r) for k, r in split.items()}), plans, d[8].long(),
-                     d[9])
+                     RaggedSeqs(d[2], d[3], d[4], d[5], d[6], **{k: get(r) for k, r in split.items()}, longest=longest), plans,
+                     d[8].long(), d[9])
 
     # ------------------------------------------------------------------- decode
     def _fixed_seqs(self, nb: int) -> dict:

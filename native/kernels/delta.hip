@@ -71,6 +71,7 @@ struct Args {
   const int4* chunks;  // per chunk (first row, rows, sequence, -), (sequence's first row, position, slot, -)
   const int4* cseqs;   // (sequence, first chunk, chunks, first row)
   int nchunks, ncseqs;
+  long longest;        // the longest chunked sequence's chunks, 0: not known
   float *cW, *cQ, *cK, *cE, *cU, *cP;  // per (chunk, head): [16][KP] x 2, [KP][16], [KP], [16][V], [16][16]
 };
 
@@ -593,9 +594,11 @@ __global__ __launch_bounds__(256) void chunk_scan(Args a) {
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l16 = lane & 15, g = lane >> 4;
   const int KP = a.KP, V = a.V, H = a.H, nslab = (V + 16 * NS - 1) / (16 * NS), ntile = KP / 16;
-  const int lid = xcd_remap(blockIdx.x, gridDim.x);  // a head's slabs share an XCD's L2
-  // (divisions run on the vector unit: back to scalars, so that bases stay uniform)
-  const int sh = __builtin_amdgcn_readfirstlane(lid / nslab), slab = __builtin_amdgcn_readfirstlane(lid - sh * nslab);
+  // A head's slabs share an XCD's L2; a sequence's heads go round the XCDs, so that each has as many of the longest chains
+  // (which come first) as the others. (Divisions run on the vector unit: back to scalars, so that bases stay uniform.)
+  const int loc = blockIdx.x >> 3, pos = __builtin_amdgcn_readfirstlane(loc / nslab);
+  const int sh = pos * 8 + (blockIdx.x & 7), slab = loc - pos * nslab;
+  if (sh >= a.ncseqs * H) return;
   const int si = __builtin_amdgcn_readfirstlane(sh / H), h = sh - si * H;
   const int4 sq = a.cseqs[si];  // sequence, first chunk, chunks, first row
   const int b = sq.x, n = a.n[b];
@@ -779,7 +782,7 @@ __global__ __launch_bounds__(256) void out(OutArgs a) {
 
 template <typename T, int NS>
 static void run_chunk_scan(const Args& a, hipStream_t s) {
-  const dim3 grid((unsigned)((a.V + 16 * NS - 1) / (16 * NS) * a.H * a.ncseqs));
+  const dim3 grid((unsigned)((a.V + 16 * NS - 1) / (16 * NS) * ((a.H * a.ncseqs + 7) / 8) * 8));  // whole rounds of the XCDs
   switch ((a.KP + 63) / 64) {
     case 1: hipLaunchKernelGGL((chunk_scan<T, 1, NS>), grid, dim3(256), 0, s, a); break;
     case 2: hipLaunchKernelGGL((chunk_scan<T, 2, NS>), grid, dim3(256), 0, s, a); break;
@@ -816,8 +819,13 @@ static hipError_t run(const Args& a, hipStream_t s) {
       if (e != hipSuccess) return e;
     }
     hipLaunchKernelGGL(prep_k, dim3((unsigned)(a.nchunks * a.H)), dim3(256), lds, s, a);
-    const long wide = (long)((a.V + 31) / 32) * a.H * a.ncseqs;
-    if (a.V > 16 && wide >= 256) run_chunk_scan<T, 2>(a, s);
+    // Slabs of 32 columns read the chunks' operands half as often; of 16 they halve a chain's step, which is what counts where
+    // there are few workgroups or the longest chain (a.longest chunks, 0: unknown) is above a CU's mean share of all
+    // chunks. us, 32 / 16 columns, longest chain over share: 6 prompts of 3580 tokens 170 / 138 (1.35), 7 of 3140 153 / 119
+    // (1.56), 8 of 3060 116 / 109 (1.06); 6 of 690 29.8 / 34.6 (1.02), 10 of 3070 92 / 111 (0.79), 32 heads: 4 of 1950 108 / 127 (0.75)
+    const long slabs = (a.V + 31) / 32, wide = slabs * a.H * a.ncseqs;
+    const bool chain = a.longest * 256.0 > 1.05 * a.nchunks * a.H * slabs;
+    if (a.V > 16 && wide >= 256 && !chain) run_chunk_scan<T, 2>(a, s);
     else run_chunk_scan<T, 1>(a, s);
   }
   return hipGetLastError();
@@ -834,7 +842,7 @@ static hipError_t run(const Args& a, bool pairs, hipStream_t s) {
 
 // ptrs (29 device pointers): z a2 cw A_log dt_bias row_seq row0 n pos0 slot q k v lg beta qk o S conv
 //   rows seqs chunks cseqs cW cQ cK cE cU cP
-// dims (20): ldz lda oq ok ov ob taps G H K V KP B T f32 nrows nseqs nchunks ncseqs, even (channel pairs aligned)
+// dims (21): ldz lda oq ok ov ob taps G H K V KP B T f32 nrows nseqs nchunks ncseqs, even (channel pairs aligned), longest
 KGS_EXPORT int kgs_delta_forward(const void* const* ptrs, const long* dims, hipStream_t s) {
   using namespace kgs::delta;
   Args a{};
@@ -886,6 +894,7 @@ KGS_EXPORT int kgs_delta_forward(const void* const* ptrs, const long* dims, hipS
   a.nseqs = (int)dims[16];
   a.nchunks = (int)dims[17];
   a.ncseqs = (int)dims[18];
+  a.longest = dims[20];
   a.C = 2 * a.G * a.K + a.H * a.V;
   if (a.taps < 1 || a.G < 1 || a.H < 1 || a.H % a.G || a.K < 1 || a.V < 1 || a.B < 1 || a.T < 1 || a.KP % 32 ||
       a.KP < a.K || a.KP > 256 || a.G > 65535 || a.H > 65535 || a.B > 65535)

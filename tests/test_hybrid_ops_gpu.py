@@ -327,6 +327,33 @@ def test_delta_ragged_batches_and_reused_slots(shape):
         close(o[lo:lo + n], c.ref(lo, n)[0], 3e-5)
 
 
+def test_delta_many_chunked_sequences_by_either_slab():
+    """Enough sequences for slabs of 32 columns, heads times sequences no multiple of the XCDs; where the longest is known to be
+    a chain of its own, slabs of 16: the same bits."""
+    import dataclasses
+
+    from kgs.ops import delta as Dl
+
+    n = [40, 65, 16, 33, 17, 48, 90, 20, 31, 50]
+    got = []
+    for longest in (0, 1, 1000):
+        c = DeltaCase(7, 7, 128, 100, 4, sum(n), slots=len(n) + 1)
+        whole = Dl.RaggedSeqs
+        try:
+            Dl.RaggedSeqs = lambda *a, **k: dataclasses.replace(whole(*a, **k), longest=longest)
+            o = c.run([[(sum(n[:i]), m, 0, 1 + i) for i, m in enumerate(n)]])
+        finally:
+            Dl.RaggedSeqs = whole
+        got.append((o, c.state.S.clone()))
+    for o, S in got[1:]:
+        assert torch.equal(o, got[0][0]) and torch.equal(S, got[0][1])
+    for i in (0, 1, 6, 9):
+        a = sum(n[:i])
+        ref, S = c.ref(a, n[i])
+        close(got[0][0][a:a + n[i]], ref, 3e-5)
+        close(got[0][1][1 + i, :, :, :128].transpose(1, 2), S, 3e-5)
+
+
 def test_delta_decay_extremes():
     """Channels that forget at once beside channels that keep everything for long."""
     c = DeltaCase(2, 1, 64, 32, 4, 600)

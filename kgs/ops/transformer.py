@@ -18,6 +18,7 @@ missing -- there is no silent PyTorch fallback.
 """
 from __future__ import annotations
 
+import ctypes
 import math
 
 import torch
@@ -54,6 +55,58 @@ def add_rmsnorm(x: torch.Tensor, d: torch.Tensor | None, w: torch.Tensor, eps: f
                                          x.stride(0), y.stride(0), float(eps), _lib.stream_handle(x.device))
     _lib.check(rc, "add_rmsnorm")
     return y
+
+
+def embeds(table: torch.Tensor) -> bool:
+    """Whether :func:`embed_rows` reads this embedding table."""
+    return (table.is_cuda and table.dtype == torch.bfloat16 and table.dim() == 2 and table.stride(1) == 1 and table.stride(0) % 8 == 0
+            and table.data_ptr() % 16 == 0 and table.shape[0] > 0 and 0 < table.shape[1] <= 8192 and table.shape[1] % 512 == 0)
+
+
+def embed_rows(table: torch.Tensor, tokens: torch.Tensor, w: torch.Tensor | None = None, eps: float = 1e-5, keep: torch.Tensor | None = None,
+               squares: torch.Tensor | None = None, positions: torch.Tensor | None = None, slots: torch.Tensor | None = None,
+               zeros=()) -> tuple:
+    """The rows ``table[tokens]`` that a step starts from, with what its first layer takes, in one launch: ``(x, y, positions,
+    slots)`` -- with ``w`` ``y = rmsnorm(x) * w`` (else None), as :func:`add_rmsnorm`; ``keep`` (int32): of those rows of ``tokens``,
+    ``positions`` and ``slots`` (int32 each) only. ``squares`` (fp32 ``[rows]``) is given the rows' sums of squares, the tensors ``zeros``
+    (two at most, contiguous, whole 4-byte words) are cleared. Numbers below zero count from the table's end, a row of
+    one that is not in the table is NaN."""
+    if not embeds(table):
+        raise ValueError("table must be bf16 rows of 16-byte chunks on the GPU, a multiple of 512 up to 8192 columns")
+    tokens = tokens.reshape(-1)
+    if tokens.dtype != torch.int32:
+        tokens = tokens.clamp(-2 ** 31, 2 ** 31 - 1).to(torch.int32)
+    tokens = tokens.contiguous()
+    dev, cols = table.device, table.shape[1]
+    rows = tokens.numel() if keep is None else keep.numel()
+    given = [t for t in (keep, positions, slots) if t is not None]
+    if tokens.device != dev or any(t.dtype != torch.int32 or t.device != dev or not t.is_contiguous() for t in given) or \
+            any(t.numel() != tokens.numel() for t in (positions, slots) if t is not None):
+        raise ValueError("tokens, keep, positions and slots must be int32 vectors on the table's GPU, the last two as long as tokens")
+    if w is not None and (w.shape != (cols,) or w.dtype != torch.bfloat16 or not w.is_contiguous() or w.device != dev):
+        raise ValueError("w must be a contiguous bf16 vector of length cols")
+    if squares is not None and (squares.dtype != torch.float32 or squares.shape != (rows,) or not squares.is_contiguous()):
+        raise ValueError("squares must be a contiguous fp32 vector, one a row")
+    words = [t.numel() * t.element_size() // 4 for t in zeros]
+    if len(words) > 2 or any(not t.is_contiguous() or t.device != dev or t.element_size() % 4 for t in zeros):
+        raise ValueError("zeros: at most two contiguous tensors of whole words on the table's GPU")
+    x = torch.empty((rows, cols), dtype=torch.bfloat16, device=dev)
+    y = None if w is None else torch.empty_like(x)
+    if keep is None or rows == 0:
+        pos, slot = (None if t is None else t if keep is None else t[:0] for t in (positions, slots))
+    else:
+        pos, slot = (None if t is None else torch.empty(rows, dtype=torch.int32, device=dev) for t in (positions, slots))
+    if rows == 0:
+        for t in zeros:
+            t.zero_()
+        return x, y, pos, slot
+    moved = keep is not None
+    ptrs = (ctypes.c_void_p * 13)(*(None if t is None else t.data_ptr() for t in (
+        table, tokens, keep, x, y, w, squares, positions if moved else None, slots if moved else None, pos if moved else None,
+        slot if moved else None, *zeros, *[None] * (2 - len(words)))))
+    dims = (ctypes.c_long * 8)(rows, cols, table.shape[0], table.stride(0), cols, cols, *words, *[0] * (2 - len(words)))
+    _lib.check(_lib.lib().kgs_embed_rows_bf16(ptrs, dims, float(eps), _lib.stream_handle(dev)), f"embed_rows[{rows}x{cols}]")
+    return x, y, pos, slot
 
 
 def splitk_add_rmsnorm(partials: torch.Tensor, x: torch.Tensor, w: torch.Tensor, eps: float = 1e-5,

@@ -59,9 +59,9 @@ def gate_up_panel_widths(n: int, k: int) -> set:
 
 
 class _PromptRows:
-    """Rows of a step's layers: ``n`` of them, ``last`` (int64) those whose logits are wanted, attention
+    """Rows of a step's layers: ``n`` of them, ``last`` (int32) those whose logits are wanted, attention
     ``items`` (and ``merges``, ``slots`` of their parts) with the gathered contexts ``past`` ``(first row, end, tokens, portion)``, and, where
-    the padding was dropped, ``keep`` (int64: the given rows that stay) and ``rows`` (int32: each
+    the padding was dropped, ``keep`` (int32: the given rows that stay) and ``rows`` (int32: each
     given row's number, -1 for padding)."""
 
     __slots__ = ("n", "past", "items", "merges", "slots", "last", "rows", "keep")
@@ -349,10 +349,7 @@ class ServingModel:
         if self._fused_prompts(sum(n for _, n, _, _ in seqs), len(seqs)):
             return self._prefill_fused(tokens, positions, slots, seqs)
         plan = self._prompt_rows(seqs, tokens.numel(), tokens.device)
-        if plan.keep is not None:
-            tokens = tokens.reshape(-1)[plan.keep]
-        x = self.embed[tokens.long()].reshape(-1, h).contiguous()
-        y = self._norm(x, None, self.ln1[0])
+        x, y = self._start(tokens, plan.keep)
         T.op("prefill embed+norm")
         m = x.shape[0]
         # few rows: the decode step's split tiles, whose sums the rotation, norms and gate take (one
@@ -389,8 +386,7 @@ class ServingModel:
             else:
                 y = self._proj_add_norm(act, i, "down", x, nxt)
             T.op(f"prefill L{i} down+norm")
-        yl = y[plan.last].contiguous()
-        out = self._proj(yl, None, "lm", True)
+        out = self._proj(y.index_select(0, plan.last), None, "lm", True)
         T.op("prefill lm_head")
         return out
 
@@ -408,19 +404,18 @@ class ServingModel:
         5 launches a layer besides the attention's (one prompt of 20 tokens, hidden 2048: 481 us by the
         split tiles, 403 so; of 30, hidden 4096: 630 and 546)."""
         plan = self._prompt_rows(seqs, tokens.numel(), tokens.device, drop=True, force=True)
-        tokens, positions, slots = (t.reshape(-1)[plan.keep] for t in (tokens, positions, slots))
         c = self.cfg
-        # counters of the step's own: nothing is shared with a decode step on another stream
+        # counters of the step's own, cleared with its first launch: nothing is shared with a decode step on another stream
         most = max(w.n for w in (*self.packed[0].values(), self.packed_lm))
-        count = torch.zeros(most // 16, dtype=torch.int32, device=tokens.device)
+        count = torch.empty(most // 16, dtype=torch.int32, device=tokens.device)
         from kgs.ops.transformer import attention_blocks
 
         def attend(qkv, i):
             a = torch.empty((plan.n, c.heads * c.head_dim), dtype=torch.bfloat16, device=qkv.device)
             return attention_blocks(qkv, *self._kv(qkv), plan.items, c.heads, c.kv_heads, a, merges=plan.merges, slots=plan.slots)
 
-        x, ss = self._fused_layers(tokens, positions, slots, attend, "prefill", count, exact=True)
-        out = D.skinny_gemm(x[plan.last], self.packed_lm, rms=ss.index_select(1, plan.last), eps=c.eps, counters=count)
+        x, ss = self._fused_layers(tokens, positions, slots, attend, "prefill", count, exact=True, keep=plan.keep)
+        out = D.skinny_gemm(x.index_select(0, plan.last), self.packed_lm, rms=ss.index_select(1, plan.last), eps=c.eps, counters=count)
         T.op("prefill-fused lm_head")
         return out
 
@@ -433,9 +428,8 @@ class ServingModel:
         c = self.cfg
         plan = self._prompt_rows([(int(s), int(n), int(p), 0) for s, n, p in zip(seq_starts, seq_lens, padded_lens)],
                                  tokens.numel(), tokens.device, drop=False)
-        x = self.embed[tokens.long()].reshape(-1, c.hidden).contiguous()
+        x, y = self._start(tokens, norm=False)
         y8, ys = add_rmsnorm_fp8(x, None, self.ln1[0], c.eps)
-        y = None
         for i in range(c.layers):
             F = self.prefill_f8[i]
             qkv = F["qkv"].forward_q(y8, ys)
@@ -448,7 +442,7 @@ class ServingModel:
                 y8, ys = add_rmsnorm_fp8(x, d, self.ln1[i + 1], c.eps)
             else:
                 y = add_rmsnorm(x, d, self.norm, c.eps)
-        return self._proj(y[plan.last].contiguous(), None, "lm", True)
+        return self._proj(y.index_select(0, plan.last), None, "lm", True)
 
     def _prompt_rows(self, seqs, total: int, device, drop: bool = True, tail: int = 0, wanted=None,
                      force: bool = False) -> "_PromptRows":
@@ -507,9 +501,9 @@ class ServingModel:
             out.items = t[:items.size].view(-1, 4)
             if merges is not None:
                 out.merges, out.slots = t[items.size:n].view(-1, 4), slots
-        out.last = t[n:n + sizes[0]].long()
+        out.last = t[n:n + sizes[0]]
         if drop:
-            out.rows, out.keep = t[n + sizes[0]:n + sizes[0] + total], t[n + sizes[0] + total:].long()
+            out.rows, out.keep = t[n + sizes[0]:n + sizes[0] + total], t[n + sizes[0] + total:]
         return out
 
     def _kv(self, qkv):
@@ -570,8 +564,6 @@ class ServingModel:
         f8 = self.prefill_f8 is not None and n_pf > 0  # W8A8 projections for the whole mixed step
         plan = self._prompt_rows([ch[:4] for ch in chunks], tokens.numel(), tokens.device, drop=not f8, tail=nd,
                                  wanted=[bool(ch[5]) for ch in chunks])
-        if plan.keep is not None:
-            tokens = tokens.reshape(-1)[plan.keep]
         n_pf = plan.n - nd  # prompt rows of the layers
         k2 = v2 = None
         if plan.items is not None:
@@ -579,13 +571,11 @@ class ServingModel:
 
             if plan.past:
                 k2, v2 = torch.empty((2, plan.past[-1][1], c.kv_heads * hd), dtype=torch.bfloat16, device=tokens.device)
-        x = self.embed[tokens.long()].reshape(-1, c.hidden).contiguous()
+        x, y = self._start(tokens, plan.keep, norm=not f8)
         if f8:
             from kgs.ops.transformer import add_rmsnorm_fp8, quantize_rows_fp8, silu_mul_fp8
 
             y8, ys = add_rmsnorm_fp8(x, None, self.ln1[0], c.eps)
-        else:
-            y = self._norm(x, None, self.ln1[0])
         for i in range(c.layers):
             qkv = self.prefill_f8[i]["qkv"].forward_q(y8, ys) if f8 else self._proj(y, i, "qkv", False)
             self._rope_cache(qkv, i, positions, slots, plan.rows)
@@ -625,8 +615,7 @@ class ServingModel:
             y = self._proj_add_norm(act, i, "down", x, nxt)
         if plan.last.numel() == 0:
             return torch.empty((0, c.vocab), dtype=torch.bfloat16, device=x.device)
-        yl = y[plan.last].contiguous()
-        return self._proj(yl, None, "lm", True)
+        return self._proj(y.index_select(0, plan.last), None, "lm", True)
 
     def _chunk_attention(self, blk, layer, n, p, ctx0, pages):
         """The plain backend's causal attention of one prompt chunk (rows = positions ctx0 ..
@@ -651,8 +640,7 @@ class ServingModel:
         c = self.cfg
         if self.backend == "kgs" and tokens.shape[0] <= self.fused_max_batch:
             return self._decode_fused(tokens, positions, slots, block_tables, ctx_lens, pages_per_split)
-        x = self.embed[tokens.long()].reshape(-1, c.hidden).contiguous()
-        y = self._norm(x, None, self.ln1[0])
+        x, y = self._start(tokens)
         m = x.shape[0]
         rq, ro, rd = (self._splitk_route(m, 0, n) for n in ("qkv", "o", "down"))  # same shapes in every layer
         rg = self._swiglu_route(m)
@@ -724,18 +712,43 @@ class ServingModel:
         T.op("decode-fused lm_head")
         return out
 
-    def _fused_layers(self, tokens, positions, slots, attend, kind: str, counters, exact: bool):
+    def _start(self, tokens, keep=None, norm: bool = True):
+        """The residual rows of a step (of the rows ``keep`` of ``tokens``) and, with ``norm``, their norm for the first layer."""
+        from kgs.ops.transformer import embed_rows, embeds
+
+        if self.backend == "kgs" and embeds(self.embed):
+            return embed_rows(self.embed, tokens, self.ln1[0] if norm else None, self.cfg.eps, keep)[:2]
+        tokens = tokens.reshape(-1) if keep is None else tokens.reshape(-1)[keep.long()]
+        x = self.embed[tokens.long()].reshape(-1, self.cfg.hidden).contiguous()
+        return x, self._norm(x, None, self.ln1[0]) if norm else None
+
+    def _fused_layers(self, tokens, positions, slots, attend, kind: str, counters, exact: bool, keep=None):
         """The residual rows after all layers and their sums of squares; ``attend(qkv, layer)`` is the
         attention of the rotated rows, whose keys and values are in the cache. ``exact``: statistics whose
-        bits do not depend on the order in which workgroups arrive, so that equal steps give equal bits."""
+        bits do not depend on the order in which workgroups arrive, so that equal steps give equal bits. ``keep``
+        (int32): of these rows of ``tokens``, ``positions`` and ``slots`` only. ``counters``: the step's own, cleared here."""
+        from kgs.ops.transformer import embed_rows, embeds
+
         c = self.cfg
         eps = c.eps
-        x = self.embed[tokens.long()].reshape(-1, c.hidden).contiguous()  # residual stream
-        ss_b = ss = x.float().pow(2).sum(-1)  # statistic for layer 0's qkv
+        m, dev = (tokens if keep is None else keep).numel(), tokens.device
+        ss = torch.empty(m, dtype=torch.float32, device=dev)  # statistic for layer 0's qkv
         if exact:
-            ss_a, ss_b = torch.zeros((2, D.SUM_WORDS, x.shape[0]), dtype=torch.int64, device=x.device)
+            zero = stats = torch.empty((2, D.SUM_WORDS, m), dtype=torch.int64, device=dev)
+            ss_a, ss_b = stats
         else:
-            ss_a = torch.zeros_like(ss)
+            zero = ss_a = torch.empty_like(ss)
+            ss_b = ss
+        clear = (zero,) if counters is None else (zero, counters)
+        if embeds(self.embed):
+            x, _, positions, slots = embed_rows(self.embed, tokens, None, eps, keep, ss, positions, slots, clear)
+        else:
+            if keep is not None:
+                tokens, positions, slots = (t.reshape(-1)[keep.long()] for t in (tokens, positions, slots))
+            x = self.embed[tokens.long()].reshape(-1, c.hidden).contiguous()  # residual stream
+            ss.copy_(x.float().pow(2).sum(-1))
+            for t in clear:
+                t.zero_()
         for i in range(c.layers):
             P = self.packed[i]
             if P["qkv"].rope:

@@ -45,6 +45,80 @@ __device__ __forceinline__ uint2 to_e4m3x8(const float* v) {
   return make_uint2(lo, hi);
 }
 
+// A step's rows from the embedding table, with all that its first layer takes: row t is table[tokens[keep ? keep[t] : t]] (a
+// negative number counts from the end; NaN where there is no such row), stored to x; rmsnorm of it times w to y; its sum of
+// squares to ss; positions and slots of the kept rows; and zeros into up to two buffers (statistics, tickets) --
+// each null where not wanted. One wave per row as add_rmsnorm, whose rounding y has. One launch for up to ten of torch's, each 2.5
+// to 5 us on the GPU in a replayed graph and 6 to 10 for the host.
+struct EmbedArgs {
+  const unsigned short* table;
+  const int *tokens, *keep;
+  unsigned short *x, *y;
+  const unsigned short* w;
+  float* ss;
+  const int *pos, *slot;
+  int *pos_out, *slot_out;
+  int* zero[2];
+  long nzero[2];
+  long ldt, ldx, ldy;
+  int rows, vocab;
+  float eps;
+};
+template <int NC>
+__global__ __launch_bounds__(256) void embed_rows(EmbedArgs a) {
+  const long id = (long)blockIdx.x * 256 + threadIdx.x;
+#pragma unroll
+  for (int z = 0; z < 2; ++z)
+    for (long i = id; i < a.nzero[z]; i += (long)gridDim.x * 256) a.zero[z][i] = 0;
+  const int lane = threadIdx.x & 63;
+  const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (row >= a.rows) return;
+  const int from = a.keep ? a.keep[row] : row;
+  int tok = a.tokens[from];
+  if (tok < 0) tok += a.vocab;
+  const bool in = tok >= 0 && tok < a.vocab;
+  const bf16x8* src = (const bf16x8*)(a.table + (long)(in ? tok : 0) * a.ldt);
+  if (lane == 0) {
+    if (a.pos_out) a.pos_out[row] = a.pos[from];
+    if (a.slot_out) a.slot_out[row] = a.slot[from];
+  }
+  bf16x8 xv[NC];
+#pragma unroll
+  for (int j = 0; j < NC; ++j) xv[j] = src[lane + 64 * j];
+  if (!in) {
+#pragma unroll
+    for (int j = 0; j < NC; ++j)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) xv[j][e] = 0x7fc0;
+  }
+  bf16x8* xw = (bf16x8*)(a.x + row * a.ldx);
+  float v[NC][8], ss = 0.f;
+#pragma unroll
+  for (int j = 0; j < NC; ++j) {
+    xw[lane + 64 * j] = xv[j];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      v[j][e] = bf2f((unsigned short)xv[j][e]);
+      ss += v[j][e] * v[j][e];
+    }
+  }
+  if (!a.y && !a.ss) return;
+  ss = wave_sum(ss);
+  if (a.ss && lane == 0) a.ss[row] = ss;
+  if (!a.y) return;
+  const float r = rsqrtf(ss / (float)(NC * 512) + a.eps);
+  const bf16x8* wr = (const bf16x8*)a.w;
+  bf16x8* yw = (bf16x8*)(a.y + row * a.ldy);
+#pragma unroll
+  for (int j = 0; j < NC; ++j) {
+    const bf16x8 wv = wr[lane + 64 * j];
+    bf16x8 o;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) o[e] = (short)f2bf(v[j][e] * r * bf2f((unsigned short)wv[e]));
+    yw[lane + 64 * j] = o;
+  }
+}
+
 // One wave per row; lane owns 16-B chunks lane + 64*j (j < NC) -- a wave reads
 // 1 KB contiguous per j. cols == 512 * NC.
 // Q8: y is written as e4m3 bytes with a per-row scale ys[row] = amax/448
@@ -454,6 +528,34 @@ KGS_EXPORT int kgs_splitk_add_rmsnorm_bf16(const float* P, int nslice, void* x, 
   }
 #undef KGS_SARN_NJ
 #undef KGS_SARN
+  return (int)hipGetLastError();
+}
+
+// ptrs (13): table tokens keep x y w ss pos slot pos_out slot_out zero0 zero1, keep (int32), y with w, ss, pos with pos_out, slot with
+// slot_out and the zeros null where not wanted; dims (8): rows cols vocab ldt ldx ldy, 4-byte words of zero0 and zero1.
+KGS_EXPORT int kgs_embed_rows_bf16(void* const* ptrs, const long* dims, float eps, hipStream_t s) {
+  using namespace kgs::tfm;
+  const long rows = dims[0], cols = dims[1], vocab = dims[2];
+  EmbedArgs a{(const unsigned short*)ptrs[0], (const int*)ptrs[1], (const int*)ptrs[2], (unsigned short*)ptrs[3],
+              (unsigned short*)ptrs[4], (const unsigned short*)ptrs[5], (float*)ptrs[6], (const int*)ptrs[7], (const int*)ptrs[8],
+              (int*)ptrs[9], (int*)ptrs[10], {(int*)ptrs[11], (int*)ptrs[12]}, {dims[6], dims[7]}, dims[3], dims[4], dims[5],
+              (int)rows, (int)vocab, eps};
+  if (rows < 0 || rows > 0x7ffffff0 || cols <= 0 || cols % 512 || cols > 8192 || vocab <= 0 || vocab > 0x7fffffff) return KGS_ERR_SHAPE;
+  if (a.ldt < cols || a.ldx < cols || (a.y && a.ldy < cols) || a.nzero[0] < 0 || a.nzero[1] < 0) return KGS_ERR_SHAPE;
+  if (!al16(a.table) || !al16(a.x) || !al16(a.y) || !al16(a.w) || a.ldt % 8 || a.ldx % 8 || a.ldy % 8) return KGS_ERR_ALIGN;
+  if (!a.table || !a.tokens || !a.x || (a.y && !a.w) || (a.pos_out && !a.pos) || (a.slot_out && !a.slot) ||
+      (a.nzero[0] && !a.zero[0]) || (a.nzero[1] && !a.zero[1]))
+    return KGS_ERR_ARG;
+  if (rows == 0) return 0;
+  const dim3 g((unsigned)((rows + 3) / 4)), b(256);
+  switch (cols / 512) {
+#define KGS_NC(n) \
+  case n: hipLaunchKernelGGL(embed_rows<n>, g, b, 0, s, a); break;
+    KGS_NC(1) KGS_NC(2) KGS_NC(3) KGS_NC(4) KGS_NC(5) KGS_NC(6) KGS_NC(7) KGS_NC(8)
+    KGS_NC(9) KGS_NC(10) KGS_NC(11) KGS_NC(12) KGS_NC(13) KGS_NC(14) KGS_NC(15) KGS_NC(16)
+#undef KGS_NC
+    default: return KGS_ERR_SHAPE;
+  }
   return (int)hipGetLastError();
 }
 

@@ -1,0 +1,53 @@
+"""Launches that take single waves as workgroups up to a size (row_waves in transformer.hip, kgs_rope_cache_bf16): both sides of it."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+@pytest.mark.parametrize("rows", [1, 5, 1023, 1024, 1025, 1027])
+@pytest.mark.parametrize("add", [False, True])
+def test_norm_rows(rows, add):
+    from kgs.ops.transformer import add_rmsnorm
+
+    x, d, w = (torch.randn(*s, device=DEV).bfloat16() for s in ((rows, 512), (rows, 512), (512,)))
+    want = (x.float() + d.float()).bfloat16() if add else x.clone()
+    guard = torch.full((rows + 1, 512), 7.0, device=DEV).bfloat16()
+    add_rmsnorm(x, d if add else None, w, out=guard[:rows])
+    f = want.double()
+    ref = f * torch.rsqrt(f.pow(2).mean(-1, keepdim=True) + 1e-5) * w.double()
+    assert torch.equal(x, want) and bool((guard[rows] == 7).all())
+    # one rounding to bf16 and a few of fp32
+    assert float(((guard[:rows].double() - ref).abs() - 2.0 ** -8 * ref.abs()).max()) <= 1e-6
+
+
+@pytest.mark.parametrize("tokens,heads,kv,slices", [(1, 2, 1, 0), (33, 2, 1, 2), (2048, 2, 1, 0), (2049, 2, 1, 0), (2048, 2, 1, 8),
+                                                    (2049, 2, 1, 8), (1023, 4, 2, 0), (1024, 4, 2, 0), (2048, 4, 2, 4)])
+def test_rotation_and_cache(tokens, heads, kv, slices):
+    from kgs.ops import decode as D
+
+    nh = heads + 2 * kv
+    cos, sin = (torch.randn(300, 64, device=DEV) for _ in range(2))
+    pos = torch.randint(0, 300, (tokens,), device=DEV, dtype=torch.int32)
+    slot = torch.randperm((tokens // 32 + 2) * 32, device=DEV)[:tokens].int()
+    slot[::7] = -1
+    cache = torch.zeros(tokens // 32 + 2, kv, 2, 4096, device=DEV).bfloat16()
+    part = torch.randn(max(1, slices), tokens, nh * 128, device=DEV)
+    total = part[0]
+    for p in part[1:]:
+        total = total + p
+    qkv = torch.full((tokens + 1, nh * 128), 7.0, device=DEV).bfloat16()
+    given = total.bfloat16()
+    if not slices:
+        qkv[:tokens] = given
+    D.rope_cache_(qkv[:tokens], cos, sin, pos, slot, cache, heads, kv, partials=part if slices else None)
+    rot = D.ref_rope_rows(given, cos, sin, pos, heads + kv).double()
+    got = qkv[:tokens].double()
+    n = (heads + kv) * 128
+    assert float(((got[:, :n] - rot).abs() - 2.0 ** -8 * rot.abs()).max()) <= 1e-5  # fp32 turned, one rounding
+    assert torch.equal(qkv[:tokens, n:], given[:, n:]) and bool((qkv[tokens] == 7).all())
+    ref = torch.zeros_like(cache)
+    k, v = (qkv[:tokens, a:a + kv * 128].reshape(tokens, kv, 128) for a in (heads * 128, n))
+    D.ref_cache_write(ref, k, v, slot)
+    assert torch.equal(cache, ref)

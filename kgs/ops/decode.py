@@ -286,6 +286,24 @@ def w4x_rule(m: int, n: int, k: int, most: int = 16, cus: int = CUS):
     return 128, ns, bm
 
 
+def gate_rule(m: int, n: int, k: int, sliced: bool) -> int | None:
+    """Rows (64 or 128) of the gate kernel's tiles (:func:`kgs.ops.gemm.gemm_gate`) for a fused gate|up of ``n`` rows at up to 128
+    rows, None where 128-wide tiles are faster, or (``sliced``: the caller has a route of K slices) those in slices.
+
+    Its tiles of 32 outputs are a workgroup for every CU at n = 16384 and half of them or fewer rows below; up to 64 rows
+    two share a CU. us in a chain of launches, weights from HBM, 128-wide tiles in slices with their sum / without / so: 16384x2048
+    at 36 rows 20.0 / 24.1 / 17.5, 100 23.6 / 25.6 / 19.9, 8192x2048 at 100 18.2 / 23.4 / 13.7, 16384x4096 42.8 / 44.7 / 33.9, 11008x2048
+    at 64 19.3 / 23.2 / 15.3; without slices 28672x4096 at 64 58.6 / 51.3, 24576x2048 28.2 / 27.9, but 32768x2048 37.6 / 39.6 and at
+    100 rows 22016x4096 52.5 / 61. A long sum on less than half of the CUs, or from 65 rows on on less than seven eighths, is
+    better in slices: 8192x4096 at 64 21.5 / 24.8, 6144x6144 27.0 / 37.6, 10240x5120 at 96 43.0 / 45.9."""
+    wgs = -(-(n // 2) // 32)
+    if not 0 < m <= 128 or n % 16 or k % 8 or wgs > (448 if m <= 64 else CUS):
+        return None
+    if sliced and ((2 * wgs <= CUS and k > 2048) or (m > 64 and 8 * wgs < 7 * CUS and k > 4096)):
+        return None
+    return 64 if m <= 64 or 2 * wgs <= CUS else 128
+
+
 _MEASURED = {key[1:] for key in (*W4X_TUNED, *SPLITK_TUNED)}
 
 

@@ -450,6 +450,30 @@ def gemm_swiglu(a: torch.Tensor, w_gate_up: torch.Tensor, act="silu") -> torch.T
     return silu_mul(gemm_nt(a, w_gate_up))
 
 
+def gemm_gate(a: torch.Tensor, w_gate_up: torch.Tensor, bm: int, act="silu", out: torch.Tensor | None = None) -> torch.Tensor:
+    """:func:`gemm_swiglu` on tiles of ``bm`` (64 or 128) rows by 32 outputs, for few rows (the same bits). Rows of whole, aligned
+    16-byte chunks, ``K`` and ``I`` multiples of 8."""
+    from .activation import Gate
+
+    _check_operand(a, "a")
+    _check_operand(w_gate_up, "w_gate_up")
+    M, K = a.shape
+    N, K2 = w_gate_up.shape
+    if K != K2 or a.device != w_gate_up.device:
+        raise ValueError(f"operands do not fit: a {tuple(a.shape)} on {a.device}, w {tuple(w_gate_up.shape)} on {w_gate_up.device}")
+    if out is None:
+        out = torch.empty((M, N // 2), dtype=torch.bfloat16, device=a.device)
+    else:
+        _check_operand(out, "out")
+        if tuple(out.shape) != (M, N // 2) or out.device != a.device:
+            raise ValueError(f"out is {tuple(out.shape)} on {out.device}, expected {(M, N // 2)} on {a.device}")
+    gate = Gate.of(act)
+    rc = _lib.lib().kgs_gemm_bf16_nt_gate(a.data_ptr(), w_gate_up.data_ptr(), out.data_ptr(), M, N, K, a.stride(0), w_gate_up.stride(0),
+                                          out.stride(0), bm, GATE_ACTS[gate.act], gate.limit_ptr(a.device), _lib.stream_handle(a.device))
+    _lib.check(rc, f"gemm_gate[{M}x{N}x{K}]")
+    return out
+
+
 FP8_DTYPE = torch.float8_e4m3fn  # OCP e4m3 -- gfx950's MFMA fp8 format (not MI300's fnuz)
 FP8_MAX = 448.0
 # fp8: "fast" = the 8-wave aligned pipeline; "w4p" = the four-wave persistent

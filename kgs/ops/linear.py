@@ -62,7 +62,7 @@ class Projection:
         return act_mul(y, act)
 
     def _gated(self, x, m):
-        from .gemm import gemm_nt_w4x_swiglu, gemm_swiglu, swiglu_fused_ok
+        from .gemm import gemm_gate, gemm_nt_w4x_swiglu, gemm_swiglu, swiglu_fused_ok
 
         if m > 512:
             return gemm_swiglu(x, self.w, self.gated)
@@ -73,6 +73,9 @@ class Projection:
         # 22.7 / 28.2; 22016x4096 64.2 / 63.0 and 88.7 / 110.2)
         if m > 128:
             return gemm_swiglu(x, self.w, self.gated)
+        bm = D.gate_rule(m, *self.w.shape, sliced=False)
+        if bm is not None:
+            return gemm_gate(x, self.w, bm, self.gated)
         return gemm_nt_w4x_swiglu(x, self.w, bn=128, bm=128, nt_weights=D.NT_WEIGHTS, act=self.gated)
 
     def _plain(self, x, m, n, k):

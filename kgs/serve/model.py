@@ -51,6 +51,8 @@ from kgs.ops import decode as D
 
 from .trace import TRACE as T
 
+GATE = 32  # outputs of the gate kernel's tiles: a route's width
+
 
 def gate_up_panel_widths(n: int, k: int) -> set:
     """Tile widths of the unsplit SwiGLU decode routes for a gate|up of shape
@@ -260,13 +262,18 @@ class ServingModel:
         return self.w[layer]["gate_up"]
 
     def _swiglu_route(self, m: int):
-        """The route when the decode gate|up projection runs on the four-wave kernel: unsplit,
-        SwiGLU goes into its epilogue, split (no measured entry is), into the slices' sum."""
+        """The route when the decode gate|up projection runs on the four-wave kernel -- unsplit,
+        SwiGLU goes into its epilogue, split (no measured entry is), into the slices' sum -- or the gate kernel (``GATE``
+        wide)."""
         if not self.fuse_splitk:
             return None
         w = self.w[0]["gate_up"]
         r = D.w4x_route(m, w.shape[0], w.shape[1])
-        return D.w4x_rule(m, w.shape[0], w.shape[1]) if r is None else r if r[1] == 1 else None
+        if r is not None:
+            return r if r[1] == 1 else None
+        rule = D.w4x_rule(m, w.shape[0], w.shape[1])
+        bm = D.gate_rule(m, w.shape[0], w.shape[1], rule is not None and rule[1] > 1)
+        return rule if bm is None else (GATE, 1, bm)
 
     def _split_proj(self, x, layer: int, name: str, r, private: bool = False):
         """fp32 partial products of a projection along route ``r``, in a buffer of the call's own if
@@ -279,8 +286,10 @@ class ServingModel:
 
     def _gate_up_split(self, y, layer: int, r):
         """gate|up and SwiGLU along route ``r`` of :meth:`_swiglu_route`."""
-        from kgs.ops.gemm import gemm_nt_w4x_splitk_swiglu, gemm_nt_w4x_swiglu
+        from kgs.ops.gemm import gemm_gate, gemm_nt_w4x_splitk_swiglu, gemm_nt_w4x_swiglu
 
+        if r[0] == GATE:
+            return gemm_gate(y, self.w[layer]["gate_up"], r[2])
         if r[1] > 1:
             return gemm_nt_w4x_splitk_swiglu(y, self.w[layer]["gate_up"], r[0], r[1], r[2], nt_weights=D.w4x_nt(r, y.shape[0]), private=True)
         return gemm_nt_w4x_swiglu(y, self._gate_up_weight(layer, r[0]), bn=r[0], bm=r[2], stages=D.w4x_stages(r),

@@ -377,6 +377,79 @@ __global__ __launch_bounds__(256) void gemm_small(Args a) {
   }
 }
 
+// act(A . gate^T) * (A . up^T) of few rows, B = [gate; up] of 2 I rows: BM rows by 32 outputs, whose gate and up columns
+// (16 of each in turn) one wave holds. For grids that 128-wide tiles leave short of the CUs: what else fills them
+// there, K slices, costs their fp32 partial products' way through memory and a launch that sums them. Four stages and one
+// barrier per K-step as gemm_small, and its order of products per element. Bound by the operands' way into LDS: A comes
+// whole to every workgroup, 16384x2048 at 100 rows 20 us where 23.6 (0.4 us a K-step). B's loads are non-temporal (21.0 by
+// default; kgs/ops/decode.py gate_rule has the rule and its other side).
+template <int BM, int SW>
+__global__ __launch_bounds__(256) void gemm_gate(Args a) {
+  constexpr int BN = 64, ST = 4, FM = BM / 32, LA = BM / 32, LB = BN / 32, STAGE = (BM + BN) * 128;
+  __shared__ __attribute__((aligned(1024))) char smem[ST * STAGE];
+  const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int I = a.N / 2, ntm = (a.M + BM - 1) / BM, ntn = (I + 31) / 32;
+  int none, tm, tn;
+  w4::tile_of<0, false>((int)blockIdx.x, (int)gridDim.x, ntm, ntn, none, tm, tn);
+  const int m0 = tm * BM, n0 = tn * 32, K = a.K, nt = (K + BK - 1) / BK;
+  const int na = min(a.M - m0, BM), nb = min(I - n0, 32);
+  // waves 0 and 1 stage gate rows, 2 and 3 up rows: 16 of each per 32-row group
+  const auto ra = __builtin_amdgcn_make_buffer_rsrc((void*)(a.A + (long)m0 * a.lda), 0, ((na - 1) * a.lda + K) * 2, 0x00020000);
+  const auto rb = __builtin_amdgcn_make_buffer_rsrc((void*)(a.B + ((long)(w >> 1) * I + n0) * a.ldb), 0, ((nb - 1) * a.ldb + K) * 2, 0x00020000);
+  const int row = w * 8 + (lane >> 3), ch = ((lane & 7) ^ ((row >> 1) & 7)) * 8;
+  const int va = (row * a.lda + ch) * 2, vb = ((row & 15) * a.ldb + ch) * 2, sa = 64 * a.lda, sb = 32 * a.ldb;
+  auto load = [&](int t) {  // K-tile t (zeros past K) into its stage
+    char* dst = smem + (t % ST) * STAGE;
+    const bool in = t * BK + ch < K;
+    const int oa = in ? va : OOB, ob = in ? vb : OOB;
+#pragma unroll
+    for (int j = 0; j < LA; ++j)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (KGS_LDS void*)(dst + (j * 4 + w) * 1024), 16, oa, j * sa + t * 128, 0, 0);
+#pragma unroll
+    for (int j = 0; j < LB; ++j)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (KGS_LDS void*)(dst + BM * 128 + (j * 4 + w) * 1024), 16, ob, j * sb + t * 128, 0, 2);
+  };
+  const int fr = lane & 15, fq = lane >> 4;
+  const int ro = fr * 128 + ((fq ^ (fr >> 1)) * 16);
+  const int pa = (w >> 1) * (BM / 2) * 128 + ro, pb = BM * 128 + (w & 1) * (BN / 2) * 128 + ro;
+  f32x4 acc[FM][2];
+#pragma unroll
+  for (int i = 0; i < FM; ++i) acc[i][0] = acc[i][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int t = 0; t < ST - 1; ++t) load(t);
+  for (int t = 0; t < nt; ++t) {
+    w4::wait_vm<(ST - 2) * (LA + LB)>();  // this wave's part of K-tile t
+    w4::bar();                            // every wave's part, and every wave has read K-tile t - 1
+    load(t + ST - 1);
+    const char* st = smem + (t % ST) * STAGE;
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+      bf16x8 fa[FM], fb[2];
+#pragma unroll
+      for (int i = 0; i < FM; ++i) fa[i] = *(const bf16x8*)(st + ((pa + i * 2048) ^ (ks * 64)));
+#pragma unroll
+      for (int n = 0; n < 2; ++n) fb[n] = *(const bf16x8*)(st + ((pb + n * 2048) ^ (ks * 64)));
+#pragma unroll
+      for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int n = 0; n < 2; ++n) acc[i][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[n], fa[i], acc[i][n], 0, 0, 0);
+    }
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the tail's loads land before LDS is released
+  const float limit = SW == GATE_CLAMPED ? *(const float*)a.bias : 0.f;
+  const int col = n0 + (w & 1) * 16 + fq * 4;
+#pragma unroll
+  for (int i = 0; i < FM; ++i) {
+    const int r = m0 + (w >> 1) * (BM / 2) + i * 16 + fr;
+    if (r >= a.M || col >= I) continue;
+    float y[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) y[e] = gated<SW>(acc[i][0][e], acc[i][1][e], limit);
+    *(uint2*)((unsigned short*)a.C + (long)r * a.ldc + col) = make_uint2(pack_bf16x2(y[0], y[1]), pack_bf16x2(y[2], y[3]));
+  }
+}
+
 // Products with operands stored K-major (A as [K, M], B as [K, N]): Linear's backward pass, whose
 // dX = dY . W reads W that way and dW = dY^T . X both operands, at the sizes where transposing them
 // first costs more than a smaller tile does (layout_plan below). 128x128 tiles, two workgroups
@@ -942,6 +1015,23 @@ int gemm_any_swiglu(const void* A, const void* B, void* C, int M, int N, int K, 
   return (int)hipGetLastError();
 }
 
+// C [M, I] = act(A . gate^T) * (A . up^T), B = [gate; up] of N = 2 I rows, on tiles of bm (64, 128) rows by 32 outputs
+int gemm_gate(const void* A, const void* B, void* C, int M, int N, int K, int lda, int ldb, int ldc, int bm, int act,
+              const float* limit, hipStream_t s) {
+  using namespace any;
+  const Args a{(const unsigned short*)A, (const unsigned short*)B, C, nullptr, (const unsigned short*)limit,
+               M, N, K, lda, ldb, ldc, 0, 0, 1, 1.f, nullptr};
+  const dim3 grid((unsigned)(ceil_div(M, bm) * ceil_div(N / 2, 32)));
+#define KGS_GATE(ACT)                                                                                  \
+  if (bm == 64) hipLaunchKernelGGL((any::gemm_gate<64, ACT>), grid, dim3(256), 0, s, a);               \
+  else hipLaunchKernelGGL((any::gemm_gate<128, ACT>), grid, dim3(256), 0, s, a)
+  if (act == GATE_CLAMPED) { KGS_GATE(GATE_CLAMPED); }
+  else if (act == GATE_GELU) { KGS_GATE(GATE_GELU); }
+  else { KGS_GATE(GATE_SILU); }
+#undef KGS_GATE
+  return (int)hipGetLastError();
+}
+
 // e4m3 operands on 64x64 tiles, sizes in 16-bit words (kgs_gemm_fp8_nt_dev)
 int gemm_any_f8(const void* A, const void* B, void* C, const void* bias, int M, int N, int Kw, int lda, int ldb, int ldc,
                 float alpha, const float* alpha_ptr, int epi, hipStream_t s) {
@@ -1012,4 +1102,15 @@ KGS_EXPORT int kgs_gemm_bf16_nt_act(const void* A, const void* B, void* Z, void*
   if (!Y || epi < kgs::EPI_BIAS_GELU || epi > kgs::EPI_BIAS_SILU) return KGS_ERR_ARG;
   if (!kgs::gemm_any_ok(A, B, M, N, K, lda, ldb) || (uintptr_t)ws % 16) return KGS_ERR_ALIGN;
   return kgs::gemm_any(A, B, Z, Y, bias, M, N, K, lda, ldb, ldc, epi, 0, 0, 0, ws, s);
+}
+
+// C [M, N / 2] = act(A . gate^T) * (A . up^T), B = [gate; up] of N rows, both products rounded to bf16 first: tiles of bm (64
+// or 128) rows by 32 outputs. act: a GateAct (limit: the clamped gate's, on the device). N / 2 and K multiples of 8.
+KGS_EXPORT int kgs_gemm_bf16_nt_gate(const void* A, const void* B, void* C, int M, int N, int K, int lda, int ldb, int ldc, int bm,
+                                     int act, const void* limit, hipStream_t s) {
+  if (M <= 0 || N <= 0 || K <= 0 || N % 16 || lda < K || ldb < K || ldc < N / 2) return KGS_ERR_SHAPE;
+  if ((bm != 64 && bm != 128) || (act != kgs::GATE_SILU && act != kgs::GATE_GELU && act != kgs::GATE_CLAMPED)) return KGS_ERR_ARG;
+  if (act == kgs::GATE_CLAMPED && (!limit || (uintptr_t)limit % 4)) return KGS_ERR_ARG;
+  if (!kgs::gemm_any_ok(A, B, M, N, K, lda, ldb) || (uintptr_t)C % 16 || ldc % 8) return KGS_ERR_ALIGN;
+  return kgs::gemm_gate(A, B, C, M, N, K, lda, ldb, ldc, bm, act, (const float*)limit, s);
 }

@@ -29,3 +29,13 @@ def pytest_collection_modifyitems(config, items):
     for it in items:
         if "gpu" in it.keywords:
             it.add_marker(skip)
+
+
+@pytest.fixture
+def own_rng():
+    """Random numbers of the test's own: those of the tests after it do not depend on it."""
+    import torch
+
+    with torch.random.fork_rng(devices=range(torch.cuda.device_count())):
+        torch.manual_seed(0)
+        yield

@@ -3,7 +3,7 @@ that it takes the place of."""
 import pytest
 import torch
 
-pytestmark = pytest.mark.gpu
+pytestmark = [pytest.mark.gpu, pytest.mark.usefixtures("own_rng")]
 DEV = "cuda"
 
 

@@ -5,6 +5,7 @@ import torch
 
 from kgs.ops import decode as D
 
+pytestmark = pytest.mark.usefixtures("own_rng")
 DEV = "cuda"
 REL = 2.0 ** -8
 

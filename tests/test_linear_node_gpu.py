@@ -4,7 +4,7 @@ Python's can run."""
 import pytest
 import torch
 
-pytestmark = pytest.mark.gpu
+pytestmark = [pytest.mark.gpu, pytest.mark.usefixtures("own_rng")]
 DEV = "cuda"
 
 

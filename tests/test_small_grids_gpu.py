@@ -2,7 +2,7 @@
 import pytest
 import torch
 
-pytestmark = pytest.mark.gpu
+pytestmark = [pytest.mark.gpu, pytest.mark.usefixtures("own_rng")]
 DEV = "cuda"
 
 

@@ -620,12 +620,17 @@ def transpose(x: torch.Tensor) -> torch.Tensor:
 
 
 TR_READ_A = False        # route K-major A through ds_read_b64_tr_b16 (else transpose + NT)
-TR_READ_B_MAX_M = 4096   # K-major B: tr reads up to this M, transpose + NT above
+TR_READ_B_MAX_M = None   # K-major B: tr reads up to this M, transpose + NT above; None: by the sizes (gemm_any.hip turn_b)
 
 
 @lru_cache(maxsize=4096)
 def _tr_slices(m: int, n: int, k: int, ta: bool, tb: bool) -> int:
     return int(_lib.lib().kgs_gemm_bf16_tr_slices(m, n, k, int(ta), int(tb)))
+
+
+@lru_cache(maxsize=4096)
+def _turn_b(m: int, n: int, k: int) -> bool:
+    return bool(_lib.lib().kgs_gemm_bf16_turn_b(m, n, k))
 
 
 def _rows16(t: torch.Tensor) -> bool:
@@ -699,9 +704,7 @@ def _general(a, b, out, M, N, K, ta, tb, bias, act) -> torch.Tensor:
         # measured: the tr-read A path runs ~20 % behind a 6.3 TB/s transpose + NT
         # at 8192^3 and ties at 4096^3 (profiles/gemm_layouts.json)
         a, ta = transpose(a), 0
-    if tb and M > TR_READ_B_MAX_M:
-        # the B transpose costs ~ 476/M of the GEMM time; above M = 4096 it is
-        # cheaper than the tr-read path's LDS cost (profiles/gemm_layouts.json)
+    if tb and (_turn_b(M, N, K) if TR_READ_B_MAX_M is None else M > TR_READ_B_MAX_M):
         b, tb = transpose(b), 0
     if not ta and not tb:
         return gemm_nt(a, b, bias=bias, act=act, out=out)

@@ -815,6 +815,24 @@ inline bool wide(long M, long N, long K, bool split, int cus) {
   return cost(M, N, K, 256, 256, 1, cus) <= cost(M, N, K, p.bm, p.bn, 1, cus) * (K >= 3072 ? 1.14 : K > 512 ? 1.03 : 1);
 }
 
+// The 256x256 kernel that reads a K-major B transposed (kgs_gemm_bf16), us; sizes of whole tiles. Measured: 2048 x 1024 x 4096 65,
+// 4096 x 2048 x 8192 132, 3072^3 58, 4096^3 95, 4096 x 8192 x 2048 106, 4096 x 14336 x 4096 347.
+inline double tr256_cost(long M, long N, long K, int cus) {
+  const long g = (M / 256) * (N / 256), full = g / cus;
+  const double rest = (double)(g - full * cus) / cus, b4 = rest * rest * rest * rest;
+  return 8 * (full + (rest > 0)) + K / 64 * (full * 1.36 + (rest > 0 ? 0.88 + 0.15 * rest + 0.33 * b4 : 0));
+}
+
+// Whether that kernel loses to a transpose of B (4 bytes a value at 6.4 TB/s) and the product's best tiles: where its tiles leave
+// most of the CUs idle. us, transposed read / transpose and tiles: 2048 x 1024 x 4096 65 / 38, 4096 x 512 x 4096 65 / 36, 4096 x
+// 2048 x 8192 132 / 118; 4096 x 8192 x 2048 106 / 114, 2048 x 14336 x 4096 172 / 217, 8192 x 2048 x 2048 52 / 59.
+inline bool turn_b(long M, long N, long K, int cus) {
+  const Plan p = refine(plan(M, N, K, true, cus), M, N, K, cus);
+  const double nt = p.ns > 1 || p.bm == 64 ? cost(M, N, K, p.bm == 64 ? 128 : p.bm, p.bm == 64 ? 128 : p.bn, p.ns, cus)
+                                           : tile_cost(p.bm, p.bn, M, N, K, cus);
+  return nt + 2.5 + 4.0 * N * K / 6.4e6 < tr256_cost(M, N, K, cus);
+}
+
 // Slices with which gemm_tr is the fastest way to a product with K-major operands, 0 where
 // another one is. The others transpose the operands first (a launch and a pass over memory each)
 // and run cost()'s best tile, or, for aligned sizes and a K-major B alone, the 256x256 kernel that
@@ -846,11 +864,7 @@ inline int layout_plan(long M, long N, long K, int ta, int tb, int cus) {
   }
   if (K % 8) return best;  // nothing else reads such operands 16 bytes at a time
   if (t0 > nt + turn_a + turn_b) return 0;
-  if (M % 256 == 0 && N % 256 == 0 && K % 128 == 0 && tb && M <= 4096) {
-    const long g = (M / 256) * (N / 256);
-    const double busy = g < cus ? (double)g / cus : 1;
-    if (t0 > 4 + ceil_div(g, cus) * (K / 64) * (0.98 + 0.32 * busy) + turn_a) return 0;
-  }
+  if (M % 256 == 0 && N % 256 == 0 && K % 128 == 0 && tb && t0 > tr256_cost(M, N, K, cus) + turn_a) return 0;
   return best;
 }
 
@@ -1087,6 +1101,11 @@ KGS_EXPORT int kgs_gemm_bf16_tr(const void* A, const void* B, void* C, int M, in
   if (M <= 0 || N <= 0 || K <= 0 || ldc < N || ns < 1 || ns > 64) return KGS_ERR_SHAPE;
   if (!kgs::gemm_tr_ok(A, B, M, N, K, lda, ldb, ta, tb) || (uintptr_t)ws % 16) return KGS_ERR_ALIGN;
   return kgs::gemm_tr(A, B, C, M, N, K, lda, ldb, ldc, ta, tb, ns, ws, s);
+}
+
+// Whether a K-major B is better transposed first than read by kgs_gemm_bf16 (turn_b).
+KGS_EXPORT int kgs_gemm_bf16_turn_b(int M, int N, int K) {
+  return M > 0 && N > 0 && K > 0 && kgs::any::turn_b(M, N, K, kgs::cu_count());
 }
 
 // Slices for kgs_gemm_bf16_tr, 0 where another route is faster (layout_plan).

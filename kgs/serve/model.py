@@ -226,7 +226,8 @@ class ServingModel:
         # the LM head (N = 128256) from batch 128 up runs faster on the kgs
         # 256x256 GEMM than on hipBLASLt (1.09x at 128, 1.21x at 256,
         # profiles/decode_wide_gemm.jsonl); the other decode shapes do not
-        if decode and (layer is not None or m < 128):
+        # up to 32 rows of it on the general kernel's small tiles (us, library / so: 32000x4096 62 / 48, 32000x2048 35 / 31)
+        if decode and (layer is not None or 32 < m < 128):
             return torch.matmul(x, w.T)
         from kgs.ops import gemm_nt
 

@@ -317,9 +317,17 @@ __global__ __launch_bounds__(256) void gemm_small(Args a) {
 #pragma unroll
     for (int j = 0; j < LA; ++j)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (KGS_LDS void*)(dst + (j * 4 + w) * 1024), 16, oa, j * sa + t * 128, 0, 0);
+    // B is read once, whole lines at a time: non-temporal loads, 5.9 TB/s of a large B where the default policy reaches 5.0 (off
+    // the 128-byte lines each would come twice: 64 x 3000 x 1032 9.1 / 12.1 us)
+    if (ntm == 1 && a.ldb % 64 == 0) {
 #pragma unroll
-    for (int j = 0; j < LB; ++j)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (KGS_LDS void*)(dst + BM * 128 + (j * 4 + w) * 1024), 16, ob, j * sb + t * 128, 0, 0);
+      for (int j = 0; j < LB; ++j)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (KGS_LDS void*)(dst + BM * 128 + (j * 4 + w) * 1024), 16, ob, j * sb + t * 128, 0, 2);
+    } else {
+#pragma unroll
+      for (int j = 0; j < LB; ++j)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (KGS_LDS void*)(dst + BM * 128 + (j * 4 + w) * 1024), 16, ob, j * sb + t * 128, 0, 0);
+    }
   };
   const int fr = lane & 15, fq = lane >> 4;
   const int ro = fr * 128 + ((fq ^ (fr >> 1)) * 16);
@@ -381,8 +389,8 @@ __global__ __launch_bounds__(256) void gemm_small(Args a) {
 // (16 of each in turn) one wave holds. For grids that 128-wide tiles leave short of the CUs: what else fills them
 // there, K slices, costs their fp32 partial products' way through memory and a launch that sums them. Four stages and one
 // barrier per K-step as gemm_small, and its order of products per element. Bound by the operands' way into LDS: A comes
-// whole to every workgroup, 16384x2048 at 100 rows 20 us where 23.6 (0.4 us a K-step). B's loads are non-temporal (21.0 by
-// default; kgs/ops/decode.py gate_rule has the rule and its other side).
+// whole to every workgroup, 16384x2048 at 100 rows 20 us where 23.6 (0.4 us a K-step). B's loads are non-temporal where its rows are whole
+// 128-byte lines (21.0 by default; kgs/ops/decode.py gate_rule has the rule and its other side).
 template <int BM, int SW>
 __global__ __launch_bounds__(256) void gemm_gate(Args a) {
   constexpr int BN = 64, ST = 4, FM = BM / 32, LA = BM / 32, LB = BN / 32, STAGE = (BM + BN) * 128;
@@ -406,9 +414,15 @@ __global__ __launch_bounds__(256) void gemm_gate(Args a) {
 #pragma unroll
     for (int j = 0; j < LA; ++j)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (KGS_LDS void*)(dst + (j * 4 + w) * 1024), 16, oa, j * sa + t * 128, 0, 0);
+    if (a.ldb % 64 == 0) {
 #pragma unroll
-    for (int j = 0; j < LB; ++j)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (KGS_LDS void*)(dst + BM * 128 + (j * 4 + w) * 1024), 16, ob, j * sb + t * 128, 0, 2);
+      for (int j = 0; j < LB; ++j)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (KGS_LDS void*)(dst + BM * 128 + (j * 4 + w) * 1024), 16, ob, j * sb + t * 128, 0, 2);
+    } else {
+#pragma unroll
+      for (int j = 0; j < LB; ++j)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (KGS_LDS void*)(dst + BM * 128 + (j * 4 + w) * 1024), 16, ob, j * sb + t * 128, 0, 0);
+    }
   };
   const int fr = lane & 15, fq = lane >> 4;
   const int ro = fr * 128 + ((fq ^ (fr >> 1)) * 16);
@@ -736,9 +750,14 @@ inline Plan plan(long M, long N, long K, bool split, int cus) {
         best = {s[0], s[1], ns};
       }
     }
-  // 64x64 tiles: a cheaper step, twice as many bytes per product; several share a CU
-  const double full = (double)ceil_div(M, 64) * ceil_div(N, 64) / cus;
-  if (3.5 + ceil_div(K, 64) * (full <= 1 ? 0.34 + 0.06 * full : 0.06 + 0.38 * full) < t0) best = {64, 64, 1};
+  if (M <= 64) t0 = t0 > 4 + 2.0 * N * K / 5.0e6 ? t0 : 4 + 2.0 * N * K / 5.0e6;  // few rows: B's way from memory
+  // 64x64 tiles: a cheaper step, twice as many bytes per product; several share a CU. Up to 64 rows B is read once, past
+  // the caches, where there are tiles for most CUs: us at 1 to 16 rows by larger tiles / so 32000x4096 57 / 45, 32000x2048 33 / 28,
+  // 14336x4096 28 / 25, 128256x4096 at 40 192 / 179, but at 64 196 / 207
+  const double full = (double)ceil_div(M, 64) * ceil_div(N, 64) / cus, steps = ceil_div(K, 64);
+  const double t = M <= 64 && full >= 0.75 && (M <= 48 || full <= 4) ? 4 + steps * (full <= 1 ? 0.20 + 0.13 * full : 0.33 * full)
+                                                                     : 3.5 + steps * (full <= 1 ? 0.34 + 0.06 * full : 0.06 + (M <= 64 ? 0.43 : 0.38) * full);
+  if (t < t0) best = {64, 64, 1};
   return best;
 }
 

@@ -51,3 +51,17 @@ def test_rotation_and_cache(tokens, heads, kv, slices):
     k, v = (qkv[:tokens, a:a + kv * 128].reshape(tokens, kv, 128) for a in (heads * 128, n))
     D.ref_cache_write(ref, k, v, slot)
     assert torch.equal(cache, ref)
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 256, 64), (64, 200, 128), (65, 128, 128), (33, 72, 200), (64, 136, 328), (17, 64, 1024)])
+def test_small_tiles_by_either_cache_policy(M, N, K):
+    """One row tile with whole-line rows of B (non-temporal), two of them, rows off the lines."""
+    from kgs.ops import _lib
+
+    a, b = (torch.randn(r, K, device=DEV).bfloat16() for r in (M, N))
+    c = torch.full((M + 1, N), 7.0, device=DEV).bfloat16()
+    rc = _lib.lib().kgs_gemm_bf16_nt_any(a.data_ptr(), b.data_ptr(), c.data_ptr(), None, M, N, K, K, K, N, 0, 64, 64, 1, None,
+                                         _lib.stream_handle(a.device))
+    want = a.double() @ b.double().T
+    assert rc == 0 and bool((c[M] == 7).all())
+    assert float((c[:M].double() - want).norm() / want.norm()) < 2.0 ** -8  # one rounding to bf16

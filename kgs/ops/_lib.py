@@ -141,6 +141,7 @@ _SIGS = {
     "kgs_head_proj": ([_c_void_p] * 6 + [_c_long] * 5 + [_c_int] * 7 + [_c_void_p] * 2 + [_c_int] * 3 + [_c_void_p],
                       _c_int),
     "kgs_latent_attn": ([_c_void_p] * 10 + [_c_int] * 10 + [ctypes.c_float, _c_void_p], _c_int),
+    "kgs_latent_attn_parts": ([_c_void_p] * 10 + [_c_int] * 9 + [ctypes.c_float, _c_void_p], _c_int),
     # residual, talking-heads attention, mixture of experts (residual.hip, talking.hip, moe.hip)
     "kgs_residual_embed": ([_c_void_p] * 3 + [_c_long, ctypes.c_float] + [_c_void_p] * 2 + [_c_long, _c_void_p]
                            + [_c_int] * 5 + [ctypes.c_float] * 2 + [_c_int, _c_void_p], _c_int),

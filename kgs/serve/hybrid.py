@@ -28,7 +28,7 @@ from kgs.ops.decode import PAGE
 from kgs.ops.delta import DeltaShape, DeltaState, delta_forward, delta_out
 from kgs.ops.hyper import MAX_STREAMS, hyper_embed, hyper_step
 from kgs.ops.latent import (LatentCache, LatentRows, head_proj, latent_attention, latent_norm, mfma_sizes,
-                            padded_latent, padded_rot, split_count, waves_for, window_pages)
+                            padded_latent, padded_rot, split_count, split_parts, waves_for, window_pages)
 from kgs.ops.linear import Projection
 from kgs.ops.transformer import attention_ragged
 
@@ -154,10 +154,11 @@ class Geometry:
     def decode_plan(self, f, nb, positions, block_tables):
         waves = waves_for(self.heads, self.rp)
         tiles = -(-self.heads // (16 * waves))
+        maxp = self.pages(block_tables.shape[1], 1)
         return LatentPlan(LatentRows(
             nt=nb, q0=f["ar"], n=f["one"], pos0=positions, bt=block_tables, tok_seq=f["ar"], tok_pos=positions,
             rows=None, items=None, ntiles=nb * tiles, tiles=tiles, waves=waves,
-            nsplit=split_count(nb * tiles, self.pages(block_tables.shape[1], 1), self.rp)), None)
+            nsplit=split_count(nb * tiles, maxp, self.rp), parts=split_parts(nb, tiles, maxp, self.rp)), None)
 
 
 # -------------------------------------------------------------------- sublayers

@@ -321,9 +321,59 @@ struct Args {
   int H, W, tiles, nsplit, Nt, RP, HR;
   float scale, sl2;  // sl2 = scale * log2(e)
   int win;           // 0: every earlier key
+  int parts;         // 0: nsplit equal splits of each; else parts by length for one token a sequence (find_part), q0[b] = b
+  int* part_of;      // then [Nt][first part, parts], written for merge
 };
 
 __device__ __forceinline__ int first_key(const Args& a, int pos) { return a.win ? max(0, pos - a.win + 1) : 0; }
+
+// Pages that a token at pos sees
+__device__ __forceinline__ int pages_seen(const Args& a, int pos) { return pos / PAGE - first_key(a, pos) / PAGE + 1; }
+
+constexpr int MAX_SPLIT = 64;   // parts of a sequence
+constexpr int LEAST_PAGES = 2;  // pages of a part
+
+// Parts by length: all sequences are cut into parts of the same number of pages, the fewest that make at most `parts`
+// of them (and MAX_SPLIT of one), and workgroup i takes part i of the list. The host sees only the block table's width:
+// equal splits of each sequence are as many as its longest needs, the longest one's are the launch's time, and the short ones'
+// workgroups are done or empty. 24 sequences of 60 to 1300 tokens with 16 heads over latents of 512: 14.9 us in equal splits,
+// 10.9 so, and the merge's 4.9 and 4.7; the page's own loads and products are about 2 us of a part, so parts are two pages
+// and more.
+struct Part {
+  int seq, pos, part, first, count, pages;  // seq -1: none
+};
+__device__ __forceinline__ Part find_part(const Args& a, int i, int lane) {
+  float total = 0.f, most = 0.f;  // whole numbers
+  for (int c = lane; c < a.Nt; c += 64) {
+    const float np = (float)pages_seen(a, a.pos0[c]);
+    total += np;
+    most = fmaxf(most, np);
+  }
+  total = wave_sum(total);
+  most = wave_max(most);
+  const int room = a.parts - a.Nt;  // every sequence's last part may be a short one
+  const int pages = __builtin_amdgcn_readfirstlane(
+      max(LEAST_PAGES, max(((int)total + room - 1) / room, ((int)most + MAX_SPLIT - 1) / MAX_SPLIT)));
+  for (int c0 = 0, before = 0; c0 < a.Nt; c0 += 64) {
+    const int c = c0 + lane, pos = a.pos0[min(c, a.Nt - 1)];
+    const int n = c < a.Nt ? (pages_seen(a, pos) + pages - 1) / pages : 0;
+    int upto = n;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int v = __shfl_up(upto, o);
+      if (lane >= o) upto += v;
+    }
+    upto += before;
+    const unsigned long long hit = __ballot(i >= upto - n && i < upto);
+    if (hit) {
+      const int src = __builtin_ctzll(hit);
+      const int first = __builtin_amdgcn_readlane(upto - n, src);
+      return {c0 + src, __builtin_amdgcn_readlane(pos, src), i - first, first, __builtin_amdgcn_readlane(n, src), pages};
+    }
+    before = __builtin_amdgcn_readlane(upto, 63);
+  }
+  return {-1, 0, 0, 0, 0, pages};
+}
 
 template <int I, int N, class F>
 __device__ __forceinline__ void static_for(F f) {
@@ -433,15 +483,26 @@ __global__ __launch_bounds__(RT > 8 ? 256 : 512) void attn(Args a) {
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int l16 = lane & 15, g = lane >> 4, tq = (lane >> 2) & 3, tp = lane & 3;
   int b, tile;  // uniform: page ids then come by scalar loads
-  if (a.items) {
+  Part pt{};
+  if (a.parts) {
+    const int i = __builtin_amdgcn_readfirstlane(blockIdx.x / a.tiles);
+    tile = blockIdx.x - i * a.tiles;
+    pt = find_part(a, i, lane);
+    b = pt.seq;
+    if (b < 0) return;
+    if (pt.part == 0 && tile == 0 && threadIdx.x == 0) {
+      a.part_of[2 * b] = pt.first;
+      a.part_of[2 * b + 1] = pt.count;
+    }
+  } else if (a.items) {
     b = a.items[2 * blockIdx.x];
     tile = a.items[2 * blockIdx.x + 1];
   } else {
     b = __builtin_amdgcn_readfirstlane(blockIdx.x / a.tiles);
     tile = blockIdx.x - b * a.tiles;
   }
-  const int rows = a.n[b] * a.H, pos0 = a.pos0[b];
-  const long base = (long)a.q0[b] * a.H;  // row 0 of the sequence
+  const int rows = a.parts ? a.H : a.n[b] * a.H, pos0 = a.parts ? pt.pos : a.pos0[b];
+  const long base = (long)(a.parts ? b : a.q0[b]) * a.H;  // row 0 of the sequence
   const int r0 = tile * 16 * nw;          // the workgroup's rows
   if (r0 >= rows) return;
   const int last = min(r0 + 16 * nw, rows) - 1;
@@ -452,8 +513,8 @@ __global__ __launch_bounds__(RT > 8 ? 256 : 512) void attn(Args a) {
   const int wmin = first_key(a, pos0 + min(r0 + 16 * w, last) / a.H);  // and first key
   const int fp = __builtin_amdgcn_readfirstlane(first_key(a, pos0 + r0 / a.H) / PAGE);
   const int npages = __builtin_amdgcn_readfirstlane((pos0 + last / a.H) / PAGE + 1);
-  const int pps = __builtin_amdgcn_readfirstlane((npages - fp + a.nsplit - 1) / a.nsplit);
-  const int p0 = fp + blockIdx.y * pps, p1 = min(p0 + pps, npages);
+  const int pps = a.parts ? pt.pages : __builtin_amdgcn_readfirstlane((npages - fp + a.nsplit - 1) / a.nsplit);
+  const int p0 = fp + (a.parts ? pt.part : (int)blockIdx.y) * pps, p1 = min(p0 + pps, npages);
   const int* bt = a.bt + (long)b * a.W;
   const unsigned short* cache = (const unsigned short*)a.cache;
   const long nrows = (long)a.Nt * a.H;
@@ -592,7 +653,7 @@ __global__ __launch_bounds__(RT > 8 ? 256 : 512) void attn(Args a) {
       *(uint2*)(op + 16 * i) = v;
     }
   } else {
-    const long pr = blockIdx.y * nrows + base + myrow;
+    const long pr = (a.parts ? (long)(pt.first + pt.part) * a.H : blockIdx.y * nrows + base) + myrow;
     float* po = a.part_o + pr * G::RP + 4 * g;
 #pragma unroll
     for (int i = 0; i < 2 * RT; ++i) *(f32x4*)(po + 16 * i) = acc[i];
@@ -604,7 +665,6 @@ __global__ __launch_bounds__(RT > 8 ? 256 : 512) void attn(Args a) {
 }
 
 // one workgroup per row: o = sum_s 2^((m_s - m) sl2) acc_s / sum_s 2^((m_s - m) sl2) l_s
-constexpr int MAX_SPLIT = 64;
 __global__ __launch_bounds__(128) void merge(Args a) {
   __shared__ float wt[MAX_SPLIT];
   const int tid = threadIdx.x;
@@ -633,6 +693,54 @@ __global__ __launch_bounds__(128) void merge(Args a) {
     o.y = pack_bf16x2(v[2], v[3]);
     *(uint2*)((unsigned short*)a.o + row * a.RP + c) = o;
   }
+}
+
+// The same over parts by length, none of which is empty: eight parts' loads are under way at once, the first of them
+// before the weights are known.
+__global__ __launch_bounds__(128) void merge_parts(Args a) {
+  constexpr int U = 8;
+  __shared__ float wt[MAX_SPLIT];
+  const int tid = threadIdx.x, b = blockIdx.x / a.H;
+  const long row = blockIdx.x;
+  const int first = a.part_of[2 * b], ns = a.part_of[2 * b + 1];
+  const long r0 = (long)first * a.H + (row - (long)b * a.H);
+  const long step = (long)a.H * a.RP;
+  const float* po = a.part_o + r0 * a.RP;
+  const int c0 = min(4 * tid, a.RP - 4);
+  f32x4 x[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) x[u] = *(const f32x4*)(po + min(u, ns - 1) * step + c0);
+  if (tid < 64) {
+    float m = NEG, l = 0.f;
+    if (tid < ns) {
+      const float* ml = a.part_ml + 2 * ((long)tid * a.H + r0);
+      l = ml[1];
+      m = l > 0.f ? ml[0] : NEG;
+    }
+    const float mx = wave_max(m);
+    const float e = l > 0.f ? __builtin_amdgcn_exp2f((m - mx) * a.sl2) : 0.f;
+    wt[tid] = e / wave_sum(e * l);
+  }
+  __syncthreads();
+  if (4 * tid >= a.RP) return;  // RP is at most 512
+  f32x4 v = f32x4{};
+  for (int s = 0; s < ns; s += U) {
+    f32x4 y[U];
+    if (s + U < ns) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) y[u] = *(const f32x4*)(po + min(s + U + u, ns - 1) * step + c0);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const float w = s + u < ns ? wt[s + u] : 0.f;
+      if (w > 0.f) v += x[u] * w;
+      x[u] = y[u];
+    }
+  }
+  uint2 o;
+  o.x = pack_bf16x2(v[0], v[1]);
+  o.y = pack_bf16x2(v[2], v[3]);
+  *(uint2*)((unsigned short*)a.o + row * a.RP + c0) = o;
 }
 
 // ---------------------------------------------------------------- attn_simple
@@ -709,7 +817,7 @@ static hipError_t launch_attn(const Args& a, int ntiles, int nw, hipStream_t s) 
         hipFuncSetAttribute((const void*)attn<RT, RK>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return e;
   }
-  hipLaunchKernelGGL((attn<RT, RK>), dim3(ntiles, a.nsplit), dim3(64 * nw), lds, s, a);
+  hipLaunchKernelGGL((attn<RT, RK>), a.parts ? dim3(a.parts * a.tiles) : dim3(ntiles, a.nsplit), dim3(64 * nw), lds, s, a);
   return hipGetLastError();
 }
 template <int RT>
@@ -770,25 +878,16 @@ KGS_EXPORT int kgs_head_proj(const void* a, const void* w, void* out, const void
   return (int)hipGetLastError();
 }
 
-// MFMA form: RP one of 32 x {1, 2, 3, 4, 6, 8, 12, 16}, HR 0, 32 or 64, bf16. ntiles workgroups
-// per split (items: ntiles (sequence, tile) pairs; null: B x tiles). A tile is
-// 16 nw rows.
-KGS_EXPORT int kgs_latent_attn(const void* q, const void* cache, void* o, void* part_o, void* part_ml, const void* q0,
-                               const void* n, const void* pos0, const void* bt, const void* items, int ntiles,
-                               int tiles, int nw, int nsplit, int H, int W, int Nt, int RP, int HR, int win,
-                               float scale, hipStream_t s) {
+static int latent_attn(const kgs::latent::Args& a, int ntiles, int nw, hipStream_t s) {
   using namespace kgs::latent;
-  if (ntiles <= 0 || H <= 0 || W <= 0 || Nt <= 0 || nw < 1 || nw > 8 || nsplit < 1 || nsplit > MAX_SPLIT ||
-      (!items && tiles <= 0) || (HR != 0 && HR != 32 && HR != 64) || win < 0)
+  if (ntiles <= 0 || a.H <= 0 || a.W <= 0 || a.Nt <= 0 || nw < 1 || nw > 8 || a.nsplit < 1 || a.nsplit > MAX_SPLIT ||
+      (!a.items && a.tiles <= 0) || (a.HR != 0 && a.HR != 32 && a.HR != 64) || a.win < 0)
     return KGS_ERR_SHAPE;
-  if (nsplit > 1 && (!part_o || !part_ml)) return KGS_ERR_ARG;
-  if (RP > 256 && nw > 4) return KGS_ERR_SHAPE;  // a wave holds 16 x RP outputs in registers
-  if (((uintptr_t)q | (uintptr_t)cache | (uintptr_t)o | (uintptr_t)part_o) & 15) return KGS_ERR_ALIGN;
-  Args a{q, cache, o, (float*)part_o, (float*)part_ml, (const int*)q0, (const int*)n, (const int*)pos0,
-         (const int*)bt, (const int*)items, nullptr, nullptr, H, W, tiles, nsplit, Nt, RP, HR, scale,
-         scale * 1.4426950408889634f, win};
+  if (a.nsplit > 1 && (!a.part_o || !a.part_ml)) return KGS_ERR_ARG;
+  if (a.RP > 256 && nw > 4) return KGS_ERR_SHAPE;  // a wave holds 16 x RP outputs in registers
+  if (((uintptr_t)a.q | (uintptr_t)a.cache | (uintptr_t)a.o | (uintptr_t)a.part_o) & 15) return KGS_ERR_ALIGN;
   hipError_t e;
-  switch (RP) {
+  switch (a.RP) {
     case 32: e = launch_attn<1>(a, ntiles, nw, s); break;
     case 64: e = launch_attn<2>(a, ntiles, nw, s); break;
     case 96: e = launch_attn<3>(a, ntiles, nw, s); break;
@@ -799,11 +898,38 @@ KGS_EXPORT int kgs_latent_attn(const void* q, const void* cache, void* o, void* 
     case 512: e = launch_attn<16>(a, ntiles, nw, s); break;
     default: return KGS_ERR_SHAPE;
   }
-  if (e == hipSuccess && nsplit > 1) {
-    hipLaunchKernelGGL(merge, dim3((unsigned)((long)Nt * H)), dim3(128), 0, s, a);
+  if (e == hipSuccess && a.nsplit > 1) {
+    const dim3 grid((unsigned)((long)a.Nt * a.H));
+    if (a.parts) hipLaunchKernelGGL(merge_parts, grid, dim3(128), 0, s, a);
+    else hipLaunchKernelGGL(merge, grid, dim3(128), 0, s, a);
     e = hipGetLastError();
   }
   return (int)e;
+}
+
+// MFMA form: RP one of 32 x {1, 2, 3, 4, 6, 8, 12, 16}, HR 0, 32 or 64, bf16. ntiles workgroups
+// per split (items: ntiles (sequence, tile) pairs; null: B x tiles). A tile is
+// 16 nw rows.
+KGS_EXPORT int kgs_latent_attn(const void* q, const void* cache, void* o, void* part_o, void* part_ml, const void* q0,
+                               const void* n, const void* pos0, const void* bt, const void* items, int ntiles,
+                               int tiles, int nw, int nsplit, int H, int W, int Nt, int RP, int HR, int win,
+                               float scale, hipStream_t s) {
+  return latent_attn({q, cache, o, (float*)part_o, (float*)part_ml, (const int*)q0, (const int*)n, (const int*)pos0,
+                      (const int*)bt, (const int*)items, nullptr, nullptr, H, W, tiles, nsplit, Nt, RP, HR, scale,
+                      scale * 1.4426950408889634f, win, 0, nullptr}, ntiles, nw, s);
+}
+
+// The same for one token of each of the Nt sequences (q0[b] = b, n[b] = 1) in `parts` > Nt parts by length: part_o
+// [parts][H][RP], part_ml [parts][H][2], part_of [Nt][2].
+KGS_EXPORT int kgs_latent_attn_parts(const void* q, const void* cache, void* o, void* part_o, void* part_ml, void* part_of,
+                                     const void* q0, const void* n, const void* pos0, const void* bt, int tiles, int nw,
+                                     int parts, int H, int W, int Nt, int RP, int HR, int win, float scale,
+                                     hipStream_t s) {
+  if (tiles <= 0 || Nt <= 0 || parts <= Nt || (long)parts * tiles > 65535 || (long)16 * nw * tiles < H) return KGS_ERR_SHAPE;
+  if (!part_of || !q0 || !n || !pos0 || !bt) return KGS_ERR_ARG;
+  return latent_attn({q, cache, o, (float*)part_o, (float*)part_ml, (const int*)q0, (const int*)n, (const int*)pos0,
+                      (const int*)bt, nullptr, nullptr, nullptr, H, W, tiles, kgs::latent::MAX_SPLIT, Nt, RP, HR, scale,
+                      scale * 1.4426950408889634f, win, parts, (int*)part_of}, parts * tiles, nw, s);
 }
 
 KGS_EXPORT int kgs_latent_attn_simple(const void* q, const void* cache, void* o, const void* tok_seq,
@@ -813,7 +939,7 @@ KGS_EXPORT int kgs_latent_attn_simple(const void* q, const void* cache, void* o,
   if (H <= 0 || W <= 0 || Nt <= 0 || RP <= 0 || RP > SIMPLE_MAX || HR < 0 || HR > SIMPLE_ROT || win < 0)
     return KGS_ERR_SHAPE;
   Args a{q, cache, o, nullptr, nullptr, nullptr, nullptr, nullptr, (const int*)bt, nullptr, (const int*)tok_seq,
-         (const int*)tok_pos, H, W, 0, 1, Nt, RP, HR, scale, 0.f, win};
+         (const int*)tok_pos, H, W, 0, 1, Nt, RP, HR, scale, 0.f, win, 0, nullptr};
   const dim3 grid((unsigned)((long)Nt * H));
   if (f32) hipLaunchKernelGGL(attn_simple<float>, grid, dim3(256), 0, s, a);
   else hipLaunchKernelGGL(attn_simple<unsigned short>, grid, dim3(256), 0, s, a);

@@ -317,19 +317,18 @@ def w4x_stages(route) -> int:
 NT_WEIGHTS = os.environ.get("KGS_NT_WEIGHTS", "1") == "1"
 
 
-def w4x_nt(route, rows: int = 0, packed: bool = False) -> bool:
-    """Whether this route's weights are streamed non-temporally (``packed``: from a tile-panel copy): those of two stages,
-    except row-major ones in K slices for up to 128 rows.
+def w4x_nt(route, packed: bool = False) -> bool:
+    """Whether this route's weights are streamed non-temporally (``packed``: from a tile-panel copy): those of two stages
+    without K slices, or packed.
 
     A product without slices reads a row-major weight in whole rows per CU and is 3 to 9 % faster so; a slice reads short
     pieces of its rows, and the default policy is the faster one. us in a chain of launches, weights (700 MB of them)
     from HBM, non-temporal / default: 28672x4096 gate|up unsliced at 40 / 90 / 256 rows 45.7 / 49.9, 49.3 / 52.1, 63.0 / 67.0,
     32000x2048 at 100 37.9 / 40.1; in slices at 100 rows 2048x8192 23.4 / 20.0, 16384x2048 28.1 / 23.5, 4096x4096 21.6 / 18.3,
-    3072x2048 16.0 / 15.8 (at 40 11.6 / 11.7). Launched back to back, with no other kernels between them, the two differ by 2 %.
-    Packed slices and more rows gain as much in such a chain (4096x4096 packed 20.6 / 17.7, 2048x8192 at 200 rows 24.3 / 21.3) and
-    not in whole steps: 90 prompt rows of hidden 4096 626 to 646 us, 655 by default; decode steps 2048 wide of 250 sequences of
-    60 415 / 430, of 150 of 200 462 / 462."""
-    return NT_WEIGHTS and w4x_stages(route) == 2 and (route[1] == 1 or packed or rows > 128)
+    3072x2048 16.0 / 15.8 (at 40 11.6 / 11.7), at 200 2048x8192 24.3 / 21.3, 4096x8192 34.5 / 31.7. Launched back to back,
+    with no other kernels between them, the two differ by 2 %. Packed slices gain as much in such a chain (4096x4096 20.6 / 17.7)
+    and not in a whole step (90 prompt rows of hidden 4096 626 to 646 us, 655 by default)."""
+    return NT_WEIGHTS and w4x_stages(route) == 2 and (route[1] == 1 or packed)
 
 
 def w4x_split_bns(n: int, k: int) -> set:

@@ -97,4 +97,4 @@ class Projection:
         if route is None:  # us at 64 rows of 4096x11008, which slices badly: 27 here, 36 by the library
             return gemm_nt(x, self.w) if m >= 128 or (n % 128 == 0 and k % 128 == 0) else None
         return gemm_nt_w4x(x, self.w, bn=route[0], nslice=route[1], bm=route[2], stages=D.w4x_stages(route),
-                           nt_weights=D.w4x_nt(route, m), private=table is None)
+                           nt_weights=D.w4x_nt(route), private=table is None)

@@ -202,7 +202,7 @@ class ServingModel:
                 from kgs.ops.gemm import gemm_nt_w4x
 
                 return gemm_nt_w4x(x, w, bn=route[0], nslice=route[1], bm=route[2], stages=D.w4x_stages(route),
-                                   nt_weights=D.w4x_nt(route, m), private=table is None)
+                                   nt_weights=D.w4x_nt(route), private=table is None)
             # slices whose sum nothing takes: the general kernel's tiles, but for small outputs of a middling K the
             # library's (us at 96 rows, the rule's slices and their sum / general / library: 1024x1024 9.5 / 7.0 / 8.3,
             # 2560x7168 18.9 / 17.7 / 20.3, 5120x5120 25.4 / 21.2 / 27.2; 1024x4096 14.5 / 11.5 / 8.9, 2048x2048 11.8 / 11.1 / 8.5)
@@ -282,7 +282,7 @@ class ServingModel:
         from kgs.ops.gemm import gemm_nt_w4x_partials
 
         w, read = self.w[layer][name], self._w4x_weight(layer, name, r[0])
-        return gemm_nt_w4x_partials(x, read, *r, nt_weights=D.w4x_nt(r, x.shape[0], read is not w),
+        return gemm_nt_w4x_partials(x, read, *r, nt_weights=D.w4x_nt(r, read is not w),
                                     private=private or D.w4x_route(x.shape[0], *w.shape) is None)
 
     def _gate_up_split(self, y, layer: int, r):
@@ -292,7 +292,7 @@ class ServingModel:
         if r[0] == GATE:
             return gemm_gate(y, self.w[layer]["gate_up"], r[2])
         if r[1] > 1:
-            return gemm_nt_w4x_splitk_swiglu(y, self.w[layer]["gate_up"], r[0], r[1], r[2], nt_weights=D.w4x_nt(r, y.shape[0]), private=True)
+            return gemm_nt_w4x_splitk_swiglu(y, self.w[layer]["gate_up"], r[0], r[1], r[2], nt_weights=D.w4x_nt(r), private=True)
         return gemm_nt_w4x_swiglu(y, self._gate_up_weight(layer, r[0]), bn=r[0], bm=r[2], stages=D.w4x_stages(r),
                                   nt_weights=D.w4x_nt(r))
 

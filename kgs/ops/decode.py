@@ -312,23 +312,22 @@ def w4x_stages(route) -> int:
     return route[3] if len(route) > 3 else 2
 
 
-# Whether the four-wave decode products may stream their weights non-temporally (gemm_w4.h AUX 52: B's loads only; the
-# activations, re-read by every workgroup from L2, keep the default policy). KGS_NT_WEIGHTS=0 turns it off.
+# Decode weights are read once per step by one CU each: their loads go
+# non-temporal (gemm_w4.h AUX 52, B's loads only; the activations, re-read by
+# every workgroup from L2, keep the default policy). gate|up at batch 256:
+# 69.1 -> 68.0 us row-major, 67.5 -> 64.9 us tile-panel packed
+# (profiles/r4/decode/README.md); batch-256 serving, two A/B/A passes on one
+# box: 18 247 -> 18 302 output tok/s (profiles/r5/decode/README.md). On by
+# default since round 5: the fault that kept it opt-in in round 4 was the
+# graph memset node of the persistent GEMM's ticket slot, not these loads
+# (profiles/r5/fault/README.md; the nt kernels differ from the default ones
+# only in the nt bit of B's buffer loads). KGS_NT_WEIGHTS=0 turns it off.
 NT_WEIGHTS = os.environ.get("KGS_NT_WEIGHTS", "1") == "1"
 
 
-def w4x_nt(route, packed: bool = False) -> bool:
-    """Whether this route's weights are streamed non-temporally (``packed``: from a tile-panel copy): those of two stages
-    without K slices, or packed.
-
-    A product without slices reads a row-major weight in whole rows per CU and is 3 to 9 % faster so; a slice reads short
-    pieces of its rows, and the default policy is the faster one. us in a chain of launches, weights (700 MB of them)
-    from HBM, non-temporal / default: 28672x4096 gate|up unsliced at 40 / 90 / 256 rows 45.7 / 49.9, 49.3 / 52.1, 63.0 / 67.0,
-    32000x2048 at 100 37.9 / 40.1; in slices at 100 rows 2048x8192 23.4 / 20.0, 16384x2048 28.1 / 23.5, 4096x4096 21.6 / 18.3,
-    3072x2048 16.0 / 15.8 (at 40 11.6 / 11.7), at 200 2048x8192 24.3 / 21.3, 4096x8192 34.5 / 31.7. Launched back to back,
-    with no other kernels between them, the two differ by 2 %. Packed slices gain as much in such a chain (4096x4096 20.6 / 17.7)
-    and not in a whole step (90 prompt rows of hidden 4096 626 to 646 us, 655 by default)."""
-    return NT_WEIGHTS and w4x_stages(route) == 2 and (route[1] == 1 or packed)
+def w4x_nt(route) -> bool:
+    """Stream this route's weights non-temporally (two-stage routes only)."""
+    return NT_WEIGHTS and w4x_stages(route) == 2
 
 
 def w4x_split_bns(n: int, k: int) -> set:

@@ -281,8 +281,8 @@ class ServingModel:
         ``private`` (prompts) and for a size without measured entries."""
         from kgs.ops.gemm import gemm_nt_w4x_partials
 
-        w, read = self.w[layer][name], self._w4x_weight(layer, name, r[0])
-        return gemm_nt_w4x_partials(x, read, *r, nt_weights=D.w4x_nt(r, read is not w),
+        w = self.w[layer][name]
+        return gemm_nt_w4x_partials(x, self._w4x_weight(layer, name, r[0]), *r, nt_weights=D.w4x_nt(r),
                                     private=private or D.w4x_route(x.shape[0], *w.shape) is None)
 
     def _gate_up_split(self, y, layer: int, r):

@@ -140,13 +140,3 @@ def test_rope_forms_by_rows(tokens):
     for a in range(0, tokens, 99):
         D.rope_cache_(one[a:a + 99], cos, sin, pos[a:a + 99].clone(), slot[a:a + 99].clone(), cb, heads, kv)
     assert torch.equal(qkv, one) and torch.equal(ca, cb)
-
-
-def test_sliced_row_major_weights_keep_the_default_cache_policy(monkeypatch):
-    monkeypatch.setattr(D, "NT_WEIGHTS", True)
-    for route in ((128, 1, 128), (128, 8, 128), (128, 8, 256, 2), (128, 4, 128, 3)):
-        stages2, sliced = D.w4x_stages(route) == 2, route[1] > 1
-        assert D.w4x_nt(route) == (stages2 and not sliced)
-        assert D.w4x_nt(route, packed=True) == stages2
-    monkeypatch.setattr(D, "NT_WEIGHTS", False)
-    assert not D.w4x_nt((128, 1, 128))

@@ -23,6 +23,7 @@
 #include "kgs_common.h"
 
 namespace kgs {
+int cu_count();  // gemm_bf16.hip
 namespace latent {
 
 constexpr int PAGE = 32;
@@ -201,12 +202,17 @@ struct ProjArgs {
   const int* pos;  // [Nt]
 };
 
-// D^T[n][token] = W[n][k] a^T[k][token]; wave: 16 outputs x 16 TT tokens of one head
-template <int TT>
+// D^T[n][token] = W[n][k] a^T[k][token]; wave: 16 outputs x 16 TT tokens of one head, D k-steps' loads in flight together.
+// A grid of one workgroup of four waves per CU or fewer is bound by the rounds of loads of a wave and by what one CU can take in:
+// single waves on all CUs then, with K = 512 in one round (D 16) and the gate's loads before them, 32 tokens each. us, 128 outputs of
+// K = 512 of 16 heads, four waves / single ones with D 4 / with D 16: 1 token 5.0 / 4.2 / 3.2, 24 tokens 8.0 / 5.5 / 4.5, of 32 heads 16
+// tokens 6.2 / 4.8 / 3.7; 33 of 32 heads 10.3 with 64 tokens a wave, 8.7 with 32, 5.9 so.
+// More workgroups hide each other's loads and lose by the registers (16 tokens of 128 heads, 512 outputs of K = 128: D 4 6.9, D 16 8.1).
+template <int TT, int D>
 __global__ __launch_bounds__(256) void head_proj(ProjArgs p) {
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int l16 = lane & 15, g = lane >> 4;
-  const int nt = blockIdx.x * 4 + w, h = blockIdx.z, t0 = blockIdx.y * 16 * TT;
+  const int nt = blockIdx.x * (blockDim.x >> 6) + w, h = blockIdx.z, t0 = blockIdx.y * 16 * TT;
   if (nt * 16 >= p.N) {
     const int c = nt * 16 - p.N + 4 * g;
     if (c >= p.hr) return;
@@ -244,20 +250,31 @@ __global__ __launch_bounds__(256) void head_proj(ProjArgs p) {
     const long r = p.idx_in ? p.idx_in[t] : t;
     ap[i] = (const unsigned short*)p.a + r * p.lda + h * p.ha + 8 * g;
   }
+  unsigned short gate[TT][4];
+  if (p.gate) {
+#pragma unroll
+    for (int i = 0; i < TT; ++i) {
+      const int t = min(t0 + 16 * i + l16, p.Nt - 1);
+      const long r = p.idx_out ? p.idx_out[t] : t;
+      const unsigned short* gp = (const unsigned short*)p.gate + r * p.ldg + (long)h * p.hg + (nt * 16 + 4 * g) * p.eg;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) gate[i][j] = gp[j * p.eg];
+    }
+  }
   f32x4 acc[TT];
 #pragma unroll
   for (int i = 0; i < TT; ++i) acc[i] = f32x4{};
-  for (int k = 0; k < p.K; k += 128) {  // four steps' loads are in flight together
-    bf16x8 wf[4], af[4][TT];
+  for (int k = 0; k < p.K; k += 32 * D) {
+    bf16x8 wf[D], af[D][TT];
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+    for (int j = 0; j < D; ++j)
       if (k + 32 * j < p.K) {
         wf[j] = *(const bf16x8*)(wp + k + 32 * j);
 #pragma unroll
         for (int i = 0; i < TT; ++i) af[j][i] = *(const bf16x8*)(ap[i] + k + 32 * j);
       }
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+    for (int j = 0; j < D; ++j)
       if (k + 32 * j < p.K) {
 #pragma unroll
         for (int i = 0; i < TT; ++i)
@@ -271,9 +288,8 @@ __global__ __launch_bounds__(256) void head_proj(ProjArgs p) {
     const long r = p.idx_out ? p.idx_out[t] : t;
     f32x4 s = f32x4{1.0f, 1.0f, 1.0f, 1.0f};
     if (p.gate) {
-      const unsigned short* gp = (const unsigned short*)p.gate + r * p.ldg + (long)h * p.hg + (nt * 16 + 4 * g) * p.eg;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) s[j] = sigmoid(bf2f(gp[j * p.eg]));
+      for (int j = 0; j < 4; ++j) s[j] = sigmoid(bf2f(gate[i][j]));
     }
     uint2 o;
     o.x = pack_bf16x2(acc[i][0] * s[0], acc[i][1] * s[1]);
@@ -335,10 +351,9 @@ constexpr int LEAST_PAGES = 2;  // pages of a part
 
 // Parts by length: all sequences are cut into parts of the same number of pages, the fewest that make at most `parts`
 // of them (and MAX_SPLIT of one), and workgroup i takes part i of the list. The host sees only the block table's width:
-// equal splits of each sequence are as many as its longest needs, the longest one's are the launch's time, and the short ones'
-// workgroups are done or empty. 24 sequences of 60 to 1300 tokens with 16 heads over latents of 512: 14.9 us in equal splits,
-// 10.9 so, and the merge's 4.9 and 4.7; the page's own loads and products are about 2 us of a part, so parts are two pages
-// and more.
+// in equal splits of each sequence the longest one's are the launch's time, and the short ones' workgroups are done or
+// empty. 24 sequences of 60 to 1300 tokens with 16 heads over latents of 512: 14.9 us in equal splits,
+// 10.9 so, and the merge's 4.9 and 4.7.
 struct Part {
   int seq, pos, part, first, count, pages;  // seq -1: none
 };
@@ -871,10 +886,15 @@ KGS_EXPORT int kgs_head_proj(const void* a, const void* w, void* out, const void
   if (N % 16 || K % 32) return KGS_ERR_SHAPE;
   if ((((uintptr_t)a | (uintptr_t)w | (uintptr_t)out) & 15) || (lda | ha) % 8 || (ldo | ho) % 4) return KGS_ERR_ALIGN;
   const int gx = ((N + hr) / 16 + 3) / 4;
-  if (Nt <= 16) hipLaunchKernelGGL(head_proj<1>, dim3(gx, 1, H), dim3(256), 0, s, p);
-  else if (Nt <= 32) hipLaunchKernelGGL(head_proj<2>, dim3(gx, 1, H), dim3(256), 0, s, p);
+  const int ny = (Nt + 31) / 32;
+  const bool few = (long)gx * ny * H <= kgs::cu_count();
+  const int gw = (N + hr) / 16;
+  if (few && Nt <= 16) hipLaunchKernelGGL((head_proj<1, 16>), dim3(gw, 1, H), dim3(64), 0, s, p);
+  else if (few) hipLaunchKernelGGL((head_proj<2, 16>), dim3(gw, ny, H), dim3(64), 0, s, p);
+  else if (Nt <= 16) hipLaunchKernelGGL((head_proj<1, 4>), dim3(gx, 1, H), dim3(256), 0, s, p);
+  else if (Nt <= 32) hipLaunchKernelGGL((head_proj<2, 4>), dim3(gx, 1, H), dim3(256), 0, s, p);
   else if ((Nt + 63) / 64 > 65535) return KGS_ERR_SHAPE;
-  else hipLaunchKernelGGL(head_proj<4>, dim3(gx, (Nt + 63) / 64, H), dim3(256), 0, s, p);
+  else hipLaunchKernelGGL((head_proj<4, 4>), dim3(gx, (Nt + 63) / 64, H), dim3(256), 0, s, p);
   return (int)hipGetLastError();
 }
 

@@ -16,7 +16,7 @@
 //                   the latter with the sigmoid output gate (a number per head or per
 //                   element) in its store;
 //   * attn          rows x pages on v_mfma_f32_16x16x32_bf16, split over the
-//                   context, + merge;
+//                   context, + merge; a decode step's in parts by length, + merge_parts;
 //   * attn_simple   the same on the VALU for any RP and for fp32 caches.
 #include <type_traits>
 

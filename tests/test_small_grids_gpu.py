@@ -65,3 +65,21 @@ def test_small_tiles_by_either_cache_policy(M, N, K):
     want = a.double() @ b.double().T
     assert rc == 0 and bool((c[M] == 7).all())
     assert float((c[:M].double() - want).norm() / want.norm()) < 2.0 ** -8  # one rounding to bf16
+
+
+@pytest.mark.parametrize("m", [17, 31, 32])
+@pytest.mark.parametrize("n,k", [(6272, 2048), (8064, 1024), (8192, 2048)])
+@pytest.mark.parametrize("swiglu", [False, True])
+def test_skinny_products_in_one_round_of_two_tile_workgroups(m, n, k, swiglu):
+    """bf16 outputs of fp32 sums over K: 2^-8 of the largest (a rounding is 2^-9, a fused gate's are two)."""
+    from kgs.ops import decode as D
+
+    g = torch.Generator(device="cuda").manual_seed(n + m)
+    w = (torch.randn(n, k, device="cuda", generator=g) * k ** -0.5).bfloat16()
+    x = torch.randn(m, k, device="cuda", generator=g).bfloat16()
+    assert D.skinny_rule(m, n, k) == (23, 1)
+    got = D.skinny_gemm(x, D.PackedWeight(w, swiglu=swiglu)).double()
+    want = x.double() @ w.double().T
+    if swiglu:
+        want = torch.nn.functional.silu(want[:, :n // 2]) * want[:, n // 2:]
+    assert (got - want).abs().max() < 2.0 ** -8 * want.abs().max()

@@ -796,12 +796,18 @@ def length_parts(batch: int, kv_heads: int, max_pages: int, waves: int, fp8: boo
     return max(1, (192 if groups < CUS or (groups == CUS and not fp8) else 384) // kv_heads)
 
 
+def part_tickets(batch: int, kv_heads: int, max_pages: int, fp8: bool) -> int:
+    """Length of the ``tickets`` that :func:`paged_decode_attention` of such a batch takes, 0: none."""
+    waves = workgroup_waves(batch * kv_heads, max_pages, fp8)
+    return batch * kv_heads if length_parts(batch, kv_heads, max_pages, waves, fp8) else 0
+
+
 _AWS: dict = {}
 
 
 def _attn_workspace(b: int, heads: int, kv_heads: int, nsplit: int, device) -> tuple:
     """(po, pml, cnt) split-merge workspace of the paged decode attention
-    (None x 3 for one split); grown on demand, one per device."""
+    (None x 3 for one split); grown on demand, one per device: calls that share it are ordered by their stream."""
     if nsplit <= 1:
         return None, None, None
     need = b * heads * nsplit
@@ -871,11 +877,14 @@ def rope_paged_decode_attention(partials: torch.Tensor, cos: torch.Tensor, sin: 
 def paged_decode_attention(q: torch.Tensor, cache_layer: torch.Tensor, block_tables: torch.Tensor,
                            ctx_lens: torch.Tensor, heads: int, kv_heads: int, out: torch.Tensor | None = None,
                            scale: float | None = None, pages_per_split: int | None = None,
-                           pipe: bool | None = None) -> torch.Tensor:
+                           pipe: bool | None = None, tickets: torch.Tensor | None = None) -> torch.Tensor:
     """One query token per sequence: ``q`` rows ``[B, >= H*128]`` (e.g. the rotated
     q heads at the front of the fused QKV rows), ``block_tables`` int32
     ``[B, max_pages]``, ``ctx_lens`` int32 ``[B]`` (cached tokens incl. the new
-    one). Returns ``[B, H*128]`` bf16."""
+    one). Returns ``[B, H*128]`` bf16. Parts that follow the lengths (:func:`length_parts`) have partial results of the call's own and take
+    ``tickets``, zeroed int32 of :func:`part_tickets` values or more, which are zero again behind it and so serve every layer of
+    a step (None: the call's own, a launch of 1.5 us more). Contexts split in any other way
+    share one workspace per GPU: calls of such batches on several streams have to be ordered."""
     b = q.shape[0]
     if q.dtype != torch.bfloat16 or not q.is_cuda or q.stride(1) != 1:
         raise ValueError("q must be a row-major bf16 GPU matrix")
@@ -887,9 +896,7 @@ def paged_decode_attention(q: torch.Tensor, cache_layer: torch.Tensor, block_tab
     fp8 = cache_layer.dtype == FP8
     waves = workgroup_waves(b * kv_heads, max_pages, fp8) if pages_per_split is None and pipe is None else 1
     target = length_parts(b, kv_heads, max_pages, waves, fp8)
-    if target:
-        nsplit = 1 + -(-target // b)  # b + target rows of partial results
-    elif waves > 1:
+    if waves > 1:
         nsplit = workgroup_splits(b, kv_heads, max_pages) if b else 1
     elif pages_per_split is None:
         pps, nsplit = decode_splits(b, kv_heads, max_pages)
@@ -897,15 +904,21 @@ def paged_decode_attention(q: torch.Tensor, cache_layer: torch.Tensor, block_tab
         pps, nsplit = pages_per_split, math.ceil(max_pages / pages_per_split)
     if out is None:
         out = torch.empty((b, heads * HEAD_DIM), dtype=torch.bfloat16, device=q.device)
-    po, pml, cnt = _attn_workspace(b, heads, kv_heads, nsplit, q.device)
     scale = 1.0 / math.sqrt(HEAD_DIM) if scale is None else scale
     if target:
+        rows = (b + target) * heads  # of partial results, then their maxima and sums
+        part = torch.empty(rows * (HEAD_DIM + 2), dtype=torch.float32, device=q.device)
+        if tickets is None:
+            tickets = torch.zeros(b * kv_heads, dtype=torch.int32, device=q.device)
+        elif tickets.dtype != torch.int32 or tickets.device != q.device or not tickets.is_contiguous() or tickets.numel() < b * kv_heads:
+            raise ValueError(f"tickets must be {b * kv_heads} contiguous int32 or more on q's GPU")
         rc = _lib.lib().kgs_paged_decode_wg_bal(q.data_ptr(), cache_layer.data_ptr(), block_tables.data_ptr(), ctx_lens.data_ptr(),
-                                                out.data_ptr(), po.data_ptr(), pml.data_ptr(), cnt.data_ptr(), b, heads, kv_heads,
-                                                HEAD_DIM, max_pages, target, PARTS_LEAST, q.stride(0), out.stride(0), float(scale),
-                                                int(fp8), _lib.stream_handle(q.device))
+                                                out.data_ptr(), part.data_ptr(), part.data_ptr() + rows * HEAD_DIM * 4,
+                                                tickets.data_ptr(), b, heads, kv_heads, HEAD_DIM, max_pages, target, PARTS_LEAST,
+                                                q.stride(0), out.stride(0), float(scale), int(fp8), _lib.stream_handle(q.device))
         _lib.check(rc, "paged_decode_attention")
         return out
+    po, pml, cnt = _attn_workspace(b, heads, kv_heads, nsplit, q.device)
     if waves > 1:
         rc = _lib.lib().kgs_paged_decode_wg_ex(q.data_ptr(), cache_layer.data_ptr(), block_tables.data_ptr(), ctx_lens.data_ptr(),
                                                out.data_ptr(), po.data_ptr() if po is not None else None,

@@ -581,7 +581,8 @@ class ServingModel:
 
             if plan.past:
                 k2, v2 = torch.empty((2, plan.past[-1][1], c.kv_heads * hd), dtype=torch.bfloat16, device=tokens.device)
-        x, y = self._start(tokens, plan.keep, norm=not f8)
+        tickets = self._tickets(dec_block_tables) if nd else None
+        x, y = self._start(tokens, plan.keep, not f8, tickets)
         if f8:
             from kgs.ops.transformer import add_rmsnorm_fp8, quantize_rows_fp8, silu_mul_fp8
 
@@ -607,7 +608,7 @@ class ServingModel:
                                                   c.kv_heads).to(torch.bfloat16)
                 else:
                     D.paged_decode_attention(qd, self.cache.layer(i), dec_block_tables, dec_ctx_lens, c.heads,
-                                             c.kv_heads, out=a[n_pf:])
+                                             c.kv_heads, out=a[n_pf:], tickets=tickets)
             nxt = self.ln1[i + 1] if i + 1 < c.layers else self.norm
             if f8:
                 F = self.prefill_f8[i]
@@ -650,7 +651,8 @@ class ServingModel:
         c = self.cfg
         if self.backend == "kgs" and tokens.shape[0] <= self.fused_max_batch:
             return self._decode_fused(tokens, positions, slots, block_tables, ctx_lens, pages_per_split)
-        x, y = self._start(tokens)
+        tickets = self._tickets(block_tables)
+        x, y = self._start(tokens, zero=tickets)
         m = x.shape[0]
         rq, ro, rd = (self._splitk_route(m, 0, n) for n in ("qkv", "o", "down"))  # same shapes in every layer
         rg = self._swiglu_route(m)
@@ -684,7 +686,7 @@ class ServingModel:
                                        c.kv_heads).to(torch.bfloat16)
             else:
                 a = D.paged_decode_attention(qkv, self.cache.layer(i), block_tables, ctx_lens, c.heads, c.kv_heads,
-                                             pages_per_split=pages_per_split)
+                                             pages_per_split=pages_per_split, tickets=tickets)
                 T.op(f"decode L{i} attention")
             if ro:
                 y = splitk_add_rmsnorm(self._split_proj(a, i, "o", ro), x, self.ln2[i], c.eps)
@@ -712,31 +714,45 @@ class ServingModel:
         ss_a / ss_b carry the residual rows' sums of squares between the
         producing GEMM (residual update) and the consuming one (folded RMSNorm)."""
         c = self.cfg
+        tickets = self._tickets(block_tables)
 
         def attend(qkv, i):
             return D.paged_decode_attention(qkv, self.cache.layer(i), block_tables, ctx_lens, c.heads, c.kv_heads,
-                                            pages_per_split=pages_per_split)
+                                            pages_per_split=pages_per_split, tickets=tickets)
 
-        x, ss = self._fused_layers(tokens, positions, slots, attend, "decode", None, exact=False)
+        x, ss = self._fused_layers(tokens, positions, slots, attend, "decode", None, exact=False, tickets=tickets)
         out = D.skinny_gemm(x, self.packed_lm, rms=ss, eps=c.eps)
         T.op("decode-fused lm_head")
         return out
 
-    def _start(self, tokens, keep=None, norm: bool = True):
-        """The residual rows of a step (of the rows ``keep`` of ``tokens``) and, with ``norm``, their norm for the first layer."""
+    def _tickets(self, block_tables):
+        """Tickets of the step's own for the decode rows' attention, to be cleared with its first launch; None: it takes none."""
+        if self.backend != "kgs":
+            return None
+        n = D.part_tickets(block_tables.shape[0], self.cfg.kv_heads, block_tables.shape[1], self.cache.fp8)
+        return torch.empty(n, dtype=torch.int32, device=block_tables.device) if n else None
+
+    def _start(self, tokens, keep=None, norm: bool = True, zero=None):
+        """The residual rows of a step (of the rows ``keep`` of ``tokens``) and, with ``norm``, their norm for the first layer;
+        ``zero`` is cleared."""
         from kgs.ops.transformer import embed_rows, embeds
 
         if self.backend == "kgs" and embeds(self.embed):
-            return embed_rows(self.embed, tokens, self.ln1[0] if norm else None, self.cfg.eps, keep)[:2]
+            return embed_rows(self.embed, tokens, self.ln1[0] if norm else None, self.cfg.eps, keep,
+                              zeros=() if zero is None else (zero,))[:2]
+        if zero is not None:
+            zero.zero_()
         tokens = tokens.reshape(-1) if keep is None else tokens.reshape(-1)[keep.long()]
         x = self.embed[tokens.long()].reshape(-1, self.cfg.hidden).contiguous()
         return x, self._norm(x, None, self.ln1[0]) if norm else None
 
-    def _fused_layers(self, tokens, positions, slots, attend, kind: str, counters, exact: bool, keep=None):
+    def _fused_layers(self, tokens, positions, slots, attend, kind: str, counters, exact: bool, keep=None,
+                      tickets=None):
         """The residual rows after all layers and their sums of squares; ``attend(qkv, layer)`` is the
         attention of the rotated rows, whose keys and values are in the cache. ``exact``: statistics whose
         bits do not depend on the order in which workgroups arrive, so that equal steps give equal bits. ``keep``
-        (int32): of these rows of ``tokens``, ``positions`` and ``slots`` only. ``counters``: the step's own, cleared here."""
+        (int32): of these rows of ``tokens``, ``positions`` and ``slots`` only. ``counters`` and
+        ``tickets``: the step's own, cleared here (not both of them)."""
         from kgs.ops.transformer import embed_rows, embeds
 
         c = self.cfg
@@ -749,7 +765,7 @@ class ServingModel:
         else:
             zero = ss_a = torch.empty_like(ss)
             ss_b = ss
-        clear = (zero,) if counters is None else (zero, counters)
+        clear = tuple(t for t in (zero, counters, tickets) if t is not None)
         if embeds(self.embed):
             x, _, positions, slots = embed_rows(self.embed, tokens, None, eps, keep, ss, positions, slots, clear)
         else:

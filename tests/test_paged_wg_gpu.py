@@ -185,3 +185,45 @@ def test_length_rule_has_room_for_its_parts():
                 n = length_parts(batch, kv, 64, 4 if fp8 else 8, fp8)
                 assert (n > 0) == (2 < batch <= 128) and n * kv <= max(384, kv)
                 assert length_parts(batch, kv, 63, 4 if fp8 else 8, fp8) == 0 == length_parts(batch, kv, 64, 2, fp8)
+
+
+def test_parts_keep_their_scratch_to_the_call(monkeypatch):
+    """Batches that had no split before their parts followed the lengths shared nothing with other calls, nor do they now: steps
+    of different lengths on two streams, and between a graph's replays, with tickets given and without."""
+    from kgs.ops import decode as D
+
+    monkeypatch.setattr(D, "_attn_workspace", lambda *a: pytest.fail("workspace of the whole GPU"))
+    g = torch.Generator().manual_seed(1)
+    sets = []
+    for _ in range(4):
+        lens = torch.randint(1, 700, (64,), generator=g).tolist()
+        lens[5] = 2040
+        sets.append(setup(lens, 8, 2, seed=len(sets)))
+    assert D.length_parts(64, 8, sets[0][2].shape[1], 8, False) and D.part_tickets(64, 8, sets[0][2].shape[1], False) == 512
+    want = [D.paged_decode_attention(*s, 16, 8) for s in sets]
+    for w, s in zip(want, sets):
+        assert float((w.float() - D.ref_paged_decode(*s, 16, 8)).abs().max()) < TOL
+    tickets = [torch.zeros(512, dtype=torch.int32, device=DEV) for _ in sets]
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    torch.cuda.synchronize()
+    got = []
+    for n in range(10):
+        for i, s in enumerate(sets):
+            with torch.cuda.stream(streams[i % 2]):
+                got.append((i, D.paged_decode_attention(*s, 16, 8, tickets=tickets[i % 2] if n % 2 else None)))
+    torch.cuda.synchronize()
+    assert all(torch.equal(o, want[i]) for i, o in got) and not any(bool(t.any()) for t in tickets)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = D.paged_decode_attention(*sets[0], 16, 8)
+    for _ in range(4):
+        out.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        with torch.cuda.stream(streams[0]):
+            other = D.paged_decode_attention(*sets[1], 16, 8)
+        torch.cuda.synchronize()
+        assert torch.equal(out, want[0]) and torch.equal(other, want[1])
+    for bad in (tickets[0][:511], tickets[0].long(), tickets[0].cpu(), torch.zeros(1024, dtype=torch.int32, device=DEV)[::2]):
+        with pytest.raises(ValueError):
+            D.paged_decode_attention(*sets[0], 16, 8, tickets=bad)

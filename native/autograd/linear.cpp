@@ -9,7 +9,7 @@
 // that run on transposed copies (tr_slices 0: such sizes keep the GPU busy for longer than the
 // host), operands that only the element-wise kernel reads, empty ones, and whatever has to see a Python
 // function (tracing, functorch transforms, forward-mode tangents, dispatch modes, tensor subclasses).
-#include <ATen/FuncTorchTLS.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/jit/frontend/tracer.h>
@@ -187,12 +187,17 @@ struct LinearNode : torch::autograd::Function<LinearNode> {
   }
 };
 
+// A functorch transform is running on this thread (its thread-local storage stays behind when it has ended)
+bool transforming() {
+  return c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode) ||
+         c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerBackMode);
+}
+
 // act(x . w^T + bias), or None where kgs/ops/gemm.py's _LinearFn has to run it (or say what is wrong)
 std::optional<at::Tensor> linear(const at::Tensor& x, const at::Tensor& w, const std::optional<at::Tensor>& b, int64_t act) {
   const at::Tensor bias = b ? *b : at::Tensor();
   if (!(act == NONE || (act >= GELU && act <= SILU)) || !plain(x, 2) || !plain(w, 2) || (b && !plain(bias, 1))) return {};
-  if (torch::jit::tracer::isTracing() || at::functorch::functorchTLSAccessor() || c10::impl::TorchDispatchModeTLS::any_modes_set())
-    return {};
+  if (torch::jit::tracer::isTracing() || transforming() || c10::impl::TorchDispatchModeTLS::any_modes_set()) return {};
   const long m = x.size(0), k = x.size(1), n = w.size(0), lim = 1L << 22;
   if (w.size(1) != k || w.device() != x.device() || (b && (bias.numel() != n || bias.device() != x.device()))) return {};
   if (m >= 1L << 24 || x.stride(0) < k || w.stride(0) < k || std::max({n, x.stride(0), w.stride(0)}) >= lim) return {};

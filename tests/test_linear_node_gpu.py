@@ -101,8 +101,23 @@ def test_python_only_calls_keep_their_answers():
                 lambda f: f(x.float(), w, b, None), lambda f: f(x, w, b[:8], "gelu"), lambda f: f(x, w, b, "tanh")):
         assert refusal(lambda: how(linear)) == refusal(lambda: how(_LinearFn.apply))
         assert refusal(lambda: how(linear)) is not None
+    assert "LinearNode" in linear(x, w, b, "gelu").grad_fn.name()  # nothing stays behind of the refused ones
     graph = torch.jit.trace(lambda *v: linear(*v, "gelu"), tuple(t.detach() for t in (x, w, b)), check_trace=False).graph
     assert "_LinearFn" in str(graph)
+
+
+def test_transforms_leave_nothing_behind():
+    """Inside a transform the Python function, which has no rule for one; after it the node again."""
+    from kgs.ops.gemm import linear
+
+    x, w, b = leaves(64, 128, 256, True)
+    one = torch.ones(3, device=DEV)
+    for transform in (lambda f: torch.vmap(f)(one), lambda f: torch.func.grad(lambda v: f(v).sum())(one), lambda f: torch.func.jvp(f, (one,), (one,))):
+        transform(lambda v: v * 2)
+        assert "LinearNode" in linear(x, w, b, "gelu").grad_fn.name()
+        with pytest.raises(RuntimeError, match="setup_context"):
+            transform(lambda v: linear(x, w, b, "gelu").sum() * v)
+        assert "LinearNode" in linear(x, w, b, "gelu").grad_fn.name()
 
 
 def test_backward_of_streams_threads_and_graphs():
@@ -111,7 +126,9 @@ def test_backward_of_streams_threads_and_graphs():
     from kgs.ops.gemm import linear
 
     def step(x, w, b, gy):
-        return torch.autograd.grad(linear(linear(x, w, b, "gelu"), w, b, "silu"), (x, w, b), gy)
+        y = linear(linear(x, w, b, "gelu"), w, b, "silu")
+        assert "LinearNode" in y.grad_fn.name()
+        return torch.autograd.grad(y, (x, w, b), gy)
 
     sets = [(*leaves(96, 256, 256, True), rnd(96, 256)) for _ in range(4)]
     want = [step(*s) for s in sets]

@@ -12,6 +12,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+import warnings
 from functools import lru_cache
 from pathlib import Path
 
@@ -215,12 +216,15 @@ def lib() -> ctypes.CDLL:
 
 @lru_cache(maxsize=1)
 def autograd():
-    """The native autograd nodes (``native/autograd``), on the kernels of :func:`lib`."""
+    """The native autograd nodes (``native/autograd``), on the kernels of :func:`lib`. None, with a warning, where they cannot be
+    loaded (built for another torch or Python): the Python functions run the same kernels."""
     so = lib()
     try:
         from .._native import _autograd
     except ImportError as e:
-        raise NativeUnavailable(f"cannot load kgs/_native/_autograd: {e}; build it with `python -m kgs.utils.build`") from e
+        warnings.warn(f"cannot load kgs/_native/_autograd, small training layers take about twice as long: {e}; build it with "
+                      "`python -m kgs.utils.build`", RuntimeWarning, stacklevel=2)
+        return None
     names = ("kgs_gemm_bf16_nt_auto", "kgs_gemm_bf16_nt_padded", "kgs_gemm_bf16_nt_act", "kgs_pad_rows_bf16", "kgs_act_grad",
              "kgs_gemm_bf16_tr", "kgs_gemm_bf16_nt_scratch", "kgs_gemm_bf16_nt_padded_scratch", "kgs_act_grad_parts",
              "kgs_gemm_bf16_tr_slices")

@@ -848,7 +848,8 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None, a
     """Differentiable ``act(x @ w.T + bias)`` on the HIP GEMM (x: [M,K], w: [N,K]): by the native node
     (``native/autograd/linear.cpp``) where the host bounds the layer, else by :class:`_LinearFn`."""
     if x.is_cuda and act in EPI:
-        y = _lib.autograd().linear(x, w, bias, EPI[act])
+        nodes = _lib.autograd()
+        y = None if nodes is None else nodes.linear(x, w, bias, EPI[act])
         if y is not None:
             return y
     return _LinearFn.apply(x, w, bias, act)

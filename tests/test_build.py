@@ -103,3 +103,22 @@ def test_manifest_check_names_a_stale_library(tmp_path):
     assert not r["ok"] and "inputs changed" in r["targets"]["one"] and str(src) in r["targets"]["one"]
     Path(t.output).write_bytes(b"not the recorded library")
     assert check_manifest(tmp_path)["targets"]["one"] == "output differs from the recorded build"
+
+
+def test_layers_run_without_the_native_node(monkeypatch):
+    """Nodes that cannot be loaded (another torch) or built (a torch without HIP) are reported and done without."""
+    import sys
+
+    import kgs._native
+    from kgs.ops import _lib
+    from kgs.utils.build import targets
+
+    assert next(t for t in targets() if t.name == "autograd").optional
+    monkeypatch.delattr(kgs._native, "_autograd", raising=False)
+    monkeypatch.setitem(sys.modules, "kgs._native._autograd", None)
+    _lib.autograd.cache_clear()
+    try:
+        with pytest.warns(RuntimeWarning, match="_autograd"):
+            assert _lib.autograd() is None
+    finally:
+        _lib.autograd.cache_clear()

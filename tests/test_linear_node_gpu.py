@@ -43,6 +43,20 @@ def test_same_bits(act, rows, din, dout, bias):
                            _LinearFn.apply(x.detach(), w.detach(), None if b is None else b.detach(), act))
 
 
+def test_without_the_node(monkeypatch):
+    from kgs.ops import _lib
+    from kgs.ops.gemm import linear
+
+    x, w, b = leaves(64, 512, 256, True)
+    gy = rnd(64, 256)
+    want = linear(x, w, b, "gelu")
+    monkeypatch.setattr(_lib, "autograd", lambda: None)
+    got = linear(x, w, b, "gelu")
+    assert "_LinearFn" in got.grad_fn.name() and torch.equal(got, want)
+    for g, t in zip(torch.autograd.grad(got, (x, w, b), gy), torch.autograd.grad(want, (x, w, b), gy)):
+        assert torch.equal(g, t)
+
+
 def test_rows_apart_and_large_products_keep_their_ways():
     from kgs.ops.gemm import _LinearFn, linear
 

@@ -81,11 +81,11 @@ def embed_rows(table: torch.Tensor, tokens: torch.Tensor, w: torch.Tensor | None
     rows = tokens.numel() if keep is None else keep.numel()
     given = [t for t in (keep, positions, slots) if t is not None]
     if tokens.device != dev or any(t.dtype != torch.int32 or t.device != dev or not t.is_contiguous() for t in given) or \
-            any(t.numel() != tokens.numel() for t in (positions, slots) if t is not None):
-        raise ValueError("tokens, keep, positions and slots must be int32 vectors on the table's GPU, the last two as long as tokens")
+            any(t.numel() < tokens.numel() for t in (positions, slots) if t is not None):
+        raise ValueError("tokens, keep, positions and slots must be int32 vectors on the table's GPU, the last two no shorter than tokens")
     if w is not None and (w.shape != (cols,) or w.dtype != torch.bfloat16 or not w.is_contiguous() or w.device != dev):
         raise ValueError("w must be a contiguous bf16 vector of length cols")
-    if squares is not None and (squares.dtype != torch.float32 or squares.shape != (rows,) or not squares.is_contiguous()):
+    if squares is not None and (squares.dtype != torch.float32 or squares.shape != (rows,) or not squares.is_contiguous() or squares.device != dev):
         raise ValueError("squares must be a contiguous fp32 vector, one a row")
     words = [t.numel() * t.element_size() // 4 for t in zeros]
     if len(words) > 2 or any(not t.is_contiguous() or t.device != dev or t.element_size() % 4 for t in zeros):

@@ -738,7 +738,7 @@ class ServingModel:
         from kgs.ops.transformer import embed_rows, embeds
 
         if self.backend == "kgs" and embeds(self.embed):
-            return embed_rows(self.embed, tokens, self.ln1[0] if norm else None, self.cfg.eps, keep,
+            return embed_rows(self.embed, tokens.to(self.embed.device), self.ln1[0] if norm else None, self.cfg.eps, keep,
                               zeros=() if zero is None else (zero,))[:2]
         if zero is not None:
             zero.zero_()
@@ -757,7 +757,8 @@ class ServingModel:
 
         c = self.cfg
         eps = c.eps
-        m, dev = (tokens if keep is None else keep).numel(), tokens.device
+        tokens, dev = tokens.to(self.embed.device), self.embed.device
+        m = (tokens if keep is None else keep).numel()
         ss = torch.empty(m, dtype=torch.float32, device=dev)  # statistic for layer 0's qkv
         if exact:
             zero = stats = torch.empty((2, D.SUM_WORDS, m), dtype=torch.int64, device=dev)
@@ -767,6 +768,8 @@ class ServingModel:
             ss_b = ss
         clear = tuple(t for t in (zero, counters, tickets) if t is not None)
         if embeds(self.embed):
+            if keep is not None:
+                positions, slots = positions.reshape(-1).contiguous(), slots.reshape(-1).contiguous()
             x, _, positions, slots = embed_rows(self.embed, tokens, None, eps, keep, ss, positions, slots, clear)
         else:
             if keep is not None:

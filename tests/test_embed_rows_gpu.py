@@ -69,3 +69,31 @@ def test_what_it_refuses_and_replays():
         graph.replay()
         assert torch.equal(x, emb[[t] * 4]) and not z.any()
         torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("batch", [5, 70])  # the fused layer, the split tiles
+def test_steps_take_what_indexing_took(batch):
+    """Tokens in host memory, positions and slots of a longer batch, prompts' positions and slots from columns of a matrix."""
+    from kgs.models.llama import LlamaConfig
+    from kgs.serve.model import ServingModel
+
+    m = ServingModel(LlamaConfig(hidden=1024, layers=1, heads=8, kv_heads=1, intermediate=512, vocab=512), device="cuda", num_pages=64,
+                     max_model_len=512)
+    i32 = dict(dtype=torch.int32, device=DEV)
+    tokens, pos = torch.randint(0, 512, (batch,), **i32), torch.zeros(batch, **i32)
+    slots, tables, ctx = torch.full((batch,), -1, **i32), torch.zeros(batch, 1, **i32), torch.ones(batch, **i32)
+    want = m.decode(tokens, pos, slots, tables, ctx).float()
+
+    def same(got):
+        # the fused layer adds its rows' squares in the order of arrival
+        assert float((got.float() - want).norm() / want.norm()) < 1e-2
+
+    same(m.decode(tokens.cpu(), pos, slots, tables, ctx))
+    same(m.decode(tokens.long(), pos, slots, tables, ctx))
+    if batch < 48:
+        same(m.decode(tokens, torch.cat([pos, pos]), torch.cat([slots, slots]), tables, ctx))
+        n = 32
+        prompt, at, to = torch.randint(0, 512, (n,), **i32), torch.arange(n, **i32), torch.arange(n, **i32) + 32
+        cols = torch.stack([at, to], 1)
+        assert not cols[:, 0].is_contiguous()
+        assert torch.equal(m.prefill(prompt, cols[:, 0], cols[:, 1], [0], [20], [32]), m.prefill(prompt, at, to, [0], [20], [32]))

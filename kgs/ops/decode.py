@@ -393,7 +393,8 @@ def skinny_rule(m: int, n: int, k: int, one: bool = False) -> tuple[int, int]:
     The K split inside the workgroup (16 rows of W each, no slabs in memory and no ticket, 2 to 3 us
     of a launch) where its strips are a workgroup per CU or so: up to 6144 rows, two tiles a wave
     above 4096 from 17 rows of x on; at 17 to 32 rows of x and K up to 2048 to 8192, one round of two-tile workgroups (us at 24 rows, slabs /
-    so: 8192x2048 13.5 / 10.9, 6656x2048 13.2 / 11.1, 8192x1024 10.2 / 7.0; 10240x2048, where it is a second round, 13.5 / 14.3). Every workgroup reads all of x, which bounds K by the rows: up to 16 rows K of
+    so: 8192x2048 13.5 / 10.9, 6656x2048 13.2 / 11.1, 8192x1024 10.2 / 7.0; 10240x2048, where it is a second round, 13.5 / 14.3), in one tile a wave (``one``: weights packed with
+    RoPE), which is a second round there, up to 48k values of x (17 rows of 8192x2048 13.8 / 11.1, 24 14.0 / 13.5, 32 14.0 / 14.7; 32 of x1024 10.7 / 8.7). Every workgroup reads all of x, which bounds K by the rows: up to 16 rows K of
     8192 (in two halves where that is no second round of workgroups; else, from 64k values of x on, only where slabs
     would not fill three quarters of the CUs), of 32k values where the strips are more than the CUs; up to 32 rows K of
     4096 (96k values on less than half of the CUs and in two tiles a wave); beyond them 160k values; from 17 rows on
@@ -407,7 +408,7 @@ def skinny_rule(m: int, n: int, k: int, one: bool = False) -> tuple[int, int]:
     shorter than 512 (1024x4096 at 48 rows 15.5 / 18.0 in 16 slices; 3584x3584 at 24 in one 18.9, in two 15.1)."""
     mt = _mt(m)
     strips = n // 16
-    if mt <= 4 and k % 1024 == 0 and n % 32 == 0 and strips <= (512 if mt == 2 and k <= 2048 else 384):
+    if mt <= 4 and k % 1024 == 0 and n % 32 == 0 and strips <= (512 if mt == 2 and k <= 2048 and (not one or m * k <= 48 << 10) else 384):
         over = strips > CUS
         wide = mt > 1 and over and not one
         v = {1: 20, 2: 23 if wide else 22, 4: 25 if wide else 24}[mt]

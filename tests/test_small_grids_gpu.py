@@ -78,6 +78,8 @@ def test_skinny_products_in_one_round_of_two_tile_workgroups(m, n, k, swiglu):
     w = (torch.randn(n, k, device="cuda", generator=g) * k ** -0.5).bfloat16()
     x = torch.randn(m, k, device="cuda", generator=g).bfloat16()
     assert D.skinny_rule(m, n, k) == (23, 1)
+    # weights packed with RoPE: one tile a wave, a second round of workgroups
+    assert D.skinny_rule(m, n, k, one=True) == ((22, 1) if m * k <= 48 << 10 else (5, 2))
     got = D.skinny_gemm(x, D.PackedWeight(w, swiglu=swiglu)).double()
     want = x.double() @ w.double().T
     if swiglu:

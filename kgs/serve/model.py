@@ -60,6 +60,17 @@ def gate_up_panel_widths(n: int, k: int) -> set:
     return {r[0] for (_, rn, rk), r in D.W4X_TUNED.items() if (rn, rk) == (n, k) and r[1] == 1}
 
 
+def head_on_small_tiles(m: int, n: int, k: int) -> bool:
+    """Whether ``m`` rows of an LM head ``[n, k]`` go by the general kernel's small tiles and not by the library.
+
+    Up to 32 rows of large vocabularies, which they read once and past the caches. us, library / so, 1 row: 32000x4096 58 / 47, 16384x2048
+    18 / 16, 128256x2048 119 / 83; 32 rows 32000x2048 35 / 30, 64000x4096 118 / 90. Not below 16384 (1 row of 8192x4096 16.7 / 18.8, 12288x8192 40.6 / 43.6,
+    5000x8192 19.9 / 23.4), nor where the rows' products are no longer hidden by the reads and the library has larger tiles that
+    fit (32 rows of 18432x3072 28.7 / 33.4, 16 of 50432x5120 90.8 / 96.5, 32 of 50257x1024, whose outputs are not aligned, 23.5 /
+    26.2). Worst within the rule: 1 row of 20480x8192 67.7 / 71.3, 32 of 18432x2048 22.1 / 22.8."""
+    return 0 < m <= 32 and n >= 16384 and n % 8 == 0 and (k <= 2048 or k % 4096 == 0 or (m <= 16 and k <= 4096))
+
+
 class _PromptRows:
     """Rows of a step's layers: ``n`` of them, ``last`` (int32) those whose logits are wanted, attention
     ``items`` (and ``merges``, ``slots`` of their parts) with the gathered contexts ``past`` ``(first row, end, tokens, portion)``, and, where
@@ -226,8 +237,7 @@ class ServingModel:
         # the LM head (N = 128256) from batch 128 up runs faster on the kgs
         # 256x256 GEMM than on hipBLASLt (1.09x at 128, 1.21x at 256,
         # profiles/decode_wide_gemm.jsonl); the other decode shapes do not
-        # up to 32 rows of it on the general kernel's small tiles (us, library / so: 32000x4096 62 / 48, 32000x2048 35 / 31)
-        if decode and (layer is not None or 32 < m < 128):
+        if decode and (layer is not None or m < 128) and not (layer is None and head_on_small_tiles(m, *w.shape)):
             return torch.matmul(x, w.T)
         from kgs.ops import gemm_nt
 

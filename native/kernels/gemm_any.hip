@@ -811,12 +811,14 @@ inline Plan refine(Plan p, long M, long N, long K, int cus, bool sw = false) {
 }
 
 // Whether a product that the aligned, the persistent or the eight-wave 256x256 kernels take is better off on refine's
-// tile here: those keep a little (persistent tiles 3 % on average, 9 % at most) that a tile has to win back first. Of rows off
-// the 128-byte lines (wide below), us by eight waves / so: 1598 x 5680 x 4144 87 / 72, 2310 x 3384 x 8568 165 / 130, where
-// the estimate promises 8 % 3567 x 15328 x 928 108 / 111, 1505 x 8296 x 4336 103 / 98.
-inline bool finer(long M, long N, long K, int cus, bool sw = false) {
+// tile here: those keep a little (persistent tiles 3 % on average, 9 % at most) that a tile has to win back first. Of 90 such products whose estimate
+// promises 7 to 20 % the tile is 6 % faster on average, 4 % slower at worst (2902 x 13312 x 1536 107 / 112 us, ragged rows). off: rows off the
+// 128-byte lines (wide below), where a K-step waits for twice the lines: 20 % have to be promised. us by eight waves / so: 2129 x 3728 x 4616
+// 103 / 89 (27 %), 1598 x 5680 x 4144 87 / 86 (22 %); below, what 55 products gain 1 % from on average 7756 x 6320 x 3816 loses 7 % of (349 / 372),
+// 3567 x 15328 x 928 6 % (108 / 114).
+inline bool finer(long M, long N, long K, int cus, bool sw = false, bool off = false) {
   const Plan p = refine({256, 256, 1}, M, N, K, cus, sw);
-  return p.bm * p.bn < 65536 && tile_cost(p.bm, p.bn, M, N, K, cus) < 0.93 * tile_cost(TILES[0], M, N, K, cus);
+  return p.bm * p.bn < 65536 && tile_cost(p.bm, p.bn, M, N, K, cus) < (off ? 0.80 : 0.93) * tile_cost(TILES[0], M, N, K, cus);
 }
 
 // Whether 256x256 tiles are plan's choice, or so near it that the eight-wave kernel of such tiles
@@ -1086,7 +1088,7 @@ int gemm_any_f8(const void* A, const void* B, void* C, const void* bias, int M, 
   return (int)hipGetLastError();
 }
 
-bool gemm_any_finer(int M, int N, int K, bool sw) { return any::finer(M, N, K, cu_count(), sw); }
+bool gemm_any_finer(int M, int N, int K, bool sw, bool off) { return any::finer(M, N, K, cu_count(), sw, off); }
 
 bool gemm_any_wide(int M, int N, int K, bool split) { return any::wide(M, N, K, split, cu_count()); }
 
@@ -1120,6 +1122,11 @@ KGS_EXPORT int kgs_gemm_bf16_tr(const void* A, const void* B, void* C, int M, in
   if (M <= 0 || N <= 0 || K <= 0 || ldc < N || ns < 1 || ns > 64) return KGS_ERR_SHAPE;
   if (!kgs::gemm_tr_ok(A, B, M, N, K, lda, ldb, ta, tb) || (uintptr_t)ws % 16) return KGS_ERR_ALIGN;
   return kgs::gemm_tr(A, B, C, M, N, K, lda, ldb, ldc, ta, tb, ns, ws, s);
+}
+
+// Whether the kernels of 256x256 tiles leave a product (gated: of a gated projection; off: A's rows off the 128-byte lines) to a finer tile.
+KGS_EXPORT int kgs_gemm_bf16_nt_finer(int M, int N, int K, int gated, int off) {
+  return M > 0 && N > 0 && K > 0 && kgs::gemm_any_finer(M, N, K, gated != 0, off != 0);
 }
 
 // Whether a K-major B is better transposed first than read by kgs_gemm_bf16 (turn_b).

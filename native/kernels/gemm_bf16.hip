@@ -171,7 +171,7 @@ int gemm_any(const void* A, const void* B, void* C, void* C2, const void* bias, 
              int ldc, int epi, int bm, int bn, int ns, float* ws, hipStream_t s);
 long gemm_any_ws(int M, int N, int K);
 bool gemm_any_wide(int M, int N, int K, bool split);
-bool gemm_any_finer(int M, int N, int K, bool sw);
+bool gemm_any_finer(int M, int N, int K, bool sw, bool off);
 int gemm_any_f8(const void* A, const void* B, void* C, const void* bias, int M, int N, int Kw, int lda, int ldb, int ldc,
                 float alpha, const float* alpha_ptr, int epi, hipStream_t s);
 int gemm_any_swiglu(const void* A, const void* B, void* C, int M, int N, int K, int lda, int ldb, int ldc, int act,
@@ -191,13 +191,13 @@ static bool rows_ok(const void* A, const void* B, const void* C, int M, int N, i
   if (M <= 0 || N % 256 || K % 128 || K < 384 || (lda | ldb | ldc) % 8) return false;
   if (((uintptr_t)A | (uintptr_t)B | (uintptr_t)C) % 16) return false;
   if ((long)lda * 512 >= (1L << 31) || (long)ldb * 512 >= (1L << 31)) return false;
-  return ((long)M + 255) / 256 * (N / 256) > cu_count() && !gemm_any_finer(M, N, K, sw);
+  return ((long)M + 255) / 256 * (N / 256) > cu_count() && !gemm_any_finer(M, N, K, sw, false);
 }
 
 // Aligned products of up to one 256x256 tile per CU that a finer tile fills better. Above that they stay on the
 // persistent kernel, on which the tests of its ticket slots and captured graphs launch such sizes through gemm_nt.
 static bool aligned_finer(int M, int N, int K) {
-  return (long)(M / 256) * (N / 256) <= cu_count() && gemm_any_finer(M, N, K, false);
+  return (long)(M / 256) * (N / 256) <= cu_count() && gemm_any_finer(M, N, K, false, false);
 }
 
 template <int EPI>
@@ -391,7 +391,7 @@ static int gemm_nt(const void* A, const void* B, void* C, const void* bias, int 
     // that nothing hides (us, its / the element-wise kernel's: 8192 x 8191 x 128 165 / 131, 3000 x 8001 x 64 65 / 50,
     // 6272 x 3085 x 128 55 / 49, x 256 57 / 56, x 512 66 / 71; 2048 x 3001 x 128 21 / 21)
     const bool short_odd = (ldc % 8 || (uintptr_t)C % 16) && K <= 256 && (long)M * N >= 1L << 23;
-    const bool off = !large && bounded && kgs_gemm_bf16_nt_off_lines(A, M, N, K, lda, ws != nullptr) && !kgs::gemm_any_finer(M, N, K, false);
+    const bool off = !large && bounded && kgs_gemm_bf16_nt_off_lines(A, M, N, K, lda, ws != nullptr) && !kgs::gemm_any_finer(M, N, K, false, true);
     if (!large && !short_odd && !off && kgs::gemm_any_ok(A, B, M, N, K, lda, ldb))
       return kgs::gemm_any(A, B, C, nullptr, bias, M, N, K, lda, ldb, ldc, epi, 0, 0, 0, ws, stream);
     v = large ? 3 : off ? 16 : 2;

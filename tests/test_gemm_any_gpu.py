@@ -426,6 +426,15 @@ def test_large_odd_outputs_of_short_sums(M, N, K, short, act):
     assert rel(got, want) < 2 * REL and rel(plain, want) < 2 * REL
 
 
+@pytest.mark.parametrize("M,N,K,off,taken", [(1598, 5680, 4144, 1, True), (2129, 3728, 4616, 1, True), (3567, 15328, 928, 1, False), (1505, 8296, 4336, 1, False),
+                                              (3567, 15328, 928, 0, True), (4467, 4608, 7296, 0, True), (2048, 5120, 2048, 0, True), (8192, 8192, 8192, 0, False)])
+def test_finer_tiles_where_they_win(M, N, K, off, taken):
+    """Rows off the 128-byte lines leave the eight-wave kernel for more than others leave theirs."""
+    from kgs.ops import _lib
+
+    assert _lib.lib().kgs_gemm_bf16_nt_finer(M, N, K, 0, off) == taken
+
+
 @pytest.mark.parametrize("M,N,K,pad,off,taken", [(2560, 3912, 264, 0, 0, True), (2560, 3912, 248, 0, 0, False), (2576, 3584, 712, 0, 0, True), (2576, 3584, 704, 0, 0, False), (2576, 3584, 704, 8, 0, True),
                                                  (2576, 3584, 704, 0, 8, True), (1500, 12344, 3080, 0, 0, True), (259, 264, 264, 0, 0, False)])
 @pytest.mark.parametrize("act", [None, "gelu", "silu"])

@@ -318,8 +318,8 @@ __global__ __launch_bounds__(256) void gemm_small(Args a) {
     for (int j = 0; j < LA; ++j)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (KGS_LDS void*)(dst + (j * 4 + w) * 1024), 16, oa, j * sa + t * 128, 0, 0);
     // B is read once, whole lines at a time: non-temporal loads, 5.9 TB/s of a large B where the default policy reaches 5.0 (off
-    // the 128-byte lines each would come twice: 64 x 3000 x 1032 9.1 / 12.1 us)
-    if (ntm == 1 && a.ldb % 64 == 0) {
+    // the 128-byte lines each would come twice: 64 x 3000 x 1032 9.1 / 12.1 us; of a few tiles they cost 0.2: 17 x 448 x 256 3.4 / 3.6)
+    if (ntm == 1 && ntn >= 64 && a.ldb % 64 == 0) {
 #pragma unroll
       for (int j = 0; j < LB; ++j)
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (KGS_LDS void*)(dst + BM * 128 + (j * 4 + w) * 1024), 16, ob, j * sb + t * 128, 0, 2);
@@ -750,13 +750,14 @@ inline Plan plan(long M, long N, long K, bool split, int cus) {
         best = {s[0], s[1], ns};
       }
     }
-  if (M <= 64) t0 = t0 > 4 + 2.0 * N * K / 5.0e6 ? t0 : 4 + 2.0 * N * K / 5.0e6;  // few rows: B's way from memory
-  // 64x64 tiles: a cheaper step, twice as many bytes per product; several share a CU. Up to 64 rows B is read once, past
+  // 64x64 tiles: a cheaper step, twice as many bytes per product; several share a CU. Up to 64 rows a B of whole 128-byte lines is read once, past
   // the caches, where there are tiles for most CUs: us at 1 to 16 rows by larger tiles / so 32000x4096 57 / 45, 32000x2048 33 / 28,
-  // 14336x4096 28 / 25, 128256x4096 at 40 192 / 179, but at 64 196 / 207
+  // 14336x4096 28 / 25, 128256x4096 at 40 192 / 179, but at 64 196 / 207; off the lines each line comes twice, 89600x1872 at 32 78 / 83
+  const bool few = M <= 64 && K % 64 == 0;
+  if (few) t0 = t0 > 4 + 2.0 * N * K / 5.0e6 ? t0 : 4 + 2.0 * N * K / 5.0e6;  // few rows: B's way from memory
   const double full = (double)ceil_div(M, 64) * ceil_div(N, 64) / cus, steps = ceil_div(K, 64);
-  const double t = M <= 64 && full >= 0.75 && (M <= 48 || full <= 4) ? 4 + steps * (full <= 1 ? 0.20 + 0.13 * full : 0.33 * full)
-                                                                     : 3.5 + steps * (full <= 1 ? 0.34 + 0.06 * full : 0.06 + (M <= 64 ? 0.43 : 0.38) * full);
+  const double t = few && full >= 0.75 && (M <= 48 || full <= 4) ? 4 + steps * (full <= 1 ? 0.20 + 0.13 * full : 0.33 * full)
+                                                                 : 3.5 + steps * (full <= 1 ? 0.34 + 0.06 * full : 0.06 + (few ? 0.43 : 0.38) * full);
   if (t < t0) best = {64, 64, 1};
   return best;
 }

@@ -53,9 +53,10 @@ def test_rotation_and_cache(tokens, heads, kv, slices):
     assert torch.equal(cache, ref)
 
 
-@pytest.mark.parametrize("M,N,K", [(1, 256, 64), (64, 200, 128), (65, 128, 128), (33, 72, 200), (64, 136, 328), (17, 64, 1024)])
+@pytest.mark.parametrize("M,N,K", [(1, 256, 64), (64, 200, 128), (65, 128, 128), (33, 72, 200), (64, 136, 328), (17, 64, 1024),
+                                   (1, 4033, 64), (64, 4040, 320), (33, 4104, 1024), (17, 4032, 128), (65, 4104, 128), (48, 4104, 72)])
 def test_small_tiles_by_either_cache_policy(M, N, K):
-    """One row tile with whole-line rows of B (non-temporal), two of them, rows off the lines."""
+    """One row tile with whole-line rows of a B of 64 column tiles (non-temporal); fewer of them, two row tiles, rows off the lines."""
     from kgs.ops import _lib
 
     a, b = (torch.randn(r, K, device=DEV).bfloat16() for r in (M, N))

@@ -845,13 +845,17 @@ inline double tr256_cost(long M, long N, long K, int cus) {
   return 8 * (full + (rest > 0)) + K / 64 * (full * 1.36 + (rest > 0 ? 0.88 + 0.15 * rest + 0.33 * b4 : 0));
 }
 
-// Whether that kernel loses to a transpose of B (4 bytes a value at 6.4 TB/s) and the product's best tiles: where its tiles leave
+// Whether that kernel loses to a transpose of B (4 bytes a value at 6.4 TB/s) and the product as gemm_nt runs it: where its tiles leave
 // most of the CUs idle. us, transposed read / transpose and tiles: 2048 x 1024 x 4096 65 / 38, 4096 x 512 x 4096 65 / 36, 4096 x
-// 2048 x 8192 132 / 118; 4096 x 8192 x 2048 106 / 114, 2048 x 14336 x 4096 172 / 217, 8192 x 2048 x 2048 52 / 59.
+// 2048 x 8192 132 / 118; 4096 x 8192 x 2048 106 / 114, 2048 x 14336 x 4096 172 / 217, 8192 x 2048 x 2048 52 / 59. Aligned products of more
+// 256x256 tiles than CUs run on these (gemm_bf16.hip aligned_finer): 2304 x 8192 x 6912 255 / 296, 3072 x 6656 x 1536 69 / 83. Of 117 sizes of
+// more than 4096 rows that read transposed now 7 % on average, none loses more than 7 (11520 x 10752 x 384 119 / 111).
 inline bool turn_b(long M, long N, long K, int cus) {
   const Plan p = refine(plan(M, N, K, true, cus), M, N, K, cus);
-  const double nt = p.ns > 1 || p.bm == 64 ? cost(M, N, K, p.bm == 64 ? 128 : p.bm, p.bm == 64 ? 128 : p.bn, p.ns, cus)
-                                           : tile_cost(p.bm, p.bn, M, N, K, cus);
+  const bool aligned = M % 256 == 0 && N % 256 == 0 && K % 128 == 0 && (M / 256) * (N / 256) > cus;
+  const double nt = aligned ? tile_cost(TILES[0], M, N, K, cus)
+                    : p.ns > 1 || p.bm == 64 ? cost(M, N, K, p.bm == 64 ? 128 : p.bm, p.bm == 64 ? 128 : p.bn, p.ns, cus)
+                                             : tile_cost(p.bm, p.bn, M, N, K, cus);
   return nt + 2.5 + 4.0 * N * K / 6.4e6 < tr256_cost(M, N, K, cus);
 }
 
@@ -886,7 +890,8 @@ inline int layout_plan(long M, long N, long K, int ta, int tb, int cus) {
   }
   if (K % 8) return best;  // nothing else reads such operands 16 bytes at a time
   if (t0 > nt + turn_a + turn_b) return 0;
-  if (M % 256 == 0 && N % 256 == 0 && K % 128 == 0 && tb && t0 > tr256_cost(M, N, K, cus) + turn_a) return 0;
+  // (3 %: few rows of tiles read a K-major B less well than that estimate; 1280 x 5376 x 11776 182 here, 208 there)
+  if (M % 256 == 0 && N % 256 == 0 && K % 128 == 0 && tb && t0 > 1.03 * tr256_cost(M, N, K, cus) + turn_a) return 0;
   return best;
 }
 

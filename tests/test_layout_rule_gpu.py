@@ -6,6 +6,14 @@ import torch
 pytestmark = [pytest.mark.gpu, pytest.mark.usefixtures("own_rng")]
 
 
+def test_prices_the_tiles_that_run():
+    """Aligned products of more tiles than CUs run on 256x256 ones, whatever finer tile would fill the CUs better."""
+    from kgs.ops.gemm import _tr_slices, _turn_b
+
+    assert not any(_turn_b(*s) for s in ((3072, 6656, 1536), (2304, 8192, 6912), (3584, 9984, 1024), (3840, 8960, 7168), (3584, 5120, 1792)))
+    assert _tr_slices(1280, 5376, 11776, False, True) and not _tr_slices(4608, 2560, 512, False, True)
+
+
 def test_transposes_where_the_reading_kernel_leaves_cus_idle():
     from kgs.ops.gemm import _turn_b
 

@@ -811,6 +811,12 @@ inline Plan refine(Plan p, long M, long N, long K, int cus, bool sw = false) {
   return p;
 }
 
+// The tile of a gated product (B of N rows, gate and up)
+inline Plan gated_plan(long M, long N, long K, int cus) {
+  const Plan p = plan(M, N, K, false, cus);
+  return refine(p.bm == 64 ? Plan{128, 128, 1} : p, M, N, K, cus, true);
+}
+
 // Whether a product that the aligned, the persistent or the eight-wave 256x256 kernels take is better off on refine's
 // tile here: those keep a little (persistent tiles 3 % on average, 9 % at most) that a tile has to win back first. Of 90 such products whose estimate
 // promises 7 to 20 % the tile is 6 % faster on average, 4 % slower at worst (2902 x 13312 x 1536 107 / 112 us, ragged rows). off: rows off the
@@ -1028,9 +1034,7 @@ int gemm_any_swiglu(const void* A, const void* B, void* C, int M, int N, int K, 
   using namespace any;
   const Args a{(const unsigned short*)A, (const unsigned short*)B, C, nullptr, (const unsigned short*)limit,
                M, N, K, lda, ldb, ldc, 0, M > N, ldc % 8 == 0 && (uintptr_t)C % 16 == 0, 1.f, nullptr};
-  Plan p = plan(M, N, K, false, cu_count());
-  if (p.bm == 64) p = {128, 128, 1};
-  p = refine(p, M, N, K, cu_count(), true);
+  const Plan p = gated_plan(M, N, K, cu_count());
   const dim3 grid((unsigned)(ceil_div(M, p.bm) * ceil_div(N / 2, p.bn / 2)));
 #define KGS_SWK(BM, BN, ...) \
   case BM << 16 | BN: hipLaunchKernelGGL((__VA_ARGS__>), grid, dim3(256), 0, s, a); break
@@ -1128,6 +1132,15 @@ KGS_EXPORT int kgs_gemm_bf16_tr(const void* A, const void* B, void* C, int M, in
   if (M <= 0 || N <= 0 || K <= 0 || ldc < N || ns < 1 || ns > 64) return KGS_ERR_SHAPE;
   if (!kgs::gemm_tr_ok(A, B, M, N, K, lda, ldb, ta, tb) || (uintptr_t)ws % 16) return KGS_ERR_ALIGN;
   return kgs::gemm_tr(A, B, C, M, N, K, lda, ldb, ldc, ta, tb, ns, ws, s);
+}
+
+// The tile that gemm_any chooses without scratch, for a gated product (N rows of gate and up) if gated: rows << 16 | columns.
+KGS_EXPORT int kgs_gemm_bf16_nt_tile(int M, int N, int K, int gated) {
+  using namespace kgs::any;
+  if (M <= 0 || N <= 0 || K <= 0) return 0;
+  const int cus = kgs::cu_count();
+  const Plan p = gated ? gated_plan(M, N, K, cus) : refine(plan(M, N, K, false, cus), M, N, K, cus);
+  return p.bm << 16 | p.bn;
 }
 
 // Whether the kernels of 256x256 tiles leave a product (gated: of a gated projection; off: A's rows off the 128-byte lines) to a finer tile.

@@ -65,14 +65,22 @@ def test_mid_tiles_repeat_the_large_tile_bits(M, N, K, bm, bn):
     assert rel(want, torch.nn.functional.gelu(a.double() @ b.double().T + bias.double(), approximate="tanh")) < 2 * REL
 
 
+def tile(M, N, K, gated=False):
+    from kgs.ops import _lib
+
+    t = _lib.lib().kgs_gemm_bf16_nt_tile(M, N, K, int(gated))
+    return t >> 16, t & 0xffff
+
+
 # sizes whose tile, by the rule, is each of MID
 @pytest.mark.parametrize("M,N,K", [(642, 5480, 128), (965, 5456, 136), (1541, 5008, 128), (1543, 5408, 128), (2035, 4832, 128),
                                    (2054, 5392, 128)])
 def test_mid_tiles_with_every_epilogue(M, N, K):
     """What is stored beside the product: the residual sum, both outputs of a training pass."""
     from kgs.ops import gemm_nt
-    from kgs.ops.gemm import add_product_, gemm_nt_act, gemm_swiglu
+    from kgs.ops.gemm import add_product_, gemm_nt_act
 
+    assert tile(M, N, K) in MID
     a, b, bias = rnd(M, K), rnd(N, K), torch.randn(N, device=DEV).bfloat16()
     z = a.double() @ b.double().T
     assert rel(gemm_nt(a, b), z) < REL
@@ -84,15 +92,32 @@ def test_mid_tiles_with_every_epilogue(M, N, K):
     assert rel(y, torch.nn.functional.silu(pre.double())) < REL
 
 
-@pytest.mark.parametrize("M,N", [(642, 5504), (965, 5504), (1541, 5120)])
-@pytest.mark.parametrize("act", ["silu", "gelu_tanh"])
-def test_mid_tiles_of_gated_products(M, N, act):
-    from kgs.ops.gemm import gemm_swiglu
+def test_the_sizes_above_have_every_tile():
+    assert {tile(*s) for s in ((642, 5480, 128), (965, 5456, 136), (1541, 5008, 128), (1543, 5408, 128), (2035, 4832, 128), (2054, 5392, 128))} == set(MID)
 
-    a, b = rnd(M, 128), rnd(N, 128)
-    g, u = (a.double() @ b.double().T).bfloat16().double().chunk(2, 1)
-    f = torch.nn.functional.silu(g) if act == "silu" else torch.nn.functional.gelu(g, approximate="tanh")
-    assert rel(gemm_swiglu(a, b, act), f * u) < 2 * REL
+
+@pytest.mark.parametrize("M,N,K,bm,bn", [(642, 5504, 128, 192, 128), (642, 5456, 136, 192, 128), (965, 5456, 136, 224, 128), (2017, 3184, 328, 224, 128),
+                                         (1541, 5120, 128, 224, 256), (1541, 5136, 200, 224, 256), (965, 5504, 128, 128, 128)])
+@pytest.mark.parametrize("act", ["silu", "gelu_tanh", "clamped"])
+def test_mid_tiles_of_gated_products(M, N, K, bm, bn, act):
+    """Each tile, with and without a K tail (which gemm_swiglu itself keeps to the unfused way)."""
+    from kgs.ops import _lib
+    from kgs.ops.activation import Gate, act_mul
+    from kgs.ops.gemm import GATE_ACTS, gemm_swiglu
+
+    assert tile(M, N, K, gated=True) == (bm, bn)
+    a, b = rnd(M, K), rnd(N, K)
+    both = (a.double() @ b.double().T).bfloat16().double()
+    g, u = both.chunk(2, 1)
+    gate = Gate("clamped", 1.5) if act == "clamped" else Gate.of(act)
+    want = act_mul(both.float(), gate).double() if act == "clamped" else u * (
+        torch.nn.functional.silu(g) if act == "silu" else torch.nn.functional.gelu(g, approximate="tanh"))
+    got = torch.full((M + 1, N // 2), 7.0, device=DEV, dtype=torch.bfloat16)
+    assert _lib.lib().kgs_gemm_bf16_nt_swiglu(a.data_ptr(), b.data_ptr(), got.data_ptr(), M, N, K, K, K, N // 2, GATE_ACTS[gate.act],
+                                              gate.limit_ptr(a.device), _lib.stream_handle(a.device)) == 0
+    assert rel(got[:M], want) < 2 * REL and bool((got[M] == 7).all())
+    if K % 128 == 0 and N % 128 == 0:
+        assert torch.equal(gemm_swiglu(a, b, gate), got[:M])
 
 
 def test_any_reads_nothing_past_its_operands():

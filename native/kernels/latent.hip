@@ -346,14 +346,15 @@ __device__ __forceinline__ int first_key(const Args& a, int pos) { return a.win 
 // Pages that a token at pos sees
 __device__ __forceinline__ int pages_seen(const Args& a, int pos) { return pos / PAGE - first_key(a, pos) / PAGE + 1; }
 
-constexpr int MAX_SPLIT = 64;   // parts of a sequence
-constexpr int LEAST_PAGES = 2;  // pages of a part
+constexpr int MAX_SPLIT = 64;  // parts of a sequence
 
 // Parts by length: all sequences are cut into parts of the same number of pages, the fewest that make at most `parts`
 // of them (and MAX_SPLIT of one), and workgroup i takes part i of the list. The host sees only the block table's width:
 // in equal splits of each sequence the longest one's are the launch's time, and the short ones' workgroups are done or
-// empty. 24 sequences of 60 to 1300 tokens with 16 heads over latents of 512: 14.9 us in equal splits,
-// 10.9 so, and the merge's 4.9 and 4.7.
+// empty. us with the merge, latents of 512, equal splits / so: 24 sequences of 500 tokens on average with 16 heads 19.2 / 17.6, 3 of 2700 30.5 / 19.8, 16 of 512
+// with 32 20.9 / 20.0. Parts of one page where there are places for them: of two pages at least 22 of 23 tokens took 13.4 (equal splits 12.2, now
+// 11.5), 8 of 79 13.0 (11.9, 11.0), and each part's largest weight is the one that its rounding to bf16 keeps exact: errors against
+// 64 bits over 40 batches 1.03 times those of the equal splits, 1.00 so.
 struct Part {
   int seq, pos, part, first, count, pages;  // seq -1: none
 };
@@ -368,7 +369,7 @@ __device__ __forceinline__ Part find_part(const Args& a, int i, int lane) {
   most = wave_max(most);
   const int room = a.parts - a.Nt;  // every sequence's last part may be a short one
   const int pages = __builtin_amdgcn_readfirstlane(
-      max(LEAST_PAGES, max(((int)total + room - 1) / room, ((int)most + MAX_SPLIT - 1) / MAX_SPLIT)));
+      max(1, max(((int)total + room - 1) / room, ((int)most + MAX_SPLIT - 1) / MAX_SPLIT)));
   for (int c0 = 0, before = 0; c0 < a.Nt; c0 += 64) {
     const int c = c0 + lane, pos = a.pos0[min(c, a.Nt - 1)];
     const int n = c < a.Nt ? (pages_seen(a, pos) + pages - 1) / pages : 0;

@@ -52,3 +52,22 @@ def test_parts_by_length(kind, batch, heads, rp, hr, window):
     assert (got.view(batch, heads, rp) - want).abs().max().item() < bound
     whole = latent_attention(q, pages, LatentRows(**rows), heads, scale, hr, window).float()
     assert (got - whole).abs().max().item() < bound
+
+
+@pytest.mark.parametrize("lens,parts,pages", [([79] * 8, 256, 1), ([500, 33, 1, 32], 256, 1), ([5000] + [1] * 7, 256, 3), ([2000] * 24, 256, 7)])
+def test_parts_are_as_short_as_the_places_allow(lens, parts, pages):
+    """A page each where there are places for all, else as few as make them fit (64 parts of a sequence at most)."""
+    from kgs.ops import _lib
+
+    nt, heads, rp = len(lens), 16, 128
+    i32 = dict(dtype=torch.int32, device="cuda")
+    W = -(-max(lens) // 32)
+    ar, pos, bt = torch.arange(nt, **i32), torch.tensor(lens, **i32) - 1, torch.zeros(nt, W, **i32)
+    cache, q = (torch.randn(*s, device="cuda").bfloat16() for s in ((1, 32, rp), (nt, heads * rp)))
+    o, po, ml, of = torch.empty_like(q), torch.empty(parts, heads, rp, device="cuda"), torch.empty(parts, heads, 2, device="cuda"), torch.full((nt, 2), -1, **i32)
+    one = torch.ones(nt, **i32)
+    assert _lib.lib().kgs_latent_attn_parts(q.data_ptr(), cache.data_ptr(), o.data_ptr(), po.data_ptr(), ml.data_ptr(), of.data_ptr(), ar.data_ptr(),
+                                            one.data_ptr(), pos.data_ptr(), bt.data_ptr(), 1, 1, parts, heads, W, nt, rp, 0, 0, 0.1,
+                                            _lib.stream_handle(q.device)) == 0
+    want = [-(-(-(-n // 32)) // pages) for n in lens]
+    assert of[:, 1].tolist() == want and of[:, 0].tolist() == [sum(want[:i]) for i in range(nt)]

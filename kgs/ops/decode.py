@@ -785,22 +785,29 @@ def length_parts(batch: int, kv_heads: int, max_pages: int, waves: int, fp8: boo
     For 3 to 128 sequences and tables of 64 pages on: up to two have equal parts that are as good (one of 4000 tokens 10.2 us /
     10.6), narrower tables hold lengths that differ by less than the longer start costs (256 sequences of 32 pages
     26.6 / 28.0), and 256 sequences of 600 on average, four rounds of workgroups that even out by themselves, take 47.9 /
-    49.4. Fewer than one workgroup per CU while the (sequence, KV head) pairs are at most that many, since
-    the parts' remainders come on top, else one and a half. us, equal parts / 192 workgroups / 384, lengths log-normal around the
-    mean: 100 of 700 tokens with 4 KV heads 38.1 / 30.8 / 29.9, 40 of 700 with 8 27.8 / 25.2 / 25.6, 70 of 1000 with 4 44.9 / - /
-    32.2, 50 of 1000 27.1 / 23.7 / 26.0, 30 of 700 with 8 23.9 / 19.4 / 20.6, 16 of 1000 17.9 / 17.1 / 18.3; 32 equal ones of 2000 47.0 /
-    43.7 / 45.3, 128 of up to 2000 with 4 53.1 / 53.5 / 52.6; e4m3 100 of 700 25.6 / 22.2 / 21.0, 64 of 900 21.0 / 21.2 / 20.0, 40 of 700
-    with 8 20.9 / 18.2 / 17.7."""
+    49.4. One and a half workgroups per CU, and fewer than one up to three fifths of the CUs in (sequence, KV head) pairs, whose short last
+    parts come on top. us, equal parts / 192 workgroups / 384, lengths log-normal around the mean: 24 of 3676 tokens with 8 KV heads
+    67.9 / 70.4 / 58.8, 27 of 2222 44.5 / 46.2 / 40.3, 51 of 1826 with 4 44.9 / 48.4 / 40.4, 100 of 700 38.1 / 30.8 / 29.9; 16 of 1000 with 8 17.9 / 17.1 /
+    18.3, 8 of 2348 19.3 / 18.4 / 21.0. Over 380 batches the geometric mean is 0.75 to 0.92 of the equal parts' time by the number of pairs. Slower are
+    short contexts in tables that are much wider (101 of 117 tokens in 256 pages 6.5 / 7.7), equal ones that just need a second part (72 of
+    605 in a batch of 128 21.2 / 27.3) and 128 of up to 2000, uniform,
+    with 4 KV heads (53.2 / 54.7)."""
     if max_pages < 64 or not 2 < batch <= 128 or waves != (4 if fp8 else 8):
         return 0
-    groups = batch * kv_heads
-    return max(1, (192 if groups < CUS or (groups == CUS and not fp8) else 384) // kv_heads)
+    return max(1, (192 if 5 * batch * kv_heads < 3 * CUS else 384) // kv_heads)
+
+
+def part_target(batch: int, kv_heads: int, max_pages: int, waves: int, fp8: bool) -> int:
+    """:func:`length_parts`, 0 where equal parts are as short: up to 40 pairs and tables of fewer than 128 pages, 8 pages a part at most
+    (us, equal / by length: 5 of 747 tokens with 4 KV heads 9.6 / 11.4, 3 of 2138 with 8 11.0 / 12.1, 14 of 3173 with 1 12.7 / 14.0; 11 of 1132 with 4,
+    44 pairs, 12.9 / 12.1, and 5 of 3098 in 128 pages 15.1 / 13.8)."""
+    return 0 if batch * kv_heads <= 40 and max_pages < 128 else length_parts(batch, kv_heads, max_pages, waves, fp8)
 
 
 def part_tickets(batch: int, kv_heads: int, max_pages: int, fp8: bool) -> int:
     """Length of the ``tickets`` that :func:`paged_decode_attention` of such a batch takes, 0: none."""
     waves = workgroup_waves(batch * kv_heads, max_pages, fp8)
-    return batch * kv_heads if length_parts(batch, kv_heads, max_pages, waves, fp8) else 0
+    return batch * kv_heads if part_target(batch, kv_heads, max_pages, waves, fp8) else 0
 
 
 _AWS: dict = {}
@@ -882,7 +889,7 @@ def paged_decode_attention(q: torch.Tensor, cache_layer: torch.Tensor, block_tab
     """One query token per sequence: ``q`` rows ``[B, >= H*128]`` (e.g. the rotated
     q heads at the front of the fused QKV rows), ``block_tables`` int32
     ``[B, max_pages]``, ``ctx_lens`` int32 ``[B]`` (cached tokens incl. the new
-    one). Returns ``[B, H*128]`` bf16. Parts that follow the lengths (:func:`length_parts`) have partial results of the call's own and take
+    one). Returns ``[B, H*128]`` bf16. Parts that follow the lengths (:func:`part_target`) have partial results of the call's own and take
     ``tickets``, zeroed int32 of :func:`part_tickets` values or more, which are zero again behind it and so serve every layer of
     a step (None: the call's own, a launch of 1.5 us more). Contexts split in any other way
     share one workspace per GPU: calls of such batches on several streams have to be ordered."""
@@ -896,7 +903,7 @@ def paged_decode_attention(q: torch.Tensor, cache_layer: torch.Tensor, block_tab
     max_pages = block_tables.shape[1]
     fp8 = cache_layer.dtype == FP8
     waves = workgroup_waves(b * kv_heads, max_pages, fp8) if pages_per_split is None and pipe is None else 1
-    target = length_parts(b, kv_heads, max_pages, waves, fp8)
+    target = part_target(b, kv_heads, max_pages, waves, fp8)
     if waves > 1:
         nsplit = workgroup_splits(b, kv_heads, max_pages) if b else 1
     elif pages_per_split is None:

@@ -187,6 +187,26 @@ def test_length_rule_has_room_for_its_parts():
                 assert length_parts(batch, kv, 63, 4 if fp8 else 8, fp8) == 0 == length_parts(batch, kv, 64, 2, fp8)
 
 
+@pytest.mark.parametrize("batch,kv,target", [(3, 8, 24), (19, 8, 24), (20, 8, 48), (153, 1, 0), (38, 4, 48), (39, 4, 96), (128, 8, 48), (100, 4, 96), (5, 300, 1)])
+@pytest.mark.parametrize("fp8", [False, True])
+def test_parts_by_the_number_of_pairs(batch, kv, target, fp8):
+    from kgs.ops.decode import length_parts
+
+    assert length_parts(batch, kv, 64, 4 if fp8 else 8, fp8) == target
+
+
+@pytest.mark.parametrize("batch,kv,pages,parts", [(5, 8, 64, False), (5, 8, 127, False), (5, 8, 128, True), (41, 1, 64, True), (11, 4, 64, True), (3, 1, 4096, True)])
+def test_few_pairs_on_narrow_tables_keep_equal_parts(batch, kv, pages, parts):
+    from kgs.ops import decode as D
+
+    assert bool(D.part_tickets(batch, kv, pages, False)) == parts
+    lens = [32 * pages - 5] + [70] * (batch - 1)
+    q, cache, tables, ctx = setup(lens, kv, 2)
+    tables = tables[:, :pages].contiguous()
+    got = D.paged_decode_attention(q, cache, tables, ctx, 2 * kv, kv).float()
+    assert float((got - D.ref_paged_decode(q, cache, tables, ctx, 2 * kv, kv)).abs().max()) < TOL
+
+
 def test_parts_keep_their_scratch_to_the_call(monkeypatch):
     """Batches that had no split before their parts followed the lengths shared nothing with other calls, nor do they now: steps
     of different lengths on two streams, and between a graph's replays, with tickets given and without."""
@@ -199,7 +219,7 @@ def test_parts_keep_their_scratch_to_the_call(monkeypatch):
         lens = torch.randint(1, 700, (64,), generator=g).tolist()
         lens[5] = 2040
         sets.append(setup(lens, 8, 2, seed=len(sets)))
-    assert D.length_parts(64, 8, sets[0][2].shape[1], 8, False) and D.part_tickets(64, 8, sets[0][2].shape[1], False) == 512
+    assert D.part_tickets(64, 8, sets[0][2].shape[1], False) == 512
     want = [D.paged_decode_attention(*s, 16, 8) for s in sets]
     for w, s in zip(want, sets):
         assert float((w.float() - D.ref_paged_decode(*s, 16, 8)).abs().max()) < TOL

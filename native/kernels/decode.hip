@@ -1873,8 +1873,9 @@ KGS_EXPORT int kgs_rope_cache_bf16(void* qkv, const float* cosv, const float* si
   const long n = tokens * (H + 2 * HKV) * 8;
   if (n == 0) return 0;
   // small grids: a wave per workgroup, so that every CU takes part (us of 256 / 64 threads, 24 heads, 8 slices: 40 tokens 3.9 / 3.2,
-  // 128 4.5 / 3.9; 48 heads: 90 5.05 / 4.6, 30 without slices 3.2 / 2.9; 4 slices at 128 4.57 / 4.65)
-  const int wg = n <= 256 * 256 ? 64 : 256;
+  // 128 4.5 / 3.9; 48 heads: 90 5.05 / 4.6, 30 without slices 3.2 / 2.9; two slices up to 24k threads only: 80 heads 51 tokens 3.4 / 3.7,
+  // 48 150 5.1 / 5.5)
+  const int wg = n <= (P != nullptr && nslice == 2 ? 96 : 256) * 256 ? 64 : 256;
   const dim3 g((unsigned)((n + wg - 1) / wg)), b(wg);
   auto q = (unsigned short*)qkv;
   if (P != nullptr) {

@@ -207,7 +207,8 @@ struct ProjArgs {
 // single waves on all CUs then, with K = 512 in one round (D 16) and the gate's loads before them, 32 tokens each. us, 128 outputs of
 // K = 512 of 16 heads, four waves / single ones with D 4 / with D 16: 1 token 5.0 / 4.2 / 3.2, 24 tokens 8.0 / 5.5 / 4.5, of 32 heads 16
 // tokens 6.2 / 4.8 / 3.7; 33 of 32 heads 10.3 with 64 tokens a wave, 8.7 with 32, 5.9 so.
-// More workgroups hide each other's loads and lose by the registers (16 tokens of 128 heads, 512 outputs of K = 128: D 4 6.9, D 16 8.1).
+// More workgroups hide each other's loads and lose by the registers (16 tokens of 128 heads, 512 outputs of K = 128: D 4 6.9, D 16 8.1; the
+// gate's loads come last there: 217 tokens of 32 heads, 128 outputs of K = 128, 8.1, before the others 8.7).
 template <int TT, int D>
 __global__ __launch_bounds__(256) void head_proj(ProjArgs p) {
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
@@ -250,17 +251,19 @@ __global__ __launch_bounds__(256) void head_proj(ProjArgs p) {
     const long r = p.idx_in ? p.idx_in[t] : t;
     ap[i] = (const unsigned short*)p.a + r * p.lda + h * p.ha + 8 * g;
   }
-  unsigned short gate[TT][4];
-  if (p.gate) {
+  constexpr bool EARLY = D > 4;
+  auto gate_of = [&](int t, unsigned short (&v)[4]) {
+    const long r = p.idx_out ? p.idx_out[t] : t;
+    const unsigned short* gp = (const unsigned short*)p.gate + r * p.ldg + (long)h * p.hg + (nt * 16 + 4 * g) * p.eg;
 #pragma unroll
-    for (int i = 0; i < TT; ++i) {
-      const int t = min(t0 + 16 * i + l16, p.Nt - 1);
-      const long r = p.idx_out ? p.idx_out[t] : t;
-      const unsigned short* gp = (const unsigned short*)p.gate + r * p.ldg + (long)h * p.hg + (nt * 16 + 4 * g) * p.eg;
+    for (int j = 0; j < 4; ++j) v[j] = gp[j * p.eg];
+  };
+  unsigned short gate[EARLY ? TT : 1][4];
+  if constexpr (EARLY)
+    if (p.gate) {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) gate[i][j] = gp[j * p.eg];
+      for (int i = 0; i < TT; ++i) gate_of(min(t0 + 16 * i + l16, p.Nt - 1), gate[i]);
     }
-  }
   f32x4 acc[TT];
 #pragma unroll
   for (int i = 0; i < TT; ++i) acc[i] = f32x4{};
@@ -288,8 +291,9 @@ __global__ __launch_bounds__(256) void head_proj(ProjArgs p) {
     const long r = p.idx_out ? p.idx_out[t] : t;
     f32x4 s = f32x4{1.0f, 1.0f, 1.0f, 1.0f};
     if (p.gate) {
+      if constexpr (!EARLY) gate_of(t, gate[0]);
 #pragma unroll
-      for (int j = 0; j < 4; ++j) s[j] = sigmoid(bf2f(gate[i][j]));
+      for (int j = 0; j < 4; ++j) s[j] = sigmoid(bf2f(gate[EARLY ? i : 0][j]));
     }
     uint2 o;
     o.x = pack_bf16x2(acc[i][0] * s[0], acc[i][1] * s[1]);

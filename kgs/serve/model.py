@@ -60,6 +60,21 @@ def gate_up_panel_widths(n: int, k: int) -> set:
     return {r[0] for (_, rn, rk), r in D.W4X_TUNED.items() if (rn, rk) == (n, k) and r[1] == 1}
 
 
+def gate_up_route(m: int, n: int, k: int):
+    """The route of :meth:`ServingModel._swiglu_route` for a gate|up ``[n, k]`` without measured entries, None: the library and the product.
+
+    The gate kernel by :func:`kgs.ops.decode.gate_rule`, beside the library's product as beside slices: 2048x3328 at 39 rows 10.6 us by the
+    library, 16.3 by the gate kernel, 2048x6912 at 104 21.6 / 30.5. Where unsplit tiles take more rows of W than CUs have 64 of, only up to 40 rows
+    and K of 4096 (33 rows of 25856x1536 19.8 / 19.3; 40 of 22528x8064 76 / 82, 56 of 23808x3840 43.5 / 47.5, 60 of 22272x7680 79 / 90). Over 170
+    sizes of 1 to 128 rows its geometric mean is 0.67 of the other route's time, the worst 1.07 (32 of 21504x6912 62.6 / 67.0)."""
+    rule = D.w4x_rule(m, n, k)
+    whole = rule is not None and rule[1] == 1
+    if whole and n > 64 * D.CUS and (m > 40 or k > 4096):
+        return rule
+    bm = D.gate_rule(m, n, k, sliced=not whole)
+    return rule if bm is None else (GATE, 1, bm)
+
+
 def head_on_small_tiles(m: int, n: int, k: int) -> bool:
     """Whether ``m`` rows of an LM head ``[n, k]`` go by the general kernel's small tiles and not by the library.
 
@@ -282,9 +297,7 @@ class ServingModel:
         r = D.w4x_route(m, w.shape[0], w.shape[1])
         if r is not None:
             return r if r[1] == 1 else None
-        rule = D.w4x_rule(m, w.shape[0], w.shape[1])
-        bm = D.gate_rule(m, w.shape[0], w.shape[1], rule is not None and rule[1] > 1)
-        return rule if bm is None else (GATE, 1, bm)
+        return gate_up_route(m, *w.shape)
 
     def _split_proj(self, x, layer: int, name: str, r, private: bool = False):
         """fp32 partial products of a projection along route ``r``, in a buffer of the call's own if

@@ -1,4 +1,4 @@
-"""Which LM heads of few rows go by the general kernel's small tiles."""
+"""Which LM heads of few rows go by the general kernel's small tiles, and which gate|up projections by the gate kernel."""
 import pytest
 
 
@@ -10,3 +10,12 @@ def test_small_tiles_where_they_are_the_faster(m, n, k, small):
     from kgs.serve.model import head_on_small_tiles
 
     assert head_on_small_tiles(m, n, k) == small
+
+
+@pytest.mark.parametrize("m,n,k,route", [
+    (39, 2048, 3328, None), (104, 2048, 6912, None), (59, 2304, 1280, (32, 1, 64)), (40, 16384, 4736, (32, 1, 64)), (33, 25856, 1536, (32, 1, 64)),
+    (40, 22528, 8064, (128, 1, 128)), (56, 23808, 3840, (128, 1, 128)), (100, 16384, 2048, (32, 1, 128)), (8, 2048, 1024, (32, 1, 64))])
+def test_gate_kernel_where_it_is_the_faster(m, n, k, route):
+    from kgs.serve.model import gate_up_route
+
+    assert gate_up_route(m, n, k) == route

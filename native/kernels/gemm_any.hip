@@ -294,7 +294,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
 // F8: e4m3 operands, seen as rows of 16-bit words (lda, ldb, K in words). A lane's 16-byte chunk is 16
 // values of K, its halves the operands of two MFMAs: which K they are does not matter as long as
 // both operands agree.
-template <int EPI, bool DUAL, bool F8 = false>
+// NT: B past the caches, for one row tile of a B of whole 128-byte lines and 64 column tiles or more (launch), which is read once: 5.9 TB/s of a large one
+// where the default policy reaches 5.0. Off the lines each would come twice (64 x 3000 x 1032 9.1 / 12.1 us), of a few tiles such loads cost 0.2 us (17 x
+// 448 x 256 3.4 / 3.6). A kernel of its own: chosen at run time inside, the others lost 2 to 8 % (e4m3 8 x 512 x 5120 13.7 / 14.5 us, 32 x 1152 x 1280 with
+// both outputs 9.0 / 9.8).
+template <int EPI, bool DUAL, bool F8 = false, bool NT = false>
 __global__ __launch_bounds__(256) void gemm_small(Args a) {
   constexpr int BM = 64, BN = 64, ST = 4;
   constexpr int FM = BM / 32, FN = BN / 32, LA = BM / 32, LB = BN / 32, STAGE = (BM + BN) * 128;
@@ -317,17 +321,9 @@ __global__ __launch_bounds__(256) void gemm_small(Args a) {
 #pragma unroll
     for (int j = 0; j < LA; ++j)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (KGS_LDS void*)(dst + (j * 4 + w) * 1024), 16, oa, j * sa + t * 128, 0, 0);
-    // B is read once, whole lines at a time: non-temporal loads, 5.9 TB/s of a large B where the default policy reaches 5.0 (off
-    // the 128-byte lines each would come twice: 64 x 3000 x 1032 9.1 / 12.1 us; of a few tiles they cost 0.2: 17 x 448 x 256 3.4 / 3.6)
-    if (ntm == 1 && ntn >= 64 && a.ldb % 64 == 0) {
 #pragma unroll
-      for (int j = 0; j < LB; ++j)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (KGS_LDS void*)(dst + BM * 128 + (j * 4 + w) * 1024), 16, ob, j * sb + t * 128, 0, 2);
-    } else {
-#pragma unroll
-      for (int j = 0; j < LB; ++j)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (KGS_LDS void*)(dst + BM * 128 + (j * 4 + w) * 1024), 16, ob, j * sb + t * 128, 0, 0);
-    }
+    for (int j = 0; j < LB; ++j)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (KGS_LDS void*)(dst + BM * 128 + (j * 4 + w) * 1024), 16, ob, j * sb + t * 128, 0, NT ? 2 : 0);
   };
   const int fr = lane & 15, fq = lane >> 4;
   const int ro = fr * 128 + ((fq ^ (fr >> 1)) * 16);
@@ -911,7 +907,13 @@ void launch_tile(const Args& a, int ns, hipStream_t s) {
 template <int EPI, bool DUAL>
 int launch(Args a, Plan p, float* ws, hipStream_t s) {
   if (p.bm == 64) {
-    hipLaunchKernelGGL((gemm_small<EPI, DUAL>), dim3((unsigned)(ceil_div(a.M, 64) * ceil_div(a.N, 64))), dim3(256), 0, s, a);
+    const dim3 grid((unsigned)(ceil_div(a.M, 64) * ceil_div(a.N, 64)));
+    if constexpr (!DUAL)
+      if (a.M <= 64 && grid.x >= 64 && a.ldb % 64 == 0) {
+        hipLaunchKernelGGL((gemm_small<EPI, false, false, true>), grid, dim3(256), 0, s, a);
+        return (int)hipGetLastError();
+      }
+    hipLaunchKernelGGL((gemm_small<EPI, DUAL>), grid, dim3(256), 0, s, a);
     return (int)hipGetLastError();
   }
   Args g = a;

@@ -3,7 +3,7 @@
 ``gemm_nt(a, b)`` computes ``a @ b.T`` for ``a: [M, K]``, ``b: [N, K]`` (both
 K-contiguous bf16 on a gfx950 device), with optional fused bias + activation in
 the kernel epilogue. :func:`gemm_bf16` covers the other layouts: operands stored
-K-major are read with ``ds_read_b64_tr_b16``, so no transpose copy is made.
+K-major are read with ``ds_read_b64_tr_b16``, or transposed first where that is faster.
 ``gemm_fp8_nt`` is the same pipeline on OCP e4m3 operands with the scaled fp8
 MFMA and a per-tensor dequant scale. ``matmul`` and ``Linear`` are built on
 these; the backward pass uses the transposed-read layouts, so every FLOP of the
@@ -731,7 +731,7 @@ def _general(a, b, out, M, N, K, ta, tb, bias, act) -> torch.Tensor:
 
 
 def matmul(a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
-    """``a @ b`` with ``b: [K, N]`` row-major (transposed-read path, no transpose copy)."""
+    """``a @ b`` with ``b: [K, N]`` row-major, read transposed or transposed first, whichever is faster for the size."""
     return gemm_bf16(a, b)
 
 

@@ -1257,6 +1257,18 @@ __global__ __launch_bounds__(64) void paged_decode(AttnArgs a) {
   store_o(op, o, L > 0.f ? 1.f / L : 0.f);
 }
 
+// Inclusive sums over the wave's lanes, all of them active: shifts by 1, 2, 4 and 8 within rows of 16, then the last
+// lane of row 0 (of 2) to row 1 (3) and of lane 31 to the upper half
+__device__ __forceinline__ int scan64(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);
+  return v;
+}
+
 // Decode attention by workgroups: W waves share a (sequence, KV head), or one of nsplit equal
 // parts of its pages. paged_decode gives every (sequence, KV head, fixed number of pages) one wave,
 // so a batch of unequal contexts waits for the longest one's wave, and at small batches a split
@@ -1273,18 +1285,6 @@ __global__ __launch_bounds__(64) void paged_decode(AttnArgs a) {
 // that keep the next page on its way in registers while they widen and multiply one (64 sequences
 // around 700 tokens, 8 KV heads: 22 us, 31 without). Fewer waves where the table holds few pages
 // (kgs/ops/decode.py workgroup_waves).
-// Inclusive sums over the wave's lanes, all of them active: shifts by 1, 2, 4 and 8 within rows of 16, then the last
-// lane of row 0 (of 2) to row 1 (3) and of lane 31 to the upper half
-__device__ __forceinline__ int scan64(int v) {
-  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true);
-  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true);
-  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true);
-  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true);
-  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);
-  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);
-  return v;
-}
-
 template <bool KV8>
 struct PageRegs;  // a page's K and V as loaded: fragment order, e4m3 pages 8 bytes a lane
 template <>
@@ -1314,11 +1314,10 @@ struct PageRegs<true> {
   __device__ bf16x8 vf(int i) const { return dequant8(v[i], 1.f); }
 };
 
-//
-// BAL (paged_parts): the parts follow the lengths, so that a long context is no longer one workgroup's (100 sequences of 60 to 2800 tokens, 4
-// KV heads: 38.1 -> 29.9 us, 70 of 4000 at most 44.9 -> 32.2; the rule is length_parts). All workgroups read all of them (a lane holds BAL of each 64) and cut
-// every sequence into equal parts of at most P pages, P such that `target` parts of P hold
-// them all (at least `least`): unit u of the grid is the u-th such part.
+// The attention itself, as described above at PageRegs. BAL (paged_parts): the parts follow the lengths, so that a long context is no longer one workgroup's (100
+// sequences of 60 to 2800 tokens, 4 KV heads: 38.1 -> 29.9 us, 70 of 4000 at most 44.9 -> 31.2; the rules are part_target and length_parts). All workgroups read
+// all of them (a lane holds BAL of each 64) and cut every sequence into equal parts of at most P pages, P such that `target` parts of P hold
+// them all (at least `least`): unit u of the grid is the u-th such part. Partial results and tickets are the caller's, of a call and a step.
 template <bool KV8, int W, bool PIPE, int BAL>
 __device__ __forceinline__ void paged_waves(const AttnArgs& a) {
   constexpr int LDO = HD + 4;  // a row of partial outputs: 16 heads' rows start on different banks

@@ -23,7 +23,8 @@ def test_norm_rows(rows, add):
 
 
 @pytest.mark.parametrize("tokens,heads,kv,slices", [(1, 2, 1, 0), (33, 2, 1, 2), (2048, 2, 1, 0), (2049, 2, 1, 0), (2048, 2, 1, 8),
-                                                    (2049, 2, 1, 8), (1023, 4, 2, 0), (1024, 4, 2, 0), (2048, 4, 2, 4)])
+                                                    (2049, 2, 1, 8), (1023, 4, 2, 0), (1024, 4, 2, 0), (2048, 4, 2, 4),
+                                                    (768, 2, 1, 2), (769, 2, 1, 2)])
 def test_rotation_and_cache(tokens, heads, kv, slices):
     from kgs.ops import decode as D
 

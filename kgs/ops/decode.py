@@ -507,9 +507,60 @@ def _workspace(device: torch.device, floats: int, ints: int):
     return ws, cnt
 
 
-EPI_SWIGLU, EPI_RMS, EPI_RESID, EPI_GELU, EPI_CLAMPED, EPI_SUMS_IN, EPI_SUMS_OUT = 1, 2, 4, 16, 32, 64, 128
+EPI_SWIGLU, EPI_RMS, EPI_RESID, EPI_ROPE, EPI_GELU, EPI_CLAMPED, EPI_SUMS_IN, EPI_SUMS_OUT = 1, 2, 4, 8, 16, 32, 64, 128
 SUM_WORDS, SUM_MAX_N = 8, 8192  # integers of a row's exact sum of squares (decode.hip add_exact), longest row
 GATE_EPI = {"silu": 0, "gelu_tanh": EPI_GELU, "clamped": EPI_CLAMPED}
+
+
+FEW_ROWS = 8  # of a fused layer; above, every workgroup's way through all of x costs what the statistics do (16 rows 4096 wide 504 us a step / 515)
+
+
+@lru_cache(maxsize=4096)
+def few_takes(m: int, n: int, k: int, fp8: bool = False) -> bool:
+    """Whether the kernel of few rows (native/kernels/decode_few.hip) runs ``m`` rows of an ``[n, k]`` weight: up to 16 of bf16 weights."""
+    return not fp8 and 0 < m <= 16 and bool(_lib.lib().kgs_skinny_few_ok(m, n, k))
+
+
+def _rope_args(rope: dict, m: int):
+    """The cache of :func:`skinny_gemm`'s ``rope``, checked."""
+    cache = rope["cache"]
+    if cache.dtype != torch.bfloat16 or not cache.is_contiguous():
+        raise ValueError("the RoPE epilogue writes a bf16 KV cache")
+    for key in ("positions", "slots"):
+        v = rope[key]
+        if v.dtype != torch.int32 or not v.is_contiguous() or v.numel() < m:
+            raise ValueError(f"{key} must be a contiguous int32 vector of >= M elements")
+    return cache
+
+
+def skinny_few(x: torch.Tensor, w: PackedWeight, out: torch.Tensor | None = None, norm: bool = False, resid: bool = False,
+               eps: float = 1e-5, rope: dict | None = None) -> torch.Tensor:
+    """:func:`skinny_gemm` of up to 16 rows (:func:`few_takes`), whose RMSNorm (``norm``; its weight folded into W) takes the rows'
+    statistics from x itself; ``resid``: ``out += x @ W^T``. ``rope`` as there."""
+    if x.dtype != torch.bfloat16 or not x.is_cuda or x.dim() != 2 or x.stride(1) != 1:
+        raise ValueError("x must be a row-major bf16 GPU matrix")
+    m, k = x.shape
+    if k != w.k or not few_takes(m, w.n, k, w.fp8):
+        raise ValueError(f"not a product of few rows: x {tuple(x.shape)}, W [{w.n}, {w.k}]")
+    if (rope is not None) != bool(w.rope) or (resid and (rope is not None or w.swiglu)):
+        raise ValueError("rope= needs a rope-packed qkv weight and vice versa; resid a plain one")
+    if out is None:
+        if resid:
+            raise ValueError("resid needs the residual stream as out [M, N]")
+        out = torch.empty((m, w.n_out), dtype=torch.bfloat16, device=x.device)
+    elif out.dtype != torch.bfloat16 or tuple(out.shape) != (m, w.n_out) or out.stride(1) != 1 or out.device != x.device:
+        raise ValueError("out must be a row-major bf16 matrix [M, N]")
+    epi = (EPI_SWIGLU | GATE_EPI[w.act.act] if w.swiglu else 0) | (EPI_RMS if norm else 0) | (EPI_RESID if resid else 0)
+    extra = (None,) * 5 + (0, 0)
+    if rope is not None:
+        cache = _rope_args(rope, m)
+        epi |= EPI_ROPE
+        extra = (rope["cos"].data_ptr(), rope["sin"].data_ptr(), rope["positions"].data_ptr(), rope["slots"].data_ptr(),
+                 cache.data_ptr(), *w.rope)
+    rc = _lib.lib().kgs_skinny_few(w.data.data_ptr(), x.data_ptr(), out.data_ptr(), m, w.n, k, x.stride(0), out.stride(0), epi,
+                                   float(eps), w.act.limit, *extra, _lib.stream_handle(x.device))
+    _lib.check(rc, f"skinny_few[{m}x{w.n}x{k}, epi={epi}]")
+    return out
 
 
 def skinny_gemm(x: torch.Tensor, w: PackedWeight, out: torch.Tensor | None = None,
@@ -579,13 +630,7 @@ def skinny_gemm(x: torch.Tensor, w: PackedWeight, out: torch.Tensor | None = Non
     if rope is not None:
         if w.fp8 or resid_ss is not None:
             raise ValueError("the RoPE epilogue is bf16-weight only and writes a fresh qkv output")
-        cache = rope["cache"]
-        if cache.dtype != torch.bfloat16 or not cache.is_contiguous():
-            raise ValueError("the RoPE epilogue writes a bf16 KV cache")
-        for key in ("positions", "slots"):
-            v = rope[key]
-            if v.dtype != torch.int32 or not v.is_contiguous() or v.numel() < m:
-                raise ValueError(f"{key} must be a contiguous int32 vector of >= M elements")
+        cache = _rope_args(rope, m)
         rc = _lib.lib().kgs_skinny_gemm_bf16_rope(
             w.data.data_ptr(), x.data_ptr(), out.data_ptr(), None if ws is None else ws.data_ptr(), cnt.data_ptr(), m, w.n, k, x.stride(0),
             out.stride(0), ks, variant, epi & (EPI_RMS | EPI_SUMS_IN),

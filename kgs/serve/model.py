@@ -448,7 +448,11 @@ class ServingModel:
             return attention_blocks(qkv, *self._kv(qkv), plan.items, c.heads, c.kv_heads, a, merges=plan.merges, slots=plan.slots)
 
         x, ss = self._fused_layers(tokens, positions, slots, attend, "prefill", count, exact=True, keep=plan.keep)
-        out = D.skinny_gemm(x.index_select(0, plan.last), self.packed_lm, rms=ss.index_select(1, plan.last), eps=c.eps, counters=count)
+        x = x.index_select(0, plan.last)
+        if ss is None:
+            out = D.skinny_few(x, self.packed_lm, norm=True, eps=c.eps)
+        else:
+            out = D.skinny_gemm(x, self.packed_lm, rms=ss.index_select(1, plan.last), eps=c.eps, counters=count)
         T.op("prefill-fused lm_head")
         return out
 
@@ -734,8 +738,9 @@ class ServingModel:
     def _decode_fused(self, tokens, positions, slots, block_tables, ctx_lens, pages_per_split):
         """Decode with every norm / SwiGLU / residual add inside the skinny GEMMs:
         5 GEMMs + RoPE/KV-write + attention per layer, no elementwise launches.
+        Up to 16 rows a GEMM takes the folded RMSNorm's statistic from its own input; above,
         ss_a / ss_b carry the residual rows' sums of squares between the
-        producing GEMM (residual update) and the consuming one (folded RMSNorm)."""
+        producing GEMM (residual update) and the consuming one."""
         c = self.cfg
         tickets = self._tickets(block_tables)
 
@@ -744,9 +749,14 @@ class ServingModel:
                                             pages_per_split=pages_per_split, tickets=tickets)
 
         x, ss = self._fused_layers(tokens, positions, slots, attend, "decode", None, exact=False, tickets=tickets)
-        out = D.skinny_gemm(x, self.packed_lm, rms=ss, eps=c.eps)
+        out = D.skinny_few(x, self.packed_lm, norm=True, eps=c.eps) if ss is None else D.skinny_gemm(x, self.packed_lm, rms=ss, eps=c.eps)
         T.op("decode-fused lm_head")
         return out
+
+    def _few(self, m: int) -> bool:
+        """Whether the fused layers and the head of ``m`` rows are products of few rows, which make the norms' statistics themselves."""
+        return m <= D.FEW_ROWS and D.few_takes(m, self.packed_lm.n, self.packed_lm.k, self.packed_lm.fp8) and \
+            all(D.few_takes(m, w.n, w.k, w.fp8) for w in self.packed[0].values())
 
     def _tickets(self, block_tables):
         """Tickets of the step's own for the decode rows' attention, to be cleared with its first launch; None: it takes none."""
@@ -771,7 +781,7 @@ class ServingModel:
 
     def _fused_layers(self, tokens, positions, slots, attend, kind: str, counters, exact: bool, keep=None,
                       tickets=None):
-        """The residual rows after all layers and their sums of squares; ``attend(qkv, layer)`` is the
+        """The residual rows after all layers and their sums of squares (None where :meth:`_few` products make their own); ``attend(qkv, layer)`` is the
         attention of the rotated rows, whose keys and values are in the cache. ``exact``: statistics whose
         bits do not depend on the order in which workgroups arrive, so that equal steps give equal bits. ``keep``
         (int32): of these rows of ``tokens``, ``positions`` and ``slots`` only. ``counters`` and
@@ -782,13 +792,16 @@ class ServingModel:
         eps = c.eps
         tokens, dev = tokens.to(self.embed.device), self.embed.device
         m = (tokens if keep is None else keep).numel()
-        ss = torch.empty(m, dtype=torch.float32, device=dev)  # statistic for layer 0's qkv
-        if exact:
-            zero = stats = torch.empty((2, D.SUM_WORDS, m), dtype=torch.int64, device=dev)
-            ss_a, ss_b = stats
-        else:
-            zero = ss_a = torch.empty_like(ss)
-            ss_b = ss
+        few = self._few(m)
+        ss = zero = None
+        if not few:
+            ss = torch.empty(m, dtype=torch.float32, device=dev)  # statistic for layer 0's qkv
+            if exact:
+                zero = stats = torch.empty((2, D.SUM_WORDS, m), dtype=torch.int64, device=dev)
+                ss_a, ss_b = stats
+            else:
+                zero = ss_a = torch.empty_like(ss)
+                ss_b = ss
         clear = tuple(t for t in (zero, counters, tickets) if t is not None)
         if embeds(self.embed):
             if keep is not None:
@@ -798,24 +811,31 @@ class ServingModel:
             if keep is not None:
                 tokens, positions, slots = (t.reshape(-1)[keep.long()] for t in (tokens, positions, slots))
             x = self.embed[tokens.long()].reshape(-1, c.hidden).contiguous()  # residual stream
-            ss.copy_(x.float().pow(2).sum(-1))
+            if ss is not None:
+                ss.copy_(x.float().pow(2).sum(-1))
             for t in clear:
                 t.zero_()
         for i in range(c.layers):
             P = self.packed[i]
-            if P["qkv"].rope:
-                qkv = D.skinny_gemm(x, P["qkv"], rms=ss, eps=eps, counters=counters,
-                                    rope={"cos": self.cos, "sin": self.sin, "positions": positions, "slots": slots,
-                                          "cache": self.cache.layer(i)})
+            rope = {"cos": self.cos, "sin": self.sin, "positions": positions, "slots": slots,
+                    "cache": self.cache.layer(i)} if P["qkv"].rope else None
+            if few:
+                qkv = D.skinny_few(x, P["qkv"], norm=True, eps=eps, rope=rope)
             else:
-                qkv = D.skinny_gemm(x, P["qkv"], rms=ss, eps=eps, counters=counters)
+                qkv = D.skinny_gemm(x, P["qkv"], rms=ss, eps=eps, counters=counters, rope=rope)
+            if rope is None:
                 self._rope_cache(qkv, i, positions, slots)
             T.op(f"{kind}-fused L{i} qkv+rope")
             a = attend(qkv, i)
             T.op(f"{kind}-fused L{i} attention")
-            D.skinny_gemm(a, P["o"], out=x, resid_ss=ss_a, zero=ss_b, counters=counters)
-            act = D.skinny_gemm(x, P["gate_up"], rms=ss_a, eps=eps, counters=counters)
-            D.skinny_gemm(act, P["down"], out=x, resid_ss=ss_b, zero=ss_a, counters=counters)
-            ss = ss_b
+            if few:
+                D.skinny_few(a, P["o"], out=x, resid=True)
+                act = D.skinny_few(x, P["gate_up"], norm=True, eps=eps)
+                D.skinny_few(act, P["down"], out=x, resid=True)
+            else:
+                D.skinny_gemm(a, P["o"], out=x, resid_ss=ss_a, zero=ss_b, counters=counters)
+                act = D.skinny_gemm(x, P["gate_up"], rms=ss_a, eps=eps, counters=counters)
+                D.skinny_gemm(act, P["down"], out=x, resid_ss=ss_b, zero=ss_a, counters=counters)
+                ss = ss_b
             T.op(f"{kind}-fused L{i} o+mlp")
         return x, ss

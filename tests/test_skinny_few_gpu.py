@@ -1,0 +1,86 @@
+"""Products of few rows (native/kernels/decode_few.hip) against the plain product in float64: the edges of its splits over waves
+and tiles, each epilogue, and the RMSNorm whose statistics it makes itself."""
+import pytest
+import torch
+
+from kgs.ops import decode as D
+
+pytestmark = pytest.mark.gpu
+
+# one strip; one and two rounds of strips with 8, 4 and 2 waves, each side of where the split changes; K at the ring's least
+SHAPES = [(16, 512), (4096, 1024), (4096, 1536), (4112, 1024), (8192, 512), (8208, 512), (8192, 4096), (2048, 8192)]
+
+
+def _operands(m, n, k, seed=0):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    x = torch.randn(m, k + 8, generator=g, device="cuda").bfloat16()[:, :k]  # rows further apart than they are long
+    return x, (torch.randn(n, k, generator=g, device="cuda") * k ** -0.5).bfloat16()
+
+
+def _close(got, ref, rows_scale=1.0):
+    """One rounding to bf16 (2^-9 of the value) and fp32 sums of at most 8192 products (1e-5 of the rows' size)."""
+    err = (got.double() - ref).abs()
+    assert bool((err <= 2.0 ** -8 * ref.abs() + 2e-5 * ref.abs().max() * rows_scale).all()), err.max()
+
+
+@pytest.mark.parametrize("m", (1, 5, 16))
+@pytest.mark.parametrize("n,k", SHAPES)
+def test_product_norm_and_residual(n, k, m):
+    x, w = _operands(m, n, k)
+    assert D.few_takes(m, n, k)
+    pw = D.PackedWeight(w)
+    ref = x.double() @ w.double().T
+    _close(D.skinny_few(x, pw), ref)
+    scale = torch.rsqrt(x.double().pow(2).mean(1, keepdim=True) + 1e-3)
+    _close(D.skinny_few(x, pw, norm=True, eps=1e-3), ref * scale)
+    out = torch.randn(m, n, device="cuda").bfloat16()
+    want = out.double() + ref
+    assert D.skinny_few(x, pw, out=out, resid=True) is out
+    _close(out, want)
+
+
+@pytest.mark.parametrize("act", ("silu", "gelu_tanh"))
+@pytest.mark.parametrize("n,k,m", ((32, 512, 1), (4128, 1024, 7), (16384, 512, 16)))
+def test_gated(n, k, m, act):
+    x, w = _operands(m, n, k, 1)
+    got = D.skinny_few(x, D.PackedWeight(w, swiglu=True, act=act), norm=True)
+    z = x.double() @ w.double().T * torch.rsqrt(x.double().pow(2).mean(1, keepdim=True) + 1e-5)
+    g, u = z.chunk(2, 1)
+    g = torch.nn.functional.silu(g) if act == "silu" else torch.nn.functional.gelu(g, approximate="tanh")
+    _close(got, g * u, rows_scale=4.0)  # both factors' errors
+
+
+@pytest.mark.parametrize("m", (1, 6, 16))
+@pytest.mark.parametrize("heads,kv", ((4, 2), (32, 8), (32, 16)))
+def test_rope_and_cache_as_the_separate_launch(heads, kv, m):
+    k = 1024
+    x, w = _operands(m, (heads + 2 * kv) * 128, k, 2)
+    from kgs.ops.transformer import rope_tables
+
+    cos, sin = rope_tables(256, 128, 10000.0, "cuda")
+    pos = torch.arange(m, dtype=torch.int32, device="cuda") * 13 % 200
+    slots = torch.randperm(8 * 32, device="cuda")[:m].int()
+    slots[m // 2] = -1
+    caches = [D.PagedKVCache(1, 8, kv, "cuda") for _ in range(2)]
+    got = D.skinny_few(x, D.PackedWeight(w, rope=(heads, kv)), norm=True,
+                       rope={"cos": cos, "sin": sin, "positions": pos, "slots": slots, "cache": caches[0].layer(0)})
+    want = D.skinny_few(x, D.PackedWeight(w), norm=True)  # the same sums, row by row
+    D.rope_cache_(want, cos, sin, pos, slots, caches[1].layer(0), heads, kv)
+    assert torch.equal(got, want) and torch.equal(caches[0].data, caches[1].data)
+
+
+def test_what_it_does_not_take():
+    for m, n, k in ((17, 4096, 4096), (0, 4096, 4096), (4, 4096, 768), (4, 4104, 512)):
+        assert not D.few_takes(m, n, k)
+    assert not D.few_takes(4, 4096, 4096, fp8=True)
+    x, w = _operands(4, 32, 512)
+    with pytest.raises(ValueError):
+        D.skinny_few(x, D.PackedWeight(w), resid=True)
+
+
+def test_infinite_and_missing_values_stay_in_their_rows():
+    x, w = _operands(5, 64, 512, 3)
+    x = x.clone()
+    x[2, 7], x[4, 9] = float("nan"), float("inf")
+    got = D.skinny_few(x, D.PackedWeight(w), norm=True).float()
+    assert got[2].isnan().all() and got[[0, 1, 3]].isfinite().all() and not (got[4].abs() > 0).logical_and(got[4].isfinite()).any()

@@ -507,18 +507,38 @@ def _workspace(device: torch.device, floats: int, ints: int):
     return ws, cnt
 
 
-EPI_SWIGLU, EPI_RMS, EPI_RESID, EPI_ROPE, EPI_GELU, EPI_CLAMPED, EPI_SUMS_IN, EPI_SUMS_OUT = 1, 2, 4, 8, 16, 32, 64, 128
+EPI_SWIGLU, EPI_RMS, EPI_RESID, EPI_ROPE, EPI_GELU, EPI_CLAMPED, EPI_SUMS_IN, EPI_SUMS_OUT, EPI_OWN = 1, 2, 4, 8, 16, 32, 64, 128, 256
 SUM_WORDS, SUM_MAX_N = 8, 8192  # integers of a row's exact sum of squares (decode.hip add_exact), longest row
 GATE_EPI = {"silu": 0, "gelu_tanh": EPI_GELU, "clamped": EPI_CLAMPED}
-
-
-FEW_ROWS = 8  # of a fused layer; above, every workgroup's way through all of x costs what the statistics do (16 rows 4096 wide 504 us a step / 515)
 
 
 @lru_cache(maxsize=4096)
 def few_takes(m: int, n: int, k: int, fp8: bool = False) -> bool:
     """Whether the kernel of few rows (native/kernels/decode_few.hip) runs ``m`` rows of an ``[n, k]`` weight: up to 16 of bf16 weights."""
     return not fp8 and 0 < m <= 16 and bool(_lib.lib().kgs_skinny_few_ok(m, n, k))
+
+
+@lru_cache(maxsize=4096)
+def _own_by_skinny(m: int, n: int, k: int, fp8: bool, rope: bool) -> bool:
+    v, ks = _skinny_plan(m, n, k, fp8, rope)
+    return skinny_takes(m, n, k, fp8, rope) and not (ks > 1 and v in KIN_VARIANTS)
+
+
+@lru_cache(maxsize=4096)
+def own_takes(m: int, n: int, k: int, fp8: bool = False, rope: bool = False) -> bool:
+    """Whether :func:`own_gemm` takes a norm in front of an ``[n, k]`` weight of ``m`` rows: up to 64 of bf16 weights that tile."""
+    return not fp8 and 0 < m <= 64 and (few_takes(m, n, k) or _own_by_skinny(m, n, k, False, rope))
+
+
+def own_gemm(x: torch.Tensor, w: PackedWeight, out: torch.Tensor | None = None, norm: bool = False, resid: bool = False,
+             eps: float = 1e-5, rope: dict | None = None, counters: torch.Tensor | None = None) -> torch.Tensor:
+    """:func:`skinny_gemm` with ``norm`` or ``resid``, by :func:`skinny_few` up to 8 rows, and up to 16 where W has at most
+    512 strips and x 128k values: beyond, x through LDS is shared by more of W, or split over workgroups (us at 16 rows, few / others: 28672x4096 51
+    / 43, 4096x14336 26.3 / 23.5, but 6144x4096 13.7 / 16.2, 4096x4096 10.5 / 11)."""
+    m, k = x.shape
+    if few_takes(m, w.n, k, w.fp8) and (m <= 8 or (w.n <= 512 * 16 and m * k <= 128 << 10) or not _own_by_skinny(m, w.n, k, w.fp8, bool(w.rope))):
+        return skinny_few(x, w, out, norm, resid, eps, rope)
+    return skinny_gemm(x, w, out, norm=norm, resid=resid, eps=eps, rope=rope, counters=counters)
 
 
 def _rope_args(rope: dict, m: int):
@@ -566,7 +586,8 @@ def skinny_few(x: torch.Tensor, w: PackedWeight, out: torch.Tensor | None = None
 def skinny_gemm(x: torch.Tensor, w: PackedWeight, out: torch.Tensor | None = None,
                 ksplit: int | None = None, variant: int = 0, rms: torch.Tensor | None = None,
                 resid_ss: torch.Tensor | None = None, zero: torch.Tensor | None = None,
-                eps: float = 1e-5, rope: dict | None = None, counters: torch.Tensor | None = None) -> torch.Tensor:
+                eps: float = 1e-5, rope: dict | None = None, counters: torch.Tensor | None = None, norm: bool = False,
+                resid: bool = False) -> torch.Tensor:
     """``x @ W^T`` (bf16, fp32 accumulate) for ``x: [M <= 256, K]`` row-major;
     ``silu(x @ Wg^T) * (x @ Wu^T)`` for a ``swiglu`` weight. Fused epilogues:
 
@@ -584,6 +605,8 @@ def skinny_gemm(x: torch.Tensor, w: PackedWeight, out: torch.Tensor | None = Non
       (fp32 ``[max_pos, 64]``), ``positions`` and ``slots`` (int32 ``[M]``) and
       ``cache`` (the layer's bf16 pages): q / k rotated at their positions, k / v
       written into their cache slots -- :func:`rope_cache_` in the epilogue;
+    * ``norm`` (instead of ``rms``; up to 64 rows of bf16 weights): RMSNorm folded in by statistics that the product
+      makes from x itself; ``resid`` (instead of ``resid_ss``): the residual update alone;
     * ``counters`` (zeroed int32, a value per W strip; left zeroed): instead of the per-GPU ones, with
       slabs of the call's own -- calls that other streams' calls may overlap."""
     if x.dtype != torch.bfloat16 or not x.is_cuda or x.dim() != 2 or x.stride(1) != 1:
@@ -600,8 +623,10 @@ def skinny_gemm(x: torch.Tensor, w: PackedWeight, out: torch.Tensor | None = Non
     rps, kpc, mpad = skinny_geometry(m, variant)
     if w.n % rps or k % kpc:
         raise ValueError(f"skinny GEMM needs N % {rps} == 0 and K % {kpc} == 0 (N={w.n}, K={k})")
+    if (norm and (rms is not None or resid or resid_ss is not None or w.fp8 or m > 64 or (ks > 1 and variant in KIN_VARIANTS))) or (resid and (resid_ss is not None or rope is not None)):
+        raise ValueError("norm: a product of up to 64 rows of bf16 weights without rms or a residual update; resid: without resid_ss and rope")
     epi = (EPI_SWIGLU | GATE_EPI[w.act.act] if w.swiglu else 0) | (EPI_RMS if rms is not None else 0) | \
-        (EPI_RESID if resid_ss is not None else 0)
+        (EPI_RMS | EPI_OWN if norm else 0) | (EPI_RESID if resid or resid_ss is not None else 0)
     for t, name, sums in ((rms, "rms", EPI_SUMS_IN), (resid_ss, "resid_ss", EPI_SUMS_OUT), (zero, "zero", EPI_SUMS_OUT)):
         if t is None:
             continue
@@ -613,12 +638,12 @@ def skinny_gemm(x: torch.Tensor, w: PackedWeight, out: torch.Tensor | None = Non
             raise ValueError(f"{name} must be contiguous")
     if epi & EPI_SUMS_OUT and resid_ss is not None and zero is not None and resid_ss.dtype != zero.dtype:
         raise ValueError("resid_ss and zero must be of one kind")
-    if resid_ss is not None:
+    if epi & EPI_RESID:
         if w.swiglu or out is None or tuple(out.shape) != (m, w.n):
             raise ValueError("resid_ss needs the residual stream as out [M, N] (and no swiglu)")
     if out is None:
         out = torch.empty((m, w.n_out), dtype=torch.bfloat16, device=x.device)
-    need = ks * mpad * w.n if ks > 1 else 0
+    need = ks * mpad * (w.n + (w.n // rps if norm else 0)) if ks > 1 else 0
     if counters is None:
         ws, cnt = _workspace(x.device, need, w.n // rps)
     else:
@@ -633,7 +658,7 @@ def skinny_gemm(x: torch.Tensor, w: PackedWeight, out: torch.Tensor | None = Non
         cache = _rope_args(rope, m)
         rc = _lib.lib().kgs_skinny_gemm_bf16_rope(
             w.data.data_ptr(), x.data_ptr(), out.data_ptr(), None if ws is None else ws.data_ptr(), cnt.data_ptr(), m, w.n, k, x.stride(0),
-            out.stride(0), ks, variant, epi & (EPI_RMS | EPI_SUMS_IN),
+            out.stride(0), ks, variant, epi & (EPI_RMS | EPI_SUMS_IN | EPI_OWN),
             rms.data_ptr() if rms is not None else None, 1.0 / k, float(eps), rope["cos"].data_ptr(),
             rope["sin"].data_ptr(), rope["positions"].data_ptr(), rope["slots"].data_ptr(), cache.data_ptr(),
             w.rope[0], w.rope[1], _lib.stream_handle(x.device))

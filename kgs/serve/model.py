@@ -447,10 +447,10 @@ class ServingModel:
             a = torch.empty((plan.n, c.heads * c.head_dim), dtype=torch.bfloat16, device=qkv.device)
             return attention_blocks(qkv, *self._kv(qkv), plan.items, c.heads, c.kv_heads, a, merges=plan.merges, slots=plan.slots)
 
-        x, ss = self._fused_layers(tokens, positions, slots, attend, "prefill", count, exact=True, keep=plan.keep)
+        x, ss = self._fused_layers(tokens, positions, slots, attend, "prefill", count, exact=True, keep=plan.keep, heads=plan.last.numel())
         x = x.index_select(0, plan.last)
         if ss is None:
-            out = D.skinny_few(x, self.packed_lm, norm=True, eps=c.eps)
+            out = D.own_gemm(x, self.packed_lm, norm=True, eps=c.eps, counters=count)
         else:
             out = D.skinny_gemm(x, self.packed_lm, rms=ss.index_select(1, plan.last), eps=c.eps, counters=count)
         T.op("prefill-fused lm_head")
@@ -738,7 +738,7 @@ class ServingModel:
     def _decode_fused(self, tokens, positions, slots, block_tables, ctx_lens, pages_per_split):
         """Decode with every norm / SwiGLU / residual add inside the skinny GEMMs:
         5 GEMMs + RoPE/KV-write + attention per layer, no elementwise launches.
-        Up to 16 rows a GEMM takes the folded RMSNorm's statistic from its own input; above,
+        The consuming GEMM takes the folded RMSNorm's statistic from its own input; where one cannot,
         ss_a / ss_b carry the residual rows' sums of squares between the
         producing GEMM (residual update) and the consuming one."""
         c = self.cfg
@@ -749,14 +749,14 @@ class ServingModel:
                                             pages_per_split=pages_per_split, tickets=tickets)
 
         x, ss = self._fused_layers(tokens, positions, slots, attend, "decode", None, exact=False, tickets=tickets)
-        out = D.skinny_few(x, self.packed_lm, norm=True, eps=c.eps) if ss is None else D.skinny_gemm(x, self.packed_lm, rms=ss, eps=c.eps)
+        out = D.own_gemm(x, self.packed_lm, norm=True, eps=c.eps) if ss is None else D.skinny_gemm(x, self.packed_lm, rms=ss, eps=c.eps)
         T.op("decode-fused lm_head")
         return out
 
-    def _few(self, m: int) -> bool:
-        """Whether the fused layers and the head of ``m`` rows are products of few rows, which make the norms' statistics themselves."""
-        return m <= D.FEW_ROWS and D.few_takes(m, self.packed_lm.n, self.packed_lm.k, self.packed_lm.fp8) and \
-            all(D.few_takes(m, w.n, w.k, w.fp8) for w in self.packed[0].values())
+    def _own(self, m: int, head: int) -> bool:
+        """Whether the products behind a norm of ``m`` rows' fused layers, and of ``head`` rows the LM head, make its statistics themselves."""
+        P = self.packed[0]
+        return all(D.own_takes(r, w.n, w.k, w.fp8, bool(w.rope)) for w, r in ((P["qkv"], m), (P["gate_up"], m), (self.packed_lm, head)))
 
     def _tickets(self, block_tables):
         """Tickets of the step's own for the decode rows' attention, to be cleared with its first launch; None: it takes none."""
@@ -780,8 +780,8 @@ class ServingModel:
         return x, self._norm(x, None, self.ln1[0]) if norm else None
 
     def _fused_layers(self, tokens, positions, slots, attend, kind: str, counters, exact: bool, keep=None,
-                      tickets=None):
-        """The residual rows after all layers and their sums of squares (None where :meth:`_few` products make their own); ``attend(qkv, layer)`` is the
+                      tickets=None, heads=None):
+        """The residual rows after all layers and their sums of squares (None where the products make their own, :meth:`_own`; ``heads``: rows of the LM head, all); ``attend(qkv, layer)`` is the
         attention of the rotated rows, whose keys and values are in the cache. ``exact``: statistics whose
         bits do not depend on the order in which workgroups arrive, so that equal steps give equal bits. ``keep``
         (int32): of these rows of ``tokens``, ``positions`` and ``slots`` only. ``counters`` and
@@ -792,9 +792,9 @@ class ServingModel:
         eps = c.eps
         tokens, dev = tokens.to(self.embed.device), self.embed.device
         m = (tokens if keep is None else keep).numel()
-        few = self._few(m)
+        own = self._own(m, m if heads is None else heads)
         ss = zero = None
-        if not few:
+        if not own:
             ss = torch.empty(m, dtype=torch.float32, device=dev)  # statistic for layer 0's qkv
             if exact:
                 zero = stats = torch.empty((2, D.SUM_WORDS, m), dtype=torch.int64, device=dev)
@@ -819,8 +819,8 @@ class ServingModel:
             P = self.packed[i]
             rope = {"cos": self.cos, "sin": self.sin, "positions": positions, "slots": slots,
                     "cache": self.cache.layer(i)} if P["qkv"].rope else None
-            if few:
-                qkv = D.skinny_few(x, P["qkv"], norm=True, eps=eps, rope=rope)
+            if own:
+                qkv = D.own_gemm(x, P["qkv"], norm=True, eps=eps, rope=rope, counters=counters)
             else:
                 qkv = D.skinny_gemm(x, P["qkv"], rms=ss, eps=eps, counters=counters, rope=rope)
             if rope is None:
@@ -828,10 +828,10 @@ class ServingModel:
             T.op(f"{kind}-fused L{i} qkv+rope")
             a = attend(qkv, i)
             T.op(f"{kind}-fused L{i} attention")
-            if few:
-                D.skinny_few(a, P["o"], out=x, resid=True)
-                act = D.skinny_few(x, P["gate_up"], norm=True, eps=eps)
-                D.skinny_few(act, P["down"], out=x, resid=True)
+            if own:
+                D.own_gemm(a, P["o"], out=x, resid=True, counters=counters)
+                act = D.own_gemm(x, P["gate_up"], norm=True, eps=eps, counters=counters)
+                D.own_gemm(act, P["down"], out=x, resid=True, counters=counters)
             else:
                 D.skinny_gemm(a, P["o"], out=x, resid_ss=ss_a, zero=ss_b, counters=counters)
                 act = D.skinny_gemm(x, P["gate_up"], rms=ss_a, eps=eps, counters=counters)

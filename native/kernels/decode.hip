@@ -97,7 +97,10 @@ __device__ __forceinline__ bf16x8 dequant8(u32x2 v, float s) {
 // first weights' way from memory, and a workgroup's tiles are summed in LDS before they are added (with each
 // tile's atomics and each output's conversion 1.2 us more a launch). us at 30 rows, floats / exact sums:
 // 28672x4096 43.4 / 43.6, 4096x14336 29.5 / 29.1, 4096x4096 16.9 / 16.5.
-template <int R, int MT, int KC_, bool W8 = false, bool EROPE = false, bool KIN = false, bool SUMS = false>
+// OWN (EPI_OWN; bf16 weights, batch <= 64): EPI_RMS by statistics that the workgroup makes itself, an
+// MFMA of x with itself per k-step, whose diagonal the rows' sums of squares are (decode_few.hip has the reason). KIN: each
+// wave of its K quarter; else wave c of column tile c, and with cross-workgroup split-K (not KIN) the splits' sums go behind their slabs.
+template <int R, int MT, int KC_, bool W8 = false, bool EROPE = false, bool KIN = false, bool SUMS = false, bool OWN = false>
 __global__ __launch_bounds__(256, (MT * KC_ > 32 || R * MT >= 16) ? 1 : 2) void skinny(const void* __restrict__ wpv, const unsigned short* __restrict__ x,
                                                  unsigned short* __restrict__ y, float* __restrict__ ws,
                                                  int* __restrict__ cnt, int M, int N, int K, long ldx, long ldy,
@@ -114,7 +117,7 @@ __global__ __launch_bounds__(256, (MT * KC_ > 32 || R * MT >= 16) ? 1 : 2) void 
   // arriver" flag reuses its first word after the main loop
   static_assert(!KIN || PF == KC, "KIN: one ring round per chunk");
   __shared__ __attribute__((aligned(16))) bf16x8 xs[2][KIN ? 2 * R * MT * 64 : C::CHUNK_SLOTS];
-  __shared__ float stat[SUMS ? 5 : 1][16 * MT];  // SUMS: the rows' scales; a wave's sums of squares in [1 + wave]
+  __shared__ float stat[SUMS || OWN ? 5 : 1][16 * MT];  // SUMS: the rows' scales; a wave's sums of squares in [1 + wave]. OWN: a wave's (KIN), the rows'
 
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int nstrip = N / ((KIN ? 16 : 64) * R);
@@ -191,6 +194,16 @@ __global__ __launch_bounds__(256, (MT * KC_ > 32 || R * MT >= 16) ? 1 : 2) void 
 #pragma unroll
     for (int c = 0; c < MT; ++c) acc[r][c] = f32x4v{0.f, 0.f, 0.f, 0.f};
 
+  f32x4v gram[OWN && KIN ? MT : 1];  // OWN: x . x^T of the column tiles (KIN), of the wave's own
+#pragma unroll
+  for (int c = 0; c < (OWN && KIN ? MT : 1); ++c) gram[c] = f32x4v{0.f, 0.f, 0.f, 0.f};
+  // its diagonal: row m in lane 16 (m / 4) + m, element m % 4
+  [[maybe_unused]] auto diagonal = [&](const f32x4v& d, float* to) {
+    const int m = lane & 15;
+    const float lo = m & 1 ? d[1] : d[0], hi = m & 1 ? d[3] : d[2];
+    if (lane >> 4 == m >> 2) to[m] = m & 2 ? hi : lo;
+  };
+
   // Every load below is unconditional (indices clamped to the last step /
   // chunk: a few redundant L2-hit reloads at the tail) so hipcc can count
   // vmcnt through the loop instead of draining the ring before each MFMA.
@@ -246,6 +259,10 @@ __global__ __launch_bounds__(256, (MT * KC_ > 32 || R * MT >= 16) ? 1 : 2) void 
 #pragma unroll
             for (int c = 0; c < MT; ++c) acc[r][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wdq, xf[p][c], acc[r][c], 0, 0, 0);
           }
+          if constexpr (OWN) {
+#pragma unroll
+            for (int c = 0; c < MT; ++c) gram[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xf[p][c], xf[p][c], gram[c], 0, 0, 0);
+          }
           const int sn = min(s0 + p + PF, nsteps - 1);
 #pragma unroll
           for (int r = 0; r < R; ++r) wf[p][r] = __builtin_nontemporal_load(wrow[r] + (long)sn * 64);
@@ -257,6 +274,10 @@ __global__ __launch_bounds__(256, (MT * KC_ > 32 || R * MT >= 16) ? 1 : 2) void 
     // the four K quarters of the strip: waves 1-3 hand theirs to wave 0 (slot 0
     // of xs stays free for the split-K flag); summed in wave order
     f32x4v* red = (f32x4v*)&xs[0][1];
+    if constexpr (OWN) {
+#pragma unroll
+      for (int c = 0; c < MT; ++c) diagonal(gram[c], &stat[1 + w][16 * c]);
+    }
     if (w > 0) {
 #pragma unroll
       for (int r = 0; r < R; ++r)
@@ -286,6 +307,10 @@ __global__ __launch_bounds__(256, (MT * KC_ > 32 || R * MT >= 16) ? 1 : 2) void 
 #pragma unroll
     for (int kk = 0; kk < KC; ++kk) {
       const int p = kk % PF;
+      if constexpr (OWN) {
+        const bf16x8 o = xb[(kk * MT + (w < MT ? w : 0)) * 64];
+        gram[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(o, o, gram[0], 0, 0, 0);
+      }
       bf16x8 wdq[R];
 #pragma unroll
       for (int r = 0; r < R; ++r) {
@@ -306,6 +331,10 @@ __global__ __launch_bounds__(256, (MT * KC_ > 32 || R * MT >= 16) ? 1 : 2) void 
     store_x((chunk + 1) & 1);
     __syncthreads();
   }
+  if constexpr (OWN) {
+    if (w < MT) diagonal(gram[0], &stat[0][16 * w]);
+    __syncthreads();
+  }
   }  // !KIN
 
   // C^T tile (r, c): lane holds column m = 16c + (lane & 15), rows n = 16*(nt0+r) + 4*(lane>>4) + i
@@ -314,7 +343,13 @@ __global__ __launch_bounds__(256, (MT * KC_ > 32 || R * MT >= 16) ? 1 : 2) void 
   // (the SWIGLU / RESID exchanges are cross-lane)
   auto emit = [&](f32x4v v, int m, int r) {
     const int ms = m < M ? m : M - 1;
-    if (ep.mode & EPI_RMS) v *= SUMS ? stat[0][ms] : rsqrtf(ep.ss_in[ms] * ep.inv_k + ep.eps);
+    if constexpr (OWN) {
+      float ss = stat[KIN ? 1 : 0][ms];
+      if constexpr (KIN) ss = ((ss + stat[2][ms]) + stat[3][ms]) + stat[4][ms];
+      v *= rsqrtf(ss * ep.inv_k + ep.eps);
+    } else {
+      if (ep.mode & EPI_RMS) v *= SUMS ? stat[0][ms] : rsqrtf(ep.ss_in[ms] * ep.inv_k + ep.eps);
+    }
     if (ep.mode & EPI_SWIGLU) {
       f32x4v u;
 #pragma unroll
@@ -346,7 +381,7 @@ __global__ __launch_bounds__(256, (MT * KC_ > 32 || R * MT >= 16) ? 1 : 2) void 
         sq = r0 * r0 + r1 * r1 + r2 * r2 + r3 * r3;
       }
       sq = wsum16(sq);  // lanes of one column m (g = 0..3)
-      if (m < M && g == 0) {
+      if (m < M && g == 0 && ep.ss_out) {
         if (SUMS && (ep.mode & EPI_SUMS_OUT)) stat[1 + w][m] = r ? stat[1 + w][m] + sq : sq;
         else atomicAdd(ep.ss_out + m, sq);
       }
@@ -458,6 +493,11 @@ __global__ __launch_bounds__(256, (MT * KC_ > 32 || R * MT >= 16) ? 1 : 2) void 
       }
     }
   }
+  constexpr int SR = 16 * MT;  // OWN: sums of squares [split][strip][SR] behind the slabs
+  const __amdgpu_buffer_rsrc_t sr = rsrc(ws + ksplit * sstride, OWN ? (unsigned)(ksplit * nstrip * SR * 4) : 0);
+  if constexpr (OWN && !KIN) {
+    if (tid < SR) st1_sc1(sr, (unsigned)(((split * nstrip + strip) * SR + tid) * 4), stat[0][tid]);
+  }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
   int* flag = (int*)&xs[0][0];
@@ -473,6 +513,14 @@ __global__ __launch_bounds__(256, (MT * KC_ > 32 || R * MT >= 16) ? 1 : 2) void 
   }
   __syncthreads();
   if (!*flag || (KIN && w != 0)) return;
+  if constexpr (OWN && !KIN) {
+    if (tid < SR) {
+      float ss = 0.f;
+      for (int sp = 0; sp < ksplit; ++sp) ss += ld1_sc1(sr, (unsigned)(((sp * nstrip + strip) * SR + tid) * 4));
+      stat[0][tid] = ss;
+    }
+    __syncthreads();
+  }
   if constexpr (MT > 8) {
     if (ep.mode == 0) {
 #pragma unroll
@@ -1570,6 +1618,16 @@ hipError_t launch_skinny(const void* wp, const void* x, void* y, float* ws, int*
     return hipGetLastError();
   };
   const bool rope = ep.mode & EPI_ROPE, sums = ep.mode & (EPI_SUMS_IN | EPI_SUMS_OUT);
+  if (ep.mode & EPI_OWN) {
+    if constexpr (!W8 && MT <= 4) {
+      if ((KIN && ksplit != 1) || sums) return hipErrorInvalidValue;
+      if constexpr (R == 1) {
+        if (rope) return run(skinny<R, MT, KC, false, true, KIN, false, true>);
+      }
+      if (!rope) return run(skinny<R, MT, KC, false, false, KIN, false, true>);
+    }
+    return hipErrorInvalidValue;
+  }
   if constexpr (!W8 && MT <= 4 && R == 1) {  // the fused layer's qkv variants (kgs/ops/decode.py rope_variant)
     if (rope) return sums ? run(skinny<R, MT, KC, false, true, KIN, true>) : run(skinny<R, MT, KC, false, true, KIN>);
   }
@@ -1604,9 +1662,9 @@ KGS_EXPORT int kgs_skinny_geometry(int M, int* rows_per_strip, int* k_per_chunk,
 
 // y[M, N] (bf16, row stride ldy) = x[M, K] (row stride ldx) . W^T with W
 // prepacked ([N/16][K/32][64][8] bf16). ksplit must divide K / k_per_chunk;
-// with ksplit > 1, ws holds ksplit * mpad * N floats and cnt N / rows_per_strip
+// with ksplit > 1, ws holds ksplit * mpad * N floats (OWN: and ksplit * mpad * N / rows_per_strip) and cnt N / rows_per_strip
 // zero-initialised ints (left zeroed on return). epi: EPI_* flags (SWIGLU: y is
-// [M, N/2]; RMS needs ss_in[M]; RESID accumulates into y and ss_out[M]);
+// [M, N/2]; RMS needs ss_in[M], or OWN; RESID accumulates into y and, unless null, ss_out[M]);
 // ss_zero (optional, [M] floats) is cleared at kernel start. With EPI_SUMS_IN ss_in, with EPI_SUMS_OUT
 // ss_out and ss_zero hold 64-bit integers [8][M] (16-B aligned), N at most 8192 for ss_out.
 namespace {
@@ -1637,7 +1695,7 @@ KGS_EXPORT int kgs_skinny_gemm_bf16_rope(const void* wp, const void* x, void* y,
                                         const float* sinv, const int* pos, const int* slot, void* cache, int H,
                                         int HKV, hipStream_t s) {
   using namespace kgs::dec;
-  if (epi & ~(EPI_RMS | EPI_SUMS_IN)) return KGS_ERR_ARG;
+  if (epi & ~(EPI_RMS | EPI_SUMS_IN | EPI_OWN)) return KGS_ERR_ARG;
   if (H <= 0 || HKV <= 0 || H % HKV || N != (H + 2 * HKV) * HD) return KGS_ERR_SHAPE;
   if (!cosv || !sinv || !pos || !slot || !al16(cache)) return KGS_ERR_ARG;
   SkinnyEpi r{};
@@ -1661,12 +1719,14 @@ int skinny_fused(const void* wp, const void* x, void* y, float* ws, int* cnt, in
   const int rc = kgs_skinny_variant_geometry(variant, M, &rps, &kpc, &mpad);
   if (rc) return rc;
   if (variant == 0) variant = default_variant(mt_for(M));
-  if (epi & ~(EPI_SWIGLU | EPI_RMS | EPI_RESID | EPI_ROPE | EPI_GELU | EPI_CLAMPED | EPI_SUMS_IN | EPI_SUMS_OUT) ||
+  if (epi & ~(EPI_SWIGLU | EPI_RMS | EPI_RESID | EPI_ROPE | EPI_GELU | EPI_CLAMPED | EPI_SUMS_IN | EPI_SUMS_OUT | EPI_OWN) ||
       ((epi & (EPI_GELU | EPI_CLAMPED)) && !(epi & EPI_SWIGLU)) || ((epi & EPI_SWIGLU) && (epi & EPI_RESID)))
     return KGS_ERR_ARG;
   if ((epi & EPI_ROPE) && (rope.cache == nullptr || (epi & (EPI_SWIGLU | EPI_RESID)) || wscale != nullptr))
     return KGS_ERR_ARG;
-  if (((epi & EPI_RMS) && ss_in == nullptr) || ((epi & EPI_RESID) && ss_out == nullptr)) return KGS_ERR_ARG;
+  if ((epi & EPI_RMS) && !(epi & EPI_OWN) && ss_in == nullptr) return KGS_ERR_ARG;
+  if ((epi & EPI_OWN) && (!(epi & EPI_RMS) || (epi & (EPI_RESID | EPI_SUMS_IN | EPI_SUMS_OUT)) || M > 64 || wscale)) return KGS_ERR_ARG;
+  if ((epi & EPI_SUMS_OUT) && (epi & EPI_RESID) && ss_out == nullptr) return KGS_ERR_ARG;
   if (N <= 0 || K <= 0 || N % rps || K % kpc || ldx < K || ldy < ((epi & EPI_SWIGLU) ? N / 2 : N))
     return KGS_ERR_SHAPE;
   if ((epi & EPI_RESID) && (epi & EPI_SUMS_OUT) && N > SUM_MAX_N) return KGS_ERR_SHAPE;

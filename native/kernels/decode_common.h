@@ -83,7 +83,7 @@ __device__ __forceinline__ float ld1_sc1(__amdgpu_buffer_rsrc_t r, unsigned off)
 //               paged cache slot slot[m] -- the rope_cache launch, folded in.
 // Together they remove both add_rmsnorm launches, the SwiGLU launch and the
 // RoPE / KV-write launch from a decode layer (kgs/serve/model.py fused path).
-enum { EPI_SWIGLU = 1, EPI_RMS = 2, EPI_RESID = 4, EPI_ROPE = 8, EPI_GELU = 16, EPI_CLAMPED = 32, EPI_SUMS_IN = 64, EPI_SUMS_OUT = 128 };
+enum { EPI_SWIGLU = 1, EPI_RMS = 2, EPI_RESID = 4, EPI_ROPE = 8, EPI_GELU = 16, EPI_CLAMPED = 32, EPI_SUMS_IN = 64, EPI_SUMS_OUT = 128, EPI_OWN = 256 };
 struct SkinnyEpi {
   int mode;
   int zero_words;  // 4-byte words of ss_zero

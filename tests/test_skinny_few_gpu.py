@@ -1,5 +1,5 @@
 """Products of few rows (native/kernels/decode_few.hip) against the plain product in float64: the edges of its splits over waves
-and tiles, each epilogue, and the RMSNorm whose statistics it makes itself."""
+and tiles, each epilogue, and the RMSNorm whose statistics it makes itself -- as decode.hip's skinny does up to 64 rows."""
 import pytest
 import torch
 
@@ -84,3 +84,49 @@ def test_infinite_and_missing_values_stay_in_their_rows():
     x[2, 7], x[4, 9] = float("nan"), float("inf")
     got = D.skinny_few(x, D.PackedWeight(w), norm=True).float()
     assert got[2].isnan().all() and got[[0, 1, 3]].isfinite().all() and not (got[4].abs() > 0).logical_and(got[4].isfinite()).any()
+
+
+# x through LDS in one K slice and in several, K split inside the workgroup, in one and in two tiles; each column tile's edge
+@pytest.mark.parametrize("variant,ksplit,n,k,m", [(None, None, *nk, m) for nk in ((6144, 4096), (2048, 2048)) for m in (12, 17, 32, 33, 64)] + [
+    (1, 1, 256, 1024, 12), (3, 2, 256, 2048, 16), (4, 4, 128, 2048, 17), (22, 1, 64, 1024, 32), (23, 1, 64, 2048, 31), (10, 2, 192, 1024, 33),
+    (24, 1, 64, 1024, 64), (25, 1, 128, 1024, 49)])
+def test_skinny_norm_by_its_own_statistics(variant, ksplit, n, k, m):
+    x, w = _operands(m, n, k, 4)
+    pw = D.PackedWeight(w)
+    ref = x.double() @ w.double().T
+    want = ref * torch.rsqrt(x.double().pow(2).mean(1, keepdim=True) + 1e-3)
+    for _ in range(2):  # the second call finds the first one's slabs and tickets
+        got = D.own_gemm(x, pw, norm=True, eps=1e-3) if variant is None else D.skinny_gemm(x, pw, ksplit=ksplit, variant=variant, norm=True, eps=1e-3)
+        _close(got, want)
+    out = torch.randn(m, n, device="cuda").bfloat16()
+    want = out.double() + ref
+    _close(D.own_gemm(x, pw, out=out, resid=True), want)
+
+
+@pytest.mark.parametrize("m", (9, 24, 40))
+def test_skinny_rope_by_its_own_statistics(m):
+    from kgs.ops.transformer import rope_tables
+
+    for n, k, heads, kv in ((6144, 4096, 32, 8), (3072, 2048, 16, 4)):
+        x, w = _operands(m, n, k, 5)
+        cos, sin = rope_tables(256, 128, 10000.0, "cuda")
+        pos, slots = torch.arange(m, dtype=torch.int32, device="cuda"), torch.randperm(256, device="cuda")[:m].int()
+        caches = [D.PagedKVCache(1, 8, kv, "cuda") for _ in range(2)]
+        rope = {"cos": cos, "sin": sin, "positions": pos, "slots": slots}
+        pw = D.PackedWeight(w, rope=(heads, kv))
+        ss = x.float().pow(2).sum(1)
+        got = D.own_gemm(x, pw, norm=True, rope={**rope, "cache": caches[0].layer(0)})
+        want = D.skinny_gemm(x, pw, rms=ss, rope={**rope, "cache": caches[1].layer(0)})
+        # the statistics' last bits and, up to 16 rows, the order of the sums: one unit of bf16 before the rotation
+        assert float((got.float() - want.float()).norm() / want.float().norm()) < 2.0 ** -8
+        assert float((caches[0].data.float() - caches[1].data.float()).norm() / caches[1].data.float().norm()) < 2.0 ** -8
+
+
+def test_norm_and_resid_are_refused_where_they_do_not_go():
+    x, w = _operands(70, 4096, 2048, 6)
+    pw = D.PackedWeight(w)
+    ss = torch.zeros(70, device="cuda")
+    for kw in ({"norm": True}, {"norm": True, "rms": ss}, {"resid": True}, {"resid": True, "resid_ss": ss, "out": x}):
+        with pytest.raises(ValueError):
+            D.skinny_gemm(x, pw, **kw)
+    assert not D.own_takes(65, 4096, 2048) and not D.own_takes(16, 4096, 2048, fp8=True)

@@ -104,6 +104,7 @@ _SIGS = {
     "kgs_skinny_gemm_bf16_fused": ([_c_void_p] * 5 + [_c_int] * 3 + [_c_long, _c_long] + [_c_int] * 3 +
                                    [_c_void_p] * 3 + [ctypes.c_float, ctypes.c_float, _c_void_p, ctypes.c_float,
                                                       _c_void_p], _c_int),
+    "kgs_skinny_slabs": ([_c_void_p] * 3 + [_c_int] * 3 + [_c_long] + [_c_int] * 2 + [_c_void_p], _c_int),
     "kgs_skinny_few_ok": ([_c_int] * 3, _c_int),
     "kgs_skinny_few": ([_c_void_p] * 3 + [_c_int] * 3 + [_c_long, _c_long, _c_int, ctypes.c_float, ctypes.c_float] + [_c_void_p] * 5 +
                        [_c_int, _c_int, _c_void_p], _c_int),
@@ -133,7 +134,7 @@ _SIGS = {
     "kgs_paged_decode_rope_bf16": ([_c_void_p, _c_int] + [_c_void_p] * 11 + [_c_int] * 7 +
                                    [_c_long, ctypes.c_float, _c_int, _c_int, _c_void_p], _c_int),
     # hyper-connections, latent attention, delta rule (hyper.hip, latent.hip, delta.hip, activation.hip)
-    "kgs_hyper_step": ([_c_void_p] * 7 + [_c_int] * 3 + [_c_long] * 2 + [ctypes.c_float, _c_int, _c_void_p], _c_int),
+    "kgs_hyper_step": ([_c_void_p] * 7 + [_c_int] * 3 + [_c_long] * 2 + [ctypes.c_float, _c_int, _c_int, _c_void_p], _c_int),
     "kgs_hyper_embed": ([_c_void_p] * 7 + [_c_int] * 3 + [_c_long] * 2 + [ctypes.c_float, _c_int, _c_void_p], _c_int),
     "kgs_act_mul": ([_c_void_p] * 2 + [_c_int] * 2 + [_c_long] * 2 + [_c_int, ctypes.c_float, _c_int, _c_void_p], _c_int),
     "kgs_softcap": ([_c_void_p] * 2 + [_c_int] * 2 + [_c_long, ctypes.c_float, _c_int, _c_void_p], _c_int),

@@ -541,6 +541,36 @@ def own_gemm(x: torch.Tensor, w: PackedWeight, out: torch.Tensor | None = None, 
     return skinny_gemm(x, w, out, norm=norm, resid=resid, eps=eps, rope=rope, counters=counters)
 
 
+@lru_cache(maxsize=4096)
+def slab_split(m: int, n: int, k: int, cus: int = CUS) -> tuple[int, int] | None:
+    """(W tiles a wave, K slices) of :func:`skinny_slabs`, or None: up to 64 rows of W of 64 rows a workgroup (128 from N = 4096 on),
+    in as many slices, 16 at most and of 128 at least, as leave one workgroup a CU. us at 32 rows in 4 / 8 / 16 slices: 2048x8192 12.9 / 8.8 /
+    9.1, 4096x14336 28.9 / 20.9 / 23.6, 6144x4096 11.8 / 14.5 / -."""
+    r = 2 if n >= 4096 and n % 128 == 0 else 1
+    if not 0 < m <= 64 or n % (64 * r) or k % 128:
+        return None
+    tiles, ns = n // (64 * r), 1
+    while ns < 16 and 2 * ns * tiles <= cus and k % (256 * ns) == 0:
+        ns *= 2
+    return r, ns
+
+
+def skinny_slabs(x: torch.Tensor, w: PackedWeight) -> torch.Tensor:
+    """``x @ W^T`` of up to 64 rows of a plain bf16 weight as fp32 parts ``[slices, M, N]`` of its sum, for a consumer that adds them
+    (native/kernels/decode_slabs.hip; :func:`slab_split`)."""
+    if x.dtype != torch.bfloat16 or not x.is_cuda or x.dim() != 2 or x.stride(1) != 1 or x.shape[1] != w.k:
+        raise ValueError("x must be a row-major bf16 GPU matrix [M, K]")
+    m, k = x.shape
+    split = None if w.fp8 or w.swiglu or w.rope else slab_split(m, w.n, k)
+    if split is None:
+        raise ValueError(f"no slices for x {tuple(x.shape)}, W [{w.n}, {w.k}]")
+    out = torch.empty((split[1], m, w.n), dtype=torch.float32, device=x.device)
+    rc = _lib.lib().kgs_skinny_slabs(w.data.data_ptr(), x.data_ptr(), out.data_ptr(), m, w.n, k, x.stride(0), *split,
+                                     _lib.stream_handle(x.device))
+    _lib.check(rc, f"skinny_slabs[{m}x{w.n}x{k}, {split}]")
+    return out
+
+
 def _rope_args(rope: dict, m: int):
     """The cache of :func:`skinny_gemm`'s ``rope``, checked."""
     cache = rope["cache"]

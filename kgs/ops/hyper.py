@@ -51,15 +51,23 @@ def hyper_embed(tokens: torch.Tensor, embed: torch.Tensor, w0: torch.Tensor, w_i
 def hyper_step(x: torch.Tensor, y: torch.Tensor | None, mix: torch.Tensor | None, w_out: torch.Tensor | None,
                w_in: torch.Tensor, w: torch.Tensor, eps: float, dtype=None, ld: int | None = None) -> torch.Tensor:
     """``x_t <- sum_s mix[s, t] x_s + w_out[t] y`` in place (``y`` None: unchanged),
-    then ``rmsnorm(sum_s w_in[s] x_s) * w`` as ``[T, ld]`` (zero past the width)."""
+    then ``rmsnorm(sum_s w_in[s] x_s) * w`` as ``[T, ld]`` (zero past the width). ``y`` fp32 ``[parts, T, >= D]``: the
+    parts of a product (:func:`kgs.ops.decode.skinny_slabs`), whose sum rounded to ``dtype`` (default bf16) it stands for."""
     T, S, D = x.shape
     _f32(x, (T, S, D), "x")
-    dtype = dtype or (y.dtype if y is not None else torch.bfloat16)
+    parts = 0
+    if y is not None and y.dim() == 3:
+        parts, dtype = y.shape[0], dtype or torch.bfloat16
+        if not parts or not y.is_contiguous():
+            raise ValueError("the parts of y must be contiguous")
+        yp = _act(y[0], T, D, torch.float32, "y")
+    else:
+        dtype = dtype or (y.dtype if y is not None else torch.bfloat16)
+        yp = 0 if y is None else _act(y, T, D, dtype, "y")
     h = _out(None, T, ld or D, dtype, x.device)
-    yp = 0 if y is None else _act(y, T, D, dtype, "y")
     rc = _lib.lib().kgs_hyper_step(x.data_ptr(), yp, 0 if y is None else _f32(mix, (S, S), "mix"),
                                    0 if y is None else _f32(w_out, (S,), "w_out"), _f32(w_in, (S,), "w_in"),
-                                   _f32(w, (D,), "w"), h.data_ptr(), T, S, D, 0 if y is None else y.stride(0),
-                                   h.stride(0), float(eps), int(dtype == torch.float32), _lib.stream_handle(x.device))
+                                   _f32(w, (D,), "w"), h.data_ptr(), T, S, D, 0 if y is None else y.stride(-2),
+                                   h.stride(0), float(eps), int(dtype == torch.float32), parts, _lib.stream_handle(x.device))
     _lib.check(rc, f"hyper_step[{T}x{S}x{D}]")
     return h

@@ -61,6 +61,15 @@ class Projection:
 
         return act_mul(y, act)
 
+    def partials(self, x: torch.Tensor) -> torch.Tensor:
+        """:meth:`__call__`, or where the product of a decode batch runs in K slices those, fp32 ``[slices, M, N]``, for a consumer
+        that adds them and rounds to bf16. One slice is stored as such (its sum is no work), and rows that 16-byte loads cannot read go the other way."""
+        p = self.packed
+        if p is None or self.gated is not None or x.dtype != torch.bfloat16 or x.stride(0) % 8 or x.data_ptr() % 16 or \
+                D.slab_split(x.shape[0], p.n, p.k) is None:
+            return self(x)
+        return D.skinny_slabs(x, p)
+
     def _gated(self, x, m):
         from .gemm import gemm_gate, gemm_nt_w4x_swiglu, gemm_swiglu, swiglu_fused_ok
 

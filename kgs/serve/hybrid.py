@@ -241,7 +241,7 @@ class LatentMixer:
             ol = latent_attention(ql, pages, r, m.heads, m.scale, hr, m.window)
             head_proj(ol, self.uv, r.nt, a, rows_out=r.rows, gate=gate, each=m.gate_each)
             T.op(f"L{self.layer} latent attention")
-        return self.o(a)
+        return self.o.partials(a) if model.adds_parts else self.o(a)
 
 
 class DeltaMixer:
@@ -270,7 +270,7 @@ class DeltaMixer:
                           b.seqs)
         y = delta_out(o, self.norm, g2, self.eps, self.ld)
         T.op(f"L{self.layer} delta rule")
-        return self.o(y)
+        return self.o.partials(y)
 
 
 class DenseFF:
@@ -282,13 +282,15 @@ class DenseFF:
         self.down = w.proj(w.mat(p + "down", model.wp, fp))
 
     def __call__(self, model, h: torch.Tensor, b: Batch) -> torch.Tensor:
-        y = self.down(self.gate_up(h))
+        y = self.down.partials(self.gate_up(h))
         T.op(f"L{self.layer} feed-forward")
         return y
 
 
 # ------------------------------------------------------------------------ model
 class HybridModel(RaggedModel):
+    adds_parts = True  # hyper_step adds a product's slices
+
     def __init__(self, cfg: RuruzenConfig, device="cuda", dtype: str = "bfloat16", seed: int = 0,
                  num_pages: int = 1024, state_slots: int = 256, weights: dict | None = None,
                  packed_decode: bool = True):

@@ -136,6 +136,7 @@ class RaggedModel:
     pad_multiple = 1  # portions are not padded
     has_state = False
     delta_chunks = False  # batches carry the delta rule's split into chunks
+    adds_parts = False  # what follows a mixer takes its product as fp32 slices too (Projection.partials)
 
     def __init__(self):
         self._fixed: dict = {}

@@ -40,6 +40,8 @@ struct Args {
   long ldy, ldh, lde;
   int D;
   float eps;
+  const float* parts;   // y as ns fp32 parts [ns, T, ldy] instead, rounded to T once they are added; ns 0: none
+  int ns;
 };
 
 template <typename T>
@@ -75,7 +77,8 @@ __device__ __forceinline__ void st4(T* p, float4 v) {
   }
 }
 
-// sum over the workgroup, the same value in every thread; red: NT / 64 floats
+// sum over the workgroup of N threads, the same value in every thread; red: N / 64 floats
+template <int N = NT>
 __device__ __forceinline__ float block_sum(float v, float* red) {
   v = wave_sum(v);
   __syncthreads();
@@ -83,8 +86,36 @@ __device__ __forceinline__ float block_sum(float v, float* red) {
   __syncthreads();
   float s = 0.f;
 #pragma unroll
-  for (int i = 0; i < NT / 64; ++i) s += red[i];
+  for (int i = 0; i < N / 64; ++i) s += red[i];
   return s;
+}
+
+// y[t][d ..] rounded to T from its parts, added in their order; eight loads at a time on their way
+template <typename T, int V>
+__device__ __forceinline__ float4 add_parts(const Args& a, long t, long rows, int d) {
+  float4 y = make_float4(0.f, 0.f, 0.f, 0.f);
+  for (int i0 = 0; i0 < a.ns; i0 += 8) {
+    float4 v[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      if (i0 + j < a.ns) {
+        const float* p = a.parts + ((i0 + j) * rows + t) * a.ldy + d;
+        if constexpr (V == 4) v[j] = *(const float4*)p;
+        else v[j].x = *p;
+      }
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      if (i0 + j < a.ns) {
+        y.x += v[j].x;
+        if constexpr (V == 4) {
+          y.y += v[j].y;
+          y.z += v[j].z;
+          y.w += v[j].w;
+        }
+      }
+  }
+  if constexpr (sizeof(T) == 2) y = make_float4(bf2f(f2bf(y.x)), bf2f(f2bf(y.y)), bf2f(f2bf(y.z)), bf2f(f2bf(y.w)));
+  return y;
 }
 
 __device__ __forceinline__ float4 f4_fma(float a, float4 b, float4 c) {
@@ -104,7 +135,7 @@ __global__ __launch_bounds__(NT) void step(Args a) {
   float in[S], outw[S], mix[S][S];
 #pragma unroll
   for (int s = 0; s < S; ++s) in[s] = a.in[s];
-  const bool wb = MODE == MODE_STEP && a.y != nullptr;
+  const bool wb = MODE == MODE_STEP && (a.y != nullptr || a.ns);
   if (wb) {
 #pragma unroll
     for (int s = 0; s < S; ++s) {
@@ -151,7 +182,7 @@ __global__ __launch_bounds__(NT) void step(Args a) {
 #pragma unroll
         for (int s = 0; s < S; ++s) x[s] = *(const float4*)(xr + (long)s * D + d);
         if (wb) {
-          const float4 yv = ld4(y + d);
+          const float4 yv = a.ns ? add_parts<T, 4>(a, t, gridDim.x, d) : ld4(y + d);
           float4 n[S];
 #pragma unroll
           for (int q = 0; q < S; ++q) {
@@ -175,7 +206,7 @@ __global__ __launch_bounds__(NT) void step(Args a) {
 #pragma unroll
         for (int s = 0; s < S; ++s) x[s] = xr[(long)s * D + d];
         if (wb) {
-          const float yv = ld(y + d);
+          const float yv = a.ns ? add_parts<T, 1>(a, t, gridDim.x, d).x : ld(y + d);
           float n[S];
 #pragma unroll
           for (int q = 0; q < S; ++q) {
@@ -210,12 +241,62 @@ __global__ __launch_bounds__(NT) void step(Args a) {
   for (int d = D + threadIdx.x; d < a.ldh; d += NT) st(h + d, 0.f);
 }
 
+// MODE_STEP of few tokens: N threads, four values of each stream a thread (D at most 4 N), everything in registers and one trip
+// through memory before the norm, one after it.
+template <typename T, int S, int N>
+__global__ __launch_bounds__(N) void step_few(Args a) {
+  __shared__ float red[N / 64];
+  const int D = a.D, d = threadIdx.x * 4;
+  const long t = blockIdx.x;
+  const bool on = d < D, wb = a.y != nullptr || a.ns;
+  float* xr = a.x + t * S * D + d;
+  float4 x[S], yv = make_float4(0.f, 0.f, 0.f, 0.f), w = yv, u = yv;
+  if (on) {
+#pragma unroll
+    for (int s = 0; s < S; ++s) x[s] = *(const float4*)(xr + (long)s * D);
+    w = *(const float4*)(a.w + d);
+    if (a.ns) yv = add_parts<T, 4>(a, t, gridDim.x, d);
+    else if (wb) yv = ld4((const T*)a.y + t * a.ldy + d);
+    if (wb) {
+      float4 n[S];
+#pragma unroll
+      for (int q = 0; q < S; ++q) {
+        const float o = a.out[q];
+        n[q] = make_float4(o * yv.x, o * yv.y, o * yv.z, o * yv.w);
+#pragma unroll
+        for (int s = 0; s < S; ++s) n[q] = f4_fma(a.mix[s * S + q], x[s], n[q]);
+      }
+#pragma unroll
+      for (int q = 0; q < S; ++q) {
+        x[q] = n[q];
+        *(float4*)(xr + (long)q * D) = n[q];
+      }
+    }
+#pragma unroll
+    for (int s = 0; s < S; ++s) u = f4_fma(a.in[s], x[s], u);
+  }
+  const float r = 1.0f / sqrtf(block_sum<N>(sq4(u), red) / D + a.eps);
+  T* h = (T*)a.h + t * a.ldh;
+  if (on) st4(h + d, make_float4(u.x * r * w.x, u.y * r * w.y, u.z * r * w.z, u.w * r * w.w));
+  for (int e = D + threadIdx.x; e < a.ldh; e += N) st(h + e, 0.f);
+}
+
+// us by the loop / here: 16 tokens 2048 wide 3.6 / 2.9, 128 4.8 / 4.0, 512 10.4 / 9.8, 768 13.7 / 13.6; 4096 wide 16 5.5 / 3.9, 256 11.3 / 9.8, 384 14.0 / 14.2
+constexpr long FEW_VALUES = 512 * 2048;
+
 template <typename T, int S, int MODE>
 static hipError_t launch_v(const Args& a, int T_, hipStream_t s) {
   const uintptr_t al = (uintptr_t)a.x | (uintptr_t)a.y | (uintptr_t)a.w | (uintptr_t)a.w0 | (uintptr_t)a.h |
-                       (uintptr_t)a.embed;
+                       (uintptr_t)a.embed | (uintptr_t)a.parts;
   const bool v4 = a.D % 4 == 0 && a.ldy % 4 == 0 && a.ldh % 4 == 0 && a.lde % 4 == 0 && (al & 15) == 0;
   const size_t lds = sizeof(float) * a.D;
+  if constexpr (MODE == MODE_STEP) {
+    if (v4 && (long)T_ * a.D <= FEW_VALUES && a.D > 1024 && a.D <= 4096) {
+      if (a.D <= 2048) hipLaunchKernelGGL((step_few<T, S, 512>), dim3(T_), dim3(512), 0, s, a);
+      else hipLaunchKernelGGL((step_few<T, S, 1024>), dim3(T_), dim3(1024), 0, s, a);
+      return hipGetLastError();
+    }
+  }
   auto k = v4 ? step<T, S, MODE, 4> : step<T, S, MODE, 1>;
   if (lds > 48 * 1024) {
     const hipError_t e = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
@@ -242,13 +323,15 @@ static hipError_t launch(const Args& a, int T_, int S, hipStream_t s) {
 }  // namespace hyper
 }  // namespace kgs
 
-// f32 != 0: y, h and embed are fp32, else bf16. y may be null (no write-back).
+// f32 != 0: y, h and embed are fp32, else bf16. y may be null (no write-back). ns > 0: y is ns fp32 parts [ns, T, ldy] whose sum,
+// rounded to h's type, it stands for.
 KGS_EXPORT int kgs_hyper_step(void* x, const void* y, const void* mix, const void* out, const void* in, const void* w,
-                              void* h, int T, int S, int D, long ldy, long ldh, float eps, int f32, hipStream_t s) {
+                              void* h, int T, int S, int D, long ldy, long ldh, float eps, int f32, int ns, hipStream_t s) {
   using namespace kgs::hyper;
+  if (ns < 0 || (ns && !y)) return KGS_ERR_ARG;
   if (T <= 0 || S <= 0 || S > MAX_STREAMS || D <= 0 || D > MAX_WIDTH || ldh < D || (y && ldy < D)) return KGS_ERR_SHAPE;
-  Args a{(float*)x, y, (const float*)mix, (const float*)out, (const float*)in, (const float*)w, h, nullptr, nullptr,
-         nullptr, y ? ldy : 0, ldh, 0, D, eps};
+  Args a{(float*)x, ns ? nullptr : y, (const float*)mix, (const float*)out, (const float*)in, (const float*)w, h, nullptr, nullptr,
+         nullptr, y ? ldy : 0, ldh, 0, D, eps, ns ? (const float*)y : nullptr, ns};
   return (int)(f32 ? launch<float, MODE_STEP>(a, T, S, s) : launch<unsigned short, MODE_STEP>(a, T, S, s));
 }
 

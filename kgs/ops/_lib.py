@@ -105,6 +105,9 @@ _SIGS = {
                                    [_c_void_p] * 3 + [ctypes.c_float, ctypes.c_float, _c_void_p, ctypes.c_float,
                                                       _c_void_p], _c_int),
     "kgs_skinny_slabs": ([_c_void_p] * 3 + [_c_int] * 3 + [_c_long] + [_c_int] * 2 + [_c_void_p], _c_int),
+    "kgs_skinny_rows": ([_c_void_p] * 3 + [_c_int] * 3 + [_c_long] * 2 + [_c_int, _c_int, _c_void_p, ctypes.c_float, ctypes.c_float, _c_void_p], _c_int),
+    "kgs_rope_cache_packed_bf16": ([_c_void_p] * 6 + [_c_long, _c_int, _c_int, _c_long, _c_void_p, _c_int, _c_void_p, ctypes.c_float,
+                                   ctypes.c_float, _c_void_p], _c_int),
     "kgs_skinny_few_ok": ([_c_int] * 3, _c_int),
     "kgs_skinny_few": ([_c_void_p] * 3 + [_c_int] * 3 + [_c_long, _c_long, _c_int, ctypes.c_float, ctypes.c_float] + [_c_void_p] * 5 +
                        [_c_int, _c_int, _c_void_p], _c_int),
@@ -118,6 +121,7 @@ _SIGS = {
                                                                                                   _c_void_p], _c_int),
     "kgs_argmax_rows_bf16": ([_c_void_p, _c_void_p, _c_int, _c_int, _c_long, _c_void_p], _c_int),
     "kgs_embed_rows_bf16": ([ctypes.POINTER(_c_void_p), ctypes.POINTER(_c_long), ctypes.c_float, _c_void_p], _c_int),
+    "kgs_splitk_add_squares_bf16": ([_c_void_p, _c_int] + [_c_void_p] * 2 + [_c_int, _c_int, _c_long, _c_void_p], _c_int),
     "kgs_splitk_add_rmsnorm_bf16": ([_c_void_p, _c_int] + [_c_void_p] * 3 + [_c_int, _c_int, _c_long, _c_long,
                                                                               ctypes.c_float, _c_void_p], _c_int),
     "kgs_paged_decode_bf16": ([_c_void_p] * 8 + [_c_int] * 7 + [_c_long, _c_long, ctypes.c_float, _c_int, _c_void_p],

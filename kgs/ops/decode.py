@@ -541,13 +541,16 @@ def own_gemm(x: torch.Tensor, w: PackedWeight, out: torch.Tensor | None = None, 
     return skinny_gemm(x, w, out, norm=norm, resid=resid, eps=eps, rope=rope, counters=counters)
 
 
+SLAB_ROWS = 96
+
+
 @lru_cache(maxsize=4096)
 def slab_split(m: int, n: int, k: int, cus: int = CUS) -> tuple[int, int] | None:
-    """(W tiles a wave, K slices) of :func:`skinny_slabs`, or None: up to 64 rows of W of 64 rows a workgroup (128 from N = 4096 on),
+    """(W tiles a wave, K slices) of :func:`skinny_slabs`, or None: up to 96 rows of W of 64 rows a workgroup (128 from N = 4096 on),
     in as many slices, 16 at most and of 128 at least, as leave one workgroup a CU. us at 32 rows in 4 / 8 / 16 slices: 2048x8192 12.9 / 8.8 /
     9.1, 4096x14336 28.9 / 20.9 / 23.6, 6144x4096 11.8 / 14.5 / -."""
     r = 2 if n >= 4096 and n % 128 == 0 else 1
-    if not 0 < m <= 64 or n % (64 * r) or k % 128:
+    if not 0 < m <= SLAB_ROWS or n % (64 * r) or k % 128:
         return None
     tiles, ns = n // (64 * r), 1
     while ns < 16 and 2 * ns * tiles <= cus and k % (256 * ns) == 0:
@@ -555,20 +558,71 @@ def slab_split(m: int, n: int, k: int, cus: int = CUS) -> tuple[int, int] | None
     return r, ns
 
 
-def skinny_slabs(x: torch.Tensor, w: PackedWeight) -> torch.Tensor:
-    """``x @ W^T`` of up to 64 rows of a plain bf16 weight as fp32 parts ``[slices, M, N]`` of its sum, for a consumer that adds them
-    (native/kernels/decode_slabs.hip; :func:`slab_split`)."""
+@lru_cache(maxsize=4096)
+def slab_rows_tiles(m: int, n: int, k: int, cus: int = CUS) -> int | None:
+    """W tiles a wave of :func:`skinny_rows`, or None: two where 128 rows a workgroup are three quarters of the CUs or more (us at 64 rows with one /
+    two: 28672x4096 58.6 / 44.4, 16384x2048 16.2 / 20.9; at 32 and fewer 32000x2048 25.3 / 30.4)."""
+    if not 0 < m <= SLAB_ROWS or n % 64 or k % 128:
+        return None
+    return 2 if m > 32 and n % 128 == 0 and 4 * (n // 128) >= 3 * cus else 1
+
+
+def _slab_operand(x: torch.Tensor, w: PackedWeight) -> tuple[int, int]:
     if x.dtype != torch.bfloat16 or not x.is_cuda or x.dim() != 2 or x.stride(1) != 1 or x.shape[1] != w.k:
         raise ValueError("x must be a row-major bf16 GPU matrix [M, K]")
-    m, k = x.shape
-    split = None if w.fp8 or w.swiglu or w.rope else slab_split(m, w.n, k)
+    return x.shape
+
+
+def skinny_slabs(x: torch.Tensor, w: PackedWeight) -> torch.Tensor:
+    """``x @ W^T`` of up to 96 rows of a bf16 weight as fp32 parts ``[slices, M, N]`` of its sum, for a consumer that adds them
+    (native/kernels/decode_slabs.hip; :func:`slab_split`). Columns in the order in which the weight is packed."""
+    m, k = _slab_operand(x, w)
+    split = None if w.fp8 or w.swiglu else slab_split(m, w.n, k)
     if split is None:
         raise ValueError(f"no slices for x {tuple(x.shape)}, W [{w.n}, {w.k}]")
     out = torch.empty((split[1], m, w.n), dtype=torch.float32, device=x.device)
     rc = _lib.lib().kgs_skinny_slabs(w.data.data_ptr(), x.data_ptr(), out.data_ptr(), m, w.n, k, x.stride(0), *split,
                                      _lib.stream_handle(x.device))
-    _lib.check(rc, f"skinny_slabs[{m}x{w.n}x{k}, {split}]")
+    if rc:
+        _lib.check(rc, f"skinny_slabs[{m}x{w.n}x{k}, {split}]")
     return out
+
+
+def skinny_rows(x: torch.Tensor, w: PackedWeight, sq: torch.Tensor | None = None, eps: float = 1e-5) -> torch.Tensor:
+    """``x @ W^T`` of up to 96 rows of a bf16 weight, or ``act(gate) * up`` of a gated one, by the kernel of :func:`skinny_slabs` in one slice;
+    ``sq`` (fp32 ``[M]``): of x's RMSNorm (its weight folded into W) by these sums of squares of its rows."""
+    m, k = _slab_operand(x, w)
+    r = None if w.fp8 or w.rope else slab_rows_tiles(m, w.n, k)
+    if r is None:
+        raise ValueError(f"no tiles for x {tuple(x.shape)}, W [{w.n}, {w.k}]")
+    if sq is not None and (sq.dtype != torch.float32 or sq.numel() != m or not sq.is_contiguous() or sq.device != x.device):
+        raise ValueError("sq must be a contiguous fp32 vector, one a row of x")
+    out = torch.empty((m, w.n_out), dtype=torch.bfloat16, device=x.device)
+    rc = _lib.lib().kgs_skinny_rows(w.data.data_ptr(), x.data_ptr(), out.data_ptr(), m, w.n, k, x.stride(0), out.stride(0), r,
+                                    EPI_SWIGLU | GATE_EPI[w.act.act] if w.swiglu else 0, None if sq is None else sq.data_ptr(),
+                                    float(eps), w.act.limit, _lib.stream_handle(x.device))
+    if rc:
+        _lib.check(rc, f"skinny_rows[{m}x{w.n}x{k}]")
+    return out
+
+
+def rope_cache_packed(parts: torch.Tensor, sq: torch.Tensor, w: PackedWeight, eps: float, rope: dict) -> torch.Tensor:
+    """The fused qkv rows ``[T, (H + 2 HKV) * 128]`` of a RoPE-packed weight whose product of the raw residual rows came as ``parts``
+    (:func:`skinny_slabs`): their sum scaled by the rows' RMSNorm (``sq``: sums of squares), rounded and rotated, k and v in the cache, as
+    :func:`skinny_gemm` with ``rope`` leaves them."""
+    slices, t, n = parts.shape
+    if not w.rope or n != w.n or parts.dtype != torch.float32 or not parts.is_contiguous() or slices not in (1, 2, 4, 8, 16):
+        raise ValueError("parts must be skinny_slabs' of a RoPE-packed weight")
+    if sq.dtype != torch.float32 or sq.numel() != t or not sq.is_contiguous():
+        raise ValueError("sq must be a contiguous fp32 vector, one a row")
+    cache = _rope_args(rope, t)
+    qkv = torch.empty((t, n), dtype=torch.bfloat16, device=parts.device)
+    rc = _lib.lib().kgs_rope_cache_packed_bf16(qkv.data_ptr(), rope["cos"].data_ptr(), rope["sin"].data_ptr(), rope["positions"].data_ptr(),
+                                               rope["slots"].data_ptr(), cache.data_ptr(), t, *w.rope, n, parts.data_ptr(), slices, sq.data_ptr(),
+                                               1.0 / w.k, float(eps), _lib.stream_handle(qkv.device))
+    if rc:
+        _lib.check(rc, "rope_cache_packed")
+    return qkv
 
 
 def _rope_args(rope: dict, m: int):

@@ -132,6 +132,21 @@ def splitk_add_rmsnorm(partials: torch.Tensor, x: torch.Tensor, w: torch.Tensor,
     return y
 
 
+def splitk_add_squares(partials: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
+    """``x += sum(partials)`` (in place, rounded once) and the new rows' sums of squares (fp32), for a product that applies
+    the norm itself. ``partials`` as :func:`splitk_add_rmsnorm`."""
+    _need(x, "x")
+    rows, cols = x.shape
+    if partials.dtype != torch.float32 or partials.dim() != 3 or tuple(partials.shape[1:]) != (rows, cols) or \
+            not partials.is_contiguous():
+        raise ValueError("partials must be a contiguous fp32 [nslice, rows, cols] tensor")
+    sq = torch.empty(rows, dtype=torch.float32, device=x.device)
+    rc = _lib.lib().kgs_splitk_add_squares_bf16(partials.data_ptr(), partials.shape[0], x.data_ptr(), sq.data_ptr(), rows, cols,
+                                                x.stride(0), _lib.stream_handle(x.device))
+    _lib.check(rc, "splitk_add_squares")
+    return sq
+
+
 def argmax_rows(x: torch.Tensor) -> torch.Tensor:
     """``x.argmax(dim=-1)`` for bf16 GPU logits ``[rows, cols]`` (cols % 8 == 0):
     int64, the first index of each row's maximum (NaN counts as the maximum)."""

@@ -379,7 +379,8 @@ class ServingModel:
         if self.prefill_f8 is not None:
             return self._prefill_fp8(tokens, positions, slots, seq_starts, seq_lens, padded_lens)
         seqs = [(int(s), int(n), int(p), 0) for s, n, p in zip(seq_starts, seq_lens, padded_lens)]
-        if self._fused_prompts(sum(n for _, n, _, _ in seqs), len(seqs)):
+        rows = sum(n for _, n, _, _ in seqs)
+        if self._slab_prompts(rows) or self._fused_prompts(rows, len(seqs)):
             return self._prefill_fused(tokens, positions, slots, seqs)
         plan = self._prompt_rows(seqs, tokens.numel(), tokens.device)
         x, y = self._start(tokens, plan.keep)
@@ -433,20 +434,26 @@ class ServingModel:
             D.skinny_takes(prompts, self.packed_lm.n, self.packed_lm.k)
 
     def _prefill_fused(self, tokens, positions, slots, seqs) -> torch.Tensor:
-        """A prompt step of few rows on the fused decode layer (:meth:`_fused_layers`), without its padding:
+        """A prompt step of few rows on the decode layers (:meth:`_fused_layers`, :meth:`_slab_layers`), without its padding:
         5 launches a layer besides the attention's (one prompt of 20 tokens, hidden 2048: 481 us by the
         split tiles, 403 so; of 30, hidden 4096: 630 and 546)."""
         plan = self._prompt_rows(seqs, tokens.numel(), tokens.device, drop=True, force=True)
         c = self.cfg
-        # counters of the step's own, cleared with its first launch: nothing is shared with a decode step on another stream
-        most = max(w.n for w in (*self.packed[0].values(), self.packed_lm))
-        count = torch.empty(most // 16, dtype=torch.int32, device=tokens.device)
         from kgs.ops.transformer import attention_blocks
 
         def attend(qkv, i):
             a = torch.empty((plan.n, c.heads * c.head_dim), dtype=torch.bfloat16, device=qkv.device)
             return attention_blocks(qkv, *self._kv(qkv), plan.items, c.heads, c.kv_heads, a, merges=plan.merges, slots=plan.slots)
 
+        if self._slab_prompts(plan.n):
+            x, y, ss = self._slab_layers(tokens, positions, slots, attend, "prefill", keep=plan.keep)
+            out = self._slab_head(x.index_select(0, plan.last) if y is None else y.index_select(0, plan.last), y is None,
+                                  None if y is not None else ss.index_select(0, plan.last), decode=False)
+            T.op("prefill-slabs lm_head")
+            return out
+        # counters of the step's own, cleared with its first launch: nothing is shared with a decode step on another stream
+        most = max(w.n for w in (*self.packed[0].values(), self.packed_lm))
+        count = torch.empty(most // 16, dtype=torch.int32, device=tokens.device)
         x, ss = self._fused_layers(tokens, positions, slots, attend, "prefill", count, exact=True, keep=plan.keep, heads=plan.last.numel())
         x = x.index_select(0, plan.last)
         if ss is None:
@@ -510,7 +517,7 @@ class ServingModel:
         parts = [np.asarray(last + list(range(at, at + tail)), np.int32)]
         past, items = [], None
         if not ref and seqs and (drop or wanted is not None or len({p for _, _, p, _ in seqs}) > 1):
-            from kgs.ops.transformer import block_items, split_items
+            from kgs.ops.transformer import SPLIT_TILES, block_items, split_items
 
             blocks, k0 = [], 0
             for j, (r, (_, n, p, ctx)) in enumerate(zip(starts, seqs)):
@@ -519,7 +526,9 @@ class ServingModel:
                 if ctx:
                     past.append((k0, k0 + ctx + m, ctx + n, j))
                     k0 += ctx + m
-            items, merges, slots = split_items(block_items(blocks, at), self.cfg.heads)
+            items, merges, slots = block_items(blocks, at), None, 0
+            if max(m + ctx for _, m, _, ctx, _ in blocks) > 64 * (SPLIT_TILES - 1):  # else no block is long enough
+                items, merges, slots = split_items(items, self.cfg.heads)
             parts.append(items.reshape(-1) if merges is None else np.concatenate([items, merges]).reshape(-1))
         if drop:
             keep = np.concatenate([np.arange(s, s + n, dtype=np.int32) for s, n, _, _ in seqs] +
@@ -676,7 +685,7 @@ class ServingModel:
     def decode(self, tokens, positions, slots, block_tables, ctx_lens, pages_per_split=None) -> torch.Tensor:
         """One token per sequence -> logits [B, vocab]."""
         c = self.cfg
-        if self.backend == "kgs" and tokens.shape[0] <= self.fused_max_batch:
+        if self.backend == "kgs" and tokens.shape[0] <= self.fused_max_batch or self._slabs(tokens.shape[0]):
             return self._decode_fused(tokens, positions, slots, block_tables, ctx_lens, pages_per_split)
         tickets = self._tickets(block_tables)
         x, y = self._start(tokens, zero=tickets)
@@ -748,6 +757,11 @@ class ServingModel:
             return D.paged_decode_attention(qkv, self.cache.layer(i), block_tables, ctx_lens, c.heads, c.kv_heads,
                                             pages_per_split=pages_per_split, tickets=tickets)
 
+        if self._slabs(tokens.shape[0]):
+            x, y, ss = self._slab_layers(tokens, positions, slots, attend, "decode", tickets=tickets)
+            out = self._slab_head(x if y is None else y, y is None, ss, decode=True)
+            T.op("decode-slabs lm_head")
+            return out
         x, ss = self._fused_layers(tokens, positions, slots, attend, "decode", None, exact=False, tickets=tickets)
         out = D.own_gemm(x, self.packed_lm, norm=True, eps=c.eps) if ss is None else D.skinny_gemm(x, self.packed_lm, rms=ss, eps=c.eps)
         T.op("decode-fused lm_head")
@@ -757,6 +771,84 @@ class ServingModel:
         """Whether the products behind a norm of ``m`` rows' fused layers, and of ``head`` rows the LM head, make its statistics themselves."""
         P = self.packed[0]
         return all(D.own_takes(r, w.n, w.k, w.fp8, bool(w.rope)) for w, r in ((P["qkv"], m), (P["gate_up"], m), (self.packed_lm, head)))
+
+    def _slabs(self, m: int) -> bool:
+        """Whether ``m`` rows take the layers of :meth:`_slab_layers`: 33 to 96 of bf16 weights and pages, where the products tile."""
+        if self.packed is None or self.decode_fp8 or self.backend != "kgs" or not self.fuse_splitk or self.rope_attn or \
+                not self.fused_max_batch or not 32 < m <= D.SLAB_ROWS:
+            return False
+        P, c = self.packed[0], self.cfg
+        return c.hidden % 2048 == 0 and c.hidden <= 8192 and bool(P["qkv"].rope) and \
+            all(D.slab_split(m, P[n].n, P[n].k) for n in ("qkv", "o", "down")) and \
+            all(D.slab_rows_tiles(m, w.n, w.k) for w in (P["gate_up"], self.packed_lm))
+
+    def _slab_prompts(self, m: int) -> bool:
+        """:meth:`_slabs` for prompts, whose launches come from the host one by one: up to 48 rows, where the fused layers have 5 a layer and these 8, only
+        with layers of 96 M weights and more (us, fused / here, one prompt of 36 tokens: 2048 wide, 63 M, 347 / 368; 4096 wide, 218 M, 612 / 487)."""
+        return self._slabs(m) and (m > 48 or sum(w.n * w.k for w in self.packed[0].values()) >= 96 << 20)
+
+    def _slab_gate(self, m: int):
+        """Gate and up of ``m`` rows of :meth:`_slab_layers`: a route of :meth:`_swiglu_route` on normed rows, or None: :func:`kgs.ops.decode.skinny_rows` on the
+        residual rows. The former from 49 rows on, where the route is the gate kernel or has tile-panel weights (us at 64 and 90 rows, so /
+        skinny_rows: 28672x4096 42.2, 48.9 / 45.9, 51.5, from row-major weights 51.6, 54.2; 16384x2048 15.9, 17.8 / 16.4, 19.2). Up to 48 rows as
+        the fused layers, whose products' inputs are not rounded behind the norm."""
+        if m <= 48:
+            return None
+        route = self._swiglu_route(m)
+        if route is None or route[1] > 1 or not (route[0] == GATE or (self.gate_up_panels is not None and route[0] in self.gate_up_panels[0])):
+            return None
+        return route
+
+    def _slab_layers(self, tokens, positions, slots, attend, kind: str, keep=None, tickets=None):
+        """As :meth:`_fused_layers`, for 33 to 96 rows: products in K slices that the rotation and the residual adds sum, gate and up whole. The
+        rows' bits depend on nothing but their own inputs. ``(x, y, ss)``: the residual rows, from 49 rows on their norm for the head
+        (else None) and else their sums of squares. Four layers 4096 wide, us a step by four-wave tiles (up to 48 rows skinny) / so: one prompt of 90
+        tokens 596 / 563, of 60 615 / 528, two of 36 in all 611 / 496; 2048 wide one of 60 401 / 362."""
+        from kgs.ops.transformer import embed_rows, embeds, splitk_add_rmsnorm, splitk_add_squares
+
+        c = self.cfg
+        tokens, dev = tokens.to(self.embed.device), self.embed.device
+        m = (tokens if keep is None else keep).numel()
+        ss, y = torch.empty(m, dtype=torch.float32, device=dev), None
+        if embeds(self.embed):
+            if keep is not None:
+                positions, slots = positions.reshape(-1).contiguous(), slots.reshape(-1).contiguous()
+            x, _, positions, slots = embed_rows(self.embed, tokens, None, c.eps, keep, ss, positions, slots, () if tickets is None else (tickets,))
+        else:
+            if keep is not None:
+                tokens, positions, slots = (t.reshape(-1)[keep.long()] for t in (tokens, positions, slots))
+            x = self.embed[tokens.long()].reshape(-1, c.hidden).contiguous()
+            ss.copy_(x.float().pow(2).sum(-1))
+            if tickets is not None:
+                tickets.zero_()
+        gate = self._slab_gate(m)
+        rope = {"cos": self.cos, "sin": self.sin, "positions": positions, "slots": slots}
+        for i, P in enumerate(self.packed):
+            rope["cache"] = self.cache.layer(i)
+            qkv = D.rope_cache_packed(D.skinny_slabs(x, P["qkv"]), ss, P["qkv"], c.eps, rope)
+            T.op(f"{kind}-slabs L{i} qkv+rope")
+            a = attend(qkv, i)
+            T.op(f"{kind}-slabs L{i} attention")
+            part = D.skinny_slabs(a, P["o"])
+            if gate:
+                act = self._gate_up_split(splitk_add_rmsnorm(part, x, self.ln2[i], c.eps), i, gate)
+            else:
+                act = D.skinny_rows(x, P["gate_up"], splitk_add_squares(part, x), c.eps)
+            part = D.skinny_slabs(act, P["down"])
+            if m > 48 and i + 1 == c.layers:
+                y = splitk_add_rmsnorm(part, x, self.norm, c.eps)
+            else:
+                ss = splitk_add_squares(part, x)
+            T.op(f"{kind}-slabs L{i} o+mlp")
+        return x, y, ss
+
+    def _slab_head(self, x, raw: bool, ss, decode: bool):
+        """Logits of rows of :meth:`_slab_layers`: residual rows with their sums of squares (``raw``), or their norm."""
+        if not raw:
+            return self._proj(x, None, "lm", decode)
+        if x.shape[0] <= 8 and D.few_takes(x.shape[0], self.packed_lm.n, self.packed_lm.k):
+            return D.skinny_few(x, self.packed_lm, norm=True, eps=self.cfg.eps)
+        return D.skinny_rows(x, self.packed_lm, ss, self.cfg.eps)
 
     def _tickets(self, block_tables):
         """Tickets of the step's own for the decode rows' attention, to be cleared with its first launch; None: it takes none."""

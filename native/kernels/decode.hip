@@ -627,13 +627,16 @@ __device__ __forceinline__ void kv_write(void* __restrict__ cache, int sl, int h
 // to bf16 exactly as kgs::splitk_reduce would, then rotated and stored to qkv
 // and the cache -- one launch instead of reduce + rope_cache. NSL > 0: the
 // slice count at compile time (all partial loads issued before the first add).
-template <bool KV8, bool SK = false, int NSL = 0>
+// PK (SK): the partials' columns are in the order of a weight packed with rope_rows (kgs/ops/decode.py), and rows of a raw residual
+// stream: they are scaled by its RMSNorm, rsqrt(sq[row] * inv_k + eps).
+template <bool KV8, bool SK = false, int NSL = 0, bool PK = false>
 __global__ __launch_bounds__(256) void rope_cache(unsigned short* __restrict__ qkv, const float* __restrict__ cosv,
                                                   const float* __restrict__ sinv, const int* __restrict__ pos,
                                                   const int* __restrict__ slot, void* __restrict__ cache,
                                                   long tokens, int H, int HKV, long ld,
                                                   const float* __restrict__ P = nullptr, int nslice = 0,
-                                                  const int* __restrict__ rows = nullptr, long prows = 0) {
+                                                  const int* __restrict__ rows = nullptr, long prows = 0,
+                                                  const float* __restrict__ sq = nullptr, float inv_k = 0.f, float eps = 0.f) {
   const int nh = H + 2 * HKV;
   const long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (idx >= tokens * nh * 8) return;
@@ -651,14 +654,17 @@ __global__ __launch_bounds__(256) void rope_cache(unsigned short* __restrict__ q
   const int sl = slot[t];
   bf16x8 a, b;
   if constexpr (SK) {
-    const long MN = prows * nh * HD, e = row * nh * HD + (long)h * HD + 8 * c;
+    const bool turned = PK && h < H + HKV;  // dims 8 c.. and 64 + 8 c.. side by side
+    const long MN = prows * nh * HD, e = row * nh * HD + (long)h * HD + (turned ? 16 : 8) * c;
+    const int far = turned ? 8 : HD / 2;
+    const float scale = PK ? rsqrtf(sq[row] * inv_k + eps) : 1.f;
     f32x4 s[4];
     if constexpr (NSL > 0) {
       f32x4 ps[NSL][4];
 #pragma unroll
       for (int sl = 0; sl < NSL; ++sl)
 #pragma unroll
-        for (int q = 0; q < 4; ++q) ps[sl][q] = *(const f32x4*)(P + sl * MN + e + (q >> 1) * (HD / 2) + (q & 1) * 4);
+        for (int q = 0; q < 4; ++q) ps[sl][q] = *(const f32x4*)(P + sl * MN + e + (q >> 1) * far + (q & 1) * 4);
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         s[q] = ps[0][q];
@@ -667,10 +673,14 @@ __global__ __launch_bounds__(256) void rope_cache(unsigned short* __restrict__ q
       }
     } else {
 #pragma unroll
-      for (int q = 0; q < 4; ++q) s[q] = *(const f32x4*)(P + e + (q >> 1) * (HD / 2) + (q & 1) * 4);
+      for (int q = 0; q < 4; ++q) s[q] = *(const f32x4*)(P + e + (q >> 1) * far + (q & 1) * 4);
       for (int sl = 1; sl < nslice; ++sl)
 #pragma unroll
-        for (int q = 0; q < 4; ++q) s[q] += *(const f32x4*)(P + sl * MN + e + (q >> 1) * (HD / 2) + (q & 1) * 4);
+        for (int q = 0; q < 4; ++q) s[q] += *(const f32x4*)(P + sl * MN + e + (q >> 1) * far + (q & 1) * 4);
+    }
+    if constexpr (PK) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) s[q] *= scale;
     }
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
@@ -1870,6 +1880,33 @@ KGS_EXPORT int kgs_rope_cache_bf16(void* qkv, const float* cosv, const float* si
 // [B, max_pages] int32; ctx_lens [B] int32 (>= 1). nsplit > 1 needs po
 // (B*H*nsplit*128 f32), pml (B*H*nsplit*2 f32) and cnt (B*HKV zeroed ints, left
 // zeroed); the splits are merged in the same launch.
+// kgs_rope_cache_bf16 of the partials (2 to 16, a power of two) of a weight packed with rope_rows, on rows of the raw residual stream
+// with sums of squares sq [tokens]: scaled by their RMSNorm, over inv_k^-1 columns. bf16 pages.
+KGS_EXPORT int kgs_rope_cache_packed_bf16(void* qkv, const float* cosv, const float* sinv, const int* pos, const int* slot, void* cache,
+                                         long tokens, int H, int HKV, long ld, const float* P, int nslice, const float* sq,
+                                         float inv_k, float eps, hipStream_t s) {
+  if (tokens < 0 || H <= 0 || HKV <= 0 || H % HKV || ld < (long)(H + 2 * HKV) * kgs::dec::HD) return KGS_ERR_SHAPE;
+  if (!al16(qkv) || !al16(cosv) || !al16(sinv) || !al16(cache) || !al16(P) || ld % 8) return KGS_ERR_ALIGN;
+  if (!P || !sq || !pos || !slot) return KGS_ERR_ARG;
+  const long n = tokens * (H + 2 * HKV) * 8;
+  if (n == 0) return 0;
+  const int wg = n <= (nslice == 2 ? 96 : 256) * 256 ? 64 : 256;  // as kgs_rope_cache_bf16
+  const dim3 g((unsigned)((n + wg - 1) / wg)), b(wg);
+#define KGS_RCP(NSL)                                                                                                                  \
+  hipLaunchKernelGGL((kgs::dec::rope_cache<false, true, NSL, true>), g, b, 0, s, (unsigned short*)qkv, cosv, sinv, pos, slot, cache, \
+                     tokens, H, HKV, ld, P, nslice, nullptr, tokens, sq, inv_k, eps)
+  switch (nslice) {
+    case 1: KGS_RCP(1); break;
+    case 2: KGS_RCP(2); break;
+    case 4: KGS_RCP(4); break;
+    case 8: KGS_RCP(8); break;
+    case 16: KGS_RCP(16); break;
+    default: return KGS_ERR_ARG;
+  }
+#undef KGS_RCP
+  return (int)hipGetLastError();
+}
+
 KGS_EXPORT int kgs_paged_decode_bf16_ex(const void* q, const void* cache, const int* block_tables,
                                        const int* ctx_lens, void* o, float* po, float* pml, int* cnt, int B, int H,
                                        int HKV, int hd, int max_pages, int pages_per_split, int nsplit, long ldq,

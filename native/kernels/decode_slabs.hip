@@ -1,14 +1,20 @@
-// Skinny products of up to 64 rows in K slices, as fp32 partial sums that the next launch adds: P[slice][M][N] of
-// x[M, K] . W^T, W packed as for decode.hip's skinny ([N/16][K/32][64][8]).
+// Skinny products of up to 96 rows past skinny's tickets and barriers: x[M, K] . W^T, W packed as for decode.hip's skinny
+// ([N/16][K/32][64][8]), in K slices as fp32 partial sums P[slice][M][N] that the next launch adds (slabs), or whole, with the
+// RMSNorm and the gate of a fused layer in the epilogue (rows).
 //
 // A workgroup of four waves takes 64 R rows of W (wave w its R tiles) over one slice. W streams into registers, PF k-steps
-// ahead and past the caches; x comes by LDS-DMA in MFMA operand order, chunks of KC k-steps in three stages, one barrier
+// ahead and past the caches; x comes by LDS-DMA in MFMA operand order, chunks of KC k-steps in NB stages, one barrier
 // each, and a k-step's fragments are read from LDS under the MFMAs of the one before. All loads are counted by hand: the
-// compiler's own schedule waits for every load in flight before it stores a chunk (twice the time).
+// compiler's own schedule waits for every load in flight before it stores a chunk (twice the time). W has to lie packed: 16 rows' pieces of 64
+// bytes, straight from its rows, take half as long again (28672x4096 at 100 rows 79 us, packed 53).
 //
-// skinny adds its slices itself: each stores its part, the last one of a strip to arrive reads them all. That is 3 to 5 us at the end of a
-// launch (2048x8192 at 24 rows 14.7 us, the same product here 8.8); where the next launch passes over the output anyway it
-// reads a few MB instead. Workgroups by slices (slab_split): about one a CU, and wide tiles only where N alone has enough.
+// Slices: skinny adds its slices itself: each stores its part, the last one of a strip to arrive reads them all. That is 3 to 5 us at the end of a
+// launch (2048x8192 at 32 rows 15.0 us, the same product here 8.8); where the next launch passes over the output anyway it
+// reads a few MB instead. Workgroups by slices (kgs/ops/decode.py slab_split): about one a CU, and wide tiles only where N alone has enough.
+// From 33 rows on these beat the four-wave tiles of gemm_w4.h too, whose weights go through LDS; us at 64 and 90 rows, those / here:
+// 6144x4096 14.9, 20.2 / 14.0, 15.8; 4096x14336 25.1, 27.6 / 23.5, 26.4; whole: 28672x4096 51.6, 54.2 / 44.4, 47.5; 32000x4096 61 / 48; not
+// above 96 rows (128: 55.0 / 53.5, 19.0 / 18.6, 13.2 / 14.2), where reading x from LDS takes as long as the MFMAs.
+// Deep rings (8 k-steps, 5 stages) help long sums of whole products only: 28672x4096 at 64 / 90 rows 46.2 / 51.0 us by short ones, 44.4 / 47.5.
 #include "decode_common.h"
 
 namespace kgs {
@@ -17,9 +23,14 @@ namespace dec {
 struct SlabArgs {
   const unsigned short* x;
   const unsigned short* w;
-  float* p;
+  void* y;  // OUT_SLABS: fp32 [ns][M][N]; else bf16 rows ldy apart
   int M, N, K, ldx, ns;
+  long ldy;
+  const float* sq;  // RMSNorm of x's rows: their sums of squares, or null
+  float inv_k, eps, limit;
+  int mode;  // OUT_GATED: EPI_GELU, EPI_CLAMPED
 };
+enum { OUT_SLABS, OUT_ROWS, OUT_GATED };
 
 __device__ __forceinline__ void dma16(__amdgpu_buffer_rsrc_t r, void* lds, int v, int s) {
   __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (KGS_LDS void*)lds, 16, v, s, 0, 0);
@@ -32,10 +43,11 @@ __device__ __forceinline__ void wait_loads() {
   asm volatile("" ::: "memory");
 }
 
-template <int MT, int R>
+template <int MT, int R, int OUT, int PF, int NB>
 __global__ __launch_bounds__(256, 2) void slabs(SlabArgs a) {
-  constexpr int KC = MT == 1 ? 4 : 2, PF = 4, XL = KC * MT / 4;  // x fragments of a wave and chunk
-  __shared__ __attribute__((aligned(16))) bf16x8 xs[3][KC * MT * 64];
+  constexpr int KC = MT == 1 ? 4 : 2, XL = KC * MT / 4;  // x fragments of a wave and chunk
+  static_assert(PF % KC == 0 && PF >= (NB - 2) * KC);
+  __shared__ __attribute__((aligned(16))) bf16x8 xs[NB][KC * MT * 64];
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), fr = lane & 15, fq = lane >> 4;
   const int M = a.M, N = a.N, nkk = a.K / 32, tiles = N / (64 * R), tile = blockIdx.x % tiles, sl = blockIdx.x / tiles;
   const int nsteps = nkk / a.ns, k0 = sl * nsteps, nchunks = nsteps / KC;
@@ -60,24 +72,26 @@ __global__ __launch_bounds__(256, 2) void slabs(SlabArgs a) {
 #pragma unroll
     for (int i = 0; i < XL; ++i) dma16(rx, &xs[to][(w * XL + i) * 64], xo[i], min(next, nchunks - 1) * (KC * 64));
     ++next;
-    to = to == 2 ? 0 : to + 1;
+    to = to == NB - 1 ? 0 : to + 1;
   };
   f32x4v acc[R][MT];
 #pragma unroll
   for (int r = 0; r < R; ++r)
 #pragma unroll
     for (int c = 0; c < MT; ++c) acc[r][c] = f32x4v{0.f, 0.f, 0.f, 0.f};
+  // KC k-steps of weights at least between two chunks, as in the loop
   send();
   send();
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-  for (int p = 0; p < PF / 2; ++p) load_w(p, p);
-  __builtin_amdgcn_sched_barrier(0);
-  send();
-  __builtin_amdgcn_sched_barrier(0);
+  for (int g = 0; g < NB - 1; ++g) {
 #pragma unroll
-  for (int p = PF / 2; p < PF; ++p) load_w(p, p);
-  wait_loads<2 * XL + PF * R, false>();  // chunk 0
+    for (int p = g * KC; p < (g == NB - 2 ? PF : (g + 1) * KC); ++p) load_w(p, p);
+    __builtin_amdgcn_sched_barrier(0);
+    if (g < NB - 2) send();
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  wait_loads<(NB - 1) * XL + PF * R, false>();  // chunk 0
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
   int from = 0;  // stage being read
@@ -89,12 +103,12 @@ __global__ __launch_bounds__(256, 2) void slabs(SlabArgs a) {
     for (int p = 0; p < PF; ++p) {
       const int kk = p % KC;
       if (kk == KC - 1) {
-        // the next chunk: at least the weights of 2 KC - 1 k-steps and one chunk were sent for after it. Every wave has read
+        // the next chunk: at least the weights of (NB - 1) KC - 1 k-steps and NB - 2 chunks were sent for after it. Every wave has read
         // this one, so its stage is free
-        wait_loads<(2 * KC - 1) * R + XL, true>();
+        wait_loads<((NB - 1) * KC - 1) * R + (NB - 2) * XL, true>();
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
-        from = from == 2 ? 0 : from + 1;
+        from = from == NB - 1 ? 0 : from + 1;
 #pragma unroll
         for (int c = 0; c < MT; ++c) b[(p + 1) & 1][c] = xs[from][c * 64 + lane];
         send();
@@ -115,9 +129,28 @@ __global__ __launch_bounds__(256, 2) void slabs(SlabArgs a) {
 #pragma unroll
   for (int c = 0; c < MT; ++c) {
     const int m = 16 * c + fr;
-    if (m < M) {
+    float scale = 1.f;
+    if constexpr (OUT != OUT_SLABS) {
+      if (a.sq) scale = rsqrtf(a.sq[min(m, M - 1)] * a.inv_k + a.eps);
+    }
 #pragma unroll
-      for (int r = 0; r < R; ++r) *(f32x4v*)(a.p + ((long)sl * M + m) * N + 16 * (nt0 + r) + 4 * fq) = acc[r][c];
+    for (int r = 0; r < R; ++r) {
+      const f32x4v v = OUT == OUT_SLABS ? acc[r][c] : acc[r][c] * scale;
+      const int nt = nt0 + r;
+      if constexpr (OUT == OUT_SLABS) {
+        if (m < M) *(f32x4v*)((float*)a.y + ((long)sl * M + m) * N + 16 * nt + 4 * fq) = v;
+      } else if constexpr (OUT == OUT_ROWS) {
+        if (m < M) *(uint2*)((unsigned short*)a.y + m * a.ldy + 16 * nt + 4 * fq) = uint2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+      } else {  // a tile's gate rows in lanes 0 .. 31, their up rows in the lanes 32 on
+        f32x4v u, o;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) u[i] = lane_xor32(v[i]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          o[i] = (a.mode & EPI_CLAMPED) ? gate_clamped(v[i], u[i], a.limit)
+                 : ((a.mode & EPI_GELU) ? gate_act<GATE_GELU>(v[i]) : gate_act<GATE_SILU>(v[i])) * u[i];
+        if (m < M && fq < 2) *(uint2*)((unsigned short*)a.y + m * a.ldy + 8 * nt + 4 * fq) = uint2{pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3])};
+      }
     }
   }
 }
@@ -125,20 +158,54 @@ __global__ __launch_bounds__(256, 2) void slabs(SlabArgs a) {
 }  // namespace dec
 }  // namespace kgs
 
-// P[ns][M][N] (fp32) = the K slices' products of x[M, K] (rows ldx apart) and W^T, W packed as for kgs_skinny_gemm_bf16: up to 64
+namespace {
+constexpr int SLAB_ROWS = 96;
+
+template <int OUT, int PF, int NB>
+int launch_slabs(const kgs::dec::SlabArgs& a, int r, hipStream_t s) {
+  using namespace kgs::dec;
+  auto run = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(a.N / (64 * r) * a.ns), dim3(256), 0, s, a);
+    return (int)hipGetLastError();
+  };
+  if constexpr (NB == 3) {
+    if (a.M <= 16) return r == 1 ? run(slabs<1, 1, OUT, PF, NB>) : run(slabs<1, 2, OUT, PF, NB>);
+    if (a.M <= 32) return r == 1 ? run(slabs<2, 1, OUT, PF, NB>) : run(slabs<2, 2, OUT, PF, NB>);
+    if (r == 1) return a.M <= 64 ? run(slabs<4, 1, OUT, PF, NB>) : run(slabs<6, 1, OUT, PF, NB>);
+  }
+  return a.M <= 64 ? run(slabs<4, 2, OUT, PF, NB>) : run(slabs<6, 2, OUT, PF, NB>);
+}
+
+int slab_shape(const void* wp, const void* x, const void* y, int M, int N, int K, long ldx, int r, int ns) {
+  if (M < 1 || M > SLAB_ROWS || N <= 0 || K <= 0 || (r != 1 && r != 2) || ns < 1 || N % (64 * r) || K % (128 * ns) || (long)N * K > (1l << 31))
+    return KGS_ERR_SHAPE;
+  if (ldx < K || ldx > 1l << 23) return KGS_ERR_SHAPE;
+  return (uintptr_t)wp % 16 || (uintptr_t)x % 16 || (uintptr_t)y % 16 || ldx % 8 ? KGS_ERR_ALIGN : 0;
+}
+}  // namespace
+
+// P[ns][M][N] (fp32) = the K slices' products of x[M, K] (rows ldx apart) and W^T, W packed as for kgs_skinny_gemm_bf16: up to 96
 // rows, r (1, 2) tiles of 16 W rows a wave, N a multiple of 64 r, K of 128 ns.
 KGS_EXPORT int kgs_skinny_slabs(const void* wp, const void* x, float* p, int M, int N, int K, long ldx, int r, int ns, hipStream_t s) {
   using namespace kgs::dec;
-  if (M < 1 || M > 64 || N <= 0 || K <= 0 || (r != 1 && r != 2) || ns < 1 || N % (64 * r) || K % (128 * ns) || (long)N * K > (1l << 31))
-    return KGS_ERR_SHAPE;
-  if (ldx < K || ldx > 1l << 23) return KGS_ERR_SHAPE;
-  if ((uintptr_t)wp % 16 || (uintptr_t)x % 16 || (uintptr_t)p % 16 || ldx % 8) return KGS_ERR_ALIGN;
-  const SlabArgs a{(const unsigned short*)x, (const unsigned short*)wp, p, M, N, K, (int)ldx, ns};
-  auto run = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, dim3(N / (64 * r) * ns), dim3(256), 0, s, a);
-    return (int)hipGetLastError();
-  };
-  if (M <= 16) return r == 1 ? run(slabs<1, 1>) : run(slabs<1, 2>);
-  if (M <= 32) return r == 1 ? run(slabs<2, 1>) : run(slabs<2, 2>);
-  return r == 1 ? run(slabs<4, 1>) : run(slabs<4, 2>);
+  const int rc = slab_shape(wp, x, p, M, N, K, ldx, r, ns);
+  if (rc) return rc;
+  const SlabArgs a{(const unsigned short*)x, (const unsigned short*)wp, p, M, N, K, (int)ldx, ns, 0, nullptr, 0.f, 0.f, 0.f, 0};
+  return launch_slabs<OUT_SLABS, 4, 3>(a, r, s);
+}
+
+// y[M, N] (bf16, rows ldy apart) = x[M, K] . W^T as kgs_skinny_slabs in one slice; sq: of x's RMSNorm (its weight folded into W) by
+// these sums of squares of its rows. epi: EPI_SWIGLU (with EPI_GELU or EPI_CLAMPED and limit): y is [M, N / 2].
+KGS_EXPORT int kgs_skinny_rows(const void* wp, const void* x, void* y, int M, int N, int K, long ldx, long ldy, int r, int epi,
+                               const float* sq, float eps, float limit, hipStream_t s) {
+  using namespace kgs::dec;
+  const int rc = slab_shape(wp, x, y, M, N, K, ldx, r, 1);
+  if (rc) return rc;
+  const bool gated = epi & EPI_SWIGLU;
+  if (ldy < (gated ? N / 2 : N)) return KGS_ERR_SHAPE;
+  if (ldy % 4) return KGS_ERR_ALIGN;
+  if (epi & ~(EPI_SWIGLU | EPI_GELU | EPI_CLAMPED) || (epi && !gated)) return KGS_ERR_ARG;
+  const SlabArgs a{(const unsigned short*)x, (const unsigned short*)wp, y, M, N, K, (int)ldx, 1, ldy, sq, 1.f / K, eps, limit, epi};
+  if (M > 32 && r == 2 && K % 256 == 0) return gated ? launch_slabs<OUT_GATED, 8, 5>(a, r, s) : launch_slabs<OUT_ROWS, 8, 5>(a, r, s);
+  return gated ? launch_slabs<OUT_GATED, 4, 3>(a, r, s) : launch_slabs<OUT_ROWS, 4, 3>(a, r, s);
 }

@@ -337,12 +337,14 @@ __global__ __launch_bounds__(256) void silu_mul(const unsigned short* __restrict
 // NSL > 0: the slice count at compile time, so every partial load of a thread
 // is issued before the first add (a run-time slice loop waits out one cache
 // latency per slice); 0 = run-time count.
-template <int NJ, int NSL>
+// SQUARES: x' = bf16(x + sum_s P[s][row]), and its row's sum of squares to sq[row] instead of y: for a product that
+// applies the norm to its own rows. Bound by the slices, 4 to 5 TB/s from the caches (more threads a row: the same).
+template <int NJ, int NSL, bool SQUARES = false>
 __global__ __launch_bounds__(256) void splitk_add_rmsnorm(const float* __restrict__ P, int nslice, long MN,
                                                           unsigned short* __restrict__ x,
                                                           const unsigned short* __restrict__ w,
                                                           unsigned short* __restrict__ y, int cols, long ldx,
-                                                          long ldy, float eps) {
+                                                          long ldy, float eps, float* __restrict__ sq = nullptr) {
   __shared__ float red[4];
   const int row = blockIdx.x, t = threadIdx.x;
   bf16x8* xr = (bf16x8*)(x + row * ldx);
@@ -354,7 +356,7 @@ __global__ __launch_bounds__(256) void splitk_add_rmsnorm(const float* __restric
 #pragma unroll
   for (int j = 0; j < NJ; ++j) {
     xin[j] = xr[t + 256 * j];
-    wv[j] = wr[t + 256 * j];
+    if constexpr (!SQUARES) wv[j] = wr[t + 256 * j];
   }
   float v[NJ][8];
   float ss = 0.f;
@@ -388,7 +390,7 @@ __global__ __launch_bounds__(256) void splitk_add_rmsnorm(const float* __restric
     bf16x8 o;
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
-      const float d = bf2f(f2bf(k < 4 ? a[k] : b[k - 4]));
+      const float p = k < 4 ? a[k] : b[k - 4], d = SQUARES ? p : bf2f(f2bf(p));
       o[k] = (short)f2bf(bf2f((unsigned short)xv[k]) + d);
       v[j][k] = bf2f((unsigned short)o[k]);
       ss += v[j][k] * v[j][k];
@@ -399,6 +401,10 @@ __global__ __launch_bounds__(256) void splitk_add_rmsnorm(const float* __restric
   if ((t & 63) == 0) red[t >> 6] = ss;
   __syncthreads();
   ss = (red[0] + red[1]) + (red[2] + red[3]);
+  if constexpr (SQUARES) {
+    if (t == 0) sq[row] = ss;
+    return;
+  }
   const float r = rsqrtf(ss / (float)cols + eps);
   bf16x8* yr = (bf16x8*)(y + row * ldy);
 #pragma unroll
@@ -499,10 +505,12 @@ KGS_EXPORT int kgs_argmax_rows_bf16(const void* x, long long* out, int rows, int
 // P: nslice fp32 partial products [nslice][rows][cols] (gemm_nt_w4x without its
 // reduce); x: [rows, ldx] residual stream, updated in place; w: [cols]; y: out.
 // cols a multiple of 2048 up to 8192.
-KGS_EXPORT int kgs_splitk_add_rmsnorm_bf16(const float* P, int nslice, void* x, const void* w, void* y, int rows,
-                                          int cols, long ldx, long ldy, float eps, hipStream_t s) {
+namespace {
+template <bool SQUARES>
+int add_slices(const float* P, int nslice, void* x, const void* w, void* y, int rows, int cols, long ldx, long ldy, float eps,
+               float* sq, hipStream_t s) {
   if (rows < 0 || cols <= 0 || nslice <= 0) return KGS_ERR_SHAPE;
-  if (cols % 2048 || cols > 8192 || ldx < cols || ldy < cols) return KGS_ERR_SHAPE;
+  if (cols % 2048 || cols > 8192 || ldx < cols || (!SQUARES && ldy < cols)) return KGS_ERR_SHAPE;
   if (!al16(P) || !al16(x) || !al16(w) || !al16(y) || ldx % 8 || ldy % 8) return KGS_ERR_ALIGN;
   if (rows == 0) return 0;
   using namespace kgs::tfm;
@@ -510,11 +518,9 @@ KGS_EXPORT int kgs_splitk_add_rmsnorm_bf16(const float* P, int nslice, void* x, 
   auto X = (unsigned short*)x;
   auto W = (const unsigned short*)w;
   auto Y = (unsigned short*)y;
-  const int nj = cols / 2048;
-  if (nj < 1 || nj > 4) return KGS_ERR_SHAPE;
-#define KGS_SARN(NJ, NSL)                                                                                           \
-  hipLaunchKernelGGL((splitk_add_rmsnorm<NJ, NSL>), dim3(rows), dim3(256), 0, s, P, nslice, MN, X, W, Y, cols, ldx, \
-                     ldy, eps)
+#define KGS_SARN(NJ, NSL)                                                                                                    \
+  hipLaunchKernelGGL((splitk_add_rmsnorm<NJ, NSL, SQUARES>), dim3(rows), dim3(256), 0, s, P, nslice, MN, X, W, Y, cols, ldx, \
+                     ldy, eps, sq)
 #define KGS_SARN_NJ(NJ)                                           \
   switch (nslice) {                                               \
     case 2: KGS_SARN(NJ, 2); break;                               \
@@ -523,7 +529,7 @@ KGS_EXPORT int kgs_splitk_add_rmsnorm_bf16(const float* P, int nslice, void* x, 
     case 16: KGS_SARN(NJ, 16); break;                             \
     default: KGS_SARN(NJ, 0); break;                              \
   }
-  switch (nj) {
+  switch (cols / 2048) {
     case 1: KGS_SARN_NJ(1); break;
     case 2: KGS_SARN_NJ(2); break;
     case 3: KGS_SARN_NJ(3); break;
@@ -532,6 +538,18 @@ KGS_EXPORT int kgs_splitk_add_rmsnorm_bf16(const float* P, int nslice, void* x, 
 #undef KGS_SARN_NJ
 #undef KGS_SARN
   return (int)hipGetLastError();
+}
+}  // namespace
+
+KGS_EXPORT int kgs_splitk_add_rmsnorm_bf16(const float* P, int nslice, void* x, const void* w, void* y, int rows,
+                                          int cols, long ldx, long ldy, float eps, hipStream_t s) {
+  return add_slices<false>(P, nslice, x, w, y, rows, cols, ldx, ldy, eps, nullptr, s);
+}
+
+// x += the sum of nslice fp32 slices [nslice, rows, cols], sq[row] = the new row's sum of squares.
+KGS_EXPORT int kgs_splitk_add_squares_bf16(const float* P, int nslice, void* x, float* sq, int rows, int cols, long ldx, hipStream_t s) {
+  if (!sq) return KGS_ERR_ARG;
+  return add_slices<true>(P, nslice, x, nullptr, nullptr, rows, cols, ldx, 0, 0.f, sq, s);
 }
 
 // ptrs (13): table tokens keep x y w ss pos slot pos_out slot_out zero0 zero1, keep (int32), y with w, ss, pos with pos_out, slot with

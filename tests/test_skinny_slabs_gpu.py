@@ -5,7 +5,7 @@ import torch
 from kgs.ops import decode as D
 from kgs.ops.hyper import hyper_step
 
-pytestmark = pytest.mark.gpu
+pytestmark = [pytest.mark.gpu, pytest.mark.usefixtures("own_rng")]
 
 
 def _operands(m, n, k, seed=0):
@@ -16,7 +16,7 @@ def _operands(m, n, k, seed=0):
 
 # the shortest slice (one round of the weights' ring), one chunk more, many; one and two tiles a wave; column tiles full, of one row and short
 @pytest.mark.parametrize("n,k", ((64, 128), (64, 256), (1024, 1024), (2048, 2048), (2048, 8192), (192, 384), (4096, 896), (4224, 2048)))
-@pytest.mark.parametrize("m", (1, 16, 17, 32, 33, 64))
+@pytest.mark.parametrize("m", (1, 16, 17, 32, 33, 64, 65, 96))
 def test_slices_add_to_the_product(n, k, m):
     x, w = _operands(m, n, k)
     r, ns = D.slab_split(m, n, k)
@@ -30,12 +30,115 @@ def test_slices_add_to_the_product(n, k, m):
 
 
 def test_what_slices_do_not_take():
-    for m, n, k in ((0, 2048, 2048), (65, 2048, 2048), (8, 2080, 2048), (8, 2048, 2080)):
+    for m, n, k in ((0, 2048, 2048), (97, 2048, 2048), (8, 2080, 2048), (8, 2048, 2080)):
         assert D.slab_split(m, n, k) is None
     x, w = _operands(4, 128, 256)
     for pw in (D.PackedWeight(w, swiglu=True), D.PackedWeight(w, fp8=True)):
         with pytest.raises(ValueError):
             D.skinny_slabs(x, pw)
+    for m, n, k in ((0, 2048, 2048), (97, 2048, 2048), (40, 2080, 2048), (40, 2048, 2080)):
+        assert D.slab_rows_tiles(m, n, k) is None
+    with pytest.raises(ValueError):
+        D.skinny_rows(x, D.PackedWeight(w, fp8=True))
+    with pytest.raises(ValueError):
+        D.skinny_rows(x, D.PackedWeight(w), sq=torch.ones(3, device="cuda"))
+
+
+# short and deep rings (the latter from 33 rows and 192 strips of 128 rows on), the latter's least and one round more
+@pytest.mark.parametrize("n,k", ((64, 128), (1024, 384), (16384, 256), (24576, 256), (24576, 512), (24576, 384), (24704, 1024)))
+@pytest.mark.parametrize("m", (1, 16, 17, 32, 33, 64, 65, 96))
+def test_whole_products_and_gates(n, k, m):
+    x, w = _operands(m, n, k, 1)
+    ref = x.double() @ w.double().T
+
+    def close(got, want, factors=1):  # one rounding to bf16, and fp32 sums' errors for each factor
+        assert bool(((got.double() - want).abs() <= 2.0 ** -8 * want.abs() + 2e-5 * factors * want.abs().max()).all())
+
+    close(D.skinny_rows(x, D.PackedWeight(w)), ref)
+    sq = x.float().pow(2).sum(1)
+    normed = ref * torch.rsqrt(x.double().pow(2).mean(1, keepdim=True) + 1e-3)
+    close(D.skinny_rows(x, D.PackedWeight(w), sq, 1e-3), normed)
+    g, u = normed.chunk(2, 1)
+    close(D.skinny_rows(x, D.PackedWeight(w, swiglu=True), sq, 1e-3), torch.nn.functional.silu(g) * u, 4)
+    close(D.skinny_rows(x, D.PackedWeight(w, swiglu=True, act="gelu_tanh"), sq, 1e-3), torch.nn.functional.gelu(g, approximate="tanh") * u, 4)
+
+
+@pytest.mark.parametrize("heads,kv,k", ((32, 8, 4096), (16, 4, 2048), (8, 1, 128), (2, 1, 1024)))  # 4, 4, 1 and 4 slices
+@pytest.mark.parametrize("m", (33, 96))
+def test_rotation_of_slices_as_of_the_whole_product(heads, kv, k, m):
+    from kgs.ops.transformer import rope_tables
+
+    x, w = _operands(m, (heads + 2 * kv) * 128, k, 2)
+    cos, sin = rope_tables(256, 128, 10000.0, "cuda")
+    pos, slots = torch.arange(m, dtype=torch.int32, device="cuda") * 7 % 250, torch.randperm(256, device="cuda")[:m].int()
+    slots[5] = -1
+    caches = [D.PagedKVCache(1, 8, kv, "cuda") for _ in range(2)]
+    pw = D.PackedWeight(w, rope=(heads, kv))
+    sq = x.float().pow(2).sum(1)
+    parts = D.skinny_slabs(x, pw)
+    got = D.rope_cache_packed(parts, sq, pw, 1e-5, {"cos": cos, "sin": sin, "positions": pos, "slots": slots, "cache": caches[0].layer(0)})
+    total = parts[0].clone()
+    for p in parts[1:]:
+        total += p
+    total *= torch.rsqrt(sq[:, None] * (1.0 / k) + 1e-5)
+    want = torch.empty_like(total)
+    want[:, D.rope_rows(pw.n, heads, kv).cuda()] = total
+    want = want.bfloat16()
+    D.rope_cache_(want, cos, sin, pos, slots, caches[1].layer(0), heads, kv)
+    # v_rsq's last bit before the rounding to bf16
+    assert float((got.float() - want.float()).abs().max()) <= 2.0 ** -7 * float(want.float().abs().max())
+    assert float((got.float() - want.float()).norm() / want.float().norm()) < 1e-3
+    assert float((caches[0].data.float() - caches[1].data.float()).norm() / caches[1].data.float().norm()) < 1e-3
+    assert torch.equal(caches[0].data == 0, caches[1].data == 0)
+
+
+@pytest.mark.parametrize("cols", (2048, 4096, 6144, 8192))
+@pytest.mark.parametrize("parts", (1, 2, 4, 8, 16))
+def test_residual_add_of_slices_and_its_squares(parts, cols):
+    from kgs.ops.transformer import splitk_add_squares
+
+    g = torch.Generator(device="cuda").manual_seed(cols)
+    p = torch.randn(parts, 5, cols, generator=g, device="cuda")
+    x = torch.randn(5, cols, generator=g, device="cuda").bfloat16()
+    total = p[0].clone()
+    for q in p[1:]:
+        total += q
+    want = (x.float() + total).bfloat16()
+    sq = splitk_add_squares(p, x)
+    assert torch.equal(x, want)
+    assert torch.allclose(sq.double(), want.double().pow(2).sum(1), rtol=1e-6)
+
+
+@pytest.mark.parametrize("rows", (33, 48, 49, 64, 96))
+@pytest.mark.parametrize("wide", (False, True))  # gate and up of a product's two tiles a wave
+def test_layers_of_slices_as_the_others(rows, wide):
+    from kgs.models.llama import LlamaConfig
+    from kgs.serve.model import ServingModel
+
+    c = LlamaConfig(hidden=2048, layers=2, heads=16, kv_heads=4, intermediate=12544 if wide else 1024, vocab=512)
+    m = ServingModel(c, device="cuda", num_pages=256, max_model_len=1024)
+    m.cache.data.normal_()
+    assert m._slabs(rows) and not m._slabs(32) and not m._slabs(97)
+    i32 = dict(dtype=torch.int32, device="cuda")
+    ctx = torch.randint(1, 300, (rows,), **i32)
+    tables = torch.stack([torch.randperm(255, device="cuda")[:16].int() + 1 for _ in range(rows)])
+    tokens, slots = torch.randint(0, 512, (rows,), **i32), torch.full((rows,), -1, **i32)
+    n = [rows // 2, rows - rows // 2]
+    starts, padded = [0, 128], [128, 128]
+    flat = torch.randint(0, 512, (256,), **i32)
+    pos = torch.cat([torch.arange(128, **i32)] * 2)
+    where = torch.cat([torch.where(torch.arange(128, device="cuda") < k, torch.arange(128, device="cuda") + o, -1) for k, o in zip(n, (32, 512))]).int()
+
+    def both():
+        m.cache.data[:, 1:32].zero_()
+        logits = m.prefill(flat, pos, where, starts, n, padded)
+        return m.decode(tokens, ctx - 1, slots, tables, ctx).float(), logits.float(), m.cache.data.float()
+
+    got, again = both(), both()
+    assert all(torch.equal(a, b) for a, b in zip(got[1:], again[1:]))  # a prompt's bits repeat
+    m._slabs = m._slab_prompts = lambda rows: False
+    for a, b in zip(got, both()):
+        assert float((a - b).norm() / b.norm()) < 2e-2  # sums in another order, rounded to bf16 through two layers
 
 
 @pytest.mark.parametrize("width", (64, 1023, 1028, 2048, 2052, 4096, 4100))  # both kernels' edges and rows that 16-byte loads cannot read

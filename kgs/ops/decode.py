@@ -513,9 +513,21 @@ GATE_EPI = {"silu": 0, "gelu_tanh": EPI_GELU, "clamped": EPI_CLAMPED}
 
 
 @lru_cache(maxsize=4096)
-def few_takes(m: int, n: int, k: int, fp8: bool = False) -> bool:
-    """Whether the kernel of few rows (native/kernels/decode_few.hip) runs ``m`` rows of an ``[n, k]`` weight: up to 16 of bf16 weights."""
-    return not fp8 and 0 < m <= 16 and bool(_lib.lib().kgs_skinny_few_ok(m, n, k))
+def few_takes(m: int, n: int, k: int, fp8: bool = False, plain: bool = False) -> bool:
+    """Whether the kernel of few rows (native/kernels/decode_few.hip) runs ``m`` rows of an ``[n, k]`` weight: up to 16 of bf16 weights,
+    32 of a product without a norm or a rotation (``plain``), which also takes any K of 64."""
+    return not fp8 and 0 < m <= 32 and bool(_lib.lib().kgs_skinny_few_ok(m, n, k, plain))
+
+
+@lru_cache(maxsize=4096)
+def few_route(m: int, n: int, k: int, plain: bool = False) -> bool:
+    """Whether the kernel of few rows is the better one, of those that take these rows: up to 8, up to 16 where W has at most 512 strips and x
+    128k values -- beyond, x through LDS is shared by more of W, or split over workgroups (us at 16 rows, few / others: 28672x4096 51 / 43,
+    4096x14336 26.3 / 23.5, but 6144x4096 13.7 / 16.2, 4096x4096 10.5 / 11, 6656x2048 7.5 / 10.3) -- and up to 32 for short sums of narrow weights and the sizes that skinny does not
+    take (24 rows: 2048x768 4.7 / 7.6, 4096x1536 6.7 / 9.6, 1344x2048 7.3 / 6.7)."""
+    if not few_takes(m, n, k, False, plain):
+        return False
+    return m <= 8 or (m <= 16 and n <= 512 * 16 and m * k <= 128 << 10) or (k <= 1536 and n <= 4096) or not _own_by_skinny(m, n, k, False, False)
 
 
 @lru_cache(maxsize=4096)
@@ -532,11 +544,9 @@ def own_takes(m: int, n: int, k: int, fp8: bool = False, rope: bool = False) -> 
 
 def own_gemm(x: torch.Tensor, w: PackedWeight, out: torch.Tensor | None = None, norm: bool = False, resid: bool = False,
              eps: float = 1e-5, rope: dict | None = None, counters: torch.Tensor | None = None) -> torch.Tensor:
-    """:func:`skinny_gemm` with ``norm`` or ``resid``, by :func:`skinny_few` up to 8 rows, and up to 16 where W has at most
-    512 strips and x 128k values: beyond, x through LDS is shared by more of W, or split over workgroups (us at 16 rows, few / others: 28672x4096 51
-    / 43, 4096x14336 26.3 / 23.5, but 6144x4096 13.7 / 16.2, 4096x4096 10.5 / 11)."""
+    """:func:`skinny_gemm` with ``norm`` or ``resid``, by :func:`skinny_few` where that is the better one (:func:`few_route`)."""
     m, k = x.shape
-    if few_takes(m, w.n, k, w.fp8) and (m <= 8 or (w.n <= 512 * 16 and m * k <= 128 << 10) or not _own_by_skinny(m, w.n, k, w.fp8, bool(w.rope))):
+    if m <= 16 and not w.fp8 and (few_route(m, w.n, k) or (few_takes(m, w.n, k) and not _own_by_skinny(m, w.n, k, False, bool(w.rope)))):
         return skinny_few(x, w, out, norm, resid, eps, rope)
     return skinny_gemm(x, w, out, norm=norm, resid=resid, eps=eps, rope=rope, counters=counters)
 
@@ -639,12 +649,12 @@ def _rope_args(rope: dict, m: int):
 
 def skinny_few(x: torch.Tensor, w: PackedWeight, out: torch.Tensor | None = None, norm: bool = False, resid: bool = False,
                eps: float = 1e-5, rope: dict | None = None) -> torch.Tensor:
-    """:func:`skinny_gemm` of up to 16 rows (:func:`few_takes`), whose RMSNorm (``norm``; its weight folded into W) takes the rows'
+    """:func:`skinny_gemm` of few rows (:func:`few_takes`), whose RMSNorm (``norm``; its weight folded into W) takes the rows'
     statistics from x itself; ``resid``: ``out += x @ W^T``. ``rope`` as there."""
     if x.dtype != torch.bfloat16 or not x.is_cuda or x.dim() != 2 or x.stride(1) != 1:
         raise ValueError("x must be a row-major bf16 GPU matrix")
     m, k = x.shape
-    if k != w.k or not few_takes(m, w.n, k, w.fp8):
+    if k != w.k or not few_takes(m, w.n, k, w.fp8, not norm and rope is None):
         raise ValueError(f"not a product of few rows: x {tuple(x.shape)}, W [{w.n}, {w.k}]")
     if (rope is not None) != bool(w.rope) or (resid and (rope is not None or w.swiglu)):
         raise ValueError("rope= needs a rope-packed qkv weight and vice versa; resid a plain one")

@@ -30,10 +30,8 @@ class Projection:
         if gated is not None and w.is_cuda:
             self.gated.limit_ptr(w.device)  # on the device before any hipGraph capture
         n, k = w.shape
-        # every default skinny tile: 64 or 128 rows of w, 8 or 16 k-steps of 32
-        fits = n % 128 == 0 and k % 512 == 0
         self.packed = None
-        if pack and fits and w.dtype == torch.bfloat16 and w.is_cuda:
+        if pack and n % (32 if gated is not None else 16) == 0 and k % 64 == 0 and w.dtype == torch.bfloat16 and w.is_cuda:
             self.packed = D.PackedWeight(self.w, swiglu=gated is not None, act=gated or "silu")
 
     def __call__(self, x: torch.Tensor) -> torch.Tensor:
@@ -42,8 +40,10 @@ class Projection:
             raise ValueError(f"x {tuple(x.shape)} {x.dtype} does not fit w {tuple(w.shape)} {w.dtype}")
         m, (n, k) = x.shape[0], w.shape
         if x.dtype == torch.bfloat16:
-            if m <= SKINNY_MAX_ROWS and self.packed is not None:
-                return D.skinny_gemm(x, self.packed)
+            if m <= D.SLAB_ROWS and self.packed is not None and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0:
+                y = self._packed(x, m, n, k)
+                if y is not None:
+                    return y
             if act is not None:
                 y = self._gated(x, m)
                 if y is not None:
@@ -60,6 +60,18 @@ class Projection:
         from .activation import act_mul
 
         return act_mul(y, act)
+
+    def _packed(self, x, m, n, k):
+        """The product by a kernel that reads the packed weight, or None. Up to 32 rows that of few rows or :func:`kgs.ops.decode.skinny_gemm` -- a gate and up of
+        one round of 64-row strips by :func:`kgs.ops.decode.skinny_rows` from 17 rows on (16384x2048 at 32 rows 16.1 us / 14.5) --, from
+        33 rows on ``skinny_rows`` where its wide tiles fill the CUs (us at 64 rows, four-wave tiles / so: 28672x4096 51.6 / 44.4, 32000x4096 61 / 48)."""
+        if m > SKINNY_MAX_ROWS:
+            return D.skinny_rows(x, self.packed) if D.slab_rows_tiles(m, n, k) == 2 else None
+        if D.few_route(m, n, k, True):
+            return D.skinny_few(x, self.packed)
+        if m > 16 and self.gated is not None and n <= 64 * D.CUS and D.slab_rows_tiles(m, n, k):
+            return D.skinny_rows(x, self.packed)
+        return D.skinny_gemm(x, self.packed) if D.skinny_takes(m, n, k) else None
 
     def partials(self, x: torch.Tensor) -> torch.Tensor:
         """:meth:`__call__`, or where the product of a decode batch runs in K slices those, fp32 ``[slices, M, N]``, for a consumer

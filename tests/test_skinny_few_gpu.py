@@ -69,9 +69,28 @@ def test_rope_and_cache_as_the_separate_launch(heads, kv, m):
     assert torch.equal(got, want) and torch.equal(caches[0].data, caches[1].data)
 
 
+# 2, 4 and 8 waves, rings of 1 to 4 k-steps, one and several rounds of them
+@pytest.mark.parametrize("n,k", ((16, 64), (48, 192), (2048, 128), (64, 384), (32, 768), (832, 1280), (2048, 768), (16, 2048), (64, 1536)))
+@pytest.mark.parametrize("m", (1, 16, 17, 32))
+def test_plain_products_of_any_short_sum(n, k, m):
+    x, w = _operands(m, n, k, 7)
+    pw = D.PackedWeight(w)
+    assert D.few_takes(m, n, k, plain=True)
+    ref = x.double() @ w.double().T
+    _close(D.skinny_few(x, pw), ref)
+    out = torch.randn(m, n, device="cuda").bfloat16()
+    want = out.double() + ref
+    _close(D.skinny_few(x, pw, out=out, resid=True), want)
+    if n % 32 == 0:
+        g, u = ref.chunk(2, 1)
+        _close(D.skinny_few(x, D.PackedWeight(w, swiglu=True)), torch.nn.functional.silu(g) * u, 4.0)
+
+
 def test_what_it_does_not_take():
     for m, n, k in ((17, 4096, 4096), (0, 4096, 4096), (4, 4096, 768), (4, 4104, 512)):
         assert not D.few_takes(m, n, k)
+    for m, n, k in ((33, 4096, 4096), (4, 4096, 96), (4, 4104, 512)):
+        assert not D.few_takes(m, n, k, plain=True)
     assert not D.few_takes(4, 4096, 4096, fp8=True)
     x, w = _operands(4, 32, 512)
     with pytest.raises(ValueError):
@@ -130,3 +149,20 @@ def test_norm_and_resid_are_refused_where_they_do_not_go():
         with pytest.raises(ValueError):
             D.skinny_gemm(x, pw, **kw)
     assert not D.own_takes(65, 4096, 2048) and not D.own_takes(16, 4096, 2048, fp8=True)
+
+
+@pytest.mark.parametrize("n,k,gated", ((2048, 768, False), (832, 2048, False), (2048, 128, False), (1504, 2048, False), (16384, 2048, True), (24576, 1024, True),
+                                       (32000, 512, False), (96, 64, True)))
+@pytest.mark.parametrize("m", (1, 9, 16, 17, 32, 33, 64, 96, 97))
+def test_projections_by_the_packed_weight(n, k, gated, m):
+    from kgs.ops.linear import Projection
+
+    x, w = _operands(m, n, k, 8)
+    ref = x.double() @ w.double().T
+    if gated:
+        g, u = ref.chunk(2, 1)
+        ref = torch.nn.functional.silu(g) * u
+    got = Projection(w, "silu" if gated else None)(x)
+    assert got.shape == ref.shape
+    # some routes round gate and up to bf16 before the product
+    assert bool(((got.double() - ref).abs() <= 2.0 ** -7 * ref.abs() + 2.0 ** -7 * (ref.abs().max() if gated else 0) + 1e-4 * ref.abs().max()).all())

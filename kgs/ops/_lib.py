@@ -55,6 +55,7 @@ _SIGS = {
     "kgs_pad_rows_bf16": ([_c_void_p] * 2 + [_c_long, _c_int, _c_long] + [_c_void_p] * 2 + [_c_long, _c_int, _c_long, _c_void_p],
                           _c_int),
     "kgs_gemm_bf16_tr": ([_c_void_p] * 3 + [_c_int] * 9 + [_c_void_p] * 2, _c_int),
+    "kgs_gemm_bf16_tr_pair": ([_c_void_p] * 5 + [_c_int] * 8 + [_c_void_p] * 3, _c_int),
     "kgs_gemm_bf16_nt_addc": ([_c_void_p, _c_void_p, _c_void_p] + [_c_int] * 6 + [_c_void_p], _c_int),
     "kgs_tile_queue_stats": ([_c_int, ctypes.POINTER(_c_long)], _c_int),
     "kgs_tile_queue_check": ([_c_int, ctypes.POINTER(_c_long)], _c_int),
@@ -236,7 +237,7 @@ def autograd():
                       "`python -m kgs.utils.build`", RuntimeWarning, stacklevel=2)
         return None
     names = ("kgs_gemm_bf16_nt_auto", "kgs_gemm_bf16_nt_padded", "kgs_gemm_bf16_nt_act", "kgs_pad_rows_bf16", "kgs_act_grad",
-             "kgs_gemm_bf16_tr", "kgs_gemm_bf16_nt_scratch", "kgs_gemm_bf16_nt_padded_scratch", "kgs_act_grad_parts",
+             "kgs_gemm_bf16_tr", "kgs_gemm_bf16_tr_pair", "kgs_gemm_bf16_nt_scratch", "kgs_gemm_bf16_nt_padded_scratch", "kgs_act_grad_parts",
              "kgs_gemm_bf16_tr_slices")
     _autograd.bind({n: ctypes.cast(getattr(so, n), ctypes.c_void_p).value for n in names})
     return _autograd

@@ -26,6 +26,7 @@ typedef int (*NtAct)(const void*, const void*, void*, void*, const void*, int, i
 typedef int (*PadRows)(const void*, void*, long, int, long, const void*, void*, long, int, long, hipStream_t);
 typedef int (*ActGrad)(const void*, const void*, void*, void*, float*, void*, int, int, int, int, hipStream_t);
 typedef int (*Tr)(const void*, const void*, void*, int, int, int, int, int, int, int, int, int, float*, hipStream_t);
+typedef int (*TrPair)(const void*, const void*, const void*, void*, void*, int, int, int, int, int, int, int, int, float*, float*, hipStream_t);
 typedef long (*Scratch)(int, int, int);
 typedef long (*PaddedScratch)(int, int, int, int, int);
 typedef int (*Parts)(int, int);
@@ -38,6 +39,7 @@ struct Entries {
   PadRows pad_rows;
   ActGrad act_grad;
   Tr tr;
+  TrPair tr_pair;
   Scratch scratch;
   PaddedScratch padded_scratch;
   Parts parts;
@@ -103,11 +105,16 @@ at::Tensor product(const at::Tensor& a, const at::Tensor& b, at::Tensor bias, in
   return out;
 }
 
+// room for the ns partial sums of an [m, n] product in K slices, none for a whole one
+at::Tensor slices(const at::Tensor& like, int ns, long m, long n) {
+  return ns > 1 ? fresh(like, {ns * m * ((n + 7) / 8 * 8)}, at::kFloat) : at::Tensor();
+}
+
 // op(a) . b over k on tiles that read K-major operands in place (a: [k, m] if ta; b: [k, n]), a's rows lda apart
 at::Tensor product_tr(const at::Tensor& a, int lda, const at::Tensor& b, int m, int n, int k, int ta, hipStream_t s) {
   const int ns = so.tr_slices(m, n, k, ta, 1);
   const at::Tensor out = fresh(a, {m, n});
-  const at::Tensor ws = ns > 1 ? fresh(a, {(long)ns * m * ((n + 7) / 8 * 8)}, at::kFloat) : at::Tensor();
+  const at::Tensor ws = slices(a, ns, m, n);
   check(so.tr(ptr(a), ptr(b), ptr(out), m, n, k, lda, (int)b.stride(0), n, ta, 1, ns, ptr<float>(ws), s), "gemm_tr", m, n, k);
   return out;
 }
@@ -181,6 +188,16 @@ struct LinearNode : torch::autograd::Function<LinearNode> {
     }
     even(need_w ? &x : nullptr, need_x ? &w : nullptr, s);
     at::Tensor gx, gw;
+    if (need_x && need_w) {  // both from one launch
+      const int nsx = so.tr_slices(m, k, n, 0, 1), nsw = so.tr_slices(n, k, m, 1, 1);
+      gx = fresh(gz, {m, k});
+      gw = fresh(gz, {n, k});
+      const at::Tensor wsx = slices(gz, nsx, m, k), wsw = slices(gz, nsw, n, k);
+      check(so.tr_pair(ptr(gz), ptr(w), ptr(x), ptr(gx), ptr(gw), m, n, k, ld, (int)w.stride(0), (int)x.stride(0), nsx, nsw,
+                       ptr<float>(wsx), ptr<float>(wsw), s),
+            "gemm_tr_pair", m, n, k);
+      return {gx, gw, gb, at::Tensor(), at::Tensor()};
+    }
     if (need_x) gx = product_tr(gz, ld, w, m, k, n, 0, s);  // dX[m, k] = dY[m, n] . W[n, k]
     if (need_w) gw = product_tr(gz, ld, x, n, k, m, 1, s);  // dW[n, k] = dY[m, n]^T . X[m, k]
     return {gx, gw, gb, at::Tensor(), at::Tensor()};
@@ -225,6 +242,7 @@ PYBIND11_MODULE(_autograd, mod) {
     bind(so.pad_rows, d, "kgs_pad_rows_bf16");
     bind(so.act_grad, d, "kgs_act_grad");
     bind(so.tr, d, "kgs_gemm_bf16_tr");
+    bind(so.tr_pair, d, "kgs_gemm_bf16_tr_pair");
     bind(so.scratch, d, "kgs_gemm_bf16_nt_scratch");
     bind(so.padded_scratch, d, "kgs_gemm_bf16_nt_padded_scratch");
     bind(so.parts, d, "kgs_act_grad_parts");

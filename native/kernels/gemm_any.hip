@@ -550,14 +550,14 @@ struct Operand {
   }
 };
 
+// workgroup `id` of the product's `wgs`
 template <bool TA, bool TB, bool SPLIT>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_tr(TrArgs a) {
-  __shared__ __attribute__((aligned(1024))) char smem[2 * 32768];
+__device__ __forceinline__ void tr_tile(const TrArgs& a, char* smem, int id, int wgs) {
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int ntm = (a.M + 127) / 128, ntn = (a.N + 127) / 128;
   int slice, tm, tn;
-  w4::tile_of<0, SPLIT>((int)blockIdx.x, (int)gridDim.x, ntm, ntn, slice, tm, tn);
+  w4::tile_of<0, SPLIT>(id, wgs, ntm, ntn, slice, tm, tn);
   const int m0 = tm * 128, n0 = tn * 128, k0 = SPLIT ? slice * a.ks : 0;
   const int kn = SPLIT ? min(a.K - k0, a.ks) : a.K, nt = (kn + BK - 1) / BK;
   Operand<TA> oa;
@@ -622,6 +622,25 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       }
     }
   }
+}
+
+template <bool TA, bool TB, bool SPLIT>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_tr(TrArgs a) {
+  __shared__ __attribute__((aligned(1024))) char smem[2 * 32768];
+  tr_tile<TA, TB, SPLIT>(a, smem, (int)blockIdx.x, (int)gridDim.x);
+}
+
+// A layer's two gradient products in one launch, dX = dY . W (its workgroups first) and dW = dY^T . X, the tiles of
+// gemm_tr and their bits. Layers of up to about a thousand rows are bound by the launches (some 4 us of host time each), and leave CUs
+// idle in either product. us, a training step by two launches / one: 64 rows, three layers, 512 - 2048 - 512 216 / 204;
+// 256 rows, three of 1024 219 / 202; 777 rows 768 - 3072 - 768 230 / 214; 1024 rows, two layers, 1024 - 4096 - 1024 186 / 175; from 2048 rows the
+// same time (2048 - 5504 - 2048 393 / 394).
+template <bool SPLIT0, bool SPLIT1>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_tr_pair(TrArgs x, TrArgs w, int wgx) {
+  __shared__ __attribute__((aligned(1024))) char smem[2 * 32768];
+  const int id = (int)blockIdx.x;
+  if (id < wgx) tr_tile<false, true, SPLIT0>(x, smem, id, wgx);
+  else tr_tile<true, true, SPLIT1>(w, smem, id - wgx, (int)gridDim.x - wgx);
 }
 
 // Sum of the K slices' partial tiles (fp32 [ns][M][ldp]) and the epilogue: a thread's 8 columns
@@ -963,31 +982,62 @@ int gemm_tr_ok(const void* A, const void* B, int M, int N, int K, int lda, int l
   return ((long)M + 127) / 128 * (((long)N + 127) / 128) * 64 < (1L << 31);
 }
 
-int gemm_tr(const void* A, const void* B, void* C, int M, int N, int K, int lda, int ldb, int ldc, int ta, int tb, int ns,
-            float* ws, hipStream_t s) {
+// A product's arguments, its slices as they come out (of ns asked for) and its workgroups
+inline any::TrArgs tr_args(const void* A, const void* B, void* C, int M, int N, int K, int lda, int ldb, int ldc, int& ns, float* ws,
+                           unsigned& wgs) {
   using namespace any;
   TrArgs a{(const unsigned short*)A, (const unsigned short*)B, C, M, N, K, lda, ldb, ldc, 0,
            ldc % 8 == 0 && (uintptr_t)C % 16 == 0};
-  const int ldp = (N + 7) / 8 * 8, vec = a.vec;
   a.ks = ceil_div(ceil_div(K, 128), ns) * 128;
   ns = ceil_div(K, a.ks);
   if (ns > 1) {
-    if (!ws) return KGS_ERR_ARG;
     a.C = ws;
-    a.ldc = ldp;
+    a.ldc = (N + 7) / 8 * 8;
   }
-  const dim3 grid((unsigned)(ceil_div(M, 128) * ceil_div(N, 128) * ns));
-#define KGS_TR(TA, TB)                                                                        \
-  if (ns > 1) hipLaunchKernelGGL((any::gemm_tr<TA, TB, true>), grid, dim3(256), 0, s, a);    \
-  else hipLaunchKernelGGL((any::gemm_tr<TA, TB, false>), grid, dim3(256), 0, s, a)
+  wgs = (unsigned)(ceil_div(M, 128) * ceil_div(N, 128) * ns);
+  return a;
+}
+
+inline void tr_reduce(const any::TrArgs& a, void* C, int ldc, int ns, float* ws, hipStream_t s) {
+  using namespace any;
+  if (ns < 2) return;
+  hipLaunchKernelGGL((any_reduce<EPI_NONE, false>), dim3((unsigned)ceil_div((long)a.M * (a.ldc / 8), 256)), dim3(256), 0, s, ws,
+                     (unsigned short*)C, nullptr, nullptr, a.M, a.N, ldc, a.ldc, ns, a.vec);
+}
+
+int gemm_tr(const void* A, const void* B, void* C, int M, int N, int K, int lda, int ldb, int ldc, int ta, int tb, int ns,
+            float* ws, hipStream_t s) {
+  using namespace any;
+  unsigned wgs;
+  const TrArgs a = tr_args(A, B, C, M, N, K, lda, ldb, ldc, ns, ws, wgs);
+  if (ns > 1 && !ws) return KGS_ERR_ARG;
+#define KGS_TR(TA, TB)                                                                            \
+  if (ns > 1) hipLaunchKernelGGL((any::gemm_tr<TA, TB, true>), dim3(wgs), dim3(256), 0, s, a);    \
+  else hipLaunchKernelGGL((any::gemm_tr<TA, TB, false>), dim3(wgs), dim3(256), 0, s, a)
   if (ta && tb) { KGS_TR(true, true); }
   else if (ta) { KGS_TR(true, false); }
   else if (tb) { KGS_TR(false, true); }
   else return KGS_ERR_ARG;
 #undef KGS_TR
-  if (ns > 1)
-    hipLaunchKernelGGL((any_reduce<EPI_NONE, false>), dim3((unsigned)ceil_div((long)M * (ldp / 8), 256)), dim3(256), 0, s, ws,
-                       (unsigned short*)C, nullptr, nullptr, M, N, ldc, ldp, ns, vec);
+  tr_reduce(a, C, ldc, ns, ws, s);
+  return (int)hipGetLastError();
+}
+
+// dX [m, k] = dY [m, n] . W [n, k] and dW [n, k] = dY^T . X [m, k]
+int gemm_tr_pair(const void* dY, const void* W, const void* X, void* dX, void* dW, int m, int n, int k, int ldy, int ldw, int ldx,
+                 int nsx, int nsw, float* wsx, float* wsw, hipStream_t s) {
+  using namespace any;
+  unsigned gx, gw;
+  const TrArgs x = tr_args(dY, W, dX, m, k, n, ldy, ldw, k, nsx, wsx, gx), w = tr_args(dY, X, dW, n, k, m, ldy, ldx, k, nsw, wsw, gw);
+  if ((nsx > 1 && !wsx) || (nsw > 1 && !wsw)) return KGS_ERR_ARG;
+  if ((long)gx + gw > 0x7fffffffL) return KGS_ERR_SHAPE;
+  const dim3 grid(gx + gw);
+  if (nsx > 1 && nsw > 1) hipLaunchKernelGGL((any::gemm_tr_pair<true, true>), grid, dim3(256), 0, s, x, w, (int)gx);
+  else if (nsx > 1) hipLaunchKernelGGL((any::gemm_tr_pair<true, false>), grid, dim3(256), 0, s, x, w, (int)gx);
+  else if (nsw > 1) hipLaunchKernelGGL((any::gemm_tr_pair<false, true>), grid, dim3(256), 0, s, x, w, (int)gx);
+  else hipLaunchKernelGGL((any::gemm_tr_pair<false, false>), grid, dim3(256), 0, s, x, w, (int)gx);
+  tr_reduce(x, dX, k, nsx, wsx, s);
+  tr_reduce(w, dW, k, nsw, wsw, s);
   return (int)hipGetLastError();
 }
 
@@ -1134,6 +1184,16 @@ KGS_EXPORT int kgs_gemm_bf16_tr(const void* A, const void* B, void* C, int M, in
   if (M <= 0 || N <= 0 || K <= 0 || ldc < N || ns < 1 || ns > 64) return KGS_ERR_SHAPE;
   if (!kgs::gemm_tr_ok(A, B, M, N, K, lda, ldb, ta, tb) || (uintptr_t)ws % 16) return KGS_ERR_ALIGN;
   return kgs::gemm_tr(A, B, C, M, N, K, lda, ldb, ldc, ta, tb, ns, ws, s);
+}
+
+// A linear layer's gradients in one launch, as two kgs_gemm_bf16_tr calls leave them: dX [m, k] = dY [m, n] . W [n, k] over nsx slices
+// of n (wsx: nsx m (k rounded up to 8) fp32 values if nsx > 1) and dW [n, k] = dY^T . X [m, k] over nsw of m (wsw alike).
+KGS_EXPORT int kgs_gemm_bf16_tr_pair(const void* dY, const void* W, const void* X, void* dX, void* dW, int m, int n, int k, int ldy,
+                                     int ldw, int ldx, int nsx, int nsw, float* wsx, float* wsw, hipStream_t s) {
+  if (m <= 0 || n <= 0 || k <= 0 || nsx < 1 || nsx > 64 || nsw < 1 || nsw > 64) return KGS_ERR_SHAPE;
+  if (!kgs::gemm_tr_ok(dY, W, m, k, n, ldy, ldw, 0, 1) || !kgs::gemm_tr_ok(dY, X, n, k, m, ldy, ldx, 1, 1)) return KGS_ERR_ALIGN;
+  if ((uintptr_t)wsx % 16 || (uintptr_t)wsw % 16) return KGS_ERR_ALIGN;
+  return kgs::gemm_tr_pair(dY, W, X, dX, dW, m, n, k, ldy, ldw, ldx, nsx, nsw, wsx, wsw, s);
 }
 
 // The tile that gemm_any chooses without scratch, for a gated product (N rows of gate and up) if gated: rows << 16 | columns.

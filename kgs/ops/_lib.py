@@ -187,6 +187,7 @@ _SIGS = {
                                  + [_c_int] * 2 + [_c_void_p, _c_long, _c_int] + [_c_void_p] * 2 + [_c_int] * 3
                                  + [_c_void_p], _c_int),
     "kgs_delta_forward": ([ctypes.POINTER(_c_void_p), ctypes.POINTER(_c_long), _c_void_p], _c_int),
+    "kgs_delta_step": ([ctypes.POINTER(_c_void_p), ctypes.POINTER(_c_long), ctypes.c_float, _c_void_p], _c_int),
     "kgs_delta_out": ([_c_void_p] * 4 + [_c_int] * 3 + [_c_long] * 2 + [ctypes.c_float, _c_int, _c_void_p], _c_int),
     # peer-to-peer all-reduce (native/kernels/allreduce_p2p.hip)
     "kgs_ar_signal_bytes": ([], _c_int),

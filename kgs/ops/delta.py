@@ -141,3 +141,33 @@ def delta_out(o: torch.Tensor, w: torch.Tensor, gate: torch.Tensor, eps: float, 
                                   int(gate.dtype == torch.float32), _lib.stream_handle(o.device))
     _lib.check(rc, f"delta_out[{T}x{H}x{V}]")
     return y
+
+
+def step_takes(z: torch.Tensor, offs: tuple[int, int, int, int], a2: torch.Tensor, gate: torch.Tensor, sh: DeltaShape, seqs: RaggedSeqs,
+               ld: int) -> bool:
+    """Whether :func:`delta_step` takes a call: as many rows as sequences, none by chunks, heads of 128 with a q / k head each, 4 taps,
+    and channel pairs on even columns."""
+    return (seqs.chunks is None or not seqs.chunks.shape[0]) and z.shape[0] == seqs.row0.shape[0] and sh.heads == sh.kv_heads and \
+        sh.dim == sh.vdim == 128 and sh.taps == 4 and \
+        not (any(x % 2 for x in (z.stride(0), a2.stride(0), gate.stride(0), ld, *offs[:3])) or
+             any(t.data_ptr() % 4 for t in (z, a2, gate)))
+
+
+def delta_step(z: torch.Tensor, offs: tuple[int, int, int, int], a2: torch.Tensor, cw: torch.Tensor, a_log: torch.Tensor,
+               dt_bias: torch.Tensor, sh: DeltaShape, state: DeltaState, seqs: RaggedSeqs, w: torch.Tensor, gate: torch.Tensor,
+               eps: float, ld: int) -> torch.Tensor:
+    """:func:`delta_forward` and :func:`delta_out` in one launch, where :func:`step_takes` it. State slot 0 is nobody's here: rows of its
+    sequences come out as zeros, and it is neither read nor written."""
+    T, dev = z.shape[0], z.device
+    H, hk, B = sh.heads, sh.heads * 128, seqs.row0.shape[0]
+    if not step_takes(z, offs, a2, gate, sh, seqs, ld):
+        raise ValueError(f"delta_step: {T} rows of {B} sequences, {sh}")
+    _act(z, T, max(*(x + hk for x in offs[:3]), offs[3] + H), z.dtype, "z")
+    y = torch.empty((T, ld), dtype=z.dtype, device=dev)
+    ptrs = (ctypes.c_void_p * 14)(
+        z.data_ptr(), _act(a2, T, hk, z.dtype, "a2"), _f32(cw, (sh.taps, sh.channels), "cw"), _f32(a_log, (H,), "a_log"),
+        _f32(dt_bias, (hk,), "dt_bias"), seqs.row0.data_ptr(), seqs.n.data_ptr(), seqs.pos0.data_ptr(), seqs.slot.data_ptr(),
+        state.S.data_ptr(), state.conv.data_ptr(), _act(gate, T, hk, z.dtype, "gate"), _f32(w, (128,), "w"), y.data_ptr())
+    dims = (ctypes.c_long * 12)(z.stride(0), a2.stride(0), *offs, H, B, T, int(z.dtype == torch.float32), gate.stride(0), ld)
+    _lib.check(_lib.lib().kgs_delta_step(ptrs, dims, float(eps), _lib.stream_handle(dev)), f"delta_step[{T}x{H}]")
+    return y

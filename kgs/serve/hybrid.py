@@ -25,7 +25,7 @@ from kgs.models.ruruzen import DeltaSpec, LatentSpec, RuruzenConfig
 from kgs.ops.activation import softcap
 from kgs.ops import decode as D
 from kgs.ops.decode import PAGE
-from kgs.ops.delta import DeltaShape, DeltaState, delta_forward, delta_out
+from kgs.ops.delta import DeltaShape, DeltaState, delta_forward, delta_out, delta_step, step_takes
 from kgs.ops.hyper import MAX_STREAMS, hyper_embed, hyper_step
 from kgs.ops.latent import (LatentCache, LatentRows, head_proj, latent_attention, latent_norm, mfma_sizes,
                             padded_latent, padded_rot, split_count, split_parts, waves_for, window_pages)
@@ -266,9 +266,11 @@ class DeltaMixer:
         a2 = self.a2(z[:, self.oa:self.oa + self.ra])
         g2 = self.g2(z[:, self.og:self.og + self.rg])
         T.op(f"L{self.layer} delta projections")
-        o = delta_forward(z, self.offs, a2, self.cw, self.a_log, self.dt_bias, self.shape, model.state[self.layer],
-                          b.seqs)
-        y = delta_out(o, self.norm, g2, self.eps, self.ld)
+        args = (z, self.offs, a2, self.cw, self.a_log, self.dt_bias, self.shape, model.state[self.layer], b.seqs)
+        if step_takes(z, self.offs, a2, g2, self.shape, b.seqs, self.ld):
+            y = delta_step(*args, self.norm, g2, self.eps, self.ld)
+        else:
+            y = delta_out(delta_forward(*args), self.norm, g2, self.eps, self.ld)
         T.op(f"L{self.layer} delta rule")
         return self.o.partials(y)
 

@@ -11,7 +11,8 @@
 // Short sequences (decode) step token by token:
 //   prep   the short causal convolutions + silu of q, k, v (tail of the previous
 //          portion from the pool), unit norms, log decays, step sizes;
-//   scan   the recurrence.
+//   scan   the recurrence;
+//   step   both and out in one, for one token a sequence of the usual sizes.
 // Longer ones go by chunks of C = 16 tokens. With b_i the log decays summed from
 // the chunk's start, S_0 the state before it and every exponent taken as a
 // difference b_i - b_j <= 0 (any decay is safe):
@@ -780,6 +781,171 @@ __global__ __launch_bounds__(256) void out(OutArgs a) {
   for (int i = lane; i < V; i += 64) st(y + i, o[i] * r * a.w[i] * sigm<FAST>(ld(gate + i)));
 }
 
+// ----------------------------------------------------------------------- step
+struct StepArgs {
+  Args a;
+  OutArgs out;
+};
+
+// One token a sequence: prep, scan and out in one launch, for K = V = 128, 4 taps and a q / k head per head. A workgroup
+// takes one head of one sequence; waves 0 to 5 prepare its q, k, v, decays, gate and step size while all eight wait for the 64 KB of state,
+// which crosses memory once each way and bounds the kernel. The arithmetic is that of the three kernels, in their order. Slot 0 is
+// nobody's: its rows are zeros (padding wrote its state 8 MB at a time). us in a captured graph, three launches / one, 16 heads: 1 sequence
+// 11.8 / 7.1, 10 in a batch of 16 17.9 / 9.0, 24 of 32 27.9 / 15.8, 60 of 64 43 / 32 (3.9 TB/s), 128 71 / 61; 32 heads, 128 125 / 116 (4.6 TB/s).
+// 128 registers, so that two workgroups share a CU (170, as prep_token's code would have it, take 24 sequences 4 us longer).
+template <typename T>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) void step(StepArgs s) {
+  constexpr bool FAST = sizeof(T) == 2;
+  constexpr int K = 128, TAPS = 4;
+  __shared__ __attribute__((aligned(16))) float sq[K], sk[K], sraw[K], sg[K], sv[K], su[K], so[K];
+  __shared__ float sbeta, srq, srk, sqk;
+  const Args& a = s.a;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), rg = lane >> 3, i0 = 2 * lane;
+  const int h = blockIdx.x, b = blockIdx.y, H = a.H;
+  const int r0 = a.row0[b], n = a.n[b], p0 = a.pos0[b];
+  const long slot = a.slot[b];
+  const bool live = slot != 0;
+  for (int t = 0; t < n; ++t) {
+    T* const y = (T*)s.out.y + (r0 + t) * s.out.ldy;
+    if (h == 0)
+      for (int i = H * K + threadIdx.x; i < s.out.ldy; i += 512) st(y + i, 0.f);
+    if (!live && threadIdx.x < K) st(y + h * K + threadIdx.x, 0.f);
+  }
+  if (!live) return;
+
+  // a wave's part of token t: its last taps of q, k or v (x), its decays, its gate (x[3]), its step size (x[3][0])
+  const T* src = w < 3    ? (const T*)a.z + (w == 0 ? a.oq : w == 1 ? a.ok : a.ov) + h * K + i0
+                 : w == 3 ? (const T*)a.a2 + h * K + i0
+                 : w == 4 ? (const T*)s.out.gate + h * K + i0
+                          : (const T*)a.z + a.ob + h;
+  const long ld_src = w == 3 ? a.lda : w == 4 ? s.out.ldg : a.ldz;
+  src += r0 * ld_src;
+  float* const tail = a.conv + slot * (TAPS - 1) * a.C + (w < 3 ? w * H * K + h * K + i0 : 0);
+  float x[TAPS][2] = {}, cw[TAPS][2] = {};
+  auto fetch = [&](int t) {
+    if (w < 5) ldn(src + t * ld_src, x[3]);
+    else x[3][0] = ld(src + t * ld_src);
+  };
+  auto pair = [](const float* p, float (&v)[2]) {
+    const float2 f = *(const float2*)p;
+    v[0] = f.x;
+    v[1] = f.y;
+  };
+  if (n > 0 && w < 6) fetch(0);
+  if (w < 3) {
+#pragma unroll
+    for (int j = 0; j < TAPS; ++j) {
+      if (j < 3 && p0 > 0) pair(tail + j * a.C, x[j]);
+      pair(a.cw + j * a.C + w * H * K + h * K + i0, cw[j]);
+    }
+  } else if (w == 3) {
+    pair(a.dt_bias + h * K + i0, cw[0]);
+    cw[1][0] = a.A_log[h];
+  } else if (w == 4) {
+    pair(s.out.w + i0, cw[0]);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  // lane (rg, c) holds rows 32 i + 4 rg + j of columns 8 w + c and 64 + 8 w + c
+  const int col = 8 * w + (lane & 7);
+  float* const Sp = a.S + ((slot * H + h) * K + col) * K + 4 * rg;
+  f32x4 S[2][4];
+#pragma unroll
+  for (int c = 0; c < 2; ++c)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) S[c][i] = p0 > 0 ? *(const f32x4*)(Sp + 64 * K * c + 32 * i) : f32x4{};
+  __builtin_amdgcn_sched_barrier(0);
+  for (int t = 0; t < n; ++t) {
+    if (t) {  // the next token's taps
+      if (w < 3) {
+#pragma unroll
+        for (int j = 0; j < TAPS - 1; ++j) x[j][0] = x[j + 1][0], x[j][1] = x[j + 1][1];
+      }
+      __syncthreads();
+      if (w < 6) fetch(t);
+    }
+    float y[2] = {};
+    if (w < 3) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        float v = 0.f;
+#pragma unroll
+        for (int j = 0; j < TAPS; ++j) v = __builtin_fmaf(cw[j][i], x[j][i], v);
+        y[i] = v * sigm<FAST>(v);
+      }
+      if (w == 2) {
+        *(float2*)&sv[i0] = make_float2(y[0], y[1]);
+      } else {
+        const float ss = wave_sum(__builtin_fmaf(y[1], y[1], __builtin_fmaf(y[0], y[0], 0.f)));
+        const float r = w == 0 ? 1.0f / sqrtf(ss + 1e-6f) / sqrtf((float)K) : 1.0f / sqrtf(ss + 1e-6f);
+        *(float2*)&(w == 0 ? sq : sk)[i0] = make_float2(y[0] * r, y[1] * r);
+        if (w == 1) *(float2*)&sraw[i0] = make_float2(y[0], y[1]);
+        if (lane == 0) (w == 0 ? srq : srk) = r;
+      }
+    } else if (w == 3) {
+      const float A = -expf(cw[1][0]);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) sg[i0 + i] = expf(A * softplus<FAST>(x[3][i] + cw[0][i]));
+    } else if (w == 5 && lane == 0) {
+      sbeta = sigm<FAST>(x[3][0]);
+    }
+    __syncthreads();
+    if (w == 0) {
+      const float2 k = *(const float2*)&sraw[i0];
+      const float qk = wave_sum(__builtin_fmaf(y[1], k.y, __builtin_fmaf(y[0], k.x, 0.f)));
+      if (lane == 0) sqk = qk * srq * srk;
+    }
+    f32x4 k[4];
+    float dk[2] = {}, dq[2] = {};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      k[i] = *(const f32x4*)&sk[32 * i + 4 * rg];
+      const f32x4 q = *(const f32x4*)&sq[32 * i + 4 * rg], g = *(const f32x4*)&sg[32 * i + 4 * rg];
+#pragma unroll
+      for (int c = 0; c < 2; ++c)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const float v = S[c][i][j] * g[j];
+          S[c][i][j] = v;
+          dk[c] = __builtin_fmaf(v, k[i][j], dk[c]);
+          dq[c] = __builtin_fmaf(v, q[j], dq[c]);
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      dk[c] = xor32_sum(xor16_sum(xor8_sum(dk[c])));
+      dq[c] = xor32_sum(xor16_sum(xor8_sum(dq[c])));
+      const float u = sbeta * (sv[64 * c + col] - dk[c]);
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) S[c][i][j] = __builtin_fmaf(k[i][j], u, S[c][i][j]);
+      if (rg == 0) {
+        su[64 * c + col] = u;
+        so[64 * c + col] = dq[c];
+      }
+    }
+    __syncthreads();
+    if (w == 4) {
+      const float2 u = *(const float2*)&su[i0], d = *(const float2*)&so[i0];
+      const float o0 = __builtin_fmaf(sqk, u.x, d.x), o1 = __builtin_fmaf(sqk, u.y, d.y);
+      const float r = 1.0f / sqrtf(wave_sum(o0 * o0 + o1 * o1) / K + s.out.eps);
+      const float y0 = o0 * r * cw[0][0] * sigm<FAST>(x[3][0]), y1 = o1 * r * cw[0][1] * sigm<FAST>(x[3][1]);
+      T* const out = (T*)s.out.y + (r0 + t) * s.out.ldy + h * K + i0;
+      if constexpr (FAST) *(unsigned*)out = pack_bf16x2(y0, y1);
+      else *(float2*)out = make_float2(y0, y1);
+    }
+  }
+#pragma unroll
+  for (int c = 0; c < 2; ++c)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) *(f32x4*)(Sp + 64 * K * c + 32 * i) = S[c][i];
+  // the tails, which these lanes alone read: the last three inputs
+  if (w < 3 && (n > 0 || p0 == 0)) {
+#pragma unroll
+    for (int j = 1; j < TAPS; ++j) *(float2*)(tail + (j - 1) * a.C) = make_float2(x[j][0], x[j][1]);
+  }
+}
+
 template <typename T, int NS>
 static void run_chunk_scan(const Args& a, hipStream_t s) {
   const dim3 grid((unsigned)((a.V + 16 * NS - 1) / (16 * NS) * ((a.H * a.ncseqs + 7) / 8) * 8));  // whole rounds of the XCDs
@@ -921,5 +1087,52 @@ KGS_EXPORT int kgs_delta_out(const void* o, const void* w, const void* gate, voi
   const dim3 grid(T, (H + 3) / 4);
   if (f32) hipLaunchKernelGGL(out<float>, grid, dim3(256), 0, s, a);
   else hipLaunchKernelGGL(out<unsigned short>, grid, dim3(256), 0, s, a);
+  return (int)hipGetLastError();
+}
+
+// kgs_delta_forward and kgs_delta_out of one token a sequence (any number of them is right, in turn) in one launch: K = V = 128, 4 taps, a q /
+// k head per head. A sequence of slot 0 is nobody's: its rows of y are zeros, and no state is read or written.
+// ptrs (14 device pointers): z a2 cw A_log dt_bias row0 n pos0 slot S conv gate w y; dims (12): ldz lda oq ok ov ob H B T f32 ldg ldy
+KGS_EXPORT int kgs_delta_step(const void* const* ptrs, const long* dims, float eps, hipStream_t s) {
+  using namespace kgs::delta;
+  StepArgs x{};
+  Args& a = x.a;
+  a.z = ptrs[0];
+  a.a2 = ptrs[1];
+  a.cw = (const float*)ptrs[2];
+  a.A_log = (const float*)ptrs[3];
+  a.dt_bias = (const float*)ptrs[4];
+  a.row0 = (const int*)ptrs[5];
+  a.n = (const int*)ptrs[6];
+  a.pos0 = (const int*)ptrs[7];
+  a.slot = (const int*)ptrs[8];
+  a.S = (float*)ptrs[9];
+  a.conv = (float*)ptrs[10];
+  a.ldz = dims[0];
+  a.lda = dims[1];
+  a.oq = (int)dims[2];
+  a.ok = (int)dims[3];
+  a.ov = (int)dims[4];
+  a.ob = (int)dims[5];
+  a.taps = 4;
+  a.G = a.H = (int)dims[6];
+  a.K = a.V = a.KP = 128;
+  a.B = (int)dims[7];
+  a.T = (int)dims[8];
+  const bool f32 = dims[9] != 0;
+  a.C = 3 * a.H * 128;
+  x.out = OutArgs{nullptr, (const float*)ptrs[12], ptrs[11], (void*)ptrs[13], dims[10], dims[11], a.H, 128, eps};
+  const long hk = 128l * a.H;
+  if (a.H < 1 || a.H > 65535 || a.B < 1 || a.B > 65535 || a.T < 1) return KGS_ERR_SHAPE;
+  if (a.oq < 0 || a.ok < 0 || a.ov < 0 || a.ob < 0 || a.ldz < a.oq + hk || a.ldz < a.ok + hk || a.ldz < a.ov + hk ||
+      a.ldz < a.ob + a.H || a.lda < hk || x.out.ldg < hk || x.out.ldy < hk || x.out.ldy > 0x7fffffff)
+    return KGS_ERR_SHAPE;
+  if ((a.ldz | a.lda | a.oq | a.ok | a.ov | x.out.ldg | x.out.ldy) % 2 ||
+      (((uintptr_t)a.z | (uintptr_t)a.a2 | (uintptr_t)x.out.gate) & 3) || ((uintptr_t)x.out.y & (f32 ? 7 : 3)) ||
+      (((uintptr_t)a.cw | (uintptr_t)a.conv | (uintptr_t)a.dt_bias | (uintptr_t)x.out.w) & 7) || ((uintptr_t)a.S & 15))
+    return KGS_ERR_ALIGN;
+  const dim3 grid(a.H, a.B);
+  if (f32) hipLaunchKernelGGL(step<float>, grid, dim3(512), 0, s, x);
+  else hipLaunchKernelGGL(step<unsigned short>, grid, dim3(512), 0, s, x);
   return (int)hipGetLastError();
 }

@@ -21,7 +21,8 @@
 //   U = T V - (T K~) S_0        K~_i = k_i e^(b_i)
 //   O = Q~ S_0 + P U            Q~_i = q_i e^(b_i)
 //   S = diag(e^(b_C)) S_0 + K^^T U   K^_j = k_j e^(b_C - b_j)
-//   chunk_prep  everything that does not need S_0, one workgroup per (chunk, head);
+//   chunk_prep  everything that does not need S_0, one workgroup per (chunk, head): 16 heads of 128, 225 chunks 67 us, 456 chunks 133,
+//               its stores (35 KB each) take 25 and 50 of it;
 //   chunk_scan  the three products with the state per chunk, on fp32 MFMAs.
 // Both scans also update the convolution tails; out applies the per-head norm and gate.
 //
@@ -109,6 +110,26 @@ __device__ __forceinline__ void ldn(const T* p, float (&v)[N]) {
   }
 }
 
+// ... as loaded, to be widened once they are needed: a load that is widened in the branch that it stands in is waited for there
+template <typename T, int N>
+struct Raw {
+  static constexpr bool WORD = N == 2 && sizeof(T) == 2;
+  typename std::conditional<WORD, unsigned, T>::type u[WORD ? 1 : N];
+  __device__ __forceinline__ void load(const T* p) {
+    if constexpr (WORD) {
+      u[0] = *(const unsigned*)p;
+    } else {
+#pragma unroll
+      for (int i = 0; i < N; ++i) u[i] = p[i];
+    }
+  }
+  __device__ __forceinline__ float operator[](int i) const {
+    if constexpr (WORD) return bf2f((unsigned short)(i ? u[0] >> 16 : u[0] & 0xffff));
+    else if constexpr (sizeof(T) == 2) return bf2f(u[i]);
+    else return u[i];
+  }
+};
+
 // channels c .. c + N - 1 (column col of z) of row src of the sequence that starts at
 // row r0 (position p0): rows ahead of it come from the pool's tail
 template <typename T, int N>
@@ -150,15 +171,30 @@ template <typename T, int N, int TAPS, class F>
 __device__ __forceinline__ void conv_rows(const Args& a, long t0, int n, int c, int col, int r0, int p0, long slot,
                                           F store) {
   if constexpr (TAPS > 0) {
+    // All rows on their way at once, those ahead of the sequence or past its portion as copies of its ends. A row at a time, each
+    // waited for behind its condition, the convolutions were 37 of chunk_prep's 86 us for 3600 chunks and heads, now 17 of 67.
+    Raw<T, N> raw[16 + TAPS - 1];
     float x[16 + TAPS - 1][N], w[TAPS][N];
 #pragma unroll
+    for (int j = 0; j < 16 + TAPS - 1; ++j)
+      raw[j].load((const T*)a.z + max((long)r0, min(t0 + n - 1, t0 - (TAPS - 1) + j)) * a.ldz + (unsigned)col);
+#pragma unroll
     for (int j = 0; j < TAPS; ++j) ldn(a.cw + (long)j * a.C + c, w[j]);
+    float old[TAPS - 1][N] = {};
+    if (t0 - (TAPS - 1) < r0 && p0 > 0) {
 #pragma unroll
-    for (int j = 0; j < 16 + TAPS - 1; ++j) {
-#pragma unroll
-      for (int i = 0; i < N; ++i) x[j][i] = 0.f;
-      if (j - (TAPS - 1) < n) conv_in<T, N>(a, t0 - (TAPS - 1) + j, c, col, r0, p0, slot, x[j]);
+      for (int j = 0; j < TAPS - 1; ++j)
+        if (t0 - (TAPS - 1) + j < r0)
+          ldn(a.conv + (slot * (TAPS - 1) + (t0 - r0 + j)) * a.C + (unsigned)c, old[j]);
     }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int j = 0; j < 16 + TAPS - 1; ++j)
+#pragma unroll
+      for (int i = 0; i < N; ++i) {
+        const float v = raw[j][i];
+        x[j][i] = j - (TAPS - 1) >= n ? 0.f : j < TAPS - 1 && t0 - (TAPS - 1) + j < r0 ? old[j < TAPS - 1 ? j : 0][i] : v;
+      }
 #pragma unroll
     for (int t = 0; t < 16; ++t) {
       float y[N] = {};
@@ -420,13 +456,10 @@ __global__ __launch_bounds__(256, 4) void chunk_prep(Args a) {
       const float A = -expf(a.A_log[h]) * LOG2E;  // b: sums of log decays, in log2 units
       float s[N] = {}, dt[N] = {};
       if (c < K) ldn(a.dt_bias + h * K + c, dt);
-      float x[CH][N];
+      Raw<T, N> x[CH];
+      const int cin = min(c, K - N);
 #pragma unroll
-      for (int t = 0; t < CH; ++t) {
-#pragma unroll
-        for (int i = 0; i < N; ++i) x[t][i] = 0.f;
-        if (t < n && c < K) ldn((const T*)a.a2 + (t0 + t) * a.lda + h * K + (unsigned)c, x[t]);
-      }
+      for (int t = 0; t < CH; ++t) x[t].load((const T*)a.a2 + (t0 + min(t, n - 1)) * a.lda + h * K + (unsigned)cin);
 #pragma unroll
       for (int t = 0; t < CH; ++t)
 #pragma unroll

@@ -621,6 +621,11 @@ __global__ __launch_bounds__(256, 4) void chunk_prep(Args a) {
 // contraction indices are 4 g + r, so state and U feed the products without
 // moving; the A operands are read as float4s in that order. The waves' partial
 // products over their rows meet in LDS, one barrier per chunk.
+// A sequence's chunks are a serial chain, W S, its sum over the waves, K U, so what is not on it is shared or kept out of its way: TV
+// enters the sum a quarter a wave, P U a wave's part of O, whose sum is stored a chunk later, a row in four a wave; and the next operands
+// are sent for in two parts, W and Q under the barrier's wait. us, one wave a chunk for O and all loads at the chunk's end / so, 16 heads: one
+// sequence of 1216 tokens 89 / 67, six of 3600 116 / 108, six of 1216 each 215 / 200. Bound by that chain's latencies (0.83 us a chunk alone), then by
+// the operands' way into the CUs (27 KB a chunk and workgroup). A fifth wave for TV and O: 80, 127 and 280 us; three waves a SIMD by a shorter ring: 69, 113, 277.
 // NS 2 reads the A operands half as often; NS 1 spreads few heads over more CUs.
 template <typename T, int MT, int NS>
 __global__ __launch_bounds__(256) void chunk_scan(Args a) {
@@ -652,7 +657,8 @@ __global__ __launch_bounds__(256) void chunk_scan(Args a) {
     }
   }
   struct Frag {
-    f32x4 W[MT], Q[MT], K[MT], E[MT], U[NS], P;
+    f32x4 W[MT], Q[MT], K[MT], E[MT];
+    float U[NS], P;  // rows 4 g + w of T V, column 4 g + w of P
   };
   // Loads without conditions (a wave's rows past the last tile repeat it, columns
   // past V the last one), so that the number in flight is known at every wait;
@@ -666,32 +672,55 @@ __global__ __launch_bounds__(256) void chunk_scan(Args a) {
     le[m] = 16 * tile + 4 * g;
   }
 #pragma unroll
-  for (int s = 0; s < NS; ++s) lu[s] = 4 * g * V + col[s];
-  const unsigned lp = l16 * CH + 4 * g;
-  auto fetch = [&](int c, Frag& f) {
-    const long base = (long)(sq.y + c) * H + h;
-    const float *W = a.cW + base * CH * KP, *Q = a.cQ + base * CH * KP, *K = a.cK + base * CH * KP;
-    const float *E = a.cE + base * KP, *U = a.cU + base * CH * V, *P = a.cP + base * CH * CH;
+  for (int s = 0; s < NS; ++s) lu[s] = (4 * g + w) * V + col[s];
+  const unsigned lp = l16 * CH + 4 * g + w;
+  // in two parts, each as its registers are free
+  auto base = [&](int c) { return (long)(sq.y + c) * H + h; };
+  auto fetch_wq = [&](int c, Frag& f) __attribute__((always_inline)) {
+    const float *W = a.cW + base(c) * CH * KP, *Q = a.cQ + base(c) * CH * KP, *U = a.cU + base(c) * CH * V;
 #pragma unroll
     for (int m = 0; m < MT; ++m) {
       f.W[m] = *(const f32x4*)(W + lw[m]);
       f.Q[m] = *(const f32x4*)(Q + lw[m]);
+    }
+#pragma unroll
+    for (int s = 0; s < NS; ++s) f.U[s] = U[lu[s]];
+    __builtin_amdgcn_sched_barrier(0);  // chunks are loaded in order: their waits are counted in it
+  };
+  auto fetch_k = [&](int c, Frag& f) __attribute__((always_inline)) {
+    const float *K = a.cK + base(c) * CH * KP, *E = a.cE + base(c) * KP;
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
       f.K[m] = *(const f32x4*)(K + lk[m]);
       f.E[m] = *(const f32x4*)(E + le[m]);
     }
-#pragma unroll
-    for (int s = 0; s < NS; ++s)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) f.U[s][r] = (U + (unsigned)(r * V))[lu[s]];
-    f.P = *(const f32x4*)(P + lp);
-    __builtin_amdgcn_sched_barrier(0);  // chunks are loaded in order: their waits are counted in it
+    f.P = (a.cP + base(c) * CH * CH)[lp];
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto fetch = [&](int c, Frag& f) __attribute__((always_inline)) {
+    fetch_wq(c, f);
+    fetch_k(c, f);
   };
   // a ring of RING chunks' operands in registers: loads run RING - 1 chunks ahead
   constexpr int RING = MT == 1 || (MT == 2 && NS == 1) ? 4 : MT == 2 ? 3 : 2;
+  auto at_w = [&](const f32x4& x) { return w == 0 ? x[0] : w == 1 ? x[1] : w == 2 ? x[2] : x[3]; };
+  auto store_o = [&](int c) {  // row 4 g + w of chunk c's O, whose parts lie there
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+      const float* p = (const float*)&part[c & 1][1][s][0][lane] + w;
+      const float o = p[0] + p[256] + p[512] + p[768];
+      const int t = CH * c + 4 * g + w;
+      if (t < n && live[s]) a.o[((long)(sq.w + t) * H + h) * V + col[s]] = o;
+    }
+  };
   auto step = [&](int c, Frag& f) __attribute__((always_inline)) {
     f32x4 pu[NS], po[NS];
 #pragma unroll
-    for (int s = 0; s < NS; ++s) pu[s] = po[s] = f32x4{};
+    for (int s = 0; s < NS; ++s) {
+      po[s] = f32x4{};
+#pragma unroll
+      for (int r = 0; r < 4; ++r) pu[s][r] = w == r ? -f.U[s] : 0.f;
+    }
 #pragma unroll
     for (int m = 0; m < MT; ++m)
 #pragma unroll
@@ -703,16 +732,15 @@ __global__ __launch_bounds__(256) void chunk_scan(Args a) {
         }
     const int buf = c & 1;
 #pragma unroll
-    for (int s = 0; s < NS; ++s) {
-      part[buf][0][s][w][lane] = pu[s];
-      part[buf][1][s][w][lane] = po[s];
-    }
+    for (int s = 0; s < NS; ++s) part[buf][0][s][w][lane] = pu[s];
+    __builtin_amdgcn_sched_barrier(0);
+    fetch_wq(min(c + RING, sq.z - 1), f);
     __syncthreads();
+    if (c > 0) store_o(c - 1);
     f32x4 U[NS];
 #pragma unroll
     for (int s = 0; s < NS; ++s)
-      U[s] = f.U[s] - (part[buf][0][s][0][lane] + part[buf][0][s][1][lane] + part[buf][0][s][2][lane] +
-                       part[buf][0][s][3][lane]);
+      U[s] = -(part[buf][0][s][0][lane] + part[buf][0][s][1][lane] + part[buf][0][s][2][lane] + part[buf][0][s][3][lane]);
 #pragma unroll
     for (int m = 0; m < MT; ++m)
 #pragma unroll
@@ -724,26 +752,19 @@ __global__ __launch_bounds__(256) void chunk_scan(Args a) {
 #pragma unroll
         for (int s = 0; s < NS; ++s)
           S[m][s] = __builtin_amdgcn_mfma_f32_16x16x4f32(f.K[m][r], U[s][r], S[m][s], 0, 0, 0);
+    // a wave's quarter of P U goes into its part of O
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+      po[s] = __builtin_amdgcn_mfma_f32_16x16x4f32(f.P, at_w(U[s]), po[s], 0, 0, 0);
+      part[buf][1][s][w][lane] = po[s];
+    }
 #pragma unroll
     for (int m = 0; m < MT; ++m)
       if (w + 4 * m >= ntile) {  // no such rows
 #pragma unroll
         for (int s = 0; s < NS; ++s) S[m][s] = f32x4{};
       }
-#pragma unroll
-    for (int s = 0; s < NS; ++s)
-      if (w == ((c + 2 * s) & 3)) {
-        f32x4 O = part[buf][1][s][0][lane] + part[buf][1][s][1][lane] + part[buf][1][s][2][lane] +
-                  part[buf][1][s][3][lane];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) O = __builtin_amdgcn_mfma_f32_16x16x4f32(f.P[r], U[s][r], O, 0, 0, 0);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int t = CH * c + 4 * g + r;
-          if (t < n && live[s]) a.o[((long)(sq.w + t) * H + h) * V + col[s]] = O[r];
-        }
-      }
-    fetch(min(c + RING, sq.z - 1), f);
+    fetch_k(min(c + RING, sq.z - 1), f);
   };
   Frag f0, f1, f2, f3;
   fetch(0, f0);
@@ -762,6 +783,8 @@ __global__ __launch_bounds__(256) void chunk_scan(Args a) {
     if (c + 1 < sq.z) step(c + 1, f1);
   if constexpr (RING > 3)
     if (c + 2 < sq.z) step(c + 2, f2);
+  __syncthreads();
+  store_o(sq.z - 1);
 #pragma unroll
   for (int s = 0; s < NS; ++s)
     if (live[s]) {
@@ -1020,8 +1043,8 @@ static hipError_t run(const Args& a, hipStream_t s) {
     hipLaunchKernelGGL(prep_k, dim3((unsigned)(a.nchunks * a.H)), dim3(256), lds, s, a);
     // Slabs of 32 columns read the chunks' operands half as often; of 16 they halve a chain's step, which is what counts where
     // there are few workgroups or the longest chain (a.longest chunks, 0: unknown) is above a CU's mean share of all
-    // chunks. us, 32 / 16 columns, longest chain over share: 6 prompts of 3580 tokens 170 / 138 (1.35), 7 of 3140 153 / 119
-    // (1.56), 8 of 3060 116 / 109 (1.06); 6 of 690 29.8 / 34.6 (1.02), 10 of 3070 92 / 111 (0.79), 32 heads: 4 of 1950 108 / 127 (0.75)
+    // chunks. us, 32 / 16 columns, longest chain over share: 6 prompts of 3600 tokens 135 / 109 (1.35), 7 of 3140 107 / 95
+    // (1.15), 8 of 3080 102 / 95 (1.06); 6 of 690 28.4 / 34.7 (0.93), 10 of 3070 81 / 99 (0.78), 6 of 7296 197 / 218 (0.67)
     const long slabs = (a.V + 31) / 32, wide = slabs * a.H * a.ncseqs;
     const bool chain = a.longest * 256.0 > 1.05 * a.nchunks * a.H * slabs;
     if (a.V > 16 && wide >= 256 && !chain) run_chunk_scan<T, 2>(a, s);

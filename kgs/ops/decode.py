@@ -677,6 +677,21 @@ def skinny_few(x: torch.Tensor, w: PackedWeight, out: torch.Tensor | None = None
     return out
 
 
+def skinny_few_two(x: torch.Tensor, w: PackedWeight, x2: torch.Tensor, w2: PackedWeight) -> tuple[torch.Tensor, torch.Tensor]:
+    """Two plain products of :func:`skinny_few` of the same sizes and row strides in one launch."""
+    m, k = x.shape
+    for t, p in ((x, w), (x2, w2)):
+        if t.dtype != torch.bfloat16 or not t.is_cuda or tuple(t.shape) != (m, p.k) or t.stride() != (x.stride(0), 1) or t.device != x.device:
+            raise ValueError("x and x2 must be row-major bf16 GPU matrices of one shape and stride")
+        if p.n != w.n or p.k != k or p.swiglu or p.rope or not few_takes(m, p.n, k, p.fp8, True):
+            raise ValueError(f"not two products of few rows: x {tuple(t.shape)}, W [{p.n}, {p.k}]")
+    out = torch.empty((2, m, w.n), dtype=torch.bfloat16, device=x.device)
+    rc = _lib.lib().kgs_skinny_few_two(w.data.data_ptr(), x.data_ptr(), out[0].data_ptr(), w2.data.data_ptr(), x2.data_ptr(), out[1].data_ptr(),
+                                       m, w.n, k, x.stride(0), w.n, _lib.stream_handle(x.device))
+    _lib.check(rc, f"skinny_few_two[{m}x{w.n}x{k}]")
+    return out[0], out[1]
+
+
 def skinny_gemm(x: torch.Tensor, w: PackedWeight, out: torch.Tensor | None = None,
                 ksplit: int | None = None, variant: int = 0, rms: torch.Tensor | None = None,
                 resid_ss: torch.Tensor | None = None, zero: torch.Tensor | None = None,

@@ -82,6 +82,15 @@ class Projection:
             return self(x)
         return D.skinny_slabs(x, p)
 
+    def two(self, x: torch.Tensor, other: Projection, x2: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
+        """``self(x), other(x2)``: one launch where both are products of few rows of the same sizes (2048x128 twice at 1 row 3.7 us / 2.0, at 32 4.3 / 2.3)."""
+        p, q, m = self.packed, other.packed, x.shape[0]
+        if p is not None and q is not None and m <= SKINNY_MAX_ROWS and self.gated is None and other.gated is None and self.w.shape == other.w.shape and \
+                x.dtype == x2.dtype == torch.bfloat16 and x.shape == x2.shape and x.stride() == x2.stride() and x.shape[1] == self.w.shape[1] and \
+                x.stride(1) == 1 and x.stride(0) % 8 == 0 and not (x.data_ptr() % 16 or x2.data_ptr() % 16) and D.few_route(m, *self.w.shape, True):
+            return D.skinny_few_two(x, p, x2, q)
+        return self(x), other(x2)
+
     def _gated(self, x, m):
         from .gemm import gemm_gate, gemm_nt_w4x_swiglu, gemm_swiglu, swiglu_fused_ok
 

@@ -263,8 +263,7 @@ class DeltaMixer:
 
     def __call__(self, model, h: torch.Tensor, b: Batch) -> torch.Tensor:
         z = self.win(h)
-        a2 = self.a2(z[:, self.oa:self.oa + self.ra])
-        g2 = self.g2(z[:, self.og:self.og + self.rg])
+        a2, g2 = self.a2.two(z[:, self.oa:self.oa + self.ra], self.g2, z[:, self.og:self.og + self.rg])
         T.op(f"L{self.layer} delta projections")
         args = (z, self.offs, a2, self.cw, self.a_log, self.dt_bias, self.shape, model.state[self.layer], b.seqs)
         if step_takes(z, self.offs, a2, g2, self.shape, b.seqs, self.ld):

@@ -38,6 +38,10 @@ struct FewArgs {
   const int* slot;
   unsigned short* cache;
   int H, HKV;
+  // a second product of the same sizes (the grid's y), plain ones only
+  const unsigned short* x2;
+  const unsigned short* w2;
+  unsigned short* y2;
 };
 
 template <int AUX>
@@ -53,6 +57,13 @@ __global__ __launch_bounds__(64 * NW) void few(FewArgs a) {
   __shared__ float stat[OWN ? NW : 1][16];
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), fr = lane & 15, fq = lane >> 4;
   const int M = a.M, nkk = a.K / 32, nsteps = nkk / NW, kk0 = w * nsteps, nt0 = blockIdx.x * R;
+  if constexpr (!ROPE && !OWN) {
+    if (blockIdx.y) {
+      a.x = a.x2;
+      a.w = a.w2;
+      a.y = a.y2;
+    }
+  }
   const auto rw = rsrc(a.w + (long)nt0 * nkk * 512, (unsigned)(R * nkk * 1024));
   const auto rx = rsrc(a.x, (unsigned)(((M - 1) * a.ldx + a.K) * 2));
   const int wo = lane * 16;
@@ -203,29 +214,12 @@ FewSplit few_split(int M, int N, int K) {
 // Whether kgs_skinny_few runs M rows of an [N, K] weight: up to 16 rows, N a multiple of 16 and K of 512; without a norm and a rotation up to 32 rows and K of 64.
 KGS_EXPORT int kgs_skinny_few_ok(int M, int N, int K, int plain) { return few_split(M, N, K).r > 0 && (plain || (M <= 16 && K % 512 == 0)); }
 
-// y[M, N] (bf16, rows ldy apart) = x[M, K] (rows ldx apart) . W^T, W packed as for kgs_skinny_gemm_bf16. epi: EPI_SWIGLU (with
-// EPI_GELU or EPI_CLAMPED and limit; y is [M, N / 2]), EPI_RESID (y += the product), EPI_RMS (the product of x's RMSNorm: its
-// rows' statistics are made here), EPI_ROPE (as kgs_skinny_gemm_bf16_rope, with cosv .. HKV).
-KGS_EXPORT int kgs_skinny_few(const void* wp, const void* x, void* y, int M, int N, int K, long ldx, long ldy, int epi, float eps,
-                              float limit, const float* cosv, const float* sinv, const int* pos, const int* slot, void* cache,
-                              int H, int HKV, hipStream_t s) {
+namespace {
+int launch_few(const kgs::dec::FewArgs& a, const FewSplit& f, bool rope, bool own, int products, hipStream_t s) {
   using namespace kgs::dec;
-  const FewSplit f = few_split(M, N, K);
-  if (!f.r) return KGS_ERR_SHAPE;
-  const bool rope = epi & EPI_ROPE, own = epi & EPI_RMS;
-  if ((rope || own) && (M > 16 || K % 512)) return KGS_ERR_SHAPE;
-  if (ldx < K || ldy < (epi & EPI_SWIGLU ? N / 2 : N) || ldx > 1l << 25) return KGS_ERR_SHAPE;
-  if ((uintptr_t)wp % 16 || (uintptr_t)x % 16 || (uintptr_t)y % 8 || ldx % 8 || ldy % 4) return KGS_ERR_ALIGN;
-  if (epi & ~(EPI_SWIGLU | EPI_GELU | EPI_CLAMPED | EPI_RMS | EPI_RESID | EPI_ROPE)) return KGS_ERR_ARG;
-  if (((epi & EPI_SWIGLU) != 0) + ((epi & EPI_RESID) != 0) + rope > 1) return KGS_ERR_ARG;
-  if (rope) {
-    if (H <= 0 || HKV <= 0 || H % HKV || N != (H + 2 * HKV) * HD) return KGS_ERR_SHAPE;
-    if (!cosv || !sinv || !pos || !slot || !cache || (uintptr_t)cache % 16) return KGS_ERR_ARG;
-  }
-  const FewArgs a{(const unsigned short*)x, (const unsigned short*)wp, (unsigned short*)y, M, N, K, (int)ldx, ldy, epi, 1.f / K, eps, limit,
-                  cosv, sinv, pos, slot, (unsigned short*)cache, H, HKV};
+  const int M = a.M, N = a.N, K = a.K;
   auto run = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, dim3(N / (16 * f.r)), dim3(64 * f.nw), 0, s, a);
+    hipLaunchKernelGGL(kernel, dim3(N / (16 * f.r), products), dim3(64 * f.nw), 0, s, a);
     return (int)hipGetLastError();
   };
   auto pick = [&](auto ro, auto ow) {
@@ -248,4 +242,44 @@ KGS_EXPORT int kgs_skinny_few(const void* wp, const void* x, void* y, int M, int
                                                                              : odd(mt, std::integral_constant<int, 2>{});
   };
   return M <= 16 ? waves(std::integral_constant<int, 1>{}) : waves(std::integral_constant<int, 2>{});
+}
+}  // namespace
+
+// y[M, N] (bf16, rows ldy apart) = x[M, K] (rows ldx apart) . W^T, W packed as for kgs_skinny_gemm_bf16. epi: EPI_SWIGLU (with
+// EPI_GELU or EPI_CLAMPED and limit; y is [M, N / 2]), EPI_RESID (y += the product), EPI_RMS (the product of x's RMSNorm: its
+// rows' statistics are made here), EPI_ROPE (as kgs_skinny_gemm_bf16_rope, with cosv .. HKV).
+KGS_EXPORT int kgs_skinny_few(const void* wp, const void* x, void* y, int M, int N, int K, long ldx, long ldy, int epi, float eps,
+                              float limit, const float* cosv, const float* sinv, const int* pos, const int* slot, void* cache,
+                              int H, int HKV, hipStream_t s) {
+  using namespace kgs::dec;
+  const FewSplit f = few_split(M, N, K);
+  if (!f.r) return KGS_ERR_SHAPE;
+  const bool rope = epi & EPI_ROPE, own = epi & EPI_RMS;
+  if ((rope || own) && (M > 16 || K % 512)) return KGS_ERR_SHAPE;
+  if (ldx < K || ldy < (epi & EPI_SWIGLU ? N / 2 : N) || ldx > 1l << 25) return KGS_ERR_SHAPE;
+  if ((uintptr_t)wp % 16 || (uintptr_t)x % 16 || (uintptr_t)y % 8 || ldx % 8 || ldy % 4) return KGS_ERR_ALIGN;
+  if (epi & ~(EPI_SWIGLU | EPI_GELU | EPI_CLAMPED | EPI_RMS | EPI_RESID | EPI_ROPE)) return KGS_ERR_ARG;
+  if (((epi & EPI_SWIGLU) != 0) + ((epi & EPI_RESID) != 0) + rope > 1) return KGS_ERR_ARG;
+  if (rope) {
+    if (H <= 0 || HKV <= 0 || H % HKV || N != (H + 2 * HKV) * HD) return KGS_ERR_SHAPE;
+    if (!cosv || !sinv || !pos || !slot || !cache || (uintptr_t)cache % 16) return KGS_ERR_ARG;
+  }
+  const FewArgs a{(const unsigned short*)x, (const unsigned short*)wp, (unsigned short*)y, M, N, K, (int)ldx, ldy, epi, 1.f / K, eps, limit,
+                  cosv, sinv, pos, slot, (unsigned short*)cache, H, HKV};
+  return launch_few(a, f, rope, own, 1, s);
+}
+
+// y = x . W^T and y2 = x2 . W2^T in one launch: sizes and strides shared, as kgs_skinny_few with epi 0.
+KGS_EXPORT int kgs_skinny_few_two(const void* wp, const void* x, void* y, const void* wp2, const void* x2, void* y2, int M, int N, int K,
+                                  long ldx, long ldy, hipStream_t s) {
+  using namespace kgs::dec;
+  const FewSplit f = few_split(M, N, K);
+  if (!f.r || ldx < K || ldy < N || ldx > 1l << 25) return KGS_ERR_SHAPE;
+  if (((uintptr_t)wp | (uintptr_t)x | (uintptr_t)wp2 | (uintptr_t)x2) % 16 || ((uintptr_t)y | (uintptr_t)y2) % 8 || ldx % 8 || ldy % 4)
+    return KGS_ERR_ALIGN;
+  FewArgs a{(const unsigned short*)x, (const unsigned short*)wp, (unsigned short*)y, M, N, K, (int)ldx, ldy};
+  a.x2 = (const unsigned short*)x2;
+  a.w2 = (const unsigned short*)wp2;
+  a.y2 = (unsigned short*)y2;
+  return launch_few(a, f, false, false, 2, s);
 }

@@ -166,3 +166,14 @@ def test_projections_by_the_packed_weight(n, k, gated, m):
     assert got.shape == ref.shape
     # some routes round gate and up to bf16 before the product
     assert bool(((got.double() - ref).abs() <= 2.0 ** -7 * ref.abs() + 2.0 ** -7 * (ref.abs().max() if gated else 0) + 1e-4 * ref.abs().max()).all())
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 16, 64), (16, 2048, 128), (7, 4128, 1024), (24, 2048, 192), (32, 48, 512)])
+def test_two_products(m, n, k):
+    """One launch's bits are two launches', of operands that are columns of a wider matrix."""
+    z, (_, w), (_, w2) = torch.randn(m, 2 * k + 8, device="cuda").bfloat16(), _operands(m, n, k), _operands(m, n, k, 1)
+    x, x2, pw, pw2 = z[:, :k], z[:, k + 8:], D.PackedWeight(w), D.PackedWeight(w2)
+    got, got2 = D.skinny_few_two(x, pw, x2, pw2)
+    assert torch.equal(got, D.skinny_few(x, pw)) and torch.equal(got2, D.skinny_few(x2, pw2))
+    with pytest.raises(ValueError):
+        D.skinny_few_two(x, pw, torch.empty(m, k, device="cuda", dtype=torch.bfloat16), pw2)

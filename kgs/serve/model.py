@@ -803,7 +803,7 @@ class ServingModel:
         """As :meth:`_fused_layers`, for 33 to 96 rows: products in K slices that the rotation and the residual adds sum, gate and up whole. The
         rows' bits depend on nothing but their own inputs. ``(x, y, ss)``: the residual rows, from 49 rows on their norm for the head
         (else None) and else their sums of squares. Four layers 4096 wide, us a step by four-wave tiles (up to 48 rows skinny) / so: one prompt of 90
-        tokens 596 / 563, of 60 615 / 528, two of 36 in all 611 / 496; 2048 wide one of 60 401 / 362."""
+        tokens 599 / 540, of 60 615 / 509, two of 36 in all 611 / 494; 2048 wide one of 60 397 / 387."""
         from kgs.ops.transformer import embed_rows, embeds, splitk_add_rmsnorm, splitk_add_squares
 
         c = self.cfg

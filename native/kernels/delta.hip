@@ -622,14 +622,15 @@ __global__ __launch_bounds__(256, 4) void chunk_prep(Args a) {
 // moving; the A operands are read as float4s in that order. The waves' partial
 // products over their rows meet in LDS, one barrier per chunk.
 // A sequence's chunks are a serial chain, W S, its sum over the waves, K U, so what is not on it is shared or kept out of its way: TV
-// enters the sum a quarter a wave, P U a wave's part of O, whose sum is stored a chunk later, a row in four a wave; and the next operands
+// is loaded a quarter a wave, P U enters a wave's part of O a quarter each, whose sum is stored a chunk later, a row in four a wave; and the next operands
 // are sent for in two parts, W and Q under the barrier's wait. us, one wave a chunk for O and all loads at the chunk's end / so, 16 heads: one
-// sequence of 1216 tokens 89 / 67, six of 3600 116 / 108, six of 1216 each 215 / 200. Bound by that chain's latencies (0.83 us a chunk alone), then by
+// sequence of 1216 tokens 89 / 67, six of 3600 116 / 108, six of 1216 each 213 / 212 (NS 2). Bound by that chain's latencies (0.83 us a chunk alone), then by
 // the operands' way into the CUs (27 KB a chunk and workgroup). A fifth wave for TV and O: 80, 127 and 280 us; three waves a SIMD by a shorter ring: 69, 113, 277.
 // NS 2 reads the A operands half as often; NS 1 spreads few heads over more CUs.
 template <typename T, int MT, int NS>
 __global__ __launch_bounds__(256) void chunk_scan(Args a) {
   __shared__ f32x4 part[2][2][NS][4][64];  // [buffer][U | O][tile][wave][lane]
+  __shared__ f32x4 tv[2][NS][64];          // T V: [buffer][tile][lane], a row in four from each wave
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l16 = lane & 15, g = lane >> 4;
   const int KP = a.KP, V = a.V, H = a.H, nslab = (V + 16 * NS - 1) / (16 * NS), ntile = KP / 16;
@@ -717,9 +718,8 @@ __global__ __launch_bounds__(256) void chunk_scan(Args a) {
     f32x4 pu[NS], po[NS];
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
-      po[s] = f32x4{};
-#pragma unroll
-      for (int r = 0; r < 4; ++r) pu[s][r] = w == r ? -f.U[s] : 0.f;
+      pu[s] = po[s] = f32x4{};
+      ((float*)&tv[c & 1][s][lane])[w] = f.U[s];
     }
 #pragma unroll
     for (int m = 0; m < MT; ++m)
@@ -740,7 +740,7 @@ __global__ __launch_bounds__(256) void chunk_scan(Args a) {
     f32x4 U[NS];
 #pragma unroll
     for (int s = 0; s < NS; ++s)
-      U[s] = -(part[buf][0][s][0][lane] + part[buf][0][s][1][lane] + part[buf][0][s][2][lane] + part[buf][0][s][3][lane]);
+      U[s] = tv[buf][s][lane] - (part[buf][0][s][0][lane] + part[buf][0][s][1][lane] + part[buf][0][s][2][lane] + part[buf][0][s][3][lane]);
 #pragma unroll
     for (int m = 0; m < MT; ++m)
 #pragma unroll
@@ -1044,7 +1044,7 @@ static hipError_t run(const Args& a, hipStream_t s) {
     // Slabs of 32 columns read the chunks' operands half as often; of 16 they halve a chain's step, which is what counts where
     // there are few workgroups or the longest chain (a.longest chunks, 0: unknown) is above a CU's mean share of all
     // chunks. us, 32 / 16 columns, longest chain over share: 6 prompts of 3600 tokens 135 / 109 (1.35), 7 of 3140 107 / 95
-    // (1.15), 8 of 3080 102 / 95 (1.06); 6 of 690 28.4 / 34.7 (0.93), 10 of 3070 81 / 99 (0.78), 6 of 7296 197 / 218 (0.67)
+    // (1.15), 8 of 3080 102 / 95 (1.06); 6 of 690 28.4 / 34.7 (0.93), 10 of 3070 81 / 99 (0.78), 6 of 7296 212 / 218 (0.67)
     const long slabs = (a.V + 31) / 32, wide = slabs * a.H * a.ncseqs;
     const bool chain = a.longest * 256.0 > 1.05 * a.nchunks * a.H * slabs;
     if (a.V > 16 && wide >= 256 && !chain) run_chunk_scan<T, 2>(a, s);

@@ -634,7 +634,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 // gemm_tr and their bits. Layers of up to about a thousand rows are bound by the launches (some 4 us of host time each), and leave CUs
 // idle in either product. us, a training step by two launches / one: 64 rows, three layers, 512 - 2048 - 512 216 / 204;
 // 256 rows, three of 1024 219 / 202; 777 rows 768 - 3072 - 768 230 / 214; 1024 rows, two layers, 1024 - 4096 - 1024 186 / 175; from 2048 rows the
-// same time (2048 - 5504 - 2048 393 / 394).
+// same time, and large grids go one by one (gemm_tr_pair below).
 template <bool SPLIT0, bool SPLIT1>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_tr_pair(TrArgs x, TrArgs w, int wgx) {
   __shared__ __attribute__((aligned(1024))) char smem[2 * 32768];
@@ -1030,7 +1030,12 @@ int gemm_tr_pair(const void* dY, const void* W, const void* X, void* dX, void* d
   unsigned gx, gw;
   const TrArgs x = tr_args(dY, W, dX, m, k, n, ldy, ldw, k, nsx, wsx, gx), w = tr_args(dY, X, dW, n, k, m, ldy, ldx, k, nsw, wsw, gw);
   if ((nsx > 1 && !wsx) || (nsw > 1 && !wsw)) return KGS_ERR_ARG;
-  if ((long)gx + gw > 0x7fffffffL) return KGS_ERR_SHAPE;
+  // Two rounds of two workgroups a CU: beyond, neither launch leaves CUs idle for long and the mixed one loses (us, two launches / one: 1500
+  // rows, three layers of 2048, 448 tiles each, 266 / 229; 3000 rows, 1536 - 6144 - 1536, up to 1728 tiles, 540 / 544)
+  if ((long)gx + gw > 4L * cu_count()) {
+    const int rc = gemm_tr(dY, W, dX, m, k, n, ldy, ldw, k, 0, 1, nsx, wsx, s);
+    return rc ? rc : gemm_tr(dY, X, dW, n, k, m, ldy, ldx, k, 1, 1, nsw, wsw, s);
+  }
   const dim3 grid(gx + gw);
   if (nsx > 1 && nsw > 1) hipLaunchKernelGGL((any::gemm_tr_pair<true, true>), grid, dim3(256), 0, s, x, w, (int)gx);
   else if (nsx > 1) hipLaunchKernelGGL((any::gemm_tr_pair<true, false>), grid, dim3(256), 0, s, x, w, (int)gx);

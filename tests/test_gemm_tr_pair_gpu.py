@@ -10,9 +10,10 @@ def rnd(*s):
     return torch.randn(*s, device="cuda").bfloat16()
 
 
-# m, n, k, slices of dX and dW: one tile each, remainders of rows, columns and sums, odd columns out, more slices than chunks of 128
+# m, n, k, slices of dX and dW: one tile each, remainders of rows, columns and sums, odd columns out, more slices than chunks of 128,
+# more tiles than one launch takes
 @pytest.mark.parametrize("m,n,k,nsx,nsw", [(128, 128, 128, 1, 1), (1, 8, 8, 1, 1), (130, 520, 264, 1, 1), (64, 2048, 512, 4, 1),
-                                           (1001, 136, 392, 1, 3), (600, 1000, 129, 2, 4), (257, 384, 515, 64, 64)])
+                                           (1001, 136, 392, 1, 3), (600, 1000, 129, 2, 4), (257, 384, 515, 64, 64), (2056, 4096, 4104, 1, 1)])
 def test_bits_of_two_launches(m, n, k, nsx, nsw):
     from kgs.ops import _lib
 

@@ -208,10 +208,16 @@ __global__ __launch_bounds__(256, (MT * KC_ > 32 || R * MT >= 16) ? 1 : 2) void 
   // chunk: a few redundant L2-hit reloads at the tail) so hipcc can count
   // vmcnt through the loop instead of draining the ring before each MFMA.
   WFrag<W8> wf[PF][R];
+  // OWN, KIN: the k-steps' order is fixed, else the compiler gives up the ring for the statistic's sake (84 registers instead of 167, every load in
+  // flight waited for several times a chunk). us at 24 rows, given statistics / own, loose /
+  // own, fixed: 8192x2048 11.7 / 15.5 / 10.9, 3072x2048 7.9 / 9.6 / 8.5.
+  constexpr bool PINNED = OWN && KIN && MT <= 2;
+  if constexpr (!PINNED) {
 #pragma unroll
-  for (int p = 0; p < PF; ++p)
+    for (int p = 0; p < PF; ++p)
 #pragma unroll
-    for (int r = 0; r < R; ++r) wf[p][r] = __builtin_nontemporal_load(wrow[r] + (long)min(p, nsteps - 1) * 64);
+      for (int r = 0; r < R; ++r) wf[p][r] = __builtin_nontemporal_load(wrow[r] + (long)min(p, nsteps - 1) * 64);
+  }
 
   if constexpr (SUMS) {
     if ((ep.mode & EPI_RMS) && tid < M) {
@@ -245,9 +251,15 @@ __global__ __launch_bounds__(256, (MT * KC_ > 32 || R * MT >= 16) ? 1 : 2) void 
       for (int c = 0; c < MT; ++c) xr[c] = x + (long)min(16 * c + (lane & 15), M - 1) * ldx + (long)kk0 * 32 + 8 * (lane >> 4);
       bf16x8 xf[PF][MT];
 #pragma unroll
-      for (int p = 0; p < PF; ++p)
+      for (int p = 0; p < PF; ++p) {
+        if constexpr (PINNED) {
+#pragma unroll
+          for (int r = 0; r < R; ++r) wf[p][r] = __builtin_nontemporal_load(wrow[r] + p * 64);
+        }
 #pragma unroll
         for (int c = 0; c < MT; ++c) xf[p][c] = *(const bf16x8*)(xr[c] + p * 32);
+        if constexpr (PINNED) __builtin_amdgcn_sched_barrier(0);
+      }
       for (int s0 = 0; s0 < nsteps; s0 += PF) {
 #pragma unroll
         for (int p = 0; p < PF; ++p) {
@@ -268,6 +280,7 @@ __global__ __launch_bounds__(256, (MT * KC_ > 32 || R * MT >= 16) ? 1 : 2) void 
           for (int r = 0; r < R; ++r) wf[p][r] = __builtin_nontemporal_load(wrow[r] + (long)sn * 64);
 #pragma unroll
           for (int c = 0; c < MT; ++c) xf[p][c] = *(const bf16x8*)(xr[c] + sn * 32);
+          if constexpr (PINNED) __builtin_amdgcn_sched_barrier(0);
         }
       }
     }

@@ -507,3 +507,21 @@ def test_paged_and_lightning_kernels_do_not_spill(tmp_path):
             assert r["VGPRs Spill"] == 0 and r["SGPRs Spill"] == 0, (name, r)
             if "6chunksILi4ELi8ELb1EE" in name:
                 assert r["VGPRs"] <= 128 and 2 * r["LDS Size"] <= 160 * 1024, r
+
+
+def test_own_statistics_keep_the_ring_of_loads(builds):
+    """The skinny products with K split over a workgroup's waves wait for one k-step of their ring at a time also where they make the norm's
+    statistics: at every wait of the loop more than a third of the ring's loads stay in flight."""
+    asm, seen = builds["decode.hip"].result()[1], set()
+    for name, body in re.findall(r"^(_ZN3kgs3dec6skinny\S+):[^\n]*\n(.*?)s_endpgm", asm, re.S | re.M):
+        m = re.match(r"_ZN3kgs3dec6skinnyILi(\d)ELi([12])ELi8ELb0ELb[01]ELb1ELb0ELb1E", name)
+        if not m:
+            continue
+        r, mt = int(m[1]), int(m[2])
+        parts = re.split(r"^(\.LBB\w+):", body, flags=re.M)
+        loops = [p for label, p in zip(parts[1::2], parts[2::2]) if p.count("v_mfma") >= 8 * r * mt and re.search(rf"s_cbranch\w+ {re.escape(label)}\b", p)]
+        assert loops, name
+        waits = [int(v) for p in loops for v in re.findall(r"s_waitcnt vmcnt\((\d+)\)", p)]
+        assert waits and min(waits) > 8 * (r + mt) // 3, (name, waits)
+        seen.add((r, mt))
+    assert seen == {(1, 1), (2, 1), (1, 2), (2, 2)}

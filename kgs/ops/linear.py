@@ -40,7 +40,7 @@ class Projection:
             raise ValueError(f"x {tuple(x.shape)} {x.dtype} does not fit w {tuple(w.shape)} {w.dtype}")
         m, (n, k) = x.shape[0], w.shape
         if x.dtype == torch.bfloat16:
-            if m <= D.SLAB_ROWS and self.packed is not None and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0:
+            if m <= D.SLAB_ROWS and self._reads(x):
                 y = self._packed(x, m, n, k)
                 if y is not None:
                     return y
@@ -61,6 +61,12 @@ class Projection:
 
         return act_mul(y, act)
 
+    def _reads(self, x) -> bool:
+        """Whether the kernels that read the packed weight can read ``x``: rows of 16-byte loads, not over one another, whose offsets fit 32 bits."""
+        ld = x.stride(0)
+        return self.packed is not None and x.is_cuda and x.dtype == torch.bfloat16 and x.stride(1) == 1 and x.shape[1] <= ld <= 1 << 23 and \
+            ld % 8 == 0 and x.data_ptr() % 16 == 0
+
     def _packed(self, x, m, n, k):
         """The product by a kernel that reads the packed weight, or None. Up to 32 rows that of few rows or :func:`kgs.ops.decode.skinny_gemm` -- a gate and up of
         one round of 64-row strips by :func:`kgs.ops.decode.skinny_rows` from 17 rows on (16384x2048 at 32 rows 16.1 us / 14.5) --, from
@@ -75,19 +81,17 @@ class Projection:
 
     def partials(self, x: torch.Tensor) -> torch.Tensor:
         """:meth:`__call__`, or where the product of a decode batch runs in K slices those, fp32 ``[slices, M, N]``, for a consumer
-        that adds them and rounds to bf16. One slice is stored as such (its sum is no work), and rows that 16-byte loads cannot read go the other way."""
+        that adds them and rounds to bf16. One slice is stored as such (its sum is no work), and rows that the kernel cannot read go the other way."""
         p = self.packed
-        if p is None or self.gated is not None or x.dtype != torch.bfloat16 or x.stride(0) % 8 or x.data_ptr() % 16 or \
-                D.slab_split(x.shape[0], p.n, p.k) is None:
+        if self.gated is not None or x.shape[1] != self.w.shape[1] or not self._reads(x) or D.slab_split(x.shape[0], p.n, p.k) is None:
             return self(x)
         return D.skinny_slabs(x, p)
 
     def two(self, x: torch.Tensor, other: Projection, x2: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
         """``self(x), other(x2)``: one launch where both are products of few rows of the same sizes (2048x128 twice at 1 row 3.7 us / 2.0, at 32 4.3 / 2.3)."""
         p, q, m = self.packed, other.packed, x.shape[0]
-        if p is not None and q is not None and m <= SKINNY_MAX_ROWS and self.gated is None and other.gated is None and self.w.shape == other.w.shape and \
-                x.dtype == x2.dtype == torch.bfloat16 and x.shape == x2.shape and x.stride() == x2.stride() and x.shape[1] == self.w.shape[1] and \
-                x.stride(1) == 1 and x.stride(0) % 8 == 0 and not (x.data_ptr() % 16 or x2.data_ptr() % 16) and D.few_route(m, *self.w.shape, True):
+        if m <= SKINNY_MAX_ROWS and self.gated is None and other.gated is None and self.w.shape == other.w.shape and x.shape == x2.shape and \
+                x.stride() == x2.stride() and x.shape[1] == self.w.shape[1] and self._reads(x) and other._reads(x2) and D.few_route(m, *self.w.shape, True):
             return D.skinny_few_two(x, p, x2, q)
         return self(x), other(x2)
 

@@ -177,3 +177,27 @@ def test_two_products(m, n, k):
     assert torch.equal(got, D.skinny_few(x, pw)) and torch.equal(got2, D.skinny_few(x2, pw2))
     with pytest.raises(ValueError):
         D.skinny_few_two(x, pw, torch.empty(m, k, device="cuda", dtype=torch.bfloat16), pw2)
+
+
+@pytest.mark.parametrize("n,k,gated", ((2048, 768, False), (24576, 512, False), (256, 512, False), (16384, 1024, True)))
+@pytest.mark.parametrize("m", (1, 8, 32, 40))
+def test_projections_of_rows_that_the_packed_kernels_cannot_read(n, k, gated, m):
+    """Columns, odd addresses and, of plain weights, one row repeated or rows that overlap go where any matrix goes, in each of the ways in."""
+    from kgs.ops.linear import Projection
+
+    g = torch.Generator(device="cuda").manual_seed(m)
+    z, (_, w) = torch.randn(m + 1, k + 8, generator=g, device="cuda").bfloat16(), _operands(m, n, k, 9)
+    p, q = Projection(w, "silu" if gated else None), Projection(w, "silu" if gated else None)
+    rows = z[:m, :k]
+    spread = torch.empty(m, 2 * k, device="cuda", dtype=torch.bfloat16)[:, ::2].copy_(rows)
+    over = () if gated else (rows[:1].expand(m, k), z.flatten().as_strided((m, k), (8, 1)))
+    for x in (rows.t().contiguous().t(), spread, z[:m, 1:k + 1], *over):
+        ref = x.double() @ w.double().T
+        if gated:
+            a, b = ref.chunk(2, 1)
+            ref = torch.nn.functional.silu(a) * b
+        for got in (p(x), *p.two(x, q, x), p.partials(x)):
+            # one rounding to bf16 and fp32 sums; of a gate with its factors rounded before
+            tol = 2.0 ** -7 * ref.abs() + 2.0 ** -7 * (ref.abs().max() if gated else 0) + 1e-4 * ref.abs().max()
+            got = got.sum(0) if got.dim() == 3 else got
+            assert got.shape == ref.shape and bool(((got.double() - ref).abs() <= tol).all())

@@ -773,9 +773,10 @@ class ServingModel:
         return all(D.own_takes(r, w.n, w.k, w.fp8, bool(w.rope)) for w, r in ((P["qkv"], m), (P["gate_up"], m), (self.packed_lm, head)))
 
     def _slabs(self, m: int) -> bool:
-        """Whether ``m`` rows take the layers of :meth:`_slab_layers`: 33 to 96 of bf16 weights and pages, where the products tile."""
+        """Whether ``m`` rows take the layers of :meth:`_slab_layers`: 33 to 96 of bf16 weights and pages, where the products tile. A
+        ``fused_max_batch`` of 32 and less leaves all rows above it to the split tiles."""
         if self.packed is None or self.decode_fp8 or self.backend != "kgs" or not self.fuse_splitk or self.rope_attn or \
-                not self.fused_max_batch or not 32 < m <= D.SLAB_ROWS:
+                not 32 < min(m, self.fused_max_batch) or m > D.SLAB_ROWS:
             return False
         P, c = self.packed[0], self.cfg
         return c.hidden % 2048 == 0 and c.hidden <= 8192 and bool(P["qkv"].rope) and \

@@ -77,6 +77,22 @@ def test_prompt_rows_of_the_fused_layer(most, rows, fused):
     assert ServingModel._fused_prompts(M, rows, 1) is fused
 
 
+@pytest.mark.parametrize("most,rows,slabs", [(48, 33, True), (48, 96, True), (48, 97, False), (48, 32, False), (33, 64, True), (32, 33, False), (16, 40, False),
+                                             (16, 96, False), (0, 64, False)])
+def test_rows_of_the_layers_in_slices(most, rows, slabs):
+    """fused_max_batch bounds these layers too: where the caller wants few rows on packed weights, larger steps take the split tiles."""
+    from types import SimpleNamespace
+
+    from kgs.serve.model import ServingModel
+
+    class M:
+        decode_fp8, backend, fuse_splitk, rope_attn, fused_max_batch = False, "kgs", True, False, most
+        packed = [{"qkv": _Weight(3072, 2048, rope=(16, 4)), "o": _Weight(2048, 2048), "gate_up": _Weight(16384, 2048), "down": _Weight(2048, 8192)}]
+        packed_lm, cfg = _Weight(1024, 2048), SimpleNamespace(hidden=2048)
+
+    assert ServingModel._slabs(M, rows) is slabs
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("m,v", [(17, 22), (32, 22), (24, 23), (33, 24), (64, 24), (40, 25)])
 def test_k_split_in_the_workgroup(m, v):

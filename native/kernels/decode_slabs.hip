@@ -177,9 +177,9 @@ int launch_slabs(const kgs::dec::SlabArgs& a, int r, hipStream_t s) {
 }
 
 int slab_shape(const void* wp, const void* x, const void* y, int M, int N, int K, long ldx, int r, int ns) {
-  if (M < 1 || M > SLAB_ROWS || N <= 0 || K <= 0 || (r != 1 && r != 2) || ns < 1 || N % (64 * r) || K % (128 * ns) || (long)N * K > (1l << 31))
+  if (M < 1 || M > SLAB_ROWS || N <= 0 || K <= 0 || (r != 1 && r != 2) || ns < 1 || N % (64 * r) || K % (128 * ns))
     return KGS_ERR_SHAPE;
-  if (ldx < K || ldx > 1l << 23) return KGS_ERR_SHAPE;
+  if (ldx < K || ldx > 1l << 23) return KGS_ERR_SHAPE;  // 32-bit offsets: x's 96 rows, and a wave's 32 rows of W, whose base has 64 bits
   return (uintptr_t)wp % 16 || (uintptr_t)x % 16 || (uintptr_t)y % 16 || ldx % 8 ? KGS_ERR_ALIGN : 0;
 }
 }  // namespace

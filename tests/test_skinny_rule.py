@@ -93,6 +93,23 @@ def test_rows_of_the_layers_in_slices(most, rows, slabs):
     assert ServingModel._slabs(M, rows) is slabs
 
 
+def test_what_the_rules_of_slices_take_the_kernel_takes():
+    """Addresses off 16 bytes are refused after the sizes and before any launch, so the entries tell here whether they take the sizes."""
+    from kgs.ops import _lib
+
+    lib = _lib.lib()
+    align = lib.kgs_skinny_slabs(1, 1, 1, 1, 64, 128, 128, 1, 1, None)
+    assert align not in (0, lib.kgs_skinny_slabs(1, 1, 1, 97, 64, 128, 128, 1, 1, None))
+    for n in (64, 128, 192, 2048, 4096, 4160, 28672, 128256, 256000, 262208, 1 << 20):
+        for k in (128, 256, 384, 2048, 4096, 8192, 12288, 14336, 16384, 65536):
+            for m in (1, 16, 17, 32, 33, 64, 65, 96):
+                split, tiles = D.slab_split(m, n, k), D.slab_rows_tiles(m, n, k)
+                if split:
+                    assert lib.kgs_skinny_slabs(1, 1, 1, m, n, k, k, *split, None) == align, (m, n, k)
+                if tiles:
+                    assert lib.kgs_skinny_rows(1, 1, 1, m, n, k, k, n, tiles, 0, None, 0.0, 0.0, None) == align, (m, n, k)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("m,v", [(17, 22), (32, 22), (24, 23), (33, 24), (64, 24), (40, 25)])
 def test_k_split_in_the_workgroup(m, v):

@@ -63,6 +63,22 @@ def test_whole_products_and_gates(n, k, m):
     close(D.skinny_rows(x, D.PackedWeight(w, swiglu=True, act="gelu_tanh"), sq, 1e-3), torch.nn.functional.gelu(g, approximate="tanh") * u, 4)
 
 
+def test_weights_of_more_than_31_bits_of_values():
+    """An LM head of 2.15e9 values: its first, middle and last strips."""
+    from kgs.ops.linear import Projection
+
+    m, n, k = 33, 131200, 16384
+    x, w = _operands(m, 128, k, 3)
+    wide = w.repeat(n // 128, 1)
+    wide[-1] *= 2
+    ref = (x.double() @ w.double().T).repeat(1, n // 128)
+    ref[:, -1] *= 2
+    p = Projection(wide)
+    assert n * k > 1 << 31 and D.slab_rows_tiles(m, n, k) == 2
+    for got in (D.skinny_rows(x, p.packed), p(x)):
+        assert bool(((got.double() - ref).abs() <= 2.0 ** -8 * ref.abs() + 2e-5 * ref.abs().max()).all())
+
+
 @pytest.mark.parametrize("heads,kv,k", ((32, 8, 4096), (16, 4, 2048), (8, 1, 128), (2, 1, 1024)))  # 4, 4, 1 and 4 slices
 @pytest.mark.parametrize("m", (33, 96))
 def test_rotation_of_slices_as_of_the_whole_product(heads, kv, k, m):

@@ -752,7 +752,7 @@ def skinny_gemm(x: torch.Tensor, w: PackedWeight, out: torch.Tensor | None = Non
             raise ValueError("resid_ss needs the residual stream as out [M, N] (and no swiglu)")
     if out is None:
         out = torch.empty((m, w.n_out), dtype=torch.bfloat16, device=x.device)
-    need = ks * mpad * (w.n + (w.n // rps if norm else 0)) if ks > 1 else 0
+    need = ks * mpad * (w.n + (2 * (w.n // rps) if norm else 0)) if ks > 1 else 0
     if counters is None:
         ws, cnt = _workspace(x.device, need, w.n // rps)
     else:

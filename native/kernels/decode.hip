@@ -97,9 +97,9 @@ __device__ __forceinline__ bf16x8 dequant8(u32x2 v, float s) {
 // first weights' way from memory, and a workgroup's tiles are summed in LDS before they are added (with each
 // tile's atomics and each output's conversion 1.2 us more a launch). us at 30 rows, floats / exact sums:
 // 28672x4096 43.4 / 43.6, 4096x14336 29.5 / 29.1, 4096x4096 16.9 / 16.5.
-// OWN (EPI_OWN; bf16 weights, batch <= 64): EPI_RMS by statistics that the workgroup makes itself, an
-// MFMA of x with itself per k-step, whose diagonal the rows' sums of squares are (decode_few.hip has the reason). KIN: each
-// wave of its K quarter; else wave c of column tile c, and with cross-workgroup split-K (not KIN) the splits' sums go behind their slabs.
+// OWN (EPI_OWN; bf16 weights, batch <= 64): EPI_RMS by statistics that the workgroup makes itself from the operands as they pass
+// (add_squares; decode_few.hip has the reason). KIN: each wave of its K quarter; else wave c of column tile c, and with cross-workgroup
+// split-K (not KIN) the splits' sums go behind their slabs.
 template <int R, int MT, int KC_, bool W8 = false, bool EROPE = false, bool KIN = false, bool SUMS = false, bool OWN = false>
 __global__ __launch_bounds__(256, (MT * KC_ > 32 || R * MT >= 16) ? 1 : 2) void skinny(const void* __restrict__ wpv, const unsigned short* __restrict__ x,
                                                  unsigned short* __restrict__ y, float* __restrict__ ws,
@@ -117,7 +117,8 @@ __global__ __launch_bounds__(256, (MT * KC_ > 32 || R * MT >= 16) ? 1 : 2) void 
   // arriver" flag reuses its first word after the main loop
   static_assert(!KIN || PF == KC, "KIN: one ring round per chunk");
   __shared__ __attribute__((aligned(16))) bf16x8 xs[2][KIN ? 2 * R * MT * 64 : C::CHUNK_SLOTS];
-  __shared__ float stat[SUMS || OWN ? 5 : 1][16 * MT];  // SUMS: the rows' scales; a wave's sums of squares in [1 + wave]. OWN: a wave's (KIN), the rows'
+  // SUMS: the rows' scales; a wave's sums of squares in [1 + wave]. OWN: a wave's (KIN), the rows'
+  __shared__ typename std::conditional<OWN, double, float>::type stat[SUMS ? 5 : OWN && KIN ? 4 : 1][16 * MT];
 
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int nstrip = N / ((KIN ? 16 : 64) * R);
@@ -194,23 +195,16 @@ __global__ __launch_bounds__(256, (MT * KC_ > 32 || R * MT >= 16) ? 1 : 2) void 
 #pragma unroll
     for (int c = 0; c < MT; ++c) acc[r][c] = f32x4v{0.f, 0.f, 0.f, 0.f};
 
-  f32x4v gram[OWN && KIN ? MT : 1];  // OWN: x . x^T of the column tiles (KIN), of the wave's own
-#pragma unroll
-  for (int c = 0; c < (OWN && KIN ? MT : 1); ++c) gram[c] = f32x4v{0.f, 0.f, 0.f, 0.f};
-  // its diagonal: row m in lane 16 (m / 4) + m, element m % 4
-  [[maybe_unused]] auto diagonal = [&](const f32x4v& d, float* to) {
-    const int m = lane & 15;
-    const float lo = m & 1 ? d[1] : d[0], hi = m & 1 ? d[3] : d[2];
-    if (lane >> 4 == m >> 2) to[m] = m & 2 ? hi : lo;
-  };
+  [[maybe_unused]] double own[OWN && KIN ? MT : 1] = {};  // OWN: this lane's part of its rows' sums of squares, of all column tiles (KIN) or the wave's own
 
   // Every load below is unconditional (indices clamped to the last step /
   // chunk: a few redundant L2-hit reloads at the tail) so hipcc can count
   // vmcnt through the loop instead of draining the ring before each MFMA.
   WFrag<W8> wf[PF][R];
   // OWN, KIN: the k-steps' order is fixed, else the compiler gives up the ring for the statistic's sake (84 registers instead of 167, every load in
-  // flight waited for several times a chunk). us at 24 rows, given statistics / own, loose /
-  // own, fixed: 8192x2048 11.7 / 15.5 / 10.9, 3072x2048 7.9 / 9.6 / 8.5.
+  // flight waited for several times a chunk). us at 24 rows, given statistics / own, loose / own, fixed: 8192x2048 11.7 / 15.5 / 10.9, 3072x2048
+  // 7.9 / 9.6 / 8.5, there with MFMAs of x with itself for the statistic; fixed with those / add_squares in one run 10.4 / 10.4, 7.9 / 7.6, two column
+  // tiles of 6144x4096 18.9 / 19.9, four of 3072x2048 at 64 rows 12.3 / 12.7.
   constexpr bool PINNED = OWN && KIN && MT <= 2;
   if constexpr (!PINNED) {
 #pragma unroll
@@ -273,7 +267,7 @@ __global__ __launch_bounds__(256, (MT * KC_ > 32 || R * MT >= 16) ? 1 : 2) void 
           }
           if constexpr (OWN) {
 #pragma unroll
-            for (int c = 0; c < MT; ++c) gram[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xf[p][c], xf[p][c], gram[c], 0, 0, 0);
+            for (int c = 0; c < MT; ++c) own[c] = add_squares(own[c], xf[p][c]);
           }
           const int sn = min(s0 + p + PF, nsteps - 1);
 #pragma unroll
@@ -289,7 +283,10 @@ __global__ __launch_bounds__(256, (MT * KC_ > 32 || R * MT >= 16) ? 1 : 2) void 
     f32x4v* red = (f32x4v*)&xs[0][1];
     if constexpr (OWN) {
 #pragma unroll
-      for (int c = 0; c < MT; ++c) diagonal(gram[c], &stat[1 + w][16 * c]);
+      for (int c = 0; c < MT; ++c) {
+        const double s = wsum16(own[c]);
+        if (lane < 16) stat[w][16 * c + lane] = s;
+      }
     }
     if (w > 0) {
 #pragma unroll
@@ -321,8 +318,7 @@ __global__ __launch_bounds__(256, (MT * KC_ > 32 || R * MT >= 16) ? 1 : 2) void 
     for (int kk = 0; kk < KC; ++kk) {
       const int p = kk % PF;
       if constexpr (OWN) {
-        const bf16x8 o = xb[(kk * MT + (w < MT ? w : 0)) * 64];
-        gram[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(o, o, gram[0], 0, 0, 0);
+        own[0] = add_squares(own[0], xb[(kk * MT + (w < MT ? w : 0)) * 64]);
       }
       bf16x8 wdq[R];
 #pragma unroll
@@ -345,7 +341,8 @@ __global__ __launch_bounds__(256, (MT * KC_ > 32 || R * MT >= 16) ? 1 : 2) void 
     __syncthreads();
   }
   if constexpr (OWN) {
-    if (w < MT) diagonal(gram[0], &stat[0][16 * w]);
+    const double s = wsum16(own[0]);
+    if (w < MT && lane < 16) stat[0][16 * w + lane] = s;
     __syncthreads();
   }
   }  // !KIN
@@ -357,9 +354,9 @@ __global__ __launch_bounds__(256, (MT * KC_ > 32 || R * MT >= 16) ? 1 : 2) void 
   auto emit = [&](f32x4v v, int m, int r) {
     const int ms = m < M ? m : M - 1;
     if constexpr (OWN) {
-      float ss = stat[KIN ? 1 : 0][ms];
-      if constexpr (KIN) ss = ((ss + stat[2][ms]) + stat[3][ms]) + stat[4][ms];
-      v *= rsqrtf(ss * ep.inv_k + ep.eps);
+      double ss = stat[0][ms];
+      if constexpr (KIN) ss = ((ss + stat[1][ms]) + stat[2][ms]) + stat[3][ms];
+      v *= rsqrtf((float)ss * ep.inv_k + ep.eps);
     } else {
       if (ep.mode & EPI_RMS) v *= SUMS ? stat[0][ms] : rsqrtf(ep.ss_in[ms] * ep.inv_k + ep.eps);
     }
@@ -507,9 +504,9 @@ __global__ __launch_bounds__(256, (MT * KC_ > 32 || R * MT >= 16) ? 1 : 2) void 
     }
   }
   constexpr int SR = 16 * MT;  // OWN: sums of squares [split][strip][SR] behind the slabs
-  const __amdgpu_buffer_rsrc_t sr = rsrc(ws + ksplit * sstride, OWN ? (unsigned)(ksplit * nstrip * SR * 4) : 0);
+  const __amdgpu_buffer_rsrc_t sr = rsrc(ws + ksplit * sstride, OWN ? (unsigned)(ksplit * nstrip * SR * 8) : 0);
   if constexpr (OWN && !KIN) {
-    if (tid < SR) st1_sc1(sr, (unsigned)(((split * nstrip + strip) * SR + tid) * 4), stat[0][tid]);
+    if (tid < SR) st2_sc1(sr, (unsigned)(((split * nstrip + strip) * SR + tid) * 8), stat[0][tid]);
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
@@ -528,8 +525,8 @@ __global__ __launch_bounds__(256, (MT * KC_ > 32 || R * MT >= 16) ? 1 : 2) void 
   if (!*flag || (KIN && w != 0)) return;
   if constexpr (OWN && !KIN) {
     if (tid < SR) {
-      float ss = 0.f;
-      for (int sp = 0; sp < ksplit; ++sp) ss += ld1_sc1(sr, (unsigned)(((sp * nstrip + strip) * SR + tid) * 4));
+      double ss = 0.;
+      for (int sp = 0; sp < ksplit; ++sp) ss += ld2_sc1(sr, (unsigned)(((sp * nstrip + strip) * SR + tid) * 8));
       stat[0][tid] = ss;
     }
     __syncthreads();
@@ -1685,7 +1682,7 @@ KGS_EXPORT int kgs_skinny_geometry(int M, int* rows_per_strip, int* k_per_chunk,
 
 // y[M, N] (bf16, row stride ldy) = x[M, K] (row stride ldx) . W^T with W
 // prepacked ([N/16][K/32][64][8] bf16). ksplit must divide K / k_per_chunk;
-// with ksplit > 1, ws holds ksplit * mpad * N floats (OWN: and ksplit * mpad * N / rows_per_strip) and cnt N / rows_per_strip
+// with ksplit > 1, ws holds ksplit * mpad * N floats (OWN: and 2 ksplit * mpad * N / rows_per_strip) and cnt N / rows_per_strip
 // zero-initialised ints (left zeroed on return). epi: EPI_* flags (SWIGLU: y is
 // [M, N/2]; RMS needs ss_in[M], or OWN; RESID accumulates into y and, unless null, ss_out[M]);
 // ss_zero (optional, [M] floats) is cleared at kernel start. With EPI_SUMS_IN ss_in, with EPI_SUMS_OUT

@@ -1,8 +1,8 @@
-// What the decode products share (decode.hip, chain.hip): the page layout of the KV cache, write-through stores for
+// What the decode products share (decode.hip, decode_few.hip, decode_slabs.hip): the page layout of the KV cache, write-through stores for
 // hand-offs inside a launch, and the fused epilogues' flags and statistics.
 #pragma once
 
-#include "kgs_common.h"
+#include "sums64.h"
 
 namespace kgs {
 namespace dec {
@@ -30,6 +30,7 @@ __host__ __device__ __forceinline__ int kv_v_index(int tau, int d) {
 // over the four 16-lane rows (lanes of one column), on the permlane swaps
 __device__ __forceinline__ float wmax16(float v) { return xor32_max(xor16_max(v)); }
 __device__ __forceinline__ float wsum16(float v) { return xor32_sum(xor16_sum(v)); }
+__device__ __forceinline__ double wsum16(double v) { return xor32_sum(xor16_sum(v)); }
 
 // In-launch hand-offs (split-K slabs, attention split partials): producers store
 // WRITE-THROUGH (sc1 buffer stores) and drain, so they need no release fence (a
@@ -53,6 +54,13 @@ __device__ __forceinline__ void st1_sc1(__amdgpu_buffer_rsrc_t r, unsigned off, 
 }
 __device__ __forceinline__ float ld1_sc1(__amdgpu_buffer_rsrc_t r, unsigned off) {
   return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 16));
+}
+typedef unsigned u32x2v __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ void st2_sc1(__amdgpu_buffer_rsrc_t r, unsigned off, double a) {
+  __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2v, a), r, off, 0, 16);
+}
+__device__ __forceinline__ double ld2_sc1(__amdgpu_buffer_rsrc_t r, unsigned off) {
+  return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 16));
 }
 
 // Fused epilogues (runtime flags in SkinnyEpi::mode, uniform per launch):

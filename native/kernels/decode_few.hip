@@ -5,8 +5,7 @@
 // MFMA operand order, straight from memory) through a ring of PF k-steps and add their sums in LDS, in the order of the waves.
 // Loads are buffer loads, so that a step waits for exactly its own.
 //
-// OWN: the RMSNorm of x from x itself. Every wave holds its part of all rows anyway, and one more MFMA of x with itself per
-// k-step has the rows' sums of squares on its diagonal. Where the producer of x adds them up instead, 256 workgroups' atomics
+// OWN: the RMSNorm of x from x itself. Every wave holds its part of all rows anyway and adds up its squares (add_squares). Where the producer of x adds them up instead, 256 workgroups' atomics
 // meet on one address, 12.5 ns each, at the end of a launch that nothing hides: a layer's o and down took 1.6 us longer at 1
 // row, 2.0 at 16. Nothing here depends on the order in which workgroups arrive.
 //
@@ -54,7 +53,7 @@ template <int R, int MT, int NW, int PF, bool ROPE, bool OWN>
 __global__ __launch_bounds__(64 * NW) void few(FewArgs a) {
   static_assert(MT == 1 || (!ROPE && !OWN && R == 1));
   __shared__ __attribute__((aligned(16))) f32x4v red[NW * R * MT * 64];
-  __shared__ float stat[OWN ? NW : 1][16];
+  __shared__ double stat[OWN ? NW : 1][16];
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), fr = lane & 15, fq = lane >> 4;
   const int M = a.M, nkk = a.K / 32, nsteps = nkk / NW, kk0 = w * nsteps, nt0 = blockIdx.x * R;
   if constexpr (!ROPE && !OWN) {
@@ -97,7 +96,8 @@ __global__ __launch_bounds__(64 * NW) void few(FewArgs a) {
     }
   }
 
-  f32x4v acc[R][MT], gram = f32x4v{0.f, 0.f, 0.f, 0.f};
+  f32x4v acc[R][MT];
+  [[maybe_unused]] double own = 0.;
 #pragma unroll
   for (int r = 0; r < R; ++r)
 #pragma unroll
@@ -111,7 +111,7 @@ __global__ __launch_bounds__(64 * NW) void few(FewArgs a) {
       for (int r = 0; r < R; ++r)
 #pragma unroll
         for (int c = 0; c < MT; ++c) acc[r][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[p][r], xf[p][c], acc[r][c], 0, 0, 0);
-      if constexpr (OWN) gram = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xf[p][0], xf[p][0], gram, 0, 0, 0);
+      if constexpr (OWN) own = add_squares(own, xf[p][0]);
       load(p, next + p);
     }
   }
@@ -119,9 +119,9 @@ __global__ __launch_bounds__(64 * NW) void few(FewArgs a) {
   for (int r = 0; r < R; ++r)
 #pragma unroll
     for (int c = 0; c < MT; ++c) red[((w * R + r) * MT + c) * 64 + lane] = acc[r][c];
-  if constexpr (OWN) {  // row m of the diagonal: lanes 4 (m / 4) .. of column m, element m % 4
-    const float lo = fr & 1 ? gram[1] : gram[0], hi = fr & 1 ? gram[3] : gram[2];
-    if (fq == fr >> 2) stat[w][fr] = fr & 2 ? hi : lo;
+  if constexpr (OWN) {
+    own = wsum16(own);
+    if (fq == 0) stat[w][fr] = own;
   }
   __syncthreads();
   if (w >= R * MT) return;
@@ -131,10 +131,10 @@ __global__ __launch_bounds__(64 * NW) void few(FewArgs a) {
 #pragma unroll
   for (int j = 1; j < NW; ++j) v += red[(j * R * MT + w) * 64 + lane];
   if constexpr (OWN) {
-    float ss = stat[0][fr];
+    double ss = stat[0][fr];
 #pragma unroll
     for (int j = 1; j < NW; ++j) ss += stat[j][fr];
-    v *= rsqrtf(ss * a.inv_k + a.eps);
+    v *= rsqrtf((float)ss * a.inv_k + a.eps);
   }
   const bool in = m < M;
   if constexpr (ROPE) {

@@ -14,7 +14,9 @@
 // the same block (kgs/models/llama.py, backend "torch") runs ~10 kernels per op
 // here with fp32 intermediates in HBM; profiles/llama_prefill_kernels_v0.md has
 // the numbers that motivated these kernels.
-#include "kgs_common.h"
+#include "sums64.h"
+
+#include <type_traits>
 
 namespace kgs {
 namespace tfm {
@@ -338,14 +340,16 @@ __global__ __launch_bounds__(256) void silu_mul(const unsigned short* __restrict
 // is issued before the first add (a run-time slice loop waits out one cache
 // latency per slice); 0 = run-time count.
 // SQUARES: x' = bf16(x + sum_s P[s][row]), and its row's sum of squares to sq[row] instead of y: for a product that
-// applies the norm to its own rows. Bound by the slices, 4 to 5 TB/s from the caches (more threads a row: the same).
+// applies the norm to its own rows; a chunk's eight in fp32, on from there in fp64, so that the sum is as good as rounded once. Bound by
+// the slices, 4 to 5 TB/s from the caches (more threads a row: the same).
 template <int NJ, int NSL, bool SQUARES = false>
 __global__ __launch_bounds__(256) void splitk_add_rmsnorm(const float* __restrict__ P, int nslice, long MN,
                                                           unsigned short* __restrict__ x,
                                                           const unsigned short* __restrict__ w,
                                                           unsigned short* __restrict__ y, int cols, long ldx,
                                                           long ldy, float eps, float* __restrict__ sq = nullptr) {
-  __shared__ float red[4];
+  using Sum = typename std::conditional<SQUARES, double, float>::type;
+  __shared__ Sum red[4];
   const int row = blockIdx.x, t = threadIdx.x;
   bf16x8* xr = (bf16x8*)(x + row * ldx);
   // the residual chunks and the norm weight are loaded next to the partials:
@@ -359,7 +363,7 @@ __global__ __launch_bounds__(256) void splitk_add_rmsnorm(const float* __restric
     if constexpr (!SQUARES) wv[j] = wr[t + 256 * j];
   }
   float v[NJ][8];
-  float ss = 0.f;
+  Sum ss = 0;
 #pragma unroll
   for (int j = 0; j < NJ; ++j) {
     const long e = (long)row * cols + 8 * (t + 256 * j);
@@ -393,16 +397,18 @@ __global__ __launch_bounds__(256) void splitk_add_rmsnorm(const float* __restric
       const float p = k < 4 ? a[k] : b[k - 4], d = SQUARES ? p : bf2f(f2bf(p));
       o[k] = (short)f2bf(bf2f((unsigned short)xv[k]) + d);
       v[j][k] = bf2f((unsigned short)o[k]);
-      ss += v[j][k] * v[j][k];
+      if constexpr (!SQUARES) ss += v[j][k] * v[j][k];
     }
+    if constexpr (SQUARES) ss = add_squares(ss, o);
     xr[t + 256 * j] = o;
   }
-  ss = wave_sum(ss);
+  if constexpr (SQUARES) ss = kgs::wave_sum(ss);
+  else ss = wave_sum(ss);
   if ((t & 63) == 0) red[t >> 6] = ss;
   __syncthreads();
   ss = (red[0] + red[1]) + (red[2] + red[3]);
   if constexpr (SQUARES) {
-    if (t == 0) sq[row] = ss;
+    if (t == 0) sq[row] = (float)ss;
     return;
   }
   const float r = rsqrtf(ss / (float)cols + eps);

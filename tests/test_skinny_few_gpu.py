@@ -122,6 +122,30 @@ def test_skinny_norm_by_its_own_statistics(variant, ksplit, n, k, m):
     _close(D.own_gemm(x, pw, out=out, resid=True), want)
 
 
+# few rows by 2, 4 and 8 waves; skinny with x through LDS, in K slices, and with K split inside the workgroup
+@pytest.mark.parametrize("form,n,k,m", [("few", 8208, 4096, 16), ("few", 4112, 4096, 16), ("few", 4096, 4096, 9), ((1, 1), 256, 4096, 16), ((4, 1), 64, 8192, 32),
+                                        ((3, 2), 256, 4096, 16), ((10, 4), 192, 4096, 64), ((22, 1), 64, 4096, 32), ((23, 1), 64, 8192, 31), ((24, 1), 64, 4096, 64)])
+@pytest.mark.parametrize("large", (1, 30))
+def test_own_statistics_are_sums_rounded_once(form, n, k, m, large):
+    """A negative eps close to the mean square lays the sum's last bits open: 1 / scale^2 = ss / k + eps, k a power of two, without a further rounding."""
+    g = torch.Generator(device="cuda").manual_seed(k + m)
+    v = torch.randn(k, generator=g, device="cuda")
+    v[:4] *= large
+    v = v.bfloat16()
+    x = torch.stack([v[torch.randperm(k, generator=g, device="cuda")] for _ in range(m)])
+    w = (torch.randn(n, k, generator=g, device="cuda") * k ** -0.5).bfloat16()
+    ss = float(v.double().pow(2).sum())
+    eps = float(torch.tensor(-ss / k * (1 - 2.0 ** -18), dtype=torch.float32))
+    pw = D.PackedWeight(w)
+    got = D.skinny_few(x, pw, norm=True, eps=eps) if form == "few" else D.skinny_gemm(x, pw, variant=form[0], ksplit=form[1], norm=True, eps=eps)
+    ref = x.double() @ w.double().T
+    scale = (got.double() * ref).sum(1) / ref.pow(2).sum(1)  # the rows' outputs differ by their roundings alone
+    err = (k * (scale.pow(-2) - eps) / ss - 1).abs()
+    # a rounding to fp32 (2^-24), the parts' before they meet in fp64 (a lane's eight values, 3 2^-24 of them; four values of 30 times the others' size are
+    # most of the sum), and what 64 roundings to bf16 and more leave of 2^-9 times 2^-18
+    assert float(err.max()) <= (1.25 if large == 1 else 3.0) * 2.0 ** -24, float(err.max()) * 2 ** 24
+
+
 @pytest.mark.parametrize("m", (9, 24, 40))
 def test_skinny_rope_by_its_own_statistics(m):
     from kgs.ops.transformer import rope_tables

@@ -125,6 +125,18 @@ def test_residual_add_of_slices_and_its_squares(parts, cols):
     assert torch.allclose(sq.double(), want.double().pow(2).sum(1), rtol=1e-6)
 
 
+@pytest.mark.parametrize("cols", (2048, 8192))
+def test_squares_are_sums_rounded_once(cols):
+    from kgs.ops.transformer import splitk_add_squares
+
+    g = torch.Generator(device="cuda").manual_seed(cols)
+    x = torch.randn(400, cols, generator=g, device="cuda").bfloat16()
+    sq = splitk_add_squares(torch.randn(2, 400, cols, generator=g, device="cuda"), x)
+    want = x.double().pow(2).sum(1)
+    # the rounding to fp32 and, averaged over 256 chunks and more of eight values, theirs
+    assert float((sq.double() / want - 1).abs().max()) <= 1.25 * 2.0 ** -24
+
+
 @pytest.mark.parametrize("rows", (33, 48, 49, 64, 96))
 @pytest.mark.parametrize("wide", (False, True))  # gate and up of a product's two tiles a wave
 def test_layers_of_slices_as_the_others(rows, wide):

@@ -521,13 +521,39 @@ def few_takes(m: int, n: int, k: int, fp8: bool = False, plain: bool = False) ->
 
 @lru_cache(maxsize=4096)
 def few_route(m: int, n: int, k: int, plain: bool = False) -> bool:
-    """Whether the kernel of few rows is the better one, of those that take these rows: up to 8, up to 16 where W has at most 512 strips and x
-    128k values -- beyond, x through LDS is shared by more of W, or split over workgroups (us at 16 rows, few / others: 28672x4096 51 / 43,
-    4096x14336 26.3 / 23.5, but 6144x4096 13.7 / 16.2, 4096x4096 10.5 / 11, 6656x2048 7.5 / 10.3) -- and up to 32 for short sums of narrow weights and the sizes that skinny does not
-    take (24 rows: 2048x768 4.7 / 7.6, 4096x1536 6.7 / 9.6, 1344x2048 7.3 / 6.7)."""
+    """Whether the kernel of few rows is the better one, of those that take these rows; us of plain products, weights from HBM, few / others.
+
+    Beside :func:`skinny_gemm`: up to 8 rows where W is not much wider than the CUs are many -- its workgroups are short, and a third
+    round of them costs more than skinny's long ones (12288x1024 at 1 row 6.6 / 7.0, 64000x1024 29 / 24.8, 24576x2048 19.6 / 20.4, 64000x2048
+    48.5 / 46.2 and at 8 rows 49 / 45.2), beyond that from K = 3584 on up to 4 rows and where K is a multiple of 4096, whose strips lie at
+    multiples of 128 KB, which skinny's four waves read at once (32000x4096 at 8 rows 44.8 / 48.3, 32000x5120 at 8 57 / 55). Not where W has as many strips
+    at multiples of 256 KB as CUs (4096x8192 at 1 row 16.0 / 14.3, in two tiles a workgroup 8192x8192 at 8 31.8 / 28.3), nor short
+    strips of long K, which skinny reads in slices (1024x14336 at 8 rows 16.9 / 13.4), nor a few more strips than CUs in four waves each (5120x13824 at
+    4 rows 30.3 / 28.0). Up to 16 rows while x is short, which every workgroup
+    reads whole (6144x4096 at 16 13.7 / 16.2, but 2048x8192 14.4 / 12.6, 8192x7168 at 12 27 / 32, 2560x6144 at 16 10.5 / 9.7); up to 32
+    for short K that does not divide by 1024 (24 rows: 2048x768 4.7 / 7.6, 4096x1536 6.7 / 9.6, but 2048x1024 5.5 / 4.6).
+
+    Beside the library, for sizes that skinny does not take: as long as neither x nor the grid is long (832x2048 at 1 row 3.6 / 7.9; 896x4864
+    at 24 25.5 / 16.6, 13824x768 at 16 1.31 times its time, 6144x11008 1.15 times)."""
     if not few_takes(m, n, k, False, plain):
         return False
-    return m <= 8 or (m <= 16 and n <= 512 * 16 and m * k <= 128 << 10) or (k <= 1536 and n <= 4096) or not _own_by_skinny(m, n, k, False, False)
+    if not (skinny_takes(m, n, k) if plain else _own_by_skinny(m, n, k, False, False)):
+        if not plain:
+            return True
+        return n <= 32768 if m <= 8 else n <= 8192 and (n <= 4096 or k <= 8192) if m <= 16 else n <= 4096 and k <= 2048
+    if m > 16:
+        return k <= 1536 and n <= 4096 and k % 1024 != 0
+    if k % 8192 == 0 and ((n == 4096 and m <= 8) or (n == 8192 and m > 4)):
+        return False
+    if n <= 2048:
+        return k <= (8192 if m <= 8 else 5120) or (k < 8192 and k % 1024 != 0)
+    if m > 8:
+        return n <= 8192 and m * k < 96 << 10
+    if 4096 < n <= 5120 and k > 8192 and k % 1024:
+        return False
+    if n <= 24576:
+        return n <= 10240 or (k > 1024 and (m <= 4 or not 12288 < n < 16384))
+    return (m <= 4 and k >= 3584) or k % 4096 == 0
 
 
 @lru_cache(maxsize=4096)
@@ -546,7 +572,9 @@ def own_gemm(x: torch.Tensor, w: PackedWeight, out: torch.Tensor | None = None, 
              eps: float = 1e-5, rope: dict | None = None, counters: torch.Tensor | None = None) -> torch.Tensor:
     """:func:`skinny_gemm` with ``norm`` or ``resid``, by :func:`skinny_few` where that is the better one (:func:`few_route`)."""
     m, k = x.shape
-    if m <= 16 and not w.fp8 and (few_route(m, w.n, k) or (few_takes(m, w.n, k) and not _own_by_skinny(m, w.n, k, False, bool(w.rope)))):
+    plain = not norm and rope is None
+    if m <= 16 and not w.fp8 and (few_route(m, w.n, k, plain) or (few_takes(m, w.n, k, False, plain) and not (
+            skinny_takes(m, w.n, k) if plain else _own_by_skinny(m, w.n, k, False, bool(w.rope))))):
         return skinny_few(x, w, out, norm, resid, eps, rope)
     return skinny_gemm(x, w, out, norm=norm, resid=resid, eps=eps, rope=rope, counters=counters)
 

@@ -110,6 +110,18 @@ def test_what_the_rules_of_slices_take_the_kernel_takes():
                     assert lib.kgs_skinny_rows(1, 1, 1, m, n, k, k, n, tiles, 0, None, 0.0, 0.0, None) == align, (m, n, k)
 
 
+def test_few_rows_keep_to_where_they_are_the_faster():
+    """Beside skinny: not for wide weights of short sums, x that is long, strips at multiples of 256 KB; beside the library: neither long sums nor wide weights."""
+    few = [(1, 28672, 4096), (8, 32000, 4096), (8, 16384, 2048), (1, 24576, 2048), (8, 10240, 1024), (16, 6144, 4096), (8, 4096, 14336), (1, 4096, 4096), (16, 2048, 3584),
+           (4, 8192, 8192), (24, 2048, 768), (24, 4096, 1536), (32, 832, 1984), (8, 22016, 768), (12, 2048, 11008)]
+    not_few = [(1, 64000, 1024), (8, 64000, 2048), (1, 32000, 2048), (8, 32000, 5120), (4, 24576, 512), (1, 4096, 8192), (8, 8192, 8192), (16, 8192, 8192), (8, 1024, 14336),
+               (16, 2048, 8192), (12, 1024, 6144), (24, 2048, 1024), (32, 4096, 1024), (24, 896, 4864), (32, 2048, 11008), (16, 13824, 768), (16, 6144, 11008), (4, 5120, 13824)]
+    for case in few:
+        assert D.few_route(*case, True), case
+    for case in not_few:
+        assert not D.few_route(*case, True), case
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("m,v", [(17, 22), (32, 22), (24, 23), (33, 24), (64, 24), (40, 25)])
 def test_k_split_in_the_workgroup(m, v):

@@ -68,18 +68,16 @@ class Projection:
             ld % 8 == 0 and x.data_ptr() % 16 == 0
 
     def _packed(self, x, m, n, k):
-        """The product by a kernel that reads the packed weight, or None. Up to 32 rows that of few rows (:func:`kgs.ops.decode.few_route`; a gate and up
-        of K off 512 where the gate kernel has few workgroups: us at 8 rows, gate kernel / so, 8192x768 5.8 / 5.6, 16384x768 6.7 / 9.2, 13824x4864
-        28.8 / 35.5) or :func:`kgs.ops.decode.skinny_gemm` -- a gate and up of one round of 64-row strips by :func:`kgs.ops.decode.skinny_rows` from 17 rows
-        on (16384x2048 at 32 rows 16.1 us / 14.5) --, from 33 rows on ``skinny_rows`` where its wide tiles fill the CUs (us at 64 rows, four-wave
-        tiles / so: 28672x4096 51.6 / 44.4, 32000x4096 61 / 48)."""
-        if m > SKINNY_MAX_ROWS:
-            return D.skinny_rows(x, self.packed) if D.slab_rows_tiles(m, n, k) == 2 else None
-        if D.few_route(m, n, k, True) and not (self.gated is not None and k % 512 and n > (8192 if m <= 8 else 4096)):
+        """The product by a kernel that reads the packed weight, or None: up to 32 rows that of few rows (:func:`kgs.ops.decode.few_route`; a gate
+        and up of K off 512 where the gate kernel has few workgroups: us at 8 rows, gate kernel / so, 8192x768 5.8 / 5.6, 16384x768 6.7 / 9.2,
+        13824x4864 28.8 / 35.5), :func:`kgs.ops.decode.skinny_rows` where it pays, or :func:`kgs.ops.decode.skinny_gemm` -- of K of 512, others
+        slice badly (2048x11008 at 32 rows 54.9 us, by the library 26.9) --, from 33 rows on ``skinny_rows``."""
+        few = m <= SKINNY_MAX_ROWS and D.few_route(m, n, k, True)
+        if few and not (self.gated is not None and k % 512 and n > (8192 if m <= 8 else 4096)):
             return D.skinny_few(x, self.packed)
-        if m > 16 and self.gated is not None and n <= 64 * D.CUS and D.slab_rows_tiles(m, n, k):
+        if D.rows_pay(m, n, k, self.gated is not None):
             return D.skinny_rows(x, self.packed)
-        return D.skinny_gemm(x, self.packed) if D.skinny_takes(m, n, k) else None
+        return D.skinny_gemm(x, self.packed) if m <= SKINNY_MAX_ROWS and k % 512 == 0 and D.skinny_takes(m, n, k) else None
 
     def partials(self, x: torch.Tensor) -> torch.Tensor:
         """:meth:`__call__`, or where the product of a decode batch runs in K slices those, fp32 ``[slices, M, N]``, for a consumer

@@ -623,6 +623,40 @@ def rows_pay(m: int, n: int, k: int, gated: bool) -> bool:
     return k >= 1536 if m <= 64 else k >= (3072 if rounds == 1 else 5120)
 
 
+def slabs_fill(m: int, n: int, k: int) -> bool:
+    """Whether the slices of :func:`slab_split` are short or fill the CUs. A K like 11008 gives two slices of 43 ring rounds in a quarter of the workgroups
+    that the CUs hold: the product and a hyper-connection step at 64 / 96 rows, over the general kernel's with the step, 4096x11008 1.65 / 1.82, 3072x14336 (slices of 3584,
+    three quarters) 1.02 / 1.09, 5120x14336 (the same in wide tiles) 0.95 / 0.97, 2048x5632 (of 2816) 0.90 / 0.99."""
+    split = slab_split(m, n, k)
+    if split is None:
+        return False
+    r, ns = split
+    wgs = n // (64 * r) * ns
+    return wgs >= CUS or (wgs >= 48 and k // ns <= (4096 if r == 2 else 3072))
+
+
+@lru_cache(maxsize=4096)
+def slabs_pay(m: int, n: int, k: int) -> bool:
+    """Whether a product left in slices to a hyper-connection step beats the whole product in front of it (times of both, in slices over whole): from 33 rows
+    on where :func:`slabs_fill` says so. Up to 32 rows a product that one launch reads whole at full rate is better whole:
+    of more than 2048 rows of W by the kernel of few rows (4096x4096 at 1 / 8 / 16 rows 1.23 / 1.24 / 1.15, 5120x2048 1.19 / 1.08 / 0.97, 2048x4096 0.94 / 0.89
+    / 0.82), and of short K by skinny with K split in the workgroup (4096x1024 at 32 1.27, 4096x2048 1.09, 2048x1024 1.01); and so are two long
+    slices in few workgroups (1024x13824 1.24 at 1 row, 4096x11008 1.23 at 32)."""
+    split = slab_split(m, n, k)
+    if split is None:
+        return False
+    if m > 32:
+        return slabs_fill(m, n, k) and not (m > 64 and n >= 4096 and k <= 1024) and not (n > 4096 and k <= 512)
+    r, ns = split
+    if k // ns > 3072 and n // (64 * r) * ns < CUS // 2:
+        return False
+    if m <= 8:
+        return not (k <= 1024 or (n > 2048 and k <= (8192 if m <= 4 else 7168)))
+    if m <= 16:
+        return not ((n >= 4096 and k <= 4096) or (n > 4096 and k <= 512))
+    return not ((n >= 4096 and k in (1024, 2048)) or (n > 2048 and k <= 1024))
+
+
 def _slab_operand(x: torch.Tensor, w: PackedWeight) -> tuple[int, int]:
     if x.dtype != torch.bfloat16 or not x.is_cuda or x.dim() != 2 or x.stride(1) != 1 or x.shape[1] != w.k:
         raise ValueError("x must be a row-major bf16 GPU matrix [M, K]")

@@ -80,10 +80,10 @@ class Projection:
         return D.skinny_gemm(x, self.packed) if m <= SKINNY_MAX_ROWS and k % 512 == 0 and D.skinny_takes(m, n, k) else None
 
     def partials(self, x: torch.Tensor) -> torch.Tensor:
-        """:meth:`__call__`, or where the product of a decode batch runs in K slices those, fp32 ``[slices, M, N]``, for a consumer
-        that adds them and rounds to bf16. One slice is stored as such (its sum is no work), and rows that the kernel cannot read go the other way."""
+        """:meth:`__call__`, or where it pays (:func:`kgs.ops.decode.slabs_pay`) the product of a decode batch in K slices, fp32 ``[slices, M, N]``, for a
+        consumer that adds them and rounds to bf16. One slice is stored as such (its sum is no work), and rows that the kernel cannot read go the other way."""
         p = self.packed
-        if self.gated is not None or x.shape[1] != self.w.shape[1] or not self._reads(x) or D.slab_split(x.shape[0], p.n, p.k) is None:
+        if self.gated is not None or x.shape[1] != self.w.shape[1] or not self._reads(x) or not D.slabs_pay(x.shape[0], p.n, p.k):
             return self(x)
         return D.skinny_slabs(x, p)
 

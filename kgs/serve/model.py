@@ -685,7 +685,7 @@ class ServingModel:
     def decode(self, tokens, positions, slots, block_tables, ctx_lens, pages_per_split=None) -> torch.Tensor:
         """One token per sequence -> logits [B, vocab]."""
         c = self.cfg
-        if self.backend == "kgs" and tokens.shape[0] <= self.fused_max_batch or self._slabs(tokens.shape[0]):
+        if self.backend == "kgs" and tokens.shape[0] <= self.fused_max_batch or self._slabs_pay(tokens.shape[0]):
             return self._decode_fused(tokens, positions, slots, block_tables, ctx_lens, pages_per_split)
         tickets = self._tickets(block_tables)
         x, y = self._start(tokens, zero=tickets)
@@ -757,7 +757,7 @@ class ServingModel:
             return D.paged_decode_attention(qkv, self.cache.layer(i), block_tables, ctx_lens, c.heads, c.kv_heads,
                                             pages_per_split=pages_per_split, tickets=tickets)
 
-        if self._slabs(tokens.shape[0]):
+        if self._slabs_pay(tokens.shape[0]):
             x, y, ss = self._slab_layers(tokens, positions, slots, attend, "decode", tickets=tickets)
             out = self._slab_head(x if y is None else y, y is None, ss, decode=True)
             T.op("decode-slabs lm_head")
@@ -783,10 +783,16 @@ class ServingModel:
             all(D.slab_split(m, P[n].n, P[n].k) for n in ("qkv", "o", "down")) and \
             all(D.slab_rows_tiles(m, w.n, w.k) for w in (P["gate_up"], self.packed_lm))
 
+    def _slabs_pay(self, m: int) -> bool:
+        """Whether they are the better ones too: up to 48 rows, where the fused layers are slower still, always, beyond where the products' slices are short or fill the
+        CUs (:func:`kgs.ops.decode.slabs_fill`; four layers 2048 wide with a feed-forward of 11008, us a step of 64 / 96 rows by four-wave tiles 363 / 378, so 420 / 495)."""
+        return self._slabs(m) and (m <= 48 or all(D.slabs_fill(m, w.n, w.k) for w in (self.packed[0][n] for n in ("qkv", "o", "down"))))
+
     def _slab_prompts(self, m: int) -> bool:
-        """:meth:`_slabs` for prompts, whose launches come from the host one by one: up to 48 rows, where the fused layers have 5 a layer and these 8, only
-        with layers of 96 M weights and more (us, fused / here, one prompt of 36 tokens: 2048 wide, 63 M, 347 / 368; 4096 wide, 218 M, 612 / 487)."""
-        return self._slabs(m) and (m > 48 or sum(w.n * w.k for w in self.packed[0].values()) >= 96 << 20)
+        """:meth:`_slabs_pay` for prompts, whose launches come from the host one by one: up to 48 rows, where the fused layers have 5 a layer and these 8, only
+        with layers of 72 M weights and more (us, fused / here, one prompt of 40 tokens among others and alone: 2048 wide, 61 M weights 331 / 379, 423 / 436; 80 M 387 / 382,
+        499 / 439; 92 M 400 / 386, 510 / 448; 4096 wide, 67 M 386 / 381, 489 / 460; 92 M 440 / 382, 544 / 472; 218 M 576 / 479, 685 / 586)."""
+        return self._slabs_pay(m) and (m > 48 or sum(w.n * w.k for w in self.packed[0].values()) >= 72_000_000)
 
     def _slab_gate(self, m: int):
         """Gate and up of ``m`` rows of :meth:`_slab_layers`: a route of :meth:`_swiglu_route` on normed rows, or None: :func:`kgs.ops.decode.skinny_rows` on the

@@ -91,6 +91,10 @@ def test_rows_of_the_layers_in_slices(most, rows, slabs):
         packed_lm, cfg = _Weight(1024, 2048), SimpleNamespace(hidden=2048)
 
     assert ServingModel._slabs(M, rows) is slabs
+    M._slabs = staticmethod(lambda m: ServingModel._slabs(M, m))
+    assert ServingModel._slabs_pay(M, rows) is slabs
+    M.packed = [{**M.packed[0], "down": _Weight(2048, 11008)}]  # slices badly: from 49 rows on the split tiles are the faster
+    assert ServingModel._slabs_pay(M, rows) is (slabs and rows <= 48)
 
 
 def test_what_the_rules_of_slices_take_the_kernel_takes():
@@ -128,6 +132,16 @@ def test_whole_products_keep_to_where_they_are_the_faster():
                                 (64, 32000, 1024, True, False), (96, 24576, 2048, True, False), (64, 32000, 4096, False, True), (96, 32000, 4096, False, True), (64, 24576, 512, False, False),
                                 (64, 40960, 4096, False, False), (64, 64000, 2048, False, True), (96, 64000, 2048, False, False), (96, 128256, 4096, False, False), (97, 32000, 4096, False, False)):
         assert D.rows_pay(m, n, k, gated) is pay, (m, n, k, gated)
+
+
+def test_slices_keep_to_where_they_are_the_faster():
+    for m, n, k, fill in ((64, 4096, 11008, False), (49, 2048, 11008, False), (96, 2560, 14336, False), (64, 512, 5632, False), (96, 4096, 14336, True), (96, 2048, 5632, True),
+                          (64, 8192, 28672, True), (64, 2048, 8192, True), (64, 2080, 2048, False)):
+        assert D.slabs_fill(m, n, k) is fill, (m, n, k)
+    for m, n, k, pay in ((1, 2048, 2048, True), (1, 4096, 4096, False), (8, 4096, 4096, False), (16, 4096, 4096, False), (24, 4096, 4096, True), (32, 4096, 1024, False),
+                         (32, 2048, 8192, True), (1, 1024, 13824, False), (32, 4096, 11008, False), (64, 4096, 11008, False), (64, 2048, 8192, True), (96, 4096, 1024, False),
+                         (8, 4096, 14336, True), (97, 2048, 2048, False)):
+        assert D.slabs_pay(m, n, k) is pay, (m, n, k)
 
 
 @pytest.mark.gpu

@@ -608,8 +608,8 @@ def slab_rows_tiles(m: int, n: int, k: int, cus: int = CUS) -> int | None:
 def rows_pay(m: int, n: int, k: int, gated: bool) -> bool:
     """Whether :func:`skinny_rows` beats what reads the weight's rows, by the time of the one over the other: of a gate and up at 17 to 32 rows one round
     of 64-row strips, or most of one of short K (16384x2048 0.93, 10240x2048 0.95, 10240x8192 1.04, 4096x4096 1.66); from 33 rows on its wide tiles in
-    most of one round or in whole ones, of K that is worth a workgroup's start -- at 64 / 96 rows 28672x1024 1.18 / 1.19, x2048 0.91 / 0.95, 40960x4096 1.15
-    / 1.16, 64000x4096 0.91 / 0.96, 128256x4096, which has a measured entry, 1.03 / 1.13, 28672x6144 0.79 / 0.82; gated 28672x1536 0.97 / 1.07, x2048 1.01 / 1.04, x5120 0.84 / 0.92."""
+    most of one round or in whole ones, of K that is worth a workgroup's start -- at 64 / 96 rows 28672x1024 1.18 / 1.19, x2048 1.04 / 1.07, 32000x2048 1.07 /
+    1.11, x4096 0.92 / 0.97, 40960x4096 1.15 / 1.16, 64000x4096 0.91 / 0.96, 128256x4096, which has a measured entry, 1.03 / 1.13, 28672x6144 0.79 / 0.82; gated 28672x1536 0.97 / 1.07, x2048 1.01 / 1.04, x5120 0.84 / 0.92."""
     if m <= 32:
         return m > 16 and gated and k % 512 == 0 and slab_rows_tiles(m, n, k) is not None and \
             (56 * CUS < n <= 64 * CUS or (10240 <= n <= 56 * CUS and k <= 4096))
@@ -620,7 +620,7 @@ def rows_pay(m: int, n: int, k: int, gated: bool) -> bool:
     wgs, rounds = n // 128, -(-n // (128 * CUS))
     if rounds > 1 and (20 * wgs < 19 * rounds * CUS or w4x_route(m, n, k) is not None):
         return False
-    return k >= 1536 if m <= 64 else k >= (3072 if rounds == 1 else 5120)
+    return k >= (3072 if m <= 64 or rounds == 1 else 5120)
 
 
 def slabs_fill(m: int, n: int, k: int) -> bool:

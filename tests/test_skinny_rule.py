@@ -130,7 +130,7 @@ def test_whole_products_keep_to_where_they_are_the_faster():
     for m, n, k, gated, pay in ((24, 16384, 2048, True, True), (32, 10240, 2048, True, True), (32, 10240, 8192, True, False), (24, 4096, 4096, True, False), (32, 8192, 14336, True, False),
                                 (24, 16384, 768, True, False), (24, 16384, 2048, False, False), (16, 16384, 2048, True, False), (64, 28672, 4096, True, True), (90, 28672, 5120, True, True),
                                 (64, 32000, 1024, True, False), (96, 24576, 2048, True, False), (64, 32000, 4096, False, True), (96, 32000, 4096, False, True), (64, 24576, 512, False, False),
-                                (64, 40960, 4096, False, False), (64, 64000, 2048, False, True), (96, 64000, 2048, False, False), (96, 128256, 4096, False, False), (97, 32000, 4096, False, False)):
+                                (64, 40960, 4096, False, False), (64, 64000, 4096, False, True), (64, 32000, 2048, False, False), (96, 64000, 2048, False, False), (96, 128256, 4096, False, False), (97, 32000, 4096, False, False)):
         assert D.rows_pay(m, n, k, gated) is pay, (m, n, k, gated)
 
 

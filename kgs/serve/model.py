@@ -426,9 +426,9 @@ class ServingModel:
 
     def _fused_prompts(self, rows: int, prompts: int) -> bool:
         """Whether a step of so many prompt rows takes the fused decode layer: as many as a decode step of it,
-        64 at most (what its rotation takes), where its products tile and its rows' statistics are exact sums."""
-        if self.packed is None or self.decode_fp8 or not 0 < rows <= min(self.fused_max_batch, 64) or \
-                self.packed[0]["o"].n > D.SUM_MAX_N:
+        64 at most (what its rotation takes), where its products tile: what tiles makes its norms' statistics itself, so that equal steps give equal bits. Not wider
+        than the norm kernels of longer prompts."""
+        if self.packed is None or self.decode_fp8 or not 0 < rows <= min(self.fused_max_batch, 64) or self.packed[0]["o"].n > 8192:
             return False
         return all(D.skinny_takes(rows, w.n, w.k, w.fp8, bool(w.rope)) for w in self.packed[0].values()) and \
             D.skinny_takes(prompts, self.packed_lm.n, self.packed_lm.k)
@@ -454,12 +454,8 @@ class ServingModel:
         # counters of the step's own, cleared with its first launch: nothing is shared with a decode step on another stream
         most = max(w.n for w in (*self.packed[0].values(), self.packed_lm))
         count = torch.empty(most // 16, dtype=torch.int32, device=tokens.device)
-        x, ss = self._fused_layers(tokens, positions, slots, attend, "prefill", count, exact=True, keep=plan.keep, heads=plan.last.numel())
-        x = x.index_select(0, plan.last)
-        if ss is None:
-            out = D.own_gemm(x, self.packed_lm, norm=True, eps=c.eps, counters=count)
-        else:
-            out = D.skinny_gemm(x, self.packed_lm, rms=ss.index_select(1, plan.last), eps=c.eps, counters=count)
+        x, _ = self._fused_layers(tokens, positions, slots, attend, "prefill", count, keep=plan.keep, heads=plan.last.numel())
+        out = D.own_gemm(x.index_select(0, plan.last), self.packed_lm, norm=True, eps=c.eps, counters=count)
         T.op("prefill-fused lm_head")
         return out
 
@@ -762,7 +758,7 @@ class ServingModel:
             out = self._slab_head(x if y is None else y, y is None, ss, decode=True)
             T.op("decode-slabs lm_head")
             return out
-        x, ss = self._fused_layers(tokens, positions, slots, attend, "decode", None, exact=False, tickets=tickets)
+        x, ss = self._fused_layers(tokens, positions, slots, attend, "decode", None, tickets=tickets)
         out = D.own_gemm(x, self.packed_lm, norm=True, eps=c.eps) if ss is None else D.skinny_gemm(x, self.packed_lm, rms=ss, eps=c.eps)
         T.op("decode-fused lm_head")
         return out
@@ -878,13 +874,10 @@ class ServingModel:
         x = self.embed[tokens.long()].reshape(-1, self.cfg.hidden).contiguous()
         return x, self._norm(x, None, self.ln1[0]) if norm else None
 
-    def _fused_layers(self, tokens, positions, slots, attend, kind: str, counters, exact: bool, keep=None,
-                      tickets=None, heads=None):
-        """The residual rows after all layers and their sums of squares (None where the products make their own, :meth:`_own`; ``heads``: rows of the LM head, all); ``attend(qkv, layer)`` is the
-        attention of the rotated rows, whose keys and values are in the cache. ``exact``: statistics whose
-        bits do not depend on the order in which workgroups arrive, so that equal steps give equal bits. ``keep``
-        (int32): of these rows of ``tokens``, ``positions`` and ``slots`` only. ``counters`` and
-        ``tickets``: the step's own, cleared here (not both of them)."""
+    def _fused_layers(self, tokens, positions, slots, attend, kind: str, counters, keep=None, tickets=None, heads=None):
+        """The residual rows after all layers and their sums of squares (None where the products make their own, :meth:`_own`; ``heads``: rows of
+        the LM head, all); ``attend(qkv, layer)`` is the attention of the rotated rows, whose keys and values are in the cache. ``keep`` (int32): of
+        these rows of ``tokens``, ``positions`` and ``slots`` only. ``counters`` and ``tickets``: the step's own, cleared here (not both of them)."""
         from kgs.ops.transformer import embed_rows, embeds
 
         c = self.cfg
@@ -895,12 +888,8 @@ class ServingModel:
         ss = zero = None
         if not own:
             ss = torch.empty(m, dtype=torch.float32, device=dev)  # statistic for layer 0's qkv
-            if exact:
-                zero = stats = torch.empty((2, D.SUM_WORDS, m), dtype=torch.int64, device=dev)
-                ss_a, ss_b = stats
-            else:
-                zero = ss_a = torch.empty_like(ss)
-                ss_b = ss
+            zero = ss_a = torch.empty_like(ss)
+            ss_b = ss
         clear = tuple(t for t in (zero, counters, tickets) if t is not None)
         if embeds(self.embed):
             if keep is not None:

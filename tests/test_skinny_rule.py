@@ -97,6 +97,14 @@ def test_rows_of_the_layers_in_slices(most, rows, slabs):
     assert ServingModel._slabs_pay(M, rows) is (slabs and rows <= 48)
 
 
+def test_what_tiles_for_prompts_makes_its_own_statistics():
+    for n in (64, 128, 1024, 1280, 2048, 3072, 4096, 6144, 8192, 10240, 28672, 32000, 128256, 262144):
+        for k in (512, 1024, 1536, 2048, 2560, 4096, 5120, 8192, 9216, 12288):
+            for m in (1, 2, 8, 9, 16, 17, 24, 32, 33, 48, 64):
+                for rope in (False, True):
+                    assert D.own_takes(m, n, k, False, rope) or not D.skinny_takes(m, n, k, False, rope), (m, n, k, rope)
+
+
 def test_what_the_rules_of_slices_take_the_kernel_takes():
     """Addresses off 16 bytes are refused after the sizes and before any launch, so the entries tell here whether they take the sizes."""
     from kgs.ops import _lib

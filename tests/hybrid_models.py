@@ -34,6 +34,9 @@ MODELS = {
     # no delta layer: no recurrent state anywhere
     "attention": dict(vocab=128, width=96, streams=5, logit_softcap=8.0, norm={"eps": 1e-4}, layers=[
         latent(17, 8, 16, 24, 56, 0.4, ff=72), latent(3, 136, 144, 40, 130, 0.09)]),
+    # heads of 128 with a key head each and four taps: a decode step's delta rule in one launch
+    "step": dict(vocab=160, width=128, streams=2, logit_softcap=20.0, norm={"eps": 1e-5}, layers=[
+        delta(2, 2, 128, 128, 4, ff=96), latent(2, 32, 32, 32, 64, 0.2, ff=64), delta(3, 3, 128, 128, 4)]),
     # only delta layers: nothing in the page cache
     "recurrent": dict(vocab=111, width=72, streams=4, logit_softcap=15.0, norm={"eps": 1e-5}, layers=[
         delta(2, 1, 130, 70, 5, ff=40), delta(4, 4, 8, 33, 4, ff=56)]),

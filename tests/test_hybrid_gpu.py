@@ -90,7 +90,7 @@ def test_residual_after_every_layer(name, dtype):
 
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
-@pytest.mark.parametrize("name", ["odd", "wide"])
+@pytest.mark.parametrize("name", ["odd", "wide", "step"])
 def test_unequal_requests_in_one_batch(name, dtype):
     """Portions beside single tokens, a request that waits, one that ends and one
     that takes over its pages and slot: each as if alone."""
@@ -118,6 +118,27 @@ def test_unequal_requests_in_one_batch(name, dtype):
     assert at == lens
     for k in lens:
         check(torch.cat(out[k]), HM.oracle_logits(name, toks[k]), dtype, k)
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+def test_padded_decode_steps_of_the_one_launch_delta_rule(dtype, monkeypatch):
+    """Three sequences in a graph of four rows, the fourth on the null slot, between portions and single tokens on the same states."""
+    from kgs.serve import hybrid
+
+    launches, real = [], hybrid.delta_step
+    monkeypatch.setattr(hybrid, "delta_step", lambda *a: launches.append(a[0].shape[0]) or real(*a))
+    eng = engine("step", dtype)
+    toks = {k: tokens("step", 70, seed=k) for k in range(3)}
+    ids, out, at = [eng.open_feed() for _ in toks], {k: [] for k in toks}, dict.fromkeys(toks, 0)
+    for st in [(20, 1, 3)] + 8 * [(1, 1, 1)] + [(1, 17, 2), (30, 1, 1)] + 6 * [(1, 1, 1)]:
+        lg, r = eng.feed([(ids[k], toks[k][at[k]:at[k] + n], list(range(n))) for k, n in enumerate(st)]), 0
+        for k, n in enumerate(st):
+            out[k].append(lg[r:r + n])
+            r += n
+            at[k] += n
+    assert 4 in launches and eng.stats["graph_replays"] > 0
+    for k in toks:
+        check(torch.cat(out[k]), HM.oracle_logits("step", toks[k][:at[k]]), dtype, k)
 
 
 def test_a_batch_changes_nothing():
@@ -197,7 +218,7 @@ def _greedy_ok(name, prompts, outs, dtype):
 
 @pytest.mark.parametrize("kw", [dict(), dict(chunked_prefill=24), dict(overlap=False), dict(cuda_graphs=False),
                                 dict(pages=9, max_model_len=200)], ids=["plain", "chunked", "no-overlap", "eager", "preempt"])
-@pytest.mark.parametrize("name", ["odd", "recurrent"])
+@pytest.mark.parametrize("name", ["odd", "recurrent", "step"])
 def test_greedy_generation(name, kw):
     """The engine's own entry point, scheduler and sampler."""
     from kgs.serve import SamplingParams

@@ -3,6 +3,7 @@ import pytest
 import torch
 
 from kgs.ops import decode as D
+from kgs.ops.activation import Gate
 from kgs.ops.hyper import hyper_step
 
 pytestmark = [pytest.mark.gpu, pytest.mark.usefixtures("own_rng")]
@@ -61,6 +62,8 @@ def test_whole_products_and_gates(n, k, m):
     g, u = normed.chunk(2, 1)
     close(D.skinny_rows(x, D.PackedWeight(w, swiglu=True), sq, 1e-3), torch.nn.functional.silu(g) * u, 4)
     close(D.skinny_rows(x, D.PackedWeight(w, swiglu=True, act="gelu_tanh"), sq, 1e-3), torch.nn.functional.gelu(g, approximate="tanh") * u, 4)
+    c, v = g.clamp(max=0.5), u.clamp(-0.5, 0.5)
+    close(D.skinny_rows(x, D.PackedWeight(w, swiglu=True, act=Gate("clamped", 0.5)), sq, 1e-3), c * torch.sigmoid(1.702 * c) * (v + 1), 4)
 
 
 def test_weights_of_more_than_31_bits_of_values():
@@ -163,7 +166,7 @@ def test_layers_of_slices_as_the_others(rows, wide):
         return m.decode(tokens, ctx - 1, slots, tables, ctx).float(), logits.float(), m.cache.data.float()
 
     got, again = both(), both()
-    assert all(torch.equal(a, b) for a, b in zip(got[1:], again[1:]))  # a prompt's bits repeat
+    assert all(torch.equal(a, b) for a, b in zip(got, again))  # both steps' bits repeat
     m._slabs = m._slab_prompts = lambda rows: False
     for a, b in zip(got, both()):
         assert float((a - b).norm() / b.norm()) < 2e-2  # sums in another order, rounded to bf16 through two layers
@@ -202,3 +205,37 @@ def test_step_of_few_tokens(width, tokens):
     got = hyper_step(x, y, mix, out, in_, w, 1e-5)
     assert float((x.double() - ref).abs().max()) < 1e-5 * float(ref.abs().max())  # four products and sums in fp32
     assert bool(((got.double() - h).abs() <= 2.0 ** -8 * h.abs() + 1e-4).all())
+
+
+def _step(m, rows, seed=3):
+    """Inputs of a decode step of ``rows`` sequences, and of one prompt of as many tokens."""
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    i32 = dict(dtype=torch.int32, device="cuda")
+    ctx = torch.randint(1, 300, (rows,), generator=g, **i32)
+    tables = torch.stack([torch.randperm(127, generator=g, device="cuda")[:16].int() + 1 for _ in range(rows)])
+    tokens, slots = torch.randint(0, 512, (128,), generator=g, **i32), torch.full((rows,), -1, **i32)
+    pos = torch.arange(128, **i32)
+    return (tokens[:rows], ctx - 1, slots, tables, ctx), (tokens, pos, torch.where(pos < rows, pos + 32, -1).int(), [0], [rows], [128])
+
+
+@pytest.mark.parametrize("rows", (1, 8, 9, 16, 17, 32, 33, 48, 49, 64, 96))
+@pytest.mark.parametrize("hidden,heads", ((2048, 16), (1024, 8)))  # layers in slices from 33 rows on, and without them
+def test_small_steps_repeat_and_agree_with_the_unfused_layers(hidden, heads, rows):
+    from kgs.models.llama import LlamaConfig
+    from kgs.serve.model import ServingModel
+
+    c = LlamaConfig(hidden=hidden, layers=2, heads=heads, kv_heads=heads // 4, intermediate=12288 if hidden == 2048 else 1024, vocab=512)
+    m = ServingModel(c, device="cuda", num_pages=128, max_model_len=1024)
+    m.cache.data.normal_(generator=torch.Generator(device="cuda").manual_seed(rows))
+    decode, prompt = _step(m, rows)
+
+    def both():
+        m.cache.data[:, 1:32].zero_()
+        return m.prefill(*prompt).float(), m.decode(*decode).float(), m.cache.data.float()
+
+    got = both()
+    for _ in range(2):
+        assert all(torch.equal(a, b) for a, b in zip(got, both()))
+    m.fused_max_batch = 0
+    for a, b in zip(got, both()):
+        assert float((a - b).norm() / b.norm()) < 2e-2  # sums in another order, rounded to bf16 through two layers

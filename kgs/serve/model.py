@@ -7,7 +7,7 @@ Two step kinds, both driven by the native scheduler's plans
 * **prefill** -- the prompts of newly admitted sequences, each padded to a
   multiple of 128 tokens and concatenated (the layers drop the padding where that
   saves a tile of rows; steps of up to ``fused_max_batch`` rows, 64 at most, run the FUSED layer
-  below, of up to 256 the split tiles): every projection is one
+  below, of up to 96 the one IN SLICES where it pays, of up to 256 the split tiles): every projection is one
   :func:`kgs.ops.gemm_nt` (256x256 MFMA pipeline), RoPE + the KV-cache scatter
   is one :func:`kgs.ops.decode.rope_cache_` launch, attention is one
   flash-attention launch over all sequences' query blocks, and only the last real token of each
@@ -17,8 +17,12 @@ Two step kinds, both driven by the native scheduler's plans
   to ``fused_max_batch`` run the FUSED layer: five
   :func:`kgs.ops.decode.skinny_gemm` launches over prepacked weights whose
   epilogues carry the RMSNorms (norm weights folded into the weights, row
-  scales from sums of squares the residual-updating GEMMs accumulate), the
-  residual adds and SwiGLU -- no elementwise kernels. Larger batches run
+  scales from sums of squares that the GEMMs make of their own input, or where
+  they cannot the residual-updating ones accumulate), the residual adds and
+  SwiGLU -- no elementwise kernels. From 33 to 96 rows (:meth:`ServingModel._slabs_pay`; a
+  ``fused_max_batch`` of 32 and less turns them off) the layer runs IN SLICES: products
+  over the prepacked weights leave their K slices to the rotation and the residual adds that
+  follow. Larger batches run
   split-K four-wave tiles (:func:`kgs.ops.decode.w4x_route`, :func:`kgs.ops.decode.w4x_rule`)
   whose partial sums go into the rotation, norm or gate that follows, and
   otherwise add_rmsnorm/silu_mul and hipBLASLt, the split-K 256x256 GEMM
@@ -803,8 +807,8 @@ class ServingModel:
         return route
 
     def _slab_layers(self, tokens, positions, slots, attend, kind: str, keep=None, tickets=None):
-        """As :meth:`_fused_layers`, for 33 to 96 rows: products in K slices that the rotation and the residual adds sum, gate and up whole. The
-        rows' bits depend on nothing but their own inputs. ``(x, y, ss)``: the residual rows, from 49 rows on their norm for the head
+        """As :meth:`_fused_layers`, for 33 to 96 rows: products in K slices that the rotation and the residual adds sum, gate and up whole. At one
+        number of rows a row's bits do not depend on the others. ``(x, y, ss)``: the residual rows, from 49 rows on their norm for the head
         (else None) and else their sums of squares. Four layers 4096 wide, us a step by four-wave tiles (up to 48 rows skinny) / so: one prompt of 90
         tokens 599 / 540, of 60 615 / 509, two of 36 in all 611 / 494; 2048 wide one of 60 397 / 387."""
         from kgs.ops.transformer import embed_rows, embeds, splitk_add_rmsnorm, splitk_add_squares

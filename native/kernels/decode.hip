@@ -1885,12 +1885,7 @@ KGS_EXPORT int kgs_rope_cache_bf16(void* qkv, const float* cosv, const float* si
   return (int)hipGetLastError();
 }
 
-// Paged decode attention for one new query token per sequence. q: [B, ldq]
-// (query heads at 128-element blocks); cache: layer base; block_tables
-// [B, max_pages] int32; ctx_lens [B] int32 (>= 1). nsplit > 1 needs po
-// (B*H*nsplit*128 f32), pml (B*H*nsplit*2 f32) and cnt (B*HKV zeroed ints, left
-// zeroed); the splits are merged in the same launch.
-// kgs_rope_cache_bf16 of the partials (2 to 16, a power of two) of a weight packed with rope_rows, on rows of the raw residual stream
+// kgs_rope_cache_bf16 of the partials (1 to 16, a power of two) of a weight packed with rope_rows, on rows of the raw residual stream
 // with sums of squares sq [tokens]: scaled by their RMSNorm, over inv_k^-1 columns. bf16 pages.
 KGS_EXPORT int kgs_rope_cache_packed_bf16(void* qkv, const float* cosv, const float* sinv, const int* pos, const int* slot, void* cache,
                                          long tokens, int H, int HKV, long ld, const float* P, int nslice, const float* sq,
@@ -1917,6 +1912,11 @@ KGS_EXPORT int kgs_rope_cache_packed_bf16(void* qkv, const float* cosv, const fl
   return (int)hipGetLastError();
 }
 
+// Paged decode attention for one new query token per sequence. q: [B, ldq]
+// (query heads at 128-element blocks); cache: layer base; block_tables
+// [B, max_pages] int32; ctx_lens [B] int32 (>= 1). nsplit > 1 needs po
+// (B*H*nsplit*128 f32), pml (B*H*nsplit*2 f32) and cnt (B*HKV zeroed ints, left
+// zeroed); the splits are merged in the same launch.
 KGS_EXPORT int kgs_paged_decode_bf16_ex(const void* q, const void* cache, const int* block_tables,
                                        const int* ctx_lens, void* o, float* po, float* pml, int* cnt, int B, int H,
                                        int HKV, int hd, int max_pages, int pages_per_split, int nsplit, long ldq,

@@ -81,8 +81,8 @@ __device__ __forceinline__ double ld2_sc1(__amdgpu_buffer_rsrc_t r, unsigned off
 //               ss_in (ss_out, ss_zero) hold SUM_WORDS integers a row instead of a
 //               float: the exact sum of the workgroups' fp32 sums of squares (add_exact),
 //               so that the order in which these arrive does not show in any bit.
-//               Prompt steps use it: the same prompts give the same logits and cached
-//               keys.
+//   EPI_OWN     EPI_RMS by statistics that the product makes from x itself (add_squares),
+//               in an order of its own.
 //   EPI_ROPE    W is the fused qkv weight packed so that in every q / k head
 //               16-row tile t holds dims 8t..8t+7 then 64+8t..64+8t+7
 //               (kgs/ops/decode.py rope_rows): lane l pairs with lane l ^ 32,

@@ -225,3 +225,16 @@ def test_projections_of_rows_that_the_packed_kernels_cannot_read(n, k, gated, m)
             tol = 2.0 ** -7 * ref.abs() + 2.0 ** -7 * (ref.abs().max() if gated else 0) + 1e-4 * ref.abs().max()
             got = got.sum(0) if got.dim() == 3 else got
             assert got.shape == ref.shape and bool(((got.double() - ref).abs() <= tol).all())
+
+
+@pytest.mark.parametrize("n,k", ((2048, 8192), (2048, 11008), (8192, 8192), (5120, 13824)))  # K in two halves, off 512, and both kernels' sides
+@pytest.mark.parametrize("m", (1, 4, 9, 16))
+def test_residual_products_of_long_sums(n, k, m):
+    x, w = _operands(m, n, k, 10)
+    pw = D.PackedWeight(w)
+    ref = x.double() @ w.double().T
+    for counters in (None, torch.zeros(n // 16, dtype=torch.int32, device="cuda")):
+        for _ in range(2):  # the second call finds the first one's slabs and tickets
+            out = torch.randn(m, n, device="cuda").bfloat16()
+            want = out.double() + ref
+            _close(D.own_gemm(x, pw, out=out, resid=True, counters=counters), want)

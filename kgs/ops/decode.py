@@ -585,8 +585,8 @@ SLAB_ROWS = 96
 @lru_cache(maxsize=4096)
 def slab_split(m: int, n: int, k: int, cus: int = CUS) -> tuple[int, int] | None:
     """(W tiles a wave, K slices) of :func:`skinny_slabs`, or None: up to 96 rows of W of 64 rows a workgroup (128 from N = 4096 on),
-    in as many slices, 16 at most and of 128 at least, as leave one workgroup a CU. us at 32 rows in 4 / 8 / 16 slices: 2048x8192 12.9 / 8.8 /
-    9.1, 4096x14336 28.9 / 20.9 / 23.6, 6144x4096 11.8 / 14.5 / -."""
+    in as many slices, 16 at most and of 128 at least, as leave one workgroup a CU. us at 32 rows in 4 / 8 / 16 slices: 2048x8192 11.6 / 8.1 /
+    8.2, 4096x14336 27.0 / 19.6 / 21.6, 6144x4096 10.8 / 12.8 / -."""
     r = 2 if n >= 4096 and n % 128 == 0 else 1
     if not 0 < m <= SLAB_ROWS or n % (64 * r) or k % 128:
         return None
@@ -598,8 +598,8 @@ def slab_split(m: int, n: int, k: int, cus: int = CUS) -> tuple[int, int] | None
 
 @lru_cache(maxsize=4096)
 def slab_rows_tiles(m: int, n: int, k: int, cus: int = CUS) -> int | None:
-    """W tiles a wave of :func:`skinny_rows`, or None: two where 128 rows a workgroup are three quarters of the CUs or more (us at 64 rows with one /
-    two: 28672x4096 58.6 / 44.4, 16384x2048 16.2 / 20.9; at 32 and fewer 32000x2048 25.3 / 30.4)."""
+    """W tiles a wave of :func:`skinny_rows`, or None: two where 128 rows a workgroup are three quarters of the CUs or more (us at 48 rows with one /
+    two: 28672x4096 48.0 / 39.8, 16384x2048 14.5 / 19.1; at 32 and fewer 32000x2048 23.4 / 28.3)."""
     if not 0 < m <= SLAB_ROWS or n % 64 or k % 128:
         return None
     return 2 if m > 32 and n % 128 == 0 and 4 * (n // 128) >= 3 * cus else 1

@@ -2,20 +2,26 @@
 // ([N/16][K/32][64][8]), in K slices as fp32 partial sums P[slice][M][N] that the next launch adds (slabs), or whole, with the
 // RMSNorm and the gate of a fused layer in the epilogue (rows).
 //
-// A workgroup of four waves takes 64 R rows of W (wave w its R tiles) over one slice. W streams into registers, PF k-steps
-// ahead and past the caches; x comes by LDS-DMA in MFMA operand order, chunks of KC k-steps in NB stages, one barrier
+// A workgroup of four waves takes 64 R rows of W (wave w its R tiles) over one slice. W streams into registers, four k-steps
+// ahead and past the caches; x comes by LDS-DMA, chunks of KC k-steps in three stages, one barrier
 // each, and a k-step's fragments are read from LDS under the MFMAs of the one before. All loads are counted by hand: the
 // compiler's own schedule waits for every load in flight before it stores a chunk (twice the time). W has to lie packed: 16 rows' pieces of 64
-// bytes, straight from its rows, take half as long again (28672x4096 at 100 rows 79 us, packed 53).
+// bytes, straight from its rows, take half as long again.
+//
+// A load instruction costs by the lines that each four lanes touch: x as 8 rows of 128 bytes comes at 120 bytes a ns and CU, in MFMA operand
+// order (16 rows of 64 bytes, each lane another row than the next) at 37. And the last round of W's ring sends for nothing: fetching its
+// k-steps again was waited for at the launch's end. us at 24 / 96 rows, operand order and full last round / so: 2048x2048 in 8 slices 4.6, 6.7 /
+// 4.0, 5.6; 3072x2048 in 4 5.4, 8.1 / 4.8, 6.5; 2048x8192 in 8 8.7, 12.1 / 8.1, 10.0; 4096x14336 in 8 20.4, 26.5 / 19.5, 24.6; whole 28672x4096 at 24 / 90 41.4, 47.7 /
+// 41.0, 45.2; 16384x2048 14.3, 19.5 / 13.5, 16.6. Deeper rings (8 k-steps, 5 stages), which long sums needed before, are 2 to 5 % slower now.
 //
 // Slices: skinny adds its slices itself: each stores its part, the last one of a strip to arrive reads them all. That is 3 to 5 us at the end of a
-// launch (2048x8192 at 32 rows 15.0 us, the same product here 8.8); where the next launch passes over the output anyway it
+// launch (2048x8192 at 32 rows 15.0 us, the same product here 8.1); where the next launch passes over the output anyway it
 // reads a few MB instead. Workgroups by slices (kgs/ops/decode.py slab_split): about one a CU, and wide tiles only where N alone has enough.
 // From 33 rows on these beat the four-wave tiles of gemm_w4.h too, whose weights go through LDS; us at 64 and 90 rows, those / here:
-// 6144x4096 14.9, 20.2 / 14.0, 15.8; 4096x14336 25.1, 27.6 / 23.5, 26.4; whole: 28672x4096 51.6, 54.2 / 44.4, 47.5; 32000x4096 61 / 48; not
-// above 96 rows (128: 55.0 / 53.5, 19.0 / 18.6, 13.2 / 14.2), where reading x from LDS takes as long as the MFMAs.
-// Deep rings (8 k-steps, 5 stages) help long sums of whole products only: 28672x4096 at 64 / 90 rows 46.2 / 51.0 us by short ones, 44.4 / 47.5.
+// 6144x4096 14.9, 20.2 / 12.6, 14.2; 4096x14336 25.1, 27.6 / 21.4, 24.2; whole: 28672x4096 51.6, 54.2 / 41.5, 45.2; 32000x4096 61 / 46.
 #include "decode_common.h"
+
+#include <type_traits>
 
 namespace kgs {
 namespace dec {
@@ -43,9 +49,9 @@ __device__ __forceinline__ void wait_loads() {
   asm volatile("" ::: "memory");
 }
 
-template <int MT, int R, int OUT, int PF, int NB>
+template <int MT, int R, int OUT>
 __global__ __launch_bounds__(256, 2) void slabs(SlabArgs a) {
-  constexpr int KC = MT == 1 ? 4 : 2, XL = KC * MT / 4;  // x fragments of a wave and chunk
+  constexpr int PF = 4, NB = 3, KC = MT == 1 ? 4 : 2, XL = KC * MT / 4;  // XL: pieces of x of a wave and chunk
   static_assert(PF % KC == 0 && PF >= (NB - 2) * KC);
   __shared__ __attribute__((aligned(16))) bf16x8 xs[NB][KC * MT * 64];
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), fr = lane & 15, fq = lane >> 4;
@@ -55,12 +61,15 @@ __global__ __launch_bounds__(256, 2) void slabs(SlabArgs a) {
   const auto rw = rsrc(a.w + (long)nt0 * nkk * 512, (unsigned)(R * nkk * 1024));
   const auto rx = rsrc(a.x, (unsigned)(((M - 1) * a.ldx + a.K) * 2));
   const int wo = lane * 16;
+  // x: piece f of a chunk is 8 rows of 64 values, row f % (2 MT) * 8 + lane / 8; a row's 16-byte chunk j lies at j ^ (row / 2 % 8), so that a
+  // fragment's reads touch every bank evenly
   int xo[XL];
 #pragma unroll
   for (int i = 0; i < XL; ++i) {
-    const int f = w * XL + i, kk = f / MT, c = f % MT;
-    xo[i] = 2 * (min(16 * c + fr, M - 1) * a.ldx + (k0 + kk) * 32 + fq * 8);  // rows from M on repeat the last one: never stored
+    const int f = w * XL + i, row = f % (2 * MT) * 8 + (lane >> 3), j = (lane & 7) ^ ((row >> 1) & 7);
+    xo[i] = 2 * (min(row, M - 1) * a.ldx + k0 * 32 + f / (2 * MT) * 64 + j * 8);  // rows from M on repeat the last one: never stored
   }
+  const int ro[2] = {fr * 8 + (fq ^ (fr >> 1)), fr * 8 + ((4 + fq) ^ (fr >> 1))};  // of a fragment's 16 bytes: even and odd k-steps
   bf16x8 wf[PF][R], b[2][MT];
   auto load_w = [&](int p, int s) {
 #pragma unroll
@@ -96,35 +105,41 @@ __global__ __launch_bounds__(256, 2) void slabs(SlabArgs a) {
   asm volatile("" ::: "memory");
   int from = 0;  // stage being read
 #pragma unroll
-  for (int c = 0; c < MT; ++c) b[0][c] = xs[0][c * 64 + lane];
-  for (int s0 = 0; s0 < nsteps; s0 += PF) {
-    const int s1 = min(s0 + PF, nsteps - PF);
+  for (int c = 0; c < MT; ++c) b[0][c] = xs[0][c * 128 + ro[0]];
+  // a round of the weights' ring; the last one sends for nothing: what it would fetch again is waited for, up to 1 us of a launch
+  auto round = [&](int s0, auto more) {
+    constexpr bool MORE = decltype(more)::value;
 #pragma unroll
     for (int p = 0; p < PF; ++p) {
       const int kk = p % KC;
-      if (kk == KC - 1) {
-        // the next chunk: at least the weights of (NB - 1) KC - 1 k-steps and NB - 2 chunks were sent for after it. Every wave has read
-        // this one, so its stage is free
-        wait_loads<((NB - 1) * KC - 1) * R + (NB - 2) * XL, true>();
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
-        from = from == NB - 1 ? 0 : from + 1;
+      if (MORE || p + 1 < PF) {
+        if (kk == KC - 1) {
+          // the next chunk: at least the weights of (NB - 1) KC - 1 k-steps and NB - 2 chunks were sent for after it. Every wave has read
+          // this one, so its stage is free
+          wait_loads<((NB - 1) * KC - 1) * R + (NB - 2) * XL, true>();
+          __builtin_amdgcn_s_barrier();
+          asm volatile("" ::: "memory");
+          from = from == NB - 1 ? 0 : from + 1;
 #pragma unroll
-        for (int c = 0; c < MT; ++c) b[(p + 1) & 1][c] = xs[from][c * 64 + lane];
-        send();
-      } else {
+          for (int c = 0; c < MT; ++c) b[(p + 1) & 1][c] = xs[from][c * 128 + ro[0]];
+          if constexpr (MORE) send();
+        } else {
 #pragma unroll
-        for (int c = 0; c < MT; ++c) b[(p + 1) & 1][c] = xs[from][((kk + 1) * MT + c) * 64 + lane];
+          for (int c = 0; c < MT; ++c) b[(p + 1) & 1][c] = xs[from][((kk + 1) / 2 * MT + c) * 128 + ro[(kk + 1) & 1]];
+        }
       }
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int c = 0; c < MT; ++c)
 #pragma unroll
         for (int r = 0; r < R; ++r) acc[r][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[p][r], b[p & 1][c], acc[r][c], 0, 0, 0);
-      load_w(p, s1 + p);
+      if constexpr (MORE) load_w(p, s0 + PF + p);
       __builtin_amdgcn_sched_barrier(0);
     }
-  }
+  };
+  int s0 = 0;
+  for (; s0 + PF < nsteps; s0 += PF) round(s0, std::true_type{});
+  round(s0, std::false_type{});
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the tail's chunks land before LDS is released
 #pragma unroll
   for (int c = 0; c < MT; ++c) {
@@ -161,19 +176,17 @@ __global__ __launch_bounds__(256, 2) void slabs(SlabArgs a) {
 namespace {
 constexpr int SLAB_ROWS = 96;
 
-template <int OUT, int PF, int NB>
+template <int OUT>
 int launch_slabs(const kgs::dec::SlabArgs& a, int r, hipStream_t s) {
   using namespace kgs::dec;
   auto run = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, dim3(a.N / (64 * r) * a.ns), dim3(256), 0, s, a);
     return (int)hipGetLastError();
   };
-  if constexpr (NB == 3) {
-    if (a.M <= 16) return r == 1 ? run(slabs<1, 1, OUT, PF, NB>) : run(slabs<1, 2, OUT, PF, NB>);
-    if (a.M <= 32) return r == 1 ? run(slabs<2, 1, OUT, PF, NB>) : run(slabs<2, 2, OUT, PF, NB>);
-    if (r == 1) return a.M <= 64 ? run(slabs<4, 1, OUT, PF, NB>) : run(slabs<6, 1, OUT, PF, NB>);
-  }
-  return a.M <= 64 ? run(slabs<4, 2, OUT, PF, NB>) : run(slabs<6, 2, OUT, PF, NB>);
+  if (a.M <= 16) return r == 1 ? run(slabs<1, 1, OUT>) : run(slabs<1, 2, OUT>);
+  if (a.M <= 32) return r == 1 ? run(slabs<2, 1, OUT>) : run(slabs<2, 2, OUT>);
+  if (a.M <= 64) return r == 1 ? run(slabs<4, 1, OUT>) : run(slabs<4, 2, OUT>);
+  return r == 1 ? run(slabs<6, 1, OUT>) : run(slabs<6, 2, OUT>);
 }
 
 int slab_shape(const void* wp, const void* x, const void* y, int M, int N, int K, long ldx, int r, int ns) {
@@ -191,7 +204,7 @@ KGS_EXPORT int kgs_skinny_slabs(const void* wp, const void* x, float* p, int M, 
   const int rc = slab_shape(wp, x, p, M, N, K, ldx, r, ns);
   if (rc) return rc;
   const SlabArgs a{(const unsigned short*)x, (const unsigned short*)wp, p, M, N, K, (int)ldx, ns, 0, nullptr, 0.f, 0.f, 0.f, 0};
-  return launch_slabs<OUT_SLABS, 4, 3>(a, r, s);
+  return launch_slabs<OUT_SLABS>(a, r, s);
 }
 
 // y[M, N] (bf16, rows ldy apart) = x[M, K] . W^T as kgs_skinny_slabs in one slice; sq: of x's RMSNorm (its weight folded into W) by
@@ -206,6 +219,5 @@ KGS_EXPORT int kgs_skinny_rows(const void* wp, const void* x, void* y, int M, in
   if (ldy % 4) return KGS_ERR_ALIGN;
   if (epi & ~(EPI_SWIGLU | EPI_GELU | EPI_CLAMPED) || (epi && !gated)) return KGS_ERR_ARG;
   const SlabArgs a{(const unsigned short*)x, (const unsigned short*)wp, y, M, N, K, (int)ldx, 1, ldy, sq, 1.f / K, eps, limit, epi};
-  if (M > 32 && r == 2 && K % 256 == 0) return gated ? launch_slabs<OUT_GATED, 8, 5>(a, r, s) : launch_slabs<OUT_ROWS, 8, 5>(a, r, s);
-  return gated ? launch_slabs<OUT_GATED, 4, 3>(a, r, s) : launch_slabs<OUT_ROWS, 4, 3>(a, r, s);
+  return gated ? launch_slabs<OUT_GATED>(a, r, s) : launch_slabs<OUT_ROWS>(a, r, s);
 }

@@ -514,24 +514,32 @@ GATE_EPI = {"silu": 0, "gelu_tanh": EPI_GELU, "clamped": EPI_CLAMPED}
 
 @lru_cache(maxsize=4096)
 def few_takes(m: int, n: int, k: int, fp8: bool = False, plain: bool = False) -> bool:
-    """Whether the kernel of few rows (native/kernels/decode_few.hip) runs ``m`` rows of an ``[n, k]`` weight: up to 16 of bf16 weights,
-    32 of a product without a norm or a rotation (``plain``), which also takes any K of 64."""
+    """Whether the kernel of few rows (native/kernels/decode_few.hip) runs ``m`` rows of an ``[n, k]`` weight: up to 16 of bf16 weights (:func:`few_wide` has
+    more), 32 of a product without a norm or a rotation (``plain``), which also takes any K of 64."""
     return not fp8 and 0 < m <= 32 and bool(_lib.lib().kgs_skinny_few_ok(m, n, k, plain))
+
+
+@lru_cache(maxsize=4096)
+def few_wide(m: int, n: int, k: int) -> bool:
+    """Whether it takes 17 to 32 rows with a norm or a rotation too, and is the better one there: K of 1024 up to 8192, up to 16384 rows of W (us at 24 rows,
+    others / so: 6144x4096 20.0 / 12.7, 2048x2048 7.6 / 5.8, 16384x2048 16.3 / 14.9; at 32 4096x14336 27.8 / 31.9, 28672x4096 42.6 / 46.6)."""
+    return 16 < m <= 32 and n <= 16384 and k <= 8192 and bool(_lib.lib().kgs_skinny_few_wide_ok(m, n, k))
 
 
 @lru_cache(maxsize=4096)
 def few_route(m: int, n: int, k: int, plain: bool = False) -> bool:
     """Whether the kernel of few rows is the better one, of those that take these rows; us of plain products, weights from HBM, few / others.
 
-    Beside :func:`skinny_gemm`: up to 8 rows where W is not much wider than the CUs are many -- its workgroups are short, and a third
-    round of them costs more than skinny's long ones (12288x1024 at 1 row 6.6 / 7.0, 64000x1024 29 / 24.8, 24576x2048 19.6 / 20.4, 64000x2048
-    48.5 / 46.2 and at 8 rows 49 / 45.2), beyond that from K = 3584 on up to 4 rows and where K is a multiple of 4096, whose strips lie at
-    multiples of 128 KB, which skinny's four waves read at once (32000x4096 at 8 rows 44.8 / 48.3, 32000x5120 at 8 57 / 55). Not where W has as many strips
+    Beside :func:`skinny_gemm`: up to 8 rows where W is not much wider than the CUs are many (64000x1024 at 1 row 29 / 24.8, 64000x2048
+    48.5 / 46.2, 32000x2048 23.8 / 23.0), beyond that from K = 3584 on up to 4 rows and where K is a multiple of 4096, whose strips lie at
+    multiples of 128 KB, which skinny's four waves read at once (28672x4096 at 8 rows 36.2 / 41.6, 32000x4096 40.0 / 45.2). Not where W has as many strips
     at multiples of 256 KB as CUs (4096x8192 at 1 row 16.0 / 14.3, in two tiles a workgroup 8192x8192 at 8 31.8 / 28.3), nor short
-    strips of long K, which skinny reads in slices (1024x14336 at 8 rows 16.9 / 13.4), nor a few more strips than CUs in four waves each (5120x13824 at
+    strips of long K, which skinny reads in slices (1024x14336 at 8 rows 16.9 / 13.4), nor a few more strips than CUs (5120x13824 at
     4 rows 30.3 / 28.0). Up to 16 rows while x is short, which every workgroup
-    reads whole (6144x4096 at 16 13.7 / 16.2, but 2048x8192 14.4 / 12.6, 8192x7168 at 12 27 / 32, 2560x6144 at 16 10.5 / 9.7); up to 32
-    for short K that does not divide by 1024 (24 rows: 2048x768 4.7 / 7.6, 4096x1536 6.7 / 9.6, but 2048x1024 5.5 / 4.6).
+    reads whole (6144x4096 at 16 11.0 / 13.6, but 2048x8192 12.7 / 11.6, 8192x7168 at 12 27 / 32), and of wide W where K is neither short nor long
+    (28672x4096 at 12 37.8 / 42.1, 16384x2048 at 16 12.4 / 14.5, 32000x4096 42.0 / 46.2, but 32000x2048 26.7 / 23.5); up to 32
+    for short K that does not divide by 1024 (24 rows: 2048x768 3.8 / 7.6, 4096x1536 6.7 / 9.6, but 2048x1024 5.5 / 4.6) and, with x by LDS,
+    for K of 2048 to 8192 up to 8192 rows of W (24 rows: 2048x2048 5.5 / 6.9, 6656x2048 7.7 / 9.9).
 
     Beside the library, for sizes that skinny does not take: as long as neither x nor the grid is long (832x2048 at 1 row 3.6 / 7.9; 896x4864
     at 24 25.5 / 16.6, 13824x768 at 16 1.31 times its time, 6144x11008 1.15 times)."""
@@ -542,13 +550,13 @@ def few_route(m: int, n: int, k: int, plain: bool = False) -> bool:
             return True
         return n <= 32768 if m <= 8 else n <= 8192 and (n <= 4096 or k <= 8192) if m <= 16 else n <= 4096 and k <= 2048
     if m > 16:
-        return k <= 1536 and n <= 4096 and k % 1024 != 0
+        return (k <= 1536 and n <= 4096 and k % 1024 != 0) or (k >= 2048 and n <= 8192 and few_wide(m, n, k))
     if k % 8192 == 0 and ((n == 4096 and m <= 8) or (n == 8192 and m > 4)):
         return False
     if n <= 2048:
         return k <= (8192 if m <= 8 else 5120) or (k < 8192 and k % 1024 != 0)
     if m > 8:
-        return n <= 8192 and m * k < 96 << 10
+        return m * k < 96 << 10 if n <= 8192 else k >= 2048 and (n <= 16384 or k >= 4096) and n <= 32768 and k <= 4096
     if 4096 < n <= 5120 and k > 8192 and k % 1024:
         return False
     if n <= 24576:
@@ -573,6 +581,8 @@ def own_gemm(x: torch.Tensor, w: PackedWeight, out: torch.Tensor | None = None, 
     """:func:`skinny_gemm` with ``norm`` or ``resid``, by :func:`skinny_few` where that is the better one (:func:`few_route`)."""
     m, k = x.shape
     plain = not norm and rope is None
+    if not w.fp8 and few_wide(m, w.n, k):
+        return skinny_few(x, w, out, norm, resid, eps, rope)
     if m <= 16 and not w.fp8 and (few_route(m, w.n, k, plain) or (few_takes(m, w.n, k, False, plain) and not (
             skinny_takes(m, w.n, k) if plain else _own_by_skinny(m, w.n, k, False, bool(w.rope))))):
         return skinny_few(x, w, out, norm, resid, eps, rope)
@@ -734,7 +744,7 @@ def skinny_few(x: torch.Tensor, w: PackedWeight, out: torch.Tensor | None = None
     if x.dtype != torch.bfloat16 or not x.is_cuda or x.dim() != 2 or x.stride(1) != 1:
         raise ValueError("x must be a row-major bf16 GPU matrix")
     m, k = x.shape
-    if k != w.k or not few_takes(m, w.n, k, w.fp8, not norm and rope is None):
+    if k != w.k or not (few_takes(m, w.n, k, w.fp8, not norm and rope is None) or (not w.fp8 and few_wide(m, w.n, k))):
         raise ValueError(f"not a product of few rows: x {tuple(x.shape)}, W [{w.n}, {w.k}]")
     if (rope is not None) != bool(w.rope) or (resid and (rope is not None or w.swiglu)):
         raise ValueError("rope= needs a rope-packed qkv weight and vice versa; resid a plain one")

@@ -197,9 +197,11 @@ __global__ __launch_bounds__(256, (MT * KC_ > 32 || R * MT >= 16) ? 1 : 2) void 
 
   [[maybe_unused]] double own[OWN && KIN ? MT : 1] = {};  // OWN: this lane's part of its rows' sums of squares, of all column tiles (KIN) or the wave's own
 
-  // Every load below is unconditional (indices clamped to the last step /
-  // chunk: a few redundant L2-hit reloads at the tail) so hipcc can count
-  // vmcnt through the loop instead of draining the ring before each MFMA.
+  // Loads in the loops below are unconditional, so that hipcc can count vmcnt instead of draining the ring before
+  // each MFMA. The last round, which sends for nothing more, stands behind them (PEEL): the last k-steps fetched again
+  // were waited for at the end. us, fetched again / so: 3072x2048 at 48 rows 11.1 / 10.2, 2048x8192 at 24 15.0 / 13.7, 16384x2048 at 32
+  // 16.3 / 14.9, 32000x2048 at 16 24.8 / 23.5. Eight tiles a wave and more spill, and four (K not split) are 3 % slower so at long K: these keep the clamped loads.
+  constexpr bool PEEL = R * MT < (KIN ? 8 : 4);
   WFrag<W8> wf[PF][R];
   // OWN, KIN: the k-steps' order is fixed, else the compiler gives up the ring for the statistic's sake (84 registers instead of 167, every load in
   // flight waited for several times a chunk). us at 24 rows, given statistics / own, loose / own, fixed: 8192x2048 11.7 / 15.5 / 10.9, 3072x2048
@@ -228,17 +230,22 @@ __global__ __launch_bounds__(256, (MT * KC_ > 32 || R * MT >= 16) ? 1 : 2) void 
       bf16x8 xf[PF];
 #pragma unroll
       for (int p = 0; p < PF; ++p) xf[p] = *(const bf16x8*)(xr + p * 32);
-      for (int s0 = 0; s0 < nsteps; s0 += PF) {
+      auto round = [&](int s0, auto more) {
 #pragma unroll
         for (int p = 0; p < PF; ++p) {
 #pragma unroll
           for (int r = 0; r < R; ++r) acc[r][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(dequant8(wf[p][r], wsc[r]), xf[p], acc[r][0], 0, 0, 0);
-          const int sn = min(s0 + p + PF, nsteps - 1);
+          if constexpr (decltype(more)::value) {
+            const int sn = s0 + p + PF;
 #pragma unroll
-          for (int r = 0; r < R; ++r) wf[p][r] = __builtin_nontemporal_load(wrow[r] + (long)sn * 64);
-          xf[p] = *(const bf16x8*)(xr + sn * 32);
+            for (int r = 0; r < R; ++r) wf[p][r] = __builtin_nontemporal_load(wrow[r] + (long)sn * 64);
+            xf[p] = *(const bf16x8*)(xr + sn * 32);
+          }
         }
-      }
+      };
+      int s0 = 0;
+      for (; s0 + PF < nsteps; s0 += PF) round(s0, std::true_type{});
+      round(s0, std::false_type{});
     } else {
       const unsigned short* xr[MT];
 #pragma unroll
@@ -254,7 +261,7 @@ __global__ __launch_bounds__(256, (MT * KC_ > 32 || R * MT >= 16) ? 1 : 2) void 
         for (int c = 0; c < MT; ++c) xf[p][c] = *(const bf16x8*)(xr[c] + p * 32);
         if constexpr (PINNED) __builtin_amdgcn_sched_barrier(0);
       }
-      for (int s0 = 0; s0 < nsteps; s0 += PF) {
+      auto round = [&](int s0, auto more) {
 #pragma unroll
         for (int p = 0; p < PF; ++p) {
 #pragma unroll
@@ -269,14 +276,19 @@ __global__ __launch_bounds__(256, (MT * KC_ > 32 || R * MT >= 16) ? 1 : 2) void 
 #pragma unroll
             for (int c = 0; c < MT; ++c) own[c] = add_squares(own[c], xf[p][c]);
           }
-          const int sn = min(s0 + p + PF, nsteps - 1);
+          if constexpr (decltype(more)::value) {
+            const int sn = PEEL ? s0 + p + PF : min(s0 + p + PF, nsteps - 1);
 #pragma unroll
-          for (int r = 0; r < R; ++r) wf[p][r] = __builtin_nontemporal_load(wrow[r] + (long)sn * 64);
+            for (int r = 0; r < R; ++r) wf[p][r] = __builtin_nontemporal_load(wrow[r] + (long)sn * 64);
 #pragma unroll
-          for (int c = 0; c < MT; ++c) xf[p][c] = *(const bf16x8*)(xr[c] + sn * 32);
+            for (int c = 0; c < MT; ++c) xf[p][c] = *(const bf16x8*)(xr[c] + sn * 32);
+          }
           if constexpr (PINNED) __builtin_amdgcn_sched_barrier(0);
         }
-      }
+      };
+      int s0 = 0;
+      for (; s0 + (PEEL ? PF : 0) < nsteps; s0 += PF) round(s0, std::true_type{});
+      if constexpr (PEEL) round(s0, std::false_type{});
     }
     // the four K quarters of the strip: waves 1-3 hand theirs to wave 0 (slot 0
     // of xs stays free for the split-K flag); summed in wave order
@@ -311,8 +323,9 @@ __global__ __launch_bounds__(256, (MT * KC_ > 32 || R * MT >= 16) ? 1 : 2) void 
   store_x(0);
   __syncthreads();
   const int nchunks = chunks_per_split;
-  for (int chunk = 0; chunk < nchunks; ++chunk) {
-    load_x(min(chunk + 1, nchunks - 1));
+  auto round = [&](int chunk, auto more) {
+    constexpr bool MORE = decltype(more)::value;
+    if constexpr (MORE) load_x(PEEL ? chunk + 1 : min(chunk + 1, nchunks - 1));
     const bf16x8* xb = xs[chunk & 1] + lane;
 #pragma unroll
     for (int kk = 0; kk < KC; ++kk) {
@@ -333,13 +346,20 @@ __global__ __launch_bounds__(256, (MT * KC_ > 32 || R * MT >= 16) ? 1 : 2) void 
         for (int r = 0; r < R; ++r)
           acc[r][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wdq[r], bfrag, acc[r][c], 0, 0, 0);
       }
-      const long sn = min(chunk * KC + kk + PF, nsteps - 1);
+      if (MORE || kk + PF < KC) {
+        const long sn = PEEL ? chunk * KC + kk + PF : min(chunk * KC + kk + PF, nsteps - 1);
 #pragma unroll
-      for (int r = 0; r < R; ++r) wf[p][r] = __builtin_nontemporal_load(wrow[r] + sn * 64);
+        for (int r = 0; r < R; ++r) wf[p][r] = __builtin_nontemporal_load(wrow[r] + sn * 64);
+      }
     }
-    store_x((chunk + 1) & 1);
-    __syncthreads();
-  }
+    if constexpr (MORE) {
+      store_x((chunk + 1) & 1);
+      __syncthreads();
+    }
+  };
+  int chunk = 0;
+  for (; chunk + PEEL < nchunks; ++chunk) round(chunk, std::true_type{});
+  if constexpr (PEEL) round(chunk, std::false_type{});
   if constexpr (OWN) {
     const double s = wsum16(own[0]);
     if (w < MT && lane < 16) stat[0][16 * w + lane] = s;

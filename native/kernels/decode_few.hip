@@ -1,24 +1,31 @@
 // Skinny products of up to 16 rows (plain ones 32): y[M, N] = x[M, K] . W^T, W packed as for decode.hip's skinny
 // ([N/16][K/32][64][8]), with that kernel's epilogues and one statistic of its own.
 //
-// A workgroup of NW waves takes R 16-row tiles of W; the waves share out K, stream their part of W and of x (in
-// MFMA operand order, straight from memory) through a ring of PF k-steps and add their sums in LDS, in the order of the waves.
-// Loads are buffer loads, so that a step waits for exactly its own.
+// A workgroup of NW waves takes R 16-row tiles of W; the waves share out K, stream their part of W and of x through a ring of PF k-steps and add
+// their sums in LDS, in the order of the waves. Loads are buffer loads, so that a step waits for exactly its own. The last round sends for nothing:
+// the last k-steps fetched again, as the ring did, were waited for at the end of the launch, 0.5 to 1 us of a short one and a
+// tenth of a long one.
+//
+// x: up to 16 rows straight from memory in MFMA operand order. There a load instruction costs by its distinct rows (137 bytes a ns and CU at 1 row, 60
+// at 8, 37 at 16, where whole lines come at 120), so that from 17 rows on (LX) x comes by LDS-DMA, 8 rows of 128 bytes a piece, into stages of
+// the wave's own: no barrier. Below, LDS on the way costs more than it gives (us at 16 rows direct / so: 2048x2048 4.8 / 4.9, 4096x4096 8.1 / 8.9).
 //
 // OWN: the RMSNorm of x from x itself. Every wave holds its part of all rows anyway and adds up its squares (add_squares). Where the producer of x adds them up instead, 256 workgroups' atomics
 // meet on one address, 12.5 ns each, at the end of a launch that nothing hides: a layer's o and down took 1.6 us longer at 1
 // row, 2.0 at 16. Nothing here depends on the order in which workgroups arrive.
 //
-// Bound by memory where W is large (28672 x 4096 at 1 row 39 us, 6.0 TB/s), else by the launch and one trip through
-// memory, the ring and LDS (4096 x 4096 7.8 us). The split by the number of strips (few_split): short grids need the waves,
-// long ones lose by them (us at 1 row with 8 / 4 / 2 waves: 2048x8192 9.1 / 12.5 / 11.5, 4096x14336 20.8 / 21.1 / 22.7, 6144x4096 11.9 /
-// 10.2 / 10.2, 28672x4096 42.0 / 40.6 / 39.8, 32000x4096 48.3 / 45.9 / 44.5). Two tiles a workgroup from 5 rows on where one makes
-// a little more than one round of the CUs: every workgroup reads all of x (6144x4096 at 12 rows 12.7 / 12.1). Any K of 64, for products that
-// were the library's: us at 1 / 32 rows, library / here: 2048x128 3.3, 3.8 / 2.1, 2.5; 2048x768 5.0, 6.8 / 2.8, 5.3; 832x2048 7.9 / 3.6 at 1 row. From 17
-// rows on the way of x bounds K (kgs/ops/decode.py few_route).
+// Bound by memory where W is large (28672 x 4096 at 1 row 36.4 us, 6.5 TB/s; 40.6 before), else by the launch and one trip through
+// memory and the ring (4096 x 4096 7.0 us, before 7.5; 2048 x 2048 3.6, 4.3). The split (few_split): few waves with long rings, whose loads are all in flight
+// at once and whose sums are soon added -- us at 8 rows with 8 / 4 / 2 / 1 waves, as long rings as fit: 2048x2048 4.3 / 4.2 / 4.0 / 4.6, 4096x4096 7.4 / 7.2 /
+// 7.0 / 8.4, 6144x4096 12.4 / 11.7 / 10.9 / 10.2, 16384x2048 12.3 / 13.6 / 12.4 / 12.2, 28672x4096 36.2 / 39.7 / 36.6 / 36.2; eight for long sums of up to 4 rows (4096x14336 at 1
+// row 18.5, by two 19.8; at 8 20.7, 19.2). Two tiles a workgroup where x counts: 6144x4096 at 16 rows 12.1 / 11.0, 28672x4096 at 16 40.8 / 40.3. At 24 / 32 rows, skinny / here:
+// 6144x4096 19.7, 19.8 / 12.6, 13.2; 4096x4096 12.3, 13.7 / 9.1, 10.1; 2048x2048 7.4, 8.1 / 5.5, 6.0; 12288x2048 16.0, 15.9 / 12.3, 12.7. Any K of 64, for products that
+// were the library's: us at 1 / 32 rows, library / here: 2048x128 3.3, 3.8 / 2.0, 2.5; 2048x768 5.0, 6.8 / 2.6, 4.0; 832x2048 7.9 / 3.3 at 1 row. Which products come here:
+// kgs/ops/decode.py few_route, few_wide.
 #include "decode_common.h"
 
 #include <type_traits>
+#include <utility>
 
 namespace kgs {
 namespace dec {
@@ -48,12 +55,23 @@ __device__ __forceinline__ bf16x8 ld_frag(__amdgpu_buffer_rsrc_t r, int v, int s
   return __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(r, v, s, AUX));
 }
 
-// MT column tiles of 16 rows of x; ROPE and OWN of one
-template <int R, int MT, int NW, int PF, bool ROPE, bool OWN>
+__device__ __forceinline__ void dma16(__amdgpu_buffer_rsrc_t r, void* lds, int v, int s) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (KGS_LDS void*)lds, 16, v, s, 0, 0);
+}
+
+template <int... I, typename F>
+__device__ __forceinline__ void each_of(std::integer_sequence<int, I...>, F&& f) { (f(std::integral_constant<int, I>{}), ...); }
+template <int N, typename F>
+__device__ __forceinline__ void each(F&& f) { each_of(std::make_integer_sequence<int, N>{}, f); }
+
+// MT column tiles of 16 rows of x. LX: x by LDS, in XP pieces of 8 rows of 64 values for two k-steps; else straight from memory in operand order
+template <int R, int MT, int NW, int PF, bool LX, bool ROPE, bool OWN>
 __global__ __launch_bounds__(64 * NW) void few(FewArgs a) {
-  static_assert(MT == 1 || (!ROPE && !OWN && R == 1));
+  static_assert(!LX || PF % 2 == 0);
+  constexpr int XP = LX ? 2 * MT : 0, NX = PF / 2 + 1;  // NX: stages of two k-steps of x, a wave's own: no barrier
   __shared__ __attribute__((aligned(16))) f32x4v red[NW * R * MT * 64];
-  __shared__ double stat[OWN ? NW : 1][16];
+  __shared__ double stat[OWN ? NW : 1][16 * MT];
+  __shared__ __attribute__((aligned(16))) bf16x8 xs[LX ? NW * NX * XP * 64 : 1];
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), fr = lane & 15, fq = lane >> 4;
   const int M = a.M, nkk = a.K / 32, nsteps = nkk / NW, kk0 = w * nsteps, nt0 = blockIdx.x * R;
   if constexpr (!ROPE && !OWN) {
@@ -66,124 +84,199 @@ __global__ __launch_bounds__(64 * NW) void few(FewArgs a) {
   const auto rw = rsrc(a.w + (long)nt0 * nkk * 512, (unsigned)(R * nkk * 1024));
   const auto rx = rsrc(a.x, (unsigned)(((M - 1) * a.ldx + a.K) * 2));
   const int wo = lane * 16;
-  int xo[MT];
+  // rows from M on repeat the last one: never stored. By LDS: row 8 j + lane / 8 of piece j, its 16-byte chunk c at c ^ (row / 2 % 8), so that a
+  // fragment's reads touch every bank evenly
+  int xo[LX ? XP : MT];
+  if constexpr (!LX) {
 #pragma unroll
-  for (int c = 0; c < MT; ++c) xo[c] = 2 * (min(16 * c + fr, M - 1) * a.ldx + fq * 8);  // rows from M on repeat the last one: never stored
-  bf16x8 wf[PF][R], xf[PF][MT];
-  auto load = [&](int p, int s) {  // k-step s of this wave; W past the caches, it comes once
+    for (int c = 0; c < MT; ++c) xo[c] = 2 * (min(16 * c + fr, M - 1) * a.ldx + fq * 8);
+  } else {
+#pragma unroll
+    for (int j = 0; j < XP; ++j) {
+      const int row = 8 * j + (lane >> 3);
+      xo[j] = 2 * (min(row, M - 1) * a.ldx + ((lane & 7) ^ ((row >> 1) & 7)) * 8);
+    }
+  }
+  bf16x8* const xw = xs + (LX ? w * NX * XP * 64 : 0);
+  const int ro[2] = {fr * 8 + (fq ^ (fr >> 1)), fr * 8 + ((4 + fq) ^ (fr >> 1))};  // a fragment's 16 bytes: even and odd k-steps
+  bf16x8 wf[PF][R], xf[LX ? 2 : PF][MT];
+  auto load_w = [&](int p, int s) {  // k-step s of this wave; W past the caches, it comes once
 #pragma unroll
     for (int r = 0; r < R; ++r) wf[p][r] = ld_frag<2>(rw, wo, (r * nkk + kk0 + s) * 1024);
+  };
+  auto load_x = [&](int p, int s) {
 #pragma unroll
     for (int c = 0; c < MT; ++c) xf[p][c] = ld_frag<0>(rx, xo[c], (kk0 + s) * 64);
   };
+  auto send_x = [&](int stage, int s) {
 #pragma unroll
-  for (int p = 0; p < PF; ++p) load(p, p);
+    for (int j = 0; j < XP; ++j) dma16(rx, xw + (stage * XP + j) * 64, xo[j], (kk0 + s) * 64);
+  };
+#pragma unroll
+  for (int p = 0; p < PF; ++p) {
+    if constexpr (!LX) {
+      load_w(p, p);
+      load_x(p, p);
+    } else {
+      if (p % 2 == 0) {
+        __builtin_amdgcn_sched_barrier(0);
+        send_x(p / 2, p);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      load_w(p, p);
+    }
+  }
 
-  // what the epilogue needs, under the main loop's way: old values or rotation of tile (r, c) = (w / MT, w % MT)
-  const int nt = nt0 + (w < R * MT ? w / MT : 0), m = 16 * (w % MT) + fr;
-  unsigned short* const yt = a.y + (long)min(m, M - 1) * a.ldy + 16 * nt + 4 * fq;
+  // what the epilogue needs of its first tile (r, c) = (w / MT, w % MT), under the main loop's way: old values or rotation
+  auto out = [&](int t) { return a.y + (long)min(16 * (t % MT) + fr, M - 1) * a.ldy + 16 * (nt0 + t / MT) + 4 * fq; };
+  const int t0 = w < R * MT ? w : 0;
   uint2 old = make_uint2(0, 0);
-  if (!ROPE && (a.mode & EPI_RESID) && w < R * MT) old = *(const uint2*)yt;
+  if (!ROPE && (a.mode & EPI_RESID) && w < R * MT) old = *(const uint2*)out(t0);
   float cs[4], sn[4];
   int slot = -1;
-  if constexpr (ROPE) {
-    const int mr = min(fr, M - 1), p = a.pos[mr], t = nt & 7, dd = 8 * t + 4 * (fq & 1);  // dim within the rotated half
-    slot = fr < M ? a.slot[mr] : -1;
+  auto turn = [&](int t) {
+    const int m = 16 * (t % MT) + fr, mr = min(m, M - 1), p = a.pos[mr], dd = 8 * ((nt0 + t / MT) & 7) + 4 * (fq & 1);  // dim within the rotated half
+    slot = m < M ? a.slot[mr] : -1;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       cs[i] = a.cosv[(long)p * (HD / 2) + dd + i];
       sn[i] = a.sinv[(long)p * (HD / 2) + dd + i];
     }
-  }
+  };
+  if constexpr (ROPE) turn(t0);
 
   f32x4v acc[R][MT];
-  [[maybe_unused]] double own = 0.;
+  [[maybe_unused]] double own[MT] = {};
 #pragma unroll
   for (int r = 0; r < R; ++r)
 #pragma unroll
     for (int c = 0; c < MT; ++c) acc[r][c] = f32x4v{0.f, 0.f, 0.f, 0.f};
-  for (int s0 = 0; s0 < nsteps; s0 += PF) {
-    const int next = min(s0 + PF, nsteps - PF);  // past the end: the last round again, from the caches
+  auto step = [&](int p, const bf16x8 (&x)[MT]) {
 #pragma unroll
-    for (int p = 0; p < PF; ++p) {
-      __builtin_amdgcn_sched_barrier(0);
+    for (int r = 0; r < R; ++r)
 #pragma unroll
-      for (int r = 0; r < R; ++r)
+      for (int c = 0; c < MT; ++c) acc[r][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[p][r], x[c], acc[r][c], 0, 0, 0);
+    if constexpr (OWN) {
 #pragma unroll
-        for (int c = 0; c < MT; ++c) acc[r][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[p][r], xf[p][c], acc[r][c], 0, 0, 0);
-      if constexpr (OWN) own = add_squares(own, xf[p][0]);
-      load(p, next + p);
+      for (int c = 0; c < MT; ++c) own[c] = add_squares(own[c], x[c]);
     }
-  }
+  };
+  [[maybe_unused]] int from = 0, to = NX - 1;  // stages being read and sent for
+  // a round of the ring; the last one sends for nothing: what it would fetch again is waited for, up to 1 us of a launch
+  auto round = [&](int s0, auto more) {
+    constexpr bool MORE = decltype(more)::value;
+    each<PF>([&](auto pc) {
+      constexpr int p = decltype(pc)::value;
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (!LX) {
+        step(p, xf[p]);
+        if constexpr (MORE) {
+          load_w(p, s0 + PF + p);
+          load_x(p, s0 + PF + p);
+        }
+      } else {
+        if constexpr (p % 2 == 0) {
+          if constexpr (MORE) {
+            send_x(to, s0 + PF + p);  // into the stage whose fragments the step before last took
+            to = to == NX - 1 ? 0 : to + 1;
+          }
+          // these k-steps' pieces: the weights of two k-steps, and the pieces and weights of the ring's others, were sent for after them
+          constexpr int AFTER = PF / 2 - (MORE ? 0 : p / 2 + 1);
+          asm volatile("s_waitcnt vmcnt(%0)" ::"n"(AFTER * (XP + 2 * R) + (MORE ? 0 : 2 * R)) : "memory");
+          const bf16x8* st = xw + from * XP * 64;
+          from = from == NX - 1 ? 0 : from + 1;
+#pragma unroll
+          for (int e = 0; e < 2; ++e)
+#pragma unroll
+            for (int c = 0; c < MT; ++c) xf[e][c] = st[c * 128 + ro[e]];
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        step(p, xf[p % 2]);
+        if constexpr (MORE) load_w(p, s0 + PF + p);
+      }
+    });
+  };
+  int s0 = 0;
+  for (; s0 + PF < nsteps; s0 += PF) round(s0, std::true_type{});
+  round(s0, std::false_type{});
 #pragma unroll
   for (int r = 0; r < R; ++r)
 #pragma unroll
     for (int c = 0; c < MT; ++c) red[((w * R + r) * MT + c) * 64 + lane] = acc[r][c];
   if constexpr (OWN) {
-    own = wsum16(own);
-    if (fq == 0) stat[w][fr] = own;
+#pragma unroll
+    for (int c = 0; c < MT; ++c) {
+      own[c] = wsum16(own[c]);
+      if (fq == 0) stat[w][16 * c + fr] = own[c];
+    }
   }
   __syncthreads();
-  if (w >= R * MT) return;
-
-  // lane: row m of x, rows 16 nt + 4 fq + i of W
-  f32x4v v = red[w * 64 + lane];
-#pragma unroll
-  for (int j = 1; j < NW; ++j) v += red[(j * R * MT + w) * 64 + lane];
-  if constexpr (OWN) {
-    double ss = stat[0][fr];
-#pragma unroll
-    for (int j = 1; j < NW; ++j) ss += stat[j][fr];
-    v *= rsqrtf((float)ss * a.inv_k + a.eps);
-  }
-  const bool in = m < M;
-  if constexpr (ROPE) {
-    const int hh = nt >> 3, t = nt & 7;  // head and tile within it
-    const bool rot = hh < a.H + a.HKV;
-    f32x4v vb, pb;  // this lane's and its partner's (lane ^ 32) values, rounded to bf16
-#pragma unroll
-    for (int i = 0; i < 4; ++i) vb[i] = bf2f(f2bf(v[i]));
-#pragma unroll
-    for (int i = 0; i < 4; ++i) pb[i] = lane_xor32(vb[i]);
-    if (!in) return;
-    const int d0 = rot ? (fq < 2 ? 8 * t + 4 * fq : 64 + 8 * t + 4 * (fq - 2)) : 16 * t + 4 * fq;
-    f32x4v o = vb;
-    if (rot) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) o[i] = fq < 2 ? rope_lo(vb[i], pb[i], cs[i], sn[i]) : rope_hi(pb[i], vb[i], cs[i], sn[i]);
+  for (int t = w; t < R * MT; t += NW) {
+    const int nt = nt0 + t / MT, m = 16 * (t % MT) + fr;
+    if (R * MT > NW && t != w) {
+      if (!ROPE && (a.mode & EPI_RESID)) old = *(const uint2*)out(t);
+      if constexpr (ROPE) turn(t);
     }
-    const uint2 pk{pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3])};
-    *(uint2*)(a.y + (long)fr * a.ldy + hh * HD + d0) = pk;
-    if (hh < a.H || slot < 0) return;
-    const int page = slot / PAGE, tau = slot - page * PAGE;
-    const bool isv = hh >= a.H + a.HKV;
-    const int kvh = isv ? hh - a.H - a.HKV : hh - a.H;
-    unsigned short* pg = a.cache + (((long)page * a.HKV + kvh) * 2 + (isv ? 1 : 0)) * PAGE_ELEMS;
-    if (!isv) {
-      *(uint2*)(pg + kv_k_index(tau, d0)) = pk;  // 4 consecutive dims: one 8-B run of the K fragment
-    } else {
-      pg[kv_v_index(tau, d0 + 0)] = (unsigned short)(pk.x & 0xffff);
-      pg[kv_v_index(tau, d0 + 1)] = (unsigned short)(pk.x >> 16);
-      pg[kv_v_index(tau, d0 + 2)] = (unsigned short)(pk.y & 0xffff);
-      pg[kv_v_index(tau, d0 + 3)] = (unsigned short)(pk.y >> 16);
-    }
-  } else if (a.mode & EPI_SWIGLU) {
-    f32x4v u, o;
+    // lane: row m of x, rows 16 nt + 4 fq + i of W
+    f32x4v v = red[t * 64 + lane];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) u[i] = lane_xor32(v[i]);
+    for (int j = 1; j < NW; ++j) v += red[(j * R * MT + t) * 64 + lane];
+    if constexpr (OWN) {
+      const int col = 16 * (t % MT) + fr;
+      double ss = stat[0][col];
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      o[i] = (a.mode & EPI_CLAMPED) ? gate_clamped(v[i], u[i], a.limit)
-             : ((a.mode & EPI_GELU) ? gate_act<GATE_GELU>(v[i]) : gate_act<GATE_SILU>(v[i])) * u[i];
-    if (in && fq < 2) *(uint2*)(a.y + (long)m * a.ldy + 8 * nt + 4 * fq) = uint2{pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3])};
-  } else if (in) {
-    if (a.mode & EPI_RESID) {
-      v[0] += bf2f(old.x & 0xffff);
-      v[1] += bf2f(old.x >> 16);
-      v[2] += bf2f(old.y & 0xffff);
-      v[3] += bf2f(old.y >> 16);
+      for (int j = 1; j < NW; ++j) ss += stat[j][col];
+      v *= rsqrtf((float)ss * a.inv_k + a.eps);
     }
-    *(uint2*)yt = uint2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+    const bool in = m < M;
+    if constexpr (ROPE) {
+      const int hh = nt >> 3, i8 = nt & 7;  // head and tile within it
+      const bool rot = hh < a.H + a.HKV;
+      f32x4v vb, pb;  // this lane's and its partner's (lane ^ 32) values, rounded to bf16
+#pragma unroll
+      for (int i = 0; i < 4; ++i) vb[i] = bf2f(f2bf(v[i]));
+#pragma unroll
+      for (int i = 0; i < 4; ++i) pb[i] = lane_xor32(vb[i]);
+      if (!in) continue;
+      const int d0 = rot ? (fq < 2 ? 8 * i8 + 4 * fq : 64 + 8 * i8 + 4 * (fq - 2)) : 16 * i8 + 4 * fq;
+      f32x4v o = vb;
+      if (rot) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) o[i] = fq < 2 ? rope_lo(vb[i], pb[i], cs[i], sn[i]) : rope_hi(pb[i], vb[i], cs[i], sn[i]);
+      }
+      const uint2 pk{pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3])};
+      *(uint2*)(a.y + (long)m * a.ldy + hh * HD + d0) = pk;
+      if (hh < a.H || slot < 0) continue;
+      const int page = slot / PAGE, tau = slot - page * PAGE;
+      const bool isv = hh >= a.H + a.HKV;
+      const int kvh = isv ? hh - a.H - a.HKV : hh - a.H;
+      unsigned short* pg = a.cache + (((long)page * a.HKV + kvh) * 2 + (isv ? 1 : 0)) * PAGE_ELEMS;
+      if (!isv) {
+        *(uint2*)(pg + kv_k_index(tau, d0)) = pk;  // 4 consecutive dims: one 8-B run of the K fragment
+      } else {
+        pg[kv_v_index(tau, d0 + 0)] = (unsigned short)(pk.x & 0xffff);
+        pg[kv_v_index(tau, d0 + 1)] = (unsigned short)(pk.x >> 16);
+        pg[kv_v_index(tau, d0 + 2)] = (unsigned short)(pk.y & 0xffff);
+        pg[kv_v_index(tau, d0 + 3)] = (unsigned short)(pk.y >> 16);
+      }
+    } else if (a.mode & EPI_SWIGLU) {
+      f32x4v u, o;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) u[i] = lane_xor32(v[i]);
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        o[i] = (a.mode & EPI_CLAMPED) ? gate_clamped(v[i], u[i], a.limit)
+               : ((a.mode & EPI_GELU) ? gate_act<GATE_GELU>(v[i]) : gate_act<GATE_SILU>(v[i])) * u[i];
+      if (in && fq < 2) *(uint2*)(a.y + (long)m * a.ldy + 8 * nt + 4 * fq) = uint2{pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3])};
+    } else if (in) {
+      if (a.mode & EPI_RESID) {
+        v[0] += bf2f(old.x & 0xffff);
+        v[1] += bf2f(old.x >> 16);
+        v[2] += bf2f(old.y & 0xffff);
+        v[3] += bf2f(old.y >> 16);
+      }
+      *(uint2*)out(t) = uint2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+    }
   }
 }
 
@@ -193,26 +286,37 @@ __global__ __launch_bounds__(64 * NW) void few(FewArgs a) {
 namespace {
 constexpr int FEW_CUS = 256;
 
-// Tiles of W (of 16 rows) and waves of a workgroup, and the k-steps of its ring; r 0: not for this kernel. Sums that neither divide as the
-// first lines' nor are short: 8, 4 or 2 waves, and as much of a wave's part in the ring as divides it.
+// Tiles of W (of 16 rows) and waves of a workgroup, the k-steps of its ring, and whether x comes by LDS; r 0: not for this kernel. Sums that neither
+// divide as the first lines' nor are short: 8, 4 or 2 waves, and as much of a wave's part in the ring as divides it.
 struct FewSplit {
-  int r, nw, pf;
+  int r, nw, pf, lx;
 };
 FewSplit few_split(int M, int N, int K) {
-  if (M < 1 || M > 32 || N <= 0 || K <= 0 || N % 16 || K % 64 || (long)N * K > (1l << 31)) return {0, 0, 0};
+  if (M < 1 || M > 32 || N <= 0 || K <= 0 || N % 16 || K % 64 || (long)N * K > (1l << 31)) return {0, 0, 0, 0};
   const int strips = N / 16;
   if (M <= 16 && K % 512 == 0) {
-    if (strips <= FEW_CUS && K % 1024 == 0) return {1, 8, 4};
-    if (strips <= 2 * FEW_CUS) return M > 4 && strips > FEW_CUS && strips % 2 == 0 ? FewSplit{2, 4, 4} : FewSplit{1, 4, 4};
-    return {1, 2, 8};
+    if (strips <= FEW_CUS) return M <= 4 && K >= 8192 && K % 1024 == 0 ? FewSplit{1, 8, 4, 0} : FewSplit{1, 2, K % 1024 == 0 ? 16 : 8, 0};
+    // two tiles a workgroup share x: where one makes little more than one round of the CUs, and where 13 rows and more bound a long grid
+    if (strips % 2 == 0 && (strips <= 2 * FEW_CUS ? M > 4 || strips <= 5 * FEW_CUS / 4 : M > 12 && strips >= 4 * FEW_CUS)) return {2, 2, 8, 0};
+    return {1, 1, 16, 0};
+  }
+  if (M > 16 && K % 1024 == 0) {
+    if (strips <= FEW_CUS) return {1, 8, 4, 1};
+    if (strips % 2 == 0) return strips <= 2 * FEW_CUS ? FewSplit{2, 8, 4, 1} : FewSplit{2, 4, 4, 1};
   }
   const int nw = K % 256 == 0 ? 8 : K % 128 == 0 ? 4 : 2, steps = K / 32 / nw;
-  return {1, nw, steps % 4 == 0 ? 4 : steps % 3 == 0 ? 3 : steps % 2 == 0 ? 2 : 1};
+  return {1, nw, steps % 4 == 0 ? 4 : steps % 3 == 0 ? 3 : steps % 2 == 0 ? 2 : 1, 0};
 }
+// With a norm or a rotation: only by the splits of the first lines
+bool few_normed(const FewSplit& f, int M, int K) { return f.r && (M <= 16 ? K % 512 == 0 : f.lx != 0); }
 }  // namespace
 
-// Whether kgs_skinny_few runs M rows of an [N, K] weight: up to 16 rows, N a multiple of 16 and K of 512; without a norm and a rotation up to 32 rows and K of 64.
+// Whether kgs_skinny_few runs M rows of an [N, K] weight: up to 32 rows, N a multiple of 16, K of 64. With a norm or a rotation (!plain) up to 16 rows
+// and K of 512; kgs_skinny_few_wide_ok has 17 to 32.
 KGS_EXPORT int kgs_skinny_few_ok(int M, int N, int K, int plain) { return few_split(M, N, K).r > 0 && (plain || (M <= 16 && K % 512 == 0)); }
+
+// Whether it runs 17 to 32 rows with x by LDS, and so with a norm and a rotation too: N a multiple of 32, or of 16 up to a strip a CU, K of 1024.
+KGS_EXPORT int kgs_skinny_few_wide_ok(int M, int N, int K) { return M > 16 && few_split(M, N, K).lx; }
 
 namespace {
 int launch_few(const kgs::dec::FewArgs& a, const FewSplit& f, bool rope, bool own, int products, hipStream_t s) {
@@ -224,18 +328,19 @@ int launch_few(const kgs::dec::FewArgs& a, const FewSplit& f, bool rope, bool ow
   };
   auto pick = [&](auto ro, auto ow) {
     constexpr bool RO = decltype(ro)::value, OW = decltype(ow)::value;
-    if (f.r == 2) return run(few<2, 1, 4, 4, RO, OW>);
-    if (f.nw == 8) return run(few<1, 1, 8, 4, RO, OW>);
-    if (f.nw == 4) return run(few<1, 1, 4, 4, RO, OW>);
-    return run(few<1, 1, 2, 8, RO, OW>);
+    if (f.lx) return f.r == 1 ? run(few<1, 2, 8, 4, true, RO, OW>) : f.nw == 8 ? run(few<2, 2, 8, 4, true, RO, OW>) : run(few<2, 2, 4, 4, true, RO, OW>);
+    if (f.r == 2) return run(few<2, 1, 2, 8, false, RO, OW>);
+    if (f.nw == 1) return run(few<1, 1, 1, 16, false, RO, OW>);
+    if (f.nw == 8) return run(few<1, 1, 8, 4, false, RO, OW>);
+    return f.pf == 16 ? run(few<1, 1, 2, 16, false, RO, OW>) : run(few<1, 1, 2, 8, false, RO, OW>);
   };
   using T = std::true_type;
   using F = std::false_type;
-  if (M <= 16 && K % 512 == 0) return rope ? (own ? pick(T{}, T{}) : pick(T{}, F{})) : own ? pick(F{}, T{}) : pick(F{}, F{});
+  if (f.lx || (M <= 16 && K % 512 == 0)) return rope ? (own ? pick(T{}, T{}) : pick(T{}, F{})) : own ? pick(F{}, T{}) : pick(F{}, F{});
   auto odd = [&](auto mt, auto nw) {
     constexpr int MT = decltype(mt)::value, NW = decltype(nw)::value;
-    return f.pf == 4 ? run(few<1, MT, NW, 4, false, false>) : f.pf == 3 ? run(few<1, MT, NW, 3, false, false>)
-           : f.pf == 2 ? run(few<1, MT, NW, 2, false, false>) : run(few<1, MT, NW, 1, false, false>);
+    return f.pf == 4 ? run(few<1, MT, NW, 4, false, false, false>) : f.pf == 3 ? run(few<1, MT, NW, 3, false, false, false>)
+           : f.pf == 2 ? run(few<1, MT, NW, 2, false, false, false>) : run(few<1, MT, NW, 1, false, false, false>);
   };
   auto waves = [&](auto mt) {
     return f.nw == 8 ? odd(mt, std::integral_constant<int, 8>{}) : f.nw == 4 ? odd(mt, std::integral_constant<int, 4>{})
@@ -255,7 +360,7 @@ KGS_EXPORT int kgs_skinny_few(const void* wp, const void* x, void* y, int M, int
   const FewSplit f = few_split(M, N, K);
   if (!f.r) return KGS_ERR_SHAPE;
   const bool rope = epi & EPI_ROPE, own = epi & EPI_RMS;
-  if ((rope || own) && (M > 16 || K % 512)) return KGS_ERR_SHAPE;
+  if ((rope || own) && !few_normed(f, M, K)) return KGS_ERR_SHAPE;
   if (ldx < K || ldy < (epi & EPI_SWIGLU ? N / 2 : N) || ldx > 1l << 25) return KGS_ERR_SHAPE;
   if ((uintptr_t)wp % 16 || (uintptr_t)x % 16 || (uintptr_t)y % 8 || ldx % 8 || ldy % 4) return KGS_ERR_ALIGN;
   if (epi & ~(EPI_SWIGLU | EPI_GELU | EPI_CLAMPED | EPI_RMS | EPI_RESID | EPI_ROPE)) return KGS_ERR_ARG;

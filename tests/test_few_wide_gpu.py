@@ -1,0 +1,58 @@
+"""Products of 17 to 32 rows with x by LDS (native/kernels/decode_few.hip), each of its splits: one tile a workgroup, two on eight waves, two on four;
+K of one ring round and of several."""
+import pytest
+import torch
+
+from kgs.ops import decode as D
+
+pytestmark = [pytest.mark.gpu, pytest.mark.usefixtures("own_rng")]
+
+SHAPES = ((16, 1024), (4096, 1024), (2048, 8192), (4128, 1024), (8192, 2048), (8224, 1024), (16384, 2048))
+
+
+def _close(got, ref, factors=1):
+    """One rounding to bf16 (2^-9 of the value) and fp32 sums of at most 8192 products (1e-5 of the rows' size) for each factor."""
+    err = (got.double() - ref).abs()
+    assert bool((err <= 2.0 ** -8 * ref.abs() + 2e-5 * factors * ref.abs().max()).all()), err.max()
+
+
+@pytest.mark.parametrize("n,k", SHAPES)
+@pytest.mark.parametrize("m", (17, 24, 32))
+def test_each_epilogue(n, k, m):
+    x = torch.randn(m, k + 8, device="cuda").bfloat16()[:, :k]  # rows further apart than they are long
+    w = (torch.randn(n, k, device="cuda") * k ** -0.5).bfloat16()
+    assert D.few_wide(m, n, k) and not D.few_takes(m, n, k)
+    pw, ref = D.PackedWeight(w), x.double() @ w.double().T
+    _close(D.skinny_few(x, pw), ref)
+    normed = ref * torch.rsqrt(x.double().pow(2).mean(1, keepdim=True) + 1e-3)
+    _close(D.skinny_few(x, pw, norm=True, eps=1e-3), normed)
+    out = torch.randn(m, n, device="cuda").bfloat16()
+    want = out.double() + ref
+    assert D.own_gemm(x, pw, out=out, resid=True) is out
+    _close(out, want)
+    if n % 32 == 0:
+        g, u = normed.chunk(2, 1)
+        _close(D.skinny_few(x, D.PackedWeight(w, swiglu=True), norm=True, eps=1e-3), torch.nn.functional.silu(g) * u, 4)
+
+
+@pytest.mark.parametrize("heads,kv", ((4, 2), (32, 8), (48, 16)))
+@pytest.mark.parametrize("m", (17, 32))
+def test_rotation_and_cache_as_the_separate_launch(heads, kv, m):
+    from kgs.ops.transformer import rope_tables
+
+    k = 1024
+    x, w = torch.randn(m, k, device="cuda").bfloat16(), (torch.randn((heads + 2 * kv) * 128, k, device="cuda") * k ** -0.5).bfloat16()
+    cos, sin = rope_tables(256, 128, 10000.0, "cuda")
+    pos, slots = torch.arange(m, dtype=torch.int32, device="cuda") * 13 % 200, torch.randperm(8 * 32, device="cuda")[:m].int()
+    slots[m // 2] = -1
+    caches = [D.PagedKVCache(1, 8, kv, "cuda") for _ in range(2)]
+    got = D.skinny_few(x, D.PackedWeight(w, rope=(heads, kv)), norm=True,
+                       rope={"cos": cos, "sin": sin, "positions": pos, "slots": slots, "cache": caches[0].layer(0)})
+    want = D.skinny_few(x, D.PackedWeight(w), norm=True)  # the same sums, row by row
+    D.rope_cache_(want, cos, sin, pos, slots, caches[1].layer(0), heads, kv)
+    assert torch.equal(got, want) and torch.equal(caches[0].data, caches[1].data)
+
+
+def test_what_goes_elsewhere():
+    for m, n, k in ((16, 4096, 4096), (33, 4096, 4096), (24, 4096, 1536), (24, 4096, 14336), (24, 28672, 4096), (24, 4112, 1024)):
+        assert not D.few_wide(m, n, k), (m, n, k)

@@ -265,7 +265,7 @@ def gemm_nt_w4x(a: torch.Tensor, b, bn: int = 256, nslice: int = 1,
     partials + reduce when > 1): the decode-batch GEMM path.
     ``N % bn == 0`` and ``(K / nslice) % 128 == 0``. ``b`` is a ``[N, K]`` tensor
     or a :class:`PanelWeight` packed with the same ``bn``. ``stages``: LDS
-    stages (3 / 4 keep more K-tiles in flight; only where they fit in 160 KiB).
+    stages asked for (refused where they do not fit in 160 KiB; tiles smaller than 256x256 take three or four in any case: the same bits).
     ``nt_weights``: ``b``'s loads non-temporal (decode weights each CU streams
     once), ``a``'s loads default (two stages only). ``private``: partials in a buffer of
     this call's own instead of the per-GPU workspace."""

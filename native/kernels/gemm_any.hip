@@ -23,6 +23,7 @@
 #include "gemm_w4.h"
 
 namespace kgs {
+int cu_count();  // gemm_bf16.hip
 namespace any {
 
 using w4::BK;
@@ -30,7 +31,7 @@ using w4::Ctx;
 using w4::Frag;
 
 typedef long i64x2 __attribute__((ext_vector_type(2)));
-constexpr int OOB = 0x7FFFFFF0;  // above every buffer resource's size (gemm_any_ok)
+constexpr int OOB = w4::OOB_OFFSET;  // above every buffer resource's size (gemm_any_ok)
 
 // What a launch stores. DUAL: C gets bf16(acc + bias) and C2 the activation of that bf16 value
 // (a training forward pass, whose backward pass needs both).
@@ -50,6 +51,14 @@ struct Args {
 
 template <int BM, int BN>
 constexpr int waves_per_simd() { return BM == 128 && BN == 128 ? 2 : 1; }
+
+// LDS stages of a tile with a CU to itself (ONE): 128 columns leave room for more than two, and so for one barrier a K-step (w4::kstep1). Of 192
+// columns three fit too and give nothing (1762 x 6144 x 4096 67.8, 68.3). Medians of runs in turn, us, two stages / so: 128x128 tiles 2048^3 21.7 / 19.8
+// (three stages 20.4, five 20.7), 1024 x 4096 x 4096 40.4 / 36.7, 1024 x 1024 x 8192 49.0 / 42.2; 192x128 1536 x 4096 x 4096 47.6 / 44.9;
+// 224x128 1762 x 4096 x 4096 55.3 / 53.2, K 14336 185 / 181, 3580 x 2048 x 2048 27.4 / 26.5; 256x128 2048 x 4096 x 4096 57.5 / 54.4. What is left there is
+// the matrix cores' clock and the operands' way in: MFMAs alone 49 us of the last.
+template <int BM, int BN, bool ONE>
+constexpr int lds_stages() { return !ONE || BN != 128 ? 2 : BM == 128 ? 4 : 3; }
 
 template <int EPI>
 __device__ __forceinline__ unsigned pack_epi(float a, float b, float ba, float bb) {
@@ -133,14 +142,15 @@ __device__ __forceinline__ void store_row(const Args& a, int r, int col, const f
 // SW (a GateAct): B is a fused gate|up weight of N rows, gate rows first, and C [M, N / 2] holds
 // act(gate) * up; a tile stages both halves' rows in turn (gemm_w4.h). `bias` then points to the
 // clamped gate's limit.
-template <int EPI, int BM, int BN, bool SPLIT, bool DUAL, int SW>
+template <int EPI, int BM, int BN, bool SPLIT, bool DUAL, int SW, bool ONE>
 __device__ __forceinline__ void tile_product(const Args& a) {
   constexpr int X = SW * 1000000, TN = SW ? BN / 2 : BN;  // TN: output columns of a tile
   const int cols = SW ? a.N / 2 : a.N;
   using S = w4::Shape<BM, BN>;
   using Kn = w4::Knobs<BM, BN>;
   constexpr int MA = S::MA, NB = S::NB, ND = w4::dma_per_stage<BM, BN>();
-  __shared__ __attribute__((aligned(1024))) char smem[2 * S::STAGE];
+  constexpr int NS = lds_stages<BM, BN, ONE>();
+  __shared__ __attribute__((aligned(1024))) char smem[NS * S::STAGE];
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int ntm = (a.M + BM - 1) / BM, ntn = (cols + TN - 1) / TN;
@@ -156,7 +166,7 @@ __device__ __forceinline__ void tile_product(const Args& a) {
   c.w = w;
   c.wr = w >> 1;
   c.wc = w & 1;
-  c.nt = (kn + 2 * BK - 1) / (2 * BK) * 2;
+  c.nt = NS > 2 ? (kn + BK - 1) / BK : (kn + 2 * BK - 1) / (2 * BK) * 2;
   // resources end with the last valid element: nothing outside the operands is ever read
   const int ra = min(a.M - m0, BM), rb = min(cols - n0, TN);
   c.ra = __builtin_amdgcn_make_buffer_rsrc((void*)(a.A + (long)m0 * a.lda + k0), 0, ((ra - 1) * a.lda + kn) * 2, 0x00020000);
@@ -183,12 +193,12 @@ __device__ __forceinline__ void tile_product(const Args& a) {
   w4::static_for<0, MA * NB>([](auto q) { accr::zero<decltype(q)::value>(); });
 
 #pragma unroll
-  for (int st = 0; st < 2; ++st) {
+  for (int st = 0; st < (NS > 2 ? NS - 1 : 2); ++st) {
     aim(st);
 #pragma unroll
-    for (int j = 0; j < ND; ++j) w4::dma_any<BM, BN, X>(c, st, j, st * BK);
+    for (int j = 0; j < ND; ++j) w4::dma_any<BM, BN, X>(c, st, j, min(st, c.nt - 1) * BK);
   }
-  w4::wait_vm<ND>();
+  w4::wait_vm<(NS > 2 ? NS - 2 : 1) * ND>();
   w4::bar();
   Frag<MA, NB> f0, f1;
   {
@@ -203,13 +213,25 @@ __device__ __forceinline__ void tile_product(const Args& a) {
   }
   __builtin_amdgcn_s_waitcnt(0xc07f);
 
-  for (int t = 0; t < c.nt; t += 2) {
-    aim(min(t + 2, c.nt - 1));
-    w4::kstep<BM, BN, 0, Kn::B1, Kn::R, Kn::P, Kn::ORD, X>(c, f0, f1, t);
-    aim(min(t + 3, c.nt - 1));
-    w4::kstep<BM, BN, 1, Kn::B1, Kn::R, Kn::P, Kn::ORD, X>(c, f0, f1, t + 1);
+  // K-tiles past the end: outside the resources, so that their DMAs fetch nothing (a fetch is waited for at the end)
+  if constexpr (NS > 2) {
+    for (int t = 0; t < c.nt; t += NS) {
+      w4::static_for<0, NS>([&](auto st) {
+        constexpr int ST = decltype(st)::value;
+        if (ST && t + ST >= c.nt) return;
+        aim(t + ST + NS - 1);
+        w4::kstep1<BM, BN, ST, Kn::R, Kn::P, Kn::ORD, X, NS>(c, f0, f1, t + ST);
+      });
+    }
+  } else {
+    for (int t = 0; t < c.nt; t += 2) {
+      aim(t + 2);
+      w4::kstep<BM, BN, 0, Kn::B1, Kn::R, Kn::P, Kn::ORD, X>(c, f0, f1, t);
+      aim(t + 3);
+      w4::kstep<BM, BN, 1, Kn::B1, Kn::R, Kn::P, Kn::ORD, X>(c, f0, f1, t + 1);
+    }
   }
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // drain the tail re-loads before LDS is released
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the tail's DMAs (zeros) land before LDS is released
   asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 3" ::: "memory");  // MFMA -> v_accvgpr_read hazard
 
   const int mw = m0 + c.wr * (BM / 2) + fr, nw = n0 + c.wc * (TN / 2);
@@ -272,15 +294,16 @@ __device__ __forceinline__ void tile_product(const Args& a) {
   });
 }
 
-// gemm_nt_any: the tiles of plan, with or without slices; gemm_nt_mid: those between them (refine), one workgroup a CU
+// gemm_nt_any: the tiles of plan, with or without slices; gemm_nt_mid: those between them (refine), one workgroup a CU, and 128x128 tiles that
+// are no more than the CUs
 template <int EPI, int BM, int BN, bool SPLIT, bool DUAL, int SW = 0>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(waves_per_simd<BM, BN>(), waves_per_simd<BM, BN>())))
 void gemm_nt_any(Args a) {
-  tile_product<EPI, BM, BN, SPLIT, DUAL, SW>(a);
+  tile_product<EPI, BM, BN, SPLIT, DUAL, SW, waves_per_simd<BM, BN>() == 1>(a);
 }
-template <int EPI, int BM, int BN, bool DUAL, int SW = 0>
+template <int EPI, int BM, int BN, bool DUAL, int SW = 0, bool SPLIT = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void gemm_nt_mid(Args a) {
-  tile_product<EPI, BM, BN, false, DUAL, SW>(a);
+  tile_product<EPI, BM, BN, SPLIT, DUAL, SW, true>(a);
 }
 
 // The same product on 64x64 tiles, for grids that leave CUs idle at 128x128. What bounds such a
@@ -780,20 +803,21 @@ inline Plan plan(long M, long N, long K, bool split, int cus) {
 // A tile's time in an unsliced product, us, fitted to 310 sizes of 160 to 10000 rows (half of the errors below 6 %; the
 // tile that these estimates choose takes 0.8 % more than the best one): start, what each round of workgroups
 // after the first adds, and a K-step alone on a CU and what the chip's filling adds to it. 128x128 tiles: of two
-// workgroups on a CU, and of the single ones that remain.
+// workgroups on a CU, and of the single ones that remain. Tiles of 128 columns (of 128x128 ones the single) scaled to their K-steps of one barrier, by 48
+// sizes: 0.33 + 0.13 full where 0.37 + 0.16, of 192 rows 0.40 + 0.25 / 0.42 + 0.29, 224 0.44 + 0.29 / 0.45 + 0.32, 256 0.46 + 0.35 / 0.49 + 0.36.
 struct Tile {
   int bm, bn;
   double start, again, step, fill;
 };
-constexpr Tile TILES[] = {{256, 256, 7.12, 7.31, 0.88, 0.50}, {256, 128, 4.61, 4.53, 0.55, 0.29}, {128, 128, 3.5, 3.2, 0.97, 0},
-                          {192, 128, 4.15, 2.97, 0.44, 0.25}, {224, 128, 4.27, 3.53, 0.49, 0.28}, {192, 192, 5.02, 4.65, 0.56, 0.29},
+constexpr Tile TILES[] = {{256, 256, 7.12, 7.31, 0.88, 0.50}, {256, 128, 4.61, 4.53, 0.53, 0.28}, {128, 128, 3.5, 3.2, 0.97, 0},
+                          {192, 128, 4.15, 2.97, 0.42, 0.22}, {224, 128, 4.27, 3.53, 0.48, 0.25}, {192, 192, 5.02, 4.65, 0.56, 0.29},
                           {224, 192, 5.40, 5.14, 0.61, 0.35}, {256, 192, 5.90, 5.94, 0.67, 0.38}, {224, 256, 6.49, 6.69, 0.78, 0.43}};
 inline double tile_cost(const Tile& t, long M, long N, long K, int cus) {
   const long wg = (long)ceil_div(M, t.bm) * ceil_div(N, t.bn);
   const int steps = 2 * ceil_div(K, 128);
   if (t.bm == 128) {
     const int two = (int)(wg / (2L * cus)), rest = (int)(wg - 2L * cus * two), pairs = two + (rest > cus);
-    const double one = rest > 0 && rest <= cus ? 0.34 + 0.26 * rest / cus : 0;
+    const double one = rest > 0 && rest <= cus ? 0.30 + 0.21 * rest / cus : 0;
     return t.start + steps * (pairs * t.step + one) + (two ? t.again * (two - (rest == 0)) : 0);
   }
   const int full = (int)(wg / cus), rest = (int)(wg - (long)full * cus), rounds = full + (rest > 0);
@@ -919,6 +943,12 @@ inline int layout_plan(long M, long N, long K, int ta, int tb, int cus) {
 template <int EPI, int BM, int BN, bool DUAL>
 void launch_tile(const Args& a, int ns, hipStream_t s) {
   const dim3 grid((unsigned)(ceil_div(a.M, BM) * ceil_div(a.N, BN) * ns));
+  if constexpr (BM == 128 && BN == 128)
+    if ((int)grid.x <= cu_count()) {
+      if (ns > 1) hipLaunchKernelGGL((gemm_nt_mid<EPI_NONE, BM, BN, false, 0, true>), grid, dim3(256), 0, s, a);
+      else hipLaunchKernelGGL((gemm_nt_mid<EPI, BM, BN, DUAL>), grid, dim3(256), 0, s, a);
+      return;
+    }
   if (ns > 1) hipLaunchKernelGGL((gemm_nt_any<EPI_NONE, BM, BN, true, false>), grid, dim3(256), 0, s, a);
   else hipLaunchKernelGGL((gemm_nt_any<EPI, BM, BN, false, DUAL>), grid, dim3(256), 0, s, a);
 }
@@ -968,8 +998,6 @@ int launch(Args a, Plan p, float* ws, hipStream_t s) {
 }
 
 }  // namespace any
-
-int cu_count();  // gemm_bf16.hip
 
 // The operands gemm_tr takes: rows of whole 16-byte chunks, readable (and zero where contracted
 // over) to the next one, 32-bit offsets over K.
@@ -1093,10 +1121,12 @@ int gemm_any_swiglu(const void* A, const void* B, void* C, int M, int N, int K, 
                M, N, K, lda, ldb, ldc, 0, M > N, ldc % 8 == 0 && (uintptr_t)C % 16 == 0, 1.f, nullptr};
   const Plan p = gated_plan(M, N, K, cu_count());
   const dim3 grid((unsigned)(ceil_div(M, p.bm) * ceil_div(N / 2, p.bn / 2)));
+  const bool one = (int)grid.x <= cu_count();
 #define KGS_SWK(BM, BN, ...) \
   case BM << 16 | BN: hipLaunchKernelGGL((__VA_ARGS__>), grid, dim3(256), 0, s, a); break
 #define KGS_SWT(ACT)           \
-  switch (p.bm << 16 | p.bn) { \
+  if (one && p.bm == 128 && p.bn == 128) hipLaunchKernelGGL((gemm_nt_mid<EPI_NONE, 128, 128, false, ACT>), grid, dim3(256), 0, s, a); \
+  else switch (p.bm << 16 | p.bn) { \
     KGS_SWK(128, 128, gemm_nt_any<EPI_NONE, 128, 128, false, false, ACT); \
     KGS_SWK(256, 128, gemm_nt_any<EPI_NONE, 256, 128, false, false, ACT); \
     KGS_SWK(256, 256, gemm_nt_any<EPI_NONE, 256, 256, false, false, ACT); \

@@ -855,44 +855,28 @@ void launch_w4x_x(dim3 grid, hipStream_t s, const unsigned short* a, const unsig
 #undef KGS_W4X
 }
 
-// LDS stages of the w4x entries: flags bits 4-5 = stages - 2 (gemm_w4.h
-// stages<MODE>), only where NS stages fit in 160 KiB
+// LDS stages of the w4x entries: four of 128x128 tiles, three where they fit in 160 KiB, else two (the flags' bits 4-5 ask for
+// stages - 2: the same bits, so the tiles take what is the fastest). us, weights from HBM, two stages and two barriers a K-step / so, 128x128
+// tiles: 6144x4096 in 4 slices at 64 rows 16.4 / 14.7, 4096x14336 in 8 26.5 / 24.4, 2048x8192 in 8 at 200 16.9 / 15.7, 28672x4096 gated from panels at 64 48.8 / 44.1;
+// 256x128 4096x14336 in 8 at 200 39.8 / 38.5; 128x256 128256x4096 at 128 200 / 190. Four K-steps a slice of whole tiles lose 0.2: 2048x2048 in 8 at 256 9.1 / 9.4.
 constexpr bool stages_fit(int bm, int bn, int ns) { return ns * (bm + bn) * 128 <= 160 * 1024; }
+constexpr int stage_bits(int bm, int bn) { return stages_fit(bm, bn, 4) ? 0x20 : stages_fit(bm, bn, 3) ? 0x10 : 0; }
+inline bool stages_given(int bm, int bn, int flags) { return stages_fit(bm, bn, 2 + ((flags >> 4) & 3)); }
 
 // flags bit 0 (packed): B stored tile-panel major ([N / bn][K / 64][bn][64],
-// gemm_w4.h PACKB); bits 4-5: extra LDS stages
+// gemm_w4.h PACKB); bit 1: weights (B) non-temporal
 template <int BN, int TM>
 int launch_w4x(dim3 grid, hipStream_t s, const unsigned short* a, const unsigned short* b, unsigned short* out,
                int M, int N, int ks, int lda, int ldb, int ld, int mode, int flags) {
-  constexpr int BM = kgs::w4::tile_m<TM>();
-  const bool packed = flags & 1;
-  if (flags & 2) {  // weights (B) non-temporal: two LDS stages only
-    if (flags & 0x30) return KGS_ERR_ARG;
-    if (packed) launch_w4x_x<BN, TM, 1000005200>(grid, s, a, b, out, M, N, ks, lda, ldb, ld, mode);
-    else launch_w4x_x<BN, TM, 5200>(grid, s, a, b, out, M, N, ks, lda, ldb, ld, mode);
-    return 0;
+  constexpr int BM = kgs::w4::tile_m<TM>(), T = TM | stage_bits(BM, BN);
+  if ((flags & 2 && flags & 0x30) || !stages_given(BM, BN, flags)) return KGS_ERR_ARG;
+  switch (flags & 3) {
+    case 0: launch_w4x_x<BN, T, 0>(grid, s, a, b, out, M, N, ks, lda, ldb, ld, mode); break;
+    case 1: launch_w4x_x<BN, T, 1000000000>(grid, s, a, b, out, M, N, ks, lda, ldb, ld, mode); break;
+    case 2: launch_w4x_x<BN, T, 5200>(grid, s, a, b, out, M, N, ks, lda, ldb, ld, mode); break;
+    default: launch_w4x_x<BN, T, 1000005200>(grid, s, a, b, out, M, N, ks, lda, ldb, ld, mode);
   }
-  switch (flags & 0x30) {
-    case 0x00:
-      if (packed) launch_w4x_x<BN, TM, 1000000000>(grid, s, a, b, out, M, N, ks, lda, ldb, ld, mode);
-      else launch_w4x_x<BN, TM, 0>(grid, s, a, b, out, M, N, ks, lda, ldb, ld, mode);
-      return 0;
-    case 0x10:
-      if constexpr (stages_fit(BM, BN, 3)) {
-        if (packed) launch_w4x_x<BN, TM | 0x10, 1000000000>(grid, s, a, b, out, M, N, ks, lda, ldb, ld, mode);
-        else launch_w4x_x<BN, TM | 0x10, 0>(grid, s, a, b, out, M, N, ks, lda, ldb, ld, mode);
-        return 0;
-      }
-      break;
-    case 0x20:
-      if constexpr (stages_fit(BM, BN, 4)) {
-        if (packed) launch_w4x_x<BN, TM | 0x20, 1000000000>(grid, s, a, b, out, M, N, ks, lda, ldb, ld, mode);
-        else launch_w4x_x<BN, TM | 0x20, 0>(grid, s, a, b, out, M, N, ks, lda, ldb, ld, mode);
-        return 0;
-      }
-      break;
-  }
-  return KGS_ERR_ARG;
+  return 0;
 }
 
 template <int BN, int TM, int X>
@@ -910,51 +894,27 @@ void launch_w4sw_x(dim3 grid, hipStream_t s, const unsigned short* a, const unsi
                        a, b, c, limit, M, N, K, lda, ldb, ldc);
 }
 
+// flags as for launch_w4x; bit 6: tanh gelu, bit 7: clamped, both with row-major weights
 template <int BN, int TM>
 int launch_w4sw(dim3 grid, hipStream_t s, const unsigned short* a, const unsigned short* b, unsigned short* c, int M,
                 int N, int K, int lda, int ldb, int ldc, bool aligned_m, int flags, const float* limit) {
-  constexpr int BM = kgs::w4::tile_m<TM>();
-  const bool packed = flags & 1;
-  if (flags & 0x80) {  // clamped: row-major weights, two LDS stages
-    if (flags & 0x31) return KGS_ERR_ARG;
-    const auto lim = (const unsigned short*)limit;
-    if (flags & 2) launch_w4sw_x<BN, TM, 4005200>(grid, s, a, b, c, M, N, K, lda, ldb, ldc, aligned_m, lim);
-    else launch_w4sw_x<BN, TM, 4000000>(grid, s, a, b, c, M, N, K, lda, ldb, ldc, aligned_m, lim);
-    return 0;
+  constexpr int BM = kgs::w4::tile_m<TM>(), T = TM | stage_bits(BM, BN);
+  if ((flags & 0xc0 && flags & 0x31) || (flags & 2 && flags & 0x30) || !stages_given(BM, BN, flags)) return KGS_ERR_ARG;
+  const auto lim = (const unsigned short*)limit;
+#define KGS_W4SW(X) launch_w4sw_x<BN, T, X>(grid, s, a, b, c, M, N, K, lda, ldb, ldc, aligned_m, lim)
+  switch (flags & 0xc3) {
+    case 0x00: KGS_W4SW(1000000); break;
+    case 0x01: KGS_W4SW(1001000000); break;
+    case 0x02: KGS_W4SW(1005200); break;
+    case 0x03: KGS_W4SW(1001005200); break;
+    case 0x40: KGS_W4SW(2000000); break;
+    case 0x42: KGS_W4SW(2005200); break;
+    case 0x80: KGS_W4SW(4000000); break;
+    case 0x82: KGS_W4SW(4005200); break;
+    default: return KGS_ERR_ARG;
   }
-  if (flags & 0x40) {  // tanh gelu: row-major weights, two LDS stages
-    if (flags & 0x31) return KGS_ERR_ARG;
-    if (flags & 2) launch_w4sw_x<BN, TM, 2005200>(grid, s, a, b, c, M, N, K, lda, ldb, ldc, aligned_m);
-    else launch_w4sw_x<BN, TM, 2000000>(grid, s, a, b, c, M, N, K, lda, ldb, ldc, aligned_m);
-    return 0;
-  }
-  if (flags & 2) {  // weights (B) non-temporal: two LDS stages only
-    if (flags & 0x30) return KGS_ERR_ARG;
-    if (packed) launch_w4sw_x<BN, TM, 1001005200>(grid, s, a, b, c, M, N, K, lda, ldb, ldc, aligned_m);
-    else launch_w4sw_x<BN, TM, 1005200>(grid, s, a, b, c, M, N, K, lda, ldb, ldc, aligned_m);
-    return 0;
-  }
-  switch (flags & 0x30) {
-    case 0x00:
-      if (packed) launch_w4sw_x<BN, TM, 1001000000>(grid, s, a, b, c, M, N, K, lda, ldb, ldc, aligned_m);
-      else launch_w4sw_x<BN, TM, 1000000>(grid, s, a, b, c, M, N, K, lda, ldb, ldc, aligned_m);
-      return 0;
-    case 0x10:
-      if constexpr (stages_fit(BM, BN, 3)) {
-        if (packed) launch_w4sw_x<BN, TM | 0x10, 1001000000>(grid, s, a, b, c, M, N, K, lda, ldb, ldc, aligned_m);
-        else launch_w4sw_x<BN, TM | 0x10, 1000000>(grid, s, a, b, c, M, N, K, lda, ldb, ldc, aligned_m);
-        return 0;
-      }
-      break;
-    case 0x20:
-      if constexpr (stages_fit(BM, BN, 4)) {
-        if (packed) launch_w4sw_x<BN, TM | 0x20, 1001000000>(grid, s, a, b, c, M, N, K, lda, ldb, ldc, aligned_m);
-        else launch_w4sw_x<BN, TM | 0x20, 1000000>(grid, s, a, b, c, M, N, K, lda, ldb, ldc, aligned_m);
-        return 0;
-      }
-      break;
-  }
-  return KGS_ERR_ARG;
+#undef KGS_W4SW
+  return 0;
 }
 }  // namespace
 

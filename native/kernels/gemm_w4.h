@@ -26,6 +26,8 @@
 // profiles/gemm_tuning.md (section "Four-wave kernel"); the measured
 // alternatives are instantiated in native/experiments/gemm_w4h.hip.
 //
+// Tiles of 128 rows or columns leave LDS for three stages and more, and so for one barrier a K-step (kstep1).
+//
 // The LDS image is the 8-wave kernel's (128-B rows, 16-B chunk c of row r at
 // c ^ ((r >> 1) & 7)): conflict-free ds_read_b128 fragments.
 //
@@ -73,6 +75,7 @@ namespace w4 {
 
 constexpr int BK = 64;
 constexpr int GM = 4;  // tile-group height (production choice)
+constexpr int OOB_OFFSET = 0x7FFFFFF0;  // above every buffer resource's size
 
 template <int BM, int BN>
 struct Shape {
@@ -348,6 +351,58 @@ __device__ __forceinline__ void kstep(const Ctx& c, Frag<BM / 32, BN / 32>& f0, 
   kbody<BM, BN, ST, B1, R, P, ORD, X, NS, 0>(c, sp, f0, f1);
 }
 
+// The same K-step on NS >= 3 stages with ONE barrier: K-tile t + NS - 1 goes into the stage of K-tile t - 1, which every wave has
+// read when it passes the barrier of step t - 1, so that the DMA issues spread over all MFMAs up to that barrier.
+//   k < NR              ds_read f1 (k-sub 1 of this K-tile) read k
+//   k < KM - R          the ND LDS-DMA issues of K-tile t + NS - 1
+//   k == KM - R - 1     lgkmcnt(0), vmcnt((NS - 2) ND) + barrier (K-tile t+1 visible, stage ST read by all)
+//   k >= KM - R         P ds_reads of f0 (K-tile t+1, k-sub 0) after each MFMA
+template <int BM, int BN, int ST, int R, int P, int ORD, int X, int NS, int K>
+__device__ __forceinline__ void kbody1(const Ctx& c, const StepPtrs& sp, Frag<BM / 32, BN / 32>& f0, Frag<BM / 32, BN / 32>& f1) {
+  using S = Shape<BM, BN>;
+  constexpr int MA = S::MA, NB = S::NB, KM = S::KM, HM = S::HM, NR = S::NR, ND = dma_per_stage<BM, BN>(), W = KM - R;
+  if constexpr (K < KM) {
+    constexpr int mi = Order<ORD, MA, NB>::o.i[K % HM], mn = Order<ORD, MA, NB>::o.n[K % HM];
+    if constexpr (K < HM) mma<MA, NB, mi, mn>(f0); else mma<MA, NB, mi, mn>(f1);
+    if constexpr (K < NR) {
+      constexpr int x = rd_idx(ORD, MA, NB, K);
+      if constexpr (rd_isa(ORD, MA, NB, K)) f1.a[x] = frag(sp.pa1 + x * 2048); else f1.b[x] = frag(sp.pb1 + x * 2048);
+    }
+    if constexpr (K < W) {
+#pragma unroll
+      for (int j = 0; j < ND; ++j) {
+        if ((j * W) / ND == K) dma_any<BM, BN, X>(c, (ST + NS - 1) % NS, j, sp.k0);
+      }
+    } else {
+      constexpr int q = K - W;
+#pragma unroll
+      for (int e = q * P; e < (q + 1) * P && e < NR; ++e) {
+        const int x = rd_idx(ORD, MA, NB, e);
+        if (rd_isa(ORD, MA, NB, e)) f0.a[x] = frag(sp.pa0 + x * 2048); else f0.b[x] = frag(sp.pb0 + x * 2048);
+      }
+    }
+    fence();
+    if constexpr (K == W - 1) {
+      __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): this wave's reads of stage ST retired
+      wait_vm<(NS - 2) * ND>();            // own DMA of K-tile t+1 landed
+      bar();
+    }
+    kbody1<BM, BN, ST, R, P, ORD, X, NS, K + 1>(c, sp, f0, f1);
+  }
+}
+template <int BM, int BN, int ST, int R, int P, int ORD, int X, int NS>
+__device__ __forceinline__ void kstep1(const Ctx& c, Frag<BM / 32, BN / 32>& f0, Frag<BM / 32, BN / 32>& f1, int t) {
+  using S = Shape<BM, BN>;
+  static_assert(NS >= 3 && S::NR <= S::KM - R && S::NR <= R * P, "bad K-step schedule");
+  StepPtrs sp;
+  sp.pa1 = abase<BM, BN, 1>(c, ST);
+  sp.pb1 = bbase<BM, BN, 1>(c, ST);
+  sp.pa0 = abase<BM, BN, 0>(c, (ST + 1) % NS);
+  sp.pb0 = bbase<BM, BN, 0>(c, (ST + 1) % NS);
+  sp.k0 = (t + NS - 1 < c.nt ? t + NS - 1 : c.nt - 1) * BK;  // past the end the caller's offsets lie outside the resources
+  kbody1<BM, BN, ST, R, P, ORD, X, NS, 0>(c, sp, f0, f1);
+}
+
 // Production knobs per tile shape: barrier 1 after MFMA B1, R MFMAs after
 // barrier 2, P reads per MFMA there, growing-square order, GROUP_M 4.
 template <int BM, int BN>
@@ -375,10 +430,8 @@ struct Knobs<128, 128> {
 template <int MODE>
 constexpr int tile_m() { return (MODE & 8) ? 128 : 256; }
 
-// MODE bits 4-5: LDS stages - 2 (round 3, decode GEMMs). With NS stages the
-// DMAs of K-tile t + NS are issued during K-step t, so NS - 1 K-tiles are in
-// flight while one is consumed: for the short-M, weight-streaming shapes the
-// K-step is bound by load latency, not by the MFMAs.
+// MODE bits 4-5: LDS stages - 2. From three on a K-step has one barrier (kstep1), and NS - 1 K-tiles are in
+// flight while one is consumed.
 template <int MODE>
 constexpr int stages() { return 2 + ((MODE >> 4) & 3); }
 
@@ -517,14 +570,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
   KGS_ACC_RESERVE();
   static_for<0, MA * NB>([](auto q) { accr::zero<decltype(q)::value>(); });
 
-  // prologue: K-tiles 0 .. NS-1 into stages 0 .. NS-1, k-sub 0 of K-tile 0 into f0
+  // prologue: the first K-tiles into their stages, k-sub 0 of K-tile 0 into f0
+  constexpr int AHEAD = NS > 2 ? NS - 1 : 2;
 #pragma unroll
-  for (int st = 0; st < NS; ++st) {
+  for (int st = 0; st < AHEAD; ++st) {
     const int kt = (st < c.nt ? st : c.nt - 1) * BK;
 #pragma unroll
     for (int j = 0; j < ND; ++j) dma_any<BM, BN, X>(c, st, j, kt);
   }
-  wait_vm<(NS - 1) * ND>();
+  wait_vm<(AHEAD - 1) * ND>();
   bar();
   Frag<MA, NB> f0, f1;
   {
@@ -546,14 +600,18 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
       kstep<BM, BN, 1, B1, R, P, ORD, X>(c, f0, f1, t + 1);
     }
   } else {
-    // K-tile t lives in stage t % NS; the tail steps of a partial round are
-    // skipped uniformly by the whole workgroup
+    // K-tile t lives in stage t % NS; the whole workgroup skips the steps past the end. K-tiles past it are sent for outside the
+    // resources: what they fetched would be waited for at the end
+    const int voa = c.voa, vob = c.vob;
     for (int t = 0; t < c.nt; t += NS) {
-      kstep<BM, BN, 0, B1, R, P, ORD, X, NS>(c, f0, f1, t);
-      if (t + 1 < c.nt) kstep<BM, BN, 1, B1, R, P, ORD, X, NS>(c, f0, f1, t + 1);
-      if (t + 2 < c.nt) kstep<BM, BN, 2 % NS, B1, R, P, ORD, X, NS>(c, f0, f1, t + 2);
-      if constexpr (NS == 4)
-        if (t + 3 < c.nt) kstep<BM, BN, 3, B1, R, P, ORD, X, NS>(c, f0, f1, t + 3);
+      static_for<0, NS>([&](auto st) {
+        constexpr int ST = decltype(st)::value;
+        if (ST && t + ST >= c.nt) return;
+        const bool in = t + ST + AHEAD < c.nt;
+        c.voa = in ? voa : OOB_OFFSET;
+        c.vob = in ? vob : OOB_OFFSET;
+        kstep1<BM, BN, ST, R, P, ORD, X, NS>(c, f0, f1, t + ST);
+      });
     }
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // drain the tail re-loads before LDS is released

@@ -65,6 +65,33 @@ def test_mid_tiles_repeat_the_large_tile_bits(M, N, K, bm, bn):
     assert rel(want, torch.nn.functional.gelu(a.double() @ b.double().T + bias.double(), approximate="tanh")) < 2 * REL
 
 
+# fewer K-tiles than LDS stages, as many, one round of them and one more; 128x128 tiles of one workgroup a CU, also in slices
+@pytest.mark.parametrize("K", [8, 64, 72, 128, 192, 200, 256, 264, 320, 448, 520, 1032])
+@pytest.mark.parametrize("bm,bn,ns", [(128, 128, 1), (128, 128, 2), (192, 128, 1), (224, 128, 1), (256, 128, 1), (256, 128, 3)])
+def test_tiles_of_one_barrier_a_step(bm, bn, ns, K):
+    M, N = 2 * bm + 1, 264
+    a, b = rnd(M, K), rnd(N, K)
+    want, got, large = a.double() @ b.double().T, *(torch.empty(M, N, device=DEV, dtype=torch.bfloat16) for _ in range(2))
+    run_any(a, b, got, bm, bn, ns)
+    run_any(a, b, large, 256, 256, 1)
+    # one rounding to bf16, and the roundings of K fp32 additions
+    assert bool(((got.double() - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -24 * K * want.abs().max()).all())
+    assert ns > 1 or torch.equal(got, large)
+
+
+@pytest.mark.parametrize("K", [128, 256, 384, 512, 640])
+@pytest.mark.parametrize("M", [128, 200])
+@pytest.mark.parametrize("bm,bn", [(128, 128), (256, 128), (128, 256)])
+def test_w4x_tiles_of_one_barrier_a_step(bm, bn, M, K):
+    from kgs.ops.gemm import gemm_nt_w4x, pack_w4x_weight
+
+    a, b = rnd(M, K), rnd(512, K)
+    want = gemm_nt_w4x(a, b, bn=256, bm=256)  # two stages
+    for w in (b, pack_w4x_weight(b, bn)):
+        for nt in (False, True):
+            assert torch.equal(gemm_nt_w4x(a, w, bn=bn, bm=bm, nt_weights=nt), want)
+
+
 def tile(M, N, K, gated=False):
     from kgs.ops import _lib
 

@@ -107,6 +107,8 @@ _SIGS = {
                                                       _c_void_p], _c_int),
     "kgs_skinny_slabs": ([_c_void_p] * 3 + [_c_int] * 3 + [_c_long] + [_c_int] * 2 + [_c_void_p], _c_int),
     "kgs_skinny_rows": ([_c_void_p] * 3 + [_c_int] * 3 + [_c_long] * 2 + [_c_int, _c_int, _c_void_p, ctypes.c_float, ctypes.c_float, _c_void_p], _c_int),
+    "kgs_wide_slabs": ([_c_void_p] * 3 + [_c_int] * 3 + [_c_long] + [_c_int] * 2 + [_c_void_p], _c_int),
+    "kgs_wide_rows": ([_c_void_p] * 3 + [_c_int] * 3 + [_c_long] * 2 + [_c_int, _c_void_p, ctypes.c_float, _c_void_p], _c_int),
     "kgs_rope_cache_packed_bf16": ([_c_void_p] * 6 + [_c_long, _c_int, _c_int, _c_long, _c_void_p, _c_int, _c_void_p, ctypes.c_float,
                                    ctypes.c_float, _c_void_p], _c_int),
     "kgs_skinny_few_ok": ([_c_int] * 4, _c_int),

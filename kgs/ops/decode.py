@@ -590,6 +590,7 @@ def own_gemm(x: torch.Tensor, w: PackedWeight, out: torch.Tensor | None = None, 
 
 
 SLAB_ROWS = 96
+WIDE_ROWS = 128
 
 
 @lru_cache(maxsize=4096)
@@ -597,8 +598,18 @@ def slab_split(m: int, n: int, k: int, cus: int = CUS) -> tuple[int, int] | None
     """(W tiles a wave, K slices) of :func:`skinny_slabs`, or None: up to 96 rows of W of 64 rows a workgroup (128 from N = 4096 on),
     in as many slices, 16 at most and of 128 at least, as leave one workgroup a CU. us at 32 rows in 4 / 8 / 16 slices: 2048x8192 11.6 / 8.1 /
     8.2, 4096x14336 27.0 / 19.6 / 21.6, 6144x4096 10.8 / 12.8 / -."""
+    return _split(n, k, cus) if 0 < m <= SLAB_ROWS else None
+
+
+def wide_split(m: int, n: int, k: int, cus: int = CUS) -> tuple[int, int] | None:
+    """:func:`slab_split` of :func:`wide_slabs`, 97 to 128 rows. The same split is the best there: us at 128 rows in 2 / 4 / 8 / 16 slices 2048x2048 9.0 /
+    6.7 / 6.5 / 8.4, 2048x8192 27.9 / 16.6 / 11.9 / 14.4, 6144x4096 by two tiles 23.6 / 17.1 / 20.3 (by one 18.6 in 2), 4096x14336 69 / 39.5 / 26.8 / 32.1."""
+    return _split(n, k, cus) if SLAB_ROWS < m <= WIDE_ROWS else None
+
+
+def _split(n: int, k: int, cus: int) -> tuple[int, int] | None:
     r = 2 if n >= 4096 and n % 128 == 0 else 1
-    if not 0 < m <= SLAB_ROWS or n % (64 * r) or k % 128:
+    if n <= 0 or k <= 0 or n % (64 * r) or k % 128:
         return None
     tiles, ns = n // (64 * r), 1
     while ns < 16 and 2 * ns * tiles <= cus and k % (256 * ns) == 0:
@@ -610,9 +621,27 @@ def slab_split(m: int, n: int, k: int, cus: int = CUS) -> tuple[int, int] | None
 def slab_rows_tiles(m: int, n: int, k: int, cus: int = CUS) -> int | None:
     """W tiles a wave of :func:`skinny_rows`, or None: two where 128 rows a workgroup are three quarters of the CUs or more (us at 48 rows with one /
     two: 28672x4096 48.0 / 39.8, 16384x2048 14.5 / 19.1; at 32 and fewer 32000x2048 23.4 / 28.3)."""
-    if not 0 < m <= SLAB_ROWS or n % 64 or k % 128:
+    return _rows_tiles(m, n, k, cus) if 0 < m <= SLAB_ROWS else None
+
+
+def _rows_tiles(m: int, n: int, k: int, cus: int) -> int | None:
+    if n % 64 or k % 128:
         return None
     return 2 if m > 32 and n % 128 == 0 and 4 * (n // 128) >= 3 * cus else 1
+
+
+def head_pays(m: int, n: int, k: int, cus: int = CUS) -> bool:
+    """Whether 49 to 128 rows of an LM head on residual rows are better off on :func:`skinny_rows` (:func:`wide_rows`) than their norm's product
+    with the rows of the weight: most of a round of workgroups or whole rounds, of K from 2048 on, where no four-wave tiles were measured to be better.
+    us at 64 / 96 / 128 rows, four-wave tiles or the library / so: 32000x2048 32.2, 33.2, 34.5 / 29.3, 30.3, 30.9; 32000x4096 58.3, 58.6, 61.7 / 44.5, 46.7, 49.3;
+    16384x2048 18.0, 19.0, 20.6 / 14.5, 16.0, 17.7; 64000x4096 119, 120, 121 / 86, 93, 100; not 32000x1024 15.7, 16.7, 17.5 / 15.7, 16.7, 17.6, nor 128256x4096,
+    which has entries of its own, 181, 187, 190 / 187, 202, 214."""
+    r = _rows_tiles(m, n, k, cus)
+    if not 48 < m <= WIDE_ROWS or r is None or k < 2048 or w4x_route(m, n, k) is not None:
+        return False
+    wgs = n // (64 * r)
+    rounds = -(-wgs // cus)
+    return 20 * wgs >= 19 * rounds * cus if rounds > 1 else 4 * wgs >= 3 * cus
 
 
 def rows_pay(m: int, n: int, k: int, gated: bool) -> bool:
@@ -677,14 +706,24 @@ def skinny_slabs(x: torch.Tensor, w: PackedWeight) -> torch.Tensor:
     """``x @ W^T`` of up to 96 rows of a bf16 weight as fp32 parts ``[slices, M, N]`` of its sum, for a consumer that adds them
     (native/kernels/decode_slabs.hip; :func:`slab_split`). Columns in the order in which the weight is packed."""
     m, k = _slab_operand(x, w)
-    split = None if w.fp8 or w.swiglu else slab_split(m, w.n, k)
+    return _slabs(x, w, m, k, slab_split, "skinny_slabs")
+
+
+def wide_slabs(x: torch.Tensor, w: PackedWeight) -> torch.Tensor:
+    """:func:`skinny_slabs` of 97 to 128 rows (:func:`wide_split`)."""
+    m, k = _slab_operand(x, w)
+    return _slabs(x, w, m, k, wide_split, "wide_slabs")
+
+
+def _slabs(x, w, m, k, rule, name):
+    split = None if w.fp8 or w.swiglu else rule(m, w.n, k)
     if split is None:
         raise ValueError(f"no slices for x {tuple(x.shape)}, W [{w.n}, {w.k}]")
     out = torch.empty((split[1], m, w.n), dtype=torch.float32, device=x.device)
-    rc = _lib.lib().kgs_skinny_slabs(w.data.data_ptr(), x.data_ptr(), out.data_ptr(), m, w.n, k, x.stride(0), *split,
-                                     _lib.stream_handle(x.device))
+    rc = getattr(_lib.lib(), "kgs_" + name)(w.data.data_ptr(), x.data_ptr(), out.data_ptr(), m, w.n, k, x.stride(0), *split,
+                                            _lib.stream_handle(x.device))
     if rc:
-        _lib.check(rc, f"skinny_slabs[{m}x{w.n}x{k}, {split}]")
+        _lib.check(rc, f"{name}[{m}x{w.n}x{k}, {split}]")
     return out
 
 
@@ -703,6 +742,22 @@ def skinny_rows(x: torch.Tensor, w: PackedWeight, sq: torch.Tensor | None = None
                                     float(eps), w.act.limit, _lib.stream_handle(x.device))
     if rc:
         _lib.check(rc, f"skinny_rows[{m}x{w.n}x{k}]")
+    return out
+
+
+def wide_rows(x: torch.Tensor, w: PackedWeight, sq: torch.Tensor | None = None, eps: float = 1e-5) -> torch.Tensor:
+    """:func:`skinny_rows` of 97 to 128 rows of a weight that is not gated."""
+    m, k = _slab_operand(x, w)
+    r = _rows_tiles(m, w.n, k, CUS) if SLAB_ROWS < m <= WIDE_ROWS and not (w.fp8 or w.rope or w.swiglu) else None
+    if r is None:
+        raise ValueError(f"no tiles for x {tuple(x.shape)}, W [{w.n}, {w.k}]")
+    if sq is not None and (sq.dtype != torch.float32 or sq.numel() != m or not sq.is_contiguous() or sq.device != x.device):
+        raise ValueError("sq must be a contiguous fp32 vector, one a row of x")
+    out = torch.empty((m, w.n), dtype=torch.bfloat16, device=x.device)
+    rc = _lib.lib().kgs_wide_rows(w.data.data_ptr(), x.data_ptr(), out.data_ptr(), m, w.n, k, x.stride(0), out.stride(0), r,
+                                  None if sq is None else sq.data_ptr(), float(eps), _lib.stream_handle(x.device))
+    if rc:
+        _lib.check(rc, f"wide_rows[{m}x{w.n}x{k}]")
     return out
 
 

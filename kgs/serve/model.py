@@ -7,7 +7,7 @@ Two step kinds, both driven by the native scheduler's plans
 * **prefill** -- the prompts of newly admitted sequences, each padded to a
   multiple of 128 tokens and concatenated (the layers drop the padding where that
   saves a tile of rows; steps of up to ``fused_max_batch`` rows, 64 at most, run the FUSED layer
-  below, of up to 96 the one IN SLICES where it pays, of up to 256 the split tiles): every projection is one
+  below, of up to 128 the one IN SLICES where it pays, of up to 256 the split tiles): every projection is one
   :func:`kgs.ops.gemm_nt` (256x256 MFMA pipeline), RoPE + the KV-cache scatter
   is one :func:`kgs.ops.decode.rope_cache_` launch, attention is one
   flash-attention launch over all sequences' query blocks, and only the last real token of each
@@ -19,7 +19,7 @@ Two step kinds, both driven by the native scheduler's plans
   epilogues carry the RMSNorms (norm weights folded into the weights, row
   scales from sums of squares that the GEMMs make of their own input, or where
   they cannot the residual-updating ones accumulate), the residual adds and
-  SwiGLU -- no elementwise kernels. From 33 to 96 rows (:meth:`ServingModel._slabs_pay`; a
+  SwiGLU -- no elementwise kernels. From 33 to 128 rows (:meth:`ServingModel._slabs_pay`, :meth:`ServingModel._wide`; a
   ``fused_max_batch`` of 32 and less turns them off) the layer runs IN SLICES: products
   over the prepacked weights leave their K slices to the rotation and the residual adds that
   follow. Larger batches run
@@ -685,7 +685,8 @@ class ServingModel:
     def decode(self, tokens, positions, slots, block_tables, ctx_lens, pages_per_split=None) -> torch.Tensor:
         """One token per sequence -> logits [B, vocab]."""
         c = self.cfg
-        if self.backend == "kgs" and tokens.shape[0] <= self.fused_max_batch or self._slabs_pay(tokens.shape[0]):
+        m = tokens.shape[0]
+        if self.backend == "kgs" and m <= self.fused_max_batch or self._slabs_pay(m) or self._wide(m):
             return self._decode_fused(tokens, positions, slots, block_tables, ctx_lens, pages_per_split)
         tickets = self._tickets(block_tables)
         x, y = self._start(tokens, zero=tickets)
@@ -757,7 +758,7 @@ class ServingModel:
             return D.paged_decode_attention(qkv, self.cache.layer(i), block_tables, ctx_lens, c.heads, c.kv_heads,
                                             pages_per_split=pages_per_split, tickets=tickets)
 
-        if self._slabs_pay(tokens.shape[0]):
+        if self._slabs_pay(tokens.shape[0]) or self._wide(tokens.shape[0]):
             x, y, ss = self._slab_layers(tokens, positions, slots, attend, "decode", tickets=tickets)
             out = self._slab_head(x if y is None else y, y is None, ss, decode=True)
             T.op("decode-slabs lm_head")
@@ -788,11 +789,22 @@ class ServingModel:
         CUs (:func:`kgs.ops.decode.slabs_fill`; four layers 2048 wide with a feed-forward of 11008, us a step of 64 / 96 rows by four-wave tiles 363 / 378, so 420 / 495)."""
         return self._slabs(m) and (m <= 48 or all(D.slabs_fill(m, w.n, w.k) for w in (self.packed[0][n] for n in ("qkv", "o", "down"))))
 
+    def _wide(self, m: int) -> bool:
+        """Whether 97 to 128 rows take those layers, under the conditions of fewer; gate and up go by their routes on normed rows. Four
+        layers, us a decode step of 97 / 112 / 128 rows by split tiles / so, contexts of 300: 2048 wide, feed-forward 8192 339, 352, 370 / 314, 326, 337; 4096,
+        14336 636, 667, 701 / 600, 627, 659; 8192, 28672 1868, 1912, 1954 / 1726, 1795, 1828; prompts 4096 wide 598, 595, 595 / 531, 553, 577; 2048, 8192 419, 414, 414 / 428, 409,
+        410, which the host bounds. Not 11008, whose slices do not fill the CUs."""
+        if self.packed is None or self.decode_fp8 or self.backend != "kgs" or not self.fuse_splitk or self.rope_attn or self.fused_max_batch <= 32:
+            return False
+        P, c = self.packed[0], self.cfg
+        return c.hidden % 2048 == 0 and c.hidden <= 8192 and bool(P["qkv"].rope) and all(
+            D.wide_split(m, w.n, w.k) and D.slabs_fill(D.SLAB_ROWS, w.n, w.k) for w in (P["qkv"], P["o"], P["down"]))
+
     def _slab_prompts(self, m: int) -> bool:
         """:meth:`_slabs_pay` for prompts, whose launches come from the host one by one: up to 48 rows, where the fused layers have 5 a layer and these 8, only
         with layers of 72 M weights and more (us, fused / here, one prompt of 40 tokens among others and alone: 2048 wide, 61 M weights 331 / 379, 423 / 436; 80 M 387 / 382,
         499 / 439; 92 M 400 / 386, 510 / 448; 4096 wide, 67 M 386 / 381, 489 / 460; 92 M 440 / 382, 544 / 472; 218 M 576 / 479, 685 / 586)."""
-        return self._slabs_pay(m) and (m > 48 or sum(w.n * w.k for w in self.packed[0].values()) >= 72_000_000)
+        return self._wide(m) or self._slabs_pay(m) and (m > 48 or sum(w.n * w.k for w in self.packed[0].values()) >= 72_000_000)
 
     def _slab_gate(self, m: int):
         """Gate and up of ``m`` rows of :meth:`_slab_layers`: a route of :meth:`_swiglu_route` on normed rows, or None: :func:`kgs.ops.decode.skinny_rows` on the
@@ -807,9 +819,9 @@ class ServingModel:
         return route
 
     def _slab_layers(self, tokens, positions, slots, attend, kind: str, keep=None, tickets=None):
-        """As :meth:`_fused_layers`, for 33 to 96 rows: products in K slices that the rotation and the residual adds sum, gate and up whole. At one
-        number of rows a row's bits do not depend on the others. ``(x, y, ss)``: the residual rows, from 49 rows on their norm for the head
-        (else None) and else their sums of squares. Four layers 4096 wide, us a step by four-wave tiles (up to 48 rows skinny) / so: one prompt of 90
+        """As :meth:`_fused_layers`, for 33 to 128 rows: products in K slices that the rotation and the residual adds sum, gate and up whole. At one
+        number of rows a row's bits do not depend on the others. ``(x, y, ss)``: the residual rows, their norm where the head wants that (else None: prompts of up
+        to 48 rows, decode steps also where :func:`kgs.ops.decode.head_pays`) and else their sums of squares. Four layers 4096 wide, us a step by four-wave tiles (up to 48 rows skinny) / so: one prompt of 90
         tokens 599 / 540, of 60 615 / 509, two of 36 in all 611 / 494; 2048 wide one of 60 397 / 387."""
         from kgs.ops.transformer import embed_rows, embeds, splitk_add_rmsnorm, splitk_add_squares
 
@@ -828,21 +840,25 @@ class ServingModel:
             ss.copy_(x.float().pow(2).sum(-1))
             if tickets is not None:
                 tickets.zero_()
-        gate = self._slab_gate(m)
+        wide = m > D.SLAB_ROWS
+        gate = self._swiglu_route(m) if wide else self._slab_gate(m)
+        slabs = D.wide_slabs if wide else D.skinny_slabs
+        raw = m <= 48 or kind == "decode" and D.head_pays(m, self.packed_lm.n, self.packed_lm.k)
         rope = {"cos": self.cos, "sin": self.sin, "positions": positions, "slots": slots}
         for i, P in enumerate(self.packed):
             rope["cache"] = self.cache.layer(i)
-            qkv = D.rope_cache_packed(D.skinny_slabs(x, P["qkv"]), ss, P["qkv"], c.eps, rope)
+            qkv = D.rope_cache_packed(slabs(x, P["qkv"]), ss, P["qkv"], c.eps, rope)
             T.op(f"{kind}-slabs L{i} qkv+rope")
             a = attend(qkv, i)
             T.op(f"{kind}-slabs L{i} attention")
-            part = D.skinny_slabs(a, P["o"])
-            if gate:
-                act = self._gate_up_split(splitk_add_rmsnorm(part, x, self.ln2[i], c.eps), i, gate)
+            part = slabs(a, P["o"])
+            if gate or wide:
+                act = splitk_add_rmsnorm(part, x, self.ln2[i], c.eps)
+                act = self._gate_up_split(act, i, gate) if gate else self._silu_mul(self._proj(act, i, "gate_up", True))
             else:
                 act = D.skinny_rows(x, P["gate_up"], splitk_add_squares(part, x), c.eps)
-            part = D.skinny_slabs(act, P["down"])
-            if m > 48 and i + 1 == c.layers:
+            part = slabs(act, P["down"])
+            if not raw and i + 1 == c.layers:
                 y = splitk_add_rmsnorm(part, x, self.norm, c.eps)
             else:
                 ss = splitk_add_squares(part, x)
@@ -855,7 +871,7 @@ class ServingModel:
             return self._proj(x, None, "lm", decode)
         if x.shape[0] <= 8 and D.few_takes(x.shape[0], self.packed_lm.n, self.packed_lm.k):
             return D.skinny_few(x, self.packed_lm, norm=True, eps=self.cfg.eps)
-        return D.skinny_rows(x, self.packed_lm, ss, self.cfg.eps)
+        return (D.wide_rows if x.shape[0] > D.SLAB_ROWS else D.skinny_rows)(x, self.packed_lm, ss, self.cfg.eps)
 
     def _tickets(self, block_tables):
         """Tickets of the step's own for the decode rows' attention, to be cleared with its first launch; None: it takes none."""

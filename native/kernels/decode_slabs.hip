@@ -1,4 +1,4 @@
-// Skinny products of up to 96 rows past skinny's tickets and barriers: x[M, K] . W^T, W packed as for decode.hip's skinny
+// Skinny products of up to 128 rows past skinny's tickets and barriers: x[M, K] . W^T, W packed as for decode.hip's skinny
 // ([N/16][K/32][64][8]), in K slices as fp32 partial sums P[slice][M][N] that the next launch adds (slabs), or whole, with the
 // RMSNorm and the gate of a fused layer in the epilogue (rows).
 //
@@ -18,7 +18,11 @@
 // launch (2048x8192 at 32 rows 15.0 us, the same product here 8.1); where the next launch passes over the output anyway it
 // reads a few MB instead. Workgroups by slices (kgs/ops/decode.py slab_split): about one a CU, and wide tiles only where N alone has enough.
 // From 33 rows on these beat the four-wave tiles of gemm_w4.h too, whose weights go through LDS; us at 64 and 90 rows, those / here:
-// 6144x4096 14.9, 20.2 / 12.6, 14.2; 4096x14336 25.1, 27.6 / 21.4, 24.2; whole: 28672x4096 51.6, 54.2 / 41.5, 45.2; 32000x4096 61 / 46.
+// 6144x4096 14.9, 20.2 / 12.6, 14.2; 4096x14336 25.1, 27.6 / 21.4, 24.2; whole: 28672x4096 51.6, 54.2 / 41.5, 45.2; 32000x4096 61 / 46; at 128 rows
+// 2048x2048 8.3 / 6.5, 3072x2048 9.7 / 7.5, 2048x8192 13.2 / 11.9, 6144x4096 18.5 / 17.1, 4096x14336 30.1 / 26.8; whole 32000x2048 34.5 / 30.9. There x counts
+// as W does: with x alone left out 16384x2048 takes 16.9 of 19.3 us, with W left out 13.1, without MFMAs or LDS reads 18.8 -- the L2s pass on x once a
+// workgroup, and deeper rings give nothing. K split over the waves with rings of their own (a quarter of the LDS reads) takes as long again as
+// the four-wave tiles.
 #include "decode_common.h"
 
 #include <type_traits>
@@ -174,7 +178,7 @@ __global__ __launch_bounds__(256, 2) void slabs(SlabArgs a) {
 }  // namespace kgs
 
 namespace {
-constexpr int SLAB_ROWS = 96;
+constexpr int SLAB_ROWS = 96, WIDE_ROWS = 128;
 
 template <int OUT>
 int launch_slabs(const kgs::dec::SlabArgs& a, int r, hipStream_t s) {
@@ -186,33 +190,31 @@ int launch_slabs(const kgs::dec::SlabArgs& a, int r, hipStream_t s) {
   if (a.M <= 16) return r == 1 ? run(slabs<1, 1, OUT>) : run(slabs<1, 2, OUT>);
   if (a.M <= 32) return r == 1 ? run(slabs<2, 1, OUT>) : run(slabs<2, 2, OUT>);
   if (a.M <= 64) return r == 1 ? run(slabs<4, 1, OUT>) : run(slabs<4, 2, OUT>);
-  return r == 1 ? run(slabs<6, 1, OUT>) : run(slabs<6, 2, OUT>);
+  if (a.M <= 96) return r == 1 ? run(slabs<6, 1, OUT>) : run(slabs<6, 2, OUT>);
+  if constexpr (OUT != OUT_GATED) return r == 1 ? run(slabs<8, 1, OUT>) : run(slabs<8, 2, OUT>);
+  return KGS_ERR_SHAPE;
 }
 
-int slab_shape(const void* wp, const void* x, const void* y, int M, int N, int K, long ldx, int r, int ns) {
-  if (M < 1 || M > SLAB_ROWS || N <= 0 || K <= 0 || (r != 1 && r != 2) || ns < 1 || N % (64 * r) || K % (128 * ns))
+int slab_shape(int most, const void* wp, const void* x, const void* y, int M, int N, int K, long ldx, int r, int ns) {
+  if (M < 1 || M > most || N <= 0 || K <= 0 || (r != 1 && r != 2) || ns < 1 || N % (64 * r) || K % (128 * ns))
     return KGS_ERR_SHAPE;
-  if (ldx < K || ldx > 1l << 23) return KGS_ERR_SHAPE;  // 32-bit offsets: x's 96 rows, and a wave's 32 rows of W, whose base has 64 bits
+  if (ldx < K || ldx > 1l << 23) return KGS_ERR_SHAPE;  // 32-bit offsets: x's rows, and a wave's 32 rows of W, whose base has 64 bits
   return (uintptr_t)wp % 16 || (uintptr_t)x % 16 || (uintptr_t)y % 16 || ldx % 8 ? KGS_ERR_ALIGN : 0;
 }
 }  // namespace
 
-// P[ns][M][N] (fp32) = the K slices' products of x[M, K] (rows ldx apart) and W^T, W packed as for kgs_skinny_gemm_bf16: up to 96
-// rows, r (1, 2) tiles of 16 W rows a wave, N a multiple of 64 r, K of 128 ns.
-KGS_EXPORT int kgs_skinny_slabs(const void* wp, const void* x, float* p, int M, int N, int K, long ldx, int r, int ns, hipStream_t s) {
+namespace {
+int parts(int most, const void* wp, const void* x, float* p, int M, int N, int K, long ldx, int r, int ns, hipStream_t s) {
   using namespace kgs::dec;
-  const int rc = slab_shape(wp, x, p, M, N, K, ldx, r, ns);
+  const int rc = slab_shape(most, wp, x, p, M, N, K, ldx, r, ns);
   if (rc) return rc;
   const SlabArgs a{(const unsigned short*)x, (const unsigned short*)wp, p, M, N, K, (int)ldx, ns, 0, nullptr, 0.f, 0.f, 0.f, 0};
   return launch_slabs<OUT_SLABS>(a, r, s);
 }
-
-// y[M, N] (bf16, rows ldy apart) = x[M, K] . W^T as kgs_skinny_slabs in one slice; sq: of x's RMSNorm (its weight folded into W) by
-// these sums of squares of its rows. epi: EPI_SWIGLU (with EPI_GELU or EPI_CLAMPED and limit): y is [M, N / 2].
-KGS_EXPORT int kgs_skinny_rows(const void* wp, const void* x, void* y, int M, int N, int K, long ldx, long ldy, int r, int epi,
-                               const float* sq, float eps, float limit, hipStream_t s) {
+int whole(int most, const void* wp, const void* x, void* y, int M, int N, int K, long ldx, long ldy, int r, int epi, const float* sq, float eps,
+          float limit, hipStream_t s) {
   using namespace kgs::dec;
-  const int rc = slab_shape(wp, x, y, M, N, K, ldx, r, 1);
+  const int rc = slab_shape(most, wp, x, y, M, N, K, ldx, r, 1);
   if (rc) return rc;
   const bool gated = epi & EPI_SWIGLU;
   if (ldy < (gated ? N / 2 : N)) return KGS_ERR_SHAPE;
@@ -220,4 +222,27 @@ KGS_EXPORT int kgs_skinny_rows(const void* wp, const void* x, void* y, int M, in
   if (epi & ~(EPI_SWIGLU | EPI_GELU | EPI_CLAMPED) || (epi && !gated)) return KGS_ERR_ARG;
   const SlabArgs a{(const unsigned short*)x, (const unsigned short*)wp, y, M, N, K, (int)ldx, 1, ldy, sq, 1.f / K, eps, limit, epi};
   return gated ? launch_slabs<OUT_GATED>(a, r, s) : launch_slabs<OUT_ROWS>(a, r, s);
+}
+}  // namespace
+
+// P[ns][M][N] (fp32) = the K slices' products of x[M, K] (rows ldx apart) and W^T, W packed as for kgs_skinny_gemm_bf16: up to 96
+// rows, r (1, 2) tiles of 16 W rows a wave, N a multiple of 64 r, K of 128 ns.
+KGS_EXPORT int kgs_skinny_slabs(const void* wp, const void* x, float* p, int M, int N, int K, long ldx, int r, int ns, hipStream_t s) {
+  return parts(SLAB_ROWS, wp, x, p, M, N, K, ldx, r, ns, s);
+}
+
+// y[M, N] (bf16, rows ldy apart) = x[M, K] . W^T as kgs_skinny_slabs in one slice; sq: of x's RMSNorm (its weight folded into W) by
+// these sums of squares of its rows. epi: EPI_SWIGLU (with EPI_GELU or EPI_CLAMPED and limit): y is [M, N / 2].
+KGS_EXPORT int kgs_skinny_rows(const void* wp, const void* x, void* y, int M, int N, int K, long ldx, long ldy, int r, int epi,
+                               const float* sq, float eps, float limit, hipStream_t s) {
+  return whole(SLAB_ROWS, wp, x, y, M, N, K, ldx, ldy, r, epi, sq, eps, limit, s);
+}
+
+// The same of up to 128 rows, without gates
+KGS_EXPORT int kgs_wide_slabs(const void* wp, const void* x, float* p, int M, int N, int K, long ldx, int r, int ns, hipStream_t s) {
+  return parts(WIDE_ROWS, wp, x, p, M, N, K, ldx, r, ns, s);
+}
+KGS_EXPORT int kgs_wide_rows(const void* wp, const void* x, void* y, int M, int N, int K, long ldx, long ldy, int r, const float* sq, float eps,
+                             hipStream_t s) {
+  return whole(WIDE_ROWS, wp, x, y, M, N, K, ldx, ldy, r, 0, sq, eps, 0.f, s);
 }

@@ -122,6 +122,26 @@ def test_what_the_rules_of_slices_take_the_kernel_takes():
                     assert lib.kgs_skinny_rows(1, 1, 1, m, n, k, k, n, tiles, 0, None, 0.0, 0.0, None) == align, (m, n, k)
 
 
+def test_what_the_rules_of_wide_slices_take_the_kernel_takes():
+    from kgs.ops import _lib
+
+    lib = _lib.lib()
+    align = lib.kgs_wide_slabs(1, 1, 1, 128, 64, 128, 128, 1, 1, None)
+    assert align not in (0, lib.kgs_wide_slabs(1, 1, 1, 129, 64, 128, 128, 1, 1, None))
+    for n in (64, 192, 2048, 4096, 4160, 28672, 128256, 1 << 20):
+        for k in (128, 384, 2048, 11008, 65536):
+            for m in (96, 97, 128, 129):
+                split, head = D.wide_split(m, n, k), D.head_pays(m, n, k)
+                assert (split is None) is (m not in (97, 128) or n % 64 != 0)
+                if split:
+                    assert lib.kgs_wide_slabs(1, 1, 1, m, n, k, k, *split, None) == align, (m, n, k)
+                if head:
+                    assert lib.kgs_wide_rows(1, 1, 1, m, n, k, k, n, D._rows_tiles(m, n, k, D.CUS), None, 0.0, None) == align, (m, n, k)
+    for m, n, k, pays in ((48, 32000, 4096, False), (49, 32000, 4096, True), (128, 32000, 2048, True), (64, 32000, 1024, False), (64, 128256, 4096, False),
+                          (100, 40960, 4096, False), (128, 64000, 4096, True), (129, 32000, 4096, False)):
+        assert D.head_pays(m, n, k) is pays, (m, n, k)
+
+
 def test_few_rows_keep_to_where_they_are_the_faster():
     """Beside skinny: not for wide weights of short sums, x that is long, strips at multiples of 256 KB; beside the library: neither long sums nor wide weights."""
     few = [(1, 28672, 4096), (8, 32000, 4096), (8, 16384, 2048), (1, 24576, 2048), (8, 10240, 1024), (16, 6144, 4096), (8, 4096, 14336), (1, 4096, 4096), (16, 2048, 3584),

@@ -111,6 +111,51 @@ def test_rotation_of_slices_as_of_the_whole_product(heads, kv, k, m):
     assert torch.equal(caches[0].data == 0, caches[1].data == 0)
 
 
+# one slice and eight, one and two tiles a wave, the last column tile full and of one row
+@pytest.mark.parametrize("n,k", ((64, 128), (2048, 2048), (4096, 384), (4224, 2048), (24576, 256)))
+@pytest.mark.parametrize("m", (97, 112, 113, 128))
+def test_wide_slices_and_products(n, k, m):
+    x, w = _operands(m, n, k, 3)
+    ns, pw = D.wide_split(m, n, k)[1], D.PackedWeight(w)
+    ref = x.double() @ w.double().T
+    got = D.wide_slabs(x, pw)
+    assert got.shape == (ns, m, n)
+    # as test_slices_add_to_the_product, whose bound holds for each slice
+    assert float((got.double().sum(0) - ref).abs().max()) <= 2.0 ** -24 * k * float(ref.abs().max())
+    y = D.wide_rows(x, pw)
+    assert bool(((y.double() - ref).abs() <= 2.0 ** -8 * ref.abs() + 2e-5 * ref.abs().max()).all())
+    sq = x.float().pow(2).sum(1)
+    normed = ref * torch.rsqrt(x.double().pow(2).mean(1, keepdim=True) + 1e-3)
+    assert bool(((D.wide_rows(x, pw, sq, 1e-3).double() - normed).abs() <= 2.0 ** -8 * normed.abs() + 2e-5 * normed.abs().max()).all())
+
+
+@pytest.mark.parametrize("rows", (97, 128))
+@pytest.mark.parametrize("inter", (1024, 8192))  # gate and up by the library and by the gate kernel
+def test_layers_of_wide_slices_as_the_others(rows, inter):
+    from kgs.models.llama import LlamaConfig
+    from kgs.serve.model import ServingModel
+
+    m = ServingModel(LlamaConfig(hidden=2048, layers=2, heads=16, kv_heads=4, intermediate=inter, vocab=12288), device="cuda", num_pages=256, max_model_len=1024)
+    m.cache.data.normal_()
+    assert m._wide(rows) and not m._wide(96) and not m._wide(129) and D.head_pays(rows, 12288, 2048)
+    i32 = dict(dtype=torch.int32, device="cuda")
+    ctx, tokens, slots = torch.randint(1, 300, (rows,), **i32), torch.randint(0, 512, (rows,), **i32), torch.full((rows,), -1, **i32)
+    tables = torch.stack([torch.randperm(255, device="cuda")[:16].int() + 1 for _ in range(rows)])
+    flat, pos = torch.randint(0, 512, (128,), **i32), torch.arange(128, **i32)
+    where = torch.where(pos < rows, pos + 32, -1).int()
+
+    def both():
+        m.cache.data[:, 1:32].zero_()
+        logits = m.prefill(flat, pos, where, [0], [rows], [128])
+        return m.decode(tokens, ctx - 1, slots, tables, ctx).float(), logits.float(), m.cache.data.float()
+
+    got, again = both(), both()
+    assert all(torch.equal(a, b) for a, b in zip(got, again))
+    m._wide = lambda rows: False
+    for a, b in zip(got, both()):
+        assert float((a - b).norm() / b.norm()) < 2e-2  # sums in another order, rounded to bf16 through two layers
+
+
 @pytest.mark.parametrize("cols", (2048, 4096, 6144, 8192))
 @pytest.mark.parametrize("parts", (1, 2, 4, 8, 16))
 def test_residual_add_of_slices_and_its_squares(parts, cols):

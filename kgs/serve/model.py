@@ -808,15 +808,18 @@ class ServingModel:
 
     def _slab_gate(self, m: int):
         """Gate and up of ``m`` rows of :meth:`_slab_layers`: a route of :meth:`_swiglu_route` on normed rows, or None: :func:`kgs.ops.decode.skinny_rows` on the
-        residual rows. The former from 49 rows on, where the route is the gate kernel or has tile-panel weights (us at 64 and 90 rows, so /
-        skinny_rows: 28672x4096 42.2, 48.9 / 45.9, 51.5, from row-major weights 51.6, 54.2; 16384x2048 15.9, 17.8 / 16.4, 19.2). Up to 48 rows as
-        the fused layers, whose products' inputs are not rounded behind the norm."""
+        residual rows, whose inputs are not rounded behind the norm. The former from 49 rows on, where the route has tile-panel weights or is the gate kernel, but of a
+        short K with many strips. us at 64 / 96 rows, route / skinny_rows: 28672x4096 from panels 42.3, 44.6 / 41.1, 45.7 (from row-major weights 51.5, 53.1); by the
+        gate kernel 16384x4096 30.0, 31.5 / 30.4, 31.3, 8192x2048 14.2, 13.8 / 13.3, 15.3, but 16384x2048 15.9, 17.6 / 15.1, 16.7, 11264x2048 15.3, 16.3 / 14.2, 15.8. A step of 49 /
+        64 rows, contexts of 300: 4096 wide, 14336 484, 512 / 493, 522; 8192 429, 443 / 438, 451; 2048 wide, 8192 263, 276 / 259, 274; 5632 260, 269 / 260, 267; 4096 236, 245 / 239, 248."""
         if m <= 48:
             return None
-        route = self._swiglu_route(m)
-        if route is None or route[1] > 1 or not (route[0] == GATE or (self.gate_up_panels is not None and route[0] in self.gate_up_panels[0])):
+        route, w = self._swiglu_route(m), self.packed[0]["gate_up"]
+        if route is None or route[1] > 1:
             return None
-        return route
+        if route[0] == GATE:
+            return None if w.n > 8192 and w.k <= 2048 else route
+        return route if self.gate_up_panels is not None and route[0] in self.gate_up_panels[0] else None
 
     def _slab_layers(self, tokens, positions, slots, attend, kind: str, keep=None, tickets=None):
         """As :meth:`_fused_layers`, for 33 to 128 rows: products in K slices that the rotation and the residual adds sum, gate and up whole. At one

@@ -596,7 +596,7 @@ WIDE_ROWS = 128
 @lru_cache(maxsize=4096)
 def slab_split(m: int, n: int, k: int, cus: int = CUS) -> tuple[int, int] | None:
     """(W tiles a wave, K slices) of :func:`skinny_slabs`, or None: up to 96 rows of W of 64 rows a workgroup (128 from N = 4096 on),
-    in as many slices, 16 at most and of 128 at least, as leave one workgroup a CU. us at 32 rows in 4 / 8 / 16 slices: 2048x8192 11.6 / 8.1 /
+    in as many slices, 16 at most and of 128 at least, as leave one workgroup a CU; the kernel then cuts W finer where that leaves CUs idle. us at 32 rows in 4 / 8 / 16 slices: 2048x8192 11.6 / 8.1 /
     8.2, 4096x14336 27.0 / 19.6 / 21.6, 6144x4096 10.8 / 12.8 / -."""
     return _split(n, k, cus) if 0 < m <= SLAB_ROWS else None
 
@@ -620,7 +620,7 @@ def _split(n: int, k: int, cus: int) -> tuple[int, int] | None:
 @lru_cache(maxsize=4096)
 def slab_rows_tiles(m: int, n: int, k: int, cus: int = CUS) -> int | None:
     """W tiles a wave of :func:`skinny_rows`, or None: two where 128 rows a workgroup are three quarters of the CUs or more (us at 48 rows with one /
-    two: 28672x4096 48.0 / 39.8, 16384x2048 14.5 / 19.1; at 32 and fewer 32000x2048 23.4 / 28.3)."""
+    two: 28672x4096 48.0 / 39.8, 16384x2048 14.5 / 19.1; at 32 and fewer 32000x2048 23.4 / 28.3). The kernel takes strips between them where they fill the CUs better."""
     return _rows_tiles(m, n, k, cus) if 0 < m <= SLAB_ROWS else None
 
 

@@ -2,7 +2,7 @@
 // ([N/16][K/32][64][8]), in K slices as fp32 partial sums P[slice][M][N] that the next launch adds (slabs), or whole, with the
 // RMSNorm and the gate of a fused layer in the epilogue (rows).
 //
-// A workgroup of four waves takes 64 R rows of W (wave w its R tiles) over one slice. W streams into registers, four k-steps
+// A workgroup of NW waves takes 16 NW R rows of W (wave w its R tiles) over one slice; the first four of them send for x. W streams into registers, four k-steps
 // ahead and past the caches; x comes by LDS-DMA, chunks of KC k-steps in three stages, one barrier
 // each, and a k-step's fragments are read from LDS under the MFMAs of the one before. All loads are counted by hand: the
 // compiler's own schedule waits for every load in flight before it stores a chunk (twice the time). W has to lie packed: 16 rows' pieces of 64
@@ -28,6 +28,7 @@
 #include <type_traits>
 
 namespace kgs {
+int cu_count();  // gemm_bf16.hip
 namespace dec {
 
 struct SlabArgs {
@@ -53,15 +54,15 @@ __device__ __forceinline__ void wait_loads() {
   asm volatile("" ::: "memory");
 }
 
-template <int MT, int R, int OUT>
-__global__ __launch_bounds__(256, 2) void slabs(SlabArgs a) {
+template <int MT, int R, int OUT, int NW>
+__global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void slabs(SlabArgs a) {
   constexpr int PF = 4, NB = 3, KC = MT == 1 ? 4 : 2, XL = KC * MT / 4;  // XL: pieces of x of a wave and chunk
   static_assert(PF % KC == 0 && PF >= (NB - 2) * KC);
   __shared__ __attribute__((aligned(16))) bf16x8 xs[NB][KC * MT * 64];
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), fr = lane & 15, fq = lane >> 4;
-  const int M = a.M, N = a.N, nkk = a.K / 32, tiles = N / (64 * R), tile = blockIdx.x % tiles, sl = blockIdx.x / tiles;
+  const int M = a.M, N = a.N, nkk = a.K / 32, T = N / (16 * R), strips = (T + NW - 1) / NW, sl = blockIdx.x / strips, at = blockIdx.x % strips * NW + w;
   const int nsteps = nkk / a.ns, k0 = sl * nsteps, nchunks = nsteps / KC;
-  const int nt0 = (tile * 4 + w) * R;
+  const int nt0 = min(at, T - 1) * R, rows = at < T ? M : 0;  // waves past the last tile repeat it and store nothing
   const auto rw = rsrc(a.w + (long)nt0 * nkk * 512, (unsigned)(R * nkk * 1024));
   const auto rx = rsrc(a.x, (unsigned)(((M - 1) * a.ldx + a.K) * 2));
   const int wo = lane * 16;
@@ -70,7 +71,7 @@ __global__ __launch_bounds__(256, 2) void slabs(SlabArgs a) {
   int xo[XL];
 #pragma unroll
   for (int i = 0; i < XL; ++i) {
-    const int f = w * XL + i, row = f % (2 * MT) * 8 + (lane >> 3), j = (lane & 7) ^ ((row >> 1) & 7);
+    const int f = (w & 3) * XL + i, row = f % (2 * MT) * 8 + (lane >> 3), j = (lane & 7) ^ ((row >> 1) & 7);
     xo[i] = 2 * (min(row, M - 1) * a.ldx + k0 * 32 + f / (2 * MT) * 64 + j * 8);  // rows from M on repeat the last one: never stored
   }
   const int ro[2] = {fr * 8 + (fq ^ (fr >> 1)), fr * 8 + ((4 + fq) ^ (fr >> 1))};  // of a fragment's 16 bytes: even and odd k-steps
@@ -80,71 +81,76 @@ __global__ __launch_bounds__(256, 2) void slabs(SlabArgs a) {
     for (int r = 0; r < R; ++r)
       wf[p][r] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(rw, wo, (r * nkk + k0 + s) * 1024, 2));
   };
-  int next = 0, to = 0;  // chunk to send for and its stage; past the end the last one again
-  auto send = [&] {
-#pragma unroll
-    for (int i = 0; i < XL; ++i) dma16(rx, &xs[to][(w * XL + i) * 64], xo[i], min(next, nchunks - 1) * (KC * 64));
-    ++next;
-    to = to == NB - 1 ? 0 : to + 1;
-  };
   f32x4v acc[R][MT];
 #pragma unroll
   for (int r = 0; r < R; ++r)
 #pragma unroll
     for (int c = 0; c < MT; ++c) acc[r][c] = f32x4v{0.f, 0.f, 0.f, 0.f};
-  // KC k-steps of weights at least between two chunks, as in the loop
-  send();
-  send();
-  __builtin_amdgcn_sched_barrier(0);
+  auto product = [&](auto sends) {
+    constexpr int XS = decltype(sends)::value ? XL : 0;  // a wave's DMAs a chunk
+    int next = 0, to = 0;  // chunk to send for and its stage; past the end the last one again
+    auto send = [&] {
 #pragma unroll
-  for (int g = 0; g < NB - 1; ++g) {
-#pragma unroll
-    for (int p = g * KC; p < (g == NB - 2 ? PF : (g + 1) * KC); ++p) load_w(p, p);
+      for (int i = 0; i < XS; ++i) dma16(rx, &xs[to][(w * XL + i) * 64], xo[i], min(next, nchunks - 1) * (KC * 64));
+      ++next;
+      to = to == NB - 1 ? 0 : to + 1;
+    };
+    // KC k-steps of weights at least between two chunks, as in the loop
+    send();
+    send();
     __builtin_amdgcn_sched_barrier(0);
-    if (g < NB - 2) send();
-    __builtin_amdgcn_sched_barrier(0);
-  }
-  wait_loads<(NB - 1) * XL + PF * R, false>();  // chunk 0
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-  int from = 0;  // stage being read
 #pragma unroll
-  for (int c = 0; c < MT; ++c) b[0][c] = xs[0][c * 128 + ro[0]];
-  // a round of the weights' ring; the last one sends for nothing: what it would fetch again is waited for, up to 1 us of a launch
-  auto round = [&](int s0, auto more) {
-    constexpr bool MORE = decltype(more)::value;
+    for (int g = 0; g < NB - 1; ++g) {
 #pragma unroll
-    for (int p = 0; p < PF; ++p) {
-      const int kk = p % KC;
-      if (MORE || p + 1 < PF) {
-        if (kk == KC - 1) {
-          // the next chunk: at least the weights of (NB - 1) KC - 1 k-steps and NB - 2 chunks were sent for after it. Every wave has read
-          // this one, so its stage is free
-          wait_loads<((NB - 1) * KC - 1) * R + (NB - 2) * XL, true>();
-          __builtin_amdgcn_s_barrier();
-          asm volatile("" ::: "memory");
-          from = from == NB - 1 ? 0 : from + 1;
-#pragma unroll
-          for (int c = 0; c < MT; ++c) b[(p + 1) & 1][c] = xs[from][c * 128 + ro[0]];
-          if constexpr (MORE) send();
-        } else {
-#pragma unroll
-          for (int c = 0; c < MT; ++c) b[(p + 1) & 1][c] = xs[from][((kk + 1) / 2 * MT + c) * 128 + ro[(kk + 1) & 1]];
-        }
-      }
+      for (int p = g * KC; p < (g == NB - 2 ? PF : (g + 1) * KC); ++p) load_w(p, p);
       __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int c = 0; c < MT; ++c)
-#pragma unroll
-        for (int r = 0; r < R; ++r) acc[r][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[p][r], b[p & 1][c], acc[r][c], 0, 0, 0);
-      if constexpr (MORE) load_w(p, s0 + PF + p);
+      if (g < NB - 2) send();
       __builtin_amdgcn_sched_barrier(0);
     }
+    wait_loads<(NB - 1) * XS + PF * R, false>();  // chunk 0
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    int from = 0;  // stage being read
+#pragma unroll
+    for (int c = 0; c < MT; ++c) b[0][c] = xs[0][c * 128 + ro[0]];
+    // a round of the weights' ring; the last one sends for nothing: what it would fetch again is waited for, up to 1 us of a launch
+    auto round = [&](int s0, auto more) {
+      constexpr bool MORE = decltype(more)::value;
+#pragma unroll
+      for (int p = 0; p < PF; ++p) {
+        const int kk = p % KC;
+        if (MORE || p + 1 < PF) {
+          if (kk == KC - 1) {
+            // the next chunk: at least the weights of (NB - 1) KC - 1 k-steps and NB - 2 chunks were sent for after it. Every wave has read
+            // this one, so its stage is free
+            wait_loads<((NB - 1) * KC - 1) * R + (NB - 2) * XS, true>();
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+            from = from == NB - 1 ? 0 : from + 1;
+#pragma unroll
+            for (int c = 0; c < MT; ++c) b[(p + 1) & 1][c] = xs[from][c * 128 + ro[0]];
+            if constexpr (MORE) send();
+          } else {
+#pragma unroll
+            for (int c = 0; c < MT; ++c) b[(p + 1) & 1][c] = xs[from][((kk + 1) / 2 * MT + c) * 128 + ro[(kk + 1) & 1]];
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int c = 0; c < MT; ++c)
+#pragma unroll
+          for (int r = 0; r < R; ++r) acc[r][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[p][r], b[p & 1][c], acc[r][c], 0, 0, 0);
+        if constexpr (MORE) load_w(p, s0 + PF + p);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    };
+    int s0 = 0;
+    for (; s0 + PF < nsteps; s0 += PF) round(s0, std::true_type{});
+    round(s0, std::false_type{});
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the tail's chunks land before LDS is released
   };
-  int s0 = 0;
-  for (; s0 + PF < nsteps; s0 += PF) round(s0, std::true_type{});
-  round(s0, std::false_type{});
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the tail's chunks land before LDS is released
+  if (NW == 4 || w < 4) product(std::true_type{});
+  else product(std::false_type{});
 #pragma unroll
   for (int c = 0; c < MT; ++c) {
     const int m = 16 * c + fr;
@@ -157,9 +163,9 @@ __global__ __launch_bounds__(256, 2) void slabs(SlabArgs a) {
       const f32x4v v = OUT == OUT_SLABS ? acc[r][c] : acc[r][c] * scale;
       const int nt = nt0 + r;
       if constexpr (OUT == OUT_SLABS) {
-        if (m < M) *(f32x4v*)((float*)a.y + ((long)sl * M + m) * N + 16 * nt + 4 * fq) = v;
+        if (m < rows) *(f32x4v*)((float*)a.y + ((long)sl * M + m) * N + 16 * nt + 4 * fq) = v;
       } else if constexpr (OUT == OUT_ROWS) {
-        if (m < M) *(uint2*)((unsigned short*)a.y + m * a.ldy + 16 * nt + 4 * fq) = uint2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+        if (m < rows) *(uint2*)((unsigned short*)a.y + m * a.ldy + 16 * nt + 4 * fq) = uint2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
       } else {  // a tile's gate rows in lanes 0 .. 31, their up rows in the lanes 32 on
         f32x4v u, o;
 #pragma unroll
@@ -168,7 +174,7 @@ __global__ __launch_bounds__(256, 2) void slabs(SlabArgs a) {
         for (int i = 0; i < 4; ++i)
           o[i] = (a.mode & EPI_CLAMPED) ? gate_clamped(v[i], u[i], a.limit)
                  : ((a.mode & EPI_GELU) ? gate_act<GATE_GELU>(v[i]) : gate_act<GATE_SILU>(v[i])) * u[i];
-        if (m < M && fq < 2) *(uint2*)((unsigned short*)a.y + m * a.ldy + 8 * nt + 4 * fq) = uint2{pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3])};
+        if (m < rows && fq < 2) *(uint2*)((unsigned short*)a.y + m * a.ldy + 8 * nt + 4 * fq) = uint2{pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3])};
       }
     }
   }
@@ -180,18 +186,41 @@ __global__ __launch_bounds__(256, 2) void slabs(SlabArgs a) {
 namespace {
 constexpr int SLAB_ROWS = 96, WIDE_ROWS = 128;
 
-template <int OUT>
-int launch_slabs(const kgs::dec::SlabArgs& a, int r, hipStream_t s) {
+// Waves of one tile each that cut T tiles of W finer than 64 r rows a workgroup, 0: none do. As few as leave one workgroup a CU: what 128 rows leave idle is
+// up to half of the CUs, and 64 rows that are more than the CUs wait for a second round. us at 24 / 64 / 90 / 128 rows by four waves / so: gated 28672x4096 (seven
+// waves) 40.2, 44.7, 49.9, 55.5 / 38.7, 42.0, 46.0, 52.6, 22016x4096 (six) 34.8, 42.9, 48.7, 53.8 / 31.5, 35.0, 39.7, 47.7; 6144x4096 in 4 slices (six) 11.5, 13.7, 15.6,
+// 17.6 / 11.0, 12.3, 13.7, 16.1, 5120x4096 (five) 10.6, 13.1, 14.8, 16.4 / 9.7, 11.0, 12.1, 13.2. Eight of one tile are as four of two. The slices stay: 3072x2048 in 8
+// by six waves 4.8, 6.0, 7.0, 8.1, in 4 by four 5.0, 5.9, 6.6, 7.4.
+inline int fine_waves(int T, int r, int ns) {
+  const int cus = kgs::cu_count();
+  if (r == 1 ? T / 4 * ns <= cus : T / 8 * ns > cus) return 0;
+  for (int nw = 5; nw < 8; ++nw)
+    if ((T + nw - 1) / nw * ns <= cus) return nw;
+  return 0;
+}
+
+template <int OUT, int MT>
+int launch_mt(const kgs::dec::SlabArgs& a, int r, hipStream_t s) {
   using namespace kgs::dec;
-  auto run = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, dim3(a.N / (64 * r) * a.ns), dim3(256), 0, s, a);
+  const int nw = fine_waves(a.N / 16, r, a.ns);
+  auto run = [&](auto kernel, int strip, int waves) {
+    hipLaunchKernelGGL(kernel, dim3((a.N + strip - 1) / strip * a.ns), dim3(64 * waves), 0, s, a);
     return (int)hipGetLastError();
   };
-  if (a.M <= 16) return r == 1 ? run(slabs<1, 1, OUT>) : run(slabs<1, 2, OUT>);
-  if (a.M <= 32) return r == 1 ? run(slabs<2, 1, OUT>) : run(slabs<2, 2, OUT>);
-  if (a.M <= 64) return r == 1 ? run(slabs<4, 1, OUT>) : run(slabs<4, 2, OUT>);
-  if (a.M <= 96) return r == 1 ? run(slabs<6, 1, OUT>) : run(slabs<6, 2, OUT>);
-  if constexpr (OUT != OUT_GATED) return r == 1 ? run(slabs<8, 1, OUT>) : run(slabs<8, 2, OUT>);
+  switch (nw) {
+    case 5: return run(slabs<MT, 1, OUT, 5>, 80, 5);
+    case 6: return run(slabs<MT, 1, OUT, 6>, 96, 6);
+    case 7: return run(slabs<MT, 1, OUT, 7>, 112, 7);
+  }
+  return r == 1 ? run(slabs<MT, 1, OUT, 4>, 64, 4) : run(slabs<MT, 2, OUT, 4>, 128, 4);
+}
+template <int OUT>
+int launch_slabs(const kgs::dec::SlabArgs& a, int r, hipStream_t s) {
+  if (a.M <= 16) return launch_mt<OUT, 1>(a, r, s);
+  if (a.M <= 32) return launch_mt<OUT, 2>(a, r, s);
+  if (a.M <= 64) return launch_mt<OUT, 4>(a, r, s);
+  if (a.M <= 96) return launch_mt<OUT, 6>(a, r, s);
+  if constexpr (OUT != kgs::dec::OUT_GATED) return launch_mt<OUT, 8>(a, r, s);
   return KGS_ERR_SHAPE;
 }
 

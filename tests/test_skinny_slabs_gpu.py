@@ -129,6 +129,26 @@ def test_wide_slices_and_products(n, k, m):
     assert bool(((D.wide_rows(x, pw, sq, 1e-3).double() - normed).abs() <= 2.0 ** -8 * normed.abs() + 2e-5 * normed.abs().max()).all())
 
 
+# five, six and seven waves of one tile: whole strips, and strips whose last waves have no tile (22016, 17408, 25088)
+@pytest.mark.parametrize("n,k", ((5120, 1024), (6144, 2048), (28672, 128), (22016, 384), (17408, 256), (25088, 128)))
+@pytest.mark.parametrize("m", (1, 17, 48, 65, 97, 128))
+def test_strips_that_fill_the_cus(n, k, m):
+    x, w = _operands(m, n, k, 4)
+    ref, pw = x.double() @ w.double().T, D.PackedWeight(w)
+    rule, slabs, rows = (D.slab_split, D.skinny_slabs, D.skinny_rows) if m <= 96 else (D.wide_split, D.wide_slabs, D.wide_rows)
+    got = slabs(x, pw)
+    assert got.shape == (rule(m, n, k)[1], m, n)
+    assert float((got.double().sum(0) - ref).abs().max()) <= 2.0 ** -24 * k * float(ref.abs().max())
+
+    def close(got, want, factors=1):  # as test_whole_products_and_gates
+        assert bool(((got.double() - want).abs() <= 2.0 ** -8 * want.abs() + 2e-5 * factors * want.abs().max()).all())
+
+    close(rows(x, pw), ref)
+    if m <= 96:
+        g, u = ref.chunk(2, 1)
+        close(D.skinny_rows(x, D.PackedWeight(w, swiglu=True)), torch.nn.functional.silu(g) * u, 4)
+
+
 @pytest.mark.parametrize("rows", (97, 128))
 @pytest.mark.parametrize("inter", (1024, 8192))  # gate and up by the library and by the gate kernel
 def test_layers_of_wide_slices_as_the_others(rows, inter):

@@ -142,7 +142,12 @@ __device__ __forceinline__ void store_row(const Args& a, int r, int col, const f
 // SW (a GateAct): B is a fused gate|up weight of N rows, gate rows first, and C [M, N / 2] holds
 // act(gate) * up; a tile stages both halves' rows in turn (gemm_w4.h). `bias` then points to the
 // clamped gate's limit.
-template <int EPI, int BM, int BN, bool SPLIT, bool DUAL, int SW, bool ONE>
+//
+// Two-stage tiles of a workgroup a CU take turns in one launch of a workgroup a CU (TURNS, take_turns): the last two K-steps of a tile send for the
+// first two K-tiles of the next and read its first fragments, so that between tiles a wave only has its epilogue. us, a
+// workgroup a tile / so: 3001 x 7000 x 200 28.2 / 24.0, 5000 x 5000 x 1000 56.9 / 53.7, 8192 x 14336 x 1024 203 / 193, 6000 x 9000 x 1000 120.5 / 111.0, 4032 x 6144 x 4096 171 /
+// 162, gated 3580 x 16384 x 2048 186.4 / 182.7, 2500 x 16000 x 4000 273 / 268. Bound by the matrix cores' power: what the gaps no longer cost comes off the clock.
+template <int EPI, int BM, int BN, bool SPLIT, bool DUAL, int SW, bool ONE, bool TURNS = false>
 __device__ __forceinline__ void tile_product(const Args& a) {
   constexpr int X = SW * 1000000, TN = SW ? BN / 2 : BN;  // TN: output columns of a tile
   const int cols = SW ? a.N / 2 : a.N;
@@ -154,10 +159,16 @@ __device__ __forceinline__ void tile_product(const Args& a) {
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int ntm = (a.M + BM - 1) / BM, ntn = (cols + TN - 1) / TN;
-  int slice, tm, tn;
-  if (a.tall) w4::tile_of<40000000, SPLIT>((int)blockIdx.x, (int)gridDim.x, ntm, ntn, slice, tm, tn);
-  else w4::tile_of<0, SPLIT>((int)blockIdx.x, (int)gridDim.x, ntm, ntn, slice, tm, tn);
-  const int m0 = tm * BM, n0 = tn * TN;
+  static_assert(!TURNS || (ONE && NS == 2 && !SPLIT));
+  int slice, m0, n0;
+  auto locate = [&](int id, int& m, int& n) {
+    int tm, tn;
+    if (a.tall) w4::tile_of<40000000, SPLIT>(id, (int)gridDim.x, ntm, ntn, slice, tm, tn);
+    else w4::tile_of<0, SPLIT>(id, (int)gridDim.x, ntm, ntn, slice, tm, tn);
+    m = tm * BM;
+    n = tn * TN;
+  };
+  locate((int)blockIdx.x, m0, n0);
   const int k0 = SPLIT ? slice * a.ks : 0;
   const int kn = SPLIT ? min(a.K - k0, a.ks) : a.K;  // this slice's valid K
 
@@ -168,11 +179,14 @@ __device__ __forceinline__ void tile_product(const Args& a) {
   c.wc = w & 1;
   c.nt = NS > 2 ? (kn + BK - 1) / BK : (kn + 2 * BK - 1) / (2 * BK) * 2;
   // resources end with the last valid element: nothing outside the operands is ever read
-  const int ra = min(a.M - m0, BM), rb = min(cols - n0, TN);
-  c.ra = __builtin_amdgcn_make_buffer_rsrc((void*)(a.A + (long)m0 * a.lda + k0), 0, ((ra - 1) * a.lda + kn) * 2, 0x00020000);
-  c.rb = __builtin_amdgcn_make_buffer_rsrc((void*)(a.B + (long)n0 * a.ldb + k0), 0, ((rb - 1) * a.ldb + kn) * 2, 0x00020000);
-  if constexpr (SW != 0)
-    c.rb2 = __builtin_amdgcn_make_buffer_rsrc((void*)(a.B + ((long)cols + n0) * a.ldb + k0), 0, ((rb - 1) * a.ldb + kn) * 2, 0x00020000);
+  auto bind = [&](int m, int n) {
+    const int ra = min(a.M - m, BM), rb = min(cols - n, TN);
+    c.ra = __builtin_amdgcn_make_buffer_rsrc((void*)(a.A + (long)m * a.lda + k0), 0, ((ra - 1) * a.lda + kn) * 2, 0x00020000);
+    c.rb = __builtin_amdgcn_make_buffer_rsrc((void*)(a.B + (long)n * a.ldb + k0), 0, ((rb - 1) * a.ldb + kn) * 2, 0x00020000);
+    if constexpr (SW != 0)
+      c.rb2 = __builtin_amdgcn_make_buffer_rsrc((void*)(a.B + ((long)cols + n) * a.ldb + k0), 0, ((rb - 1) * a.ldb + kn) * 2, 0x00020000);
+  };
+  bind(m0, n0);
   c.sa32 = 32 * a.lda * 2;
   c.sb32 = 32 * a.ldb * 2;
   const int row = w * 8 + (lane >> 3);
@@ -213,97 +227,113 @@ __device__ __forceinline__ void tile_product(const Args& a) {
   }
   __builtin_amdgcn_s_waitcnt(0xc07f);
 
-  // K-tiles past the end: outside the resources, so that their DMAs fetch nothing (a fetch is waited for at the end)
-  if constexpr (NS > 2) {
-    for (int t = 0; t < c.nt; t += NS) {
-      w4::static_for<0, NS>([&](auto st) {
-        constexpr int ST = decltype(st)::value;
-        if (ST && t + ST >= c.nt) return;
-        aim(t + ST + NS - 1);
-        w4::kstep1<BM, BN, ST, Kn::R, Kn::P, Kn::ORD, X, NS>(c, f0, f1, t + ST);
+  for (int id = (int)blockIdx.x;;) {
+    const int next = id + (int)gridDim.x;
+    const bool more = TURNS && next < ntm * ntn;
+    int m1 = 0, n1 = 0;
+    if (more) locate(next, m1, n1);
+    // K-tiles past the end: the next tile's, or outside the resources, so that their DMAs fetch nothing (a fetch is waited for at the end)
+    if constexpr (NS > 2) {
+      for (int t = 0; t < c.nt; t += NS) {
+        w4::static_for<0, NS>([&](auto st) {
+          constexpr int ST = decltype(st)::value;
+          if (ST && t + ST >= c.nt) return;
+          aim(t + ST + NS - 1);
+          w4::kstep1<BM, BN, ST, Kn::R, Kn::P, Kn::ORD, X, NS>(c, f0, f1, t + ST);
+        });
+      }
+    } else {
+      for (int t = 0; t + 2 < c.nt; t += 2) {
+        aim(t + 2);
+        w4::kstep<BM, BN, 0, Kn::B1, Kn::R, Kn::P, Kn::ORD, X>(c, f0, f1, t);
+        aim(t + 3);
+        w4::kstep<BM, BN, 1, Kn::B1, Kn::R, Kn::P, Kn::ORD, X>(c, f0, f1, t + 1);
+      }
+      if (more) bind(m1, n1);
+      aim(more ? 0 : c.nt);
+      w4::kstep<BM, BN, 0, Kn::B1, Kn::R, Kn::P, Kn::ORD, X>(c, f0, f1, -2);
+      aim(more ? 1 : c.nt);
+      w4::kstep<BM, BN, 1, Kn::B1, Kn::R, Kn::P, Kn::ORD, X>(c, f0, f1, -1);
+    }
+    if (!more) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the tail's DMAs (zeros) land before LDS is released
+    asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 3" ::: "memory");  // MFMA -> v_accvgpr_read hazard
+
+    const int mw = m0 + c.wr * (BM / 2) + fr, nw = n0 + c.wc * (TN / 2);
+    const int lc = (fq & 1) * 16 + (fq >> 1) * 8;  // this lane's 8 of a fragment pair's 32 columns
+    if constexpr (SW != 0) {
+      // output fragment q: gate fragment ng = 4 (q / 2) + q % 2 and the up fragment two further
+      const float limit = SW == GATE_CLAMPED ? *(const float*)a.bias : 0.f;
+      w4::static_for<0, MA>([&](auto ic) {
+        constexpr int i = decltype(ic)::value;
+        f32x4 v[NB];
+        w4::read_row<NB, i>(v);
+        if (mw + i * 16 >= a.M) return;
+        unsigned short* crow = (unsigned short*)a.C + (long)(mw + i * 16) * a.ldc;
+#pragma unroll
+        for (int q = 0; q < NB / 2; q += 2) {
+          uint2 o[2];
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            const int ng = 4 * ((q + h) / 2) + (q + h) % 2;
+            float r[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) r[e] = gated<SW>(v[ng][e], v[ng + 2][e], limit);
+            o[h] = make_uint2(pack_bf16x2(r[0], r[1]), pack_bf16x2(r[2], r[3]));
+          }
+          auto sx = __builtin_amdgcn_permlane16_swap(o[0].x, o[1].x, false, false);
+          auto sy = __builtin_amdgcn_permlane16_swap(o[0].y, o[1].y, false, false);
+          const int col = nw + q * 16 + lc;
+          if (col < cols) store8(crow, col, cols, a.vec, make_uint4(sx[0], sy[0], sx[1], sy[1]));
+        }
+      });
+    } else if constexpr (SPLIT) {
+      // ldc is a multiple of 8: a fragment's four columns are inside the row or all outside
+      float* part = (float*)a.C + (long)slice * a.M * a.ldc;
+      w4::static_for<0, MA>([&](auto ic) {
+        constexpr int i = decltype(ic)::value;
+        f32x4 v[NB];
+        w4::read_row<NB, i>(v);
+        if (mw + i * 16 >= a.M) return;
+        float* prow = part + (long)(mw + i * 16) * a.ldc;
+#pragma unroll
+        for (int n = 0; n < NB; ++n) {
+          const int col = nw + n * 16 + fq * 4;
+          if (col < a.ldc) *(f32x4*)(prow + col) = v[n];
+        }
+      });
+    } else {
+      float bv[NB][4];
+      load_bias<EPI, NB>(a, nw + fq * 4, bv);
+      w4::static_for<0, MA>([&](auto ic) {
+        constexpr int i = decltype(ic)::value;
+        const int r = mw + i * 16;
+        uint4 old[NB / 2];
+        load_old<EPI, NB>(a, r, nw + lc, old);
+        f32x4 v[NB];
+        w4::read_row<NB, i>(v);
+        store_row<EPI, NB, DUAL>(a, r, nw + lc, v, bv, old);
       });
     }
-  } else {
-    for (int t = 0; t < c.nt; t += 2) {
-      aim(t + 2);
-      w4::kstep<BM, BN, 0, Kn::B1, Kn::R, Kn::P, Kn::ORD, X>(c, f0, f1, t);
-      aim(t + 3);
-      w4::kstep<BM, BN, 1, Kn::B1, Kn::R, Kn::P, Kn::ORD, X>(c, f0, f1, t + 1);
-    }
+    if (!more) break;
+    id = next;
+    m0 = m1;
+    n0 = n1;
+    w4::static_for<0, MA * NB>([](auto q) { accr::zero<decltype(q)::value>(); });
+    asm volatile("s_nop 7" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0xc07f);
   }
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the tail's DMAs (zeros) land before LDS is released
-  asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 3" ::: "memory");  // MFMA -> v_accvgpr_read hazard
-
-  const int mw = m0 + c.wr * (BM / 2) + fr, nw = n0 + c.wc * (TN / 2);
-  const int lc = (fq & 1) * 16 + (fq >> 1) * 8;  // this lane's 8 of a fragment pair's 32 columns
-  if constexpr (SW != 0) {
-    // output fragment q: gate fragment ng = 4 (q / 2) + q % 2 and the up fragment two further
-    const float limit = SW == GATE_CLAMPED ? *(const float*)a.bias : 0.f;
-    w4::static_for<0, MA>([&](auto ic) {
-      constexpr int i = decltype(ic)::value;
-      f32x4 v[NB];
-      w4::read_row<NB, i>(v);
-      if (mw + i * 16 >= a.M) return;
-      unsigned short* crow = (unsigned short*)a.C + (long)(mw + i * 16) * a.ldc;
-#pragma unroll
-      for (int q = 0; q < NB / 2; q += 2) {
-        uint2 o[2];
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          const int ng = 4 * ((q + h) / 2) + (q + h) % 2;
-          float r[4];
-#pragma unroll
-          for (int e = 0; e < 4; ++e) r[e] = gated<SW>(v[ng][e], v[ng + 2][e], limit);
-          o[h] = make_uint2(pack_bf16x2(r[0], r[1]), pack_bf16x2(r[2], r[3]));
-        }
-        auto sx = __builtin_amdgcn_permlane16_swap(o[0].x, o[1].x, false, false);
-        auto sy = __builtin_amdgcn_permlane16_swap(o[0].y, o[1].y, false, false);
-        const int col = nw + q * 16 + lc;
-        if (col < cols) store8(crow, col, cols, a.vec, make_uint4(sx[0], sy[0], sx[1], sy[1]));
-      }
-    });
-    return;
-  }
-  if constexpr (SPLIT) {
-    // ldc is a multiple of 8: a fragment's four columns are inside the row or all outside
-    float* part = (float*)a.C + (long)slice * a.M * a.ldc;
-    w4::static_for<0, MA>([&](auto ic) {
-      constexpr int i = decltype(ic)::value;
-      f32x4 v[NB];
-      w4::read_row<NB, i>(v);
-      if (mw + i * 16 >= a.M) return;
-      float* prow = part + (long)(mw + i * 16) * a.ldc;
-#pragma unroll
-      for (int n = 0; n < NB; ++n) {
-        const int col = nw + n * 16 + fq * 4;
-        if (col < a.ldc) *(f32x4*)(prow + col) = v[n];
-      }
-    });
-    return;
-  }
-  float bv[NB][4];
-  load_bias<EPI, NB>(a, nw + fq * 4, bv);
-  w4::static_for<0, MA>([&](auto ic) {
-    constexpr int i = decltype(ic)::value;
-    const int r = mw + i * 16;
-    uint4 old[NB / 2];
-    load_old<EPI, NB>(a, r, nw + lc, old);
-    f32x4 v[NB];
-    w4::read_row<NB, i>(v);
-    store_row<EPI, NB, DUAL>(a, r, nw + lc, v, bv, old);
-  });
 }
 
 // gemm_nt_any: the tiles of plan, with or without slices; gemm_nt_mid: those between them (refine), one workgroup a CU, and 128x128 tiles that
-// are no more than the CUs
+// are no more than the CUs. TURNS: a kernel of its own, since a launch of one round loses up to 0.5 us by it (2080 x 5504 x 128 11.7 / 12.2)
 template <int EPI, int BM, int BN, bool SPLIT, bool DUAL, int SW = 0>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(waves_per_simd<BM, BN>(), waves_per_simd<BM, BN>())))
 void gemm_nt_any(Args a) {
   tile_product<EPI, BM, BN, SPLIT, DUAL, SW, waves_per_simd<BM, BN>() == 1>(a);
 }
-template <int EPI, int BM, int BN, bool DUAL, int SW = 0, bool SPLIT = false>
+template <int EPI, int BM, int BN, bool DUAL, int SW = 0, bool SPLIT = false, bool TURNS = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void gemm_nt_mid(Args a) {
-  tile_product<EPI, BM, BN, SPLIT, DUAL, SW, true>(a);
+  tile_product<EPI, BM, BN, SPLIT, DUAL, SW, true, TURNS>(a);
 }
 
 // The same product on 64x64 tiles, for grids that leave CUs idle at 128x128. What bounds such a
@@ -752,6 +782,23 @@ struct Plan {
 
 inline int ceil_div(long a, long b) { return (int)((a + b - 1) / b); }
 
+// Whether the tiles of an unsliced launch take turns (tile_product): two-stage ones of more than a round, but not for long sums over rows off the
+// 128-byte lines (us, a workgroup a tile / taking turns: 4000 x 6000 x 2000 108 / 116, of 2048 91.5 / 91.6; 6000 x 9000 x 3000 295 / 304.5, 6144 x 9216 x 3072 278 / 272)
+inline bool take_turns(const Args& a, long tiles) { return tiles > cu_count() && ((a.lda % 64 == 0 && a.ldb % 64 == 0) || a.K <= 1024); }
+
+// An unsliced launch of tiles with a CU each
+template <int EPI, int BM, int BN, bool DUAL, int SW = 0>
+void launch_mid(const Args& a, hipStream_t s) {
+  const long tiles = (long)ceil_div(a.M, BM) * (SW ? ceil_div(a.N / 2, BN / 2) : ceil_div(a.N, BN));
+  if constexpr (BN != 128)
+    if (take_turns(a, tiles)) {
+      hipLaunchKernelGGL((gemm_nt_mid<EPI, BM, BN, DUAL, SW, false, true>), dim3((unsigned)cu_count()), dim3(256), 0, s, a);
+      return;
+    }
+  if constexpr (BM == 256 && BN == 256) hipLaunchKernelGGL((gemm_nt_any<EPI, BM, BN, false, DUAL, SW>), dim3((unsigned)tiles), dim3(256), 0, s, a);
+  else hipLaunchKernelGGL((gemm_nt_mid<EPI, BM, BN, DUAL, SW>), dim3((unsigned)tiles), dim3(256), 0, s, a);
+}
+
 // Microseconds of a launch, as measured on an MI355X (weights streamed from HBM).
 inline double cost(long M, long N, long K, int bm, int bn, int ns, int cus) {
   const int pairs = ceil_div(K, 128), steps = 2 * ceil_div(pairs, ns);
@@ -804,14 +851,15 @@ inline Plan plan(long M, long N, long K, bool split, int cus) {
 // tile that these estimates choose takes 0.8 % more than the best one): start, what each round of workgroups
 // after the first adds, and a K-step alone on a CU and what the chip's filling adds to it. 128x128 tiles: of two
 // workgroups on a CU, and of the single ones that remain. Tiles of 128 columns (of 128x128 ones the single) scaled to their K-steps of one barrier, by 48
-// sizes: 0.33 + 0.13 full where 0.37 + 0.16, of 192 rows 0.40 + 0.25 / 0.42 + 0.29, 224 0.44 + 0.29 / 0.45 + 0.32, 256 0.46 + 0.35 / 0.49 + 0.36.
+// sizes: 0.33 + 0.13 full where 0.37 + 0.16, of 192 rows 0.40 + 0.25 / 0.42 + 0.29, 224 0.44 + 0.29 / 0.45 + 0.32, 256 0.46 + 0.35 / 0.49 + 0.36. Further rounds of two-stage
+// tiles cost 1.5 to 3 us less since they take turns.
 struct Tile {
   int bm, bn;
   double start, again, step, fill;
 };
-constexpr Tile TILES[] = {{256, 256, 7.12, 7.31, 0.88, 0.50}, {256, 128, 4.61, 4.53, 0.53, 0.28}, {128, 128, 3.5, 3.2, 0.97, 0},
-                          {192, 128, 4.15, 2.97, 0.42, 0.22}, {224, 128, 4.27, 3.53, 0.48, 0.25}, {192, 192, 5.02, 4.65, 0.56, 0.29},
-                          {224, 192, 5.40, 5.14, 0.61, 0.35}, {256, 192, 5.90, 5.94, 0.67, 0.38}, {224, 256, 6.49, 6.69, 0.78, 0.43}};
+constexpr Tile TILES[] = {{256, 256, 7.12, 5.3, 0.88, 0.50}, {256, 128, 4.61, 4.53, 0.53, 0.28}, {128, 128, 3.5, 3.2, 0.97, 0},
+                          {192, 128, 4.15, 2.97, 0.42, 0.22}, {224, 128, 4.27, 3.53, 0.48, 0.25}, {192, 192, 5.02, 3.3, 0.56, 0.29},
+                          {224, 192, 5.40, 3.6, 0.61, 0.35}, {256, 192, 5.90, 4.3, 0.67, 0.38}, {224, 256, 6.49, 4.9, 0.78, 0.43}};
 inline double tile_cost(const Tile& t, long M, long N, long K, int cus) {
   const long wg = (long)ceil_div(M, t.bm) * ceil_div(N, t.bn);
   const int steps = 2 * ceil_div(K, 128);
@@ -950,6 +998,7 @@ void launch_tile(const Args& a, int ns, hipStream_t s) {
       return;
     }
   if (ns > 1) hipLaunchKernelGGL((gemm_nt_any<EPI_NONE, BM, BN, true, false>), grid, dim3(256), 0, s, a);
+  else if constexpr (BN == 256) launch_mid<EPI, BM, BN, DUAL>(a, s);
   else hipLaunchKernelGGL((gemm_nt_any<EPI, BM, BN, false, DUAL>), grid, dim3(256), 0, s, a);
 }
 
@@ -974,10 +1023,8 @@ int launch(Args a, Plan p, float* ws, hipStream_t s) {
     g.ldc = ldp;
   }
   if (p.ns > 1 && (p.bn == 192 || (p.bm != 128 && p.bm != 256))) return KGS_ERR_ARG;  // slices run on plan's tiles
-#define KGS_MID(BM, BN)                                                                                                \
-  case BM << 16 | BN:                                                                                                  \
-    hipLaunchKernelGGL((gemm_nt_mid<EPI, BM, BN, DUAL>), dim3((unsigned)(ceil_div(a.M, BM) * ceil_div(a.N, BN))), dim3(256), 0, s, g); \
-    break
+#define KGS_MID(BM, BN) \
+  case BM << 16 | BN: launch_mid<EPI, BM, BN, DUAL>(g, s); break
   switch (p.bm << 16 | p.bn) {
     case 128 << 16 | 128: launch_tile<EPI, 128, 128, DUAL>(g, p.ns, s); break;
     case 256 << 16 | 128: launch_tile<EPI, 256, 128, DUAL>(g, p.ns, s); break;
@@ -1122,18 +1169,18 @@ int gemm_any_swiglu(const void* A, const void* B, void* C, int M, int N, int K, 
   const Plan p = gated_plan(M, N, K, cu_count());
   const dim3 grid((unsigned)(ceil_div(M, p.bm) * ceil_div(N / 2, p.bn / 2)));
   const bool one = (int)grid.x <= cu_count();
-#define KGS_SWK(BM, BN, ...) \
-  case BM << 16 | BN: hipLaunchKernelGGL((__VA_ARGS__>), grid, dim3(256), 0, s, a); break
-#define KGS_SWT(ACT)           \
-  if (one && p.bm == 128 && p.bn == 128) hipLaunchKernelGGL((gemm_nt_mid<EPI_NONE, 128, 128, false, ACT>), grid, dim3(256), 0, s, a); \
-  else switch (p.bm << 16 | p.bn) { \
-    KGS_SWK(128, 128, gemm_nt_any<EPI_NONE, 128, 128, false, false, ACT); \
-    KGS_SWK(256, 128, gemm_nt_any<EPI_NONE, 256, 128, false, false, ACT); \
-    KGS_SWK(256, 256, gemm_nt_any<EPI_NONE, 256, 256, false, false, ACT); \
-    KGS_SWK(192, 128, gemm_nt_mid<EPI_NONE, 192, 128, false, ACT);        \
-    KGS_SWK(224, 128, gemm_nt_mid<EPI_NONE, 224, 128, false, ACT);        \
-    KGS_SWK(224, 256, gemm_nt_mid<EPI_NONE, 224, 256, false, ACT);        \
-    default: return KGS_ERR_ARG;                                          \
+#define KGS_SWT(ACT)                                                                                                                     \
+  switch (p.bm << 16 | p.bn) {                                                                                                          \
+    case 128 << 16 | 128:                                                                                                               \
+      if (one) hipLaunchKernelGGL((gemm_nt_mid<EPI_NONE, 128, 128, false, ACT>), grid, dim3(256), 0, s, a);                             \
+      else hipLaunchKernelGGL((gemm_nt_any<EPI_NONE, 128, 128, false, false, ACT>), grid, dim3(256), 0, s, a);                          \
+      break;                                                                                                                            \
+    case 256 << 16 | 128: hipLaunchKernelGGL((gemm_nt_any<EPI_NONE, 256, 128, false, false, ACT>), grid, dim3(256), 0, s, a); break;    \
+    case 256 << 16 | 256: launch_mid<EPI_NONE, 256, 256, false, ACT>(a, s); break;                                                      \
+    case 192 << 16 | 128: launch_mid<EPI_NONE, 192, 128, false, ACT>(a, s); break;                                                      \
+    case 224 << 16 | 128: launch_mid<EPI_NONE, 224, 128, false, ACT>(a, s); break;                                                      \
+    case 224 << 16 | 256: launch_mid<EPI_NONE, 224, 256, false, ACT>(a, s); break;                                                      \
+    default: return KGS_ERR_ARG;                                                                                                        \
   }
   if (act == GATE_CLAMPED) {
     KGS_SWT(GATE_CLAMPED)
@@ -1143,7 +1190,6 @@ int gemm_any_swiglu(const void* A, const void* B, void* C, int M, int N, int K, 
     KGS_SWT(GATE_SILU)
   }
 #undef KGS_SWT
-#undef KGS_SWK
   return (int)hipGetLastError();
 }
 

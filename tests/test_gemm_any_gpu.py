@@ -92,6 +92,20 @@ def test_w4x_tiles_of_one_barrier_a_step(bm, bn, M, K):
             assert torch.equal(gemm_nt_w4x(a, w, bn=bn, bm=bm, nt_weights=nt), want)
 
 
+# more tiles than CUs, taking turns: two and three rounds, a last one of one tile and of most CUs; one, two and three pairs of K-tiles; off the lines
+@pytest.mark.parametrize("M,N,K", [(2049, 8200, 64), (4100, 4104, 128), (3001, 7000, 200), (5000, 8000, 264), (4000, 4200, 1096)])
+@pytest.mark.parametrize("bm,bn", [(256, 256), (224, 256), (192, 192)])
+def test_tiles_that_take_turns_keep_the_bits(bm, bn, M, N, K):
+    a, b, bias = rnd(M, K), rnd(N, K), torch.randn(N, device=DEV).bfloat16()
+    got, want = (torch.empty(M, N, device=DEV, dtype=torch.bfloat16) for _ in range(2))
+    for epi in (0, 2):
+        run_any(a, b, want, 128, 128, 1, bias, epi)  # a workgroup a tile
+        for _ in range(2):
+            got.fill_(7)
+            run_any(a, b, got, bm, bn, 1, bias, epi)
+            assert torch.equal(got, want)
+
+
 def tile(M, N, K, gated=False):
     from kgs.ops import _lib
 

@@ -596,25 +596,35 @@ WIDE_ROWS = 128
 @lru_cache(maxsize=4096)
 def slab_split(m: int, n: int, k: int, cus: int = CUS) -> tuple[int, int] | None:
     """(W tiles a wave, K slices) of :func:`skinny_slabs`, or None: up to 96 rows of W of 64 rows a workgroup (128 from N = 4096 on),
-    in as many slices, 16 at most and of 128 at least, as leave one workgroup a CU; the kernel then cuts W finer where that leaves CUs idle. us at 32 rows in 4 / 8 / 16 slices: 2048x8192 11.6 / 8.1 /
-    8.2, 4096x14336 27.0 / 19.6 / 21.6, 6144x4096 10.8 / 12.8 / -."""
-    return _split(n, k, cus) if 0 < m <= SLAB_ROWS else None
+    in as many slices, 16 at most and of 128 at least, as leave one workgroup a CU, or half as many where :func:`_split` says so; the kernel then cuts W finer where that leaves CUs idle.
+    us at 32 rows in 4 / 8 / 16 slices: 2048x8192 11.6 / 8.1 / 8.2, 4096x14336 27.0 / 19.6 / 21.6, 6144x4096 10.8 / 12.8 / -."""
+    return _split(m, n, k, cus) if 0 < m <= SLAB_ROWS else None
 
 
 def wide_split(m: int, n: int, k: int, cus: int = CUS) -> tuple[int, int] | None:
-    """:func:`slab_split` of :func:`wide_slabs`, 97 to 128 rows. The same split is the best there: us at 128 rows in 2 / 4 / 8 / 16 slices 2048x2048 9.0 /
+    """:func:`slab_split` of :func:`wide_slabs`, 97 to 128 rows. As many workgroups are the best there: us of the product alone at 128 rows in 2 / 4 / 8 / 16 slices 2048x2048 9.0 /
     6.7 / 6.5 / 8.4, 2048x8192 27.9 / 16.6 / 11.9 / 14.4, 6144x4096 by two tiles 23.6 / 17.1 / 20.3 (by one 18.6 in 2), 4096x14336 69 / 39.5 / 26.8 / 32.1."""
-    return _split(n, k, cus) if SLAB_ROWS < m <= WIDE_ROWS else None
+    return _split(m, n, k, cus) if SLAB_ROWS < m <= WIDE_ROWS else None
 
 
-def _split(n: int, k: int, cus: int) -> tuple[int, int] | None:
+def _split(m: int, n: int, k: int, cus: int) -> tuple[int, int] | None:
+    """(tiles of 64 rows to a strip, K slices). A slice more shortens the product and costs the launch that sums its parts, so the line lies where the two together are least.
+    us of the product with the residual add and norm behind it, at 24 / 64 / 96 / 128 rows:
+
+    * strips of 128 rows in 8 slices against strips of 64 in 4, as many workgroups: 4096x4096 13.2, 15.5, 17.7, 18.8 / 12.8, 13.9, 15.1, 16.8; 4096x2048 10.0, 13.0, 15.6, 18.0 /
+      8.9, 10.7, 12.4, 14.0; 4096x8192 17.7, 20.7, 22.8, 23.4 / 16.9, 19.0, 21.6, 23.3; but 4096x14336 24.6, 27.6, 29.2, 31.6 / 25.1, 27.8, 30.8, 33.9, so up to K = 8192; and
+      8192x8192 in 4 against 2 slices 30.1, 32.1, 33.9, 35.3 / 29.6, 30.7, 35.2, 39.5, so from 8 slices on;
+    * strips of 64 rows in 8 slices against 4: 2048x2048 7.2, 9.1, 10.7, 12.2 / 7.3, 8.3, 9.5, 10.7; 2048x1024 6.3, 8.1, 9.5, 11.0 / 6.1, 7.1, 8.3, 9.5 (at 33 rows 7.9 / 7.7 and
+      6.9 / 6.4, so above 32); but 2048x4096 8.9, 10.6, 12.1, 13.8 / 9.7, 10.9, 12.4, 14.1, so up to K = 2048."""
     r = 2 if n >= 4096 and n % 128 == 0 else 1
     if n <= 0 or k <= 0 or n % (64 * r) or k % 128:
         return None
     tiles, ns = n // (64 * r), 1
     while ns < 16 and 2 * ns * tiles <= cus and k % (256 * ns) == 0:
         ns *= 2
-    return r, ns
+    if r == 2 and ns >= 8 and k <= 8192:
+        return 1, ns // 2
+    return r, min(ns, 4) if m > 32 and k <= 2048 else ns
 
 
 @lru_cache(maxsize=4096)

@@ -791,8 +791,8 @@ class ServingModel:
 
     def _wide(self, m: int) -> bool:
         """Whether 97 to 128 rows take those layers, under the conditions of fewer; gate and up go by their routes on normed rows. Four
-        layers, us a decode step of 97 / 112 / 128 rows by split tiles / so, contexts of 300: 2048 wide, feed-forward 8192 339, 352, 370 / 314, 326, 337; 4096,
-        14336 636, 667, 701 / 600, 627, 659; 8192, 28672 1868, 1912, 1954 / 1726, 1795, 1828; prompts 4096 wide 598, 595, 595 / 531, 553, 577; 2048, 8192 419, 414, 414 / 428, 409,
+        layers, us a decode step of 97 / 128 rows by split tiles / so, contexts of 300: 2048 wide, feed-forward 8192 339, 370 / 312, 333; 4096,
+        14336 636, 701 / 593, 652; 8192, 28672 1868, 1954 / 1726, 1828; prompts 4096 wide 598, 595, 595 / 531, 553, 577; 2048, 8192 419, 414, 414 / 428, 409,
         410, which the host bounds. Not 11008, whose slices do not fill the CUs."""
         if self.packed is None or self.decode_fp8 or self.backend != "kgs" or not self.fuse_splitk or self.rope_attn or self.fused_max_batch <= 32:
             return False

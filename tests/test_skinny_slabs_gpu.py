@@ -30,6 +30,18 @@ def test_slices_add_to_the_product(n, k, m):
         assert float((got[i].double() - ref).abs().max()) <= 2.0 ** -24 * ks * float(ref.abs().max())
 
 
+# each side of the lines between 128-row strips in eight slices and 64-row ones in four, and between eight slices and four of a short K
+@pytest.mark.parametrize("m,n,k,split", ((1, 4096, 2048, (1, 4)), (96, 4096, 8192, (1, 4)), (96, 4096, 12288, (2, 8)), (33, 8192, 8192, (2, 4)), (97, 4096, 4096, (1, 4)),
+                                         (128, 4096, 16384, (2, 8)), (32, 2048, 2048, (1, 8)), (33, 2048, 2048, (1, 4)), (128, 2048, 1024, (1, 4)), (33, 2048, 4096, (1, 8)), (40, 1024, 512, (1, 4))))
+def test_fewer_slices(m, n, k, split):
+    x, w = _operands(m, n, k)
+    rule, slabs = (D.slab_split, D.skinny_slabs) if m <= 96 else (D.wide_split, D.wide_slabs)
+    assert rule(m, n, k) == split and (m > 96 or D.slabs_fill(m, n, k) or (n, k) == (1024, 512))
+    got, ks, ref = slabs(x, D.PackedWeight(w)), k // split[1], x.double() @ w.double().T
+    # fp32 sums of ks products of bf16 in each of the slices: the roundings of ks additions, on average their root
+    assert got.shape == (split[1], m, n) and float((got.double().sum(0) - ref).abs().max()) <= 2.0 ** -24 * ks * float(ref.abs().max())
+
+
 def test_what_slices_do_not_take():
     for m, n, k in ((0, 2048, 2048), (97, 2048, 2048), (8, 2080, 2048), (8, 2048, 2080)):
         assert D.slab_split(m, n, k) is None

@@ -169,7 +169,8 @@ def test_layers_of_wide_slices_as_the_others(rows, inter):
 
     m = ServingModel(LlamaConfig(hidden=2048, layers=2, heads=16, kv_heads=4, intermediate=inter, vocab=12288), device="cuda", num_pages=256, max_model_len=1024)
     m.cache.data.normal_()
-    assert m._wide(rows) and not m._wide(96) and not m._wide(129) and D.head_pays(rows, 12288, 2048)
+    assert m._wide(rows) and not m._wide(96) and not m._wide(129) and D.head_pays(rows, 12288, 2048) and not m._slab_prompts(rows)
+    m._slab_prompts = lambda rows: m._wide(rows)  # prompts as well, which the host bounds with layers of so few weights
     i32 = dict(dtype=torch.int32, device="cuda")
     ctx, tokens, slots = torch.randint(1, 300, (rows,), **i32), torch.randint(0, 512, (rows,), **i32), torch.full((rows,), -1, **i32)
     tables = torch.stack([torch.randperm(255, device="cuda")[:16].int() + 1 for _ in range(rows)])

@@ -86,6 +86,26 @@ def test_split_rule_stays_in_its_bounds(batch, kv, pages):
 
 
 @pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("lens,kv,pages", [([512], 8, 16), ([1, 0, 33, 512], 8, 16), ([70] * 8, 4, 16), ([992], 8, 31), ([1024], 8, 32), ([40, 513], 4, 32), ([2000], 8, 63)])
+def test_shorter_parts(lens, kv, pages, fp8):
+    """Few pairs in tables of 16 to 63 pages: parts with no page, with one and with all of theirs."""
+    from kgs.ops import decode as D
+
+    b = len(lens)
+    parts, waves = D.shorter_parts(b, kv, pages, 4 if fp8 else 8, fp8)
+    if pages < 32 or not fp8:
+        assert (parts, waves) == (4 if pages < 32 else 8, 4) and D.shorter_parts(33, 1, pages, 8, fp8)[1] == 8
+    g = torch.Generator(device=DEV).manual_seed(pages)
+    cache = torch.randn(70, kv, 2, 4096, device=DEV, generator=g).to(D.FP8 if fp8 else torch.bfloat16)
+    tables, ctx = torch.randint(0, 70, (b, pages), generator=g, device=DEV, dtype=torch.int32), torch.tensor(lens, device=DEV, dtype=torch.int32)
+    q = (2 * torch.randn(b, 4 * kv * 128, device=DEV, generator=g)).bfloat16()
+    got = D.paged_decode_attention(q, cache, tables, ctx, 4 * kv, kv)
+    want = D.ref_paged_decode(q, cache, tables, ctx.clamp(min=1), 4 * kv, kv)
+    want[ctx == 0] = 0
+    assert float((got.float() - want).abs().max()) < TOL
+
+
+@pytest.mark.parametrize("fp8", [False, True])
 @pytest.mark.parametrize("groups", [1, 639, 640, 1023, 1024, 1151, 1152, 1535, 1536, 2047, 2048, 8192])
 @pytest.mark.parametrize("pages", [1, 2, 3, 4, 5, 8, 9, 16, 17, 4096])
 def test_wave_rule(fp8, groups, pages):

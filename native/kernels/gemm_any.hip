@@ -147,19 +147,18 @@ __device__ __forceinline__ void store_row(const Args& a, int r, int col, const f
 // first two K-tiles of the next and read its first fragments, so that between tiles a wave only has its epilogue. us, a
 // workgroup a tile / so: 3001 x 7000 x 200 28.2 / 24.0, 5000 x 5000 x 1000 56.9 / 53.7, 8192 x 14336 x 1024 203 / 193, 6000 x 9000 x 1000 120.5 / 111.0, 4032 x 6144 x 4096 171 /
 // 162, gated 3580 x 16384 x 2048 186.4 / 182.7, 2500 x 16000 x 4000 273 / 268. Bound by the matrix cores' power: what the gaps no longer cost comes off the clock.
-template <int EPI, int BM, int BN, bool SPLIT, bool DUAL, int SW, bool ONE, bool TURNS = false>
+template <int EPI, int BM, int BN, bool SPLIT, bool DUAL, int SW, int NS, bool TURNS = false>
 __device__ __forceinline__ void tile_product(const Args& a) {
   constexpr int X = SW * 1000000, TN = SW ? BN / 2 : BN;  // TN: output columns of a tile
   const int cols = SW ? a.N / 2 : a.N;
   using S = w4::Shape<BM, BN>;
   using Kn = w4::Knobs<BM, BN>;
   constexpr int MA = S::MA, NB = S::NB, ND = w4::dma_per_stage<BM, BN>();
-  constexpr int NS = lds_stages<BM, BN, ONE>();
   __shared__ __attribute__((aligned(1024))) char smem[NS * S::STAGE];
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int ntm = (a.M + BM - 1) / BM, ntn = (cols + TN - 1) / TN;
-  static_assert(!TURNS || (ONE && NS == 2 && !SPLIT));
+  static_assert(!TURNS || (NS == 2 && !SPLIT));
   int slice, m0, n0;
   auto locate = [&](int id, int& m, int& n) {
     int tm, tn;
@@ -324,16 +323,25 @@ __device__ __forceinline__ void tile_product(const Args& a) {
   }
 }
 
-// gemm_nt_any: the tiles of plan, with or without slices; gemm_nt_mid: those between them (refine), one workgroup a CU, and 128x128 tiles that
-// are no more than the CUs. TURNS: a kernel of its own, since a launch of one round loses up to 0.5 us by it (2080 x 5504 x 128 11.7 / 12.2)
+// gemm_nt_any: the tiles of plan, with or without slices; gemm_nt_mid: those between them (refine), one workgroup a CU, on two stages; gemm_nt_deep: tiles
+// of 128 columns on the stages of lds_stages, 128x128 ones where they are no more than the CUs; gemm_nt_turn: tiles that take turns, kernels of their own,
+// since a launch of one round loses up to 0.5 us by it (2080 x 5504 x 128 11.7 / 12.2)
 template <int EPI, int BM, int BN, bool SPLIT, bool DUAL, int SW = 0>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(waves_per_simd<BM, BN>(), waves_per_simd<BM, BN>())))
 void gemm_nt_any(Args a) {
-  tile_product<EPI, BM, BN, SPLIT, DUAL, SW, waves_per_simd<BM, BN>() == 1>(a);
+  tile_product<EPI, BM, BN, SPLIT, DUAL, SW, lds_stages<BM, BN, waves_per_simd<BM, BN>() == 1>()>(a);
 }
-template <int EPI, int BM, int BN, bool DUAL, int SW = 0, bool SPLIT = false, bool TURNS = false>
+template <int EPI, int BM, int BN, bool DUAL, int SW = 0>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void gemm_nt_mid(Args a) {
-  tile_product<EPI, BM, BN, SPLIT, DUAL, SW, true, TURNS>(a);
+  tile_product<EPI, BM, BN, false, DUAL, SW, 2>(a);
+}
+template <int EPI, int BM, int BN, bool DUAL, int SW = 0, bool SPLIT = false>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void gemm_nt_deep(Args a) {
+  tile_product<EPI, BM, BN, SPLIT, DUAL, SW, lds_stages<BM, BN, true>()>(a);
+}
+template <int EPI, int BM, int BN, bool DUAL, int SW = 0>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void gemm_nt_turn(Args a) {
+  tile_product<EPI, BM, BN, false, DUAL, SW, 2, true>(a);
 }
 
 // The same product on 64x64 tiles, for grids that leave CUs idle at 128x128. What bounds such a
@@ -786,15 +794,19 @@ inline int ceil_div(long a, long b) { return (int)((a + b - 1) / b); }
 // 128-byte lines (us, a workgroup a tile / taking turns: 4000 x 6000 x 2000 108 / 116, of 2048 91.5 / 91.6; 6000 x 9000 x 3000 295 / 304.5, 6144 x 9216 x 3072 278 / 272)
 inline bool take_turns(const Args& a, long tiles) { return tiles > cu_count() && ((a.lda % 64 == 0 && a.ldb % 64 == 0) || a.K <= 1024); }
 
-// An unsliced launch of tiles with a CU each
+// An unsliced launch of tiles with a CU each; two stages hold all of a K up to 128
 template <int EPI, int BM, int BN, bool DUAL, int SW = 0>
 void launch_mid(const Args& a, hipStream_t s) {
   const long tiles = (long)ceil_div(a.M, BM) * (SW ? ceil_div(a.N / 2, BN / 2) : ceil_div(a.N, BN));
-  if constexpr (BN != 128)
+  if constexpr (BN != 128) {
     if (take_turns(a, tiles)) {
-      hipLaunchKernelGGL((gemm_nt_mid<EPI, BM, BN, DUAL, SW, false, true>), dim3((unsigned)cu_count()), dim3(256), 0, s, a);
+      hipLaunchKernelGGL((gemm_nt_turn<EPI, BM, BN, DUAL, SW>), dim3((unsigned)cu_count()), dim3(256), 0, s, a);
       return;
     }
+  } else if (a.K > 2 * BK) {
+    hipLaunchKernelGGL((gemm_nt_deep<EPI, BM, BN, DUAL, SW>), dim3((unsigned)tiles), dim3(256), 0, s, a);
+    return;
+  }
   if constexpr (BM == 256 && BN == 256) hipLaunchKernelGGL((gemm_nt_any<EPI, BM, BN, false, DUAL, SW>), dim3((unsigned)tiles), dim3(256), 0, s, a);
   else hipLaunchKernelGGL((gemm_nt_mid<EPI, BM, BN, DUAL, SW>), dim3((unsigned)tiles), dim3(256), 0, s, a);
 }
@@ -993,8 +1005,8 @@ void launch_tile(const Args& a, int ns, hipStream_t s) {
   const dim3 grid((unsigned)(ceil_div(a.M, BM) * ceil_div(a.N, BN) * ns));
   if constexpr (BM == 128 && BN == 128)
     if ((int)grid.x <= cu_count()) {
-      if (ns > 1) hipLaunchKernelGGL((gemm_nt_mid<EPI_NONE, BM, BN, false, 0, true>), grid, dim3(256), 0, s, a);
-      else hipLaunchKernelGGL((gemm_nt_mid<EPI, BM, BN, DUAL>), grid, dim3(256), 0, s, a);
+      if (ns > 1) hipLaunchKernelGGL((gemm_nt_deep<EPI_NONE, BM, BN, false, 0, true>), grid, dim3(256), 0, s, a);
+      else hipLaunchKernelGGL((gemm_nt_deep<EPI, BM, BN, DUAL>), grid, dim3(256), 0, s, a);
       return;
     }
   if (ns > 1) hipLaunchKernelGGL((gemm_nt_any<EPI_NONE, BM, BN, true, false>), grid, dim3(256), 0, s, a);
@@ -1172,7 +1184,7 @@ int gemm_any_swiglu(const void* A, const void* B, void* C, int M, int N, int K, 
 #define KGS_SWT(ACT)                                                                                                                     \
   switch (p.bm << 16 | p.bn) {                                                                                                          \
     case 128 << 16 | 128:                                                                                                               \
-      if (one) hipLaunchKernelGGL((gemm_nt_mid<EPI_NONE, 128, 128, false, ACT>), grid, dim3(256), 0, s, a);                             \
+      if (one) hipLaunchKernelGGL((gemm_nt_deep<EPI_NONE, 128, 128, false, ACT>), grid, dim3(256), 0, s, a);                            \
       else hipLaunchKernelGGL((gemm_nt_any<EPI_NONE, 128, 128, false, false, ACT>), grid, dim3(256), 0, s, a);                          \
       break;                                                                                                                            \
     case 256 << 16 | 128: hipLaunchKernelGGL((gemm_nt_any<EPI_NONE, 256, 128, false, false, ACT>), grid, dim3(256), 0, s, a); break;    \

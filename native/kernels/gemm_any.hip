@@ -49,6 +49,17 @@ struct Args {
   const float* alpha_ptr;
 };
 
+// The launch's arguments, read anew: behind the asm the compiler cannot know them for the ones that it has
+__device__ __forceinline__ Args again() {
+  typedef const Args __attribute__((address_space(4)))* Kernarg;
+  Kernarg p = (Kernarg)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  Args g;
+  __builtin_memcpy(&g, p, sizeof g);
+  return g;
+}
+__device__ __forceinline__ int ceil_div_dev(int a, int b) { return (a + b - 1) / b; }
+
 template <int BM, int BN>
 constexpr int waves_per_simd() { return BM == 128 && BN == 128 ? 2 : 1; }
 
@@ -145,56 +156,57 @@ __device__ __forceinline__ void store_row(const Args& a, int r, int col, const f
 //
 // Two-stage tiles of a workgroup a CU take turns in one launch of a workgroup a CU (TURNS, take_turns): the last two K-steps of a tile send for the
 // first two K-tiles of the next and read its first fragments, so that between tiles a wave only has its epilogue. us, a
-// workgroup a tile / so: 3001 x 7000 x 200 28.2 / 24.0, 5000 x 5000 x 1000 56.9 / 53.7, 8192 x 14336 x 1024 203 / 193, 6000 x 9000 x 1000 120.5 / 111.0, 4032 x 6144 x 4096 171 /
-// 162, gated 3580 x 16384 x 2048 186.4 / 182.7, 2500 x 16000 x 4000 273 / 268. Bound by the matrix cores' power: what the gaps no longer cost comes off the clock.
+// workgroup a tile / so: 3001 x 7000 x 200 23.4 / 21.3, 5000 x 5000 x 1000 56.1 / 54.1, 6000 x 9000 x 1000 120.8 / 114.6, 8192 x 14336 x 1024 227 / 213. Bound by
+// the matrix cores' power: what the gaps no longer cost comes off the clock. Tiles and resources are worked out from the arguments read anew at each turn:
+// held through the K loop and the stores they spilled 26 to 53 scalar registers, and up to 8 in kernels of one tile that shared the loop.
 template <int EPI, int BM, int BN, bool SPLIT, bool DUAL, int SW, int NS, bool TURNS = false>
 __device__ __forceinline__ void tile_product(const Args& a) {
   constexpr int X = SW * 1000000, TN = SW ? BN / 2 : BN;  // TN: output columns of a tile
-  const int cols = SW ? a.N / 2 : a.N;
   using S = w4::Shape<BM, BN>;
   using Kn = w4::Knobs<BM, BN>;
   constexpr int MA = S::MA, NB = S::NB, ND = w4::dma_per_stage<BM, BN>();
+  static_assert(!TURNS || (NS == 2 && !SPLIT));
   __shared__ __attribute__((aligned(1024))) char smem[NS * S::STAGE];
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int ntm = (a.M + BM - 1) / BM, ntn = (cols + TN - 1) / TN;
-  static_assert(!TURNS || (NS == 2 && !SPLIT));
-  int slice, m0, n0;
-  auto locate = [&](int id, int& m, int& n) {
+  int slice = 0, m0, n0;
+  auto locate = [&](const Args& g, int id, int& m, int& n) {
+    const int ntm = (g.M + BM - 1) / BM, ntn = ((SW ? g.N / 2 : g.N) + TN - 1) / TN;
     int tm, tn;
-    if (a.tall) w4::tile_of<40000000, SPLIT>(id, (int)gridDim.x, ntm, ntn, slice, tm, tn);
+    if (g.tall) w4::tile_of<40000000, SPLIT>(id, (int)gridDim.x, ntm, ntn, slice, tm, tn);
     else w4::tile_of<0, SPLIT>(id, (int)gridDim.x, ntm, ntn, slice, tm, tn);
     m = tm * BM;
     n = tn * TN;
   };
-  locate((int)blockIdx.x, m0, n0);
+  locate(a, (int)blockIdx.x, m0, n0);
   const int k0 = SPLIT ? slice * a.ks : 0;
-  const int kn = SPLIT ? min(a.K - k0, a.ks) : a.K;  // this slice's valid K
+  int kn = SPLIT ? min(a.K - k0, a.ks) : a.K;  // this slice's valid K
 
   Ctx c;
   c.smem = smem;
   c.w = w;
   c.wr = w >> 1;
   c.wc = w & 1;
-  c.nt = NS > 2 ? (kn + BK - 1) / BK : (kn + 2 * BK - 1) / (2 * BK) * 2;
   // resources end with the last valid element: nothing outside the operands is ever read
-  auto bind = [&](int m, int n) {
-    const int ra = min(a.M - m, BM), rb = min(cols - n, TN);
-    c.ra = __builtin_amdgcn_make_buffer_rsrc((void*)(a.A + (long)m * a.lda + k0), 0, ((ra - 1) * a.lda + kn) * 2, 0x00020000);
-    c.rb = __builtin_amdgcn_make_buffer_rsrc((void*)(a.B + (long)n * a.ldb + k0), 0, ((rb - 1) * a.ldb + kn) * 2, 0x00020000);
+  auto bind = [&](const Args& g, int m, int n) {
+    if constexpr (TURNS) kn = g.K;
+    c.nt = NS > 2 ? (kn + BK - 1) / BK : (kn + 2 * BK - 1) / (2 * BK) * 2;
+    c.sa32 = 32 * g.lda * 2;
+    c.sb32 = 32 * g.ldb * 2;
+    const int cols = SW ? g.N / 2 : g.N, ra = min(g.M - m, BM), rb = min(cols - n, TN);
+    c.ra = __builtin_amdgcn_make_buffer_rsrc((void*)(g.A + (long)m * g.lda + k0), 0, ((ra - 1) * g.lda + kn) * 2, 0x00020000);
+    c.rb = __builtin_amdgcn_make_buffer_rsrc((void*)(g.B + (long)n * g.ldb + k0), 0, ((rb - 1) * g.ldb + kn) * 2, 0x00020000);
     if constexpr (SW != 0)
-      c.rb2 = __builtin_amdgcn_make_buffer_rsrc((void*)(a.B + ((long)cols + n) * a.ldb + k0), 0, ((rb - 1) * a.ldb + kn) * 2, 0x00020000);
+      c.rb2 = __builtin_amdgcn_make_buffer_rsrc((void*)(g.B + ((long)cols + n) * g.ldb + k0), 0, ((rb - 1) * g.ldb + kn) * 2, 0x00020000);
   };
-  bind(m0, n0);
-  c.sa32 = 32 * a.lda * 2;
-  c.sb32 = 32 * a.ldb * 2;
+  bind(a, m0, n0);
   const int row = w * 8 + (lane >> 3);
   const int ch = ((lane & 7) ^ ((row >> 1) & 7)) * 8;  // first column of this lane's chunk in a K-tile
   const int voa = (row * a.lda + ch) * 2, vob = (row * a.ldb + ch) * 2;
   const int fr = lane & 15, fq = lane >> 4;
   c.ro0 = fr * 128 + ((fq ^ (fr >> 1)) * 16);
   c.ro1 = fr * 128 + (((4 + fq) ^ (fr >> 1)) * 16);
-  // offsets of the next DMAs: outside the resources where K-tile kt's chunk lies past K
+  // offsets of the next DMAs: outside the resources where K-tile kt's chunk lies past K, so that nothing is fetched (a fetch is waited for at the end)
   auto aim = [&](int kt) {
     const bool in = kt * BK + ch < kn;
     c.voa = in ? voa : OOB;
@@ -226,48 +238,26 @@ __device__ __forceinline__ void tile_product(const Args& a) {
   }
   __builtin_amdgcn_s_waitcnt(0xc07f);
 
-  for (int id = (int)blockIdx.x;;) {
-    const int next = id + (int)gridDim.x;
-    const bool more = TURNS && next < ntm * ntn;
-    int m1 = 0, n1 = 0;
-    if (more) locate(next, m1, n1);
-    // K-tiles past the end: the next tile's, or outside the resources, so that their DMAs fetch nothing (a fetch is waited for at the end)
-    if constexpr (NS > 2) {
-      for (int t = 0; t < c.nt; t += NS) {
-        w4::static_for<0, NS>([&](auto st) {
-          constexpr int ST = decltype(st)::value;
-          if (ST && t + ST >= c.nt) return;
-          aim(t + ST + NS - 1);
-          w4::kstep1<BM, BN, ST, Kn::R, Kn::P, Kn::ORD, X, NS>(c, f0, f1, t + ST);
-        });
-      }
-    } else {
-      for (int t = 0; t + 2 < c.nt; t += 2) {
-        aim(t + 2);
-        w4::kstep<BM, BN, 0, Kn::B1, Kn::R, Kn::P, Kn::ORD, X>(c, f0, f1, t);
-        aim(t + 3);
-        w4::kstep<BM, BN, 1, Kn::B1, Kn::R, Kn::P, Kn::ORD, X>(c, f0, f1, t + 1);
-      }
-      if (more) bind(m1, n1);
-      aim(more ? 0 : c.nt);
-      w4::kstep<BM, BN, 0, Kn::B1, Kn::R, Kn::P, Kn::ORD, X>(c, f0, f1, -2);
-      aim(more ? 1 : c.nt);
-      w4::kstep<BM, BN, 1, Kn::B1, Kn::R, Kn::P, Kn::ORD, X>(c, f0, f1, -1);
-    }
-    if (!more) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the tail's DMAs (zeros) land before LDS is released
-    asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 3" ::: "memory");  // MFMA -> v_accvgpr_read hazard
-
-    const int mw = m0 + c.wr * (BM / 2) + fr, nw = n0 + c.wc * (TN / 2);
+  // K-steps of K-tiles t, t + 1, which send for K-tiles s and s + 1
+  auto pair = [&](int s) {
+    aim(s);
+    w4::kstep<BM, BN, 0, Kn::B1, Kn::R, Kn::P, Kn::ORD, X>(c, f0, f1, s - 2);
+    aim(s + 1);
+    w4::kstep<BM, BN, 1, Kn::B1, Kn::R, Kn::P, Kn::ORD, X>(c, f0, f1, s - 1);
+  };
+  auto store = [&](const Args& g, int m, int n) {
+    const int mw = m + c.wr * (BM / 2) + fr, nw = n + c.wc * (TN / 2);
     const int lc = (fq & 1) * 16 + (fq >> 1) * 8;  // this lane's 8 of a fragment pair's 32 columns
     if constexpr (SW != 0) {
       // output fragment q: gate fragment ng = 4 (q / 2) + q % 2 and the up fragment two further
-      const float limit = SW == GATE_CLAMPED ? *(const float*)a.bias : 0.f;
+      const int cols = g.N / 2;
+      const float limit = SW == GATE_CLAMPED ? *(const float*)g.bias : 0.f;
       w4::static_for<0, MA>([&](auto ic) {
         constexpr int i = decltype(ic)::value;
         f32x4 v[NB];
         w4::read_row<NB, i>(v);
-        if (mw + i * 16 >= a.M) return;
-        unsigned short* crow = (unsigned short*)a.C + (long)(mw + i * 16) * a.ldc;
+        if (mw + i * 16 >= g.M) return;
+        unsigned short* crow = (unsigned short*)g.C + (long)(mw + i * 16) * g.ldc;
 #pragma unroll
         for (int q = 0; q < NB / 2; q += 2) {
           uint2 o[2];
@@ -282,44 +272,82 @@ __device__ __forceinline__ void tile_product(const Args& a) {
           auto sx = __builtin_amdgcn_permlane16_swap(o[0].x, o[1].x, false, false);
           auto sy = __builtin_amdgcn_permlane16_swap(o[0].y, o[1].y, false, false);
           const int col = nw + q * 16 + lc;
-          if (col < cols) store8(crow, col, cols, a.vec, make_uint4(sx[0], sy[0], sx[1], sy[1]));
+          if (col < cols) store8(crow, col, cols, g.vec, make_uint4(sx[0], sy[0], sx[1], sy[1]));
         }
       });
     } else if constexpr (SPLIT) {
       // ldc is a multiple of 8: a fragment's four columns are inside the row or all outside
-      float* part = (float*)a.C + (long)slice * a.M * a.ldc;
+      float* part = (float*)g.C + (long)slice * g.M * g.ldc;
       w4::static_for<0, MA>([&](auto ic) {
         constexpr int i = decltype(ic)::value;
         f32x4 v[NB];
         w4::read_row<NB, i>(v);
-        if (mw + i * 16 >= a.M) return;
-        float* prow = part + (long)(mw + i * 16) * a.ldc;
+        if (mw + i * 16 >= g.M) return;
+        float* prow = part + (long)(mw + i * 16) * g.ldc;
 #pragma unroll
-        for (int n = 0; n < NB; ++n) {
-          const int col = nw + n * 16 + fq * 4;
-          if (col < a.ldc) *(f32x4*)(prow + col) = v[n];
+        for (int q = 0; q < NB; ++q) {
+          const int col = nw + q * 16 + fq * 4;
+          if (col < g.ldc) *(f32x4*)(prow + col) = v[q];
         }
       });
     } else {
       float bv[NB][4];
-      load_bias<EPI, NB>(a, nw + fq * 4, bv);
+      load_bias<EPI, NB>(g, nw + fq * 4, bv);
       w4::static_for<0, MA>([&](auto ic) {
         constexpr int i = decltype(ic)::value;
         const int r = mw + i * 16;
         uint4 old[NB / 2];
-        load_old<EPI, NB>(a, r, nw + lc, old);
+        load_old<EPI, NB>(g, r, nw + lc, old);
         f32x4 v[NB];
         w4::read_row<NB, i>(v);
-        store_row<EPI, NB, DUAL>(a, r, nw + lc, v, bv, old);
+        store_row<EPI, NB, DUAL>(g, r, nw + lc, v, bv, old);
       });
     }
-    if (!more) break;
-    id = next;
-    m0 = m1;
-    n0 = n1;
-    w4::static_for<0, MA * NB>([](auto q) { accr::zero<decltype(q)::value>(); });
-    asm volatile("s_nop 7" ::: "memory");
-    __builtin_amdgcn_s_waitcnt(0xc07f);
+  };
+  auto settle = [] { asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 3" ::: "memory"); };  // MFMA -> v_accvgpr_read hazard
+
+  if constexpr (!TURNS) {
+    if constexpr (NS > 2) {
+      for (int t = 0; t < c.nt; t += NS) {
+        w4::static_for<0, NS>([&](auto st) {
+          constexpr int ST = decltype(st)::value;
+          if (ST && t + ST >= c.nt) return;
+          aim(t + ST + NS - 1);
+          w4::kstep1<BM, BN, ST, Kn::R, Kn::P, Kn::ORD, X, NS>(c, f0, f1, t + ST);
+        });
+      }
+    } else {
+      for (int t = 0; t < c.nt; t += 2) pair(t + 2);
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the tail's DMAs (zeros) land before LDS is released
+    settle();
+    store(a, m0, n0);
+  } else {
+    for (int id = (int)blockIdx.x;;) {
+      for (int t = 0; t + 2 < c.nt; t += 2) pair(t + 2);
+      const int next = id + (int)gridDim.x;
+      // the arguments again, instead of registers that hold them through the K-steps
+      const Args g = again();
+      const bool more = next < ceil_div_dev(g.M, BM) * ceil_div_dev(SW ? g.N / 2 : g.N, TN);
+      int m1 = 0, n1 = 0;
+      if (more) {
+        locate(g, next, m1, n1);
+        bind(g, m1, n1);
+      }
+      pair(more ? 0 : c.nt);
+      if (!more) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // as above
+      settle();
+      const Args h = again();
+      store(h, m0, n0);
+      if (!more) break;
+      id = next;
+      m0 = m1;
+      n0 = n1;
+      bind(again(), m0, n0);  // again: not held through the stores
+      w4::static_for<0, MA * NB>([](auto q) { accr::zero<decltype(q)::value>(); });
+      asm volatile("s_nop 7" ::: "memory");
+      __builtin_amdgcn_s_waitcnt(0xc07f);
+    }
   }
 }
 

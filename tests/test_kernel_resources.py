@@ -302,6 +302,32 @@ def test_tiles_between_the_three_keep_their_accumulators(gemm_build):
         assert r["VGPRs Spill"] == 0 and r["SGPRs Spill"] == 0 and r["LDS Size"] == 2 * (bm + bn) * 128, (name, r)
 
 
+def test_deep_tiles_and_tiles_that_take_turns_keep_their_accumulators(gemm_build):
+    """gemm_nt_deep: two tiles x (6 epilogues, 3 with two outputs, 3 gates), 128x128 with slices as well; gemm_nt_turn: five tiles x (6, 3) and two of them
+    x 3 gates. The rules of gemm_nt_mid; nor does one of gemm_nt_any hold so much between its loops that scalar registers spill."""
+    res, asm = gemm_build
+    funcs = _functions(asm, r"gemm_nt_(deep|turn)I")
+    assert len([n for n in funcs if "gemm_nt_deepI" in n]) == 3 * (6 + 3 + 3) + 1, sorted(funcs)
+    assert len([n for n in funcs if "gemm_nt_turnI" in n]) == 5 * (6 + 3) + 2 * 3, sorted(funcs)
+    for name, body in funcs.items():
+        kind, bm, bn = re.search(r"gemm_nt_(deep|turn)ILi\dELi(\d+)ELi(\d+)E", name).groups()
+        bm, bn = int(bm), int(bn)
+        seen, stray = _stray_agpr_lines(body)
+        assert seen >= bm // 32 * (bn // 32) * 4 and not stray, (name, seen, stray[:5])
+        lines = body.splitlines()
+        assert not any("v_accvgpr_mov" in ln for ln in lines), name
+        assert all(re.search(r"v_accvgpr_write_b32 a\d+, 0\b", ln) for ln in lines if "v_accvgpr_write" in ln), name
+        mfma, pads = -1, -1  # a fragment is read behind a padding that follows every MFMA above it
+        for i, ln in enumerate(lines):
+            mfma, pads = i if "v_mfma" in ln else mfma, i if "s_nop 7" in ln else pads
+            assert "v_accvgpr_read" not in ln or pads > mfma, (name, i, ln)
+        r, stages = res[name], 2 if kind == "turn" else 4 if bm == 128 else 3
+        assert r["VGPRs Spill"] == 0 and r["SGPRs Spill"] == 0, (name, r)
+        assert 0 <= r["LDS Size"] - stages * (bm + bn) * 128 <= 16, (name, r)
+    spilt = {n: r["SGPRs Spill"] for n, r in res.items() if "gemm_nt_anyI" in n and r["SGPRs Spill"]}
+    assert not spilt, spilt
+
+
 def _vregs(text: str) -> set:
     out = set()
     for a, b in re.findall(r"(?<![\w.])v\[(\d+):(\d+)\]", text):

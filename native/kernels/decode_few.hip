@@ -64,12 +64,14 @@ __device__ __forceinline__ void each_of(std::integer_sequence<int, I...>, F&& f)
 template <int N, typename F>
 __device__ __forceinline__ void each(F&& f) { each_of(std::make_integer_sequence<int, N>{}, f); }
 
-// MT column tiles of 16 rows of x. LX: x by LDS, in XP pieces of 8 rows of 64 values for two k-steps; else straight from memory in operand order
-template <int R, int MT, int NW, int PF, bool LX, bool ROPE, bool OWN>
+// MT column tiles of 16 rows of x. LX: x by LDS, in XP pieces of 8 rows of 64 values for two k-steps; else straight from memory in operand order. PARTS: K's
+// parts, which are summed apart and added in their order (few_parts); a wave takes as many as are left for it one after the other
+template <int R, int MT, int NW, int PF, bool LX, bool ROPE, bool OWN, int PARTS = NW>
 __global__ __launch_bounds__(64 * NW) void few(FewArgs a) {
   static_assert(!LX || PF % 2 == 0);
+  static_assert(PARTS % NW == 0 && (PARTS == NW || (!LX && PF % 4 == 0)));
   constexpr int XP = LX ? 2 * MT : 0, NX = PF / 2 + 1;  // NX: stages of two k-steps of x, a wave's own: no barrier
-  __shared__ __attribute__((aligned(16))) f32x4v red[NW * R * MT * 64];
+  __shared__ __attribute__((aligned(16))) f32x4v red[PARTS * R * MT * 64];
   __shared__ double stat[OWN ? NW : 1][16 * MT];
   __shared__ __attribute__((aligned(16))) bf16x8 xs[LX ? NW * NX * XP * 64 : 1];
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), fr = lane & 15, fq = lane >> 4;
@@ -161,6 +163,21 @@ __global__ __launch_bounds__(64 * NW) void few(FewArgs a) {
       for (int c = 0; c < MT; ++c) own[c] = add_squares(own[c], x[c]);
     }
   };
+  // a part's sums to LDS, at its last k-step (a part has a multiple of four)
+  const int psteps = nkk / PARTS;
+  int part = w * (PARTS / NW);
+  [[maybe_unused]] int end = psteps;
+  auto hand_over = [&] {
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+      for (int c = 0; c < MT; ++c) {
+        red[((part * R + r) * MT + c) * 64 + lane] = acc[r][c];
+        acc[r][c] = f32x4v{0.f, 0.f, 0.f, 0.f};
+      }
+    ++part;
+    end += psteps;
+  };
   [[maybe_unused]] int from = 0, to = NX - 1;  // stages being read and sent for
   // a round of the ring; the last one sends for nothing: what it would fetch again is waited for, up to 1 us of a launch
   auto round = [&](int s0, auto more) {
@@ -173,6 +190,10 @@ __global__ __launch_bounds__(64 * NW) void few(FewArgs a) {
         if constexpr (MORE) {
           load_w(p, s0 + PF + p);
           load_x(p, s0 + PF + p);
+        }
+        if constexpr (PARTS > NW && p % 4 == 3) {
+          if constexpr (OWN) asm volatile("" : "+v"(own[0]));  // here: else the squares wait behind the branch, with x in 64 registers more
+          if (s0 + p + 1 == end) hand_over();
         }
       } else {
         if constexpr (p % 2 == 0) {
@@ -199,10 +220,7 @@ __global__ __launch_bounds__(64 * NW) void few(FewArgs a) {
   int s0 = 0;
   for (; s0 + PF < nsteps; s0 += PF) round(s0, std::true_type{});
   round(s0, std::false_type{});
-#pragma unroll
-  for (int r = 0; r < R; ++r)
-#pragma unroll
-    for (int c = 0; c < MT; ++c) red[((w * R + r) * MT + c) * 64 + lane] = acc[r][c];
+  if constexpr (PARTS == NW) hand_over();
   if constexpr (OWN) {
 #pragma unroll
     for (int c = 0; c < MT; ++c) {
@@ -220,7 +238,7 @@ __global__ __launch_bounds__(64 * NW) void few(FewArgs a) {
     // lane: row m of x, rows 16 nt + 4 fq + i of W
     f32x4v v = red[t * 64 + lane];
 #pragma unroll
-    for (int j = 1; j < NW; ++j) v += red[(j * R * MT + t) * 64 + lane];
+    for (int j = 1; j < PARTS; ++j) v += red[(j * R * MT + t) * 64 + lane];
     if constexpr (OWN) {
       const int col = 16 * (t % MT) + fr;
       double ss = stat[0][col];
@@ -307,6 +325,10 @@ FewSplit few_split(int M, int N, int K) {
   const int nw = K % 256 == 0 ? 8 : K % 128 == 0 ? 4 : 2, steps = K / 32 / nw;
   return {1, nw, steps % 4 == 0 ? 4 : steps % 3 == 0 ? 3 : steps % 2 == 0 ? 2 : 1, 0};
 }
+// Parts of K that a product of up to 16 rows and K of 512 sums apart, whatever its waves: one chain a wave would be up to four times as long. rms error of
+// sums that cancel, against 64 bits, a chain a wave / so: 4096x4096 2.1e-7 / 1.2e-7, 4096x14336 4.3e-7 / 2.4e-7, 2048x1024 1.0e-7 / 0.65e-7, 6144x4096 2.1e-7 / 1.7e-7. us, the
+// same: 4096x4096 at 1 / 8 / 16 rows 7.0, 7.2, 7.9 / 7.1, 7.3, 8.1; 28672x4096 and 16384x2048 do not differ.
+int few_parts(int N, int K) { return N <= 16 * FEW_CUS && K % 1024 == 0 ? 8 : N <= 32 * FEW_CUS ? 4 : 2; }
 // With a norm or a rotation: only by the splits of the first lines
 bool few_normed(const FewSplit& f, int M, int K) { return f.r && (M <= 16 ? K % 512 == 0 : f.lx != 0); }
 }  // namespace
@@ -329,10 +351,11 @@ int launch_few(const kgs::dec::FewArgs& a, const FewSplit& f, bool rope, bool ow
   auto pick = [&](auto ro, auto ow) {
     constexpr bool RO = decltype(ro)::value, OW = decltype(ow)::value;
     if (f.lx) return f.r == 1 ? run(few<1, 2, 8, 4, true, RO, OW>) : f.nw == 8 ? run(few<2, 2, 8, 4, true, RO, OW>) : run(few<2, 2, 4, 4, true, RO, OW>);
-    if (f.r == 2) return run(few<2, 1, 2, 8, false, RO, OW>);
-    if (f.nw == 1) return run(few<1, 1, 1, 16, false, RO, OW>);
+    const bool four = few_parts(N, K) == 4;
+    if (f.r == 2) return four ? run(few<2, 1, 2, 8, false, RO, OW, 4>) : run(few<2, 1, 2, 8, false, RO, OW>);
+    if (f.nw == 1) return four ? run(few<1, 1, 1, 16, false, RO, OW, 4>) : run(few<1, 1, 1, 16, false, RO, OW, 2>);
     if (f.nw == 8) return run(few<1, 1, 8, 4, false, RO, OW>);
-    return f.pf == 16 ? run(few<1, 1, 2, 16, false, RO, OW>) : run(few<1, 1, 2, 8, false, RO, OW>);
+    return f.pf == 16 ? run(few<1, 1, 2, 16, false, RO, OW, 8>) : run(few<1, 1, 2, 8, false, RO, OW, 4>);
   };
   using T = std::true_type;
   using F = std::false_type;

@@ -56,3 +56,21 @@ def test_rotation_and_cache_as_the_separate_launch(heads, kv, m):
 def test_what_goes_elsewhere():
     for m, n, k in ((16, 4096, 4096), (33, 4096, 4096), (24, 4096, 1536), (24, 4096, 14336), (24, 28672, 4096), (24, 4112, 1024)):
         assert not D.few_wide(m, n, k), (m, n, k)
+
+
+# K's parts are summed apart and added in their order, however few waves take them: eight of up to 4096 rows of W and K of 1024, four of up to 8192 rows, else two. One
+# tile a workgroup by one, two and eight waves, two tiles by two; a part of four k-steps and of several rounds, its end at every fourth step of a round
+@pytest.mark.parametrize("n,k,parts", ((64, 1024, 8), (2048, 1024, 8), (2048, 3072, 8), (4096, 5120, 8), (4096, 8192, 8), (2048, 512, 4), (2048, 2560, 4), (4160, 1024, 4),
+                                       (6144, 1536, 4), (8192, 2048, 4), (8256, 512, 2), (16384, 1536, 2), (28672, 1024, 2)))
+@pytest.mark.parametrize("m", (1, 5, 13, 16))
+def test_parts_are_summed_apart(n, k, parts, m):
+    from kgs.ops import _lib
+
+    x, w = torch.randn(m, k, device="cuda").bfloat16(), (torch.randn(n, k, device="cuda") * k ** -0.5).bfloat16()
+    pw, p = D.PackedWeight(w), torch.empty(parts, m, n, device="cuda")
+    rc = _lib.lib().kgs_skinny_slabs(pw.data.data_ptr(), x.data_ptr(), p.data_ptr(), m, n, k, k, 2 if n >= 4096 and n % 128 == 0 else 1, parts, _lib.stream_handle(x.device))
+    assert rc == 0 and D.few_takes(m, n, k)
+    want = p[0]
+    for part in p[1:]:
+        want = want + part
+    assert torch.equal(D.skinny_few(x, pw), want.bfloat16())  # the same products in the same order: the same bits

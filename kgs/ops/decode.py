@@ -615,7 +615,10 @@ def _split(m: int, n: int, k: int, cus: int) -> tuple[int, int] | None:
       8.9, 10.7, 12.4, 14.0; 4096x8192 17.7, 20.7, 22.8, 23.4 / 16.9, 19.0, 21.6, 23.3; but 4096x14336 24.6, 27.6, 29.2, 31.6 / 25.1, 27.8, 30.8, 33.9, so up to K = 8192; and
       8192x8192 in 4 against 2 slices 30.1, 32.1, 33.9, 35.3 / 29.6, 30.7, 35.2, 39.5, so from 8 slices on;
     * strips of 64 rows in 8 slices against 4: 2048x2048 7.2, 9.1, 10.7, 12.2 / 7.3, 8.3, 9.5, 10.7; 2048x1024 6.3, 8.1, 9.5, 11.0 / 6.1, 7.1, 8.3, 9.5 (at 33 rows 7.9 / 7.7 and
-      6.9 / 6.4, so above 32); but 2048x4096 8.9, 10.6, 12.1, 13.8 / 9.7, 10.9, 12.4, 14.1, so up to K = 2048."""
+      6.9 / 6.4, so above 32); but 2048x4096 8.9, 10.6, 12.1, 13.8 / 9.7, 10.9, 12.4, 14.1, so up to K = 2048; of 16 slices half as well (1024x2048 with a hyper-connection
+      step behind it at 33 / 64 / 96 rows in 16, 8, 4: 7.9, 7.3, 7.9 / 9.3, 8.1, 8.3 / 10.9, 9.4, 9.5).
+
+    The kernel sums the halves of such a slice apart, so that no chain is longer than those of the most slices."""
     r = 2 if n >= 4096 and n % 128 == 0 else 1
     if n <= 0 or k <= 0 or n % (64 * r) or k % 128:
         return None
@@ -624,7 +627,7 @@ def _split(m: int, n: int, k: int, cus: int) -> tuple[int, int] | None:
         ns *= 2
     if r == 2 and ns >= 8 and k <= 8192:
         return 1, ns // 2
-    return r, min(ns, 4) if m > 32 and k <= 2048 else ns
+    return r, ns // 2 if ns >= 8 and m > 32 and k <= 2048 else ns
 
 
 @lru_cache(maxsize=4096)

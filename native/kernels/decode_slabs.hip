@@ -54,7 +54,8 @@ __device__ __forceinline__ void wait_loads() {
   asm volatile("" ::: "memory");
 }
 
-template <int MT, int R, int OUT, int NW>
+// HALVES: of one slice, summed apart (halves)
+template <int MT, int R, int OUT, int NW, bool HALVES = false>
 __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void slabs(SlabArgs a) {
   constexpr int PF = 4, NB = 3, KC = MT == 1 ? 4 : 2, XL = KC * MT / 4;  // XL: pieces of x of a wave and chunk
   static_assert(PF % KC == 0 && PF >= (NB - 2) * KC);
@@ -81,11 +82,13 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void slabs(SlabArgs a) {
     for (int r = 0; r < R; ++r)
       wf[p][r] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(rw, wo, (r * nkk + k0 + s) * 1024, 2));
   };
-  f32x4v acc[R][MT];
+  typedef f32x4v Sums[R][MT];
+  Sums acc;
+  [[maybe_unused]] Sums first;
 #pragma unroll
   for (int r = 0; r < R; ++r)
 #pragma unroll
-    for (int c = 0; c < MT; ++c) acc[r][c] = f32x4v{0.f, 0.f, 0.f, 0.f};
+    for (int c = 0; c < MT; ++c) acc[r][c] = first[r][c] = f32x4v{0.f, 0.f, 0.f, 0.f};
   auto product = [&](auto sends) {
     constexpr int XS = decltype(sends)::value ? XL : 0;  // a wave's DMAs a chunk
     int next = 0, to = 0;  // chunk to send for and its stage; past the end the last one again
@@ -114,7 +117,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void slabs(SlabArgs a) {
 #pragma unroll
     for (int c = 0; c < MT; ++c) b[0][c] = xs[0][c * 128 + ro[0]];
     // a round of the weights' ring; the last one sends for nothing: what it would fetch again is waited for, up to 1 us of a launch
-    auto round = [&](int s0, auto more) {
+    auto round = [&](int s0, auto more, Sums& acc) {
       constexpr bool MORE = decltype(more)::value;
 #pragma unroll
       for (int p = 0; p < PF; ++p) {
@@ -145,8 +148,10 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void slabs(SlabArgs a) {
       }
     };
     int s0 = 0;
-    for (; s0 + PF < nsteps; s0 += PF) round(s0, std::true_type{});
-    round(s0, std::false_type{});
+    if constexpr (HALVES)
+      for (; 2 * s0 < nsteps; s0 += PF) round(s0, std::true_type{}, first);
+    for (; s0 + PF < nsteps; s0 += PF) round(s0, std::true_type{}, acc);
+    round(s0, std::false_type{}, acc);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the tail's chunks land before LDS is released
   };
   if (NW == 4 || w < 4) product(std::true_type{});
@@ -160,7 +165,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void slabs(SlabArgs a) {
     }
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-      const f32x4v v = OUT == OUT_SLABS ? acc[r][c] : acc[r][c] * scale;
+      const f32x4v v = HALVES ? first[r][c] + acc[r][c] : OUT == OUT_SLABS ? acc[r][c] : acc[r][c] * scale;
       const int nt = nt0 + r;
       if constexpr (OUT == OUT_SLABS) {
         if (m < rows) *(f32x4v*)((float*)a.y + ((long)sl * M + m) * N + 16 * nt + 4 * fq) = v;
@@ -199,6 +204,18 @@ inline int fine_waves(int T, int r, int ns) {
   return 0;
 }
 
+constexpr int SLAB_CUS = 256;  // kgs/ops/decode.py CUS
+
+// Whether a slice's halves are summed apart: where more slices would leave one workgroup a CU and the caller takes fewer (kgs/ops/decode.py _split). A chain of
+// twice the length costs the sums precision; rms error against 64 bits of unit sums, most slices / fewer, in one chain / so: 4096x4096 1.37e-7 / 1.89e-7 /
+// 1.35e-7, 4096x8192 1.93e-7 / 2.74e-7 / 1.91e-7, 2048x2048 1.03e-7 / 1.32e-7 / 0.99e-7. It takes no time (4096x4096 at 64 / 128 rows 9.6, 11.7 us both).
+inline bool halves(int N, int K, int r, int ns) {
+  const int tiles = N / (N >= 4096 && N % 128 == 0 ? 128 : 64);
+  int most = 1;
+  while (most < 16 && 2 * most * tiles <= SLAB_CUS && K % (256 * most) == 0) most *= 2;
+  return r == 1 && ns < most && most % ns == 0;
+}
+
 template <int OUT, int MT>
 int launch_mt(const kgs::dec::SlabArgs& a, int r, hipStream_t s) {
   using namespace kgs::dec;
@@ -207,12 +224,14 @@ int launch_mt(const kgs::dec::SlabArgs& a, int r, hipStream_t s) {
     hipLaunchKernelGGL(kernel, dim3((a.N + strip - 1) / strip * a.ns), dim3(64 * waves), 0, s, a);
     return (int)hipGetLastError();
   };
-  switch (nw) {
-    case 5: return run(slabs<MT, 1, OUT, 5>, 80, 5);
-    case 6: return run(slabs<MT, 1, OUT, 6>, 96, 6);
-    case 7: return run(slabs<MT, 1, OUT, 7>, 112, 7);
-  }
-  return r == 1 ? run(slabs<MT, 1, OUT, 4>, 64, 4) : run(slabs<MT, 2, OUT, 4>, 128, 4);
+  auto one = [&](auto apart) {
+    constexpr bool H = decltype(apart)::value;
+    return nw == 5 ? run(slabs<MT, 1, OUT, 5, H>, 80, 5) : nw == 6 ? run(slabs<MT, 1, OUT, 6, H>, 96, 6) : nw == 7 ? run(slabs<MT, 1, OUT, 7, H>, 112, 7)
+                                                                                                         : run(slabs<MT, 1, OUT, 4, H>, 64, 4);
+  };
+  if constexpr (OUT == OUT_SLABS)
+    if (halves(a.N, a.K, r, a.ns)) return one(std::true_type{});
+  return r == 1 || nw ? one(std::false_type{}) : run(slabs<MT, 2, OUT, 4>, 128, 4);
 }
 template <int OUT>
 int launch_slabs(const kgs::dec::SlabArgs& a, int r, hipStream_t s) {

@@ -317,3 +317,36 @@ def test_small_steps_repeat_and_agree_with_the_unfused_layers(hidden, heads, row
     m.fused_max_batch = 0
     for a, b in zip(got, both()):
         assert float((a - b).norm() / b.norm()) < 2e-2  # sums in another order, rounded to bf16 through two layers
+
+
+# slices of twice the K that one workgroup a CU would have
+@pytest.mark.parametrize("m,n,k", ((1, 4096, 2048), (16, 4096, 4096), (48, 4096, 8192), (96, 4096, 2048), (128, 4096, 4096), (33, 2048, 2048), (97, 2048, 1024)))
+def test_longer_slices_sum_their_halves_apart(m, n, k):
+    from kgs.ops import _lib
+
+    x, w = _operands(m, n, k, 5)
+    rule, slabs = (D.slab_split, D.skinny_slabs) if m <= 96 else (D.wide_split, D.wide_slabs)
+    assert rule(m, n, k) == (1, 4)
+    pw, p = D.PackedWeight(w), torch.empty(8, m, n, device="cuda")
+    rc = _lib.lib().kgs_wide_slabs(pw.data.data_ptr(), x.data_ptr(), p.data_ptr(), m, n, k, x.stride(0), 2 if n >= 4096 else 1, 8, _lib.stream_handle(x.device))
+    assert rc == 0 and torch.equal(slabs(x, pw), p[0::2] + p[1::2])  # as many slices' sums, added in pairs
+
+
+# and of four times: (2048 columns of x, 1024 rows of W) 4 for 16
+@pytest.mark.parametrize("m,n,k,most", ((64, 4096, 4096, 8), (64, 2048, 2048, 8), (64, 1024, 2048, 16)))
+def test_fewer_slices_lose_no_precision(m, n, k, most):
+    """The sums of four slices against 64 bits are no further off than those of the most: the same chains or half as many, then fewer additions."""
+    from kgs.ops import _lib
+
+    x, w = _operands(m, n, k, 6)
+    pw, p = D.PackedWeight(w), torch.empty(most, m, n, device="cuda")
+    assert _lib.lib().kgs_skinny_slabs(pw.data.data_ptr(), x.data_ptr(), p.data_ptr(), m, n, k, x.stride(0), 2 if n >= 4096 else 1, most, _lib.stream_handle(x.device)) == 0
+    ref = x.double() @ w.double().T
+
+    def off(parts):
+        total = parts[0]
+        for part in parts[1:]:
+            total = total + part
+        return float((total.double() - ref).pow(2).mean())
+
+    assert off(D.skinny_slabs(x, pw)) <= off(p)

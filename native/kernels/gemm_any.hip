@@ -20,7 +20,8 @@
 // any_reduce sums in a fixed order before the epilogue.
 #include <utility>
 
-#include "gemm_w4.h"
+#include "gemm_w4p.h"
+#include "tile_queue.h"
 
 namespace kgs {
 int cu_count();  // gemm_bf16.hip
@@ -58,7 +59,6 @@ __device__ __forceinline__ Args again() {
   __builtin_memcpy(&g, p, sizeof g);
   return g;
 }
-__device__ __forceinline__ int ceil_div_dev(int a, int b) { return (a + b - 1) / b; }
 
 template <int BM, int BN>
 constexpr int waves_per_simd() { return BM == 128 && BN == 128 ? 2 : 1; }
@@ -159,19 +159,35 @@ __device__ __forceinline__ void store_row(const Args& a, int r, int col, const f
 // workgroup a tile / so: 3001 x 7000 x 200 23.4 / 21.3, 5000 x 5000 x 1000 56.1 / 54.1, 6000 x 9000 x 1000 120.8 / 114.6, 8192 x 14336 x 1024 227 / 213. Bound by
 // the matrix cores' power: what the gaps no longer cost comes off the clock. Tiles and resources are worked out from the arguments read anew at each turn:
 // held through the K loop and the stores they spilled 26 to 53 scalar registers, and up to 8 in kernels of one tile that shared the loop.
+// A workgroup's first tile is its own, the others are tickets of its XCD label in the launch's row q (tile_queue.h), so that a CU held by another
+// stream's kernel leaves its share to the others. us with 16 CUs held for a millisecond, a fixed list / tickets / a workgroup a tile: 8192 x 14336 x 1024 336 /
+// 212 / 241, 6000 x 9000 x 1000 156 / 135 / 119 (a late workgroup still has its first tile); else as the list (2049 x 8200 x 64 12.6 / 13.1 / 13.6, 6000 x 9000 x 1000 112 / 111 /
+// 118). A ticket is drawn one tile ahead and handed over between the last two K-steps, whose waits and barriers are all that it needs.
 template <int EPI, int BM, int BN, bool SPLIT, bool DUAL, int SW, int NS, bool TURNS = false>
-__device__ __forceinline__ void tile_product(const Args& a) {
+__device__ __forceinline__ void tile_product(const Args& a, [[maybe_unused]] int* q = nullptr) {
   constexpr int X = SW * 1000000, TN = SW ? BN / 2 : BN;  // TN: output columns of a tile
   using S = w4::Shape<BM, BN>;
   using Kn = w4::Knobs<BM, BN>;
   constexpr int MA = S::MA, NB = S::NB, ND = w4::dma_per_stage<BM, BN>();
   static_assert(!TURNS || (NS == 2 && !SPLIT));
-  __shared__ __attribute__((aligned(1024))) char smem[NS * S::STAGE];
+  // TURNS: and a ticket. One object: with a second one each fragment read waits for every DMA
+  __shared__ __attribute__((aligned(1024))) char smem[NS * S::STAGE + (TURNS ? 16 : 0)];
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // TURNS: the next ticket, through an address that is not known to be uniform (for a uniform one the compiler waits at once, for everything in flight)
+  const int label = (int)blockIdx.x & 7;
+  [[maybe_unused]] int zero = 0, ticket = 0;
+  [[maybe_unused]] int* const slot = (int*)(smem + NS * S::STAGE);
+  if constexpr (TURNS) asm volatile("v_mov_b32 %0, 0" : "=v"(zero));
+  auto draw = [&] {
+    if (threadIdx.x == 0) ticket = atomicAdd(q + label * TQ_INTS + zero, 1);
+  };
+  if constexpr (TURNS) draw();
   int slice = 0, m0, n0;
+  auto rows = [](const Args& g) { return (g.M + BM - 1) / BM; };  // of tiles, and their columns
+  auto columns = [](const Args& g) { return ((SW ? g.N / 2 : g.N) + TN - 1) / TN; };
   auto locate = [&](const Args& g, int id, int& m, int& n) {
-    const int ntm = (g.M + BM - 1) / BM, ntn = ((SW ? g.N / 2 : g.N) + TN - 1) / TN;
+    const int ntm = rows(g), ntn = columns(g);
     int tm, tn;
     if (g.tall) w4::tile_of<40000000, SPLIT>(id, (int)gridDim.x, ntm, ntn, slice, tm, tn);
     else w4::tile_of<0, SPLIT>(id, (int)gridDim.x, ntm, ntn, slice, tm, tn);
@@ -238,13 +254,15 @@ __device__ __forceinline__ void tile_product(const Args& a) {
   }
   __builtin_amdgcn_s_waitcnt(0xc07f);
 
-  // K-steps of K-tiles t, t + 1, which send for K-tiles s and s + 1
-  auto pair = [&](int s) {
+  // K-steps of K-tiles t, t + 1, which send for K-tiles s and s + 1; between them `middle`
+  auto pair = [&](int s, auto&& middle) {
     aim(s);
     w4::kstep<BM, BN, 0, Kn::B1, Kn::R, Kn::P, Kn::ORD, X>(c, f0, f1, s - 2);
+    middle();
     aim(s + 1);
     w4::kstep<BM, BN, 1, Kn::B1, Kn::R, Kn::P, Kn::ORD, X>(c, f0, f1, s - 1);
   };
+  auto steady = [&](int s) { pair(s, [] {}); };
   auto store = [&](const Args& g, int m, int n) {
     const int mw = m + c.wr * (BM / 2) + fr, nw = n + c.wc * (TN / 2);
     const int lc = (fq & 1) * 16 + (fq >> 1) * 8;  // this lane's 8 of a fragment pair's 32 columns
@@ -317,33 +335,58 @@ __device__ __forceinline__ void tile_product(const Args& a) {
         });
       }
     } else {
-      for (int t = 0; t < c.nt; t += 2) pair(t + 2);
+      for (int t = 0; t < c.nt; t += 2) steady(t + 2);
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the tail's DMAs (zeros) land before LDS is released
     settle();
     store(a, m0, n0);
   } else {
-    for (int id = (int)blockIdx.x;;) {
-      for (int t = 0; t + 2 < c.nt; t += 2) pair(t + 2);
-      const int next = id + (int)gridDim.x;
+    // tickets of a label are numbered behind its workgroups' first tiles; its tile t is label + 8 t
+    const int first = ((int)gridDim.x - label + 7) >> 3;
+    auto limit = [&](const Args& g) { return (rows(g) * columns(g) - label + 7) >> 3; };
+    auto hand_over = [&] {
+      if (threadIdx.x == 0) *slot = ticket;
+    };
+    // unsigned: a ticket that no launch can have issued ends the workgroup, no address comes of it
+    auto taken = [&](int lim) {
+      const int raw = __builtin_amdgcn_readfirstlane(*slot);
+      w4p::mark_bad_ticket(q + label * TQ_INTS, raw, lim);
+      if (raw == lim - 1 && threadIdx.x == 0) atomicExch(q + label * TQ_INTS, 0);  // the label's last draw: each tile of it and each end of a workgroup is one
+      return first + raw;
+    };
+    bool begun = false;
+    for (int next = 0;;) {
+      for (int t = 0; t + 2 < c.nt; t += 2) steady(t + 2);
       // the arguments again, instead of registers that hold them through the K-steps
       const Args g = again();
-      const bool more = next < ceil_div_dev(g.M, BM) * ceil_div_dev(SW ? g.N / 2 : g.N, TN);
+      const int lim = limit(g);
+      if (!begun) {
+        hand_over();
+        __builtin_amdgcn_s_waitcnt(0xc07f);
+        w4::bar();
+        next = taken(lim);
+        if ((unsigned)next < (unsigned)lim) draw();
+        begun = true;
+      }
+      const bool more = (unsigned)next < (unsigned)lim;
       int m1 = 0, n1 = 0;
       if (more) {
-        locate(g, next, m1, n1);
+        locate(g, label + 8 * next, m1, n1);
         bind(g, m1, n1);
       }
-      pair(more ? 0 : c.nt);
+      pair(more ? 0 : c.nt, hand_over);
       if (!more) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // as above
       settle();
       const Args h = again();
       store(h, m0, n0);
       if (!more) break;
-      id = next;
       m0 = m1;
       n0 = n1;
-      bind(again(), m0, n0);  // again: not held through the stores
+      const Args k = again();  // again: not held through the stores
+      bind(k, m0, n0);
+      const int most = limit(k);
+      next = taken(most);
+      if ((unsigned)next < (unsigned)most) draw();
       w4::static_for<0, MA * NB>([](auto q) { accr::zero<decltype(q)::value>(); });
       asm volatile("s_nop 7" ::: "memory");
       __builtin_amdgcn_s_waitcnt(0xc07f);
@@ -368,8 +411,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
   tile_product<EPI, BM, BN, SPLIT, DUAL, SW, lds_stages<BM, BN, true>()>(a);
 }
 template <int EPI, int BM, int BN, bool DUAL, int SW = 0>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void gemm_nt_turn(Args a) {
-  tile_product<EPI, BM, BN, false, DUAL, SW, 2, true>(a);
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void gemm_nt_turn(Args a, int* q) {
+  tile_product<EPI, BM, BN, false, DUAL, SW, 2, true>(a, q);
 }
 
 // The same product on 64x64 tiles, for grids that leave CUs idle at 128x128. What bounds such a
@@ -827,10 +870,11 @@ template <int EPI, int BM, int BN, bool DUAL, int SW = 0>
 void launch_mid(const Args& a, hipStream_t s) {
   const long tiles = (long)ceil_div(a.M, BM) * (SW ? ceil_div(a.N / 2, BN / 2) : ceil_div(a.N, BN));
   if constexpr (BN != 128) {
-    if (take_turns(a, tiles)) {
-      hipLaunchKernelGGL((gemm_nt_turn<EPI, BM, BN, DUAL, SW>), dim3((unsigned)cu_count()), dim3(256), 0, s, a);
-      return;
-    }
+    if (take_turns(a, tiles))
+      if (int* q = tile_queue_row(s)) {  // null in a capture: a workgroup a tile
+        hipLaunchKernelGGL((gemm_nt_turn<EPI, BM, BN, DUAL, SW>), dim3((unsigned)cu_count()), dim3(256), 0, s, a, q);
+        return;
+      }
   } else if (a.K > 2 * BK) {
     hipLaunchKernelGGL((gemm_nt_deep<EPI, BM, BN, DUAL, SW>), dim3((unsigned)tiles), dim3(256), 0, s, a);
     return;

@@ -272,6 +272,12 @@ KGS_EXPORT int kgs_tile_queue_slot(hipStream_t s, void** out) {
   return *out ? 0 : KGS_ERR_ARG;
 }
 
+// The same of the row of slots of tiles that take turns on `s`.
+KGS_EXPORT int kgs_tile_queue_row(hipStream_t s, void** out) {
+  *out = kgs::tile_queue_row(s);
+  return *out ? 0 : KGS_ERR_ARG;
+}
+
 // The quiescent-pool invariant (tile_queue.h tile_queue_check): out = {dirty
 // slots, dirty words, first dirty value, its word index, the first dirty slot's
 // address, its 16 words, slots with the impossible-ticket error word set}. No

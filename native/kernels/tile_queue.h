@@ -28,6 +28,12 @@
 //  * no slot (reserve empty during a capture, allocation failure): nullptr and
 //    the caller runs the one-shot grid, which needs no counters.
 //
+// Tiles that take turns (gemm_any.hip) are shorter than a persistent launch's, and tickets in one line cost them: 256 workgroups' atomics on it come one
+// after the other, 3 us at the start of a launch and as much for the exit counter at its end. Their launches have a row of eight slots, one
+// a label, of their (device, stream) -- eager ones only, a capture runs a workgroup a tile -- and no exit counter: a label's draws in a launch are as many
+// as its tiles, so the last of them clears it. us, one slot with an exit counter / a row: 2049 x 8200 x 64 17.0 / 13.1, 5000 x 5000 x 200 25.1 / 22.3, 3001 x 7000 x 200
+// 22.4 / 20.8; rows of 128-byte lines are no faster.
+//
 // Pool memory is allocated and zeroed outside any capture and outside the pool
 // lock, and never freed: 64 B per stream or captured launch. A new chunk is
 // zeroed on the pool's own non-blocking stream and only THAT stream is
@@ -53,6 +59,7 @@ constexpr int TQ_ERR = 15;      // padding word a kernel sets when it read an im
 constexpr int TQ_CHUNK = 256;   // slots per pool allocation (16 KiB)
 constexpr int TQ_RESERVE = 64;  // free slots kept for captures
 constexpr int TQ_DEVICES = 64;
+constexpr int TQ_ROW = 8;       // slots of a row
 
 struct TileQueueStats {
   long slots;          // allocated
@@ -95,6 +102,8 @@ struct OwnerHash {
 struct DevicePool {
   std::vector<int*> chunks;  // every allocation, for tile_queue_check
   std::vector<int*> free_slots;
+  std::vector<int*> row_chunks, free_rows;  // the same of rows
+  std::unordered_map<OwnerKey, int*, OwnerHash> row_owners;
   std::unordered_map<OwnerKey, int*, OwnerHash> owners;
   hipStream_t zero_stream = nullptr;  // private, non-blocking; touched only by the growing thread
   bool growing = false;               // one growth at a time per device
@@ -151,7 +160,7 @@ inline int* new_chunk(DevicePool& P, int dev) {
 // After a failure (memory nearly full, no stream) the next TQ_GROW_BACKOFF
 // eager calls do not retry: hipMalloc and stream creation stay off the hot path.
 constexpr int TQ_GROW_BACKOFF = 256;
-inline bool grow(DevicePool& P, int dev, std::unique_lock<std::mutex>& lock) {
+inline bool grow(DevicePool& P, int dev, std::unique_lock<std::mutex>& lock, bool rows = false) {
   if (P.growing) return false;
   if (P.grow_backoff > 0) {
     --P.grow_backoff;
@@ -167,13 +176,44 @@ inline bool grow(DevicePool& P, int dev, std::unique_lock<std::mutex>& lock) {
     ++P.grow_failures;
     return false;
   }
+  if (rows) {
+    for (int i = TQ_CHUNK / TQ_ROW - 1; i >= 0; --i) P.free_rows.push_back(p + i * TQ_ROW * TQ_INTS);
+    P.row_chunks.push_back(p);
+    return true;
+  }
   for (int i = TQ_CHUNK - 1; i >= 0; --i) P.free_slots.push_back(p + i * TQ_INTS);
   P.chunks.push_back(p);
   P.slots += TQ_CHUNK;
   return true;
 }
 
+inline OwnerKey owner_of(hipStream_t stream) {
+  return {stream, stream == hipStreamPerThread ? std::this_thread::get_id() : std::thread::id()};
+}
+
 }  // namespace tq_detail
+
+// The row of an eager launch on `stream`: TQ_ROW slots, all zero when no launch of the stream's runs. nullptr: captured, or none to be had
+inline int* tile_queue_row(hipStream_t stream) {
+  using namespace tq_detail;
+  int dev = 0;
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(stream, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) return nullptr;
+  if (hipStreamGetDevice(stream, &dev) != hipSuccess || dev < 0 || dev >= TQ_DEVICES) return nullptr;
+  std::unique_lock<std::mutex> lock(mu());
+  DevicePool& P = pools()[dev];
+  const OwnerKey key = owner_of(stream);
+  const auto it = P.row_owners.find(key);
+  if (it != P.row_owners.end()) return it->second;
+  if ((P.free_rows.empty() && !grow(P, dev, lock, true)) || P.free_rows.empty()) {
+    ++P.fallbacks;
+    return nullptr;
+  }
+  int* r = P.free_rows.back();
+  P.free_rows.pop_back();
+  P.row_owners.emplace(key, r);
+  return r;
+}
 
 inline int* tile_queue(hipStream_t stream) {
   using namespace tq_detail;
@@ -200,8 +240,7 @@ inline int* tile_queue(hipStream_t stream) {
     ++P.capture_slots;
     return s;
   }
-  const bool per_thread = stream == hipStreamPerThread;
-  const OwnerKey key{stream, per_thread ? std::this_thread::get_id() : std::thread::id()};
+  const OwnerKey key = owner_of(stream);
   auto it = P.owners.find(key);
   int* s = it == P.owners.end() ? nullptr : it->second;
   // keep the capture reserve filled: captures cannot allocate, eager calls can
@@ -240,7 +279,9 @@ inline int tile_queue_check(int dev, long* out) {
   const DevicePool& P = pools()[dev];
   std::vector<int> h(TQ_INTS * TQ_CHUNK);
   long base = 0;
-  for (int* c : P.chunks) {
+  std::vector<int*> all = P.chunks;
+  all.insert(all.end(), P.row_chunks.begin(), P.row_chunks.end());
+  for (int* c : all) {
     const hipError_t e = hipMemcpy(h.data(), c, sizeof(int) * h.size(), hipMemcpyDeviceToHost);
     if (e != hipSuccess) return (int)e;
     for (int sl = 0; sl < TQ_CHUNK; ++sl) {

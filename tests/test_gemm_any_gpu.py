@@ -106,6 +106,73 @@ def test_tiles_that_take_turns_keep_the_bits(bm, bn, M, N, K):
             assert torch.equal(got, want)
 
 
+def test_tiles_that_take_turns_draw_tickets():
+    """A workgroup's tiles behind its first one are tickets of the stream's row of slots: with all of them drawn beforehand each computes that one alone. A
+    launch leaves the row cleared, and impossible tickets end its workgroups and are reported."""
+    import ctypes
+
+    from kgs.ops import _lib
+    from kgs.utils.graph_audit import hip_runtime
+
+    (M, N, K), s, row = (5120, 8192, 192), torch.cuda.Stream(), ctypes.c_void_p()
+    a, b, got, want = rnd(M, K), rnd(N, K), torch.zeros(M, N, device=DEV, dtype=torch.bfloat16), torch.empty(M, N, device=DEV, dtype=torch.bfloat16)
+    run_any(a, b, want, 128, 128, 1)
+    _lib.check(_lib.lib().kgs_tile_queue_row(s.cuda_stream, ctypes.byref(row)), "kgs_tile_queue_row")
+    torch.cuda.synchronize()
+    hip = hip_runtime()
+    hip.hipMemcpy.argtypes, hip.hipMemcpy.restype = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_int], ctypes.c_int
+    tiles, cus = M // 256 * (N // 256), torch.cuda.get_device_properties(DEV).multi_processor_count
+
+    def go(ticket):
+        words = (ctypes.c_int * 128)(*([ticket] + [0] * 15) * 8)
+        assert hip.hipMemcpy(row, words, 512, 1) == 0  # host to device
+        got.zero_()
+        torch.cuda.synchronize()
+        with torch.cuda.stream(s):
+            run_any(a, b, got, 256, 256, 1)
+        torch.cuda.synchronize()
+        same = (got.view(M // 256, 256, N // 256, 256) == want.view(M // 256, 256, N // 256, 256)).all(dim=3).all(dim=1)
+        return int(same.sum()), _lib.tile_queue_check()
+
+    assert go(tiles // 8)[0] == cus < tiles
+    done, check = go(0x40000000)
+    assert done == cus and check["error_slots"] == 8
+    done, check = go(0)
+    assert done == tiles and check["dirty_slots"] == check["error_slots"] == 0
+
+
+# one K-step pair a tile, where a tile's ticket is drawn and handed over within it, and several
+@pytest.mark.parametrize("K", [64, 1000])
+def test_tiles_that_take_turns_beside_held_cus_and_in_a_graph(K):
+    from kgs.ops import _lib
+    from kgs.ops.elementwise import cu_hold
+
+    M, N = 4100, 9000
+    a, b, want = rnd(M, K), rnd(N, K), torch.empty(M, N, device=DEV, dtype=torch.bfloat16)
+    run_any(a, b, want, 128, 128, 1)
+    side, out = torch.cuda.Stream(), [torch.zeros_like(want) for _ in range(2)]
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        cu_hold(48, 200.0, lds_kb=64)
+        run_any(a, b, out[1], 224, 256, 1)  # a slot of its own
+    for _ in range(2):
+        out[0].zero_()
+        run_any(a, b, out[0], 224, 256, 1)
+    torch.cuda.synchronize()
+    assert all(torch.equal(o, want) for o in out)
+    before, g = _lib.tile_queue_stats()["capture_slots"], torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        run_any(a, b, out[0], 224, 256, 1)
+    assert _lib.tile_queue_stats()["capture_slots"] == before  # a workgroup a tile
+    for _ in range(3):
+        out[0].zero_()
+        g.replay()
+        run_any(a, b, out[1].zero_(), 224, 256, 1)
+        torch.cuda.synchronize()
+        assert all(torch.equal(o, want) for o in out)
+    assert _lib.tile_queue_check()["dirty_slots"] == 0
+
+
 def tile(M, N, K, gated=False):
     from kgs.ops import _lib
 

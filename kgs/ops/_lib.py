@@ -49,6 +49,7 @@ _SIGS = {
     "kgs_gemm_bf16_turn_b": ([_c_int] * 3, _c_int),
     "kgs_gemm_bf16_nt_finer": ([_c_int] * 5, _c_int),
     "kgs_gemm_bf16_nt_tile": ([_c_int] * 4, _c_int),
+    "kgs_gemm_bf16_nt_tile_rows": ([_c_int] * 6, _c_int),
     "kgs_gemm_bf16_tr_slices": ([_c_int] * 5, _c_int),
     "kgs_act_grad_parts": ([_c_int] * 2, _c_int),
     "kgs_act_grad": ([_c_void_p] * 6 + [_c_int] * 4 + [_c_void_p], _c_int),

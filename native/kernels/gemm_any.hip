@@ -861,16 +861,18 @@ struct Plan {
 
 inline int ceil_div(long a, long b) { return (int)((a + b - 1) / b); }
 
-// Whether the tiles of an unsliced launch take turns (tile_product): two-stage ones of more than a round, but not for long sums over rows off the
+// Whether the two-stage tiles of an unsliced launch take turns (tile_product) when they are more than a round: not for long sums over rows off the
 // 128-byte lines (us, a workgroup a tile / taking turns: 4000 x 6000 x 2000 108 / 116, of 2048 91.5 / 91.6; 6000 x 9000 x 3000 295 / 304.5, 6144 x 9216 x 3072 278 / 272)
-inline bool take_turns(const Args& a, long tiles) { return tiles > cu_count() && ((a.lda % 64 == 0 && a.ldb % 64 == 0) || a.K <= 1024); }
+inline bool turns_pay(const void* A, const void* B, int K, int lda, int ldb) {
+  return (lda % 64 == 0 && ldb % 64 == 0 && ((uintptr_t)A | (uintptr_t)B) % 128 == 0) || K <= 1024;
+}
 
 // An unsliced launch of tiles with a CU each; two stages hold all of a K up to 128
 template <int EPI, int BM, int BN, bool DUAL, int SW = 0>
 void launch_mid(const Args& a, hipStream_t s) {
   const long tiles = (long)ceil_div(a.M, BM) * (SW ? ceil_div(a.N / 2, BN / 2) : ceil_div(a.N, BN));
   if constexpr (BN != 128) {
-    if (take_turns(a, tiles))
+    if (tiles > cu_count() && turns_pay(a.A, a.B, a.K, a.lda, a.ldb))
       if (int* q = tile_queue_row(s)) {  // null in a capture: a workgroup a tile
         hipLaunchKernelGGL((gemm_nt_turn<EPI, BM, BN, DUAL, SW>), dim3((unsigned)cu_count()), dim3(256), 0, s, a, q);
         return;
@@ -935,16 +937,20 @@ inline Plan plan(long M, long N, long K, bool split, int cus) {
 // tile that these estimates choose takes 0.8 % more than the best one): start, what each round of workgroups
 // after the first adds, and a K-step alone on a CU and what the chip's filling adds to it. 128x128 tiles: of two
 // workgroups on a CU, and of the single ones that remain. Tiles of 128 columns (of 128x128 ones the single) scaled to their K-steps of one barrier, by 48
-// sizes: 0.33 + 0.13 full where 0.37 + 0.16, of 192 rows 0.40 + 0.25 / 0.42 + 0.29, 224 0.44 + 0.29 / 0.45 + 0.32, 256 0.46 + 0.35 / 0.49 + 0.36. Further rounds of two-stage
-// tiles cost 1.5 to 3 us less since they take turns.
+// sizes: 0.33 + 0.13 full where 0.37 + 0.16, of 192 rows 0.40 + 0.25 / 0.42 + 0.29, 224 0.44 + 0.29 / 0.45 + 0.32, 256 0.46 + 0.35 / 0.49 + 0.36. turn: what a
+// further round costs tiles that take turns (turns_pay), 1.5 to 2 us less.
 struct Tile {
   int bm, bn;
-  double start, again, step, fill;
+  double start, again, turn, step, fill;
 };
-constexpr Tile TILES[] = {{256, 256, 7.12, 5.3, 0.88, 0.50}, {256, 128, 4.61, 4.53, 0.53, 0.28}, {128, 128, 3.5, 3.2, 0.97, 0},
-                          {192, 128, 4.15, 2.97, 0.42, 0.22}, {224, 128, 4.27, 3.53, 0.48, 0.25}, {192, 192, 5.02, 3.3, 0.56, 0.29},
-                          {224, 192, 5.40, 3.6, 0.61, 0.35}, {256, 192, 5.90, 4.3, 0.67, 0.38}, {224, 256, 6.49, 4.9, 0.78, 0.43}};
-inline double tile_cost(const Tile& t, long M, long N, long K, int cus) {
+constexpr Tile TILES[] = {{256, 256, 7.12, 7.31, 5.3, 0.88, 0.50}, {256, 128, 4.61, 4.53, 4.53, 0.53, 0.28}, {128, 128, 3.5, 3.2, 3.2, 0.97, 0},
+                          {192, 128, 4.15, 2.97, 2.97, 0.42, 0.22}, {224, 128, 4.27, 3.53, 3.53, 0.48, 0.25}, {192, 192, 5.02, 4.65, 3.3, 0.56, 0.29},
+                          {224, 192, 5.40, 5.14, 3.6, 0.61, 0.35}, {256, 192, 5.90, 5.94, 4.3, 0.67, 0.38}, {224, 256, 6.49, 6.69, 4.9, 0.78, 0.43}};
+// The persistent and the eight-wave kernels of 256x256 tiles, as finer and turn_b see them. With the 5.3 us of tiles that take turns for a further round, 36
+// products with a K-major B that read it faster on average (up to 29 %: 3584 x 11264 x 384 48.0 us, transposed first 61.9) were transposed first, and 24
+// of ragged rows kept to persistent tiles that lose 2 % to finer ones on average (0.92 to 1.03 of their time).
+constexpr Tile LARGE = {256, 256, 7.12, 7.31, 7.31, 0.88, 0.50};
+inline double tile_cost(const Tile& t, long M, long N, long K, int cus, bool turns) {
   const long wg = (long)ceil_div(M, t.bm) * ceil_div(N, t.bn);
   const int steps = 2 * ceil_div(K, 128);
   if (t.bm == 128) {
@@ -953,11 +959,11 @@ inline double tile_cost(const Tile& t, long M, long N, long K, int cus) {
     return t.start + steps * (pairs * t.step + one) + (two ? t.again * (two - (rest == 0)) : 0);
   }
   const int full = (int)(wg / cus), rest = (int)(wg - (long)full * cus), rounds = full + (rest > 0);
-  return t.start + (rounds - 1) * t.again + steps * (rounds * t.step + (full + (double)rest / cus) * t.fill);
+  return t.start + (rounds - 1) * (turns ? t.turn : t.again) + steps * (rounds * t.step + (full + (double)rest / cus) * t.fill);
 }
-inline double tile_cost(int bm, int bn, long M, long N, long K, int cus) {
+inline double tile_cost(int bm, int bn, long M, long N, long K, int cus, bool turns) {
   for (const Tile& t : TILES)
-    if (t.bm == bm && t.bn == bn) return tile_cost(t, M, N, K, cus);
+    if (t.bm == bm && t.bn == bn) return tile_cost(t, M, N, K, cus, turns);
   return 1e30;
 }
 
@@ -967,12 +973,12 @@ inline double tile_cost(int bm, int bn, long M, long N, long K, int cus) {
 // slower per product. The bits are the same. us, plan's tile / this one: 1762 x 6144 x 4096 81 / 66, 2830 x 6144 x 5504 199 / 145,
 // 1762 x 28672 x 4096 349 / 309, 590 x 11776 x 3472 75 / 57, 1382 x 6144 x 1152 28 / 21. sw: a gated product's tiles, whose
 // waves hold gate and up columns in turn, are 128 or 256 wide.
-inline Plan refine(Plan p, long M, long N, long K, int cus, bool sw = false) {
+inline Plan refine(Plan p, long M, long N, long K, int cus, bool turns, bool sw = false) {
   if (p.ns > 1 || p.bm == 64) return p;
-  double t0 = tile_cost(p.bm, p.bn, M, N, K, cus) * 0.97;
+  double t0 = tile_cost(p.bm, p.bn, M, N, K, cus, turns) * 0.97;
   for (const Tile& t : TILES) {
     if (sw && t.bn == 192) continue;
-    const double c = tile_cost(t, M, N, K, cus);
+    const double c = tile_cost(t, M, N, K, cus, turns);
     if (c < t0) {
       t0 = c;
       p.bm = t.bm;
@@ -983,9 +989,16 @@ inline Plan refine(Plan p, long M, long N, long K, int cus, bool sw = false) {
 }
 
 // The tile of a gated product (B of N rows, gate and up)
-inline Plan gated_plan(long M, long N, long K, int cus) {
+inline Plan gated_plan(long M, long N, long K, int cus, bool turns) {
   const Plan p = plan(M, N, K, false, cus);
-  return refine(p.bm == 64 ? Plan{128, 128, 1} : p, M, N, K, cus, true);
+  return refine(p.bm == 64 ? Plan{128, 128, 1} : p, M, N, K, cus, turns, true);
+}
+
+inline int tile_of_rows(int M, int N, int K, int lda, int ldb, int gated) {
+  const bool turns = turns_pay(nullptr, nullptr, K, lda, ldb);
+  const int cus = cu_count();
+  const Plan p = gated ? gated_plan(M, N, K, cus, turns) : refine(plan(M, N, K, false, cus), M, N, K, cus, turns);
+  return p.bm << 16 | p.bn;
 }
 
 // Whether a product that the aligned, the persistent or the eight-wave 256x256 kernels take is better off on refine's
@@ -994,9 +1007,9 @@ inline Plan gated_plan(long M, long N, long K, int cus) {
 // 128-byte lines (wide below), where a K-step waits for twice the lines: 20 % have to be promised. us by eight waves / so: 2129 x 3728 x 4616
 // 103 / 89 (27 %), 1598 x 5680 x 4144 87 / 86 (22 %); below, what 55 products gain 1 % from on average 7756 x 6320 x 3816 loses 7 % of (349 / 372),
 // 3567 x 15328 x 928 6 % (108 / 114).
-inline bool finer(long M, long N, long K, int cus, bool sw = false, bool off = false) {
-  const Plan p = refine({256, 256, 1}, M, N, K, cus, sw);
-  return p.bm * p.bn < 65536 && tile_cost(p.bm, p.bn, M, N, K, cus) < (off ? 0.80 : 0.93) * tile_cost(TILES[0], M, N, K, cus);
+inline bool finer(long M, long N, long K, int cus, bool turns, bool sw, bool off) {
+  const Plan p = refine({256, 256, 1}, M, N, K, cus, turns, sw);
+  return p.bm * p.bn < 65536 && tile_cost(p.bm, p.bn, M, N, K, cus, turns) < (off ? 0.80 : 0.93) * tile_cost(LARGE, M, N, K, cus, false);
 }
 
 // Whether 256x256 tiles are plan's choice, or so near it that the eight-wave kernel of such tiles
@@ -1028,11 +1041,11 @@ inline double tr256_cost(long M, long N, long K, int cus) {
 // 256x256 tiles than CUs run on these (gemm_bf16.hip aligned_finer): 2304 x 8192 x 6912 255 / 296, 3072 x 6656 x 1536 69 / 83. Of 117 sizes of
 // more than 4096 rows that read transposed now 7 % on average, none loses more than 7 (11520 x 10752 x 384 119 / 111).
 inline bool turn_b(long M, long N, long K, int cus) {
-  const Plan p = refine(plan(M, N, K, true, cus), M, N, K, cus);
+  const Plan p = refine(plan(M, N, K, true, cus), M, N, K, cus, true);  // rows of a transposed B: as long as the plan takes them
   const bool aligned = M % 256 == 0 && N % 256 == 0 && K % 128 == 0 && (M / 256) * (N / 256) > cus;
-  const double nt = aligned ? tile_cost(TILES[0], M, N, K, cus)
+  const double nt = aligned ? tile_cost(LARGE, M, N, K, cus, false)
                     : p.ns > 1 || p.bm == 64 ? cost(M, N, K, p.bm == 64 ? 128 : p.bm, p.bm == 64 ? 128 : p.bn, p.ns, cus)
-                                             : tile_cost(p.bm, p.bn, M, N, K, cus);
+                                             : tile_cost(p.bm, p.bn, M, N, K, cus, true);
   return nt + 2.5 + 4.0 * N * K / 6.4e6 < tr256_cost(M, N, K, cus);
 }
 
@@ -1220,7 +1233,7 @@ int gemm_any(const void* A, const void* B, void* C, void* C2, const void* bias, 
   using namespace any;
   const int vec = ldc % 8 == 0 && (uintptr_t)C % 16 == 0 && (uintptr_t)C2 % 16 == 0;
   if (epi == EPI_ADDC && (!vec || N % 8)) return KGS_ERR_ALIGN;
-  const Plan p = bm ? Plan{bm, bn, ns} : refine(plan(M, N, K, ws != nullptr, cu_count()), M, N, K, cu_count());
+  const Plan p = bm ? Plan{bm, bn, ns} : refine(plan(M, N, K, ws != nullptr, cu_count()), M, N, K, cu_count(), turns_pay(A, B, K, lda, ldb));
   if (p.ns > 1 && ws == nullptr) return KGS_ERR_ARG;
   const Args a{(const unsigned short*)A, (const unsigned short*)B, C, (unsigned short*)C2, (const unsigned short*)bias,
                M, N, K, lda, ldb, ldc, 0, M > N, vec, 1.f, nullptr};
@@ -1250,7 +1263,7 @@ int gemm_any_swiglu(const void* A, const void* B, void* C, int M, int N, int K, 
   using namespace any;
   const Args a{(const unsigned short*)A, (const unsigned short*)B, C, nullptr, (const unsigned short*)limit,
                M, N, K, lda, ldb, ldc, 0, M > N, ldc % 8 == 0 && (uintptr_t)C % 16 == 0, 1.f, nullptr};
-  const Plan p = gated_plan(M, N, K, cu_count());
+  const Plan p = gated_plan(M, N, K, cu_count(), turns_pay(A, B, K, lda, ldb));
   const dim3 grid((unsigned)(ceil_div(M, p.bm) * ceil_div(N / 2, p.bn / 2)));
   const bool one = (int)grid.x <= cu_count();
 #define KGS_SWT(ACT)                                                                                                                     \
@@ -1315,7 +1328,9 @@ int gemm_any_f8(const void* A, const void* B, void* C, const void* bias, int M, 
   return (int)hipGetLastError();
 }
 
-bool gemm_any_finer(int M, int N, int K, bool sw, bool off) { return any::finer(M, N, K, cu_count(), sw, off); }
+bool gemm_any_finer(const void* A, const void* B, int M, int N, int K, int lda, int ldb, bool sw, bool off) {
+  return any::finer(M, N, K, cu_count(), any::turns_pay(A, B, K, lda, ldb), sw, off);
+}
 
 bool gemm_any_wide(int M, int N, int K, bool split) { return any::wide(M, N, K, split, cu_count()); }
 
@@ -1363,16 +1378,17 @@ KGS_EXPORT int kgs_gemm_bf16_tr_pair(const void* dY, const void* W, const void* 
 
 // The tile that gemm_any chooses without scratch, for a gated product (N rows of gate and up) if gated: rows << 16 | columns.
 KGS_EXPORT int kgs_gemm_bf16_nt_tile(int M, int N, int K, int gated) {
-  using namespace kgs::any;
-  if (M <= 0 || N <= 0 || K <= 0) return 0;
-  const int cus = kgs::cu_count();
-  const Plan p = gated ? gated_plan(M, N, K, cus) : refine(plan(M, N, K, false, cus), M, N, K, cus);
-  return p.bm << 16 | p.bn;
+  return M > 0 && N > 0 && K > 0 ? kgs::any::tile_of_rows(M, N, K, 64, 64, gated) : 0;
+}
+
+// The same of rows lda and ldb apart.
+KGS_EXPORT int kgs_gemm_bf16_nt_tile_rows(int M, int N, int K, int lda, int ldb, int gated) {
+  return M > 0 && N > 0 && K > 0 && lda >= K && ldb >= K ? kgs::any::tile_of_rows(M, N, K, lda, ldb, gated) : 0;
 }
 
 // Whether the kernels of 256x256 tiles leave a product (gated: of a gated projection; off: A's rows off the 128-byte lines) to a finer tile.
 KGS_EXPORT int kgs_gemm_bf16_nt_finer(int M, int N, int K, int gated, int off) {
-  return M > 0 && N > 0 && K > 0 && kgs::gemm_any_finer(M, N, K, gated != 0, off != 0);
+  return M > 0 && N > 0 && K > 0 && kgs::gemm_any_finer(nullptr, nullptr, M, N, K, off ? 8 : 64, 64, gated != 0, off != 0);
 }
 
 // Whether a K-major B is better transposed first than read by kgs_gemm_bf16 (turn_b).

@@ -171,7 +171,7 @@ int gemm_any(const void* A, const void* B, void* C, void* C2, const void* bias, 
              int ldc, int epi, int bm, int bn, int ns, float* ws, hipStream_t s);
 long gemm_any_ws(int M, int N, int K);
 bool gemm_any_wide(int M, int N, int K, bool split);
-bool gemm_any_finer(int M, int N, int K, bool sw, bool off);
+bool gemm_any_finer(const void* A, const void* B, int M, int N, int K, int lda, int ldb, bool sw, bool off);
 int gemm_any_f8(const void* A, const void* B, void* C, const void* bias, int M, int N, int Kw, int lda, int ldb, int ldc,
                 float alpha, const float* alpha_ptr, int epi, hipStream_t s);
 int gemm_any_swiglu(const void* A, const void* B, void* C, int M, int N, int K, int lda, int ldb, int ldc, int act,
@@ -191,14 +191,14 @@ static bool rows_ok(const void* A, const void* B, const void* C, int M, int N, i
   if (M <= 0 || N % 256 || K % 128 || K < 384 || (lda | ldb | ldc) % 8) return false;
   if (((uintptr_t)A | (uintptr_t)B | (uintptr_t)C) % 16) return false;
   if ((long)lda * 512 >= (1L << 31) || (long)ldb * 512 >= (1L << 31)) return false;
-  return ((long)M + 255) / 256 * (N / 256) > cu_count() && !gemm_any_finer(M, N, K, sw, false);
+  return ((long)M + 255) / 256 * (N / 256) > cu_count() && !gemm_any_finer(A, B, M, N, K, lda, ldb, sw, false);
 }
 
 // Aligned products of up to one 256x256 tile per CU that a finer tile fills better. Above that they stay on the
 // persistent kernel, on which the tests of its ticket slots and captured graphs launch such sizes through gemm_nt, though some lose by it:
 // us, so / on refine's tile, 5120 x 4096 x 4096 158 / 133, 2816 x 6144 x 5504 201 / 157, 8192 x 2560 x 4096 159 / 141, 4096 x 5120 x 14336 548 / 471.
-static bool aligned_finer(int M, int N, int K) {
-  return (long)(M / 256) * (N / 256) <= cu_count() && gemm_any_finer(M, N, K, false, false);
+static bool aligned_finer(const void* A, const void* B, int M, int N, int K, int lda, int ldb) {
+  return (long)(M / 256) * (N / 256) <= cu_count() && gemm_any_finer(A, B, M, N, K, lda, ldb, false, false);
 }
 
 template <int EPI>
@@ -342,7 +342,7 @@ KGS_EXPORT int kgs_gemm_bf16_nt_addc(const void* A, const void* B, void* C, int 
   using namespace kgs;
   if (M <= 0 || N <= 0 || K <= 0 || lda < K || ldb < K || ldc < N) return KGS_ERR_SHAPE;
   if (!kgs_gemm_bf16_nt_w4_ok(A, B, C, M, N, K, lda, ldb, ldc)) return KGS_ERR_ALIGN;
-  if (aligned_finer(M, N, K))
+  if (aligned_finer(A, B, M, N, K, lda, ldb))
     return gemm_any(A, B, C, nullptr, nullptr, M, N, K, lda, ldb, ldc, EPI_ADDC, 0, 0, 0, nullptr, stream);
   auto a = (const unsigned short*)A;
   auto b = (const unsigned short*)B;
@@ -388,7 +388,7 @@ static int gemm_nt(const void* A, const void* B, void* C, const void* bias, int 
   const int bounded = kgs_gemm_bf16_nt_bounded_ok(A, B, C, M, N, K, lda, ldb, ldc) && bias_ok;
   int v;
   if (variant == 0) {
-    const bool large = w4 && (long)(M / 256) * (N / 256) > 128 && !kgs::aligned_finer(M, N, K);
+    const bool large = w4 && (long)(M / 256) * (N / 256) > 128 && !kgs::aligned_finer(A, B, M, N, K, lda, ldb);
     if (!large && epi == kgs::EPI_NONE && kgs::rows_ok(A, B, C, M, N, K, lda, ldb, ldc)) {
       if (int* tq = kgs::tile_queue(stream))
         return (int)kgs::launch_w4p<kgs::EPI_NONE>((const unsigned short*)A, (const unsigned short*)B, (unsigned short*)C,
@@ -398,7 +398,7 @@ static int gemm_nt(const void* A, const void* B, void* C, const void* bias, int 
     // that nothing hides (us, its / the element-wise kernel's: 8192 x 8191 x 128 165 / 131, 3000 x 8001 x 64 65 / 50,
     // 6272 x 3085 x 128 55 / 49, x 256 57 / 56, x 512 66 / 71; 2048 x 3001 x 128 21 / 21)
     const bool short_odd = (ldc % 8 || (uintptr_t)C % 16) && K <= 256 && (long)M * N >= 1L << 23;
-    const bool off = !large && bounded && kgs_gemm_bf16_nt_off_lines(A, M, N, K, lda, ws != nullptr) && !kgs::gemm_any_finer(M, N, K, false, true);
+    const bool off = !large && bounded && kgs_gemm_bf16_nt_off_lines(A, M, N, K, lda, ws != nullptr) && !kgs::gemm_any_finer(A, B, M, N, K, lda, ldb, false, true);
     if (!large && !short_odd && !off && kgs::gemm_any_ok(A, B, M, N, K, lda, ldb))
       return kgs::gemm_any(A, B, C, nullptr, bias, M, N, K, lda, ldb, ldc, epi, 0, 0, 0, ws, stream);
     v = large ? 3 : off ? 16 : 2;

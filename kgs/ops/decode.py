@@ -601,6 +601,7 @@ def slab_split(m: int, n: int, k: int, cus: int = CUS) -> tuple[int, int] | None
     return _split(m, n, k, cus) if 0 < m <= SLAB_ROWS else None
 
 
+@lru_cache(maxsize=4096)
 def wide_split(m: int, n: int, k: int, cus: int = CUS) -> tuple[int, int] | None:
     """:func:`slab_split` of :func:`wide_slabs`, 97 to 128 rows. As many workgroups are the best there: us of the product alone at 128 rows in 2 / 4 / 8 / 16 slices 2048x2048 9.0 /
     6.7 / 6.5 / 8.4, 2048x8192 27.9 / 16.6 / 11.9 / 14.4, 6144x4096 by two tiles 23.6 / 17.1 / 20.3 (by one 18.6 in 2), 4096x14336 69 / 39.5 / 26.8 / 32.1."""
@@ -643,6 +644,7 @@ def _rows_tiles(m: int, n: int, k: int, cus: int) -> int | None:
     return 2 if m > 32 and n % 128 == 0 and 4 * (n // 128) >= 3 * cus else 1
 
 
+@lru_cache(maxsize=4096)
 def head_pays(m: int, n: int, k: int, cus: int = CUS) -> bool:
     """Whether 49 to 128 rows of an LM head on residual rows are better off on :func:`skinny_rows` (:func:`wide_rows`) than their norm's product
     with the rows of the weight: most of a round of workgroups or whole rounds, of K from 2048 on, where no four-wave tiles were measured to be better.
@@ -675,6 +677,7 @@ def rows_pay(m: int, n: int, k: int, gated: bool) -> bool:
     return k >= (3072 if m <= 64 or rounds == 1 else 5120)
 
 
+@lru_cache(maxsize=4096)
 def slabs_fill(m: int, n: int, k: int) -> bool:
     """Whether the slices of :func:`slab_split` are short or fill the CUs. A K like 11008 gives two slices of 43 ring rounds in a quarter of the workgroups
     that the CUs hold: the product and a hyper-connection step at 64 / 96 rows, over the general kernel's with the step, 4096x11008 1.65 / 1.82, 3072x14336 (slices of 3584,
@@ -719,24 +722,23 @@ def skinny_slabs(x: torch.Tensor, w: PackedWeight) -> torch.Tensor:
     """``x @ W^T`` of up to 96 rows of a bf16 weight as fp32 parts ``[slices, M, N]`` of its sum, for a consumer that adds them
     (native/kernels/decode_slabs.hip; :func:`slab_split`). Columns in the order in which the weight is packed."""
     m, k = _slab_operand(x, w)
-    return _slabs(x, w, m, k, slab_split, "skinny_slabs")
+    return _slabs(x, w, m, k, slab_split, _lib.lib().kgs_skinny_slabs)
 
 
 def wide_slabs(x: torch.Tensor, w: PackedWeight) -> torch.Tensor:
     """:func:`skinny_slabs` of 97 to 128 rows (:func:`wide_split`)."""
     m, k = _slab_operand(x, w)
-    return _slabs(x, w, m, k, wide_split, "wide_slabs")
+    return _slabs(x, w, m, k, wide_split, _lib.lib().kgs_wide_slabs)
 
 
-def _slabs(x, w, m, k, rule, name):
+def _slabs(x, w, m, k, rule, kernel):
     split = None if w.fp8 or w.swiglu else rule(m, w.n, k)
     if split is None:
         raise ValueError(f"no slices for x {tuple(x.shape)}, W [{w.n}, {w.k}]")
     out = torch.empty((split[1], m, w.n), dtype=torch.float32, device=x.device)
-    rc = getattr(_lib.lib(), "kgs_" + name)(w.data.data_ptr(), x.data_ptr(), out.data_ptr(), m, w.n, k, x.stride(0), *split,
-                                            _lib.stream_handle(x.device))
+    rc = kernel(w.data.data_ptr(), x.data_ptr(), out.data_ptr(), m, w.n, k, x.stride(0), *split, _lib.stream_handle(x.device))
     if rc:
-        _lib.check(rc, f"{name}[{m}x{w.n}x{k}, {split}]")
+        _lib.check(rc, f"slabs[{m}x{w.n}x{k}, {split}]")
     return out
 
 

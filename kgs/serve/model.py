@@ -793,7 +793,8 @@ class ServingModel:
         """Whether 97 to 128 rows take those layers, under the conditions of fewer; gate and up go by their routes on normed rows. Four
         layers, us a decode step of 97 / 128 rows by split tiles / so, contexts of 300: 2048 wide, feed-forward 8192 339, 370 / 312, 333; 4096,
         14336 636, 701 / 593, 652; 8192, 28672 1868, 1954 / 1726, 1828; Not 11008, whose slices do not fill the CUs."""
-        if self.packed is None or self.decode_fp8 or self.backend != "kgs" or not self.fuse_splitk or self.rope_attn or self.fused_max_batch <= 32:
+        if not D.SLAB_ROWS < m <= D.WIDE_ROWS or self.packed is None or self.decode_fp8 or self.backend != "kgs" or not self.fuse_splitk or self.rope_attn or \
+                self.fused_max_batch <= 32:
             return False
         P, c = self.packed[0], self.cfg
         return c.hidden % 2048 == 0 and c.hidden <= 8192 and bool(P["qkv"].rope) and all(
@@ -805,10 +806,9 @@ class ServingModel:
         499 / 439; 92 M 400 / 386, 510 / 448; 4096 wide, 67 M 386 / 381, 489 / 460; 92 M 440 / 382, 544 / 472; 218 M 576 / 479, 685 / 586). So with 97 to 128 rows, of 90 M
         on: split tiles / here, four layers and one prompt of 97, 112, 128 tokens, 2048 wide 61 M 403, 401, 402 / 421, 402, 406; 73 M 402, 403, 405 / 410, 412, 404; 4096 wide
         92 M 463, 464, 464 / 440, 450, 447; 143 M 510, 505, 516 / 451, 461, 474; 218 M at 97 and 128 599, 601 / 523, 567."""
-        if not (self._wide(m) or self._slabs_pay(m)):
+        if not (self._wide(m) if m > D.SLAB_ROWS else self._slabs_pay(m)):
             return False
-        weights = sum(w.n * w.k for w in self.packed[0].values())
-        return weights >= (72_000_000 if m <= 48 else 90_000_000 if m > D.SLAB_ROWS else 0)
+        return 48 < m <= D.SLAB_ROWS or sum(w.n * w.k for w in self.packed[0].values()) >= (72_000_000 if m <= 48 else 90_000_000)
 
     def _slab_gate(self, m: int):
         """Gate and up of ``m`` rows of :meth:`_slab_layers`: a route of :meth:`_swiglu_route` on normed rows, or None: :func:`kgs.ops.decode.skinny_rows` on the

@@ -867,7 +867,9 @@ inline bool turns_pay(const void* A, const void* B, int K, int lda, int ldb) {
   return (lda % 64 == 0 && ldb % 64 == 0 && ((uintptr_t)A | (uintptr_t)B) % 128 == 0) || K <= 1024;
 }
 
-// An unsliced launch of tiles with a CU each; two stages hold all of a K up to 128
+// An unsliced launch of tiles with a CU each. Those of 128 columns run on lds_stages but for K of 65 to 128, all of which two stages hold: there is no
+// difference (192x128 tiles of 965 x 5456 x 72 and x 128 9.8, 9.8 us on two, 9.8, 9.7 on three), while of one K-tile two stages walk two (x 64 9.9 / 8.9; 4000 x 6000 x 64 by
+// 224x128 20.2 / 18.2).
 template <int EPI, int BM, int BN, bool DUAL, int SW = 0>
 void launch_mid(const Args& a, hipStream_t s) {
   const long tiles = (long)ceil_div(a.M, BM) * (SW ? ceil_div(a.N / 2, BN / 2) : ceil_div(a.N, BN));
@@ -877,7 +879,7 @@ void launch_mid(const Args& a, hipStream_t s) {
         hipLaunchKernelGGL((gemm_nt_turn<EPI, BM, BN, DUAL, SW>), dim3((unsigned)cu_count()), dim3(256), 0, s, a, q);
         return;
       }
-  } else if (a.K > 2 * BK) {
+  } else if (a.K <= BK || a.K > 2 * BK) {
     hipLaunchKernelGGL((gemm_nt_deep<EPI, BM, BN, DUAL, SW>), dim3((unsigned)tiles), dim3(256), 0, s, a);
     return;
   }

@@ -581,7 +581,8 @@ def own_gemm(x: torch.Tensor, w: PackedWeight, out: torch.Tensor | None = None, 
     """:func:`skinny_gemm` with ``norm`` or ``resid``, by :func:`skinny_few` where that is the better one (:func:`few_route`)."""
     m, k = x.shape
     plain = not norm and rope is None
-    if not w.fp8 and few_wide(m, w.n, k):
+    # what skinny_gemm takes and skinny_few does not stays there: rows further apart than 32-bit offsets reach, an out of another shape; and what it refuses
+    if not w.fp8 and few_wide(m, w.n, k) and x.stride(0) <= 1 << 25 and (out is None or out.shape == (m, w.n_out)) and not (norm and resid):
         return skinny_few(x, w, out, norm, resid, eps, rope)
     if m <= 16 and not w.fp8 and (few_route(m, w.n, k, plain) or (few_takes(m, w.n, k, False, plain) and not (
             skinny_takes(m, w.n, k) if plain else _own_by_skinny(m, w.n, k, False, bool(w.rope))))):

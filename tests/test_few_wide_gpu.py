@@ -74,3 +74,20 @@ def test_parts_are_summed_apart(n, k, parts, m):
     for part in p[1:]:
         want = want + part
     assert torch.equal(D.skinny_few(x, pw), want.bfloat16())  # the same products in the same order: the same bits
+
+
+def test_calls_that_only_the_other_kernel_takes():
+    """own_gemm of 17 to 32 rows, as it was before these rows had a kernel of few: rows far apart and an out inside a wider one are computed, a norm with a residual is refused."""
+    m, n, k, ld = 17, 2048, 1024, (1 << 25) + 8
+    w = (torch.randn(n, k, device="cuda") * k ** -0.5).bfloat16()
+    pw, rows = D.PackedWeight(w), torch.randn(m, k, device="cuda").bfloat16()
+    far = torch.empty((m - 1) * ld + k, device="cuda", dtype=torch.bfloat16).as_strided((m, k), (ld, 1))
+    far.copy_(rows)
+    ref = rows.double() @ w.double().T
+    _close(D.own_gemm(far, pw), ref)
+    out = torch.full((m + 2, n), 7.0, device="cuda", dtype=torch.bfloat16)
+    D.own_gemm(rows, pw, out=out)
+    _close(out[:m], ref)
+    assert bool((out[m:] == 7).all())
+    with pytest.raises(ValueError):
+        D.own_gemm(rows, pw, out=out[:m], norm=True, resid=True)

@@ -308,7 +308,7 @@ _MEASURED = {key[1:] for key in (*W4X_TUNED, *SPLITK_TUNED)}
 
 
 def w4x_stages(route) -> int:
-    """LDS stages of a W4X_TUNED route (2 unless the entry names 3 or 4)."""
+    """LDS stages that a W4X_TUNED route asks for (2 unless the entry names 3 or 4; tiles smaller than 256x256 run on three or four in any case)."""
     return route[3] if len(route) > 3 else 2
 
 

@@ -230,7 +230,7 @@ def _w4x_flags(packed: int, stages: int, nt_weights: bool = False) -> int:
     if stages not in (2, 3, 4):
         raise ValueError(f"stages must be 2, 3 or 4, got {stages}")
     if nt_weights and stages != 2:
-        raise ValueError("nt_weights runs with two LDS stages only")
+        raise ValueError("nt_weights goes with the default stages only")
     return packed | (2 if nt_weights else 0) | (stages - 2) << 4
 
 
@@ -267,7 +267,7 @@ def gemm_nt_w4x(a: torch.Tensor, b, bn: int = 256, nslice: int = 1,
     or a :class:`PanelWeight` packed with the same ``bn``. ``stages``: LDS
     stages asked for (refused where they do not fit in 160 KiB; tiles smaller than 256x256 take three or four in any case: the same bits).
     ``nt_weights``: ``b``'s loads non-temporal (decode weights each CU streams
-    once), ``a``'s loads default (two stages only). ``private``: partials in a buffer of
+    once; with the default ``stages``), ``a``'s loads default. ``private``: partials in a buffer of
     this call's own instead of the per-GPU workspace."""
     _check_operand(a, "a")
     b, bshape, ldb, packed = _packed_operand(b, bn, False)
@@ -373,7 +373,7 @@ def gemm_nt_w4x_swiglu(a: torch.Tensor, w_gate_up, bn: int = 128,
                        out: torch.Tensor | None = None, bm: int = 256, stages: int = 2,
                        nt_weights: bool = False, act="silu") -> torch.Tensor:
     """``act(a @ gate.T) * (a @ up.T)`` (``act``: silu, or gelu_tanh or a clamped
-    :class:`kgs.ops.activation.Gate` with a row-major weight and two stages) for a fused gate|up weight ``[2I, K]``
+    :class:`kgs.ops.activation.Gate` with a row-major weight and the default ``stages``) for a fused gate|up weight ``[2I, K]``
     (gate rows first) on the four-wave kernel, the SwiGLU applied in the GEMM
     epilogue: returns ``[M, I]`` (both products rounded to bf16 first, as
     ``gemm_nt`` + ``kgs.ops.transformer.silu_mul`` round them). Any M;

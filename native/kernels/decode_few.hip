@@ -1,8 +1,8 @@
-// Skinny products of up to 16 rows (plain ones 32): y[M, N] = x[M, K] . W^T, W packed as for decode.hip's skinny
+// Skinny products of up to 32 rows (with a norm or a rotation of K of 512, from 17 rows on of 1024): y[M, N] = x[M, K] . W^T, W packed as for decode.hip's skinny
 // ([N/16][K/32][64][8]), with that kernel's epilogues and one statistic of its own.
 //
 // A workgroup of NW waves takes R 16-row tiles of W; the waves share out K, stream their part of W and of x through a ring of PF k-steps and add
-// their sums in LDS, in the order of the waves. Loads are buffer loads, so that a step waits for exactly its own. The last round sends for nothing:
+// their sums in LDS, in the order of K's parts (few_parts). Loads are buffer loads, so that a step waits for exactly its own. The last round sends for nothing:
 // the last k-steps fetched again, as the ring did, were waited for at the end of the launch, 0.5 to 1 us of a short one and a
 // tenth of a long one.
 //

@@ -935,8 +935,8 @@ KGS_EXPORT int kgs_gemm_bf16_nt_w4x(const void* A, const void* B, void* C, float
 
 // flags bit 0: B is the tile-panel-major copy of a [N, K] weight
 // ([N / bn][K / 64][bn][64], kgs.ops.gemm.pack_w4x_weight) and ldb must be K;
-// bit 1: B's loads non-temporal (two stages only); bits 4-5: LDS stages - 2
-// (0..2, where they fit in 160 KiB)
+// bit 1: B's loads non-temporal (then bits 4-5 are 0); bits 4-5: LDS stages - 2 asked
+// for (0..2, refused where they do not fit in 160 KiB; a tile's own are stage_bits')
 KGS_EXPORT int kgs_gemm_bf16_nt_w4x_ex(const void* A, const void* B, void* C, float* ws, int M, int N, int K,
                                        int lda, int ldb, int ldc, int bn, int nslice, int bm, int flags,
                                        hipStream_t stream) {
@@ -988,10 +988,10 @@ KGS_EXPORT int kgs_gemm_bf16_nt_w4x_swiglu(const void* A, const void* B, void* C
 }
 
 // flags bit 0: B is the SwiGLU-packed copy of the fused gate|up weight
-// (kgs.ops.gemm.pack_w4x_weight(..., swiglu=True)), ldb must be K; bits 4-5:
-// LDS stages - 2 (as kgs_gemm_bf16_nt_w4x_ex); bit 6: tanh gelu instead of silu;
+// (kgs.ops.gemm.pack_w4x_weight(..., swiglu=True)), ldb must be K; bits 1, 4-5
+// as for kgs_gemm_bf16_nt_w4x_ex; bit 6: tanh gelu instead of silu;
 // bit 7: the clamped gate with the limit at `limit` (fp32, on the device); both with
-// row-major B, two stages
+// row-major B and bits 4-5 0
 KGS_EXPORT int kgs_gemm_bf16_nt_w4x_swiglu_ex(const void* A, const void* B, void* C, int M, int N, int K, int lda,
                                               int ldb, int ldc, int bn, int bm, int flags, const void* limit,
                                               hipStream_t stream) {

@@ -15,7 +15,7 @@
 // row, 2.0 at 16. Nothing here depends on the order in which workgroups arrive.
 //
 // Bound by memory where W is large (28672 x 4096 at 1 row 36.4 us, 6.5 TB/s; 40.6 before), else by the launch and one trip through
-// memory and the ring (4096 x 4096 7.0 us, before 7.5; 2048 x 2048 3.6, 4.3). The split (few_split): few waves with long rings, whose loads are all in flight
+// memory and the ring (4096 x 4096 7.1 us, before 7.5; 2048 x 2048 3.6, 4.3). The split (few_split): few waves with long rings, whose loads are all in flight
 // at once and whose sums are soon added -- us at 8 rows with 8 / 4 / 2 / 1 waves, as long rings as fit: 2048x2048 4.3 / 4.2 / 4.0 / 4.6, 4096x4096 7.4 / 7.2 /
 // 7.0 / 8.4, 6144x4096 12.4 / 11.7 / 10.9 / 10.2, 16384x2048 12.3 / 13.6 / 12.4 / 12.2, 28672x4096 36.2 / 39.7 / 36.6 / 36.2; eight for long sums of up to 4 rows (4096x14336 at 1
 // row 18.5, by two 19.8; at 8 20.7, 19.2). Two tiles a workgroup where x counts: 6144x4096 at 16 rows 12.1 / 11.0, 28672x4096 at 16 40.8 / 40.3. At 24 / 32 rows, skinny / here:

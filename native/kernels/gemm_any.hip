@@ -154,7 +154,7 @@ __device__ __forceinline__ void store_row(const Args& a, int r, int col, const f
 // act(gate) * up; a tile stages both halves' rows in turn (gemm_w4.h). `bias` then points to the
 // clamped gate's limit.
 //
-// Two-stage tiles of a workgroup a CU take turns in one launch of a workgroup a CU (TURNS, take_turns): the last two K-steps of a tile send for the
+// Two-stage tiles of a workgroup a CU take turns in one launch of a workgroup a CU (TURNS, turns_pay): the last two K-steps of a tile send for the
 // first two K-tiles of the next and read its first fragments, so that between tiles a wave only has its epilogue. us, a
 // workgroup a tile / so: 3001 x 7000 x 200 23.4 / 21.3, 5000 x 5000 x 1000 56.1 / 54.1, 6000 x 9000 x 1000 120.8 / 114.6, 8192 x 14336 x 1024 227 / 213. Bound by
 // the matrix cores' power: what the gaps no longer cost comes off the clock. Tiles and resources are worked out from the arguments read anew at each turn:
